@@ -97,13 +97,11 @@ struct NttArgs {
     const uint64_t *barrett;  // [tables][2]
     const LimbJob *jobs;      // explicit list (then in/out limbs are absolute, no prologue/epilogue)
     uint32_t n_jobs;
-    const LimbGroup *groups;  // partition of `jobs` into runs with one table each (required with `jobs`)
+    const LimbGroup *groups;  // partition of `jobs` into runs with one table each, or nullptr
     uint32_t n_groups;
     uint32_t items;           // list mode: the whole list is applied to `items` buffers (0 = 1) ...
     size_t item_stride;       // ... that lie item_stride words apart
     uint32_t batch, n_polys;  // filled in by the launcher
-    uint32_t unit_filter;     // blocks pass of a mixed launch run as two kernels (filled in by the launcher): 1 = only the
-                              // units whose prime is below 2^50, 2 = only the others, 0 = every unit
     uint32_t log_n;
     LimbMap map;
     int pro_mode;
@@ -149,8 +147,11 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
 // rows_skipped: only the blocks pass is launched; a forward transform with NTT_PRO_SOURCE_INTT_REDUCE finishes it.
 hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, hipStream_t s, bool blocks_done = false,
                               bool rows_skipped = false);
-// whether a forward launch of n_jobs limbs may take NTT_PRO_SOURCE_INTT_REDUCE (2^15 <= N <= 2^16, a launch small
-// enough to run on quarter tiles, every table below 64)
+// The passes by themselves (ntt_passes.hip), prologue / epilogue included; the rows pass of an inverse transform takes
+// its input from a.in.
+hipError_t launch_ntt_rows(const NttArgs &a, uint32_t n_jobs, bool forward, int backend, hipStream_t s);
+hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int backend, hipStream_t s);
+// whether a forward launch of n_jobs limbs may take NTT_PRO_SOURCE_INTT_REDUCE
 bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables);
 
 // Tensor product of two size-2 ciphertexts fused with the blocks pass of the inverse transform of its third polynomial

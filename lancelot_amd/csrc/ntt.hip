@@ -7,17 +7,14 @@
 //
 // Decomposition for the GPU: N = R x 256.  A limb is an R x 256 row-major matrix.
 //   rows pass   : the first log2(R) stages pair elements that are whole rows apart.  A workgroup owns a
-//                 tile of R rows x C columns (4096 elements, 32 KiB) in LDS; global accesses run along the
-//                 columns (C consecutive words per row).
-//   blocks pass : the last 8 stages stay inside one row (256 consecutive words).  A workgroup owns 16
-//                 rows (4096 consecutive words).
-// Inside a pass each thread takes 2^r elements into registers, runs r stages on them (r <= 4, radix-16) and
-// hands them on; the stages of a pass form two such register blocks.  In the blocks pass both blocks take
-// their elements from LDS and write them back.  In the rows pass (N >= 2^12) the outer block works on the
-// words that a coalesced access of the tile gives the thread anyway, straight from or to global memory, and
-// only the exchange between the two blocks goes through LDS (rows_direct below).  LDS indices are skewed by
+//                 tile of R rows x C columns in LDS; global accesses run along the columns (C consecutive words
+//                 per row).
+//   blocks pass : the last 8 stages stay inside one row (256 consecutive words), which a wave owns.
+// The passes themselves are in ntt_passes.hip.  The forward transform runs rows pass then blocks pass, the inverse
+// the other way round.  This file holds what replaces or fuses them: the whole-limb kernel of the small degrees, the base
+// conversions with the rows pass that follows, the inner product with the blocks pass before it, the tensor product
+// with the inverse blocks pass after it.  Fused kernels work on 8 or 16 words per thread; their LDS indices are skewed by
 // one word per 16 so that both the stride-16 and the stride-256 gathers of a wave hit distinct banks.
-// The forward transform runs rows pass then blocks pass, the inverse the other way round.
 //
 // Two arithmetic back ends share this skeleton:
 //   integer : 64-bit Shoup/Harvey butterflies, any prime below 2^61 (~35 VALU instructions per butterfly);
@@ -32,557 +29,14 @@
 
 #include "kernels.h"
 #include "modarith.cuh"
+#include "ntt_common.cuh"
 
 namespace he {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr int kTileLog = 12;
-constexpr uint32_t kTile = 1u << kTileLog;
-constexpr uint32_t kLdsWords = kTile + (kTile >> 4);
-
-__device__ __forceinline__ uint32_t skew(uint32_t e) { return e + (e >> 4); }
-
-// Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global load and
-// store of the wave, which would serialise a prefetch issued before it with the butterflies after it.
-__device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
-
-// Workgroups are dealt round-robin to the 8 XCDs; give every XCD a contiguous range of logical ids so
-// that the tiles of one limb (which share a twiddle table) meet in one L2.
-__device__ __forceinline__ uint32_t logical_block() {
-    uint32_t b = blockIdx.x, n = gridDim.x;
-    if (n % 8 == 0) return (b % 8) * (n / 8) + b / 8;
-    return b;
-}
-
-struct Job {
-    const uint64_t *in;
-    uint64_t *out;
-    uint32_t table;
-    uint32_t poly;
-    uint32_t limb;
-    const uint64_t *src;   // NTT_PRO_SOURCE_[INTT_]REDUCE (rows pass only): the limb that is reduced into this one
-    uint32_t src_table;    // NTT_PRO_SOURCE_INTT_REDUCE: its prime
-};
-
-__device__ __forceinline__ Job decode_job(const NttArgs &a, uint32_t job) {
-    Job j;
-    const size_t n = (size_t)1 << a.log_n;
-    if (a.jobs) {
-        // job = item * n_jobs + entry of the list
-        const uint32_t item = job / a.n_jobs;
-        LimbJob lj = a.jobs[job - item * a.n_jobs];
-        j.in = a.in + item * a.item_stride + (size_t)lj.data_limb * n;
-        j.out = a.out + item * a.item_stride + (size_t)lj.data_limb * n;
-        j.table = lj.table;
-        j.poly = 0;
-        j.limb = 0;
-        const bool sourced = a.pro_mode == NTT_PRO_SOURCE_REDUCE || a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE;
-        j.src_table = sourced ? lj.data_limb / a.pro_lk : 0;
-        j.src = sourced ? a.pro_src + item * a.pro_item_stride + (size_t)j.src_table * n : nullptr;
-    } else {
-        j.poly = job / a.map.limbs;
-        j.limb = job % a.map.limbs;
-        j.in = a.in ? a.in + ((size_t)j.poly * a.in_poly_stride + j.limb) * n : nullptr;
-        j.out = a.out + ((size_t)j.poly * a.out_poly_stride + j.limb) * n;
-        j.table = map_table(a.map, j.limb);
-        j.src = a.pro_src + ((size_t)j.poly * a.pro_poly_stride << a.log_n);
-        j.src_table = a.pro_src_table;
-    }
-    return j;
-}
-
-// Per-limb constants of one back end.
-struct IntCtx {
-    uint64_t q;
-    const uint64_t *tw;
-};
-
-struct FpCtx {
-    FpMod m;
-    const double *tw;
-};
-
-__device__ __forceinline__ IntCtx int_ctx(const NttArgs &a, uint32_t table) {
-    return IntCtx{a.moduli[table], a.tw + ((size_t)table << (a.log_n + 1))};
-}
-
-__device__ __forceinline__ FpCtx fp_ctx(const NttArgs &a, uint32_t table) {
-    const double *c = a.fp_consts + 4 * (size_t)table;
-    return FpCtx{FpMod{c[0], c[1]}, a.tw_fp + ((size_t)table << a.log_n)};
-}
-
-// r stages on a tile held in LDS.  Tile index bits: [upper][mid: r bits][lower: low_bits]; the 2^r
-// elements of a group differ in `mid`.  idx_base + upper is the twiddle index of the group's first stage.
-template <int LOGR, bool FWD>
-__device__ __forceinline__ void tile_pass(uint64_t *lds, uint32_t tile_elems, uint32_t low_bits, uint32_t idx_base,
-                                          IntCtx c) {
-    constexpr int R = 1 << LOGR;
-    const uint32_t groups = tile_elems >> LOGR;
-    const uint32_t low_mask = (1u << low_bits) - 1;
-    for (uint32_t g = threadIdx.x; g < groups; g += blockDim.x) {
-        const uint32_t upper = g >> low_bits;
-        const uint32_t base = (upper << (low_bits + LOGR)) | (g & low_mask);
-        uint64_t v[R];
-#pragma unroll
-        for (int j = 0; j < R; j++) v[j] = lds[skew(base + ((uint32_t)j << low_bits))];
-        if (FWD)
-            ct_block<LOGR>(v, c.tw, idx_base + upper, c.q);
-        else
-            gs_block<LOGR>(v, c.tw, idx_base + upper, c.q);
-#pragma unroll
-        for (int j = 0; j < R; j++) lds[skew(base + ((uint32_t)j << low_bits))] = v[j];
-    }
-}
-
-template <int LOGR, bool FWD, bool REDUCE_FIRST>
-__device__ __forceinline__ void tile_pass_fp(uint64_t *lds, uint32_t tile_elems, uint32_t low_bits, uint32_t idx_base,
-                                             FpCtx c, uint32_t first = threadIdx.x, uint32_t stride = blockDim.x) {
-    constexpr int R = 1 << LOGR;
-    double *ld = reinterpret_cast<double *>(lds);
-    const uint32_t groups = tile_elems >> LOGR;
-    const uint32_t low_mask = (1u << low_bits) - 1;
-    for (uint32_t g = first; g < groups; g += stride) {
-        const uint32_t upper = g >> low_bits;
-        const uint32_t base = (upper << (low_bits + LOGR)) | (g & low_mask);
-        double v[R];
-#pragma unroll
-        for (int j = 0; j < R; j++) v[j] = ld[skew(base + ((uint32_t)j << low_bits))];
-        if (FWD)
-            fp_ct_block<LOGR, REDUCE_FIRST>(v, c.tw, idx_base + upper, c.m);
-        else
-            fp_gs_block<LOGR, REDUCE_FIRST>(v, c.tw, idx_base + upper, c.m);
-#pragma unroll
-        for (int j = 0; j < R; j++) ld[skew(base + ((uint32_t)j << low_bits))] = v[j];
-    }
-}
-
-template <int LD>
-struct Split {
-    static constexpr int p0 = LD >= 7 ? 4 : (LD >= 5 ? 3 : LD);
-    static constexpr int p1 = LD - p0;
-};
-
-// TL = log2(words per tile): 12, or 10 when a launch has too few limbs to give every CU a 4096-word tile
-template <int LD, int TL>
-__device__ __forceinline__ constexpr int log_cols() {
-    return (TL - LD) < 8 ? (TL - LD) : 8;
-}
-
-// (N^-1 [* w]) as an FP twiddle for the last multiplication of the inverse transform
-__device__ __forceinline__ FpTw inverse_scale(const NttArgs &a, const Job &job, FpMod m) {
-    const double *c = a.fp_consts + 4 * (size_t)job.table;
-    FpTw ninv{c[2], c[3]};
-    if (a.epi_mode != NTT_EPI_MUL) return ninv;
-    const double w = fp_canonical(fp_mulmod(fp_from_u64(a.w[2 * job.limb]), ninv, m), m);
-    return FpTw{w, w * m.qinv};
-}
-
-// ---------------------------------------------------------------------------------------------------
-// rows pass with 16 words per thread (N >= 2^12: a tile of 2^LD rows x C columns is 16 T words for its T threads).
-// The stages split into an outer block of p0 and an inner block of p1 = LD - p0 stages.  The words of a thread's
-// outer groups are t, t + T, ..., t + 15 T in tile order, i.e. what a coalesced load of the tile hands to thread t
-// anyway, so the outer block runs on registers straight from (forward) or to (inverse) global memory and the
-// tile crosses LDS once, between the blocks, instead of three times (no LDS at all when p1 = 0): the pass is
-// bound by the latency of one workgroup, and two of its three LDS round trips and barriers go away.  Same
-// arithmetic, same words.
-//   outer: register i is tile word t + T i; group k of 16 >> p0 holds registers k + (16 >> p0) j; twiddle index 1
-//   inner: group k of 16 >> p1 is group g = t + T k of the tile: registers k 2^p1 + j are the tile words
-//          ((g / C) << (LOGC + p1)) + g mod C + j C; twiddle index 2^p0 + g / C
-// Tile word e lives at row e / C, column col0 + e mod C of the limb's (N / 256) x 256 view.
-// ---------------------------------------------------------------------------------------------------
-// SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first, on the
-// same registers: its last block leaves the coefficient of tile word t + T i in register i, which is where the forward
-// pass's first block takes its input from.
-template <int LD, bool FWD, int BE, int LOGC, bool SRC_INTT = false>
-__device__ __forceinline__ void rows_direct(const NttArgs &a, const Job &job, uint32_t col0, uint64_t *lds) {
-    constexpr int p0 = Split<LD>::p0, p1 = Split<LD>::p1;
-    constexpr int R0 = 1 << p0, R1 = 1 << p1, NG0 = 16 >> p0, NG1 = 16 >> p1;
-    constexpr uint32_t C = 1u << LOGC, T = 1u << (LD + LOGC - 4);
-    const uint32_t t = threadIdx.x, col = t & (C - 1);
-    double *ld = reinterpret_cast<double *>(lds);
-    // tile word, global offset and LDS slot of register i in the outer and in the inner layout (folded to a few
-    // shifts and adds where they are used; tables of them would have to stay live across both back ends)
-    auto e_far = [&](int i) { return t + T * (uint32_t)i; };
-    auto e_near = [&](int i) {
-        const uint32_t upper = (t + T * (uint32_t)(i >> p1)) >> LOGC;
-        return (upper << (LOGC + p1)) + col + ((uint32_t)(i & (R1 - 1)) << LOGC);
-    };
-    auto glob = [&](uint32_t e) { return (size_t)(e >> LOGC) * 256 + col0 + col; };
-    auto idx_near = [&](int k) { return (1u << p0) + ((t + T * (uint32_t)k) >> LOGC); };
-    // the outer / inner block on every group of the 16 registers
-    auto outer = [&](auto *v, auto block) {
-#pragma unroll
-        for (int k = 0; k < NG0; k++) {
-            std::remove_reference_t<decltype(v[0])> w[R0];
-#pragma unroll
-            for (int j = 0; j < R0; j++) w[j] = v[k + NG0 * j];
-            block(w, 1u);
-#pragma unroll
-            for (int j = 0; j < R0; j++) v[k + NG0 * j] = w[j];
-        }
-    };
-    auto inner = [&](auto *v, auto block) {
-#pragma unroll
-        for (int k = 0; k < NG1; k++) block(v + k * R1, idx_near(k));
-    };
-    // canonical coefficients of the source limb at the tile words t + T i
-    uint64_t s[SRC_INTT ? 16 : 1];
-    if constexpr (SRC_INTT) {
-        const uint32_t st = job.src_table;
-        // (the tables of the inverse transform lie behind the forward ones: a.tw / a.tw_fp are the forward launch's)
-        if ((a.pro_src_fp_mask >> st) & 1) {
-            const FpMod m = fp_ctx(a, st).m;
-            const double *itw = a.pro_itw_fp + ((size_t)st << a.log_n);
-            double v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = __longlong_as_double((long long)job.src[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))]);
-            if (p1 > 0) {
-                inner(v, [&](double *w, uint32_t idx) { fp_gs_block<(p1 > 0 ? p1 : 1), true>(w, itw, idx, m); });
-#pragma unroll
-                for (int j = 0; j < 16; j++) ld[skew(e_near(j))] = v[j];
-                __syncthreads();
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = ld[skew(e_far(j))];
-            }
-            outer(v, [&](double *w, uint32_t idx) { fp_gs_block<p0, true>(w, itw, idx, m); });
-            const double *cc = a.fp_consts + 4 * (size_t)st;
-            const FpTw ninv{cc[2], cc[3]};
-#pragma unroll
-            for (int j = 0; j < 16; j++) s[SRC_INTT ? j : 0] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, m), m));
-        } else {
-            const uint64_t q = a.moduli[st];
-            const uint64_t *itw = a.pro_itw + ((size_t)st << (a.log_n + 1));
-            uint64_t v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = job.src[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))];
-            if (p1 > 0) {
-                inner(v, [&](uint64_t *w, uint32_t idx) { gs_block<(p1 > 0 ? p1 : 1)>(w, itw, idx, q); });
-#pragma unroll
-                for (int j = 0; j < 16; j++) lds[skew(e_near(j))] = v[j];
-                __syncthreads();
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = lds[skew(e_far(j))];
-            }
-            outer(v, [&](uint64_t *w, uint32_t idx) { gs_block<p0>(w, itw, idx, q); });
-#pragma unroll
-            for (int j = 0; j < 16; j++) s[SRC_INTT ? j : 0] = reduce_2q(v[j], q);
-        }
-        // (the forward pass below writes and reads the same LDS slots in the same order as the inverse pass read and
-        // wrote them: a thread's own slots t + T i first, then a barrier)
-    }
-    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) {
-        const FpCtx c = fp_ctx(a, job.table);
-        double v[16];
-        if (FWD) {
-            bool reduce_first = true;
-            if constexpr (SRC_INTT) {
-                const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = fp_from_u64(barrett64(s[SRC_INTT ? j : 0], q, r1));
-                reduce_first = false;
-            } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
-                const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-                const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
-                const FpMod ml = fp_ctx(a, a.pro_last).m;
-                const double wd = fp_from_u64(a.pro_w[2 * job.limb]), wl = fp_from_u64(a.pro_w[2 * a.pro_last]);
-                const FpTw w{wd, wd * c.m.qinv}, wlast{wl, wl * ml.qinv};
-                const uint64_t qj = a.moduli[job.table], rj = a.barrett[2 * job.table + 1];
-                const uint64_t qlast = a.moduli[a.pro_last], rlast = a.barrett[2 * a.pro_last + 1];
-#pragma unroll
-                for (int j = 0; j < 16; j++) {
-                    const uint64_t ds = dsrc[glob(e_far(j))];
-                    const uint64_t dl = a.pro_k1 ? barrett64(ds, qlast, rlast) : ds;
-                    const uint64_t dj = a.pro_k1 ? barrett64(ds, qj, rj) : job.in[glob(e_far(j))];
-                    // coefficient of the dropped limb of the ModDown result, canonical mod q_last
-                    const double r = fp_canonical(fp_from_u64(tsrc[glob(e_far(j))]) - fp_mulmod(fp_from_u64(dl), wlast, ml), ml);
-                    v[j] = fp_mulmod(fp_from_u64(dj), w, c.m) + fp_reduce(r, c.m);
-                }
-            } else if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE) {
-                // one source limb for every limb: it may exceed this limb's prime, so reduce first
-                const uint64_t *src = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = fp_from_u64(src[glob(e_far(j))]);
-            } else if (a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
-                const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = fp_from_u64(barrett64(job.src[glob(e_far(j))], q, r1));
-                reduce_first = false;
-            } else {
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = fp_from_u64(job.in[glob(e_far(j))]);
-                reduce_first = false;
-            }
-            if (reduce_first)
-                outer(v, [&](double *w, uint32_t idx) { fp_ct_block<p0, true>(w, c.tw, idx, c.m); });
-            else
-                outer(v, [&](double *w, uint32_t idx) { fp_ct_block<p0, false>(w, c.tw, idx, c.m); });
-            if (p1 > 0) {
-#pragma unroll
-                for (int j = 0; j < 16; j++) ld[skew(e_far(j))] = v[j];
-                __syncthreads();
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = ld[skew(e_near(j))];
-                inner(v, [&](double *w, uint32_t idx) { fp_ct_block<(p1 > 0 ? p1 : 1), true>(w, c.tw, idx, c.m); });
-            }
-            // lazy signed doubles go to the blocks pass
-#pragma unroll
-            for (int j = 0; j < 16; j++) job.out[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))] = (uint64_t)__double_as_longlong(v[j]);
-        } else {
-            // input: lazy signed doubles from the blocks pass; output: canonical residues
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = __longlong_as_double((long long)job.in[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))]);
-            if (p1 > 0) {
-                inner(v, [&](double *w, uint32_t idx) { fp_gs_block<(p1 > 0 ? p1 : 1), true>(w, c.tw, idx, c.m); });
-#pragma unroll
-                for (int j = 0; j < 16; j++) ld[skew(e_near(j))] = v[j];
-                __syncthreads();
-#pragma unroll
-                for (int j = 0; j < 16; j++) v[j] = ld[skew(e_far(j))];
-            }
-            outer(v, [&](double *w, uint32_t idx) { fp_gs_block<p0, true>(w, c.tw, idx, c.m); });
-            const FpTw scale = inverse_scale(a, job, c.m);
-#pragma unroll
-            for (int j = 0; j < 16; j++)
-                job.out[glob(e_far(j))] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, c.m), c.m));
-        }
-        return;
-    }
-
-    const IntCtx c = int_ctx(a, job.table);
-    const uint64_t q = c.q;
-    uint64_t v[16];
-    if (FWD) {
-        if constexpr (SRC_INTT) {
-            const uint64_t r1 = a.barrett[2 * job.table + 1];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = barrett64(s[SRC_INTT ? j : 0], q, r1);
-        } else if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE || a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
-            const uint64_t r1 = a.barrett[2 * job.table + 1];
-            const uint64_t *src = a.pro_mode == NTT_PRO_SOURCE_REDUCE ? job.src : a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = barrett64(src[glob(e_far(j))], q, r1);
-        } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
-            const uint64_t r1 = a.barrett[2 * job.table + 1];
-            const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-            const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
-            const uint64_t ql = a.moduli[a.pro_last];
-            const Shoup w = load_shoup(a.pro_w, job.limb), wlast = load_shoup(a.pro_w, a.pro_last);
-            const uint64_t rlast = a.barrett[2 * a.pro_last + 1];
-#pragma unroll
-            for (int j = 0; j < 16; j++) {
-                const uint64_t ds = dsrc[glob(e_far(j))];
-                const uint64_t dl = a.pro_k1 ? barrett64(ds, ql, rlast) : ds;
-                const uint64_t dj = a.pro_k1 ? barrett64(ds, q, r1) : job.in[glob(e_far(j))];
-                const uint64_t r = sub_mod(tsrc[glob(e_far(j))], mul_shoup(dl, wlast, ql), ql);
-                v[j] = add_mod(mul_shoup(dj, w, q), barrett64(r, q, r1), q);
-            }
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = job.in[glob(e_far(j))];
-        }
-        outer(v, [&](uint64_t *w, uint32_t idx) { ct_block<p0>(w, c.tw, idx, q); });
-        if (p1 > 0) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) lds[skew(e_far(j))] = v[j];
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = lds[skew(e_near(j))];
-            inner(v, [&](uint64_t *w, uint32_t idx) { ct_block<(p1 > 0 ? p1 : 1)>(w, c.tw, idx, q); });
-        }
-        // lazy values in [0, 4q) go to the blocks pass
-#pragma unroll
-        for (int j = 0; j < 16; j++) job.out[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))] = v[j];
-    } else {
-#pragma unroll
-        for (int j = 0; j < 16; j++) v[j] = job.in[p1 > 0 ? glob(e_near(j)) : glob(e_far(j))];
-        if (p1 > 0) {
-            inner(v, [&](uint64_t *w, uint32_t idx) { gs_block<(p1 > 0 ? p1 : 1)>(w, c.tw, idx, q); });
-#pragma unroll
-            for (int j = 0; j < 16; j++) lds[skew(e_near(j))] = v[j];
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = lds[skew(e_far(j))];
-        }
-        outer(v, [&](uint64_t *w, uint32_t idx) { gs_block<p0>(w, c.tw, idx, q); });
-        if (a.epi_mode == NTT_EPI_MUL) {
-            const Shoup w = load_shoup(a.w, job.limb);
-#pragma unroll
-            for (int j = 0; j < 16; j++) job.out[glob(e_far(j))] = mul_shoup(v[j], w, q);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; j++) job.out[glob(e_far(j))] = reduce_2q(v[j], q);
-        }
-    }
-}
-
-// ---------------------------------------------------------------------------------------------------
-// rows pass: stages 0 .. LD-1 (forward) over an R = 2^LD rows x 256 matrix
-// ---------------------------------------------------------------------------------------------------
-template <int LD, bool FWD, int BE, int TL, bool SRC_INTT = false>
-__global__ __launch_bounds__((1 << TL) / 16) void ntt_rows_kernel(NttArgs a) {
-    __shared__ uint64_t lds[(1 << TL) + (1 << (TL - 4))];
-    constexpr uint32_t kRowThreads = (1u << TL) / 16;
-    constexpr int LOGC = log_cols<LD, TL>();
-    constexpr uint32_t C = 1u << LOGC;
-    constexpr uint32_t tile_elems = 1u << (LD + LOGC);
-    constexpr uint32_t tiles_per_limb = 256u >> LOGC;
-    constexpr int p0 = Split<LD>::p0, p1 = Split<LD>::p1;
-
-    const uint32_t lb = logical_block();
-    const Job job = decode_job(a, lb / tiles_per_limb);
-    const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
-    // (N = 2^17, 512 rows: the inner block would be five stages, 32 words a thread; that degree takes the tile
-    // through LDS between its blocks, below)
-    if constexpr (LD >= 4 && LD <= 8 && tile_elems == 16 * kRowThreads) {
-        rows_direct<LD, FWD, BE, LOGC, SRC_INTT>(a, job, col0, lds);
-        return;
-    }
-    static_assert(!SRC_INTT || (LD >= 4 && LD <= 8 && tile_elems == 16 * kRowThreads), "only the register rows pass");
-    double *ld = reinterpret_cast<double *>(lds);
-
-    // the back end of this workgroup's limb: fixed by the launch, or (mixed) by the limb's prime
-    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) {
-        const FpCtx c = fp_ctx(a, job.table);
-        if (FWD) {
-            // input: canonical residues (or one broadcast source limb); output: lazy signed doubles
-            const uint64_t *bsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-            const uint64_t *src = a.pro_mode == NTT_PRO_BROADCAST_REDUCE ? bsrc : job.in;
-            if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
-                const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
-                const FpMod ml = fp_ctx(a, a.pro_last).m;
-                const double wd = fp_from_u64(a.pro_w[2 * job.limb]), wl = fp_from_u64(a.pro_w[2 * a.pro_last]);
-                const FpTw w{wd, wd * c.m.qinv}, wlast{wl, wl * ml.qinv};
-                const uint64_t qj = a.moduli[job.table], rj = a.barrett[2 * job.table + 1];
-                const uint64_t qlast = a.moduli[a.pro_last], rlast = a.barrett[2 * a.pro_last + 1];
-                for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                    uint32_t row = e >> LOGC, col = e & (C - 1);
-                    const size_t g = (size_t)row * 256 + col0 + col;
-                    const uint64_t ds = dsrc[g];
-                    const uint64_t dl = a.pro_k1 ? barrett64(ds, qlast, rlast) : ds;
-                    const uint64_t dj = a.pro_k1 ? barrett64(ds, qj, rj) : src[g];
-                    // coefficient of the dropped limb of the ModDown result, canonical mod q_last
-                    const double r = fp_canonical(fp_from_u64(bsrc[g]) - fp_mulmod(fp_from_u64(dl), wlast, ml), ml);
-                    ld[skew(e)] = fp_mulmod(fp_from_u64(dj), w, c.m) + fp_reduce(r, c.m);
-                }
-            } else if (a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
-                const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
-                for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                    uint32_t row = e >> LOGC, col = e & (C - 1);
-                    ld[skew(e)] = fp_from_u64(barrett64(job.src[(size_t)row * 256 + col0 + col], q, r1));
-                }
-            } else {
-                for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                    uint32_t row = e >> LOGC, col = e & (C - 1);
-                    ld[skew(e)] = fp_from_u64(src[(size_t)row * 256 + col0 + col]);
-                }
-            }
-            __syncthreads();
-            // a broadcast source may exceed this limb's prime: reduce first in that case
-            if (a.pro_mode != NTT_PLAIN)
-                tile_pass_fp<p0, true, true>(lds, tile_elems, LD - p0 + LOGC, 1u, c);
-            else
-                tile_pass_fp<p0, true, false>(lds, tile_elems, LD - p0 + LOGC, 1u, c);
-            __syncthreads();
-            if (p1 > 0) {
-                tile_pass_fp<(p1 > 0 ? p1 : 1), true, true>(lds, tile_elems, LOGC, 1u << p0, c);
-                __syncthreads();
-            }
-            for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                uint32_t row = e >> LOGC, col = e & (C - 1);
-                job.out[(size_t)row * 256 + col0 + col] = lds[skew(e)];
-            }
-        } else {
-            // input: lazy signed doubles from the blocks pass; output: canonical residues
-            for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                uint32_t row = e >> LOGC, col = e & (C - 1);
-                lds[skew(e)] = job.in[(size_t)row * 256 + col0 + col];
-            }
-            __syncthreads();
-            if (p1 > 0) {
-                tile_pass_fp<(p1 > 0 ? p1 : 1), false, true>(lds, tile_elems, LOGC, 1u << p0, c);
-                __syncthreads();
-            }
-            tile_pass_fp<p0, false, true>(lds, tile_elems, LD - p0 + LOGC, 1u, c);
-            __syncthreads();
-            const FpTw scale = inverse_scale(a, job, c.m);
-            for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                uint32_t row = e >> LOGC, col = e & (C - 1);
-                job.out[(size_t)row * 256 + col0 + col] = fp_to_u64(fp_canonical(fp_mulmod(ld[skew(e)], scale, c.m), c.m));
-            }
-        }
-        return;
-    }
-
-    const IntCtx c = int_ctx(a, job.table);
-    const uint64_t q = c.q;
-    if (FWD && (a.pro_mode == NTT_PRO_BROADCAST_REDUCE || a.pro_mode == NTT_PRO_SOURCE_REDUCE)) {
-        const uint64_t r1 = a.barrett[2 * job.table + 1];
-        const uint64_t *src = a.pro_mode == NTT_PRO_SOURCE_REDUCE ? job.src : a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-        for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-            uint32_t row = e >> LOGC, col = e & (C - 1);
-            lds[skew(e)] = barrett64(src[(size_t)row * 256 + col0 + col], q, r1);
-        }
-    } else if (FWD && a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
-        const uint64_t r1 = a.barrett[2 * job.table + 1];
-        const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
-        const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
-        const uint64_t ql = a.moduli[a.pro_last];
-        const Shoup w = load_shoup(a.pro_w, job.limb), wlast = load_shoup(a.pro_w, a.pro_last);
-        const uint64_t rlast = a.barrett[2 * a.pro_last + 1];
-        for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-            uint32_t row = e >> LOGC, col = e & (C - 1);
-            const size_t g = (size_t)row * 256 + col0 + col;
-            const uint64_t ds = dsrc[g];
-            const uint64_t dl = a.pro_k1 ? barrett64(ds, ql, rlast) : ds;
-            const uint64_t dj = a.pro_k1 ? barrett64(ds, q, r1) : job.in[g];
-            const uint64_t r = sub_mod(tsrc[g], mul_shoup(dl, wlast, ql), ql);
-            lds[skew(e)] = add_mod(mul_shoup(dj, w, q), barrett64(r, q, r1), q);
-        }
-    } else {
-        for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-            uint32_t row = e >> LOGC, col = e & (C - 1);
-            lds[skew(e)] = job.in[(size_t)row * 256 + col0 + col];
-        }
-    }
-    __syncthreads();
-
-    if (FWD) {
-        tile_pass<p0, true>(lds, tile_elems, LD - p0 + LOGC, 1u, c);
-        __syncthreads();
-        if (p1 > 0) {
-            tile_pass<(p1 > 0 ? p1 : 1), true>(lds, tile_elems, LOGC, 1u << p0, c);
-            __syncthreads();
-        }
-        // lazy values in [0, 4q) go to the blocks pass
-        for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-            uint32_t row = e >> LOGC, col = e & (C - 1);
-            job.out[(size_t)row * 256 + col0 + col] = lds[skew(e)];
-        }
-    } else {
-        if (p1 > 0) {
-            tile_pass<(p1 > 0 ? p1 : 1), false>(lds, tile_elems, LOGC, 1u << p0, c);
-            __syncthreads();
-        }
-        tile_pass<p0, false>(lds, tile_elems, LD - p0 + LOGC, 1u, c);
-        __syncthreads();
-        if (a.epi_mode == NTT_EPI_MUL) {
-            const Shoup w = load_shoup(a.w, job.limb);
-            for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                uint32_t row = e >> LOGC, col = e & (C - 1);
-                job.out[(size_t)row * 256 + col0 + col] = mul_shoup(lds[skew(e)], w, q);
-            }
-        } else {
-            for (uint32_t e = threadIdx.x; e < tile_elems; e += kRowThreads) {
-                uint32_t row = e >> LOGC, col = e & (C - 1);
-                job.out[(size_t)row * 256 + col0 + col] = reduce_2q(lds[skew(e)], q);
-            }
-        }
-    }
-}
+constexpr uint32_t kLdsWords = 4096 + 256;   // a skewed tile of 16 words per thread
 
 // ---------------------------------------------------------------------------------------------------
 // Whole-limb transform for N <= 2^14 (FP64 back end, plain forward / inverse with the optional inverse scaling):
@@ -697,15 +151,16 @@ hipError_t launch_limb_fp(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
 }
 
 // The launches that the whole-limb kernel covers and wins.  A limb is one workgroup on one CU: up to N = 2^12 that is
-// faster than two launches whatever the number of limbs (10-12 us against 15-16 us for a forward + inverse pair);
-// a limb of 2^13 or 2^14 words takes one CU 9 or 17 us, so there the kernel pays only when the launch has enough limbs
-// to occupy the chip (measured break-even: 64 and 192 limbs; at 256 limbs 23 against 34 us and 50 against 60 us).
-// a.one_pass = 2 forces it (tests).
+// faster than two launches whatever the number of limbs (5.5 against 8.5 us); a limb of 2^13 or 2^14 words takes one CU
+// longer than two launches of a few limbs take, so there the kernel pays only when the launch has enough limbs to occupy
+// the chip: from 64 limbs on at 2^13 (192 limbs 10.7 against 13.8 us, 576 limbs 25.6 against 33.3 us), from 192 on in the
+// forward direction at 2^14 (19.4 against 25.1 us, 576 limbs 55.7 against 59.9 us; its inverse, whose first blocks wait for the whole
+// limb, takes 28.4 against 25.4 us and 82 against 56 us).  a.one_pass = 2 forces it (tests).
 inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_jobs) {
     if (!a.one_pass || backend != NTT_BACKEND_FP || a.log_n > 14 || a.jobs || a.pro_mode != NTT_PLAIN || a.in_galois ||
         !(a.epi_mode == NTT_PLAIN || (!forward && a.epi_mode == NTT_EPI_MUL)))
         return false;
-    return a.one_pass == 2 || a.log_n <= 12 || n_jobs >= (a.log_n == 13 ? 64u : 192u);
+    return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && n_jobs >= 64) || (a.log_n == 14 && forward && n_jobs >= 192);
 }
 
 // ---------------------------------------------------------------------------------------------------
@@ -1253,263 +708,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
     }
 }
 
-// ---------------------------------------------------------------------------------------------------
-// blocks pass: the 8 stages that stay inside 256 consecutive words
-//
-// A workgroup of T threads owns a tile of 16 T consecutive words (T = 128 or 256) and walks through every
-// limb of its unit: the limbs of one unit share a modulus, hence a twiddle table, and the table is as large
-// as a limb, so reading it once per unit instead of once per limb removes up to half of the pass's HBM
-// traffic.  The next limb's tile is fetched into registers while the current one is transformed.
-// ---------------------------------------------------------------------------------------------------
-struct Unit {
-    uint32_t j0, jstride, count;
-};
-
-// map mode: unit = (limb i, group of `batch` polynomials); list mode: unit = group of consecutive jobs
-__device__ __forceinline__ Unit decode_unit(const NttArgs &a, uint32_t u) {
-    if (a.jobs) {
-        const uint32_t item = u / a.n_groups;
-        const LimbGroup g = a.groups[u - item * a.n_groups];
-        return Unit{item * a.n_jobs + g.first, 1u, g.count};
-    }
-    const uint32_t limb = u % a.map.limbs, pg = u / a.map.limbs;
-    const uint32_t p0 = pg * a.batch;
-    const uint32_t cnt = a.n_polys - p0 < a.batch ? a.n_polys - p0 : a.batch;
-    return Unit{p0 * a.map.limbs + limb, a.map.limbs, cnt};
-}
-
-// A workgroup of T threads owns 16 T consecutive words: T = 256 or 128 for N >= 2048, N / 16 below that, so
-// that every thread moves exactly 16 words and no access needs a bounds check (straight-line code lets the
-// compiler count the loads and stores in flight instead of draining them at every step).
-struct BlocksGeom {
-    uint32_t idx0, idx1;
-    size_t off;
-    Unit unit;
-};
-
-__device__ __forceinline__ BlocksGeom blocks_geom(const NttArgs &a) {
-    const uint32_t lr = a.log_n - 8;                       // log2(number of 256-blocks per limb)
-    const uint32_t tile_elems = blockDim.x << 4;
-    const uint32_t log_b = 31 - __builtin_clz(tile_elems >> 8);  // blocks per tile = 2^log_b
-    const uint32_t tiles_per_limb = 1u << (lr - log_b);
-    const uint32_t lb = logical_block();
-    BlocksGeom g;
-    g.unit = decode_unit(a, lb / tiles_per_limb);
-    const uint32_t tile = lb % tiles_per_limb;
-    g.off = (size_t)tile * tile_elems;
-    const uint32_t blk0 = tile << log_b;                   // first 256-block of this tile within the limb
-    g.idx0 = (1u << lr) + blk0;
-    g.idx1 = (1u << (lr + 4)) + (blk0 << 4);
-    return g;
-}
-
-constexpr int kPer = 16;  // words per thread in the blocks pass
-constexpr int kMaxGroup = 4;  // most jobs in one LimbGroup
-
-// FP64 back end.  EPI compiles the fused forward epilogues in (they cost 64 registers).  Two waves per SIMD: with
-// the epilogues the kernel needs 254 registers; left to itself the compiler spreads into the accumulation registers
-// and a single wave, which costs a third more time (three waves would spill, and measure slower).
-// GAL: the inverse pass gathers its input through a Galois permutation (a.in_galois); an instantiation of its own, so
-// that the index arithmetic costs the other launches no registers
-// TW_LDS (forward pass with an epilogue): the 30 twiddles of a thread live in LDS behind the tile instead of in 60
-// registers, which leaves room for the next tile's words in registers while the current one is transformed and its
-// epilogue operands travel: without it that fetch waits until the epilogue has stored, and every tile of the loop
-// exposes one round trip to memory.  LDS: the tile (17 T words), 15 T / 16 words of the first block's twiddles (one set
-// per 16 threads), 15 T of the second block's.
-template <bool FWD, bool EPI, bool GAL, bool TW_LDS = false>
-__device__ __forceinline__ void ntt_blocks_fp_body(const NttArgs &a, uint64_t *lds) {
-    const uint32_t nthreads = blockDim.x;
-    const BlocksGeom g = blocks_geom(a);
-    const size_t off = g.off;
-    const size_t n = (size_t)1 << a.log_n;
-    double *ld = reinterpret_cast<double *>(lds);
-    const bool fma_mode = EPI && a.epi_mode == NTT_EPI_FMA_SUB_MUL;   // ((a * pro_w + b) - v) * w
-    const bool has_addend = EPI && (a.epi_mode == NTT_EPI_SUB_MUL_ADD || fma_mode);
-
-    Job job = decode_job(a, g.unit.j0);
-    if (a.unit_filter == 1 && !((a.fp_mask >> job.table) & 1)) return;   // (the whole workgroup: a unit has one prime)
-    const FpCtx fc = fp_ctx(a, job.table);
-    const FpMod m = fc.m;
-
-    // this thread's group in either register pass, and its twiddles (the same for every limb of the unit)
-    const uint32_t gi = threadIdx.x;
-    const uint32_t base0 = ((gi >> 4) << 8) | (gi & 15);   // pass with stride 16
-    const uint32_t base1 = gi << 4;                        // pass with stride 1
-    double tw0[15], tw1[15];
-    fp_load_block_tw<4>(tw0, fc.tw, g.idx0 + (gi >> 4));
-    fp_load_block_tw<4>(tw1, fc.tw, g.idx1 + gi);
-    double *ltw0 = ld + 17 * nthreads, *ltw1 = ltw0 + 15 * (nthreads >> 4);
-
-    // list mode: the unit's jobs are read before the first store, so that they stay scalar loads
-    LimbJob pre[kMaxGroup];
-    const uint32_t item = a.jobs ? g.unit.j0 / a.n_jobs : 0;
-    const uint32_t first = g.unit.j0 - item * (a.jobs ? a.n_jobs : 0);
-#pragma unroll
-    for (int i = 0; i < kMaxGroup; i++) pre[i] = (a.jobs && (uint32_t)i < g.unit.count) ? a.jobs[first + i] : LimbJob{0, 0};
-    const size_t item_off = a.jobs ? item * a.item_stride : 0;
-    auto entry = [&](uint32_t b) {
-        if (!a.jobs) return decode_job(a, g.unit.j0 + b * g.unit.jstride);
-        LimbJob lj = pre[0];
-#pragma unroll
-        for (int i = 1; i < kMaxGroup; i++) lj = b == (uint32_t)i ? pre[i] : lj;
-        return Job{a.in + item_off + (size_t)lj.data_limb * n, a.out + item_off + (size_t)lj.data_limb * n, lj.table, 0, 0, nullptr};
-    };
-
-    uint64_t nx[kPer];
-    auto stage = [&]() {  // prefetched words -> LDS
-#pragma unroll
-        for (int i = 0; i < kPer; i++) {
-            const uint32_t e = threadIdx.x + i * nthreads;
-            if (!FWD)
-                ld[skew(e)] = fp_from_u64(nx[i]);
-            else
-                lds[skew(e)] = nx[i];
-        }
-        lds_barrier();
-    };
-    // inverse pass of a rotation: the input is sigma(in), gathered here (map mode only)
-    const uint32_t in_elt = (FWD || !GAL) ? 0u : a.in_galois;
-    auto fetch = [&](const Job &j) {
-        const uint64_t *src = (FWD ? j.out : j.in) + off;  // the forward blocks pass continues on the rows pass's output
-        if (!FWD && GAL && in_elt) {
-#pragma unroll
-            for (int i = 0; i < kPer; i++)
-                nx[i] = j.in[galois_index((uint32_t)off + threadIdx.x + i * nthreads, in_elt, a.log_n)];
-        } else {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) nx[i] = src[threadIdx.x + i * nthreads];
-        }
-    };
-    fetch(job);
-    if (TW_LDS) {
-        // (stride 15: the threads of a wave read their sets from distinct banks; 16 threads share a set of the first block)
-#pragma unroll
-        for (int i = 0; i < 15; i++) {
-            if ((gi & 15) == 0) ltw0[(gi >> 4) * 15 + i] = tw0[i];
-            ltw1[gi * 15 + i] = tw1[i];
-        }
-    } else {
-        // the twiddles have arrived before the loop starts: inside it only the prefetch is in flight
-#pragma unroll
-        for (int i = 0; i < 15; i++) asm volatile("" ::"v"(tw0[i]), "v"(tw1[i]));
-    }
-    stage();
-
-    for (uint32_t b = 0;; b++) {
-        // the next limb's tile and this limb's epilogue operands travel while the butterflies run
-        const bool more = b + 1 < g.unit.count;
-        // (with a fused epilogue the registers go to its operands instead and the next tile is fetched late)
-        Job next = job;
-        if (more) next = entry(b + 1);
-        if (more && (!EPI || TW_LDS)) fetch(next);
-        const size_t epi_off = off + (size_t)job.limb * n;
-        // SUB_MUL_ADD adds onto the polynomials named by epi_b_mask only (a rotation adds onto c0, not c1)
-        const bool add_b = has_addend && (fma_mode || ((a.epi_b_mask >> (job.poly & 31)) & 1));
-        uint64_t *dst = (FWD && EPI) ? a.epi_dst + (size_t)job.poly * a.epi_dst_poly_stride * n + epi_off : job.out + off;
-        uint64_t pre_a[EPI ? kPer : 1], pre_b[EPI ? kPer : 1];
-        if (FWD && EPI) {
-            const uint64_t *minuend = a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + epi_off;
-            const uint64_t *addend = add_b ? a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + epi_off : minuend;
-#pragma unroll
-            for (int i = 0; i < kPer; i++) pre_a[EPI ? i : 0] = minuend[threadIdx.x + i * nthreads];
-#pragma unroll
-            for (int i = 0; i < kPer; i++) pre_b[EPI ? i : 0] = addend[threadIdx.x + i * nthreads];
-        }
-
-        double v[16];
-        if (FWD) {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = ld[skew(base0 + (j << 4))];
-            if (TW_LDS) {
-                double t[15];
-#pragma unroll
-                for (int i = 0; i < 15; i++) t[i] = ltw0[(gi >> 4) * 15 + i];
-                fp_ct_block_tw<4, true>(v, t, m);
-            } else {
-                fp_ct_block_tw<4, true>(v, tw0, m);
-            }
-#pragma unroll
-            for (int j = 0; j < 16; j++) ld[skew(base0 + (j << 4))] = v[j];
-            lds_barrier();
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = ld[skew(base1 + j)];
-            if (TW_LDS) {
-                double t[15];
-#pragma unroll
-                for (int i = 0; i < 15; i++) t[i] = ltw1[gi * 15 + i];
-                fp_ct_block_tw<4, true>(v, t, m);
-            } else {
-                fp_ct_block_tw<4, true>(v, tw1, m);
-            }
-#pragma unroll
-            for (int j = 0; j < 16; j++) ld[skew(base1 + j)] = v[j];
-            lds_barrier();
-#pragma unroll
-            // (an epilogue subtracts the word as the second block left it, at most 5.3 q in magnitude: its difference from
-            // a minuend below 1.9 q stays below 2^53 and goes through one modular product)
-            for (int i = 0; i < kPer; i++) v[i] = EPI ? ld[skew(threadIdx.x + i * nthreads)] : fp_canonical(ld[skew(threadIdx.x + i * nthreads)], m);
-            if (EPI) {
-                const double wd = fp_from_u64(a.w[2 * job.limb]);
-                const FpTw w{wd, wd * m.qinv};
-                if (fma_mode) {
-                    const double pd = fp_from_u64(a.pro_w[2 * job.limb]);
-                    const FpTw pw{pd, pd * m.qinv};
-#pragma unroll
-                    for (int i = 0; i < kPer; i++) {
-                        const double lhs = fp_mulmod(fp_from_u64(pre_a[EPI ? i : 0]), pw, m) + fp_from_u64(pre_b[EPI ? i : 0]);
-                        v[i] = fp_canonical(fp_mulmod(lhs - v[i], w, m), m);
-                    }
-                } else {
-#pragma unroll
-                    for (int i = 0; i < kPer; i++) {
-                        double r = fp_mulmod(fp_from_u64(pre_a[EPI ? i : 0]) - v[i], w, m);
-                        if (add_b) r += fp_from_u64(pre_b[EPI ? i : 0]);
-                        v[i] = fp_canonical(r, m);
-                    }
-                }
-            }
-#pragma unroll
-            for (int i = 0; i < kPer; i++) dst[threadIdx.x + i * nthreads] = fp_to_u64(v[i]);
-        } else {
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = ld[skew(base1 + j)];
-            fp_gs_block_tw<4, false>(v, tw1, m);
-#pragma unroll
-            for (int j = 0; j < 16; j++) ld[skew(base1 + j)] = v[j];
-            lds_barrier();
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = ld[skew(base0 + (j << 4))];
-            fp_gs_block_tw<4, true>(v, tw0, m);
-#pragma unroll
-            for (int j = 0; j < 16; j++) ld[skew(base0 + (j << 4))] = v[j];
-            lds_barrier();
-            // lazy signed doubles go to the rows pass
-            uint64_t o[kPer];
-#pragma unroll
-            for (int i = 0; i < kPer; i++) o[i] = lds[skew(threadIdx.x + i * nthreads)];
-#pragma unroll
-            for (int i = 0; i < kPer; i++) dst[threadIdx.x + i * nthreads] = o[i];
-        }
-        if (!more) break;
-        if (EPI && !TW_LDS) fetch(next);
-        lds_barrier();  // every read of this tile is done before the next one overwrites it
-        stage();
-        job = next;
-    }
-}
-
-template <bool FWD, bool EPI, bool GAL>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void ntt_blocks_fp_kernel(NttArgs a) {
-    __shared__ uint64_t lds[kLdsWords];
-    ntt_blocks_fp_body<FWD, EPI, GAL>(a, lds);
-}
-
-// the forward pass with an epilogue: twiddles in LDS (blocks_epi_lds_bytes of dynamic LDS)
-extern __shared__ uint64_t dyn_lds[];
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void ntt_blocks_fp_epi_kernel(NttArgs a) {
-    ntt_blocks_fp_body<true, true, false, true>(a, dyn_lds);
-}
-inline size_t blocks_epi_lds_bytes(uint32_t threads) { return 8 * (size_t)(17 * threads + 15 * (threads >> 4) + 15 * threads); }
+constexpr int kPer = 16;  // words per thread in the fused blocks passes
 
 // Forward blocks pass of ModUp fused with the key-switch inner product.  Workgroup = (limb t of Ql u P, tile of
 // 16 T words): its first T threads transform that tile of every digit in turn; all 2 T threads then multiply
@@ -1689,19 +888,20 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1))) v
     __shared__ uint64_t lds[kLdsWords];
     double *ld = reinterpret_cast<double *>(lds);
     const uint32_t nthreads = blockDim.x;
-    const BlocksGeom g = blocks_geom(a);
-    const Job job = decode_job(a, g.unit.j0);
+    const uint32_t lr = a.log_n - 8, log_b = 31 - __builtin_clz(nthreads >> 4);   // 256-word blocks of a limb, of a tile
+    const uint32_t lb = logical_block(), tile = lb & ((1u << (lr - log_b)) - 1), blk0 = tile << log_b;
+    const Job job = decode_job(a, lb >> (lr - log_b));
     const FpCtx fc = fp_ctx(a, job.table);
     const FpMod m = fc.m;
-    const size_t n = (size_t)1 << a.log_n;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)tile * nthreads * kPer;
     const uint32_t gi = threadIdx.x;
     const uint32_t base0 = ((gi >> 4) << 8) | (gi & 15);
     const uint32_t base1 = gi << 4;
     double tw0[15], tw1[15];
-    fp_load_block_tw<4>(tw0, fc.tw, g.idx0 + (gi >> 4));
-    fp_load_block_tw<4>(tw1, fc.tw, g.idx1 + gi);
+    fp_load_block_tw<4>(tw0, fc.tw, (1u << lr) + blk0 + (gi >> 4));
+    fp_load_block_tw<4>(tw1, fc.tw, (1u << (lr + 4)) + (blk0 << 4) + gi);
 
-    const size_t lo = (size_t)job.limb * n + g.off, poly = (size_t)x.L * n;
+    const size_t lo = (size_t)job.limb * n + off, poly = (size_t)x.L * n;
     // the launch has 1.5 waves per SIMD at N = 2^16, L = 24: all 64 loads of a thread are in flight at once
 #pragma unroll
     for (int i = 0; i < kPer; i++) {
@@ -1745,241 +945,12 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1))) v
     for (int j = 0; j < 16; j++) ld[skew(base0 + (j << 4))] = v[j];
     lds_barrier();
     // lazy signed doubles go to the rows pass
-    uint64_t *dst = job.out + g.off;
+    uint64_t *dst = job.out + off;
     uint64_t o[kPer];
 #pragma unroll
     for (int i = 0; i < kPer; i++) o[i] = lds[skew(threadIdx.x + i * nthreads)];
 #pragma unroll
     for (int i = 0; i < kPer; i++) dst[threadIdx.x + i * nthreads] = o[i];
-}
-
-// Integer back end (twiddles stay in the table: 30 Shoup pairs per thread do not fit in registers).  Three waves
-// per SIMD (168 registers, 24 bytes of spill in the forward kernel) hide the latency of the epilogue's operand loads
-// better than the two waves that 196 registers allow.
-// PRE: the operands of a fused epilogue are requested together with the tile, so that they travel while the
-// butterflies run (32 more registers: for the mixed kernel, which is compiled for two waves per SIMD and serves the
-// small launches, where nothing else covers that round trip).
-template <bool FWD, bool GAL, bool PRE = false>
-__device__ __forceinline__ void ntt_blocks_int_body(const NttArgs &a, uint64_t *lds) {
-    const uint32_t nthreads = blockDim.x;
-    const uint32_t tile_elems = nthreads << 4;
-    const BlocksGeom g = blocks_geom(a);
-    const size_t off = g.off;
-    const size_t n = (size_t)1 << a.log_n;
-    const bool fma_mode = FWD && a.epi_mode == NTT_EPI_FMA_SUB_MUL;
-    const bool epi = FWD && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || fma_mode);
-    const bool has_addend = FWD && (a.epi_mode == NTT_EPI_SUB_MUL_ADD || fma_mode);
-
-    if (a.unit_filter == 2 && ((a.fp_mask >> decode_job(a, g.unit.j0).table) & 1)) return;
-    for (uint32_t b = 0; b < g.unit.count; b++) {
-        const Job job = decode_job(a, g.unit.j0 + b * g.unit.jstride);
-        const IntCtx ic = int_ctx(a, job.table);
-        const uint64_t q = ic.q;
-        const uint64_t *src = (FWD ? job.out : job.in) + off;
-        if (!FWD && GAL && a.in_galois) {
-#pragma unroll
-            for (int i = 0; i < kPer; i++)
-                lds[skew(threadIdx.x + i * nthreads)] = job.in[galois_index((uint32_t)off + threadIdx.x + i * nthreads, a.in_galois, a.log_n)];
-        } else {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) lds[skew(threadIdx.x + i * nthreads)] = src[threadIdx.x + i * nthreads];
-        }
-        const size_t epi_off = off + (size_t)job.limb * n;
-        const uint64_t *minuend = epi ? a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + epi_off : nullptr;
-        const bool add_b = has_addend && (fma_mode || ((a.epi_b_mask >> (job.poly & 31)) & 1));
-        const uint64_t *addend = add_b ? a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + epi_off : minuend;
-        uint64_t pre_a[PRE ? kPer : 1], pre_b[PRE ? kPer : 1];
-        if (PRE && epi) {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) pre_a[PRE ? i : 0] = minuend[threadIdx.x + i * nthreads];
-#pragma unroll
-            for (int i = 0; i < kPer; i++) pre_b[PRE ? i : 0] = addend[threadIdx.x + i * nthreads];
-        }
-        __syncthreads();
-        if (FWD) {
-            tile_pass<4, true>(lds, tile_elems, 4, g.idx0, ic);
-            __syncthreads();
-            tile_pass<4, true>(lds, tile_elems, 0, g.idx1, ic);
-            __syncthreads();
-            if (epi) {
-                uint64_t *dst = a.epi_dst + (size_t)job.poly * a.epi_dst_poly_stride * n + epi_off;
-                const Shoup w = load_shoup(a.w, job.limb);
-                const Shoup pw = fma_mode ? load_shoup(a.pro_w, job.limb) : w;
-#pragma unroll
-                for (int i = 0; i < kPer; i++) {
-                    const uint32_t e = threadIdx.x + i * nthreads;
-                    const uint64_t c = reduce_4q(lds[skew(e)], q);
-                    const uint64_t ma = PRE ? pre_a[PRE ? i : 0] : minuend[e];
-                    uint64_t r;
-                    if (fma_mode) {
-                        const uint64_t mb = PRE ? pre_b[PRE ? i : 0] : addend[e];
-                        r = mul_shoup(sub_mod(add_mod(mul_shoup(ma, pw, q), mb, q), c, q), w, q);
-                    } else {
-                        r = mul_shoup(sub_mod(ma, c, q), w, q);
-                        if (add_b) r = add_mod(r, PRE ? pre_b[PRE ? i : 0] : addend[e], q);
-                    }
-                    dst[e] = r;
-                }
-            } else {
-#pragma unroll
-                for (int i = 0; i < kPer; i++) {
-                    const uint32_t e = threadIdx.x + i * nthreads;
-                    job.out[off + e] = reduce_4q(lds[skew(e)], q);
-                }
-            }
-        } else {
-            tile_pass<4, false>(lds, tile_elems, 0, g.idx1, ic);
-            __syncthreads();
-            tile_pass<4, false>(lds, tile_elems, 4, g.idx0, ic);
-            __syncthreads();
-            // lazy values in [0, 2q) go to the rows pass
-#pragma unroll
-            for (int i = 0; i < kPer; i++) {
-                const uint32_t e = threadIdx.x + i * nthreads;
-                job.out[off + e] = lds[skew(e)];
-            }
-        }
-        __syncthreads();  // every read of this tile is done before the next one overwrites it
-    }
-}
-
-template <bool FWD, bool GAL>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(3, 3))) void ntt_blocks_int_kernel(NttArgs a) {
-    __shared__ uint64_t lds[kLdsWords];
-    ntt_blocks_int_body<FWD, GAL>(a, lds);
-}
-
-// Mixed back end: the limbs of a unit share a modulus, so the whole workgroup takes one branch.  EPI as in
-// ntt_blocks_fp_kernel: the FP64 body compiled with the fused epilogues addresses their operands unconditionally,
-// so it is only launched when the launch has an epilogue.
-template <bool FWD, bool EPI, bool GAL>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2))) void ntt_blocks_mixed_kernel(NttArgs a) {
-    __shared__ uint64_t lds[kLdsWords];
-    const Job first = decode_job(a, blocks_geom(a).unit.j0);
-    if ((a.fp_mask >> first.table) & 1)
-        ntt_blocks_fp_body<FWD, EPI, GAL>(a, lds);
-    else
-        ntt_blocks_int_body<FWD, GAL, FWD && EPI>(a, lds);
-}
-
-template <bool FWD, int FP>
-hipError_t launch_rows(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
-    const int ld = (int)a.log_n - 8;
-    auto grid = [&](int ldv, int tl) {
-        int logc = (tl - ldv) < 8 ? (tl - ldv) : 8;
-        return dim3(n_jobs * (256u >> logc));
-    };
-    // small launches (fewer 4096-word tiles than CUs) are bound by the latency of one workgroup: quarter tiles
-    const bool small = ld >= 5 && n_jobs * (256u >> (kTileLog - ld < 8 ? kTileLog - ld : 8)) < 256;
-    if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
-        // one instantiation per degree, on quarter tiles, which follows fp_mask limb by limb: the mask stands for the
-        // launch's back end here
-        if (!FWD || !ntt_source_intt_ok(a.log_n, n_jobs, 0) || !a.pro_itw || (a.pro_src_fp_mask && !a.pro_itw_fp))
-            return hipErrorInvalidValue;
-        NttArgs b = a;
-        b.fp_mask = FP == NTT_BACKEND_INT ? 0 : (FP == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
-        if (ld == 7)
-            hipLaunchKernelGGL((ntt_rows_kernel<7, true, NTT_BACKEND_MIXED, 10, true>), grid(7, 10), dim3(64), 0, s, b);
-        else
-            hipLaunchKernelGGL((ntt_rows_kernel<8, true, NTT_BACKEND_MIXED, 10, true>), grid(8, 10), dim3(64), 0, s, b);
-        return hipGetLastError();
-    }
-    switch (ld) {
-#define HE_CASE(LD)                                                                               \
-    case LD:                                                                                      \
-        hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, FP, 12>), grid(LD, 12), dim3(256), 0, s, a); \
-        break;
-#define HE_CASE2(LD)                                                                                  \
-    case LD:                                                                                          \
-        if (small)                                                                                    \
-            hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, FP, 10>), grid(LD, 10), dim3(64), 0, s, a);  \
-        else                                                                                          \
-            hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, FP, 12>), grid(LD, 12), dim3(256), 0, s, a); \
-        break;
-        HE_CASE(1) HE_CASE(2) HE_CASE(3) HE_CASE(4) HE_CASE2(5) HE_CASE2(6) HE_CASE2(7) HE_CASE2(8) HE_CASE(9)
-#undef HE_CASE
-#undef HE_CASE2
-        default:
-            return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
-}
-
-// Geometry of the blocks pass: polynomials per unit (map mode) and workgroup size, chosen so that the grid
-// still fills 256 CUs a few times over.
-struct BlocksPlan {
-    uint32_t batch, threads, grid;
-};
-
-BlocksPlan plan_blocks(const NttArgs &a, uint32_t n_polys) {
-    const uint32_t n = 1u << a.log_n;
-    // threads of a workgroup for a wished tile of `want` words (a limb may be smaller than that)
-    auto threads = [&](uint32_t want) { return (n < want ? n : want) >> 4; };
-    auto tiles = [&](uint32_t want) { return n / (threads(want) << 4); };
-    BlocksPlan p;
-    uint32_t units;
-    if (a.jobs) {
-        p.batch = 1;
-        units = a.n_groups * (a.items ? a.items : 1);
-    } else {
-        // batching pays once the launch has enough workgroups without splitting the polynomials
-        p.batch = (n_polys > 1 && a.map.limbs * tiles(2048) >= 512) ? n_polys : 1;
-        units = a.map.limbs * ((n_polys + p.batch - 1) / p.batch);
-    }
-    const uint32_t want = units * tiles(4096) >= 1024 ? 4096 : (units * tiles(2048) >= 256 ? 2048 : 1024);
-    p.threads = threads(want);
-    p.grid = units * tiles(want);
-    return p;
-}
-
-constexpr uint32_t kSplitMixedGrid = 1024;   // workgroups from which a mixed blocks pass runs as two kernels
-
-template <bool FWD, int FP>
-hipError_t launch_blocks(NttArgs a, uint32_t n_polys, hipStream_t s) {
-    const BlocksPlan p = plan_blocks(a, n_polys);
-    a.batch = p.batch;
-    a.n_polys = n_polys;
-    const bool epi = FWD && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD ||
-                             a.epi_mode == NTT_EPI_FMA_SUB_MUL);
-    // the Galois gather of an inverse pass's input lives in instantiations of its own
-    const bool gal = !FWD && a.in_galois != 0 && !a.jobs;
-    const dim3 grid(p.grid), block(p.threads);
-    if (FP == NTT_BACKEND_MIXED && p.grid >= kSplitMixedGrid) {
-        // A large mixed launch runs as two kernels over the same grid, each leaving the other's units at once: the
-        // integer body then has its own three waves per SIMD (the mixed kernel is compiled for the FP64 body's
-        // registers: two), which its unpipelined load -> butterflies -> store sequence needs.
-        a.unit_filter = 1;
-        if (gal)
-            hipLaunchKernelGGL((ntt_blocks_fp_kernel<false, false, true>), grid, block, 0, s, a);
-        else if (epi)
-            hipLaunchKernelGGL((ntt_blocks_fp_kernel<FWD, FWD, false>), grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL((ntt_blocks_fp_kernel<FWD, false, false>), grid, block, 0, s, a);
-        a.unit_filter = 2;
-        if (gal)
-            hipLaunchKernelGGL((ntt_blocks_int_kernel<false, true>), grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL((ntt_blocks_int_kernel<FWD, false>), grid, block, 0, s, a);
-        return hipGetLastError();
-    }
-    if (gal) {
-        if (FP == NTT_BACKEND_MIXED)
-            hipLaunchKernelGGL((ntt_blocks_mixed_kernel<false, false, true>), grid, block, 0, s, a);
-        else if (!FP)
-            hipLaunchKernelGGL((ntt_blocks_int_kernel<false, true>), grid, block, 0, s, a);
-        else
-            hipLaunchKernelGGL((ntt_blocks_fp_kernel<false, false, true>), grid, block, 0, s, a);
-    } else if (FP == NTT_BACKEND_MIXED && epi)
-        hipLaunchKernelGGL((ntt_blocks_mixed_kernel<FWD, FWD, false>), grid, block, 0, s, a);
-    else if (FP == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL((ntt_blocks_mixed_kernel<FWD, false, false>), grid, block, 0, s, a);
-    else if (!FP)
-        hipLaunchKernelGGL((ntt_blocks_int_kernel<FWD, false>), grid, block, 0, s, a);
-    else if (epi)
-        hipLaunchKernelGGL(ntt_blocks_fp_epi_kernel, grid, block, blocks_epi_lds_bytes(p.threads), s, a);
-    else
-        hipLaunchKernelGGL((ntt_blocks_fp_kernel<FWD, false, false>), grid, block, 0, s, a);
-    return hipGetLastError();
 }
 
 }  // namespace
@@ -2047,14 +1018,8 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
     if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb_fp<true>(a, n_jobs, s);
-    hipError_t e = rows_done                    ? hipSuccess
-                   : backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED>(a, n_jobs, s)
-                   : backend                    ? launch_rows<true, NTT_BACKEND_FP>(a, n_jobs, s)
-                                                : launch_rows<true, NTT_BACKEND_INT>(a, n_jobs, s);
-    if (e != hipSuccess) return e;
-    return backend == NTT_BACKEND_MIXED ? launch_blocks<true, NTT_BACKEND_MIXED>(a, n_polys, s)
-           : backend                    ? launch_blocks<true, NTT_BACKEND_FP>(a, n_polys, s)
-                                        : launch_blocks<true, NTT_BACKEND_INT>(a, n_polys, s);
+    const hipError_t e = rows_done ? hipSuccess : launch_ntt_rows(a, n_jobs, true, backend, s);
+    return e != hipSuccess ? e : launch_ntt_blocks(a, n_polys, true, backend, s);
 }
 
 hipError_t launch_ntt_forward_inner(const NttArgs &a, const KsFuseArgs &x, hipStream_t s, bool rows_done) {
@@ -2062,7 +1027,7 @@ hipError_t launch_ntt_forward_inner(const NttArgs &a, const KsFuseArgs &x, hipSt
     const uint32_t items = x.items ? x.items : 1;
     if (items > 1 && (x.own_galois || x.add_c0 || (a.items ? a.items : 1) != items)) return hipErrorInvalidValue;
     if (a.n_jobs && !rows_done) {
-        hipError_t e = launch_rows<true, NTT_BACKEND_FP>(a, a.n_jobs * items, s);
+        hipError_t e = launch_ntt_rows(a, a.n_jobs * items, true, NTT_BACKEND_FP, s);
         if (e != hipSuccess) return e;
     }
     const uint32_t n = 1u << a.log_n;
@@ -2080,20 +1045,16 @@ hipError_t launch_ntt_forward_inner(const NttArgs &a, const KsFuseArgs &x, hipSt
 
 hipError_t launch_tensor_intt_blocks(NttArgs a, const TensorFuse &x, hipStream_t s) {
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0) return hipErrorInvalidValue;
-    const BlocksPlan p = plan_blocks(a, 1);
-    a.batch = 1;
-    a.n_polys = 1;
+    const uint32_t n = 1u << a.log_n;
+    // the largest of 4096-, 2048- and 1024-word tiles that still gives the chip workgroups enough (a limb may be smaller)
+    const uint32_t want = x.L * (n / (n < 4096 ? n : 4096)) >= 1024 ? 4096 : x.L * (n / (n < 2048 ? n : 2048)) >= 256 ? 2048 : 1024;
+    const uint32_t tile = n < want ? n : want;
+    const dim3 grid(x.L * (n / tile)), block(tile / kPer);
     if (x.square)
-        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<true>, dim3(p.grid), dim3(p.threads), 0, s, a, x);
+        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<true>, grid, block, 0, s, a, x);
     else
-        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<false>, dim3(p.grid), dim3(p.threads), 0, s, a, x);
+        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<false>, grid, block, 0, s, a, x);
     return hipGetLastError();
-}
-
-bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
-    if (log_n < 15 || log_n > 16 || n_tables > 64) return false;
-    const uint32_t ld = log_n - 8;
-    return n_jobs * (256u >> (kTileLog - ld)) < 256;   // what launch_rows calls a small launch
 }
 
 hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, hipStream_t s, bool blocks_done,
@@ -2102,17 +1063,12 @@ hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, h
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
     if (!blocks_done && !rows_skipped && one_pass_ok(a, backend, false, n_jobs)) return launch_limb_fp<false>(a, n_jobs, s);
-    hipError_t e = blocks_done                    ? hipSuccess
-                   : backend == NTT_BACKEND_MIXED ? launch_blocks<false, NTT_BACKEND_MIXED>(a, n_polys, s)
-                   : backend                    ? launch_blocks<false, NTT_BACKEND_FP>(a, n_polys, s)
-                                                : launch_blocks<false, NTT_BACKEND_INT>(a, n_polys, s);
+    const hipError_t e = blocks_done ? hipSuccess : launch_ntt_blocks(a, n_polys, false, backend, s);
     if (e != hipSuccess || rows_skipped) return e;
     NttArgs rows = a;
     rows.in = a.out;  // the rows pass continues in place on the output buffer
     rows.in_poly_stride = a.out_poly_stride;
-    return backend == NTT_BACKEND_MIXED ? launch_rows<false, NTT_BACKEND_MIXED>(rows, n_jobs, s)
-           : backend                    ? launch_rows<false, NTT_BACKEND_FP>(rows, n_jobs, s)
-                                        : launch_rows<false, NTT_BACKEND_INT>(rows, n_jobs, s);
+    return launch_ntt_rows(rows, n_jobs, false, backend, s);
 }
 
 }  // namespace he

@@ -1,0 +1,606 @@
+// The two passes of the transform (ntt.hip's header says how a limb splits into them), 4 words per thread.
+//
+// What bounds a pass is how many waves a SIMD has to switch between while loads, twiddle look-ups and LDS exchanges are on
+// their way, so a thread holds little: 4 words, its twiddles (at most 12, requested together with the words) and no more, 52
+// to 110 registers, 4 to 8 waves per SIMD.  The stages run as register blocks of two; the exchanges between them go through
+// LDS, and all of a blocks pass's, and all but the first (two for 2048-word tiles) of a rows pass's, stay inside one wave and
+// need no barrier.  Passes with 16 words per thread (radix-16 blocks, half the LDS exchanges, at most 2 waves per SIMD on
+// FP64 and 3 on integers), which this layout replaced, measured against it: 2 x 24 limbs at N = 2^16 30.0 against 27.3 us
+// (50 bits) and 43.5 against 37.5 us (60 bits), 8 x 24 limbs of 60 bits 139 against 112 us, 12 x 24 of 50 bits the same
+// 112 us (5.3 TB/s: the two trips through memory), 2 limbs at N = 2^13 9.8 against 8.1 us (50 bits) and 13 against 8.5 us
+// (60 bits).
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "kernels.h"
+#include "modarith.cuh"
+#include "ntt_common.cuh"
+
+namespace he {
+
+namespace {
+
+// Orders the LDS accesses of one wave's lanes: the hardware runs them in program order, so only the compiler is held.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// Two stages (ST = 1: only the first of them) on four words; tw entries: the first stage's twiddle, then the two of the
+// second.
+struct IntArith {
+    using V = uint64_t;
+    struct Tw {
+        Shoup s[3];
+    };
+    IntMod m;
+    const uint64_t *table;
+    static __device__ __forceinline__ V from_word(uint64_t x) { return x; }
+    static __device__ __forceinline__ uint64_t to_word(V v) { return v; }
+    template <int ST>
+    __device__ __forceinline__ Tw load(uint32_t idx) const {
+        Tw t;
+        t.s[0] = load_shoup(table, idx);
+        t.s[1] = t.s[2] = Shoup{0, 0};
+        if (ST == 2) {
+            t.s[1] = load_shoup(table, 2 * (size_t)idx);
+            t.s[2] = load_shoup(table, 2 * (size_t)idx + 1);
+        }
+        return t;
+    }
+    template <int ST>
+    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
+        ct_butterfly(v[0], v[2], t.s[0], m);
+        ct_butterfly(v[1], v[3], t.s[0], m);
+        if (ST == 2) {
+            ct_butterfly(v[0], v[1], t.s[1], m);
+            ct_butterfly(v[2], v[3], t.s[2], m);
+        }
+    }
+    template <int ST>
+    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
+        if (ST == 2) {
+            gs_butterfly(v[0], v[1], t.s[1], m);
+            gs_butterfly(v[2], v[3], t.s[2], m);
+        }
+        gs_butterfly(v[0], v[2], t.s[0], m);
+        gs_butterfly(v[1], v[3], t.s[0], m);
+    }
+    __device__ __forceinline__ void reduce(V *) const {}
+};
+
+// Bounds (in units of q, |v| < 8 keeps every value exact): forward, a stage takes b to 1.375 b + 0.5, so four stages
+// between reductions end at 5.3 (7.1 from canonical words); inverse, words are reduced before every two stages, whose
+// sums end at 2 (4 from canonical words) and whose products stay below that.
+struct FpArith {
+    using V = double;
+    struct Tw {
+        double w[3];
+    };
+    FpMod m;
+    const double *table;
+    static __device__ __forceinline__ V from_word(uint64_t x) { return __longlong_as_double((long long)x); }
+    static __device__ __forceinline__ uint64_t to_word(V v) { return (uint64_t)__double_as_longlong(v); }
+    template <int ST>
+    __device__ __forceinline__ Tw load(uint32_t idx) const {
+        Tw t;
+        t.w[0] = table[idx];
+        t.w[1] = t.w[2] = 0.0;
+        if (ST == 2) {
+            t.w[1] = table[2 * (size_t)idx];
+            t.w[2] = table[2 * (size_t)idx + 1];
+        }
+        return t;
+    }
+    __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
+        asm volatile("" : "+v"(w));   // keeps w * qinv out of the registers that a loop over limbs holds
+        const double t = fp_mulmod(y, FpTw{w, w * m.qinv}, m);
+        y = x - t;
+        x = x + t;
+    }
+    __device__ __forceinline__ void gs1(V &x, V &y, double w) const {
+        asm volatile("" : "+v"(w));
+        const double d = x - y;
+        x = x + y;
+        y = fp_mulmod(d, FpTw{w, w * m.qinv}, m);
+    }
+    template <int ST>
+    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
+        ct1(v[0], v[2], t.w[0]);
+        ct1(v[1], v[3], t.w[0]);
+        if (ST == 2) {
+            ct1(v[0], v[1], t.w[1]);
+            ct1(v[2], v[3], t.w[2]);
+        }
+    }
+    template <int ST>
+    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
+        if (ST == 2) {
+            gs1(v[0], v[1], t.w[1]);
+            gs1(v[2], v[3], t.w[2]);
+        }
+        gs1(v[0], v[2], t.w[0]);
+        gs1(v[1], v[3], t.w[0]);
+    }
+    __device__ __forceinline__ void reduce(V *v) const {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = fp_reduce(v[j], m);
+    }
+};
+
+// A tile of 2^B words, 4 per thread, whose stages 0 .. LD-1 pair the tile bits B-1, B-2, ...; block k holds the stages
+// 2k and 2k+1.  In block k thread t has the words ((t >> low) << (low + 2)) | (j << low) | (t mod 2^low), low = B - 2k - 2,
+// and the twiddle index of its first stage is 2^(2k) + (t >> low).  Between the blocks k and k+1 words move inside groups
+// of 2^low threads: inside a wave from low = 6 on.
+template <int B, int LD>
+struct Tile4 {
+    static constexpr int kBlocks = (LD + 1) / 2;
+    static_assert(B >= 8 && 2 * kBlocks <= B, "four words of every block lie inside the tile");
+    static constexpr int stages(int k) { return LD - 2 * k >= 2 ? 2 : 1; }
+    static __device__ __forceinline__ uint32_t word(int k, uint32_t t, int j) {
+        const int low = B - 2 * k - 2;
+        return ((t >> low) << (low + 2)) | ((uint32_t)j << low) | (t & ((1u << low) - 1));
+    }
+    static __device__ __forceinline__ uint32_t index(int k, uint32_t t) { return (1u << (2 * k)) + (t >> (B - 2 * k - 2)); }
+
+    template <class A, int K>
+    static __device__ __forceinline__ void load_tw(typename A::Tw *tw, const A &ar, uint32_t scale, uint32_t t) {
+        // scale: the tile's number within the limb enters the index as its upper bits (blocks pass), 1 for a rows pass
+        tw[K] = ar.template load<stages(K)>(((scale - 1) << (2 * K)) + index(K, t));
+        if constexpr (K + 1 < kBlocks) load_tw<A, K + 1>(tw, ar, scale, t);
+    }
+    template <int KLO>
+    static __device__ __forceinline__ void sync() {
+        if constexpr (B - 2 * KLO - 2 > 6)
+            lds_barrier();
+        else
+            wave_sync();
+    }
+    template <class A, int K = 0>
+    static __device__ __forceinline__ void forward(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
+        ar.template ct<stages(K)>(v, tw[K]);
+        if constexpr (K + 1 < kBlocks) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
+            sync<K>();
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K + 1, t, j))]);
+            if constexpr ((K + 1) % 2 == 0) ar.reduce(v);
+            forward<A, K + 1>(v, tw, ar, lds, t);
+        }
+    }
+    template <class A, int K = kBlocks - 1>
+    static __device__ __forceinline__ void inverse(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
+        ar.template gs<stages(K)>(v, tw[K]);
+        if constexpr (K > 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
+            sync<K - 1>();
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K - 1, t, j))]);
+            ar.reduce(v);
+            inverse<A, K - 1>(v, tw, ar, lds, t);
+        }
+    }
+};
+
+__device__ __forceinline__ IntArith int_arith(const NttArgs &a, uint32_t table) {
+    const IntCtx c = int_ctx(a, table);
+    return IntArith{int_mod(c.q), c.tw};
+}
+
+__device__ __forceinline__ FpArith fp_arith(const NttArgs &a, uint32_t table) {
+    const FpCtx c = fp_ctx(a, table);
+    return FpArith{c.m, c.tw};
+}
+
+
+// Rows pass.  The thread index is (wave, lane), the wave the same scalar in all its lanes, so that the twiddles of the
+// first two blocks come through scalar loads.
+// SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first; it leaves the
+// coefficients where the forward pass takes them from.
+// B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
+template <int LD, bool FWD, int BE, bool SRC_INTT, int B>
+__global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
+    using T4 = Tile4<B, LD>;
+    constexpr int LOGC = B - LD, NB = T4::kBlocks;
+    constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
+    __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
+    const uint32_t lb = logical_block();
+    const Job job = decode_job(a, lb / tiles_per_limb);
+    const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
+    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    auto glob = [&](int k, int j) {
+        const uint32_t e = T4::word(k, t, j);
+        return (size_t)(e >> LOGC) * 256 + col0 + (e & (C - 1));
+    };
+    uint64_t s[4];   // canonical coefficients of the source limb
+    if constexpr (SRC_INTT) {
+        const uint32_t st = job.src_table;
+        if ((a.pro_src_fp_mask >> st) & 1) {
+            const FpArith ar{fp_ctx(a, st).m, a.pro_itw_fp + ((size_t)st << a.log_n)};
+            double v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(job.src[glob(NB - 1, j)]);
+            FpArith::Tw tw[NB];
+            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+            ar.reduce(v);
+            T4::template inverse<FpArith>(v, tw, ar, lds, t);
+            const double *cc = a.fp_consts + 4 * (size_t)st;
+            const FpTw ninv{cc[2], cc[3]};
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
+        } else {
+            const uint64_t q = a.moduli[st];
+            const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
+            uint64_t v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = job.src[glob(NB - 1, j)];
+            IntArith::Tw tw[NB];
+            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            T4::template inverse<IntArith>(v, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] = reduce_2q(v[j], q);
+        }
+    }
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) {
+        const FpCtx c = fp_ctx(a, job.table);
+        const FpArith ar{c.m, c.tw};
+        double v[4];
+        FpArith::Tw tw[NB];
+        if (FWD) {
+            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+            if constexpr (SRC_INTT) {
+                const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
+            } else if (rows_input_fp(v, a, job, c, [&](int j) { return glob(0, j); })) {
+                ar.reduce(v);
+            }
+            T4::template forward<FpArith>(v, tw, ar, lds, t);
+            // lazy signed doubles go to the blocks pass
+#pragma unroll
+            for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = FpArith::to_word(v[j]);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(job.in[glob(NB - 1, j)]);
+            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+            const FpTw scale = inverse_scale(a, job, c.m);
+            ar.reduce(v);
+            T4::template inverse<FpArith>(v, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) job.out[glob(0, j)] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, c.m), c.m));
+        }
+        return;
+    }
+    if constexpr (BE != NTT_BACKEND_FP) {
+        const IntArith ar = int_arith(a, job.table);
+        const uint64_t q = a.moduli[job.table];
+        uint64_t v[4];
+        IntArith::Tw tw[NB];
+        if (FWD) {
+            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            if constexpr (SRC_INTT) {
+                const uint64_t r1 = a.barrett[2 * job.table + 1];
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
+            } else {
+                rows_input_int(v, a, job, q, [&](int j) { return glob(0, j); });
+            }
+            T4::template forward<IntArith>(v, tw, ar, lds, t);
+            // lazy values in [0, 4q) go to the blocks pass
+#pragma unroll
+            for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = v[j];
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = job.in[glob(NB - 1, j)];
+            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            T4::template inverse<IntArith>(v, tw, ar, lds, t);
+            if (a.epi_mode == NTT_EPI_MUL) {
+                const Shoup w = load_shoup(a.w, job.limb);
+#pragma unroll
+                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = mul_shoup(v[j], w, q);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = reduce_2q(v[j], q);
+            }
+        }
+    }
+}
+
+// four consecutive words of a lane, as two 16-byte accesses (the polynomials are only 8-byte aligned for certain)
+typedef uint64_t Words2 __attribute__((ext_vector_type(2), aligned(8)));
+
+__device__ __forceinline__ void load4(uint64_t *v, const uint64_t *p) {
+    const Words2 a = reinterpret_cast<const Words2 *>(p)[0], b = reinterpret_cast<const Words2 *>(p)[1];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
+__device__ __forceinline__ void store4(uint64_t *p, const uint64_t *v) {
+    reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
+    reinterpret_cast<Words2 *>(p)[1] = Words2{v[2], v[3]};
+}
+
+constexpr int kBlockWaves = 2;   // 256-word blocks of a workgroup, one per wave
+
+// Operands of a fused forward epilogue at the lane's four consecutive words
+struct EpiOperands {
+    bool fma, add;
+    uint64_t a[4], b[4];
+    uint64_t *dst;
+};
+
+__device__ __forceinline__ EpiOperands load_epilogue(const NttArgs &a, const Job &job, size_t off) {
+    EpiOperands o;
+    o.fma = a.epi_mode == NTT_EPI_FMA_SUB_MUL;
+    o.add = o.fma || (a.epi_mode == NTT_EPI_SUB_MUL_ADD && ((a.epi_b_mask >> (job.poly & 31)) & 1));
+    const size_t n = (size_t)1 << a.log_n, at = off + (size_t)job.limb * n;
+    o.dst = a.epi_dst + (size_t)job.poly * a.epi_dst_poly_stride * n + at;
+    load4(o.a, a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + at);
+    if (o.add) load4(o.b, a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + at);
+    return o;
+}
+
+// The limbs that a wave takes in turn at its block: they share a prime, so its twiddles are loaded once.
+// Map mode: limb `limb` of the polynomials p0 .. p0 + count - 1.  List mode: the jobs of one group, for the items i0 ...
+struct BlockUnit {
+    uint32_t first, per, stride, count;   // job b of the unit: first + (b / per) * stride + b % per
+    __device__ __forceinline__ uint32_t job(uint32_t b) const { return per == 1 ? first + b * stride : first + (b / per) * stride + b % per; }
+};
+
+__device__ __forceinline__ BlockUnit block_unit(const NttArgs &a, uint32_t u) {
+    if (a.jobs) {
+        const uint32_t items = a.items ? a.items : 1;
+        uint32_t first, per, chunk;
+        if (a.groups) {
+            chunk = u / a.n_groups;
+            const LimbGroup g = a.groups[u - chunk * a.n_groups];
+            first = g.first;
+            per = g.count;
+        } else {
+            chunk = u / a.n_jobs;
+            first = u - chunk * a.n_jobs;
+            per = 1;
+        }
+        const uint32_t i0 = chunk * a.batch, n = items - i0 < a.batch ? items - i0 : a.batch;
+        return BlockUnit{i0 * a.n_jobs + first, per, a.n_jobs, n * per};
+    }
+    const uint32_t limb = u % a.map.limbs, p0 = (u / a.map.limbs) * a.batch;
+    return BlockUnit{p0 * a.map.limbs + limb, 1, a.map.limbs, a.n_polys - p0 < a.batch ? a.n_polys - p0 : a.batch};
+}
+
+// Blocks pass: a wave owns one block of 256 consecutive words of every limb of its unit, every exchange stays inside the
+// wave.  The next limb's words are requested before the current one's butterflies.
+template <bool FWD, bool EPI, bool LOOP, class A>
+__device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &unit, Job job, const A &ar, uint64_t q, uint32_t blk,
+                                              uint32_t lane, uint64_t *lds) {
+    using T4 = Tile4<8, 8>;
+    constexpr bool FP = std::is_same<A, FpArith>::value;
+    const size_t off = (size_t)blk * 256;
+    auto fetch = [&](uint64_t *x, const Job &j) {
+        if (FWD) {
+            // the rows pass left its words in out
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = j.out[off + T4::word(0, lane, i)];
+        } else if (a.in_galois) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) x[i] = j.in[galois_index((uint32_t)off + 4 * lane + i, a.in_galois, a.log_n)];
+        } else {
+            load4(x, j.in + off + 4 * lane);
+        }
+    };
+    uint64_t x[4], nx[4];
+    fetch(nx, job);
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    for (uint32_t b = 0;; b++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = nx[j];
+        const bool more = LOOP && b + 1 < unit.count;
+        EpiOperands e;
+        if (FWD && EPI) e = load_epilogue(a, job, off + 4 * lane);
+        Job next = job;
+        if (more) {
+            next = decode_job(a, unit.job(b + 1));
+            fetch(nx, next);
+        }
+        typename A::V v[4];
+        if constexpr (FP) {
+            const FpMod m = ar.m;
+            if (FWD) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
+                ar.reduce(v);
+                T4::template forward<A>(v, tw, ar, lds, lane);
+                if (EPI) {
+                    // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
+                    const double wd = fp_from_u64(a.w[2 * job.limb]);
+                    const FpTw ew{wd, wd * m.qinv};
+                    if (e.fma) {
+                        const double pd = fp_from_u64(a.pro_w[2 * job.limb]);
+                        const FpTw pw{pd, pd * m.qinv};
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            const double lhs = fp_mulmod(fp_from_u64(e.a[j]), pw, m) + fp_from_u64(e.b[j]);
+                            v[j] = fp_mulmod(lhs - v[j], ew, m);
+                        }
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            v[j] = fp_mulmod(fp_from_u64(e.a[j]) - v[j], ew, m);
+                            if (e.add) v[j] += fp_from_u64(e.b[j]);
+                        }
+                    }
+                }
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(v[j], m));
+                store4(EPI ? e.dst : job.out + off + 4 * lane, x);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(x[j]);
+                T4::template inverse<A>(v, tw, ar, lds, lane);
+            }
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = x[j];
+            if (FWD) {
+                T4::template forward<A>(v, tw, ar, lds, lane);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[j] = reduce_4q(v[j], q);
+                if (EPI) {
+                    const Shoup ew = load_shoup(a.w, job.limb);
+                    if (e.fma) {
+                        const Shoup pw = load_shoup(a.pro_w, job.limb);
+#pragma unroll
+                        for (int j = 0; j < 4; j++)
+                            x[j] = mul_shoup(sub_mod(add_mod(mul_shoup(e.a[j], pw, q), e.b[j], q), x[j], q), ew, q);
+                    } else {
+#pragma unroll
+                        for (int j = 0; j < 4; j++) {
+                            x[j] = mul_shoup(sub_mod(e.a[j], x[j], q), ew, q);
+                            if (e.add) x[j] = add_mod(x[j], e.b[j], q);
+                        }
+                    }
+                }
+                store4(EPI ? e.dst : job.out + off + 4 * lane, x);
+            } else {
+                T4::template inverse<A>(v, tw, ar, lds, lane);
+            }
+        }
+        if (!FWD) {
+            // lazy words (signed doubles, or integers in [0, 2q)) go to the rows pass
+#pragma unroll
+            for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(v[j]);
+        }
+        if (!more) break;
+        job = next;
+        wave_sync();   // (the next limb's exchanges reuse the LDS words that this one's lanes have read)
+    }
+}
+
+template <bool FWD, bool EPI, bool LOOP, int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a) {
+    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = logical_block() * kBlockWaves + w;   // (a limb has an even number of blocks)
+    const BlockUnit unit = block_unit(a, id >> lr);
+    const uint32_t blk = id & ((1u << lr) - 1);
+    const Job job = decode_job(a, unit.job(0));
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane, lds_all[w]);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), a.moduli[job.table], blk, lane, lds_all[w]);
+    }
+}
+
+// Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
+// (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
+// tiles of one wave, N = 2^17 needs 2048.
+template <bool FWD, int BE, bool SRC_INTT = false>
+hipError_t launch_rows(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
+    const uint32_t ld = a.log_n - 8;
+    const bool large = ((uint64_t)n_jobs << a.log_n) >= ((uint64_t)32 << 16);
+    const uint32_t b = ld < 4 ? 8 : (large || ld > 8) ? 11 : 10;
+    const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
+#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, B>), grid, block, 0, s, a)
+#define HE_CASE(LD)         \
+    case LD:                \
+        if (large)          \
+            HE_ROWS(LD, 11); \
+        else                \
+            HE_ROWS(LD, 10); \
+        break;
+    if constexpr (!SRC_INTT) {
+        switch (ld) {
+            case 1: HE_ROWS(1, 8); return hipGetLastError();
+            case 2: HE_ROWS(2, 8); return hipGetLastError();
+            case 3: HE_ROWS(3, 8); return hipGetLastError();
+            case 9: HE_ROWS(9, 11); return hipGetLastError();
+            default: break;
+        }
+    }
+    switch (ld) {
+        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+        default: return hipErrorInvalidValue;
+    }
+#undef HE_CASE
+#undef HE_ROWS
+    return hipGetLastError();
+}
+
+}  // namespace
+
+bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
+    return log_n >= 12 && log_n <= 16 && n_tables <= 64 && ((uint64_t)n_jobs << log_n) <= ((uint64_t)16 << 16);
+}
+
+hipError_t launch_ntt_rows(const NttArgs &a, uint32_t n_jobs, bool forward, int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
+    if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
+        // one instantiation per degree, which follows fp_mask limb by limb: the mask stands for the launch's back end here
+        if (!forward || !a.pro_itw || (a.pro_src_fp_mask && !a.pro_itw_fp)) return hipErrorInvalidValue;
+        NttArgs b = a;
+        b.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+        return launch_rows<true, NTT_BACKEND_MIXED, true>(b, n_jobs, s);
+    }
+    if (forward)
+        return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED>(a, n_jobs, s)
+               : backend                    ? launch_rows<true, NTT_BACKEND_FP>(a, n_jobs, s)
+                                            : launch_rows<true, NTT_BACKEND_INT>(a, n_jobs, s);
+    return backend == NTT_BACKEND_MIXED ? launch_rows<false, NTT_BACKEND_MIXED>(a, n_jobs, s)
+           : backend                    ? launch_rows<false, NTT_BACKEND_FP>(a, n_jobs, s)
+                                        : launch_rows<false, NTT_BACKEND_INT>(a, n_jobs, s);
+}
+
+// Limbs of one prime in turn on one wave, which reads its twiddles once: saves up to a third of the traffic (FP64; half of it
+// on the integer back end), but each wave then works longer and there are fewer.  It pays from four limbs in turn on
+// (two: 29.9 against 27.1 us for 2 x 24 limbs) as long as the launch keeps six waves per SIMD: 12 x 24 limbs 130 -> 112 us,
+// 8 x 24 of 60 bits 126 -> 112 us.
+constexpr uint32_t kLoopWaves = 6144;
+
+hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
+    const uint32_t blocks = 1u << (a.log_n - 8), repeats = a.jobs ? (a.items ? a.items : 1) : n_polys;
+    // (job lists: the groups of one table come into play when even four-limb units leave that many waves)
+    if (a.jobs && (uint64_t)a.n_groups * repeats * blocks < 4 * kLoopWaves) a.groups = nullptr;
+    const uint32_t kinds = !a.jobs ? a.map.limbs : a.groups ? a.n_groups : a.n_jobs;
+    const uint64_t waves = (uint64_t)kinds * blocks;
+    const uint32_t split = waves >= kLoopWaves ? 1 : (uint32_t)((kLoopWaves + waves - 1) / waves);
+    a.batch = (repeats + split - 1) / split;
+    if (a.batch < 4 && !a.groups) a.batch = 1;
+    a.n_polys = n_polys;
+    const dim3 grid(kinds * ((repeats + a.batch - 1) / a.batch) * (blocks / kBlockWaves)), block(64 * kBlockWaves);
+#define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
+    do {                                                                                                                \
+        if (backend == NTT_BACKEND_MIXED)                                                                               \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_MIXED>), grid, block, 0, s, a);    \
+        else if (backend)                                                                                               \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_FP>), grid, block, 0, s, a);       \
+        else                                                                                                            \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT>), grid, block, 0, s, a);      \
+    } while (0)
+    const bool epi = forward && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || a.epi_mode == NTT_EPI_FMA_SUB_MUL);
+    const bool loop = a.batch > 1 || a.groups;
+    if (epi && loop)
+        HE_LAUNCH(true, true, true);
+    else if (epi)
+        HE_LAUNCH(true, true, false);
+    else if (forward && loop)
+        HE_LAUNCH(true, false, true);
+    else if (forward)
+        HE_LAUNCH(true, false, false);
+    else if (loop)
+        HE_LAUNCH(false, false, true);
+    else
+        HE_LAUNCH(false, false, false);
+#undef HE_LAUNCH
+    return hipGetLastError();
+}
+
+}  // namespace he
