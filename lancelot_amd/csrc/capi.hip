@@ -888,8 +888,12 @@ namespace {
 // ModUp of `items` polynomials: item k reads c + k * c_item_stride * N (stride in limbs), writes out [k][beta][L+K][N];
 // ws holds items * L limbs
 // in_galois != 0 (one item, skip_own): the input is sigma(c), X -> X^in_galois, gathered by the inverse blocks pass
+// lazy: the forward transform of the converted limbs stops after its rows pass (launch_ntt_inner goes on from there); the
+// digits' own limbs are not copied.  tin: c is the third polynomial of a tensor product that has not been formed yet; the
+// inverse blocks pass forms it (FP64 back end).
 int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_item_stride, uint32_t items,
-               uint64_t *out, uint64_t *ws, he_stream s, bool skip_own = false, uint32_t in_galois = 0) {
+               uint64_t *out, uint64_t *ws, he_stream s, bool skip_own = false, uint32_t in_galois = 0, bool lazy = false,
+               const TensorFuse *tin = nullptr) {
     if (!ctx || !c || !out || !ws || ctx->size_p == 0 || items == 0 || c_item_stride < L) return HE_E_INVALID_ARGUMENT;
     const Level *lv = level_of(ctx, L);
     if (!lv) return HE_E_LEVEL_NOT_SET;
@@ -906,7 +910,8 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     inv.epi_mode = NTT_EPI_MUL;
     inv.w = lv->d_part_hat_inv;
     // skip_own (batched levels only): the consumer reads a digit's own limbs from c, their slots in out stay unwritten
-    if (skip_own && !lv->batched) return HE_E_INVALID_ARGUMENT;
+    if (lazy) skip_own = true;
+    if (skip_own && !lv->batched && !lazy) return HE_E_INVALID_ARGUMENT;
     if (in_galois && (items != 1 || !skip_own)) return HE_E_INVALID_ARGUMENT;   // (own limbs are copied from c as it is)
     inv.in_galois = in_galois;
     const bool fused = fuse_rows_ok(ctx, lv, L);
@@ -917,7 +922,8 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     // ... and a small launch finishes the inverse transform there as well
     const int inv_backend = backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, lv->n_modup_jobs * items);
-    HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), false, source_intt));
+    if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, S(s)));
+    HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), tin != nullptr, source_intt));
     const uint32_t copy_rows = skip_own ? 0 : lv->modup_max_copy;
     if (reduce_in_ntt) {
         for (uint32_t d = 0; d < lv->beta && !skip_own; d++)
@@ -939,7 +945,7 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
         const Digit &g = lv->digits[d];
         uint64_t *od = out + (size_t)d * LK * n;
         // the digit's own limbs keep their NTT form
-        HE_HIP(hipMemcpyAsync(od + (size_t)g.start * n, c + (size_t)g.start * n, (size_t)g.size * n * sizeof(uint64_t),
+        if (!skip_own) HE_HIP(hipMemcpyAsync(od + (size_t)g.start * n, c + (size_t)g.start * n, (size_t)g.size * n * sizeof(uint64_t),
                               hipMemcpyDeviceToDevice, S(s)));
         BconvArgs b{ws + (size_t)g.start * n, od, lv->d_mats + g.mat_off, g.d_out_limb, g.d_out_table, g.size, g.n_out};
         HE_HIP(launch_bconv(ctx->tables(), b, S(s)));
@@ -959,6 +965,10 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
         fwd.pro_item_stride = (size_t)L * n;
         fwd.pro_lk = LK;
         if (source_intt) set_source_intt(ctx, fwd, inv_backend);
+    }
+    if (lazy) {
+        if (!fused) HE_HIP(launch_ntt_rows(fwd, lv->n_modup_jobs * items, true, backend_for_level(ctx, L), S(s)));
+        return HE_OK;
     }
     HE_HIP(launch_ntt_forward(fwd, 1, backend_for_level(ctx, L), S(s), fused));
     return HE_OK;
@@ -1111,15 +1121,15 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
                   uint32_t items, const uint64_t *const *evk, uint32_t galois_elt, const uint64_t *fold_ct, uint64_t *ws,
                   he_stream s, const uint64_t *add_c0 = nullptr, const TensorFuse *tin = nullptr) {
     if (items == 0 || (items > 1 && (galois_elt || add_c0))) return HE_E_INVALID_ARGUMENT;
+    if (galois_elt && (!(galois_elt & 1) || galois_elt >= (2u << ctx->log_n))) return HE_E_INVALID_ARGUMENT;
     const uint64_t *fold_w = fold_ct ? ctx->d_pinv_mod_q + 2 * (size_t)(L - 1) : nullptr;
     const size_t n = ctx->n();
     const KsWorkspace w = ks_workspace(ctx, lv, L, items, ws);
     uint64_t *y = w.y, *cx = w.cx, *tmp = w.tmp;
     const uint64_t *src = c;
-    const bool fused_inner = ctx->fuse_inner && lv->batched && fp_for_level(ctx, L) &&
-                             (items == 1 || (ctx->batch_fused_inner && !tin));
-    // levels whose inner product reads a digit's own limbs from the input gather sigma(c) where they read c (the
-    // inverse blocks pass and the inner product); the others stage it
+    const bool fused_inner = ctx->fuse_inner && (items == 1 || ctx->batch_fused_inner);
+    // the separate kernels: levels whose inner product reads a digit's own limbs from the input gather sigma(c) where they
+    // read c (the inverse blocks pass and the inner product); the others stage it
     const bool gather = galois_elt && !fused_inner && lv->batched && items == 1;
     if (galois_elt && !fused_inner && !gather) {
         // sigma(c) is staged in the second half of the ModDown workspace, which ModUp leaves alone and ModDown
@@ -1129,47 +1139,17 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         src = staged;
     }
     if (fused_inner) {
-        // ModUp without the copy of a digit's own limbs, then the forward NTT fused with the inner product: the
-        // transformed digits are never written (216 limb transfers less at L = 24, K = 8)
-        // (a batch: the items are the polynomials of the inverse transform and the items of everything after it)
-        NttArgs inv = base_args(ctx, false);
-        inv.in = src;
-        inv.out = tmp;
-        inv.in_poly_stride = items == 1 ? L : c_item_stride;
-        inv.out_poly_stride = L;
-        inv.map = plain_map(L, 0);
-        inv.epi_mode = NTT_EPI_MUL;
-        inv.w = lv->d_part_hat_inv;
-        inv.in_galois = galois_elt;
-        // tin: c is the third polynomial of a tensor product that has not been formed yet; the blocks pass forms it
-        if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, S(s)));
-        HE_HIP(launch_ntt_inverse(inv, items, NTT_BACKEND_FP, S(s), tin != nullptr));
+        // ModUp up to the rows pass of its forward transform (no copy of a digit's own limbs), then the blocks pass
+        // fused with the inner product: the transformed digits are never written (216 limb transfers less at L = 24, K = 8)
+        for (uint32_t d = 0; d < lv->beta; d++)
+            if (!evk[d]) return HE_E_INVALID_ARGUMENT;
+        if (int rc = modup_impl(ctx, L, src, items == 1 ? L : c_item_stride, items, y, tmp, s, true, galois_elt, true, tin)) return rc;
         NttArgs fwd = base_args(ctx, true);
-        fwd.in = y;
         fwd.out = y;
-        fwd.jobs = lv->d_modup_jobs;
-        fwd.n_jobs = lv->n_modup_jobs;
-        fwd.groups = lv->d_modup_groups;
-        fwd.n_groups = lv->n_modup_groups;
-        fwd.items = items;
         fwd.item_stride = (size_t)lv->beta * (L + ctx->size_p) * n;
-        const bool rows_done = fuse_rows_ok(ctx, lv, L);
-        if (rows_done) {
-            BconvRows b{tmp, y, nullptr, lv->d_mats_fp, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
-                        lv->beta, lv->modup_max_rows, 0, items, (size_t)L * n, fwd.item_stride, 0, 0, lv->d_mx_up};
-            HE_HIP(launch_bconv_rows(fwd, b, ctx->tune, S(s)));
-        } else {
-            BconvBatch b{tmp, y, src, lv->d_mats, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
-                         lv->beta, lv->modup_max_rows, 0, lv->d_mats_fp, ctx->d_fp_consts, items, (size_t)L * n,
-                         fwd.item_stride, 0};
-            HE_HIP(launch_bconv_batched(ctx->tables(), b, ctx->tune, S(s)));
-        }
         KsFuseArgs x;
         memset(&x, 0, sizeof(x));
-        for (uint32_t d = 0; d < lv->beta; d++) {
-            if (!evk[d]) return HE_E_INVALID_ARGUMENT;
-            x.evk.p[d] = evk[d];
-        }
+        for (uint32_t d = 0; d < lv->beta; d++) x.evk.p[d] = evk[d];
         x.own = src;
         x.own_galois = galois_elt;
         x.add_c0 = add_c0;
@@ -1185,7 +1165,7 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         x.items = items;
         x.own_item_stride = (size_t)c_item_stride * n;
         x.fold_item_stride = 2 * (size_t)L * n;
-        HE_HIP(launch_ntt_forward_inner(fwd, x, S(s), rows_done));
+        HE_HIP(launch_ntt_inner(fwd, x, backend_for_level(ctx, L), S(s)));
     } else {
         // a batch on the FP64 back end shares each key word among the items of a group and reads a digit's own limbs
         // where they are

@@ -309,10 +309,10 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
                               size_t ct_item_stride, hipStream_t s, const double *fp_consts = nullptr, uint64_t fp_mask = 0,
                               bool own_from_ct = false);
 
-// Forward NTT of ModUp's converted limbs fused with the key-switch inner product (FP64 back end only).
-// `a` describes the converted limbs as launch_ntt_forward's job list does (a.out = the beta x (L+K) x N digit
-// buffer, whose own-digit limbs are never touched); the blocks pass multiplies every transformed tile by the
-// matching key tile and accumulates over the digits, so the transformed limbs are never written:
+// Blocks pass of the forward transform of ModUp's converted limbs fused with the key-switch inner product, on any back end.
+// a.out holds the words that the rows pass left (beta x (L+K) x N per item, whose own-digit limbs are never touched); every
+// transformed block is multiplied by the matching key words and summed over the digits, so the transformed limbs
+// are never written:
 //   out[k][t] = sum_d y_d[t] * evk_d[k][t],  y_d[t] = own[t] for the limbs t of digit d itself.
 struct KsFuseArgs {
     EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form
@@ -335,7 +335,7 @@ struct KsFuseArgs {
     uint32_t items;
     size_t own_item_stride, fold_item_stride;
 };
-hipError_t launch_ntt_forward_inner(const NttArgs &a, const KsFuseArgs &x, hipStream_t s, bool rows_done = false);
+hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s);
 
 hipError_t launch_decompose_real(const Tables &t, const double *coeffs, uint64_t *out, uint32_t limbs, uint32_t first,
                                  uint32_t items, size_t out_item_stride, hipStream_t s);

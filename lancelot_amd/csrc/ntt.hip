@@ -710,174 +710,6 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
 
 constexpr int kPer = 16;  // words per thread in the fused blocks passes
 
-// Forward blocks pass of ModUp fused with the key-switch inner product.  Workgroup = (limb t of Ql u P, tile of
-// 16 T words): its first T threads transform that tile of every digit in turn; all 2 T threads then multiply
-// it by a key polynomial (threads below T by the first, the others by the second) and accumulate in registers.
-// The key tiles are fetched before the butterflies start, so that they travel meanwhile; the digit that owns
-// limb t contributes the input itself.
-template <uint32_t T>
-__global__ __launch_bounds__(2 * T) __attribute__((amdgpu_waves_per_eu(2))) void ntt_blocks_fp_inner_kernel(NttArgs a, KsFuseArgs x) {
-    constexpr uint32_t kInnerTile = 16 * T + T;   // words of one skewed tile
-    __shared__ uint64_t lds[2 * kInnerTile];
-    constexpr uint32_t half = T, tile_elems = half << 4;
-    const uint32_t role = threadIdx.x >= half ? 1u : 0u;       // which key polynomial this thread accumulates
-    const uint32_t tid = threadIdx.x - role * half;
-    const uint32_t lr = a.log_n - 8;
-    const uint32_t log_b = 31 - __builtin_clz(tile_elems >> 8);
-    const uint32_t tiles_per_limb = 1u << (lr - log_b);
-    const uint32_t LK = x.L + x.K;
-    const size_t n = (size_t)1 << a.log_n;
-    uint32_t lb, item = 0;
-    if (x.items > 1) {
-        // hardware id -> XCD id & 7; inside an XCD the items of one (limb, tile) are consecutive
-        const uint32_t pairs = LK * tiles_per_limb, id = blockIdx.x;
-        if (pairs % 8 == 0) {
-            const uint32_t s = id >> 3;
-            item = s % x.items;
-            lb = (s / x.items) * 8 + (id & 7);
-        } else {
-            item = id / pairs;
-            lb = id - item * pairs;
-        }
-    } else {
-        // plain order, last limb first: the special limbs have one digit more to transform than the others, so their
-        // workgroups start first and are spread over all XCDs (a tile's twiddles are its own: nothing to share)
-        lb = gridDim.x - 1 - blockIdx.x;
-    }
-    const uint32_t t = lb / tiles_per_limb, tile = lb % tiles_per_limb;
-    const size_t off = (size_t)tile * tile_elems;
-    const uint32_t blk0 = tile << log_b;
-    const uint32_t table = t < x.L ? t : x.size_q + (t - x.L);
-    const uint32_t own = t < x.L ? t / x.K : 0xffffffffu;
-    // (locals: a modified copy of the argument structs would move their pointer tables to scratch memory)
-    const uint64_t *own_base = x.own + item * x.own_item_stride;
-    const uint64_t *lazy_base = a.out + item * a.item_stride;
-    uint64_t *out_base = x.out + item * (2 * (size_t)LK * n);
-    const uint64_t *fold_base = x.fold_ct ? x.fold_ct + item * x.fold_item_stride : nullptr;
-    double *ld = reinterpret_cast<double *>(lds);
-    const FpCtx fc = fp_ctx(a, table);
-    const FpMod m = fc.m;
-
-    const uint32_t base0 = ((tid >> 4) << 8) | (tid & 15);
-    const uint32_t base1 = tid << 4;
-    // the twiddles stay in the table (the digits after the first find them in cache)
-    const uint32_t idx0 = (1u << lr) + blk0 + (tid >> 4), idx1 = (1u << (lr + 4)) + (blk0 << 4) + tid;
-
-    // the 15 + 15 twiddles of the two register blocks are the same for every digit: loaded once, ahead of everything
-    // else (fetched inside the blocks they would each cost a round trip to L2 that nothing covers)
-    double twA[15], twB[15];
-    fp_load_block_tw<4>(twA, fc.tw, idx0);
-    fp_load_block_tw<4>(twB, fc.tw, idx1);
-
-    const size_t key_off = ((size_t)role * x.size_qp + table) * n + off;
-    double acc[kPer];
-    if (own != 0xffffffffu) {
-        const uint64_t *src = own_base + (size_t)t * n;
-        const uint64_t *key = x.evk.p[own] + key_off;
-        uint64_t c[kPer];
-        if (x.own_galois) {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) c[i] = src[galois_index((uint32_t)off + tid + i * half, x.own_galois, a.log_n)];
-        } else {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) c[i] = src[(uint32_t)off + tid + i * half];
-        }
-#pragma unroll
-        for (int i = 0; i < kPer; i++) {
-            const double w = fp_from_u64(key[tid + i * half]);
-            acc[i] = fp_mulmod(fp_from_u64(c[i]), FpTw{w, w * m.qinv}, m);
-        }
-    } else {
-#pragma unroll
-        for (int i = 0; i < kPer; i++) acc[i] = 0.0;
-    }
-
-    // The other digits two at a time: the threads of role 0 transform the first one's tile, those of role 1 the
-    // second one's (each into its own LDS tile, the same sequence of steps at the same time), then every thread
-    // multiplies both tiles by its key polynomial.  With the transforms on one role only, half of the workgroup's
-    // waves (and the SIMDs they sit on) would idle during the butterflies.
-    auto skip_own = [&](uint32_t d) { return d == own ? d + 1 : d; };
-    for (uint32_t da = skip_own(0); da < x.beta;) {
-        const uint32_t db = skip_own(da + 1);
-        const bool two = db < x.beta;
-        const uint32_t mine = role ? db : da;
-        const bool work = role ? two : true;
-        // key words of the first digit are requested before the butterflies, those of the second after them (they
-        // arrive while the first tile is multiplied): both sets up front would not fit the register file
-        uint64_t pka[kPer], pkb[kPer];
-        const uint64_t *ka = x.evk.p[da] + key_off, *kb = x.evk.p[two ? db : da] + key_off;
-#pragma unroll
-        for (int i = 0; i < kPer; i++) pka[i] = ka[tid + i * half];
-        double *ldm = ld + role * kInnerTile;
-        const uint64_t *src = lazy_base + ((size_t)mine * LK + t) * n + off;  // lazy values left by the rows pass
-        if (work) {
-            // the 16 words of the first register block (stride 16 inside a 256-block) straight from global memory:
-            // 16 neighbouring threads read one 128-byte line per access
-            double v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = __longlong_as_double((long long)src[base0 + (j << 4)]);
-            fp_ct_block_tw<4, true>(v, twA, m);
-#pragma unroll
-            for (int j = 0; j < 16; j++) ldm[skew(base0 + (j << 4))] = v[j];
-        }
-        lds_barrier();
-#pragma unroll
-        for (int i = 0; i < kPer / 2; i++) pkb[i] = kb[tid + i * half];
-        if (work) {
-            double v[16];
-#pragma unroll
-            for (int j = 0; j < 16; j++) v[j] = ldm[skew(base1 + j)];
-            fp_ct_block_tw<4, true>(v, twB, m);
-#pragma unroll
-            for (int j = 0; j < 16; j++) ldm[skew(base1 + j)] = v[j];
-        }
-#pragma unroll
-        for (int i = kPer / 2; i < kPer; i++) pkb[i] = kb[tid + i * half];
-        lds_barrier();
-        // The transformed words go into the products as the second block leaves them (at most 5.3 q in magnitude):
-        // each term is then at most (1/2 + 0.375 x 5.3) q < 2.5 q, and an accumulator that starts a pair below q ends
-        // it below 6 q < 2^53; one reduction per pair instead of one per word and digit.
-#pragma unroll
-        for (int i = 0; i < kPer; i++) {
-            const double w = fp_from_u64(pka[i]);
-            acc[i] += fp_mulmod(ld[skew(tid + i * half)], FpTw{w, w * m.qinv}, m);
-        }
-        if (two) {
-#pragma unroll
-            for (int i = 0; i < kPer; i++) {
-                const double w = fp_from_u64(pkb[i]);
-                acc[i] += fp_mulmod(ld[kInnerTile + skew(tid + i * half)], FpTw{w, w * m.qinv}, m);
-            }
-        }
-#pragma unroll
-        for (int i = 0; i < kPer; i++) acc[i] = fp_reduce(acc[i], m);
-        lds_barrier();  // every read of these tiles is done before the next pair overwrites them
-        da = skip_own(db + 1);
-    }
-    if (x.add_c0 && !role && t < x.L) {
-        // a rotation: polynomial 0 gains P sigma(c0), which ModDown's division by P turns into sigma(c0)
-        const uint64_t *c0 = x.add_c0 + (size_t)t * n;
-        const double pd = fp_from_u64(x.p_mod_q[2 * t]);
-        const FpTw pw{pd, pd * m.qinv};
-#pragma unroll
-        for (int i = 0; i < kPer; i++) {
-            const uint32_t e = (uint32_t)off + tid + i * half;
-            acc[i] += fp_mulmod(fp_from_u64(c0[x.own_galois ? galois_index(e, x.own_galois, a.log_n) : e]), pw, m);
-        }
-    }
-    uint64_t *o = out_base + ((size_t)role * LK + t) * n + off;
-    if (fold_base && t == x.L - 1) {
-        const uint64_t *cl = fold_base + ((size_t)role * x.L + t) * n + off;
-        const double wd = fp_from_u64(x.fold_w[0]);
-        const FpTw w{wd, wd * m.qinv};
-#pragma unroll
-        for (int i = 0; i < kPer; i++)
-            acc[i] = fp_mulmod(fp_canonical(acc[i], m), w, m) + fp_from_u64(cl[tid + i * half]);
-    }
-#pragma unroll
-    for (int i = 0; i < kPer; i++) o[tid + i * half] = fp_to_u64(fp_canonical(acc[i], m));
-}
-
 // Tensor product fused with the blocks pass of the inverse transform of its third polynomial (FP64 back end, one
 // workgroup per (limb, tile of 16 T words)): (d0, d1, d2) = (a0 b0, a0 b1 + a1 b0, a1 b1) from the four input tiles,
 // all three written as canonical residues (d2 in NTT form is what the key switch multiplies by its own digit's key),
@@ -1020,27 +852,6 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
     if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb_fp<true>(a, n_jobs, s);
     const hipError_t e = rows_done ? hipSuccess : launch_ntt_rows(a, n_jobs, true, backend, s);
     return e != hipSuccess ? e : launch_ntt_blocks(a, n_polys, true, backend, s);
-}
-
-hipError_t launch_ntt_forward_inner(const NttArgs &a, const KsFuseArgs &x, hipStream_t s, bool rows_done) {
-    if (a.log_n < 9 || a.log_n > 17 || !a.jobs) return hipErrorInvalidValue;
-    const uint32_t items = x.items ? x.items : 1;
-    if (items > 1 && (x.own_galois || x.add_c0 || (a.items ? a.items : 1) != items)) return hipErrorInvalidValue;
-    if (a.n_jobs && !rows_done) {
-        hipError_t e = launch_ntt_rows(a, a.n_jobs * items, true, NTT_BACKEND_FP, s);
-        if (e != hipSuccess) return e;
-    }
-    const uint32_t n = 1u << a.log_n;
-    // tiles of 1024 words (workgroups of two waves, four of them on a CU): 229 us against 244 us with 2048-word tiles
-    // for 8 x (24 + 8) limbs of 2^16 words, 39.7 against 42.8 us for one ciphertext's; 512-word tiles measure the same
-    const uint32_t tile = n < 1024 ? n : 1024;
-    if ((uint64_t)(x.L + x.K) * (n / tile) * items > 0x7fffffffu) return hipErrorInvalidValue;
-    const dim3 grid((x.L + x.K) * (n / tile) * items);
-    if (tile == 1024)
-        hipLaunchKernelGGL(ntt_blocks_fp_inner_kernel<64>, grid, dim3(128), 0, s, a, x);
-    else
-        hipLaunchKernelGGL(ntt_blocks_fp_inner_kernel<32>, grid, dim3(64), 0, s, a, x);
-    return hipGetLastError();
 }
 
 hipError_t launch_tensor_intt_blocks(NttArgs a, const TensorFuse &x, hipStream_t s) {

@@ -499,6 +499,208 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a)
     }
 }
 
+// Sum over the digits of (word x key word) for four words of both key polynomials.
+// FP64: a transformed word enters as the last stage leaves it (at most 5.3 q: a term below 2.5 q), the sums are reduced after
+// every second digit and stay below 6 q.  Integers: canonical words, 128-bit sums of at most 64 products below 2^122.
+struct FpSums {
+    double s[2][4];
+    uint32_t pending = 0;
+    __device__ __forceinline__ FpSums() {
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[0][j] = s[1][j] = 0.0;
+    }
+    __device__ __forceinline__ void add(const double *v, const uint64_t (*k)[4], const FpArith &ar) {
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double w = fp_from_u64(k[r][j]);
+                s[r][j] += fp_mulmod(v[j], FpTw{w, w * ar.m.qinv}, ar.m);
+            }
+        if (++pending == 2) {
+            pending = 0;
+            ar.reduce(s[0]);
+            ar.reduce(s[1]);
+        }
+    }
+};
+
+struct IntSums {
+    U128 s[2][4];
+    __device__ __forceinline__ IntSums() {
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[0][j] = s[1][j] = U128{0, 0};
+    }
+    __device__ __forceinline__ void add(const uint64_t *v, const uint64_t (*k)[4], const IntArith &ar) {
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) mac128(s[r][j], v[j], k[r][j]);
+    }
+};
+
+// Blocks pass of ModUp's forward transform fused with the key-switch inner product: a wave owns one block of 256 words of limb t of
+// Ql u P, takes it through the last 8 stages for every digit in turn and multiplies it by both key polynomials; the digit
+// that owns limb t contributes the input itself.  The transformed limbs never reach memory.
+template <class A>
+__device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &x, uint32_t t, uint32_t table, uint32_t blk,
+                                            uint32_t item, uint32_t lane, const A &ar, uint64_t *lds) {
+    using T4 = Tile4<8, 8>;
+    constexpr bool FP = std::is_same<A, FpArith>::value;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const uint32_t LK = x.L + x.K, own = t < x.L ? t / x.K : 0xffffffffu;
+    const uint64_t *lazy = a.out + item * a.item_stride + (size_t)t * n + off;   // words left by the rows pass, digit 0
+    const size_t digit_stride = (size_t)LK * n, key_off = (size_t)table * n + at, key_poly = (size_t)x.size_qp * n;
+    auto skip_own = [&](uint32_t d) { return d == own ? d + 1 : d; };
+    auto fetch = [&](uint64_t *w, uint32_t d) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
+    };
+    auto keys = [&](uint64_t (*k)[4], uint32_t d) {
+        load4(k[0], x.evk.p[d] + key_off);
+        load4(k[1], x.evk.p[d] + key_poly + key_off);
+    };
+    typename A::Tw tw[4];
+    uint64_t nx[4];
+    uint32_t d = skip_own(0);
+    if (d < x.beta) fetch(nx, d);
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    typename std::conditional<FP, FpSums, IntSums>::type sums;
+    if (own != 0xffffffffu) {
+        const uint64_t *src = x.own + item * x.own_item_stride + (size_t)t * n;
+        uint64_t c[4], k[2][4];
+        keys(k, own);
+        if (x.own_galois) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) c[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+        } else {
+            load4(c, src + at);
+        }
+        typename A::V v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (FP)
+                v[j] = fp_from_u64(c[j]);
+            else
+                v[j] = c[j];
+        }
+        sums.add(v, k, ar);
+    }
+    while (d < x.beta) {
+        uint64_t k[2][4];
+        keys(k, d);
+        typename A::V v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = A::from_word(nx[j]);
+        d = skip_own(d + 1);
+        if (d < x.beta) fetch(nx, d);
+        ar.reduce(v);
+        T4::template forward<A>(v, tw, ar, lds, lane);
+        if constexpr (!FP) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = reduce_4q(v[j], ar.m.q);
+        }
+        sums.add(v, k, ar);
+        wave_sync();   // (the next digit's exchanges reuse the LDS words that this one's lanes have read)
+    }
+    uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)t * n + at;
+    const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
+    const bool fold = x.fold_ct && t == x.L - 1;
+    uint64_t c0[4], cl[2][4];
+    if (add) {
+        const uint64_t *src = x.add_c0 + (size_t)t * n;
+        if (x.own_galois) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+        } else {
+            load4(c0, src + at);
+        }
+    }
+    if (fold) {
+        const uint64_t *src = x.fold_ct + item * x.fold_item_stride + (size_t)t * n + at;
+        load4(cl[0], src);
+        load4(cl[1], src + (size_t)x.L * n);
+    }
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        uint64_t res[4];
+        if constexpr (FP) {
+            const FpMod m = ar.m;
+            double v[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = sums.s[r][j];
+            if (add && r == 0) {
+                const double pd = fp_from_u64(x.p_mod_q[2 * t]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] += fp_mulmod(fp_from_u64(c0[j]), FpTw{pd, pd * m.qinv}, m);
+            }
+            if (fold) {
+                const double wd = fp_from_u64(x.fold_w[0]);
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], FpTw{wd, wd * m.qinv}, m) + fp_from_u64(cl[r][j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; j++) res[j] = fp_to_u64(fp_canonical(v[j], m));
+        } else {
+            const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+#pragma unroll
+            for (int j = 0; j < 4; j++) res[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
+            if (add && r == 0) {
+                const Shoup w = load_shoup(x.p_mod_q, t);
+#pragma unroll
+                for (int j = 0; j < 4; j++) res[j] = add_mod(res[j], mul_shoup(c0[j], w, q), q);
+            }
+            if (fold) {
+                const Shoup w = load_shoup(x.fold_w, 0);
+#pragma unroll
+                for (int j = 0; j < 4; j++) res[j] = add_mod(mul_shoup(res[j], w, q), cl[r][j], q);
+            }
+        }
+        store4(o + (size_t)r * LK * n, res);
+    }
+}
+
+// Waves of a workgroup: of one item, neighbouring blocks; of a batch, the same block of neighbouring items, which find the
+// key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
+#ifndef INNER_WAVES
+#define INNER_WAVES 4
+#endif
+constexpr int kInnerWaves = INNER_WAVES;
+
+template <int BE>
+__global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
+    __shared__ uint64_t lds_all[kInnerWaves][256 + 16];
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = (x.L + x.K) << lr;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t pair, item = 0;
+    if (x.items > 1) {
+        const uint32_t groups = (x.items + kInnerWaves - 1) / kInnerWaves, id = blockIdx.x;
+        uint32_t g;
+        if (pairs % 8 == 0) {
+            // hardware id -> XCD id & 7; inside an XCD the groups of one pair are consecutive
+            const uint32_t s = id >> 3;
+            g = s % groups;
+            pair = (s / groups) * 8 + (id & 7);
+        } else {
+            g = id / pairs;
+            pair = id - g * pairs;
+        }
+        item = g * kInnerWaves + w;
+        if (item >= x.items) return;
+    } else {
+        // last limb first: the special limbs have one digit more to transform than the others
+        pair = blockIdx.x * kInnerWaves + w;
+        if (pair >= pairs) return;
+        pair = pairs - 1 - pair;
+    }
+    const uint32_t t = pair >> lr, blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) inner_block(a, x, t, table, blk, item, lane, fp_arith(a, table), lds_all[w]);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) inner_block(a, x, t, table, blk, item, lane, int_arith(a, table), lds_all[w]);
+    }
+}
+
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
@@ -600,6 +802,23 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     else
         HE_LAUNCH(false, false, false);
 #undef HE_LAUNCH
+    return hipGetLastError();
+}
+
+hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
+    const uint32_t items = x.items ? x.items : 1;
+    if (items > 1 && (x.own_galois || x.add_c0)) return hipErrorInvalidValue;
+    const uint64_t pairs = (uint64_t)(x.L + x.K) << (a.log_n - 8);
+    const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs + kInnerWaves - 1) / kInnerWaves;
+    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kInnerWaves);
+    if (backend == NTT_BACKEND_MIXED)
+        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
+    else if (backend)
+        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
+    else
+        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
     return hipGetLastError();
 }
 
