@@ -263,7 +263,7 @@ bool fp_for_level(const he_context *ctx, uint32_t L) {
 
 // base conversion fused with the rows pass of the forward transform that follows it (launch_bconv_rows)
 bool fuse_rows_ok(const he_context *ctx, const Level *lv, uint32_t L) {
-    return ctx->fuse_rows && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16 && fp_for_level(ctx, L);
+    return ctx->fuse_rows && !ctx->single_limb_digits && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16 && fp_for_level(ctx, L);
 }
 
 int check_map(const he_context *ctx, uint32_t limbs, uint32_t first, uint32_t split, uint32_t tail) {
@@ -922,7 +922,7 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     // ... and a small launch finishes the inverse transform there as well
     const int inv_backend = backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, lv->n_modup_jobs * items);
-    if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, S(s)));
+    if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, items, inv_backend, S(s)));
     HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), tin != nullptr, source_intt));
     const uint32_t copy_rows = skip_own ? 0 : lv->modup_max_copy;
     if (reduce_in_ntt) {
@@ -1174,7 +1174,7 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         bool fp_batch = items > 1 && lv->batched && fp_for_level(ctx, L) && n >= 512 && !galois_elt && !add_c0 &&
                         aligned16(src) && aligned16(cx) && aligned16(y) && aligned16(fold_ct);
         for (uint32_t d = 0; d < lv->beta && fp_batch; d++) fp_batch = aligned16(evk[d]);
-        if (tin) return HE_E_INVALID_ARGUMENT;
+        if (tin) return HE_E_INVALID_ARGUMENT;   // (the fused inner product only)
         // (batched levels: neither kernel needs the copy of a digit's own limbs into y)
         const bool skip_own = fp_batch || lv->batched;
         const uint32_t src_stride = (galois_elt && !gather) ? L : c_item_stride;
@@ -1267,9 +1267,9 @@ int he_hoisted_rotations(const he_context *ctx, uint32_t L, const uint64_t *ct_i
 
 namespace {
 
-// the fused tensor + key switch of he_multiply_relin_rescale applies: one input, FP64 back end, fused inner product
-bool tensor_fusion_ok(const he_context *ctx, const Level *lv, uint32_t L) {
-    return lv && ctx->fuse_tensor && ctx->fuse_inner && lv->batched && fp_for_level(ctx, L);
+// the fused tensor + key switch of he_multiply_relin_rescale[_batch] applies (its third polynomial is never read back)
+bool tensor_fusion_ok(const he_context *ctx, uint32_t items) {
+    return ctx->fuse_tensor && ctx->fuse_inner && (items == 1 || ctx->batch_fused_inner);
 }
 
 int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *c, uint32_t c_item_stride,
@@ -1377,7 +1377,7 @@ int he_multiply_relin_rescale(const he_context *ctx, uint32_t L, const uint64_t 
     if (!lv) return HE_E_LEVEL_NOT_SET;
     const size_t n = ctx->n();
     uint64_t *d01 = ws + he_keyswitch_workspace_words(ctx, L), *d2 = d01 + 2 * (size_t)L * n;
-    if (tensor_fusion_ok(ctx, lv, L)) {
+    if (tensor_fusion_ok(ctx, 1)) {
         const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0};
         return ksr_impl(ctx, L, 1, d2, L, evk, d01, out, 0, ws, s, &tin);
     }
@@ -1404,8 +1404,10 @@ int he_multiply_relin_rescale_batch(const he_context *ctx, uint32_t L, uint32_t 
     const size_t n = ctx->n();
     // [items] key-switch workspaces | (d0, d1) [items][2][L][N] | d2 [items][L][N]
     uint64_t *d01 = ws + (size_t)items * he_keyswitch_workspace_words(ctx, L), *d2 = d01 + (size_t)items * 2 * L * n;
-    // (a tensor product formed inside the key switch's first pass, as the single call does it, measures slower here:
-    // with many items in one launch the plain tensor kernel streams at a higher rate than the fused one computes)
+    if (tensor_fusion_ok(ctx, items)) {
+        const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0};
+        return ksr_impl(ctx, L, items, d2, L, evk, d01, out, 0, ws, s, &tin);
+    }
     HE_HIP(launch_tensor(ctx->tables(), ct1, ct2, d01, L, ct1 == ct2, S(s),
                          fp_for(ctx, plain_map(L)) ? ctx->d_fp_consts : nullptr, items, d2));
     return ksr_impl(ctx, L, items, d2, L, evk, d01, out, 0, ws, s, nullptr);

@@ -154,9 +154,9 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
 // whether a forward launch of n_jobs limbs may take NTT_PRO_SOURCE_INTT_REDUCE
 bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables);
 
-// Tensor product of two size-2 ciphertexts fused with the blocks pass of the inverse transform of its third polynomial
-// (FP64 back end; every prime of the L limbs below 2^50).  `a`: inverse base arguments with map = the L data limbs
-// and out = where the lazy words of INTT(d2) go ([L][N]); finish with launch_ntt_inverse(a, 1, FP, s, true).
+// Tensor product of two size-2 ciphertexts fused with the blocks pass of the inverse transform of its third polynomial, for
+// `items` products (operands and d01 [items][2][L][N], d2 [items][L][N]).  `a`: inverse base arguments with map = the L data
+// limbs and out = where the lazy words of INTT(d2) go; finish with launch_ntt_inverse(a, items, backend, s, true).
 struct TensorFuse {
     const uint64_t *ct1, *ct2;   // [2][L][N]
     uint64_t *d01;               // [2][L][N]: d0, d1
@@ -164,7 +164,7 @@ struct TensorFuse {
     uint32_t L;
     int square;                  // ct2 is ignored, (d0, d1, d2) = (a0^2, 2 a0 a1, a1^2)
 };
-hipError_t launch_tensor_intt_blocks(NttArgs a, const TensorFuse &x, hipStream_t s);
+hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s);
 
 struct Tables {
     const uint64_t *moduli;

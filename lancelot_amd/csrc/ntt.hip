@@ -35,9 +35,6 @@ namespace he {
 
 namespace {
 
-constexpr int kThreads = 256;
-constexpr uint32_t kLdsWords = 4096 + 256;   // a skewed tile of 16 words per thread
-
 // ---------------------------------------------------------------------------------------------------
 // Whole-limb transform for N <= 2^14 (FP64 back end, plain forward / inverse with the optional inverse scaling):
 // one workgroup of N / 16 threads per limb keeps the limb in LDS (at most 136 KiB of the CU's 160) between its
@@ -708,83 +705,6 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
     }
 }
 
-constexpr int kPer = 16;  // words per thread in the fused blocks passes
-
-// Tensor product fused with the blocks pass of the inverse transform of its third polynomial (FP64 back end, one
-// workgroup per (limb, tile of 16 T words)): (d0, d1, d2) = (a0 b0, a0 b1 + a1 b0, a1 b1) from the four input tiles,
-// all three written as canonical residues (d2 in NTT form is what the key switch multiplies by its own digit's key),
-// and d2 goes on through the 8 inverse stages inside 256 consecutive words; the lazy words are left in a.out for the
-// rows pass.  One read of d2 and one launch less than tensor kernel + inverse transform.
-template <bool SQUARE>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(1))) void tensor_intt_blocks_fp_kernel(NttArgs a, TensorFuse x) {
-    __shared__ uint64_t lds[kLdsWords];
-    double *ld = reinterpret_cast<double *>(lds);
-    const uint32_t nthreads = blockDim.x;
-    const uint32_t lr = a.log_n - 8, log_b = 31 - __builtin_clz(nthreads >> 4);   // 256-word blocks of a limb, of a tile
-    const uint32_t lb = logical_block(), tile = lb & ((1u << (lr - log_b)) - 1), blk0 = tile << log_b;
-    const Job job = decode_job(a, lb >> (lr - log_b));
-    const FpCtx fc = fp_ctx(a, job.table);
-    const FpMod m = fc.m;
-    const size_t n = (size_t)1 << a.log_n, off = (size_t)tile * nthreads * kPer;
-    const uint32_t gi = threadIdx.x;
-    const uint32_t base0 = ((gi >> 4) << 8) | (gi & 15);
-    const uint32_t base1 = gi << 4;
-    double tw0[15], tw1[15];
-    fp_load_block_tw<4>(tw0, fc.tw, (1u << lr) + blk0 + (gi >> 4));
-    fp_load_block_tw<4>(tw1, fc.tw, (1u << (lr + 4)) + (blk0 << 4) + gi);
-
-    const size_t lo = (size_t)job.limb * n + off, poly = (size_t)x.L * n;
-    // the launch has 1.5 waves per SIMD at N = 2^16, L = 24: all 64 loads of a thread are in flight at once
-#pragma unroll
-    for (int i = 0; i < kPer; i++) {
-        const uint32_t e = threadIdx.x + i * nthreads;
-        const double a0 = fp_from_u64(x.ct1[lo + e]), a1 = fp_from_u64(x.ct1[poly + lo + e]);
-        double d0, d1, d2;
-        if (SQUARE) {
-            d0 = fp_canonical(fp_mulmod(a0, FpTw{a0, a0 * m.qinv}, m), m);
-            d2 = fp_canonical(fp_mulmod(a1, FpTw{a1, a1 * m.qinv}, m), m);
-            const double mm = fp_mulmod(a0, FpTw{a1, a1 * m.qinv}, m);
-            d1 = fp_canonical(mm + mm, m);
-        } else {
-            const double b0 = fp_from_u64(x.ct2[lo + e]), b1 = fp_from_u64(x.ct2[poly + lo + e]);
-            d0 = fp_canonical(fp_mulmod(a0, FpTw{b0, b0 * m.qinv}, m), m);
-            d2 = fp_canonical(fp_mulmod(a1, FpTw{b1, b1 * m.qinv}, m), m);
-            // Karatsuba: (a0 + a1)(b0 + b1) - d0 - d2; both factors are below 2 q, the product is reduced to
-            // |r| <= 2 q and the difference stays below 4 q < 2^53
-            const double sb = b0 + b1;
-            const double mm = fp_mulmod(a0 + a1, FpTw{sb, sb * m.qinv}, m);
-            d1 = fp_canonical(mm - d0 - d2, m);
-        }
-        x.d01[lo + e] = fp_to_u64(d0);
-        x.d01[poly + lo + e] = fp_to_u64(d1);
-        x.d2[lo + e] = fp_to_u64(d2);
-        ld[skew(e)] = d2;
-    }
-#pragma unroll
-    for (int i = 0; i < 15; i++) asm volatile("" ::"v"(tw0[i]), "v"(tw1[i]));
-    lds_barrier();
-    double v[16];
-#pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = ld[skew(base1 + j)];
-    fp_gs_block_tw<4, false>(v, tw1, m);
-#pragma unroll
-    for (int j = 0; j < 16; j++) ld[skew(base1 + j)] = v[j];
-    lds_barrier();
-#pragma unroll
-    for (int j = 0; j < 16; j++) v[j] = ld[skew(base0 + (j << 4))];
-    fp_gs_block_tw<4, true>(v, tw0, m);
-#pragma unroll
-    for (int j = 0; j < 16; j++) ld[skew(base0 + (j << 4))] = v[j];
-    lds_barrier();
-    // lazy signed doubles go to the rows pass
-    uint64_t *dst = job.out + off;
-    uint64_t o[kPer];
-#pragma unroll
-    for (int i = 0; i < kPer; i++) o[i] = lds[skew(threadIdx.x + i * nthreads)];
-#pragma unroll
-    for (int i = 0; i < kPer; i++) dst[threadIdx.x + i * nthreads] = o[i];
-}
-
 }  // namespace
 
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, const Tuning &tune, hipStream_t s) {
@@ -852,20 +772,6 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
     if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb_fp<true>(a, n_jobs, s);
     const hipError_t e = rows_done ? hipSuccess : launch_ntt_rows(a, n_jobs, true, backend, s);
     return e != hipSuccess ? e : launch_ntt_blocks(a, n_polys, true, backend, s);
-}
-
-hipError_t launch_tensor_intt_blocks(NttArgs a, const TensorFuse &x, hipStream_t s) {
-    if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0) return hipErrorInvalidValue;
-    const uint32_t n = 1u << a.log_n;
-    // the largest of 4096-, 2048- and 1024-word tiles that still gives the chip workgroups enough (a limb may be smaller)
-    const uint32_t want = x.L * (n / (n < 4096 ? n : 4096)) >= 1024 ? 4096 : x.L * (n / (n < 2048 ? n : 2048)) >= 256 ? 2048 : 1024;
-    const uint32_t tile = n < want ? n : want;
-    const dim3 grid(x.L * (n / tile)), block(tile / kPer);
-    if (x.square)
-        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<true>, grid, block, 0, s, a, x);
-    else
-        hipLaunchKernelGGL(tensor_intt_blocks_fp_kernel<false>, grid, block, 0, s, a, x);
-    return hipGetLastError();
 }
 
 hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, hipStream_t s, bool blocks_done,

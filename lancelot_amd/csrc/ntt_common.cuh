@@ -1,6 +1,8 @@
 // What the kernels of the transform share: how a job names its limb, the per-limb constants of the two back ends, and the
 // prologues that form the input of a forward rows pass.
 #pragma once
+#include <type_traits>
+
 #include "kernels.h"
 #include "modarith.cuh"
 
@@ -156,6 +158,206 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = job.in[glob(j)];
     }
+}
+
+// Orders the LDS accesses of one wave's lanes: the hardware runs them in program order, so only the compiler is held.
+__device__ __forceinline__ void wave_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+// read-only tables that every lane of a wave reads at one address: through the scalar cache
+typedef const double __attribute__((address_space(4))) *ScalarF64;
+typedef const uint64_t __attribute__((address_space(4))) *ScalarU64;
+__device__ __forceinline__ ScalarF64 scalar(const double *p) { return (ScalarF64)(uintptr_t)p; }
+__device__ __forceinline__ ScalarU64 scalar(const uint64_t *p) { return (ScalarU64)(uintptr_t)p; }
+
+// Two stages (ST = 1: only the first of them) on four words; tw entries: the first stage's twiddle, then the two of the
+// second.
+struct IntArith {
+    using V = uint64_t;
+    struct Tw {
+        Shoup s[3];
+    };
+    IntMod m;
+    const uint64_t *table;
+    static __device__ __forceinline__ V from_word(uint64_t x) { return x; }
+    static __device__ __forceinline__ uint64_t to_word(V v) { return v; }
+    template <int ST, bool UNIFORM>
+    __device__ __forceinline__ Tw load(uint32_t idx) const {
+        auto at = [&](size_t i) { return UNIFORM ? Shoup{scalar(table)[2 * i], scalar(table)[2 * i + 1]} : load_shoup(table, i); };
+        Tw t;
+        t.s[0] = at(idx);
+        t.s[1] = t.s[2] = Shoup{0, 0};
+        if (ST == 2) {
+            t.s[1] = at(2 * (size_t)idx);
+            t.s[2] = at(2 * (size_t)idx + 1);
+        }
+        return t;
+    }
+    template <int ST>
+    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
+        ct_butterfly(v[0], v[2], t.s[0], m);
+        ct_butterfly(v[1], v[3], t.s[0], m);
+        if (ST == 2) {
+            ct_butterfly(v[0], v[1], t.s[1], m);
+            ct_butterfly(v[2], v[3], t.s[2], m);
+        }
+    }
+    template <int ST>
+    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
+        if (ST == 2) {
+            gs_butterfly(v[0], v[1], t.s[1], m);
+            gs_butterfly(v[2], v[3], t.s[2], m);
+        }
+        gs_butterfly(v[0], v[2], t.s[0], m);
+        gs_butterfly(v[1], v[3], t.s[0], m);
+    }
+    __device__ __forceinline__ void reduce(V *) const {}
+};
+
+// Bounds (in units of q, |v| < 8 keeps every value exact): forward, a stage takes b to 1.375 b + 0.5, so four stages
+// between reductions end at 5.3 (7.1 from canonical words); inverse, words are reduced before every two stages, whose
+// sums end at 2 (4 from canonical words) and whose products stay below that.
+struct FpArith {
+    using V = double;
+    struct Tw {
+        double w[3];
+    };
+    FpMod m;
+    const double *table;
+    static __device__ __forceinline__ V from_word(uint64_t x) { return __longlong_as_double((long long)x); }
+    static __device__ __forceinline__ uint64_t to_word(V v) { return (uint64_t)__double_as_longlong(v); }
+    // UNIFORM: idx is the same in every lane of the wave
+    template <int ST, bool UNIFORM>
+    __device__ __forceinline__ Tw load(uint32_t idx) const {
+        auto at = [&](size_t i) { return UNIFORM ? (double)scalar(table)[i] : table[i]; };
+        Tw t;
+        t.w[0] = at(idx);
+        t.w[1] = t.w[2] = 0.0;
+        if (ST == 2) {
+            t.w[1] = at(2 * (size_t)idx);
+            t.w[2] = at(2 * (size_t)idx + 1);
+        }
+        return t;
+    }
+    __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
+        asm volatile("" : "+v"(w));   // keeps w * qinv out of the registers that a loop over limbs holds
+        const double t = fp_mulmod(y, FpTw{w, w * m.qinv}, m);
+        y = x - t;
+        x = x + t;
+    }
+    __device__ __forceinline__ void gs1(V &x, V &y, double w) const {
+        asm volatile("" : "+v"(w));
+        const double d = x - y;
+        x = x + y;
+        y = fp_mulmod(d, FpTw{w, w * m.qinv}, m);
+    }
+    template <int ST>
+    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
+        ct1(v[0], v[2], t.w[0]);
+        ct1(v[1], v[3], t.w[0]);
+        if (ST == 2) {
+            ct1(v[0], v[1], t.w[1]);
+            ct1(v[2], v[3], t.w[2]);
+        }
+    }
+    template <int ST>
+    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
+        if (ST == 2) {
+            gs1(v[0], v[1], t.w[1]);
+            gs1(v[2], v[3], t.w[2]);
+        }
+        gs1(v[0], v[2], t.w[0]);
+        gs1(v[1], v[3], t.w[0]);
+    }
+    __device__ __forceinline__ void reduce(V *v) const {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = fp_reduce(v[j], m);
+    }
+};
+
+// A tile of 2^B words, 4 per thread, whose stages 0 .. LD-1 pair the tile bits B-1, B-2, ...; block k holds the stages
+// 2k and 2k+1.  In block k thread t has the words ((t >> low) << (low + 2)) | (j << low) | (t mod 2^low), low = B - 2k - 2,
+// and the twiddle index of its first stage is 2^(2k) + (t >> low).  Between the blocks k and k+1 words move inside groups
+// of 2^low threads: inside a wave from low = 6 on.
+template <int B, int LD>
+struct Tile4 {
+    static constexpr int kBlocks = (LD + 1) / 2;
+    static_assert(B >= 8 && 2 * kBlocks <= B, "four words of every block lie inside the tile");
+    static constexpr int stages(int k) { return LD - 2 * k >= 2 ? 2 : 1; }
+    static __device__ __forceinline__ uint32_t word(int k, uint32_t t, int j) {
+        const int low = B - 2 * k - 2;
+        return ((t >> low) << (low + 2)) | ((uint32_t)j << low) | (t & ((1u << low) - 1));
+    }
+    static __device__ __forceinline__ uint32_t index(int k, uint32_t t) { return (1u << (2 * k)) + (t >> (B - 2 * k - 2)); }
+
+    template <class A, int K>
+    static __device__ __forceinline__ void load_tw(typename A::Tw *tw, const A &ar, uint32_t scale, uint32_t t) {
+        // scale: the tile's number within the limb enters the index as its upper bits (blocks pass), 1 for a rows pass
+        tw[K] = ar.template load<stages(K), (B - 2 * K - 2 >= 6)>(((scale - 1) << (2 * K)) + index(K, t));
+        if constexpr (K + 1 < kBlocks) load_tw<A, K + 1>(tw, ar, scale, t);
+    }
+    template <int KLO>
+    static __device__ __forceinline__ void sync() {
+        if constexpr (B - 2 * KLO - 2 > 6)
+            lds_barrier();
+        else
+            wave_sync();
+    }
+    template <class A, int K = 0>
+    static __device__ __forceinline__ void forward(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
+        ar.template ct<stages(K)>(v, tw[K]);
+        if constexpr (K + 1 < kBlocks) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
+            sync<K>();
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K + 1, t, j))]);
+            if constexpr ((K + 1) % 2 == 0) ar.reduce(v);
+            forward<A, K + 1>(v, tw, ar, lds, t);
+        }
+    }
+    template <class A, int K = kBlocks - 1>
+    static __device__ __forceinline__ void inverse(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
+        ar.template gs<stages(K)>(v, tw[K]);
+        if constexpr (K > 0) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
+            sync<K - 1>();
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K - 1, t, j))]);
+            ar.reduce(v);
+            inverse<A, K - 1>(v, tw, ar, lds, t);
+        }
+    }
+};
+
+__device__ __forceinline__ IntArith int_arith(const NttArgs &a, uint32_t table) {
+    const IntCtx c = int_ctx(a, table);
+    return IntArith{int_mod(c.q), c.tw};
+}
+
+__device__ __forceinline__ FpArith fp_arith(const NttArgs &a, uint32_t table) {
+    const FpCtx c = fp_ctx(a, table);
+    return FpArith{c.m, c.tw};
+}
+
+
+// four consecutive words of a lane, as two 16-byte accesses (the polynomials are only 8-byte aligned for certain)
+typedef uint64_t Words2 __attribute__((ext_vector_type(2), aligned(8)));
+
+__device__ __forceinline__ void load4(uint64_t *v, const uint64_t *p) {
+    const Words2 a = reinterpret_cast<const Words2 *>(p)[0], b = reinterpret_cast<const Words2 *>(p)[1];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
+__device__ __forceinline__ void store4(uint64_t *p, const uint64_t *v) {
+    reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
+    reinterpret_cast<Words2 *>(p)[1] = Words2{v[2], v[3]};
 }
 
 }  // namespace

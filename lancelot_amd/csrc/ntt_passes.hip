@@ -21,181 +21,6 @@ namespace he {
 
 namespace {
 
-// Orders the LDS accesses of one wave's lanes: the hardware runs them in program order, so only the compiler is held.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
-// Two stages (ST = 1: only the first of them) on four words; tw entries: the first stage's twiddle, then the two of the
-// second.
-struct IntArith {
-    using V = uint64_t;
-    struct Tw {
-        Shoup s[3];
-    };
-    IntMod m;
-    const uint64_t *table;
-    static __device__ __forceinline__ V from_word(uint64_t x) { return x; }
-    static __device__ __forceinline__ uint64_t to_word(V v) { return v; }
-    template <int ST>
-    __device__ __forceinline__ Tw load(uint32_t idx) const {
-        Tw t;
-        t.s[0] = load_shoup(table, idx);
-        t.s[1] = t.s[2] = Shoup{0, 0};
-        if (ST == 2) {
-            t.s[1] = load_shoup(table, 2 * (size_t)idx);
-            t.s[2] = load_shoup(table, 2 * (size_t)idx + 1);
-        }
-        return t;
-    }
-    template <int ST>
-    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
-        ct_butterfly(v[0], v[2], t.s[0], m);
-        ct_butterfly(v[1], v[3], t.s[0], m);
-        if (ST == 2) {
-            ct_butterfly(v[0], v[1], t.s[1], m);
-            ct_butterfly(v[2], v[3], t.s[2], m);
-        }
-    }
-    template <int ST>
-    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
-        if (ST == 2) {
-            gs_butterfly(v[0], v[1], t.s[1], m);
-            gs_butterfly(v[2], v[3], t.s[2], m);
-        }
-        gs_butterfly(v[0], v[2], t.s[0], m);
-        gs_butterfly(v[1], v[3], t.s[0], m);
-    }
-    __device__ __forceinline__ void reduce(V *) const {}
-};
-
-// Bounds (in units of q, |v| < 8 keeps every value exact): forward, a stage takes b to 1.375 b + 0.5, so four stages
-// between reductions end at 5.3 (7.1 from canonical words); inverse, words are reduced before every two stages, whose
-// sums end at 2 (4 from canonical words) and whose products stay below that.
-struct FpArith {
-    using V = double;
-    struct Tw {
-        double w[3];
-    };
-    FpMod m;
-    const double *table;
-    static __device__ __forceinline__ V from_word(uint64_t x) { return __longlong_as_double((long long)x); }
-    static __device__ __forceinline__ uint64_t to_word(V v) { return (uint64_t)__double_as_longlong(v); }
-    template <int ST>
-    __device__ __forceinline__ Tw load(uint32_t idx) const {
-        Tw t;
-        t.w[0] = table[idx];
-        t.w[1] = t.w[2] = 0.0;
-        if (ST == 2) {
-            t.w[1] = table[2 * (size_t)idx];
-            t.w[2] = table[2 * (size_t)idx + 1];
-        }
-        return t;
-    }
-    __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
-        asm volatile("" : "+v"(w));   // keeps w * qinv out of the registers that a loop over limbs holds
-        const double t = fp_mulmod(y, FpTw{w, w * m.qinv}, m);
-        y = x - t;
-        x = x + t;
-    }
-    __device__ __forceinline__ void gs1(V &x, V &y, double w) const {
-        asm volatile("" : "+v"(w));
-        const double d = x - y;
-        x = x + y;
-        y = fp_mulmod(d, FpTw{w, w * m.qinv}, m);
-    }
-    template <int ST>
-    __device__ __forceinline__ void ct(V *v, const Tw &t) const {
-        ct1(v[0], v[2], t.w[0]);
-        ct1(v[1], v[3], t.w[0]);
-        if (ST == 2) {
-            ct1(v[0], v[1], t.w[1]);
-            ct1(v[2], v[3], t.w[2]);
-        }
-    }
-    template <int ST>
-    __device__ __forceinline__ void gs(V *v, const Tw &t) const {
-        if (ST == 2) {
-            gs1(v[0], v[1], t.w[1]);
-            gs1(v[2], v[3], t.w[2]);
-        }
-        gs1(v[0], v[2], t.w[0]);
-        gs1(v[1], v[3], t.w[0]);
-    }
-    __device__ __forceinline__ void reduce(V *v) const {
-#pragma unroll
-        for (int j = 0; j < 4; j++) v[j] = fp_reduce(v[j], m);
-    }
-};
-
-// A tile of 2^B words, 4 per thread, whose stages 0 .. LD-1 pair the tile bits B-1, B-2, ...; block k holds the stages
-// 2k and 2k+1.  In block k thread t has the words ((t >> low) << (low + 2)) | (j << low) | (t mod 2^low), low = B - 2k - 2,
-// and the twiddle index of its first stage is 2^(2k) + (t >> low).  Between the blocks k and k+1 words move inside groups
-// of 2^low threads: inside a wave from low = 6 on.
-template <int B, int LD>
-struct Tile4 {
-    static constexpr int kBlocks = (LD + 1) / 2;
-    static_assert(B >= 8 && 2 * kBlocks <= B, "four words of every block lie inside the tile");
-    static constexpr int stages(int k) { return LD - 2 * k >= 2 ? 2 : 1; }
-    static __device__ __forceinline__ uint32_t word(int k, uint32_t t, int j) {
-        const int low = B - 2 * k - 2;
-        return ((t >> low) << (low + 2)) | ((uint32_t)j << low) | (t & ((1u << low) - 1));
-    }
-    static __device__ __forceinline__ uint32_t index(int k, uint32_t t) { return (1u << (2 * k)) + (t >> (B - 2 * k - 2)); }
-
-    template <class A, int K>
-    static __device__ __forceinline__ void load_tw(typename A::Tw *tw, const A &ar, uint32_t scale, uint32_t t) {
-        // scale: the tile's number within the limb enters the index as its upper bits (blocks pass), 1 for a rows pass
-        tw[K] = ar.template load<stages(K)>(((scale - 1) << (2 * K)) + index(K, t));
-        if constexpr (K + 1 < kBlocks) load_tw<A, K + 1>(tw, ar, scale, t);
-    }
-    template <int KLO>
-    static __device__ __forceinline__ void sync() {
-        if constexpr (B - 2 * KLO - 2 > 6)
-            lds_barrier();
-        else
-            wave_sync();
-    }
-    template <class A, int K = 0>
-    static __device__ __forceinline__ void forward(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
-        ar.template ct<stages(K)>(v, tw[K]);
-        if constexpr (K + 1 < kBlocks) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
-            sync<K>();
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K + 1, t, j))]);
-            if constexpr ((K + 1) % 2 == 0) ar.reduce(v);
-            forward<A, K + 1>(v, tw, ar, lds, t);
-        }
-    }
-    template <class A, int K = kBlocks - 1>
-    static __device__ __forceinline__ void inverse(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
-        ar.template gs<stages(K)>(v, tw[K]);
-        if constexpr (K > 0) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
-            sync<K - 1>();
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K - 1, t, j))]);
-            ar.reduce(v);
-            inverse<A, K - 1>(v, tw, ar, lds, t);
-        }
-    }
-};
-
-__device__ __forceinline__ IntArith int_arith(const NttArgs &a, uint32_t table) {
-    const IntCtx c = int_ctx(a, table);
-    return IntArith{int_mod(c.q), c.tw};
-}
-
-__device__ __forceinline__ FpArith fp_arith(const NttArgs &a, uint32_t table) {
-    const FpCtx c = fp_ctx(a, table);
-    return FpArith{c.m, c.tw};
-}
-
-
 // Rows pass.  The thread index is (wave, lane), the wave the same scalar in all its lanes, so that the twiddles of the
 // first two blocks come through scalar loads.
 // SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first; it leaves the
@@ -308,22 +133,6 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
             }
         }
     }
-}
-
-// four consecutive words of a lane, as two 16-byte accesses (the polynomials are only 8-byte aligned for certain)
-typedef uint64_t Words2 __attribute__((ext_vector_type(2), aligned(8)));
-
-__device__ __forceinline__ void load4(uint64_t *v, const uint64_t *p) {
-    const Words2 a = reinterpret_cast<const Words2 *>(p)[0], b = reinterpret_cast<const Words2 *>(p)[1];
-    v[0] = a.x;
-    v[1] = a.y;
-    v[2] = b.x;
-    v[3] = b.y;
-}
-
-__device__ __forceinline__ void store4(uint64_t *p, const uint64_t *v) {
-    reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
-    reinterpret_cast<Words2 *>(p)[1] = Words2{v[2], v[3]};
 }
 
 constexpr int kBlockWaves = 2;   // 256-word blocks of a workgroup, one per wave
@@ -701,6 +510,97 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
     }
 }
 
+// (d0, d1, d2) = (a0 b0, a0 b1 + a1 b0, a1 b1) mod q, canonical, of four words each
+__device__ __forceinline__ void tensor4(const FpArith &ar, const NttArgs &, uint32_t, const uint64_t *a0, const uint64_t *a1,
+                                        const uint64_t *b0, const uint64_t *b1, double *d0, double *d1, double *d2) {
+    const FpMod m = ar.m;
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const double x0 = fp_from_u64(a0[j]), x1 = fp_from_u64(a1[j]), y0 = fp_from_u64(b0[j]), y1 = fp_from_u64(b1[j]);
+        d0[j] = fp_canonical(fp_mulmod(x0, FpTw{y0, y0 * m.qinv}, m), m);
+        d2[j] = fp_canonical(fp_mulmod(x1, FpTw{y1, y1 * m.qinv}, m), m);
+        // Karatsuba: both factors are below 2 q, the product is reduced to |r| <= 2 q, the difference stays below 4 q
+        const double sy = y0 + y1, mm = fp_mulmod(x0 + x1, FpTw{sy, sy * m.qinv}, m);
+        d1[j] = fp_canonical(mm - d0[j] - d2[j], m);
+    }
+}
+
+__device__ __forceinline__ void tensor4(const IntArith &ar, const NttArgs &a, uint32_t table, const uint64_t *a0, const uint64_t *a1,
+                                        const uint64_t *b0, const uint64_t *b1, uint64_t *d0, uint64_t *d1, uint64_t *d2) {
+    const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        d0[j] = mul_mod(a0[j], b0[j], q, r0, r1);
+        d2[j] = mul_mod(a1[j], b1[j], q, r0, r1);
+        // Karatsuba; the sums stay below 2^62
+        d1[j] = sub_mod(sub_mod(mul_mod(a0[j] + a1[j], b0[j] + b1[j], q, r0, r1), d0[j], q), d2[j], q);
+    }
+}
+
+// Tensor product fused with the blocks pass of the inverse transform of its third polynomial: a wave forms the three products
+// of one block of 256 words, stores them (d2 in NTT form is what the key switch multiplies by its own digit's key) and takes d2
+// through the 8 inverse stages; the lazy words are left in a.out for the rows pass.  One read of d2 and one launch less
+// than tensor kernel + inverse transform.
+template <class A>
+__device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse &x, const Job &job, const A &ar, uint32_t blk,
+                                             uint32_t lane, uint64_t *lds) {
+    using T4 = Tile4<8, 8>;
+    constexpr bool FP = std::is_same<A, FpArith>::value;
+    const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const size_t ct = 2 * job.poly * poly + job.limb * n + at;
+    uint64_t a0[4], a1[4], b0[4], b1[4];
+    load4(a0, x.ct1 + ct);
+    load4(a1, x.ct1 + ct + poly);
+    if (!x.square) {
+        load4(b0, x.ct2 + ct);
+        load4(b1, x.ct2 + ct + poly);
+    }
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    if (x.square) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            b0[j] = a0[j];
+            b1[j] = a1[j];
+        }
+    }
+    typename A::V d0[4], d1[4], d2[4];
+    tensor4(ar, a, job.table, a0, a1, b0, b1, d0, d1, d2);
+    uint64_t o0[4], o1[4], o2[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        if constexpr (FP) {
+            o0[j] = fp_to_u64(d0[j]);
+            o1[j] = fp_to_u64(d1[j]);
+            o2[j] = fp_to_u64(d2[j]);
+        } else {
+            o0[j] = d0[j];
+            o1[j] = d1[j];
+            o2[j] = d2[j];
+        }
+    }
+    store4(x.d01 + ct, o0);
+    store4(x.d01 + ct + poly, o1);
+    store4(x.d2 + job.poly * poly + job.limb * n + at, o2);
+    T4::template inverse<A>(d2, tw, ar, lds, lane);
+#pragma unroll
+    for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(d2[j]);
+}
+
+template <int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(NttArgs a, TensorFuse x) {
+    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const Job job = decode_job(a, id >> lr);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane, lds_all[w]);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) tensor_block(a, x, job, int_arith(a, job.table), blk, lane, lds_all[w]);
+    }
+}
+
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
@@ -819,6 +719,20 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
         hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
     else
         hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
+    return hipGetLastError();
+}
+
+hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0 || items == 0) return hipErrorInvalidValue;
+    const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
+    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    if (backend == NTT_BACKEND_MIXED)
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
+    else if (backend)
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
+    else
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
     return hipGetLastError();
 }
 
