@@ -1004,8 +1004,9 @@ int he_ks_inner_product(const he_context *ctx, uint32_t L, const uint64_t *y, co
 namespace {
 
 // add_mask: which polynomials of `out` are added onto (bit p set) instead of overwritten
+// inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
-                 uint64_t *ws, he_stream s) {
+                 uint64_t *ws, he_stream s, bool inverted = false) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     const int accumulate = add_mask != 0;
     const size_t n = ctx->n();
@@ -1026,9 +1027,9 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     // limb's coefficients modulo each q_j, done where the forward transform reads its input
     const bool reduce_in_ntt = ctx->single_limb_digits && !fused;
     // ... and a small launch finishes the special limb's inverse transform there as well
-    const int inv_backend = backend_for(ctx, inv.map);
+    const int inv_backend = inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, n_polys * L);
-    HE_HIP(launch_ntt_inverse(inv, n_polys, inv_backend, S(s), false, source_intt));
+    HE_HIP(launch_ntt_inverse(inv, n_polys, inv_backend, S(s), inverted, source_intt));
     if (reduce_in_ntt) {
     } else if (batched) {
         const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
@@ -1117,9 +1118,11 @@ KsWorkspace ks_workspace(const he_context *ctx, const Level *lv, uint32_t L, uin
 // fold_ct != nullptr: limb L-1 of cx becomes cx * P^-1 + fold_ct (see KsFuseArgs); fold_ct holds [items][2][L][N].
 // add_c0 != nullptr (a rotation, items = 1): polynomial 0 of cx gains P sigma(add_c0) on its data limbs, sigma =
 // X -> X^galois_elt, so that the ModDown of cx yields sigma(add_c0) + KeySwitch(sigma(c)) with no pass for sigma.
+// *inverted: the limbs of cx that ModDown transforms back (the special ones, and limb L-1 with fold_ct) have been through
+// their inverse blocks pass, on the level's back end.
 int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint64_t *c, uint32_t c_item_stride,
                   uint32_t items, const uint64_t *const *evk, uint32_t galois_elt, const uint64_t *fold_ct, uint64_t *ws,
-                  he_stream s, const uint64_t *add_c0 = nullptr, const TensorFuse *tin = nullptr) {
+                  he_stream s, bool *inverted, const uint64_t *add_c0 = nullptr, const TensorFuse *tin = nullptr) {
     if (items == 0 || (items > 1 && (galois_elt || add_c0))) return HE_E_INVALID_ARGUMENT;
     if (galois_elt && (!(galois_elt & 1) || galois_elt >= (2u << ctx->log_n))) return HE_E_INVALID_ARGUMENT;
     const uint64_t *fold_w = fold_ct ? ctx->d_pinv_mod_q + 2 * (size_t)(L - 1) : nullptr;
@@ -1128,6 +1131,7 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
     uint64_t *y = w.y, *cx = w.cx, *tmp = w.tmp;
     const uint64_t *src = c;
     const bool fused_inner = ctx->fuse_inner && (items == 1 || ctx->batch_fused_inner);
+    *inverted = fused_inner;
     // the separate kernels: levels whose inner product reads a digit's own limbs from the input gather sigma(c) where they
     // read c (the inverse blocks pass and the inner product); the others stage it
     const bool gather = galois_elt && !fused_inner && lv->batched && items == 1;
@@ -1147,6 +1151,8 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         NttArgs fwd = base_args(ctx, true);
         fwd.out = y;
         fwd.item_stride = (size_t)lv->beta * (L + ctx->size_p) * n;
+        fwd.pro_itw = ctx->d_ipsi;
+        fwd.pro_itw_fp = ctx->d_ipsi_fp;
         KsFuseArgs x;
         memset(&x, 0, sizeof(x));
         for (uint32_t d = 0; d < lv->beta; d++) x.evk.p[d] = evk[d];
@@ -1162,6 +1168,7 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         x.beta = lv->beta;
         x.fold_ct = fold_ct;
         x.fold_w = fold_w;
+        x.inv_first = fold_ct ? L - 1 : L;
         x.items = items;
         x.own_item_stride = (size_t)c_item_stride * n;
         x.fold_item_stride = 2 * (size_t)L * n;
@@ -1208,8 +1215,9 @@ int he_keyswitch(const he_context *ctx, uint32_t L, const uint64_t *c, const uin
     const Level *lv = level_of(ctx, L);
     if (!lv) return HE_E_LEVEL_NOT_SET;
     const KsWorkspace w = ks_workspace(ctx, lv, L, 1, ws);
-    if (int rc = ks_accumulate(ctx, lv, L, c, L, 1, evk, galois_elt, nullptr, ws, s)) return rc;
-    return he_moddown(ctx, L, w.cx, ct, 2, 1, w.tmp, s);
+    bool inverted = false;
+    if (int rc = ks_accumulate(ctx, lv, L, c, L, 1, evk, galois_elt, nullptr, ws, s, &inverted)) return rc;
+    return moddown_impl(ctx, L, w.cx, ct, 2, 0xffffffffu, w.tmp, s, inverted);
 }
 
 int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const uint64_t *const *evk, uint64_t *ct_out,
@@ -1222,9 +1230,10 @@ int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const ui
     if (!(galois_elt & 1) || galois_elt >= (2u << ctx->log_n)) return HE_E_INVALID_ARGUMENT;
     // the automorphism is never a pass of its own: sigma(c1) is gathered where the key switch reads its input,
     // sigma(c0) where the inner product adds P sigma(c0) to its first polynomial
-    if (int rc = ks_accumulate(ctx, lv, L, ct_in + (size_t)L * n, L, 1, evk, galois_elt, nullptr, ws, s, ct_in)) return rc;
+    bool inverted = false;
+    if (int rc = ks_accumulate(ctx, lv, L, ct_in + (size_t)L * n, L, 1, evk, galois_elt, nullptr, ws, s, &inverted, ct_in)) return rc;
     // out0 = sigma(c0) + ks0 (the inner product carries P sigma(c0)), out1 = ks1
-    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s);
+    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s, inverted);
 }
 
 int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *ct_in,
@@ -1291,7 +1300,8 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     // so ModDown and rescale share one inverse and one forward transform.  Every step is exact modular arithmetic:
     // the limbs equal he_keyswitch followed by he_rescale.
     // (1) inner product; limb L-1 of cx leaves as cx_{L-1} P^-1 + ct_{L-1}
-    if (int rc = ks_accumulate(ctx, lv, L, c, c_item_stride, items, evk, galois_elt, ct, ws, s, nullptr, tin)) return rc;
+    bool inverted = false;
+    if (int rc = ks_accumulate(ctx, lv, L, c, c_item_stride, items, evk, galois_elt, ct, ws, s, &inverted, nullptr, tin)) return rc;
     // (2) limb L-1 and the special limbs -> coefficient form, the latter scaled by (P / p_k)^-1
     NttArgs inv = base_args(ctx, false);
     inv.in = cx + (size_t)(L - 1) * n;
@@ -1300,7 +1310,7 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     inv.map = LimbMap{K + 1, L - 1, 1, ctx->size_q};
     inv.epi_mode = NTT_EPI_MUL;
     inv.w = lv->d_mdr_w;
-    HE_HIP(launch_ntt_inverse(inv, polys, backend_for(ctx, inv.map), S(s)));
+    HE_HIP(launch_ntt_inverse(inv, polys, inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map), S(s), inverted));
     // (3) delta = P -> Ql conversion of the special limbs
     const bool fused = fuse_rows_ok(ctx, lv, L);
     // one special prime: the conversion is the reduction of its coefficients modulo every q_j, which the prologue of (4)

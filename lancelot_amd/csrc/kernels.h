@@ -328,6 +328,9 @@ struct KsFuseArgs {
     // transforms back to coefficients); fold_ct = nullptr leaves the inner product as it is
     const uint64_t *fold_ct;  // [2][L][N]
     const uint64_t *fold_w;   // Shoup pair of P^-1 mod q_{L-1}
+    // limbs t >= inv_first leave as the lazy words of their inverse blocks pass (what ModDown transforms back; the launch's
+    // NttArgs::pro_itw / pro_itw_fp hold the inverse tables); L + K: none
+    uint32_t inv_first;
     // items > 1: that many inputs in one launch (no Galois element, no add_c0); item i's own limbs, output and fold_ct
     // lie i * own_item_stride, i * 2 (L+K) N and i * fold_item_stride words further on, its lazy digits
     // i * NttArgs::item_stride.  The workgroups of one (limb, tile) for all items are placed on one XCD next to each

@@ -350,7 +350,10 @@ struct IntSums {
 
 // Blocks pass of ModUp's forward transform fused with the key-switch inner product: a wave owns one block of 256 words of limb t of
 // Ql u P, takes it through the last 8 stages for every digit in turn and multiplies it by both key polynomials; the digit
-// that owns limb t contributes the input itself.  The transformed limbs never reach memory.
+// that owns limb t contributes the input itself.  The transformed limbs never reach memory, and the limbs of the sum that
+// ModDown needs in coefficient form leave through the inverse blocks pass (a launch and two trips of those limbs less: one
+// product at L = 24, K = 8 157 -> 153 us, n = 2^14, 4 + 1 limbs 38 -> 34 us, although the second set of twiddles takes the
+// FP64 kernel from 96 registers to 120).
 template <class A>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &x, uint32_t t, uint32_t table, uint32_t blk,
                                             uint32_t item, uint32_t lane, const A &ar, uint64_t *lds) {
@@ -412,30 +415,34 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         sums.add(v, k, ar);
         wave_sync();   // (the next digit's exchanges reuse the LDS words that this one's lanes have read)
     }
-    uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)t * n + at;
     const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
     const bool fold = x.fold_ct && t == x.L - 1;
-    uint64_t c0[4], cl[2][4];
-    if (add) {
-        const uint64_t *src = x.add_c0 + (size_t)t * n;
-        if (x.own_galois) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
-        } else {
-            load4(c0, src + at);
-        }
-    }
-    if (fold) {
-        const uint64_t *src = x.fold_ct + item * x.fold_item_stride + (size_t)t * n + at;
-        load4(cl[0], src);
-        load4(cl[1], src + (size_t)x.L * n);
+    // (the words of a limb that ModDown transforms back go through the inverse blocks pass before they leave the wave)
+    const bool invert = t >= x.inv_first;
+    A iar = ar;
+    if (invert) {
+        if constexpr (FP)
+            iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
+        else
+            iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
+        T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
     }
 #pragma unroll
     for (int r = 0; r < 2; r++) {
-        uint64_t res[4];
+        typename A::V v[4];
+        uint64_t c0[4], cl[4];
+        if (add && r == 0) {
+            const uint64_t *src = x.add_c0 + (size_t)t * n;
+            if (x.own_galois) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+            } else {
+                load4(c0, src + at);
+            }
+        }
+        if (fold) load4(cl, x.fold_ct + item * x.fold_item_stride + ((size_t)r * x.L + t) * n + at);
         if constexpr (FP) {
             const FpMod m = ar.m;
-            double v[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = sums.s[r][j];
             if (add && r == 0) {
@@ -446,35 +453,48 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
             if (fold) {
                 const double wd = fp_from_u64(x.fold_w[0]);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], FpTw{wd, wd * m.qinv}, m) + fp_from_u64(cl[r][j]);
+                for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], FpTw{wd, wd * m.qinv}, m) + fp_from_u64(cl[j]);
             }
 #pragma unroll
-            for (int j = 0; j < 4; j++) res[j] = fp_to_u64(fp_canonical(v[j], m));
+            for (int j = 0; j < 4; j++) v[j] = fp_canonical(v[j], m);
         } else {
             const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
 #pragma unroll
-            for (int j = 0; j < 4; j++) res[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
+            for (int j = 0; j < 4; j++) v[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
             if (add && r == 0) {
                 const Shoup w = load_shoup(x.p_mod_q, t);
 #pragma unroll
-                for (int j = 0; j < 4; j++) res[j] = add_mod(res[j], mul_shoup(c0[j], w, q), q);
+                for (int j = 0; j < 4; j++) v[j] = add_mod(v[j], mul_shoup(c0[j], w, q), q);
             }
             if (fold) {
                 const Shoup w = load_shoup(x.fold_w, 0);
 #pragma unroll
-                for (int j = 0; j < 4; j++) res[j] = add_mod(mul_shoup(res[j], w, q), cl[r][j], q);
+                for (int j = 0; j < 4; j++) v[j] = add_mod(mul_shoup(v[j], w, q), cl[j], q);
             }
         }
-        store4(o + (size_t)r * LK * n, res);
+        uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)r * LK * n + (size_t)t * n;
+        if (invert) {
+            T4::template inverse<A>(v, tw, iar, lds, lane);
+#pragma unroll
+            for (int j = 0; j < 4; j++) o[off + T4::word(0, lane, j)] = A::to_word(v[j]);
+            wave_sync();
+        } else {
+            uint64_t res[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (FP)
+                    res[j] = fp_to_u64(v[j]);
+                else
+                    res[j] = v[j];
+            }
+            store4(o + at, res);
+        }
     }
 }
 
 // Waves of a workgroup: of one item, neighbouring blocks; of a batch, the same block of neighbouring items, which find the
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
-#ifndef INNER_WAVES
-#define INNER_WAVES 4
-#endif
-constexpr int kInnerWaves = INNER_WAVES;
+constexpr int kInnerWaves = 4;
 
 template <int BE>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
