@@ -334,6 +334,15 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
                          double scale, uint32_t limbs, uint32_t items, size_t value_stride, uint64_t *out,
                          uint32_t out_poly_stride, uint64_t *workspace, he_stream stream);
 
+/* he_ckks_encode_batch for a caller that knows that no coefficient reaches 2^62 (none exceeds scale / slots times the sum of
+ * the values' magnitudes): no maximum is formed, so there is nothing to wait for, and the rounding happens where the
+ * transform reads its input.  The same plaintexts.  re and im may also be page-locked host memory (he_host_malloc), which
+ * the caller leaves alone until the stream has passed the call.  workspace as for he_ckks_encode_batch.  No counterpart in the
+ * reference. */
+int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t slots,
+                           double scale, uint32_t limbs, uint32_t items, size_t value_stride, uint64_t *out,
+                           uint32_t out_poly_stride, uint64_t *workspace, he_stream stream);
+
 /* Public-key encryption of `items` plaintexts with one launch per stage: cts [items][2][L][N] holds plaintext k in
  * polynomial 0 of ciphertext k on entry and ciphertext k on return: (u pk_0 + e_0, u pk_1 + e_1) over Ql u P, divided
  * by P, plus the plaintext.  pk: [2][size_q + size_p][N] at the key level.  Item k draws u, e_0, e_1 from the
@@ -343,6 +352,33 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
 size_t he_encrypt_batch_workspace_words(const he_context *ctx, uint32_t L, uint32_t items);
 int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
                      uint64_t stream_id, uint64_t *cts, uint64_t *workspace, he_stream stream);
+
+/* One encryption of plain [L][N] (NTT form) into ct [2][L][N]: he_encrypt_batch of one item without the copy of the plaintext.
+ * workspace: he_encrypt_batch_workspace_words(ctx, L, 1) words. */
+int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],
+               uint64_t stream_id, uint64_t *ct, uint64_t *workspace, he_stream stream);
+
+/* plain [limbs][N] = c0 + c1 s (+ c2 s^2) + e for ct [size][limbs][N] of 2 or 3 polynomials, e the discrete Gaussian that
+ * he_sample (kind 3) draws from the same stream: the noise's samples stay bytes, and the sums are formed by its transform's last
+ * pass.  sk: s in NTT form, s^2 sk_stride words behind it.  cdt: DEVICE, at most 127 entries (HE_E_UNSUPPORTED beyond).
+ * workspace: N / 8 words.  Replaces ckks_decrypt (src/secretkey.cu:594-654). */
+int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t size, uint32_t limbs, const uint64_t *sk, size_t sk_stride,
+                     const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain,
+                     uint64_t *workspace, he_stream stream);
+
+/* he_ckks_decode for the real parts of the first `count` values: out [count], DEVICE or page-locked host memory (written by the
+ * last kernel; the caller synchronises the stream before it reads).  The same values. */
+size_t he_ckks_decode_real_workspace_words(const he_context *ctx, uint32_t limbs, uint32_t slots);
+int he_ckks_decode_real(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t slots, double scale, double *out,
+                        uint32_t count, uint64_t *workspace, he_stream stream);
+
+/* he_decrypt_decode_batch with the flooding noise drawn inside (key = NULL: none; item k from stream_id + k, as `items` calls of
+ * he_decrypt_flood) and real parts only: out [items][count], DEVICE or page-locked host memory. */
+size_t he_decrypt_decode_real_workspace_words(const he_context *ctx, uint32_t limbs, uint32_t slots, uint32_t items);
+int he_decrypt_decode_real_batch(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs,
+                                 const uint64_t *sk, const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt,
+                                 uint32_t cdt_len, uint32_t slots, double scale, uint32_t count, double *out,
+                                 uint64_t *workspace, he_stream stream);
 
 /* Decryption and decoding of `items` size-2 ciphertexts in one launch per stage: for the ciphertexts [2][limbs][N]
  * named by the DEVICE pointer table d_cts, m = c0 + c1 s (+ noise [items][limbs][N] in NTT form, or NULL), inverse

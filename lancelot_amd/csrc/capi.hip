@@ -1004,9 +1004,10 @@ int he_ks_inner_product(const he_context *ctx, uint32_t L, const uint64_t *y, co
 namespace {
 
 // add_mask: which polynomials of `out` are added onto (bit p set) instead of overwritten
+// (addend: where the words to add come from, limb stride addend_stride between polynomials; nullptr: out itself)
 // inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
-                 uint64_t *ws, he_stream s, bool inverted = false) {
+                 uint64_t *ws, he_stream s, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     const int accumulate = add_mask != 0;
     const size_t n = ctx->n();
@@ -1056,8 +1057,8 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     fwd.epi_mode = accumulate ? NTT_EPI_SUB_MUL_ADD : NTT_EPI_SUB_MUL;
     fwd.epi_a = cx;
     fwd.epi_a_poly_stride = LK;
-    fwd.epi_b = out;
-    fwd.epi_b_poly_stride = L;
+    fwd.epi_b = addend ? addend : out;
+    fwd.epi_b_poly_stride = addend ? addend_stride : L;
     fwd.epi_b_mask = add_mask;
     fwd.w = ctx->d_pinv_mod_q;
     fwd.epi_dst = out;
@@ -1471,6 +1472,31 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     return he_ntt_forward(ctx, out, items, out_poly_stride, limbs, 0, limbs, 0, s);
 }
 
+int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t slots,
+                           double scale, uint32_t limbs, uint32_t items, size_t value_stride, uint64_t *out,
+                           uint32_t out_poly_stride, uint64_t *ws, he_stream s) {
+    if (!ctx || !re || !out || !ws || limbs == 0 || limbs > ctx->size_qp || items == 0 || items > 16384 ||
+        out_poly_stride < limbs)
+        return HE_E_INVALID_ARGUMENT;
+    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || count > slots || !(scale > 0) ||
+        (items > 1 && value_stride < count))
+        return HE_E_INVALID_ARGUMENT;
+    double2 *v = reinterpret_cast<double2 *>(ws + (((size_t)items + 7) & ~(size_t)7));
+    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    HE_HIP(launch_ckks_fft_inverse(ft, re, im, count, slots, v, items, value_stride, S(s)));
+    // rounding and residues happen where the transform reads its input
+    NttArgs a = base_args(ctx, true);
+    a.out = out;
+    a.out_poly_stride = out_poly_stride;
+    a.map = plain_map(limbs);
+    a.pro_mode = NTT_PRO_ROUND;
+    a.pro_src = reinterpret_cast<const uint64_t *>(v);
+    a.pro_fix = scale / (double)slots;
+    a.pro_log_slots = 31 - __builtin_clz(slots);
+    HE_HIP(launch_ntt_forward(a, items, backend_for(ctx, a.map), S(s)));
+    return HE_OK;
+}
+
 int he_ckks_encode(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t slots,
                    double scale, uint32_t limbs, uint64_t *out, uint64_t *ws, he_stream s) {
     // one item: the maximum in ws[0], then the scratch (the layout of he_ckks_workspace_words)
@@ -1484,33 +1510,148 @@ size_t he_encrypt_batch_workspace_words(const he_context *ctx, uint32_t L, uint3
     return (size_t)items * (3 * LK + 2 * L) * n;
 }
 
-int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
-                     uint64_t stream_id, uint64_t *cts, uint64_t *ws, he_stream s) {
+}  // extern "C"
+
+namespace {
+
+// plain: [items] plaintexts plain_stride limbs apart; nullptr: they lie in polynomial 0 of the ciphertexts
+int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],
+                 uint64_t stream_id, uint64_t *cts, uint64_t *ws, he_stream s) {
     if (!ctx || !pk || !key || !cts || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q || items == 0 || items > 8192)
         return HE_E_INVALID_ARGUMENT;
     const size_t n = ctx->n();
     const uint32_t K = ctx->size_p, Q = ctx->size_q, LK = L + K;
+    // u and wide lie one after the other: 3 * items polynomials of the same limbs
     uint64_t *u = ws, *wide = u + (size_t)items * LK * n, *tmp = wide + (size_t)items * 2 * LK * n;
     ChaChaKey k;
     memcpy(k.k, key, sizeof(k.k));
-    const LimbMap map{LK, 0, L, Q};
-    // item k draws u, e0, e1 from the stream ids stream_id + 3 k, + 1, + 2: what `items` encryptions in a row draw
-    // (one launch: u and wide lie one after the other, 3 * items polynomials LK * N words apart)
-    HE_HIP(launch_sample_encrypt(ctx->tables(), k, stream_id, u, map, items, (size_t)LK * n, S(s)));
-    // u and wide lie one after the other: 3 * items polynomials of the same limbs
-    if (int rc = he_ntt_forward(ctx, u, 3 * items, LK, LK, 0, L, Q, s)) return rc;
-    HE_HIP(launch_encrypt_fma(ctx->tables(), u, pk, wide, L, K, Q, items, S(s)));
-    // divide by P; polynomial 0 of every ciphertext already holds the plaintext and is added onto
-    return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s);
+    // item k draws u, e0, e1 from the stream ids stream_id + 3 k, + 1, + 2: what `items` encryptions in a row draw.  The
+    // samples stay bytes (in ModDown's scratch, which is written later) until the transform reads them.
+    int8_t *small = reinterpret_cast<int8_t *>(tmp);
+    HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, small, items, S(s)));
+    const int backend = backend_for_level(ctx, L);
+    NttArgs a = base_args(ctx, true);
+    a.out = u;
+    a.out_poly_stride = LK;
+    a.map = LimbMap{LK, 0, L, Q};
+    a.pro_mode = NTT_PRO_SMALL;
+    a.pro_src = tmp;
+    a.pro_itw = ctx->d_ipsi;
+    a.pro_itw_fp = ctx->d_ipsi_fp;
+    HE_HIP(launch_ntt_rows(a, 3 * items * LK, true, backend, S(s)));
+    HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
+    // divide by P onto the plaintexts
+    return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s, true, plain, plain ? L : 0);
+}
+
+// the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
+int decode_real_impl(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t items, uint32_t slots, double scale,
+                     uint64_t *coeff, double2 *v, double *out, uint32_t count, he_stream s) {
+    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    NttArgs inv = base_args(ctx, false);
+    inv.in = plain;
+    inv.out = coeff;
+    inv.in_poly_stride = inv.out_poly_stride = limbs;
+    inv.map = plain_map(limbs);
+    const int backend = backend_for(ctx, inv.map);
+    if (limbs <= 4 && ctx->log_n >= 12 && ctx->log_n <= 16 && ctx->size_qp <= 64) {
+        HE_HIP(launch_ntt_blocks(inv, items, false, backend, S(s)));
+        inv.in = coeff;
+        HE_HIP(launch_ckks_decode_real(ft, inv, backend, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, out, count, S(s)));
+        return HE_OK;
+    }
+    HE_HIP(launch_ntt_inverse(inv, items, backend, S(s)));
+    HE_HIP(launch_ckks_compose(ft, ctx->tables(), coeff, limbs, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, S(s)));
+    HE_HIP(launch_ckks_fft_real(ft, slots, v, items, out, count, S(s)));
+    return HE_OK;
+}
+
+// plain [items][limbs][N] = c0 + c1 s [+ c2 s^2] + flooding noise from the streams stream_id + item; noise: items * N bytes
+int decrypt_flood_impl(const he_context *ctx, const DecryptArgs &d, uint32_t limbs, uint32_t items, const uint32_t key[8], uint64_t stream_id,
+                       const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain, uint64_t *noise, he_stream s) {
+    ChaChaKey k;
+    memcpy(k.k, key, sizeof(k.k));
+    HE_HIP(launch_sample_gauss_small(ctx->log_n, k, stream_id, reinterpret_cast<int8_t *>(noise), cdt, cdt_len, items, S(s)));
+    NttArgs a = base_args(ctx, true);
+    a.out = plain;
+    a.out_poly_stride = limbs;
+    a.map = plain_map(limbs);
+    a.pro_mode = NTT_PRO_SMALL;
+    a.pro_src = noise;
+    const int backend = backend_for(ctx, a.map);
+    HE_HIP(launch_ntt_rows(a, items * limbs, true, backend, S(s)));
+    HE_HIP(launch_decrypt_blocks(a, d, items, backend, S(s)));
+    return HE_OK;
+}
+
+}  // namespace
+
+extern "C" {
+
+int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
+                     uint64_t stream_id, uint64_t *cts, uint64_t *ws, he_stream s) {
+    return encrypt_impl(ctx, L, items, nullptr, pk, key, stream_id, cts, ws, s);
+}
+
+int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],
+               uint64_t stream_id, uint64_t *ct, uint64_t *ws, he_stream s) {
+    if (!plain) return HE_E_INVALID_ARGUMENT;
+    return encrypt_impl(ctx, L, 1, plain, pk, key, stream_id, ct, ws, s);
+}
+
+int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t size, uint32_t limbs, const uint64_t *sk, size_t sk_stride,
+                     const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain,
+                     uint64_t *ws, he_stream s) {
+    if (!ctx || !ct || !sk || !key || !cdt || !plain || !ws || limbs == 0 || limbs > ctx->size_q || size < 2) return HE_E_INVALID_ARGUMENT;
+    if (size > 3 || cdt_len == 0 || cdt_len >= 128) return HE_E_UNSUPPORTED;
+    return decrypt_flood_impl(ctx, DecryptArgs{ct, nullptr, sk, sk_stride, size}, limbs, 1, key, stream_id, cdt, cdt_len, plain, ws, s);
+}
+
+size_t he_ckks_decode_real_workspace_words(const he_context *ctx, uint32_t limbs, uint32_t slots) {
+    // [limbs][N] words of the inverse transform | slots complex values
+    return ctx ? (size_t)limbs * ctx->n() + 2 * (size_t)slots : 0;
+}
+
+int he_ckks_decode_real(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t slots, double scale, double *out,
+                        uint32_t count, uint64_t *ws, he_stream s) {
+    if (!ctx || !plain || !out || !ws || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
+    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0) || count == 0 || count > slots) return HE_E_INVALID_ARGUMENT;
+    return decode_real_impl(ctx, plain, limbs, 1, slots, scale, ws, reinterpret_cast<double2 *>(ws + (size_t)limbs * ctx->n()), out, count, s);
+}
+
+size_t he_decrypt_decode_real_workspace_words(const he_context *ctx, uint32_t limbs, uint32_t slots, uint32_t items) {
+    // [items][limbs][N] plaintexts | [items][slots] complex values | noise, a byte a coefficient
+    return ctx ? (size_t)items * (limbs * ctx->n() + 2 * (size_t)slots + ctx->n() / 8) : 0;
+}
+
+int he_decrypt_decode_real_batch(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs, const uint64_t *sk,
+                                 const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t slots,
+                                 double scale, uint32_t count, double *out, uint64_t *ws, he_stream s) {
+    if (!ctx || !d_cts || !sk || !out || !ws || items == 0 || items > 16384 || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
+    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0) || count == 0 || count > slots || (key && !cdt))
+        return HE_E_INVALID_ARGUMENT;
+    if (key && (cdt_len == 0 || cdt_len >= 128)) return HE_E_UNSUPPORTED;
+    const size_t n = ctx->n();
+    uint64_t *plain = ws, *v = ws + (size_t)items * limbs * n, *noise = v + 2 * (size_t)items * slots;
+    if (key) {
+        if (int rc = decrypt_flood_impl(ctx, DecryptArgs{nullptr, d_cts, sk, 0, 2}, limbs, items, key, stream_id, cdt, cdt_len, plain, noise, s))
+            return rc;
+    } else {
+        HE_HIP(launch_decrypt_gather(ctx->tables(), d_cts, sk, nullptr, plain, limbs, items, S(s)));
+    }
+    return decode_real_impl(ctx, plain, limbs, items, slots, scale, plain, reinterpret_cast<double2 *>(v), out, count, s);
 }
 
 int he_ckks_decode(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t slots, double scale,
                    double *out, uint64_t *ws, he_stream s) {
     if (!ctx || !plain || !out || !ws || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0)) return HE_E_INVALID_ARGUMENT;
-    const size_t n = ctx->n();
-    HE_HIP(hipMemcpyAsync(ws, plain, (size_t)limbs * n * sizeof(uint64_t), hipMemcpyDeviceToDevice, S(s)));
-    if (int rc = he_ntt_inverse(ctx, ws, 1, limbs, limbs, 0, limbs, 0, s)) return rc;
+    NttArgs inv = base_args(ctx, false);
+    inv.in = plain;
+    inv.out = ws;
+    inv.in_poly_stride = inv.out_poly_stride = limbs;
+    inv.map = plain_map(limbs);
+    HE_HIP(launch_ntt_inverse(inv, 1, backend_for(ctx, inv.map), S(s)));
     const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
     HE_HIP(launch_ckks_decode(ft, ctx->tables(), ws, limbs, slots, scale, ctx->d_garner_inv, ctx->size_q,
                               reinterpret_cast<double2 *>(out), 1, S(s)));

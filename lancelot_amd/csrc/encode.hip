@@ -6,18 +6,16 @@
 // contraction): a butterfly is u = a + b, t = (a - b) * w with the four-multiplication complex product, so
 // the result does not depend on how the butterflies are spread over threads.
 //
-// Layout: v = `slots` complex values as double2.  The stages whose span exceeds one tile of 2048 values (at most 5)
-// run as one kernel over global memory, every thread holding the values that those stages combine; all the others
-// run inside LDS in a single kernel.
+// Layout: v = `slots` complex values as double2.
 #include "kernels.h"
 #include "modarith.cuh"
+#include "ntt_common.cuh"
 
 namespace he {
 
 namespace {
 
 constexpr int kThreads = 256;
-constexpr uint32_t kFftTile = 2048;  // complex values per workgroup in the LDS kernel (32 KiB)
 
 __device__ __forceinline__ double2 cmul(double2 a, double2 w) {
     return double2{a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x};
@@ -63,50 +61,23 @@ __device__ __forceinline__ double2 source_value(const FftSource &src, uint32_t i
     return double2{src.re[at], src.im ? src.im[at] : 0.0};
 }
 
-constexpr int kTopThreads = 64;
+// Where a decoding ends: with `re` the real parts of the first `count` values of every item, packed, instead of the vector.
+struct FftTarget {
+    double *re;
+    uint32_t count;
+    size_t value_stride;   // doubles between the items' values
+};
 
-// The R stages of span > tile in one kernel over global memory: thread `id` of an item holds the 2^R values
-// id + h * tile, which those stages combine among themselves only; every butterfly is the one that a launch per
-// stage with a thread per butterfly would compute (same operands, same twiddle).  blockIdx.y = item (vectors `slots`
-// apart).  INVERSE runs the spans slots, slots / 2, .., 2 tile; forward 2 tile, .., slots.
-template <bool INVERSE, int R>
-__global__ __launch_bounds__(kTopThreads) void cfft_top_kernel(double2 *v, uint32_t tile, FftTables t, uint32_t slots,
-                                                               FftSource src) {
-    constexpr int E = 1 << R;
-    const uint32_t id = blockIdx.x * kTopThreads + threadIdx.x;
-    v += (size_t)blockIdx.y * slots;
-    double2 e[E];
-    if (INVERSE && src.re) {
-        if (id == 0) src.max_bits[blockIdx.y] = 0;
-#pragma unroll
-        for (int h = 0; h < E; h++) e[h] = source_value(src, blockIdx.y, id + h * tile);
-    } else {
-#pragma unroll
-        for (int h = 0; h < E; h++) e[h] = v[id + h * tile];
-    }
-#pragma unroll
-    for (int st = 0; st < R; st++) {
-        const int half = INVERSE ? E >> (st + 1) : 1 << st;   // distance of a butterfly's operands, in h
-        const uint32_t len = tile * 2 * half;
-#pragma unroll
-        for (int b = 0; b < E / 2; b++) {
-            const int lo = b & (half - 1), h0 = (b / half) * 2 * half + lo;
-            butterfly<INVERSE>(e[h0], e[h0 + half], stage_twiddle<INVERSE>(t, len, id + lo * tile));
-        }
-    }
-#pragma unroll
-    for (int h = 0; h < E; h++) v[id + h * tile] = e[h];
-}
+constexpr uint32_t kSmallSlots = 256;   // below this the small kernel runs
 
-// every stage of span <= tile inside LDS; tile = min(slots, kFftTile) values per workgroup
+// fewer than 256 slots: every stage inside LDS, one workgroup per item
 template <bool INVERSE>
 __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t tile, FftTables t, uint32_t slots,
-                                                            FftSource src) {
-    __shared__ double2 s[kFftTile];
+                                                            FftSource src, FftTarget dst) {
+    __shared__ double2 s[kSmallSlots];
     double2 *g = v + (size_t)blockIdx.y * slots + (size_t)blockIdx.x * tile;
     if (INVERSE && src.re) {
-        // (only when the whole vector is this one tile: otherwise the wider stages have run before)
-        if (threadIdx.x == 0) src.max_bits[blockIdx.y] = 0;
+        if (threadIdx.x == 0 && src.max_bits) src.max_bits[blockIdx.y] = 0;
         for (uint32_t i = threadIdx.x; i < tile; i += kThreads) s[i] = source_value(src, blockIdx.y, i);
     } else {
         for (uint32_t i = threadIdx.x; i < tile; i += kThreads) s[i] = g[i];
@@ -124,109 +95,175 @@ __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t
         }
         __syncthreads();
     }
-    for (uint32_t i = threadIdx.x; i < tile; i += kThreads) g[i] = s[i];
+    if (!INVERSE && dst.re) {
+        for (uint32_t i = threadIdx.x; i < dst.count; i += kThreads) dst.re[blockIdx.y * dst.value_stride + i] = s[i].x;
+    } else {
+        for (uint32_t i = threadIdx.x; i < tile; i += kThreads) g[i] = s[i];
+    }
 }
 
-// The same for a full tile of kFftTile = 2048 values, 8 values per thread: the 11 stages run as register blocks of
-// 3 + 3 + 3 + 2 stages with the tile in LDS between them (4 exchanges instead of 11), and the 24 twiddles a thread
-// needs are fetched ahead of everything (each is a table look-up behind a table look-up: inside the stages, 11 such
-// round trips to L2 in a row were most of the kernel's time).  Every butterfly has the operands and the twiddle it
-// has in cfft_lds_kernel, so the results are the same bit for bit.
-// Block of top span Lb = 8 S (S = 256, 32, 4): thread (hi, lo) = (tid / S, tid mod S) holds hi Lb + lo + k S, k < 8;
-// stage i of it (span Lb >> i) pairs k with k + (4 >> i) and takes twiddle lo + (k mod (4 >> i)) S.
-template <bool INVERSE>
-__global__ __launch_bounds__(kThreads) void cfft_lds8_kernel(double2 *v, FftTables t, uint32_t slots, FftSource src) {
-    constexpr uint32_t T = kFftTile;
-    static_assert(T == 2048 && kThreads == 256, "8 values per thread");
-    __shared__ double2 s[T + T / 32];
-    auto sk = [](uint32_t e) { return e + (e >> 5); };   // (a group of 4 lanes reads 32 values apart in the S = 4 block)
-    double2 *g = v + (size_t)blockIdx.y * slots + (size_t)blockIdx.x * T;
-    const uint32_t tid = threadIdx.x;
-    double2 tw[3][7], twd[3];
-#pragma unroll
-    for (int b = 0; b < 3; b++) {
-        const uint32_t S = 256u >> (3 * b), Lb = 8 * S, lo = tid & (S - 1);
-#pragma unroll
-        for (int k = 0; k < 4; k++) tw[b][k] = stage_twiddle<INVERSE>(t, Lb, lo + k * S);
-#pragma unroll
-        for (int k = 0; k < 2; k++) tw[b][4 + k] = stage_twiddle<INVERSE>(t, Lb / 2, lo + k * S);
-        tw[b][6] = stage_twiddle<INVERSE>(t, Lb / 4, lo);
+// A transform of 2^s >= 256 values as two passes, like the number-theoretic one: the vector is 2^(s - 8) rows x 256 columns;
+// the rows pass holds the stages of span above 256 (a workgroup owns all rows of a few columns), the blocks pass the 8 stages
+// inside 256 consecutive values (a wave owns one block).  A thread holds 4 values in register blocks of two stages (Tile4's
+// layout); its 12 twiddles, each a look-up behind a look-up, are fetched together with the values.  Every butterfly has the
+// operands and the twiddle that a launch per stage would give it, so the results do not depend on the split.  (One
+// workgroup per 2048 values and one thread per 16 wide ones, which this replaced, left most of the chip idle: 12.4 + 10.1 us
+// on the way in, 7.2 + 4.1 us on the way out at 32,768 slots.)
+// Stage sigma of the inverse direction (the forward runs them backwards) pairs index bit s - 1 - sigma; a value's twiddle
+// is chosen by the bits below it.
+template <bool INVERSE, int B, int LD>
+struct FftTile {
+    using T4 = Tile4<B, LD>;
+    struct Tw {
+        double2 a0, a1, b;   // first stage: pairs (0, 2) and (1, 3); second: pairs (0, 1) and (2, 3)
+    };
+    template <typename Pos, int K = 0>
+    static __device__ __forceinline__ void load_tw(Tw *tw, const FftTables &t, uint32_t log_slots, uint32_t stage0, Pos pos) {
+        const uint32_t len = 1u << (log_slots - stage0 - 2 * K), mask = (len >> 1) - 1;
+        tw[K].a0 = stage_twiddle<INVERSE>(t, len, pos(K, 0) & mask);
+        tw[K].a1 = stage_twiddle<INVERSE>(t, len, pos(K, 1) & mask);
+        tw[K].b = T4::stages(K) == 2 ? stage_twiddle<INVERSE>(t, len >> 1, pos(K, 0) & (mask >> 1)) : double2{0.0, 0.0};
+        if constexpr (K + 1 < T4::kBlocks) load_tw<Pos, K + 1>(tw, t, log_slots, stage0, pos);
     }
-    twd[0] = stage_twiddle<INVERSE>(t, 4, 0);
-    twd[1] = stage_twiddle<INVERSE>(t, 4, 1);
-    twd[2] = stage_twiddle<INVERSE>(t, 2, 0);
-    if (INVERSE && src.re) {
-        // (only when the whole vector is this one tile: otherwise the wider stages have run before)
-        if (tid == 0) src.max_bits[blockIdx.y] = 0;
+    static __device__ __forceinline__ void put(const double2 *v, double *re, double *im, int k, uint32_t t) {
 #pragma unroll
-        for (int i = 0; i < 8; i++) s[sk(tid + i * kThreads)] = source_value(src, blockIdx.y, tid + i * kThreads);
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++) s[sk(tid + i * kThreads)] = g[tid + i * kThreads];
+        for (int j = 0; j < 4; j++) {
+            const uint32_t e = skew(T4::word(k, t, j));
+            re[e] = v[j].x;
+            im[e] = v[j].y;
+        }
     }
-    __syncthreads();
-    auto block3 = [&](int b) {
-        const uint32_t S = 256u >> (3 * b), Lb = 8 * S;
-        const uint32_t base = (tid / S) * Lb + (tid & (S - 1));
-        double2 e[8];
+    static __device__ __forceinline__ void get(double2 *v, const double *re, const double *im, int k, uint32_t t) {
 #pragma unroll
-        for (int k = 0; k < 8; k++) e[k] = s[sk(base + k * S)];
-        if (INVERSE) {
+        for (int j = 0; j < 4; j++) {
+            const uint32_t e = skew(T4::word(k, t, j));
+            v[j] = double2{re[e], im[e]};
+        }
+    }
+    // the stages in order (INVERSE), values of block 0 -> values of the last block
+    template <int K = 0>
+    static __device__ __forceinline__ void down(double2 *v, const Tw *tw, double *re, double *im, uint32_t t) {
+        butterfly<INVERSE>(v[0], v[2], tw[K].a0);
+        butterfly<INVERSE>(v[1], v[3], tw[K].a1);
+        if (T4::stages(K) == 2) {
+            butterfly<INVERSE>(v[0], v[1], tw[K].b);
+            butterfly<INVERSE>(v[2], v[3], tw[K].b);
+        }
+        if constexpr (K + 1 < T4::kBlocks) {
+            put(v, re, im, K, t);
+            T4::template sync<K>();
+            get(v, re, im, K + 1, t);
+            down<K + 1>(v, tw, re, im, t);
+        }
+    }
+    // backwards (forward direction), values of the last block -> values of block 0
+    template <int K = T4::kBlocks - 1>
+    static __device__ __forceinline__ void up(double2 *v, const Tw *tw, double *re, double *im, uint32_t t) {
+        if (T4::stages(K) == 2) {
+            butterfly<INVERSE>(v[0], v[1], tw[K].b);
+            butterfly<INVERSE>(v[2], v[3], tw[K].b);
+        }
+        butterfly<INVERSE>(v[0], v[2], tw[K].a0);
+        butterfly<INVERSE>(v[1], v[3], tw[K].a1);
+        if constexpr (K > 0) {
+            put(v, re, im, K, t);
+            T4::template sync<K - 1>();
+            get(v, re, im, K - 1, t);
+            up<K - 1>(v, tw, re, im, t);
+        }
+    }
+};
+
+// blockIdx.x = tile of 2^(B - LD) columns, blockIdx.y = item
+template <bool INVERSE, int B, int LD>
+__global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, FftTables t, uint32_t log_slots, FftSource src,
+                                                                 FftTarget dst) {
+    using F = FftTile<INVERSE, B, LD>;
+    using T4 = typename F::T4;
+    constexpr int LOGC = B - LD, NB = T4::kBlocks;
+    __shared__ double re[(1 << B) + (1 << (B - 4))], im[(1 << B) + (1 << (B - 4))];
+    const uint32_t item = blockIdx.y, col0 = blockIdx.x << LOGC, tid = threadIdx.x;
+    v += (size_t)item << log_slots;
+    auto pos = [&](int k, int j) {
+        const uint32_t e = T4::word(k, tid, j);
+        return ((e >> LOGC) << 8) + col0 + (e & ((1u << LOGC) - 1));
+    };
+    double2 x[4];
+    typename F::Tw tw[NB];
+    if (INVERSE) {
+        if (src.re) {
+            if (src.max_bits && blockIdx.x == 0 && tid == 0) src.max_bits[item] = 0;
 #pragma unroll
-            for (int k = 0; k < 4; k++) butterfly<true>(e[k], e[k + 4], tw[b][k]);
-#pragma unroll
-            for (int k = 0; k < 4; k++) butterfly<true>(e[(k & 1) + 4 * (k >> 1)], e[(k & 1) + 4 * (k >> 1) + 2], tw[b][4 + (k & 1)]);
-#pragma unroll
-            for (int k = 0; k < 8; k += 2) butterfly<true>(e[k], e[k + 1], tw[b][6]);
+            for (int j = 0; j < 4; j++) x[j] = source_value(src, item, pos(0, j));
         } else {
 #pragma unroll
-            for (int k = 0; k < 8; k += 2) butterfly<false>(e[k], e[k + 1], tw[b][6]);
-#pragma unroll
-            for (int k = 0; k < 4; k++) butterfly<false>(e[(k & 1) + 4 * (k >> 1)], e[(k & 1) + 4 * (k >> 1) + 2], tw[b][4 + (k & 1)]);
-#pragma unroll
-            for (int k = 0; k < 4; k++) butterfly<false>(e[k], e[k + 4], tw[b][k]);
+            for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
         }
+        F::load_tw(tw, t, log_slots, 0, pos);
+        F::down(x, tw, re, im, tid);
 #pragma unroll
-        for (int k = 0; k < 8; k++) s[sk(base + k * S)] = e[k];
-        __syncthreads();
-    };
-    // spans 4 and 2: two groups of 4 consecutive values per thread
-    auto block2 = [&]() {
-#pragma unroll
-        for (int r = 0; r < 2; r++) {
-            const uint32_t base = 4 * (tid + r * kThreads);
-            double2 e[4];
-#pragma unroll
-            for (int k = 0; k < 4; k++) e[k] = s[sk(base + k)];
-            if (INVERSE) {
-                butterfly<true>(e[0], e[2], twd[0]);
-                butterfly<true>(e[1], e[3], twd[1]);
-                butterfly<true>(e[0], e[1], twd[2]);
-                butterfly<true>(e[2], e[3], twd[2]);
-            } else {
-                butterfly<false>(e[0], e[1], twd[2]);
-                butterfly<false>(e[2], e[3], twd[2]);
-                butterfly<false>(e[0], e[2], twd[0]);
-                butterfly<false>(e[1], e[3], twd[1]);
-            }
-#pragma unroll
-            for (int k = 0; k < 4; k++) s[sk(base + k)] = e[k];
-        }
-        __syncthreads();
-    };
-    if (INVERSE) {
-        block3(0);
-        block3(1);
-        block3(2);
-        block2();
+        for (int j = 0; j < 4; j++) v[pos(NB - 1, j)] = x[j];
     } else {
-        block2();
-        block3(2);
-        block3(1);
-        block3(0);
-    }
 #pragma unroll
-    for (int i = 0; i < 8; i++) g[tid + i * kThreads] = s[sk(tid + i * kThreads)];
+        for (int j = 0; j < 4; j++) x[j] = v[pos(NB - 1, j)];
+        F::load_tw(tw, t, log_slots, 0, pos);
+        F::up(x, tw, re, im, tid);
+        if (dst.re) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (pos(0, j) < dst.count) dst.re[item * dst.value_stride + pos(0, j)] = x[j].x;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
+        }
+    }
+}
+
+constexpr int kFftWaves = 2;   // 256-value blocks of a workgroup
+
+// blockIdx.y = item
+template <bool INVERSE>
+__global__ __launch_bounds__(64 * kFftWaves) void cfft_blocks_kernel(double2 *v, FftTables t, uint32_t log_slots, FftSource src,
+                                                                     FftTarget dst) {
+    using F = FftTile<INVERSE, 8, 8>;
+    using T4 = typename F::T4;
+    __shared__ double re_all[kFftWaves][256 + 16], im_all[kFftWaves][256 + 16];
+    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63, item = blockIdx.y;
+    const uint32_t blk = blockIdx.x * kFftWaves + w;
+    if (blk >= 1u << (log_slots - 8)) return;   // (256 slots: one block)
+    double *re = re_all[w], *im = im_all[w];
+    v += ((size_t)item << log_slots) + (size_t)blk * 256;
+    auto pos = [&](int k, int j) { return T4::word(k, lane, j); };   // (the twiddles depend on the position inside the block)
+    double2 x[4];
+    typename F::Tw tw[4];
+    if (INVERSE) {
+        if (src.re) {
+            // (only when the whole vector is this one block: otherwise the rows pass has run before)
+            if (src.max_bits && lane == 0) src.max_bits[item] = 0;
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = source_value(src, item, pos(0, j));
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
+        }
+        F::load_tw(tw, t, log_slots, log_slots - 8, pos);
+        F::down(x, tw, re, im, lane);
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[pos(3, j)] = x[j];
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = v[pos(3, j)];
+        F::load_tw(tw, t, log_slots, log_slots - 8, pos);
+        F::up(x, tw, re, im, lane);
+        if (dst.re && log_slots == 8) {
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+                if (pos(0, j) < dst.count) dst.re[item * dst.value_stride + pos(0, j)] = x[j].x;
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
+        }
+    }
 }
 
 // The largest magnitude of an item's coefficients (the bit patterns of non-negative doubles order like the values):
@@ -329,30 +366,17 @@ __global__ __launch_bounds__(kThreads) void encode_round_tiled_kernel(const doub
 
 constexpr int kMaxComposeLimbs = 64;
 
-// Garner's mixed-radix composition of one coefficient, centred around zero, as a double divided by the scale.
-// thread s < slots: real part of value s, else imaginary part of value s - slots; stored at position bitrev.
-// LIMBS > 0: the number of limbs at compile time (the digits then stay in registers; with a run-time count the array
-// lives in scratch memory), 0: any number up to kMaxComposeLimbs.
+// Garner's mixed-radix composition of one coefficient from its residues d[0 .. limbs-1] (overwritten), centred around zero,
+// as a double divided by the scale.  LIMBS > 0: the number of limbs at compile time (the digits then stay in registers;
+// with a run-time count the array lives in scratch memory), 0: any number up to kMaxComposeLimbs.
 template <int LIMBS>
-__global__ __launch_bounds__(kThreads) void decode_compose_kernel(const uint64_t *res, uint32_t limbs_rt, uint32_t log_n,
-                                                                  uint32_t log_slots, uint32_t gap, double inv_scale,
-                                                                  const uint64_t *moduli, const uint64_t *barrett,
-                                                                  const uint64_t *garner_inv, uint32_t garner_stride,
-                                                                  double2 *v) {
+__device__ __forceinline__ double compose(uint64_t *d, uint32_t limbs_rt, double inv_scale, const uint64_t *moduli, const uint64_t *barrett,
+                                          const uint64_t *garner_inv, uint32_t garner_stride) {
     const uint32_t limbs = LIMBS ? (uint32_t)LIMBS : limbs_rt;
-    const uint32_t s = blockIdx.x * kThreads + threadIdx.x;
-    const uint32_t slots = 1u << log_slots, half = 1u << (log_n - 1);
-    if (s >= 2 * slots) return;
-    res += ((size_t)blockIdx.y * limbs) << log_n;   // blockIdx.y = item: dense plaintexts, dense slot vectors
-    v += (size_t)blockIdx.y * slots;
-    const bool imag = s >= slots;
-    const uint32_t i0 = imag ? s - slots : s;
-    const size_t coeff = (imag ? half : 0) + (size_t)i0 * gap;
-    uint64_t d[LIMBS ? LIMBS : kMaxComposeLimbs];
 #pragma unroll
     for (uint32_t i = 0; i < limbs; i++) {
         const uint64_t q = moduli[i], r0 = barrett[2 * i], r1 = barrett[2 * i + 1];
-        uint64_t t = res[((size_t)i << log_n) + coeff];
+        uint64_t t = d[i];
 #pragma unroll
         for (uint32_t j = 0; j < i; j++) {
             const uint64_t dj = barrett64(d[j], q, r1);
@@ -392,44 +416,120 @@ __global__ __launch_bounds__(kThreads) void decode_compose_kernel(const uint64_t
         const uint32_t i = limbs - 1 - k;
         acc = acc * (double)moduli[i] + (double)d[i];
     }
-    const double val = (negative ? -acc : acc) * inv_scale;
+    return (negative ? -acc : acc) * inv_scale;
+}
+
+// thread s < slots: real part of value s, else imaginary part of value s - slots; stored at position bitrev.
+template <int LIMBS>
+__global__ __launch_bounds__(kThreads) void decode_compose_kernel(const uint64_t *res, uint32_t limbs_rt, uint32_t log_n,
+                                                                  uint32_t log_slots, uint32_t gap, double inv_scale,
+                                                                  const uint64_t *moduli, const uint64_t *barrett,
+                                                                  const uint64_t *garner_inv, uint32_t garner_stride,
+                                                                  double2 *v) {
+    const uint32_t limbs = LIMBS ? (uint32_t)LIMBS : limbs_rt;
+    const uint32_t s = blockIdx.x * kThreads + threadIdx.x;
+    const uint32_t slots = 1u << log_slots, half = 1u << (log_n - 1);
+    if (s >= 2 * slots) return;
+    res += ((size_t)blockIdx.y * limbs) << log_n;   // blockIdx.y = item: dense plaintexts, dense slot vectors
+    v += (size_t)blockIdx.y * slots;
+    const bool imag = s >= slots;
+    const uint32_t i0 = imag ? s - slots : s;
+    const size_t coeff = (imag ? half : 0) + (size_t)i0 * gap;
+    uint64_t d[LIMBS ? LIMBS : kMaxComposeLimbs];
+#pragma unroll
+    for (uint32_t i = 0; i < limbs; i++) d[i] = res[((size_t)i << log_n) + coeff];
     double *slot = reinterpret_cast<double *>(&v[__brev(i0) >> (32 - log_slots)]);
-    slot[imag ? 1 : 0] = val;
+    slot[imag ? 1 : 0] = compose<LIMBS>(d, limbs, inv_scale, moduli, barrett, garner_inv, garner_stride);
+}
+
+// The inverse rows pass of all limbs of a plaintext and the composition in one kernel: a workgroup takes one tile of every
+// limb in turn through the pass, which leaves rows r, r + R/4 (real parts of two values) and r + R/2, r + 3R/4 (their
+// imaginary parts) of one column in each thread, and composes them.  The two values go to neighbouring positions of the
+// slot vector.  Full and sparse packing; blockIdx.y = item.
+template <int LD, int LIMBS>
+__global__ __launch_bounds__(256) void decode_rows_compose_kernel(NttArgs a, uint32_t log_slots, double inv_scale,
+                                                                  const uint64_t *garner_inv, uint32_t garner_stride, double2 *v) {
+    constexpr int B = 10, LOGC = B - LD;
+    using T4 = Tile4<B, LD>;
+    constexpr int NB = T4::kBlocks;
+    __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
+    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    const uint32_t col0 = blockIdx.x << LOGC, item = blockIdx.y;
+    auto glob = [&](int k, int j) {
+        const uint32_t e = T4::word(k, t, j);
+        return (size_t)(e >> LOGC) * 256 + col0 + (e & ((1u << LOGC) - 1));
+    };
+    uint64_t d[4][LIMBS];
+#pragma unroll
+    for (int l = 0; l < LIMBS; l++) {
+        const Job job = decode_job(a, item * LIMBS + l);
+        uint64_t x[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = job.in[glob(NB - 1, j)];
+        if ((a.fp_mask >> job.table) & 1) {
+            const FpArith ar = fp_arith(a, job.table);
+            FpArith::Tw tw[NB];
+            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+            const FpTw scale = inverse_scale(a, job, ar.m);
+            double w[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = FpArith::from_word(x[j]);
+            ar.reduce(w);
+            T4::template inverse<FpArith>(w, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) d[j][l] = fp_to_u64(fp_canonical(fp_mulmod(w[j], scale, ar.m), ar.m));
+        } else {
+            const IntArith ar = int_arith(a, job.table);
+            IntArith::Tw tw[NB];
+            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            T4::template inverse<IntArith>(x, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) d[j][l] = reduce_2q(x[j], ar.m.q);
+        }
+        lds_barrier();   // (the next limb's tile overwrites this one's)
+    }
+    double val[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) val[j] = compose<LIMBS>(d[j], LIMBS, inv_scale, a.moduli, a.barrett, garner_inv, garner_stride);
+    const uint32_t log_gap = a.log_n - 1 - log_slots;
+    v += (size_t)item << log_slots;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        const uint32_t k = (uint32_t)glob(0, j);   // (below N / 2)
+        if ((k & ((1u << log_gap) - 1)) == 0) v[__brev(k >> log_gap) >> (32 - log_slots)] = double2{val[j], val[j + 2]};
+    }
 }
 
 template <bool INVERSE>
-hipError_t run_fft(double2 *v, uint32_t slots, uint32_t items, const FftTables &t, hipStream_t s, FftSource src) {
-    const uint32_t tile = slots < kFftTile ? slots : kFftTile;
-    const dim3 top_grid(tile / kTopThreads, items), lds_grid(slots / tile, items);
-    const uint32_t wide = 31 - __builtin_clz(slots / tile);   // stages of span > tile
+hipError_t run_fft(double2 *v, uint32_t slots, uint32_t items, const FftTables &t, hipStream_t s, FftSource src, FftTarget dst) {
+    const uint32_t log_slots = 31 - __builtin_clz(slots);
+    if (slots < kSmallSlots) {
+        hipLaunchKernelGGL(cfft_lds_kernel<INVERSE>, dim3(1, items), dim3(kThreads), 0, s, v, slots, t, slots, src, dst);
+        return hipGetLastError();
+    }
+    const uint32_t ld = log_slots - 8;
     const FftSource none{nullptr, nullptr, 0, 0, nullptr};
-    auto top = [&](FftSource from) {
-        switch (wide) {
-            case 1: hipLaunchKernelGGL((cfft_top_kernel<INVERSE, 1>), top_grid, dim3(kTopThreads), 0, s, v, tile, t, slots, from); break;
-            case 2: hipLaunchKernelGGL((cfft_top_kernel<INVERSE, 2>), top_grid, dim3(kTopThreads), 0, s, v, tile, t, slots, from); break;
-            case 3: hipLaunchKernelGGL((cfft_top_kernel<INVERSE, 3>), top_grid, dim3(kTopThreads), 0, s, v, tile, t, slots, from); break;
-            case 4: hipLaunchKernelGGL((cfft_top_kernel<INVERSE, 4>), top_grid, dim3(kTopThreads), 0, s, v, tile, t, slots, from); break;
-            case 5: hipLaunchKernelGGL((cfft_top_kernel<INVERSE, 5>), top_grid, dim3(kTopThreads), 0, s, v, tile, t, slots, from); break;
+    auto rows = [&]() {
+        // tiles of 1024 values (8 columns at 32,768 slots)
+#define HE_CASE(LD, B) \
+    case LD: hipLaunchKernelGGL((cfft_rows_kernel<INVERSE, B, LD>), dim3(256u >> (B - LD), items), dim3(1u << (B - 2)), 0, s, v, t, log_slots, src, dst); break;
+        switch (ld) {
+            HE_CASE(1, 8) HE_CASE(2, 10) HE_CASE(3, 10) HE_CASE(4, 10) HE_CASE(5, 10) HE_CASE(6, 10) HE_CASE(7, 10) HE_CASE(8, 10)
             default: return hipErrorInvalidValue;
         }
-        return hipSuccess;
+#undef HE_CASE
+        return hipGetLastError();
     };
-    if (INVERSE) {
-        if (wide)
-            if (hipError_t e = top(src)) return e;
-        if (tile == kFftTile)
-            hipLaunchKernelGGL(cfft_lds8_kernel<true>, lds_grid, dim3(kThreads), 0, s, v, t, slots, wide ? none : src);
-        else
-            hipLaunchKernelGGL(cfft_lds_kernel<true>, lds_grid, dim3(kThreads), 0, s, v, tile, t, slots, wide ? none : src);
-    } else {
-        if (tile == kFftTile)
-            hipLaunchKernelGGL(cfft_lds8_kernel<false>, lds_grid, dim3(kThreads), 0, s, v, t, slots, none);
-        else
-            hipLaunchKernelGGL(cfft_lds_kernel<false>, lds_grid, dim3(kThreads), 0, s, v, tile, t, slots, none);
-        if (wide)
-            if (hipError_t e = top(none)) return e;
-    }
-    return hipGetLastError();
+    auto blocks = [&]() {
+        hipLaunchKernelGGL(cfft_blocks_kernel<INVERSE>, dim3(((1u << ld) + kFftWaves - 1) / kFftWaves, items), dim3(64 * kFftWaves), 0, s, v, t,
+                           log_slots, ld ? none : src, dst);
+        return hipGetLastError();
+    };
+    if (INVERSE && ld)
+        if (hipError_t e = rows()) return e;
+    if (hipError_t e = blocks()) return e;
+    if (!INVERSE && ld) return rows();
+    return hipSuccess;
 }
 
 // out[item][i] = v[item][i] for i < count: the leading slots of every item, packed
@@ -447,7 +547,7 @@ hipError_t launch_ckks_encode(const FftTables &t, const double *re, const double
     const uint32_t n = 1u << t.log_n, log_slots = 31 - __builtin_clz(slots);
     if (items == 0 || items > 65535 || (out ? (!tab || limbs == 0) : !coeffs)) return hipErrorInvalidValue;
     unsigned long long *maxima = reinterpret_cast<unsigned long long *>(max_bits);
-    hipError_t e = run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, maxima});
+    hipError_t e = run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, maxima}, FftTarget{nullptr, 0, 0});
     if (e != hipSuccess) return e;
     const RoundSink sink{coeffs, out, out ? tab->moduli : nullptr, out ? tab->barrett : nullptr, limbs, out_item_stride};
     if (slots == n / 2 && log_slots >= 8)
@@ -459,9 +559,21 @@ hipError_t launch_ckks_encode(const FftTables &t, const double *re, const double
     return hipGetLastError();
 }
 
-hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs,
-                              uint32_t slots, double scale, const uint64_t *garner_inv, uint32_t garner_stride,
-                              double2 *v, uint32_t items, hipStream_t s) {
+hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
+                                   double2 *v, uint32_t items, size_t value_stride, hipStream_t s) {
+    if (items == 0 || items > 65535 || !re) return hipErrorInvalidValue;
+    return run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, nullptr}, FftTarget{nullptr, 0, 0});
+}
+
+hipError_t launch_ckks_fft_real(const FftTables &t, uint32_t slots, double2 *v, uint32_t items, double *re, uint32_t count,
+                                hipStream_t s) {
+    if (items == 0 || items > 65535 || !re || count == 0 || count > slots) return hipErrorInvalidValue;
+    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{re, count, count});
+}
+
+hipError_t launch_ckks_compose(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs,
+                               uint32_t slots, double scale, const uint64_t *garner_inv, uint32_t garner_stride,
+                               double2 *v, uint32_t items, hipStream_t s) {
     const uint32_t n = 1u << t.log_n, log_slots = 31 - __builtin_clz(slots);
     if (limbs == 0 || limbs > (uint32_t)kMaxComposeLimbs || items == 0 || items > 65535) return hipErrorInvalidValue;
     const dim3 grid((2 * slots + kThreads - 1) / kThreads, items);
@@ -476,7 +588,43 @@ hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint6
         default: HE_COMPOSE(0); break;
     }
 #undef HE_COMPOSE
-    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr});
+    return hipGetLastError();
+}
+
+hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs,
+                              uint32_t slots, double scale, const uint64_t *garner_inv, uint32_t garner_stride,
+                              double2 *v, uint32_t items, hipStream_t s) {
+    if (hipError_t e = launch_ckks_compose(t, tab, res, limbs, slots, scale, garner_inv, garner_stride, v, items, s)) return e;
+    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{nullptr, 0, 0});
+}
+
+hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int backend, uint32_t slots, double scale,
+                                   const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items, double *re,
+                                   uint32_t count, hipStream_t s) {
+    const uint32_t limbs = inv.map.limbs, log_slots = 31 - __builtin_clz(slots);
+    if (inv.log_n < 12 || inv.log_n > 16 || inv.jobs || limbs == 0 || limbs > 4 || items == 0 || items > 65535) return hipErrorInvalidValue;
+    NttArgs a = inv;   // (the mask stands for the launch's back end)
+    a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : inv.fp_mask);
+    const dim3 grid(1u << (a.log_n - 10), items);
+#define HE_LIMBS(LD, L)                                                                                                            \
+    hipLaunchKernelGGL((decode_rows_compose_kernel<LD, L>), grid, dim3(256), 0, s, a, log_slots, 1.0 / scale, garner_inv, garner_stride, v)
+#define HE_CASE(LD)                         \
+    case LD:                                \
+        switch (limbs) {                    \
+            case 1: HE_LIMBS(LD, 1); break; \
+            case 2: HE_LIMBS(LD, 2); break; \
+            case 3: HE_LIMBS(LD, 3); break; \
+            default: HE_LIMBS(LD, 4);       \
+        }                                   \
+        break;
+    switch (a.log_n - 8) {
+        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+        default: return hipErrorInvalidValue;
+    }
+#undef HE_CASE
+#undef HE_LIMBS
+    if (hipError_t e = hipGetLastError()) return e;
+    return launch_ckks_fft_real(t, slots, v, items, re, count, s);
 }
 
 hipError_t launch_take_slots(const double2 *v, uint32_t slots, uint32_t items, uint32_t count, double2 *out, hipStream_t s) {

@@ -161,13 +161,13 @@ PYBIND11_MODULE(pyCAHEL, m) {
         .def("decrypt_decode_many",
              [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, const std::vector<const CAHELGPUCiphertext *> &cts,
                 std::size_t slots, std::size_t count) {
-                 std::vector<double> out;
+                 // (a count out of range has no array: it is an error below)
+                 py::array_t<double> a({(py::ssize_t)cts.size(), (py::ssize_t)(count > slots || slots > c.poly_degree() ? 0 : count)});
+                 double *values = a.mutable_data();
                  {
                      py::gil_scoped_release release;
-                     out = k.decrypt_decode_many(c, cts, slots, count);
+                     k.decrypt_decode_many(c, cts, slots, count, values);
                  }
-                 py::array_t<double> a({(py::ssize_t)cts.size(), (py::ssize_t)count});
-                 std::copy(out.begin(), out.end(), a.mutable_data());
                  return a;
              },
              py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count") = 1)
@@ -242,12 +242,14 @@ PYBIND11_MODULE(pyCAHEL, m) {
              py::arg("context"), py::arg("public_key"), py::arg("values").noconvert(), py::arg("scale"))
         .def("decode_array",
              [](CAHELGPUCKKSEncoder &e, const CAHELGPUContext &c, const CAHELGPUPlaintext &p, std::size_t count) {
-                 std::vector<double> out;
+                 py::array_t<double> out((py::ssize_t)e.decode_count(c, p, count));
+                 double *values = out.mutable_data();
+                 const std::size_t size = (std::size_t)out.size();
                  {
                      py::gil_scoped_release release;
-                     e.decode_prefix(c, p, count, out);
+                     e.decode_real(c, p, size, values);
                  }
-                 return py::array_t<double>((py::ssize_t)out.size(), out.data());
+                 return out;
              },
              py::arg("context"), py::arg("plain"), py::arg("count") = 0)
         .def("encode", py::overload_cast<const CAHELGPUContext &, const std::vector<double> &, double>(

@@ -183,6 +183,7 @@ private:
     std::size_t n_ = 0, size_q_ = 0, size_p_ = 0;
     int log_n_ = 0;
     std::vector<std::size_t> chain_limbs_;
+    std::vector<int> chain_bits_;   // bits of the product of a level's moduli
     std::vector<cahel::parms_id_type> parms_ids_;
     std::vector<uint32_t> galois_elts_;
     he_context *he_ = nullptr;
@@ -363,9 +364,15 @@ public:
     // Real parts of the first `count` slots of every ciphertext, [items][count] row-major: decrypt + decode of all of
     // them with one launch per stage (not in the reference).  All ciphertexts: size 2, one level, one scale;
     // `slots` = the encoder's slot count.
+    void decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
+                             std::size_t slots, std::size_t count, double *destination);
     std::vector<double> decrypt_decode_many(const CAHELGPUContext &context,
                                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots,
-                                            std::size_t count);
+                                            std::size_t count) {
+        std::vector<double> out(count > slots || slots > context.poly_degree() ? 0 : ciphers.size() * count);
+        decrypt_decode_many(context, ciphers, slots, count, out.data());
+        return out;
+    }
     const uint64_t *secret_key_array() const { return sk_powers_.get(); }
 
 private:
@@ -415,9 +422,13 @@ public:
         return destination;
     }
     void decode(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::vector<double> &destination);
-    // real parts of the first `count` slots only (0: all): the transform runs in full, the download is `count` values
+    // complex values of the first `count` slots, interleaved
     void decode_values(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count,
                        std::vector<double> &interleaved);
+    // Real parts of the first `count` slots only (0: all): the transform runs in full, the download is `count` values.  In two
+    // steps for a caller with memory of its own: how many values there will be, then the values.
+    std::size_t decode_count(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count);
+    void decode_real(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count, double *destination);
     void decode_prefix(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count,
                        std::vector<double> &destination);
     void decode_complex(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::vector<double> &re,

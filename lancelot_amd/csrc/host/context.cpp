@@ -383,8 +383,10 @@ CAHELGPUContext::CAHELGPUContext(const EncryptionParameters &params, bool expand
         // a single-modulus chain has no special modulus
         std::vector<uint64_t> vals;
         for (auto &m : mods) vals.push_back(m.value());
-        for (std::size_t limbs : chain_limbs_)
+        for (std::size_t limbs : chain_limbs_) {
             parms_ids_.push_back(compute_parms_id(params.scheme(), n_, size_p_, vals, limbs));
+            chain_bits_.push_back(BigUInt::product({vals.begin(), vals.begin() + limbs}).bit_count());
+        }
     }
     galois_elts_ = params.galois_elts();
     if (galois_elts_.empty()) {
@@ -425,10 +427,8 @@ parms_id_type CAHELGPUContext::parms_id_at(std::size_t chain_index) const {
 }
 
 int CAHELGPUContext::total_coeff_modulus_bit_count(std::size_t chain_index) const {
-    std::vector<uint64_t> vals;
-    const auto &mods = params_.coeff_modulus();
-    for (std::size_t i = 0; i < limbs_at(chain_index); i++) vals.push_back(mods[i].value());
-    return BigUInt::product(vals).bit_count();
+    if (chain_index >= chain_bits_.size()) throw std::invalid_argument("chain index out of range");
+    return chain_bits_[chain_index];
 }
 
 uint32_t CAHELGPUContext::get_elt_from_step(int step) const { return elt_from_step(step, n_); }

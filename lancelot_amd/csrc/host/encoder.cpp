@@ -6,44 +6,45 @@
 // butterfly network in FP64, rounding, residues, CRT composition, NTTs); the host moves the slot values in and
 // out and keeps the reference's argument checks.  Decoded values agree with the reference up to FP64 operation
 // order (bounded by the 2^-20 acceptance tolerance), not bit for bit.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 
 #include "cahel.h"
+#include "staging.h"
 
 using namespace cahel;
 
 namespace {
 
-// Page-locked staging for the values of an encoding, one buffer per host thread (the lanes of the host layer encode
-// from several threads), grown on demand and kept until the thread ends.  The values are copied into it and uploaded
-// without waiting; every encoding ends with a blocking download (its largest coefficient), after which the buffer is
-// free for the thread's next call.
-struct PinnedStage {
-    void *ptr = nullptr;
-    std::size_t bytes = 0;
-    PinnedStage() = default;
-    PinnedStage(const PinnedStage &) = delete;
-    PinnedStage &operator=(const PinnedStage &) = delete;
-    ~PinnedStage() {
-        if (ptr) (void)he_host_free(ptr);   // (worker threads of a pool come and go: no buffer is left behind)
-    }
-    double *ensure(std::size_t want) {
-        if (want > bytes) {
-            void *old = ptr;
-            ptr = nullptr;
-            bytes = 0;
-            if (old) check_status(he_host_free(old), "he_host_free");
-            check_status(he_host_malloc(&ptr, want), "he_host_malloc");
-            bytes = want;
-        }
-        return static_cast<double *>(ptr);
-    }
-};
+// how much of a batch's values travels at once: 1 MiB takes the link about 20 us, several times what starting a copy costs
+constexpr std::size_t kChunkBytes = std::size_t(1) << 20;
 
-double *pinned_stage(std::size_t bytes) {
-    thread_local PinnedStage stage;
-    return stage.ensure(bytes);
+// dst = src, and the sum of the magnitudes
+double copy_sum(double *dst, const double *src, std::size_t count) {
+    double s = 0.0;
+#pragma omp simd reduction(+ : s)
+    for (std::size_t i = 0; i < count; i++) {
+        dst[i] = src[i];
+        s += std::fabs(src[i]);
+    }
+    return s;
+}
+
+// No coefficient of an encoding exceeds scale / slots times the sum of the values' magnitudes (the transform's twiddles have
+// magnitude 1; the margin covers its rounding).  When that already stays inside the bounds that the largest coefficient has to
+// keep, the coefficients need not be looked at: the encoding is enqueued and nothing waits for it.
+bool surely_small(double sum, double scale, std::size_t slots, int total_bits) {
+    const double bound = 1.001 * (scale / static_cast<double>(slots)) * sum + 1.0;
+    if (!(bound < 0x1p61)) return false;   // (also: not a number)
+    return static_cast<int>(std::ceil(std::log2(bound))) + 1 < total_bits;
+}
+
+void check_largest(double max_coeff, int total_bits) {
+    const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
+    if (max_coeff_bit_count >= total_bits) throw std::invalid_argument("encoded values are too large");
+    if (max_coeff_bit_count > 63)
+        throw std::invalid_argument("encoded values are too large: coefficients above 2^62 are not supported");
 }
 
 }  // namespace
@@ -86,29 +87,40 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_many(const C
     he_context *h = context.handle();
     he_stream st = context.stream();
 
-    // values -> device, packed
+    // values -> device, packed, some messages at a time through page-locked memory (the next ones are copied while the last
+    // travel)
     DeviceBuffer staging(items * count);
     double *d_values = reinterpret_cast<double *>(staging.get());
-    if (count) {
-        if (value_stride == count) {
-            check_status(he_memcpy_h2d(d_values, values, items * count * sizeof(double), st), "upload");
-        } else {
-            for (std::size_t k = 0; k < items; k++)
-                check_status(he_memcpy_h2d(d_values + k * count, values + k * value_stride, count * sizeof(double), st), "upload");
-        }
+    PinnedRing &ring = PinnedRing::of_thread();
+    const std::size_t rows = count ? std::max<std::size_t>(1, kChunkBytes / (count * sizeof(double))) : items;
+    bool small = true;
+    for (std::size_t first = 0; count && first < items; first += rows) {
+        const std::size_t taken = std::min(rows, items - first), bytes = taken * count * sizeof(double);
+        double *host = static_cast<double *>(ring.take(bytes));
+        for (std::size_t k = 0; k < taken; k++)
+            small = surely_small(copy_sum(host + k * count, values + (first + k) * value_stride, count), scale, ss, total_bits) && small;
+        const int status = he_memcpy_h2d_async(d_values + first * count, host, bytes, st);
+        ring.fence(st);
+        check_status(status, "upload");
     }
     // plaintexts straight into polynomial 0 of the ciphertexts
     const std::size_t words = 2 * (std::size_t)L * n;
     DeviceBuffer batch(items * words), ws(he_ckks_encode_batch_workspace_words(h, (uint32_t)items));
-    check_status(he_ckks_encode_batch(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
-                                      batch.get(), 2 * L, ws.get(), st),
-                 "he_ckks_encode_batch");
-    std::vector<double> maxima(items);
-    check_status(he_memcpy_d2h(maxima.data(), ws.get(), items * sizeof(double), st), "download");
-    for (double max_coeff : maxima) {
-        const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
-        if (max_coeff_bit_count >= total_bits || max_coeff_bit_count > 63)
-            throw std::invalid_argument("encoded values are too large");
+    if (small) {
+        check_status(he_ckks_encode_bounded(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
+                                            batch.get(), 2 * L, ws.get(), st),
+                     "he_ckks_encode_bounded");
+    } else {
+        check_status(he_ckks_encode_batch(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
+                                          batch.get(), 2 * L, ws.get(), st),
+                     "he_ckks_encode_batch");
+        std::vector<double> maxima(items);
+        check_status(he_memcpy_d2h(maxima.data(), ws.get(), items * sizeof(double), st), "download");
+        for (double max_coeff : maxima) {
+            const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
+            if (max_coeff_bit_count >= total_bits || max_coeff_bit_count > 63)
+                throw std::invalid_argument("encoded values are too large");
+        }
     }
     DeviceBuffer ews(he_encrypt_batch_workspace_words(h, L, (uint32_t)items));
     check_status(he_encrypt_batch(h, L, (uint32_t)items, pk.pk_.data(), context.prng_key(), context.next_stream(3 * items),
@@ -144,29 +156,27 @@ void CAHELGPUCKKSEncoder::encode_complex(const CAHELGPUContext &context, const d
     const uint32_t limbs = (uint32_t)context.limbs_at(chain_index);
     destination.resize(limbs, n);
     he_context *h = context.handle();
-    DeviceBuffer ws(he_ckks_workspace_words(h, limbs));
-    DeviceBuffer staging(2 * ss);  // the values, real parts then imaginary parts
-    double *d_re = reinterpret_cast<double *>(staging.get());
-    double *d_im = im ? d_re + ss : nullptr;
-    if (count) {
-        // (through page-locked memory, without waiting: the download of the largest coefficient below is the wait)
-        double *host = pinned_stage((im ? 2 : 1) * count * sizeof(double));
-        std::memcpy(host, re, count * sizeof(double));
-        check_status(he_memcpy_h2d_async(d_re, host, count * sizeof(double), context.stream()), "upload");
-        if (im) {
-            std::memcpy(host + count, im, count * sizeof(double));
-            check_status(he_memcpy_h2d_async(d_im, host + count, count * sizeof(double), context.stream()), "upload");
-        }
+    he_stream st = context.stream();
+    DeviceBuffer ws(he_ckks_encode_batch_workspace_words(h, 1));
+    // the values, real parts then imaginary parts, in page-locked memory that the first kernel reads where it is
+    PinnedRing &ring = PinnedRing::of_thread();
+    double *host_re = static_cast<double *>(ring.take(2 * ss * sizeof(double))), *host_im = im ? host_re + ss : nullptr;
+    double sum = copy_sum(host_re, re, count);
+    if (im) sum += copy_sum(host_im, im, count);
+    if (surely_small(sum, scale, ss, total_bits)) {
+        const int status = he_ckks_encode_bounded(h, host_re, host_im, (uint32_t)count, (uint32_t)ss, scale, limbs, 1, count,
+                                                  destination.data(), limbs, ws.get(), st);
+        ring.fence(st);
+        check_status(status, "he_ckks_encode_bounded");
+    } else {
+        const int status = he_ckks_encode(h, host_re, host_im, (uint32_t)count, (uint32_t)ss, scale, limbs, destination.data(),
+                                          ws.get(), st);
+        ring.fence(st);
+        check_status(status, "he_ckks_encode");
+        double max_coeff = 0.0;
+        check_status(he_memcpy_d2h(&max_coeff, ws.get(), sizeof(double), st), "download");
+        check_largest(max_coeff, total_bits);
     }
-    check_status(he_ckks_encode(h, d_re, d_im, (uint32_t)count, (uint32_t)ss, scale, limbs, destination.data(),
-                                ws.get(), context.stream()),
-                 "he_ckks_encode");
-    double max_coeff = 0.0;
-    check_status(he_memcpy_d2h(&max_coeff, ws.get(), sizeof(double), context.stream()), "download");
-    const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
-    if (max_coeff_bit_count >= total_bits) throw std::invalid_argument("encoded values are too large");
-    if (max_coeff_bit_count > 63)
-        throw std::invalid_argument("encoded values are too large: coefficients above 2^62 are not supported");
     destination.chain_index() = chain_index;
     destination.scale() = scale;
     destination.parms_id() = context.parms_id_at(chain_index);
@@ -181,15 +191,9 @@ void CAHELGPUCKKSEncoder::encode(const CAHELGPUContext &context, const std::vect
 // the first `count` complex values of the decoding, interleaved (re, im), into v
 void CAHELGPUCKKSEncoder::decode_values(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain,
                                         std::size_t count, std::vector<double> &v) {
-    if (!plain.is_ntt_form()) throw std::invalid_argument("plain is not in NTT form");
+    count = decode_count(context, plain, count);
     const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
-    if (limbs == 0 || !plain.data()) throw std::invalid_argument("plain is empty");
-    const int total_bits = context.total_coeff_modulus_bit_count(plain.chain_index());
-    if (plain.scale() <= 0 || (static_cast<int>(std::log2(plain.scale())) >= total_bits))
-        throw std::invalid_argument("scale out of bounds");
-    if (sparse_slots_ == 0) sparse_slots_ = slots_;   // as the reference: decoding first fixes the full slot count
     const std::size_t ss = sparse_slots_;
-    if (count == 0 || count > ss) count = ss;
 
     he_context *h = context.handle();
     DeviceBuffer ws(he_ckks_workspace_words(h, limbs));
@@ -214,16 +218,39 @@ void CAHELGPUCKKSEncoder::decode_complex(const CAHELGPUContext &context, const C
     }
 }
 
+std::size_t CAHELGPUCKKSEncoder::decode_count(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count) {
+    if (!plain.is_ntt_form()) throw std::invalid_argument("plain is not in NTT form");
+    if (plain.coeff_modulus_size() == 0 || !plain.data()) throw std::invalid_argument("plain is empty");
+    const int total_bits = context.total_coeff_modulus_bit_count(plain.chain_index());
+    if (plain.scale() <= 0 || (static_cast<int>(std::log2(plain.scale())) >= total_bits))
+        throw std::invalid_argument("scale out of bounds");
+    if (sparse_slots_ == 0) sparse_slots_ = slots_;   // as the reference: decoding first fixes the full slot count
+    return count == 0 || count > sparse_slots_ ? sparse_slots_ : count;
+}
+
+// the real parts of the first `count` values (decode_count's answer) to `destination`; the last kernel writes them to
+// page-locked memory
+void CAHELGPUCKKSEncoder::decode_real(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count,
+                                      double *destination) {
+    he_context *h = context.handle();
+    const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
+    DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)sparse_slots_));
+    double *host = static_cast<double *>(PinnedRing::of_thread().take(count * sizeof(double)));
+    check_status(he_ckks_decode_real(h, plain.data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
+                                     context.stream()),
+                 "he_ckks_decode_real");
+    check_status(he_stream_synchronize(context.stream()), "synchronisation failed");
+    std::memcpy(destination, host, count * sizeof(double));
+}
+
 void CAHELGPUCKKSEncoder::decode_prefix(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain,
                                         std::size_t count, std::vector<double> &destination) {
-    std::vector<double> v;
-    decode_values(context, plain, count, v);
-    destination.resize(v.size() / 2);
-    for (std::size_t i = 0; i < destination.size(); i++) destination[i] = v[2 * i];
+    count = decode_count(context, plain, count);
+    destination.resize(count);
+    decode_real(context, plain, count, destination.data());
 }
 
 void CAHELGPUCKKSEncoder::decode(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain,
                                  std::vector<double> &destination) {
-    std::vector<double> im;
-    decode_complex(context, plain, destination, im);
+    decode_prefix(context, plain, 0, destination);
 }

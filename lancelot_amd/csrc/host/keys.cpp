@@ -4,9 +4,11 @@
 // ckks_decrypt :594-654).  Randomness comes from the context's seeded ChaCha20 streams, one stream id per
 // sampled polynomial, handed out in the order the polynomials are drawn.
 #include <cmath>
+#include <cstring>
 #include <string>
 
 #include "cahel.h"
+#include "staging.h"
 
 using namespace cahel;
 
@@ -177,15 +179,13 @@ void CAHELGPUPublicKey::encrypt_asymmetric(const CAHELGPUContext &context, const
         check_status(he_add(h, cipher.data(), plain.data(), cipher.data(), 1, limbs, 0, st), "he_add");
     } else {
         // encrypt over Ql u P, then divide by P (ModDown) onto the L limbs of the plaintext's level: the batched
-        // pipeline with one item (u, e0, e1 from the next three stream ids; the plaintext lies in polynomial 0 and the
-        // division adds onto it)
+        // pipeline with one item (u, e0, e1 from the next three stream ids; the division adds onto the plaintext)
         const uint32_t L = (uint32_t)context.limbs_at(chain);
         cipher.resize(context, chain, 2);
-        check_status(he_memcpy_d2d(cipher.data(), plain.data(), (std::size_t)L * n * sizeof(uint64_t), st), "copy");
         DeviceBuffer ws(he_encrypt_batch_workspace_words(h, L, 1));
-        check_status(he_encrypt_batch(h, L, 1, pk_.data(), context.prng_key(), context.next_stream(3), cipher.data(),
-                                      ws.get(), st),
-                     "he_encrypt_batch");
+        check_status(he_encrypt(h, L, plain.data(), pk_.data(), context.prng_key(), context.next_stream(3), cipher.data(),
+                                ws.get(), st),
+                     "he_encrypt");
     }
     cipher.is_ntt_form() = true;
     cipher.is_asymmetric() = true;
@@ -204,16 +204,24 @@ void CAHELGPUSecretKey::decrypt(const CAHELGPUContext &context, const CAHELGPUCi
     he_context *h = context.handle();
     he_stream st = context.stream();
     plain.resize(limbs, n);
-    // c0 + c1 s (+ c2 s^2 ...): the first product reads c0 directly
-    for (std::size_t i = 1; i <= needed; i++)
-        check_status(he_multiply_add(h, cipher.data() + i * poly, sk_powers_.get() + (i - 1) * sk_poly,
-                                     i == 1 ? cipher.data() : plain.data(), plain.data(), 1, limbs, 0, 0, st),
-                     "he_multiply_add");
-    if (noise_flooding_) {
-        DeviceBuffer noise(poly);
-        sample(context, 3, noise.get(), limbs, limbs, 0);
-        check_status(he_ntt_forward(h, noise.get(), 1, limbs, limbs, 0, limbs, 0, st), "he_ntt_forward");
-        check_status(he_add(h, plain.data(), noise.get(), plain.data(), 1, limbs, 0, st), "he_add");
+    if (noise_flooding_ && needed <= 2) {
+        DeviceBuffer noise(n / 8);
+        check_status(he_decrypt_flood(h, cipher.data(), (uint32_t)cipher.size(), limbs, sk_powers_.get(), sk_poly, context.prng_key(),
+                                      context.next_stream(), context.gauss_cdt(), context.gauss_cdt_len(), plain.data(), noise.get(),
+                                      st),
+                     "he_decrypt_flood");
+    } else {
+        // c0 + c1 s (+ c2 s^2 ...): the first product reads c0 directly
+        for (std::size_t i = 1; i <= needed; i++)
+            check_status(he_multiply_add(h, cipher.data() + i * poly, sk_powers_.get() + (i - 1) * sk_poly,
+                                         i == 1 ? cipher.data() : plain.data(), plain.data(), 1, limbs, 0, 0, st),
+                         "he_multiply_add");
+        if (noise_flooding_) {
+            DeviceBuffer noise(poly);
+            sample(context, 3, noise.get(), limbs, limbs, 0);
+            check_status(he_ntt_forward(h, noise.get(), 1, limbs, limbs, 0, limbs, 0, st), "he_ntt_forward");
+            check_status(he_add(h, plain.data(), noise.get(), plain.data(), 1, limbs, 0, st), "he_add");
+        }
     }
     plain.chain_index() = cipher.chain_index();
     plain.scale() = cipher.scale();
@@ -221,11 +229,10 @@ void CAHELGPUSecretKey::decrypt(const CAHELGPUContext &context, const CAHELGPUCi
     plain.is_ntt_form_ = true;
 }
 
-std::vector<double> CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context,
-                                                           const std::vector<const CAHELGPUCiphertext *> &ciphers,
-                                                           std::size_t slots, std::size_t count) {
+void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
+                                            std::size_t slots, std::size_t count, double *destination) {
     if (!gen_flag_) throw std::logic_error("secret key has not been generated");
-    if (ciphers.empty()) return {};
+    if (ciphers.empty()) return;
     if (ciphers.size() > 16384) throw std::invalid_argument("too many ciphertexts");
     const CAHELGPUCiphertext &first = *ciphers[0];
     for (const CAHELGPUCiphertext *ct : ciphers) {
@@ -242,28 +249,31 @@ std::vector<double> CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext
         throw std::invalid_argument("scale out of bounds");
     he_context *h = context.handle();
     he_stream st = context.stream();
-    std::vector<const uint64_t *> table;
-    for (const CAHELGPUCiphertext *ct : ciphers) table.push_back(ct->data());
+    // the table of the ciphertexts goes through page-locked memory without waiting; the values come back there, written by the
+    // last kernel, unless they would take more than a block of the ring
+    PinnedRing &ring = PinnedRing::of_thread();
+    const uint64_t **table = static_cast<const uint64_t **>(ring.take(items * sizeof(uint64_t)));
+    for (uint32_t k = 0; k < items; k++) table[k] = ciphers[k]->data();
     DeviceBuffer d_table(items);
-    check_status(he_memcpy_h2d(d_table.get(), table.data(), table.size() * sizeof(uint64_t), st), "upload");
-    DeviceBuffer noise;
-    if (noise_flooding_) {
-        // one flooding-noise polynomial per ciphertext, the stream ids that `items` calls of decrypt would draw
-        noise.allocate((std::size_t)items * limbs * n);
-        check_status(he_sample_batch(h, 3, context.prng_key(), context.next_stream(items), noise.get(), limbs, 0, limbs, 0,
-                                     context.gauss_cdt(), context.gauss_cdt_len(), items, st),
-                     "he_sample_batch");
-        check_status(he_ntt_forward(h, noise.get(), items, limbs, limbs, 0, limbs, 0, st), "he_ntt_forward");
+    const int status = he_memcpy_h2d_async(d_table.get(), table, items * sizeof(uint64_t), st);
+    ring.fence(st);
+    check_status(status, "upload");
+    const std::size_t bytes = (std::size_t)items * count * sizeof(double);
+    const bool staged = bytes <= PinnedRing::kMaxBytes;
+    DeviceBuffer ws(he_decrypt_decode_real_workspace_words(h, limbs, (uint32_t)slots, items)), d_out;
+    if (!staged) d_out.allocate((std::size_t)items * count);
+    double *out = staged ? static_cast<double *>(ring.take(bytes)) : reinterpret_cast<double *>(d_out.get());
+    // flooding noise: the stream ids that `items` calls of decrypt would draw
+    check_status(he_decrypt_decode_real_batch(h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs,
+                                              sk_powers_.get(), noise_flooding_ ? context.prng_key() : nullptr,
+                                              noise_flooding_ ? context.next_stream(items) : 0, context.gauss_cdt(),
+                                              context.gauss_cdt_len(), (uint32_t)slots, first.scale(), (uint32_t)count, out,
+                                              ws.get(), st),
+                 "he_decrypt_decode_real_batch");
+    if (staged) {
+        check_status(he_stream_synchronize(st), "synchronisation failed");
+        std::memcpy(destination, out, bytes);
+    } else {
+        check_status(he_memcpy_d2h(destination, out, bytes, st), "download");
     }
-    DeviceBuffer ws(he_decrypt_decode_batch_workspace_words(h, limbs, (uint32_t)slots, items));
-    DeviceBuffer out(2 * (std::size_t)items * count);
-    check_status(he_decrypt_decode_batch(h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs,
-                                         sk_powers_.get(), noise.get(), (uint32_t)slots, first.scale(), (uint32_t)count,
-                                         reinterpret_cast<double *>(out.get()), ws.get(), st),
-                 "he_decrypt_decode_batch");
-    std::vector<double> v(2 * (std::size_t)items * count);
-    check_status(he_memcpy_d2h(v.data(), out.get(), v.size() * sizeof(double), st), "download");
-    std::vector<double> re((std::size_t)items * count);
-    for (std::size_t i = 0; i < re.size(); i++) re[i] = v[2 * i];
-    return re;
 }

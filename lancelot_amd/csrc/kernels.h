@@ -81,6 +81,13 @@ enum : int {
     // in map mode; bit t of pro_src_fp_mask says whether the blocks pass of table t ran on the FP64 back end.  The
     // inverse transform's scaling must be N^-1 alone (digits of one limb each).
     NTT_PRO_SOURCE_INTT_REDUCE = 9,
+    // forward prologue: small signed coefficients, one byte each: polynomial p at (const int8_t *)pro_src + p * N, the same
+    // for every limb (sampled polynomials: their residues are never stored)
+    NTT_PRO_SMALL = 10,
+    // forward prologue of an encoding: coefficient c of polynomial p is round(x * pro_fix) for the real (c < N/2) or
+    // imaginary part x of value (c mod N/2) / gap of the transformed slot vector (const double2 *)pro_src + p * 2^pro_log_slots,
+    // which holds value i at bitrev(i); 0 where gap does not divide c.  Magnitudes below 2^62.
+    NTT_PRO_ROUND = 11,
 };
 
 struct NttArgs {
@@ -111,6 +118,8 @@ struct NttArgs {
     size_t pro_item_stride;   // NTT_PRO_SOURCE_REDUCE in list mode: words between the sources of consecutive items
     uint32_t pro_lk;          // ... and limbs per digit of the list's buffer (L + K)
     uint32_t pro_src_table;   // NTT_PRO_SOURCE_INTT_REDUCE in map mode: table of the source limb
+    double pro_fix;           // NTT_PRO_ROUND: scale / slots
+    uint32_t pro_log_slots;
     uint64_t pro_src_fp_mask; // NTT_PRO_SOURCE_INTT_REDUCE: tables whose inverse blocks pass left FP64 lazy words
     const uint64_t *pro_itw;  // ... and the inverse transform's twiddle tables (laid out like tw and tw_fp)
     const double *pro_itw_fp;
@@ -340,6 +349,24 @@ struct KsFuseArgs {
 };
 hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s);
 
+// Blocks pass of the transforms of an encryption fused with its products: a.out holds the words that the rows pass left for
+// u [items][L+K][N] and, behind it, e0, e1 [items][2][L+K][N] (the polynomials of a.map, 3 * items of them);
+// e_i + u pk_i replaces e_i.  Limbs t >= L leave as the lazy words of their inverse blocks pass (a.pro_itw / pro_itw_fp), the
+// others as canonical residues.
+hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
+                                 int backend, hipStream_t s);
+
+// Blocks pass of the flooding noise's transform fused with a decryption: a.out [items][limbs][N] holds the words that the
+// rows pass left; c0 + sum_i c_i s^i of the ciphertext is added to them (sizes 2 and 3).
+struct DecryptArgs {
+    const uint64_t *ct;               // [size][limbs][N], or
+    const uint64_t *const *cts;       // a device pointer table of `items` such ciphertexts
+    const uint64_t *sk;               // s at sk, s^2 at sk + sk_stride
+    size_t sk_stride;
+    uint32_t size;
+};
+hipError_t launch_decrypt_blocks(const NttArgs &a, const DecryptArgs &d, uint32_t items, int backend, hipStream_t s);
+
 hipError_t launch_decompose_real(const Tables &t, const double *coeffs, uint64_t *out, uint32_t limbs, uint32_t first,
                                  uint32_t items, size_t out_item_stride, hipStream_t s);
 
@@ -352,13 +379,12 @@ struct ChaChaKey {
 hipError_t launch_sample(const Tables &t, int kind, ChaChaKey key, uint64_t stream_id, uint64_t *out, LimbMap map,
                          const uint64_t *cdt, uint32_t cdt_len, uint32_t items, uint32_t stream_stride,
                          size_t out_item_stride, hipStream_t s);
-// u, e0, e1 of `items` public-key encryptions in one launch: out = [items] ternary polynomials, then [items][2]
-// error polynomials, poly_stride words apart; item k draws from the streams stream_id + 3 k, + 1, + 2
-hipError_t launch_sample_encrypt(const Tables &t, ChaChaKey key, uint64_t stream_id, uint64_t *out, LimbMap map,
-                                 uint32_t items, size_t poly_stride, hipStream_t s);
-// wide [items][2][L+K][N] += u [items][L+K][N] * pk [2][size_q+K][N] (both polynomials of the public key)
-hipError_t launch_encrypt_fma(const Tables &t, const uint64_t *u, const uint64_t *pk, uint64_t *wide, uint32_t L,
-                              uint32_t K, uint32_t size_q, uint32_t items, hipStream_t s);
+// The same polynomials as one signed byte per coefficient, out [polys][N] (NTT_PRO_SMALL makes their residues): u of every
+// item of `items` public-key encryptions, then its e0, e1 (item k draws from the streams stream_id + 3 k, + 1, + 2) ...
+hipError_t launch_sample_encrypt(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, uint32_t items, hipStream_t s);
+// ... or the discrete Gaussian by the cumulative table cdt (at most 128 entries), item k from stream_id + k
+hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, const uint64_t *cdt,
+                                     uint32_t cdt_len, uint32_t items, hipStream_t s);
 
 // CKKS encoder tables: 5^j mod 2N for j < N/2 and e^{2 pi i k / 2N} for k <= 2N.
 struct FftTables {
@@ -374,12 +400,29 @@ hipError_t launch_ckks_encode(const FftTables &t, const double *re, const double
                               double scale, double2 *v, double *coeffs, uint64_t *max_bits, uint32_t items,
                               size_t value_stride, hipStream_t s, const Tables *tab = nullptr, uint64_t *out = nullptr,
                               uint32_t limbs = 0, size_t out_item_stride = 0);
+// Only the transform: the slot vectors stay in v [items][slots] for NTT_PRO_ROUND.  re / im may be page-locked host memory.
+hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
+                                   double2 *v, uint32_t items, size_t value_stride, hipStream_t s);
 // res: [limbs][N] coefficient-form residues of the first `limbs` primes -> v: `slots` complex values.
 // garner_inv[i * stride + j] = q_j^-1 mod q_i for j < i.
 // items: that many dense plaintexts res [items][limbs][N] -> v [items][slots].
 hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs,
                               uint32_t slots, double scale, const uint64_t *garner_inv, uint32_t garner_stride,
                               double2 *v, uint32_t items, hipStream_t s);
+// The same from plaintexts in NTT form that have been through their inverse blocks pass (inv: the inverse transform's
+// arguments, map = the limbs, in = the lazy words), real parts of the first `count` values only, to re [items][count] (device
+// or page-locked host memory): the inverse rows pass of all limbs and the composition are one kernel.  2^12 <= N <= 2^16,
+// at most 4 limbs.
+hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int backend, uint32_t slots, double scale,
+                                   const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items, double *re,
+                                   uint32_t count, hipStream_t s);
+// the forward transform of v and the real parts of the first `count` values, for the other cases
+hipError_t launch_ckks_fft_real(const FftTables &t, uint32_t slots, double2 *v, uint32_t items, double *re, uint32_t count,
+                                hipStream_t s);
+// only the composition of launch_ckks_decode
+hipError_t launch_ckks_compose(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs, uint32_t slots,
+                               double scale, const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items,
+                               hipStream_t s);
 // out [items][count] = the first `count` values of every v [items][slots]
 hipError_t launch_take_slots(const double2 *v, uint32_t slots, uint32_t items, uint32_t count, double2 *out, hipStream_t s);
 // out [items][limbs][N] = c0 + c1 * s (+ noise [items][limbs][N]) for the size-2 ciphertexts [2][limbs][N] named by the

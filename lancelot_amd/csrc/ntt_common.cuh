@@ -90,6 +90,16 @@ __device__ __forceinline__ FpTw inverse_scale(const NttArgs &a, const Job &job, 
     return FpTw{w, w * m.qinv};
 }
 
+// coefficient at `at` of polynomial job.poly of an encoding, rounded (NTT_PRO_ROUND)
+__device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Job &job, uint32_t at) {
+    const uint32_t half = 1u << (a.log_n - 1), log_gap = a.log_n - 1 - a.pro_log_slots;
+    const uint32_t k = at & (half - 1);
+    if (k & ((1u << log_gap) - 1)) return 0.0;
+    const double *v = reinterpret_cast<const double *>(a.pro_src) + ((size_t)job.poly << (a.pro_log_slots + 1));
+    const uint32_t slot = __brev(k >> log_gap) >> (32 - a.pro_log_slots);
+    return round(v[2 * slot + (at >= half ? 1 : 0)] * a.pro_fix);
+}
+
 // Input of a forward rows pass (a.pro_mode): word j of the thread from global offset glob(j) of its limb, as exact
 // doubles; returns whether they have to be reduced before the first stage (else they are canonical).
 template <int W, typename Glob>
@@ -124,6 +134,14 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(barrett64(job.src[glob(j)], q, r1));
+    } else if (a.pro_mode == NTT_PRO_SMALL) {
+        const int8_t *src = reinterpret_cast<const int8_t *>(a.pro_src) + ((size_t)job.poly << a.log_n);
+#pragma unroll
+        for (int j = 0; j < W; j++) v[j] = (double)src[glob(j)];
+    } else if (a.pro_mode == NTT_PRO_ROUND) {
+        // (an integer below 2^62 in magnitude: the quotient estimate is off by at most 1, the fused multiply-add exact)
+#pragma unroll
+        for (int j = 0; j < W; j++) v[j] = fp_reduce(rounded_coefficient(a, job, (uint32_t)glob(j)), c.m);
     } else {
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(job.in[glob(j)]);
@@ -153,6 +171,21 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
             const uint64_t dj = a.pro_k1 ? barrett64(ds, q, r1) : job.in[glob(j)];
             const uint64_t r = sub_mod(tsrc[glob(j)], mul_shoup(dl, wlast, ql), ql);
             v[j] = add_mod(mul_shoup(dj, w, q), barrett64(r, q, r1), q);
+        }
+    } else if (a.pro_mode == NTT_PRO_SMALL) {
+        const int8_t *src = reinterpret_cast<const int8_t *>(a.pro_src) + ((size_t)job.poly << a.log_n);
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const int64_t x = src[glob(j)];
+            v[j] = (uint64_t)x + (x < 0 ? q : 0);
+        }
+    } else if (a.pro_mode == NTT_PRO_ROUND) {
+        const uint64_t r1 = a.barrett[2 * job.table + 1];
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const double x = rounded_coefficient(a, job, (uint32_t)glob(j));
+            const uint64_t r = barrett64((uint64_t)fabs(x), q, r1);
+            v[j] = x < 0 ? neg_mod(r, q) : r;
         }
     } else {
 #pragma unroll

@@ -621,6 +621,148 @@ __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(Nt
     }
 }
 
+// a word that the forward stages have left (lazy) as a canonical residue, and a canonical word as the arithmetic's value
+__device__ __forceinline__ uint64_t canonical_word(double v, const FpArith &ar) { return fp_to_u64(fp_canonical(v, ar.m)); }
+__device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &ar) { return reduce_4q(v, ar.m.q); }
+
+// v + x * y mod q for canonical words x, y and v as the forward stages have left it; canonical
+__device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y, const FpArith &ar, uint64_t, uint64_t) {
+    const double w = fp_from_u64(y);
+    return fp_to_u64(fp_canonical(v + fp_mulmod(fp_from_u64(x), FpTw{w, w * ar.m.qinv}, ar.m), ar.m));
+}
+__device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t y, const IntArith &ar, uint64_t r0, uint64_t r1) {
+    return add_mod(reduce_4q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
+}
+
+// Encryption: a wave takes its block of u, e0 and e1 of one limb through the last 8 stages, adds u pk_i to e_i and stores
+// the sums; a special limb's go through the inverse blocks pass first (ModDown follows).  The transformed u never reaches memory.
+template <class A>
+__device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t LK, uint32_t size_qp, uint32_t t,
+                                              uint32_t table, uint32_t blk, uint32_t item, uint32_t items, uint32_t lane, const A &ar,
+                                              uint64_t *lds) {
+    using T4 = Tile4<8, 8>;
+    constexpr bool FP = std::is_same<A, FpArith>::value;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const uint64_t r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+    uint64_t *poly[3] = {a.out + ((size_t)item * LK + t) * n, a.out + ((size_t)(items + 2 * item) * LK + t) * n,
+                         a.out + ((size_t)(items + 2 * item + 1) * LK + t) * n};
+    uint64_t x[3][4], k[2][4], u[4];
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[i][j] = poly[i][off + T4::word(0, lane, j)];
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    load4(k[0], pk + (size_t)table * n + at);
+    load4(k[1], pk + (size_t)(size_qp + table) * n + at);
+    typename A::V v[3][4];
+#pragma unroll
+    for (int i = 0; i < 3; i++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[i][j] = A::from_word(x[i][j]);
+        ar.reduce(v[i]);
+        T4::template forward<A>(v[i], tw, ar, lds, lane);
+        wave_sync();
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) u[j] = canonical_word(v[0][j], ar);
+    A iar = ar;
+    if (t >= L) {
+        if constexpr (FP)
+            iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
+        else
+            iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
+        T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; i++) {
+        uint64_t o[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] = add_product(v[1 + i][j], u[j], k[i][j], ar, r0, r1);
+        if (t >= L) {
+            typename A::V w[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (FP)
+                    w[j] = fp_from_u64(o[j]);
+                else
+                    w[j] = o[j];
+            }
+            T4::template inverse<A>(w, tw, iar, lds, lane);
+#pragma unroll
+            for (int j = 0; j < 4; j++) poly[1 + i][off + T4::word(0, lane, j)] = A::to_word(w[j]);
+            wave_sync();
+        } else {
+            store4(poly[1 + i] + at, o);
+        }
+    }
+}
+
+template <int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
+                                                                          uint32_t items) {
+    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1), it = id >> lr;
+    const uint32_t item = it / LK, t = it - item * LK, table = t < L ? t : size_q + (t - L);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
+    if (BE != NTT_BACKEND_INT && fp)
+        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, lane, fp_arith(a, table), lds_all[w]);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, lane, int_arith(a, table), lds_all[w]);
+    }
+}
+
+// Decryption: the flooding noise's block through the last 8 stages, plus c0 + c1 s [+ c2 s^2].
+template <class A>
+__device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArgs &d, const Job &job, uint32_t blk, uint32_t lane,
+                                              const A &ar, uint64_t *lds) {
+    using T4 = Tile4<8, 8>;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane, poly = (size_t)a.map.limbs * n;
+    const uint64_t q = a.moduli[job.table], r0 = a.barrett[2 * job.table], r1 = a.barrett[2 * job.table + 1];
+    const uint64_t *ct = (d.cts ? d.cts[job.poly] : d.ct) + job.limb * n + at;
+    const uint64_t *sk = d.sk + job.limb * n + at;
+    uint64_t x[4], c0[4], c1[4], s1[4], c2[4], s2[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) x[j] = job.out[off + T4::word(0, lane, j)];
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    load4(c0, ct);
+    load4(c1, ct + poly);
+    load4(s1, sk);
+    if (d.size > 2) {
+        load4(c2, ct + 2 * poly);
+        load4(s2, sk + d.sk_stride);
+    }
+    typename A::V v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
+    ar.reduce(v);
+    T4::template forward<A>(v, tw, ar, lds, lane);
+    uint64_t o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        o[j] = add_mod(add_product(v[j], c1[j], s1[j], ar, r0, r1), c0[j], q);
+        if (d.size > 2) o[j] = add_mod(o[j], mul_mod(c2[j], s2[j], q, r0, r1), q);
+    }
+    store4(job.out + at, o);
+}
+
+template <int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArgs a, DecryptArgs d) {
+    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const Job job = decode_job(a, id >> lr);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) decrypt_block(a, d, job, blk, lane, fp_arith(a, job.table), lds_all[w]);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) decrypt_block(a, d, job, blk, lane, int_arith(a, job.table), lds_all[w]);
+    }
+}
+
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
@@ -753,6 +895,35 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
     else
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
+    return hipGetLastError();
+}
+
+hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
+                                 int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17 || items == 0) return hipErrorInvalidValue;
+    const uint64_t wgs = ((uint64_t)(L + K) * items << (a.log_n - 8)) / kBlockWaves;
+    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    if (backend == NTT_BACKEND_MIXED)
+        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, pk, L, K, size_q, items);
+    else if (backend)
+        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, pk, L, K, size_q, items);
+    else
+        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, pk, L, K, size_q, items);
+    return hipGetLastError();
+}
+
+hipError_t launch_decrypt_blocks(const NttArgs &a, const DecryptArgs &d, uint32_t items, int backend, hipStream_t s) {
+    if (a.log_n < 9 || a.log_n > 17 || a.jobs || items == 0 || d.size < 2 || d.size > 3) return hipErrorInvalidValue;
+    const uint64_t wgs = ((uint64_t)a.map.limbs * items << (a.log_n - 8)) / kBlockWaves;
+    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    if (backend == NTT_BACKEND_MIXED)
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, d);
+    else if (backend)
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, d);
+    else
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, d);
     return hipGetLastError();
 }
 

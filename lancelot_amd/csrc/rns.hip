@@ -72,24 +72,6 @@ __global__ __launch_bounds__(kThreads) void decompose_real_kernel(const double *
     out[blockIdx.z * out_item_stride + ((size_t)blockIdx.y << log_n) + i] = c < 0 ? neg_mod(r, q) : r;
 }
 
-// grid: (N / 256, L + K, items).  wide[item][i][t] += u[item][t] * pk[i][table(t)] for both polynomials of the public
-// key: the products of an encryption over Ql u P
-__global__ __launch_bounds__(kThreads) void encrypt_fma_kernel(const uint64_t *u, const uint64_t *pk, uint64_t *wide,
-                                                               const uint64_t *moduli, const uint64_t *barrett,
-                                                               uint32_t L, uint32_t K, uint32_t size_q, uint32_t log_n) {
-    const uint32_t t = blockIdx.y, LK = L + K;
-    const uint32_t table = t < L ? t : size_q + (t - L);
-    const uint64_t q = moduli[table], r0 = barrett[2 * table], r1 = barrett[2 * table + 1];
-    const uint32_t j = blockIdx.x * kThreads + threadIdx.x;
-    const uint64_t uv = u[(((size_t)blockIdx.z * LK + t) << log_n) + j];
-    const size_t key_poly = (size_t)(size_q + K) << log_n;
-    const uint64_t *k = pk + ((size_t)table << log_n) + j;
-    uint64_t *w = wide + (((size_t)blockIdx.z * 2 * LK + t) << log_n) + j;
-    const size_t wpoly = (size_t)LK << log_n;
-    w[0] = add_mod(w[0], mul_mod(uv, k[0], q, r0, r1), q);
-    w[wpoly] = add_mod(w[wpoly], mul_mod(uv, k[key_poly], q, r0, r1), q);
-}
-
 struct TensorArgs {
     const uint64_t *ct1, *ct2;
     uint64_t *out;
@@ -741,6 +723,19 @@ struct SampleArgs {
     size_t out_item_stride;
 };
 
+// the first entry of the cumulative table above u (the table ascends)
+__device__ __forceinline__ uint32_t cdt_magnitude(const uint64_t *cdt, uint32_t len, uint64_t u) {
+    uint32_t lo = 0, hi = len;
+    while (lo < hi) {
+        const uint32_t mid = (lo + hi) >> 1;
+        if (u >= cdt[mid])
+            lo = mid + 1;
+        else
+            hi = mid;
+    }
+    return lo;
+}
+
 // ternary / error / gauss: one thread = one ChaCha block = 16 (ternary) or 8 coefficients, the same
 // signed value written to every limb.  uniform: one thread = one block = 4 residues of one limb.
 // KIND is a template parameter so that the loops over the block's words unroll and the words stay in registers (with
@@ -779,15 +774,10 @@ __global__ __launch_bounds__(kThreads) void sample_kernel(SampleArgs p) {
     sample_signed<KIND>(p, b, stream, out);
 }
 
-// ternary / error / gauss coefficients of ChaCha block b of `stream`, the same signed value to every limb of `out`
+// the signed coefficients of one ChaCha block (16 words w)
 template <int KIND>
-__device__ __forceinline__ void sample_signed(const SampleArgs &p, uint32_t b, uint64_t stream, uint64_t *out) {
-    const uint32_t n = 1u << p.log_n;
-    uint32_t w[16];
+__device__ __forceinline__ void signed_values(int *v, const uint32_t *w, const uint64_t *cdt, uint32_t cdt_len) {
     constexpr int per_block = KIND == SAMPLE_TERNARY ? 16 : 8;
-    if (b >= n / per_block) return;
-    chacha20_block(p.key, b, stream, w);
-    int v[per_block];
 #pragma unroll
     for (int e = 0; e < per_block; e++) {
         if (KIND == SAMPLE_TERNARY) {
@@ -798,11 +788,22 @@ __device__ __forceinline__ void sample_signed(const SampleArgs &p, uint32_t b, u
             uint64_t u = ((uint64_t)w[2 * e + 1] << 32) | w[2 * e];
             const bool neg = u >> 63;
             u &= 0x7FFFFFFFFFFFFFFFull;
-            uint32_t mag = 0;
-            while (mag < p.cdt_len && u >= p.cdt[mag]) mag++;
+            const uint32_t mag = cdt_magnitude(cdt, cdt_len, u);
             v[e] = neg ? -(int)mag : (int)mag;
         }
     }
+}
+
+// ternary / error / gauss coefficients of ChaCha block b of `stream`, the same signed value to every limb of `out`
+template <int KIND>
+__device__ __forceinline__ void sample_signed(const SampleArgs &p, uint32_t b, uint64_t stream, uint64_t *out) {
+    const uint32_t n = 1u << p.log_n;
+    uint32_t w[16];
+    constexpr int per_block = KIND == SAMPLE_TERNARY ? 16 : 8;
+    if (b >= n / per_block) return;
+    chacha20_block(p.key, b, stream, w);
+    int v[per_block];
+    signed_values<KIND>(v, w, p.cdt, p.cdt_len);
     for (uint32_t limb = 0; limb < p.map.limbs; limb++) {
         const uint64_t q = p.moduli[map_table(p.map, limb)];
         ulonglong2 *dst = reinterpret_cast<ulonglong2 *>(out + ((size_t)limb << p.log_n) + (size_t)per_block * b);
@@ -813,18 +814,53 @@ __device__ __forceinline__ void sample_signed(const SampleArgs &p, uint32_t b, u
     }
 }
 
-// The three polynomials of `items` public-key encryptions in one launch: out holds [items] ternary polynomials u and
-// behind them [items][2] error polynomials (e0, e1), all out_item_stride words apart; item k draws u, e0, e1 from the
-// streams p.stream + 3 k, + 1, + 2.  blockIdx.y = polynomial, blockIdx.z = 0.
-__global__ __launch_bounds__(kThreads) void sample_encrypt_kernel(SampleArgs p, uint32_t items) {
-    const uint32_t b = blockIdx.x * kThreads + threadIdx.x, y = blockIdx.y;
-    uint64_t *out = p.out + y * p.out_item_stride;
-    if (y < items) {
-        sample_signed<SAMPLE_TERNARY>(p, b, p.stream + 3 * (uint64_t)y, out);
+// Sampled polynomials as one signed byte per coefficient (the residues are made where the transform reads them: a launch
+// that wrote them for every limb took 12 us for u, e0, e1 of one encryption and 16 us for one noise polynomial; its threads, one per
+// ChaCha block, had 8 to 16 words to store per limb and the table of the Gaussian to walk in memory, which is in LDS here).
+// One wave per workgroup: a polynomial has at most 8,192 blocks.
+struct SmallArgs {
+    int8_t *out;
+    const uint64_t *cdt;
+    ChaChaKey key;
+    uint64_t stream;
+    uint32_t log_n, cdt_len, items;
+};
+constexpr int kSmallThreads = 64;
+constexpr uint32_t kSmallCdt = 128;
+
+template <int KIND>
+__device__ __forceinline__ void sample_bytes(const SmallArgs &p, uint64_t stream, int8_t *out, const uint64_t *cdt) {
+    constexpr int per_block = KIND == SAMPLE_TERNARY ? 16 : 8;
+    const uint32_t b = blockIdx.x * kSmallThreads + threadIdx.x;
+    if (b >= (1u << p.log_n) / per_block) return;
+    uint32_t w[16];
+    chacha20_block(p.key, b, stream, w);
+    int v[per_block];
+    signed_values<KIND>(v, w, cdt, p.cdt_len);
+    uint32_t *dst = reinterpret_cast<uint32_t *>(out + (size_t)per_block * b);
+#pragma unroll
+    for (int e = 0; e < per_block; e += 4)
+        dst[e / 4] = (uint32_t)(v[e] & 255) | ((uint32_t)(v[e + 1] & 255) << 8) | ((uint32_t)(v[e + 2] & 255) << 16) | ((uint32_t)(v[e + 3] & 255) << 24);
+}
+
+// u of every item, then e0, e1 of every item; blockIdx.y = polynomial
+__global__ __launch_bounds__(kSmallThreads) void sample_encrypt_kernel(SmallArgs p) {
+    const uint32_t y = blockIdx.y;
+    int8_t *out = p.out + ((size_t)y << p.log_n);
+    if (y < p.items) {
+        sample_bytes<SAMPLE_TERNARY>(p, p.stream + 3 * (uint64_t)y, out, nullptr);
     } else {
-        const uint32_t e = y - items;
-        sample_signed<SAMPLE_ERROR>(p, b, p.stream + 3 * (uint64_t)(e >> 1) + 1 + (e & 1), out);
+        const uint32_t e = y - p.items;
+        sample_bytes<SAMPLE_ERROR>(p, p.stream + 3 * (uint64_t)(e >> 1) + 1 + (e & 1), out, nullptr);
     }
+}
+
+// blockIdx.y = item
+__global__ __launch_bounds__(kSmallThreads) void sample_gauss_small_kernel(SmallArgs p) {
+    __shared__ uint64_t cdt[kSmallCdt];
+    for (uint32_t i = threadIdx.x; i < p.cdt_len; i += kSmallThreads) cdt[i] = p.cdt[i];
+    __syncthreads();
+    sample_bytes<SAMPLE_GAUSS>(p, p.stream + blockIdx.y, p.out + ((size_t)blockIdx.y << p.log_n), cdt);
 }
 
 }  // namespace
@@ -851,14 +887,6 @@ hipError_t launch_decompose_real(const Tables &t, const double *coeffs, uint64_t
     if (items > 65535) return hipErrorInvalidValue;
     hipLaunchKernelGGL(decompose_real_kernel, dim3((1u << t.log_n) / kThreads, limbs, items), dim3(kThreads), 0, s, coeffs,
                        out, t.moduli, t.barrett, first, t.log_n, out_item_stride);
-    return hipGetLastError();
-}
-
-hipError_t launch_encrypt_fma(const Tables &t, const uint64_t *u, const uint64_t *pk, uint64_t *wide, uint32_t L,
-                              uint32_t K, uint32_t size_q, uint32_t items, hipStream_t s) {
-    if (items == 0 || items > 65535) return hipErrorInvalidValue;
-    hipLaunchKernelGGL(encrypt_fma_kernel, dim3((1u << t.log_n) / kThreads, L + K, items), dim3(kThreads), 0, s, u, pk, wide,
-                       t.moduli, t.barrett, L, K, size_q, t.log_n);
     return hipGetLastError();
 }
 
@@ -1146,16 +1174,21 @@ hipError_t launch_sample(const Tables &t, int kind, ChaChaKey key, uint64_t stre
     return hipGetLastError();
 }
 
-hipError_t launch_sample_encrypt(const Tables &t, ChaChaKey key, uint64_t stream_id, uint64_t *out, LimbMap map,
-                                 uint32_t items, size_t poly_stride, hipStream_t s) {
-    if (items == 0 || 3 * (uint64_t)items > 65535) return hipErrorInvalidValue;
-    if ((reinterpret_cast<uintptr_t>(out) & 15) || (poly_stride & 1)) return hipErrorInvalidValue;
-    const uint32_t n = 1u << t.log_n;
-    SampleArgs p{out, t.moduli, t.barrett, nullptr, key, stream_id, map, t.log_n, 0, SAMPLE_ERROR, 0, poly_stride};
-    // (a ChaCha block yields 16 ternary or 8 error coefficients: the grid covers the error polynomials, the surplus
-    // threads of the ternary ones leave at once)
-    const dim3 grid((n / 8 + kThreads - 1) / kThreads, 3 * items);
-    hipLaunchKernelGGL(sample_encrypt_kernel, grid, dim3(kThreads), 0, s, p, items);
+hipError_t launch_sample_encrypt(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, uint32_t items, hipStream_t s) {
+    if (items == 0 || 3 * (uint64_t)items > 65535 || log_n < 7) return hipErrorInvalidValue;
+    const SmallArgs p{out, nullptr, key, stream_id, log_n, 0, items};
+    // (the grid covers the error polynomials' blocks; the surplus threads of the ternary ones leave at once)
+    const dim3 grid(((1u << log_n) / 8 + kSmallThreads - 1) / kSmallThreads, 3 * items);
+    hipLaunchKernelGGL(sample_encrypt_kernel, grid, dim3(kSmallThreads), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, const uint64_t *cdt,
+                                     uint32_t cdt_len, uint32_t items, hipStream_t s) {
+    if (items == 0 || items > 65535 || log_n < 7 || cdt_len == 0 || cdt_len >= kSmallCdt) return hipErrorInvalidValue;
+    const SmallArgs p{out, cdt, key, stream_id, log_n, cdt_len, items};
+    const dim3 grid(((1u << log_n) / 8 + kSmallThreads - 1) / kSmallThreads, items);
+    hipLaunchKernelGGL(sample_gauss_small_kernel, grid, dim3(kSmallThreads), 0, s, p);
     return hipGetLastError();
 }
 

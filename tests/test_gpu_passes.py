@@ -1,0 +1,120 @@
+"""Edges of the transform passes and of what is fused with them, against the oracle: batches on both sides of the sizes at
+which a launch changes its tile or walks several limbs per wave, the encoding that forms no maximum, encryption and decryption
+from byte samples, and the decoding that is composed where the inverse transform ends; on all three back ends."""
+import ctypes as C
+
+import numpy as np
+import pytest
+
+from gpu_util import DeviceArray, make_pair, rand_limbs
+
+pytestmark = pytest.mark.gpu
+
+CHAINS = {"fp": [50, 49, 50, 48, 50, 50], "int": [60, 58, 60, 60, 55, 60], "mixed": [60, 40, 40, 50, 60, 60]}
+
+
+@pytest.fixture(scope="module")
+def capi():
+    from lancelot_amd import capi as c
+    c.lib()
+    return c
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,limbs,polys", [(15, 5, 30), (15, 5, 41), (16, 4, 7), (16, 4, 8), (16, 1, 1)])
+def test_batched_transforms(oracle, capi, chain, logn, limbs, polys):
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], 1)
+    lib, h = capi.lib(), ctx.he_handle()
+    x = rand_limbs(p, np.random.default_rng(polys), range(limbs), n_polys=polys)
+    x[0, 0, :4] = [0, 1, p.moduli[0] - 1, p.moduli[0] - 2]
+    d = DeviceArray(capi, host=x)
+    capi.check(lib.he_ntt_forward(h, d.ptr, polys, limbs, limbs, 0, limbs, 0, None))
+    got = d.numpy()
+    for k in sorted({0, 1, polys // 2, polys - 1} & set(range(polys))):
+        assert (got[k] == p.ntt_fwd(x[k].copy())).all(), k
+    capi.check(lib.he_ntt_inverse(h, d.ptr, polys, limbs, limbs, 0, limbs, 0, None))
+    assert (d.numpy() == x).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,size_p,L", [(12, 1, 5), (13, 2, 3), (14, 1, 1), (15, 2, 4), (16, 1, 2)])
+def test_encrypt_and_decrypt(oracle, capi, chain, logn, size_p, L):
+    """he_encrypt of a plaintext elsewhere, he_encrypt_batch of three in place, he_decrypt_flood of 2 and 3 polynomials."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], size_p)
+    lib, h = capi.lib(), ctx.he_handle()
+    rng = np.random.default_rng(logn)
+    n, Q, K, items, first = p.n, p.size_q, p.size_p, 3, 11
+    key = oracle.chacha_key(3)
+    kp = key.ctypes.data_as(C.POINTER(C.c_uint32))
+    pk = rand_limbs(p, rng, range(p.size_qp), n_polys=2)
+    plain = rand_limbs(p, rng, range(L), n_polys=items)
+    dpk, dplain = DeviceArray(capi, host=pk), DeviceArray(capi, host=plain)
+    cts = np.zeros((items, 2, L, n), dtype=np.uint64)
+    cts[:, 0] = plain
+    dcts, dct = DeviceArray(capi, host=cts), DeviceArray(capi, shape=(2, L, n))
+    ws = DeviceArray(capi, shape=(lib.he_encrypt_batch_workspace_words(h, L, items),))
+    capi.check(lib.he_encrypt_batch(h, L, items, dpk.ptr, kp, first, dcts.ptr, ws.ptr, None))
+    capi.check(lib.he_encrypt(h, L, dplain.at(L * n), dpk.ptr, kp, first + 3, dct.ptr, ws.ptr, None))
+    got = dcts.numpy()
+    assert (dct.numpy() == got[1]).all()
+    # the oracle's division works on L + K limbs: those of Q that are in use, then the special ones
+    tidx = list(range(L)) + list(range(Q, Q + K))
+    for k in range(items):
+        u = p.ntt_fwd(p.sample_ternary(key, first + 3 * k, p.size_qp))
+        for i in range(2):
+            e = p.ntt_fwd(p.sample_error(key, first + 3 * k + 1 + i, p.size_qp))
+            want = p.moddown(np.ascontiguousarray(p.mul_add(u, pk[i], e)[tidx]))
+            assert (got[k, i] == (p.add(want, plain[k]) if i == 0 else want)).all(), (k, i)
+    cdt = oracle.gauss_cdt()
+    dcdt, noise = DeviceArray(capi, host=cdt), DeviceArray(capi, shape=(n // 8,))
+    sk = rand_limbs(p, rng, range(L), n_polys=2)
+    ct = rand_limbs(p, rng, range(L), n_polys=3)
+    dsk, dct3, out = DeviceArray(capi, host=sk), DeviceArray(capi, host=ct), DeviceArray(capi, shape=(L, n))
+    e = p.ntt_fwd(p.sample_gauss(key, 5, L, cdt))
+    for size in (2, 3):
+        capi.check(lib.he_decrypt_flood(h, dct3.ptr, size, L, dsk.ptr, L * n, kp, 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None))
+        want = p.mul_add(ct[1], sk[0], ct[0])
+        want = p.mul_add(ct[2], sk[1], want) if size == 3 else want
+        assert (out.numpy() == p.add(want, e)).all(), size
+    assert lib.he_decrypt_flood(h, dct3.ptr, 4, L, dsk.ptr, L * n, kp, 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None) != 0
+    assert lib.he_decrypt_flood(h, dct3.ptr, 2, L, dsk.ptr, L * n, kp, 5, dcdt.ptr, 128, out.ptr, noise.ptr, None) != 0
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,slots,limbs", [(12, 2, 1), (12, 2048, 5), (13, 128, 2), (13, 4096, 3), (14, 512, 4), (15, 16384, 2),
+                                              (16, 32768, 4), (17, 65536, 2)])
+def test_bounded_encoding_and_real_decoding(oracle, capi, chain, logn, slots, limbs):
+    """he_ckks_encode_bounded gives he_ckks_encode_batch's plaintexts, up to the largest coefficients it is for;
+    he_ckks_decode_real and he_decrypt_decode_real_batch give he_ckks_decode's real parts."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], 1)
+    lib, h = capi.lib(), ctx.he_handle()
+    rng = np.random.default_rng(slots)
+    items, n, count, scale = 2, p.n, slots - slots // 3, 2.0 ** 40
+    z = rng.uniform(-1, 1, (2, items, count)) * np.array([2.0 ** 20, 1.0])[None, :, None]
+    z[:, 0] *= slots / count / 2.0                 # item 0: sums of magnitudes below 2^20 slots, coefficients up to 2^60
+    re, im = DeviceArray(capi, host=z[0]), DeviceArray(capi, host=z[1])
+    ws = DeviceArray(capi, shape=(lib.he_ckks_encode_batch_workspace_words(h, items),))
+    want, got = (DeviceArray(capi, host=np.zeros((items, limbs, n), dtype=np.uint64)) for _ in range(2))
+    capi.check(lib.he_ckks_encode_batch(h, re.ptr, im.ptr, count, slots, scale, limbs, items, count, want.ptr, limbs, ws.ptr, None))
+    capi.check(lib.he_ckks_encode_bounded(h, re.ptr, im.ptr, count, slots, scale, limbs, items, count, got.ptr, limbs, ws.ptr, None))
+    plain = want.numpy()
+    assert (got.numpy() == plain).all()
+    # ciphertexts (plain, 0): whatever the key, they decrypt to the plaintext
+    cts = np.zeros((items, 2, limbs, n), dtype=np.uint64)
+    cts[:, 0] = plain
+    dcts, sk = DeviceArray(capi, host=cts), DeviceArray(capi, host=np.ones((limbs, n), dtype=np.uint64))
+    table = DeviceArray(capi, host=np.array([dcts.at(k * 2 * limbs * n) for k in range(items)], dtype=np.uint64))
+    take = max(1, slots - 1)
+    dws = DeviceArray(capi, shape=(lib.he_ckks_workspace_words(h, limbs),))
+    rws = DeviceArray(capi, shape=(lib.he_decrypt_decode_real_workspace_words(h, limbs, slots, items),))
+    full, real = DeviceArray(capi, shape=(slots, 2), dtype=np.float64), DeviceArray(capi, shape=(items, take), dtype=np.float64)
+    capi.check(lib.he_decrypt_decode_real_batch(h, table.ptr, items, limbs, sk.ptr, None, 0, None, 0, slots, scale, take, real.ptr,
+                                                rws.ptr, None))
+    batch = real.numpy()
+    for k in range(items):
+        capi.check(lib.he_ckks_decode(h, want.at(k * limbs * n), limbs, slots, scale, full.ptr, dws.ptr, None))
+        capi.check(lib.he_ckks_decode_real(h, want.at(k * limbs * n), limbs, slots, scale, real.ptr, take, rws.ptr, None))
+        values = full.numpy()[:take, 0]
+        assert (real.numpy()[0] == values).all() and (batch[k] == values).all(), k
+        if limbs > 1 or k == 1:
+            assert np.abs(values[:count] - z[0, k][:take]).max() < 2.0 ** -18, k
