@@ -354,16 +354,25 @@ struct IntSums {
 // ModDown needs in coefficient form leave through the inverse blocks pass (a launch and two trips of those limbs less: one
 // product at L = 24, K = 8 157 -> 153 us, n = 2^14, 4 + 1 limbs 38 -> 34 us, although the second set of twiddles takes the
 // FP64 kernel from 96 registers to 120).
-template <class A>
+// SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
+// and waves 0 and 1 finish one polynomial each.
+template <int SPLIT, class A>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &x, uint32_t t, uint32_t table, uint32_t blk,
-                                            uint32_t item, uint32_t lane, const A &ar, uint64_t *lds) {
+                                            uint32_t item, uint32_t lane, const A &ar, uint64_t *lds, uint32_t part,
+                                            uint64_t *sums_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
     const uint32_t LK = x.L + x.K, own = t < x.L ? t / x.K : 0xffffffffu;
     const uint64_t *lazy = a.out + item * a.item_stride + (size_t)t * n + off;   // words left by the rows pass, digit 0
     const size_t digit_stride = (size_t)LK * n, key_off = (size_t)table * n + at, key_poly = (size_t)x.size_qp * n;
+    // the digits to transform: all but the own one, the own one counting as the first for the deal
     auto skip_own = [&](uint32_t d) { return d == own ? d + 1 : d; };
+    auto next_digit = [&](uint32_t d) {
+#pragma unroll
+        for (int i = 0; i < SPLIT; i++) d = skip_own(d + 1);
+        return d;
+    };
     auto fetch = [&](uint64_t *w, uint32_t d) {
 #pragma unroll
         for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
@@ -375,10 +384,14 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     typename A::Tw tw[4];
     uint64_t nx[4];
     uint32_t d = skip_own(0);
+    if constexpr (SPLIT > 1) {
+        const uint32_t skip = own == 0xffffffffu ? part : (part + SPLIT - 1) % SPLIT;
+        for (uint32_t i = 0; i < skip; i++) d = skip_own(d + 1);
+    }
     if (d < x.beta) fetch(nx, d);
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
     typename std::conditional<FP, FpSums, IntSums>::type sums;
-    if (own != 0xffffffffu) {
+    if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = x.own + item * x.own_item_stride + (size_t)t * n;
         uint64_t c[4], k[2][4];
         keys(k, own);
@@ -404,7 +417,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         typename A::V v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = A::from_word(nx[j]);
-        d = skip_own(d + 1);
+        d = next_digit(d);
         if (d < x.beta) fetch(nx, d);
         ar.reduce(v);
         T4::template forward<A>(v, tw, ar, lds, lane);
@@ -414,6 +427,23 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         }
         sums.add(v, k, ar);
         wave_sync();   // (the next digit's exchanges reuse the LDS words that this one's lanes have read)
+    }
+    if constexpr (SPLIT > 1) {
+#pragma unroll
+        for (int r = 0; r < 2; r++) {
+            uint64_t w[4];
+            if constexpr (FP) ar.reduce(sums.s[r]);
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                if constexpr (FP)
+                    w[j] = A::to_word(sums.s[r][j]);
+                else
+                    w[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, ar.m.q, a.barrett[2 * table], a.barrett[2 * table + 1]);
+            }
+            store4(sums_lds + (2 * part + r) * 256 + 4 * lane, w);
+        }
+        lds_barrier();
+        if (part > 1) return;
     }
     const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
     const bool fold = x.fold_ct && t == x.L - 1;
@@ -429,8 +459,13 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     }
 #pragma unroll
     for (int r = 0; r < 2; r++) {
+        if (SPLIT > 1 && (uint32_t)r != part) continue;
         typename A::V v[4];
-        uint64_t c0[4], cl[4];
+        uint64_t c0[4], cl[4], parts[SPLIT][4];
+        if constexpr (SPLIT > 1) {
+#pragma unroll
+            for (int i = 0; i < SPLIT; i++) load4(parts[i], sums_lds + (2 * i + r) * 256 + 4 * lane);
+        }
         if (add && r == 0) {
             const uint64_t *src = x.add_c0 + (size_t)t * n;
             if (x.own_galois) {
@@ -444,7 +479,15 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         if constexpr (FP) {
             const FpMod m = ar.m;
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = sums.s[r][j];
+            for (int j = 0; j < 4; j++) {
+                if constexpr (SPLIT > 1) {
+                    v[j] = 0.0;
+#pragma unroll
+                    for (int i = 0; i < SPLIT; i++) v[j] += A::from_word(parts[i][j]);
+                } else {
+                    v[j] = sums.s[r][j];
+                }
+            }
             if (add && r == 0) {
                 const double pd = fp_from_u64(x.p_mod_q[2 * t]);
 #pragma unroll
@@ -460,7 +503,15 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         } else {
             const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
+            for (int j = 0; j < 4; j++) {
+                if constexpr (SPLIT > 1) {
+                    v[j] = parts[0][j];
+#pragma unroll
+                    for (int i = 1; i < SPLIT; i++) v[j] = add_mod(v[j], parts[i][j], q);
+                } else {
+                    v[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
+                }
+            }
             if (add && r == 0) {
                 const Shoup w = load_shoup(x.p_mod_q, t);
 #pragma unroll
@@ -496,13 +547,14 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
 constexpr int kInnerWaves = 4;
 
-template <int BE>
+template <int BE, int SPLIT>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
     __shared__ uint64_t lds_all[kInnerWaves][256 + 16];
+    __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = (x.L + x.K) << lr;
-    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = w % SPLIT;
     uint32_t pair, item = 0;
-    if (x.items > 1) {
+    if (SPLIT == 1 && x.items > 1) {
         const uint32_t groups = (x.items + kInnerWaves - 1) / kInnerWaves, id = blockIdx.x;
         uint32_t g;
         if (pairs % 8 == 0) {
@@ -518,15 +570,17 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
         if (item >= x.items) return;
     } else {
         // last limb first: the special limbs have one digit more to transform than the others
-        pair = blockIdx.x * kInnerWaves + w;
-        if (pair >= pairs) return;
+        // (a limb has an even number of blocks: with SPLIT > 1 no wave is left over, and a workgroup's blocks share their limb)
+        pair = blockIdx.x * (kInnerWaves / SPLIT) + w / SPLIT;
+        if (SPLIT == 1 && pair >= pairs) return;
         pair = pairs - 1 - pair;
     }
     const uint32_t t = pair >> lr, blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) inner_block(a, x, t, table, blk, item, lane, fp_arith(a, table), lds_all[w]);
+    uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
+    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, fp_arith(a, table), lds_all[w], part, sums);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) inner_block(a, x, t, table, blk, item, lane, int_arith(a, table), lds_all[w]);
+        if (!fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, int_arith(a, table), lds_all[w], part, sums);
     }
 }
 
@@ -634,83 +688,77 @@ __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t
     return add_mod(reduce_4q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
 }
 
-// Encryption: a wave takes its block of u, e0 and e1 of one limb through the last 8 stages, adds u pk_i to e_i and stores
-// the sums; a special limb's go through the inverse blocks pass first (ModDown follows).  The transformed u never reaches memory.
+// Encryption: three waves take their block of u, e0 and e1 of one limb through the last 8 stages; the transformed u stays in
+// LDS, from where the other two add u pk_i to their e_i and store the sums, a special limb's through the inverse blocks pass
+// (ModDown follows).  (One wave for all three: 14.8 against 11.4 us for 4 limbs of 2^16 words.)
 template <class A>
 __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t LK, uint32_t size_qp, uint32_t t,
-                                              uint32_t table, uint32_t blk, uint32_t item, uint32_t items, uint32_t lane, const A &ar,
-                                              uint64_t *lds) {
+                                              uint32_t table, uint32_t blk, uint32_t item, uint32_t items, uint32_t w, uint32_t lane,
+                                              const A &ar, uint64_t *lds, uint64_t *u_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
-    const uint64_t r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
-    uint64_t *poly[3] = {a.out + ((size_t)item * LK + t) * n, a.out + ((size_t)(items + 2 * item) * LK + t) * n,
-                         a.out + ((size_t)(items + 2 * item + 1) * LK + t) * n};
-    uint64_t x[3][4], k[2][4], u[4];
+    uint64_t *poly = a.out + ((size_t)(w == 0 ? item : items + 2 * item + w - 1) * LK + t) * n;
+    uint64_t x[4], k[4], u[4];
 #pragma unroll
-    for (int i = 0; i < 3; i++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) x[i][j] = poly[i][off + T4::word(0, lane, j)];
+    for (int j = 0; j < 4; j++) x[j] = poly[off + T4::word(0, lane, j)];
     typename A::Tw tw[4];
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
-    load4(k[0], pk + (size_t)table * n + at);
-    load4(k[1], pk + (size_t)(size_qp + table) * n + at);
-    typename A::V v[3][4];
+    if (w) load4(k, pk + ((size_t)(w - 1) * size_qp + table) * n + at);
+    typename A::V v[4];
 #pragma unroll
-    for (int i = 0; i < 3; i++) {
+    for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
+    ar.reduce(v);
+    T4::template forward<A>(v, tw, ar, lds, lane);
+    if (w == 0) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[i][j] = A::from_word(x[i][j]);
-        ar.reduce(v[i]);
-        T4::template forward<A>(v[i], tw, ar, lds, lane);
-        wave_sync();
+        for (int j = 0; j < 4; j++) u[j] = canonical_word(v[j], ar);
+        store4(u_lds + 4 * lane, u);
     }
-#pragma unroll
-    for (int j = 0; j < 4; j++) u[j] = canonical_word(v[0][j], ar);
     A iar = ar;
-    if (t >= L) {
+    if (w && t >= L) {
         if constexpr (FP)
             iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
         else
             iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
         T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
     }
+    lds_barrier();
+    if (w == 0) return;
+    load4(u, u_lds + 4 * lane);
+    const uint64_t r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+    uint64_t o[4];
 #pragma unroll
-    for (int i = 0; i < 2; i++) {
-        uint64_t o[4];
+    for (int j = 0; j < 4; j++) o[j] = add_product(v[j], u[j], k[j], ar, r0, r1);
+    if (t >= L) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) o[j] = add_product(v[1 + i][j], u[j], k[i][j], ar, r0, r1);
-        if (t >= L) {
-            typename A::V w[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (FP)
-                    w[j] = fp_from_u64(o[j]);
-                else
-                    w[j] = o[j];
-            }
-            T4::template inverse<A>(w, tw, iar, lds, lane);
-#pragma unroll
-            for (int j = 0; j < 4; j++) poly[1 + i][off + T4::word(0, lane, j)] = A::to_word(w[j]);
-            wave_sync();
-        } else {
-            store4(poly[1 + i] + at, o);
+        for (int j = 0; j < 4; j++) {
+            if constexpr (FP)
+                v[j] = fp_from_u64(o[j]);
+            else
+                v[j] = o[j];
         }
+        T4::template inverse<A>(v, tw, iar, lds, lane);
+#pragma unroll
+        for (int j = 0; j < 4; j++) poly[off + T4::word(0, lane, j)] = A::to_word(v[j]);
+    } else {
+        store4(poly + at, o);
     }
 }
 
 template <int BE>
-__global__ __launch_bounds__(64 * kBlockWaves) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
-                                                                          uint32_t items) {
-    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+__global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
+                                                             uint32_t items) {
+    __shared__ uint64_t lds_all[3][256 + 16], u_lds[256];
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1), it = id >> lr;
+    const uint32_t id = logical_block(), blk = id & ((1u << lr) - 1), it = id >> lr;
     const uint32_t item = it / LK, t = it - item * LK, table = t < L ? t : size_q + (t - L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     if (BE != NTT_BACKEND_INT && fp)
-        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, lane, fp_arith(a, table), lds_all[w]);
+        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, fp_arith(a, table), lds_all[w], u_lds);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, lane, int_arith(a, table), lds_all[w]);
+        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, int_arith(a, table), lds_all[w], u_lds);
     }
 }
 
@@ -872,15 +920,31 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
     const uint32_t items = x.items ? x.items : 1;
     if (items > 1 && (x.own_galois || x.add_c0)) return hipErrorInvalidValue;
     const uint64_t pairs = (uint64_t)(x.L + x.K) << (a.log_n - 8);
-    const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs + kInnerWaves - 1) / kInnerWaves;
+    // Few blocks: what a wave does in turn (a transform per digit, for a special limb two inverse ones) is the kernel's time, so
+    // two or four waves share a block as long as the chip has room for them (two, four waves per SIMD).  One product, one
+    // wave against two against four a block: n = 2^12, 3 limbs 35.6 / 30.6 / 23.8 us; n = 2^14, 4 limbs 37.9 / 33.8 / 27.0;
+    // n = 2^16, 2 limbs of two digits 44.5 / 38.3; n = 2^15, 10 limbs in 5 digits 78.5 / 74.5 / 76.1; n = 2^16, 6 limbs (2048
+    // blocks) 64.4 / 64.3 / 64.5; from 3072 blocks on nothing is gained, at 8192 four waves lose 5 %.
+    const int split = items > 1 || x.beta < 2 ? 1 : x.beta > 2 && pairs <= 512 ? 4 : pairs <= 2048 ? 2 : 1;
+    const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs * split + kInnerWaves - 1) / kInnerWaves;
     if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kInnerWaves);
-    if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
-    else if (backend)
-        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
+#define HE_INNER(SPLIT)                                                                                           \
+    do {                                                                                                          \
+        if (backend == NTT_BACKEND_MIXED)                                                                         \
+            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_MIXED, SPLIT>), grid, block, 0, s, a, x);            \
+        else if (backend)                                                                                         \
+            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_FP, SPLIT>), grid, block, 0, s, a, x);               \
+        else                                                                                                      \
+            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_INT, SPLIT>), grid, block, 0, s, a, x);              \
+    } while (0)
+    if (split == 4)
+        HE_INNER(4);
+    else if (split == 2)
+        HE_INNER(2);
     else
-        hipLaunchKernelGGL(ntt_inner_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
+        HE_INNER(1);
+#undef HE_INNER
     return hipGetLastError();
 }
 
@@ -901,9 +965,9 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint
 hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
                                  int backend, hipStream_t s) {
     if (a.log_n < 9 || a.log_n > 17 || items == 0) return hipErrorInvalidValue;
-    const uint64_t wgs = ((uint64_t)(L + K) * items << (a.log_n - 8)) / kBlockWaves;
+    const uint64_t wgs = (uint64_t)(L + K) * items << (a.log_n - 8);
     if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    const dim3 grid((uint32_t)wgs), block(192);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, pk, L, K, size_q, items);
     else if (backend)
