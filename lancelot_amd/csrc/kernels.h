@@ -324,7 +324,6 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
 // are never written:
 //   out[k][t] = sum_d y_d[t] * evk_d[k][t],  y_d[t] = own[t] for the limbs t of digit d itself.
 struct KsFuseArgs {
-    EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form
     const uint64_t *own;  // the key-switch input c, [L][N], NTT form
     uint32_t own_galois;  // != 0: the input is sigma(own), gathered while it is read
     // optional (a rotation): out[0][t] += P * sigma(add_c0)[t] on the data limbs, with the same sigma; the ModDown that
@@ -346,6 +345,7 @@ struct KsFuseArgs {
     // other, so that the key tile is read from memory by the first and from that XCD's L2 by the others.
     uint32_t items;
     size_t own_item_stride, fold_item_stride;
+    EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form (last: of its lines a launch reads the first ones)
 };
 hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s);
 

@@ -12,6 +12,30 @@ namespace {
 
 __device__ __forceinline__ uint32_t skew(uint32_t e) { return e + (e >> 4); }
 
+// read-only tables that every lane of a wave reads at one address: through the scalar cache
+typedef const double __attribute__((address_space(4))) *ScalarF64;
+typedef const uint64_t __attribute__((address_space(4))) *ScalarU64;
+__device__ __forceinline__ ScalarF64 scalar(const double *p) { return (ScalarF64)(uintptr_t)p; }
+__device__ __forceinline__ ScalarU64 scalar(const uint64_t *p) { return (ScalarU64)(uintptr_t)p; }
+
+// entry idx of a table of (operand, Shoup quotient) pairs
+__device__ __forceinline__ Shoup scalar_shoup(const uint64_t *table, size_t idx) { return Shoup{scalar(table)[2 * idx], scalar(table)[2 * idx + 1]}; }
+
+// The arguments of a launch lie in memory that no cache holds yet: the first read of each of their 64-byte lines takes as long as
+// one from memory, and the compiler reads a field where it is used, one line after the other in a chain.  A kernel that begins with
+// this has asked for all lines at once.
+template <int BYTES>
+__device__ __forceinline__ void touch_arguments() {
+    typedef const uint32_t __attribute__((address_space(4))) *Line;
+    const Line p = (Line)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int LINES = BYTES / 64;
+    uint32_t x[LINES];
+#pragma unroll
+    for (int i = 0; i < LINES; i++) x[i] = p[16 * i];
+#pragma unroll
+    for (int i = 0; i < LINES; i++) asm volatile("" ::"s"(x[i]));
+}
+
 // Workgroup barrier that orders LDS traffic only.  __syncthreads() also waits for every global load and
 // store of the wave, which would serialise a prefetch issued before it with the butterflies after it.
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
@@ -73,20 +97,20 @@ struct FpCtx {
 };
 
 __device__ __forceinline__ IntCtx int_ctx(const NttArgs &a, uint32_t table) {
-    return IntCtx{a.moduli[table], a.tw + ((size_t)table << (a.log_n + 1))};
+    return IntCtx{scalar(a.moduli)[table], a.tw + ((size_t)table << (a.log_n + 1))};
 }
 
 __device__ __forceinline__ FpCtx fp_ctx(const NttArgs &a, uint32_t table) {
-    const double *c = a.fp_consts + 4 * (size_t)table;
+    const ScalarF64 c = scalar(a.fp_consts) + 4 * (size_t)table;
     return FpCtx{FpMod{c[0], c[1]}, a.tw_fp + ((size_t)table << a.log_n)};
 }
 
 // (N^-1 [* w]) as an FP twiddle for the last multiplication of the inverse transform
 __device__ __forceinline__ FpTw inverse_scale(const NttArgs &a, const Job &job, FpMod m) {
-    const double *c = a.fp_consts + 4 * (size_t)job.table;
+    const ScalarF64 c = scalar(a.fp_consts) + 4 * (size_t)job.table;
     FpTw ninv{c[2], c[3]};
     if (a.epi_mode != NTT_EPI_MUL) return ninv;
-    const double w = fp_canonical(fp_mulmod(fp_from_u64(a.w[2 * job.limb]), ninv, m), m);
+    const double w = fp_canonical(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
     return FpTw{w, w * m.qinv};
 }
 
@@ -108,10 +132,10 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
         const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
         const FpMod ml = fp_ctx(a, a.pro_last).m;
-        const double wd = fp_from_u64(a.pro_w[2 * job.limb]), wl = fp_from_u64(a.pro_w[2 * a.pro_last]);
+        const double wd = fp_from_u64(scalar(a.pro_w)[2 * job.limb]), wl = fp_from_u64(scalar(a.pro_w)[2 * a.pro_last]);
         const FpTw w{wd, wd * c.m.qinv}, wlast{wl, wl * ml.qinv};
-        const uint64_t qj = a.moduli[job.table], rj = a.barrett[2 * job.table + 1];
-        const uint64_t qlast = a.moduli[a.pro_last], rlast = a.barrett[2 * a.pro_last + 1];
+        const uint64_t qj = scalar(a.moduli)[job.table], rj = scalar(a.barrett)[2 * job.table + 1];
+        const uint64_t qlast = scalar(a.moduli)[a.pro_last], rlast = scalar(a.barrett)[2 * a.pro_last + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) {
             const uint64_t ds = dsrc[glob(j)];
@@ -131,7 +155,7 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         return true;
     }
     if (a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
-        const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
+        const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(barrett64(job.src[glob(j)], q, r1));
     } else if (a.pro_mode == NTT_PRO_SMALL) {
@@ -153,17 +177,17 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
 template <int W, typename Glob>
 __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &a, const Job &job, uint64_t q, Glob glob) {
     if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE || a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
-        const uint64_t r1 = a.barrett[2 * job.table + 1];
+        const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
         const uint64_t *src = a.pro_mode == NTT_PRO_SOURCE_REDUCE ? job.src : a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = barrett64(src[glob(j)], q, r1);
     } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
-        const uint64_t r1 = a.barrett[2 * job.table + 1];
+        const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
         const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
         const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
-        const uint64_t ql = a.moduli[a.pro_last];
-        const Shoup w = load_shoup(a.pro_w, job.limb), wlast = load_shoup(a.pro_w, a.pro_last);
-        const uint64_t rlast = a.barrett[2 * a.pro_last + 1];
+        const uint64_t ql = scalar(a.moduli)[a.pro_last];
+        const Shoup w = scalar_shoup(a.pro_w, job.limb), wlast = scalar_shoup(a.pro_w, a.pro_last);
+        const uint64_t rlast = scalar(a.barrett)[2 * a.pro_last + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) {
             const uint64_t ds = dsrc[glob(j)];
@@ -180,7 +204,7 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
             v[j] = (uint64_t)x + (x < 0 ? q : 0);
         }
     } else if (a.pro_mode == NTT_PRO_ROUND) {
-        const uint64_t r1 = a.barrett[2 * job.table + 1];
+        const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) {
             const double x = rounded_coefficient(a, job, (uint32_t)glob(j));
@@ -199,11 +223,38 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_wave_barrier();
 }
 
-// read-only tables that every lane of a wave reads at one address: through the scalar cache
-typedef const double __attribute__((address_space(4))) *ScalarF64;
-typedef const uint64_t __attribute__((address_space(4))) *ScalarU64;
-__device__ __forceinline__ ScalarF64 scalar(const double *p) { return (ScalarF64)(uintptr_t)p; }
-__device__ __forceinline__ ScalarU64 scalar(const uint64_t *p) { return (ScalarU64)(uintptr_t)p; }
+// a of the lanes whose bit BIT is set and b of the lanes where it is not change places: the words' register bit becomes that
+// bit of the lane
+template <int BIT>
+__device__ __forceinline__ void swap_lane_bit(uint32_t &a, uint32_t &b) {
+    if constexpr (BIT >= 4) {
+        const auto r = BIT == 5 ? __builtin_amdgcn_permlane32_swap(a, b, false, false) : __builtin_amdgcn_permlane16_swap(a, b, false, false);
+        a = r[0];
+        b = r[1];
+    } else if constexpr (BIT >= 2) {
+        // a row's lanes shifted by 8 or 4; the banks (4 lanes) with the bit take b from below, the others a from above
+        constexpr int SHIFT = 1 << BIT, WITH = BIT == 3 ? 0xc : 0xa;
+        const uint32_t x = (uint32_t)__builtin_amdgcn_update_dpp((int)a, (int)b, 0x110 + SHIFT, 0xf, WITH, false);
+        b = (uint32_t)__builtin_amdgcn_update_dpp((int)b, (int)a, 0x100 + SHIFT, 0xf, 0xf ^ WITH, false);
+        a = x;
+    } else {
+        constexpr int PERM = BIT == 1 ? 0x4e : 0xb1;   // lanes 2 3 0 1, or 1 0 3 2, of every four
+        const bool with = (__lane_id() >> BIT) & 1;
+        const uint32_t pa = (uint32_t)__builtin_amdgcn_mov_dpp((int)a, PERM, 0xf, 0xf, true);
+        const uint32_t pb = (uint32_t)__builtin_amdgcn_mov_dpp((int)b, PERM, 0xf, 0xf, true);
+        a = with ? pb : a;
+        b = with ? b : pa;
+    }
+}
+
+template <int BIT>
+__device__ __forceinline__ void swap_lane_bit(uint64_t &a, uint64_t &b) {
+    uint32_t al = (uint32_t)a, ah = (uint32_t)(a >> 32), bl = (uint32_t)b, bh = (uint32_t)(b >> 32);
+    swap_lane_bit<BIT>(al, bl);
+    swap_lane_bit<BIT>(ah, bh);
+    a = ((uint64_t)ah << 32) | al;
+    b = ((uint64_t)bh << 32) | bl;
+}
 
 // Two stages (ST = 1: only the first of them) on four words; tw entries: the first stage's twiddle, then the two of the
 // second.
@@ -218,7 +269,7 @@ struct IntArith {
     static __device__ __forceinline__ uint64_t to_word(V v) { return v; }
     template <int ST, bool UNIFORM>
     __device__ __forceinline__ Tw load(uint32_t idx) const {
-        auto at = [&](size_t i) { return UNIFORM ? Shoup{scalar(table)[2 * i], scalar(table)[2 * i + 1]} : load_shoup(table, i); };
+        auto at = [&](size_t i) { return UNIFORM ? scalar_shoup(table, i) : load_shoup(table, i); };
         Tw t;
         t.s[0] = at(idx);
         t.s[1] = t.s[2] = Shoup{0, 0};
@@ -331,22 +382,35 @@ struct Tile4 {
         tw[K] = ar.template load<stages(K), (B - 2 * K - 2 >= 6)>(((scale - 1) << (2 * K)) + index(K, t));
         if constexpr (K + 1 < kBlocks) load_tw<A, K + 1>(tw, ar, scale, t);
     }
-    template <int KLO>
-    static __device__ __forceinline__ void sync() {
-        if constexpr (B - 2 * KLO - 2 > 6)
+    // From the layout of block KLO to that of block KLO + 1, or back: the register bits and the thread bits low - 1 and low - 2
+    // change places.  Inside a wave that is done in registers (8 to 16 instructions for 4 words; through LDS 8 accesses
+    // and about 300 cycles before the next butterfly starts).
+    template <class A, int KLO, bool BACK>
+    static __device__ __forceinline__ void exchange(typename A::V *v, uint64_t *lds, uint32_t t) {
+        constexpr int LOW = B - 2 * KLO - 2;
+        uint64_t w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = A::to_word(v[j]);
+        if constexpr (LOW > 6) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) lds[skew(word(BACK ? KLO + 1 : KLO, t, j))] = w[j];
             lds_barrier();
-        else
-            wave_sync();
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = lds[skew(word(BACK ? KLO : KLO + 1, t, j))];
+        } else {
+            swap_lane_bit<LOW - 1>(w[0], w[2]);
+            swap_lane_bit<LOW - 1>(w[1], w[3]);
+            swap_lane_bit<LOW - 2>(w[0], w[1]);
+            swap_lane_bit<LOW - 2>(w[2], w[3]);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = A::from_word(w[j]);
     }
     template <class A, int K = 0>
     static __device__ __forceinline__ void forward(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
         ar.template ct<stages(K)>(v, tw[K]);
         if constexpr (K + 1 < kBlocks) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
-            sync<K>();
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K + 1, t, j))]);
+            exchange<A, K, false>(v, lds, t);
             if constexpr ((K + 1) % 2 == 0) ar.reduce(v);
             forward<A, K + 1>(v, tw, ar, lds, t);
         }
@@ -355,11 +419,7 @@ struct Tile4 {
     static __device__ __forceinline__ void inverse(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
         ar.template gs<stages(K)>(v, tw[K]);
         if constexpr (K > 0) {
-#pragma unroll
-            for (int j = 0; j < 4; j++) lds[skew(word(K, t, j))] = A::to_word(v[j]);
-            sync<K - 1>();
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = A::from_word(lds[skew(word(K - 1, t, j))]);
+            exchange<A, K - 1, true>(v, lds, t);
             ar.reduce(v);
             inverse<A, K - 1>(v, tw, ar, lds, t);
         }

@@ -32,6 +32,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
     constexpr int LOGC = B - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
     __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
+    touch_arguments<sizeof(NttArgs)>();
     const uint32_t lb = logical_block();
     const Job job = decode_job(a, lb / tiles_per_limb);
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
@@ -52,12 +53,12 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
             ar.reduce(v);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
-            const double *cc = a.fp_consts + 4 * (size_t)st;
+            const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
             const FpTw ninv{cc[2], cc[3]};
 #pragma unroll
             for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
         } else {
-            const uint64_t q = a.moduli[st];
+            const uint64_t q = scalar(a.moduli)[st];
             const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
             uint64_t v[4];
 #pragma unroll
@@ -78,7 +79,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
         if (FWD) {
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) {
-                const uint64_t q = a.moduli[job.table], r1 = a.barrett[2 * job.table + 1];
+                const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
             } else if (rows_input_fp(v, a, job, c, [&](int j) { return glob(0, j); })) {
@@ -102,13 +103,13 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
     }
     if constexpr (BE != NTT_BACKEND_FP) {
         const IntArith ar = int_arith(a, job.table);
-        const uint64_t q = a.moduli[job.table];
+        const uint64_t q = scalar(a.moduli)[job.table];
         uint64_t v[4];
         IntArith::Tw tw[NB];
         if (FWD) {
             T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) {
-                const uint64_t r1 = a.barrett[2 * job.table + 1];
+                const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
             } else {
@@ -122,9 +123,10 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = job.in[glob(NB - 1, j)];
             T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            Shoup w{0, 0};
+            if (a.epi_mode == NTT_EPI_MUL) w = scalar_shoup(a.w, job.limb);
             T4::template inverse<IntArith>(v, tw, ar, lds, t);
             if (a.epi_mode == NTT_EPI_MUL) {
-                const Shoup w = load_shoup(a.w, job.limb);
 #pragma unroll
                 for (int j = 0; j < 4; j++) job.out[glob(0, j)] = mul_shoup(v[j], w, q);
             } else {
@@ -137,11 +139,12 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
 
 constexpr int kBlockWaves = 2;   // 256-word blocks of a workgroup, one per wave
 
-// Operands of a fused forward epilogue at the lane's four consecutive words
+// Operands of a fused forward epilogue at the lane's four consecutive words, and its constants
 struct EpiOperands {
     bool fma, add;
     uint64_t a[4], b[4];
     uint64_t *dst;
+    Shoup w, pro_w;
 };
 
 __device__ __forceinline__ EpiOperands load_epilogue(const NttArgs &a, const Job &job, size_t off) {
@@ -152,6 +155,9 @@ __device__ __forceinline__ EpiOperands load_epilogue(const NttArgs &a, const Job
     o.dst = a.epi_dst + (size_t)job.poly * a.epi_dst_poly_stride * n + at;
     load4(o.a, a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + at);
     if (o.add) load4(o.b, a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + at);
+    o.w = scalar_shoup(a.w, job.limb);
+    o.pro_w = Shoup{0, 0};
+    if (o.fma) o.pro_w = scalar_shoup(a.pro_w, job.limb);
     return o;
 }
 
@@ -228,10 +234,10 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 T4::template forward<A>(v, tw, ar, lds, lane);
                 if (EPI) {
                     // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
-                    const double wd = fp_from_u64(a.w[2 * job.limb]);
+                    const double wd = fp_from_u64(e.w.w);
                     const FpTw ew{wd, wd * m.qinv};
                     if (e.fma) {
-                        const double pd = fp_from_u64(a.pro_w[2 * job.limb]);
+                        const double pd = fp_from_u64(e.pro_w.w);
                         const FpTw pw{pd, pd * m.qinv};
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
@@ -262,9 +268,9 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
 #pragma unroll
                 for (int j = 0; j < 4; j++) x[j] = reduce_4q(v[j], q);
                 if (EPI) {
-                    const Shoup ew = load_shoup(a.w, job.limb);
+                    const Shoup ew = e.w;
                     if (e.fma) {
-                        const Shoup pw = load_shoup(a.pro_w, job.limb);
+                        const Shoup pw = e.pro_w;
 #pragma unroll
                         for (int j = 0; j < 4; j++)
                             x[j] = mul_shoup(sub_mod(add_mod(mul_shoup(e.a[j], pw, q), e.b[j], q), x[j], q), ew, q);
@@ -295,6 +301,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
 template <bool FWD, bool EPI, bool LOOP, int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a) {
     __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    touch_arguments<sizeof(NttArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block() * kBlockWaves + w;   // (a limb has an even number of blocks)
@@ -304,7 +311,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a)
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane, lds_all[w]);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), a.moduli[job.table], blk, lane, lds_all[w]);
+        if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), scalar(a.moduli)[job.table], blk, lane, lds_all[w]);
     }
 }
 
@@ -390,6 +397,12 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     }
     if (d < x.beta) fetch(nx, d);
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
+    const bool fold = x.fold_ct && t == x.L - 1;
+    Shoup add_w{0, 0}, fold_w{0, 0};
+    if (add) add_w = scalar_shoup(x.p_mod_q, t);
+    if (fold) fold_w = scalar_shoup(x.fold_w, 0);
+    const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = x.own + item * x.own_item_stride + (size_t)t * n;
@@ -438,15 +451,13 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
                 if constexpr (FP)
                     w[j] = A::to_word(sums.s[r][j]);
                 else
-                    w[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, ar.m.q, a.barrett[2 * table], a.barrett[2 * table + 1]);
+                    w[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, ar.m.q, r0, r1);
             }
             store4(sums_lds + (2 * part + r) * 256 + 4 * lane, w);
         }
         lds_barrier();
         if (part > 1) return;
     }
-    const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
-    const bool fold = x.fold_ct && t == x.L - 1;
     // (the words of a limb that ModDown transforms back go through the inverse blocks pass before they leave the wave)
     const bool invert = t >= x.inv_first;
     A iar = ar;
@@ -489,19 +500,19 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
                 }
             }
             if (add && r == 0) {
-                const double pd = fp_from_u64(x.p_mod_q[2 * t]);
+                const double pd = fp_from_u64(add_w.w);
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] += fp_mulmod(fp_from_u64(c0[j]), FpTw{pd, pd * m.qinv}, m);
             }
             if (fold) {
-                const double wd = fp_from_u64(x.fold_w[0]);
+                const double wd = fp_from_u64(fold_w.w);
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], FpTw{wd, wd * m.qinv}, m) + fp_from_u64(cl[j]);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = fp_canonical(v[j], m);
         } else {
-            const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+            const uint64_t q = ar.m.q;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 if constexpr (SPLIT > 1) {
@@ -513,14 +524,12 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
                 }
             }
             if (add && r == 0) {
-                const Shoup w = load_shoup(x.p_mod_q, t);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = add_mod(v[j], mul_shoup(c0[j], w, q), q);
+                for (int j = 0; j < 4; j++) v[j] = add_mod(v[j], mul_shoup(c0[j], add_w, q), q);
             }
             if (fold) {
-                const Shoup w = load_shoup(x.fold_w, 0);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = add_mod(mul_shoup(v[j], w, q), cl[j], q);
+                for (int j = 0; j < 4; j++) v[j] = add_mod(mul_shoup(v[j], fold_w, q), cl[j], q);
             }
         }
         uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)r * LK * n + (size_t)t * n;
@@ -551,6 +560,7 @@ template <int BE, int SPLIT>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
     __shared__ uint64_t lds_all[kInnerWaves][256 + 16];
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
+    touch_arguments<sizeof(NttArgs) + sizeof(KsFuseArgs) - (kMaxDigits - 8) * sizeof(uint64_t *)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = (x.L + x.K) << lr;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = w % SPLIT;
     uint32_t pair, item = 0;
@@ -601,7 +611,7 @@ __device__ __forceinline__ void tensor4(const FpArith &ar, const NttArgs &, uint
 
 __device__ __forceinline__ void tensor4(const IntArith &ar, const NttArgs &a, uint32_t table, const uint64_t *a0, const uint64_t *a1,
                                         const uint64_t *b0, const uint64_t *b1, uint64_t *d0, uint64_t *d1, uint64_t *d2) {
-    const uint64_t q = ar.m.q, r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
+    const uint64_t q = ar.m.q, r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         d0[j] = mul_mod(a0[j], b0[j], q, r0, r1);
@@ -664,6 +674,7 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
 template <int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(NttArgs a, TensorFuse x) {
     __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    touch_arguments<sizeof(NttArgs) + sizeof(TensorFuse)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
@@ -699,6 +710,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
     uint64_t *poly = a.out + ((size_t)(w == 0 ? item : items + 2 * item + w - 1) * LK + t) * n;
+    const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
     uint64_t x[4], k[4], u[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) x[j] = poly[off + T4::word(0, lane, j)];
@@ -726,7 +738,6 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
     lds_barrier();
     if (w == 0) return;
     load4(u, u_lds + 4 * lane);
-    const uint64_t r0 = a.barrett[2 * table], r1 = a.barrett[2 * table + 1];
     uint64_t o[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) o[j] = add_product(v[j], u[j], k[j], ar, r0, r1);
@@ -750,6 +761,7 @@ template <int BE>
 __global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
                                                              uint32_t items) {
     __shared__ uint64_t lds_all[3][256 + 16], u_lds[256];
+    touch_arguments<sizeof(NttArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block(), blk = id & ((1u << lr) - 1), it = id >> lr;
@@ -768,7 +780,7 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
                                               const A &ar, uint64_t *lds) {
     using T4 = Tile4<8, 8>;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane, poly = (size_t)a.map.limbs * n;
-    const uint64_t q = a.moduli[job.table], r0 = a.barrett[2 * job.table], r1 = a.barrett[2 * job.table + 1];
+    const uint64_t q = scalar(a.moduli)[job.table], r0 = scalar(a.barrett)[2 * job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
     const uint64_t *ct = (d.cts ? d.cts[job.poly] : d.ct) + job.limb * n + at;
     const uint64_t *sk = d.sk + job.limb * n + at;
     uint64_t x[4], c0[4], c1[4], s1[4], c2[4], s2[4];
@@ -800,6 +812,7 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
 template <int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArgs a, DecryptArgs d) {
     __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
+    touch_arguments<sizeof(NttArgs) + sizeof(DecryptArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
