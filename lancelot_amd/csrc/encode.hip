@@ -125,19 +125,34 @@ struct FftTile {
         tw[K].b = T4::stages(K) == 2 ? stage_twiddle<INVERSE>(t, len >> 1, pos(K, 0) & (mask >> 1)) : double2{0.0, 0.0};
         if constexpr (K + 1 < T4::kBlocks) load_tw<Pos, K + 1>(tw, t, log_slots, stage0, pos);
     }
-    static __device__ __forceinline__ void put(const double2 *v, double *re, double *im, int k, uint32_t t) {
+    // from the layout of block FROM to that of its neighbour TO
+    template <int FROM, int TO>
+    static __device__ __forceinline__ void move(double2 *v, double *re, double *im, uint32_t t) {
+        constexpr int KLO = FROM < TO ? FROM : TO;
+        if constexpr (T4::in_wave(KLO)) {
+            uint64_t x[4], y[4];
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t e = skew(T4::word(k, t, j));
-            re[e] = v[j].x;
-            im[e] = v[j].y;
-        }
-    }
-    static __device__ __forceinline__ void get(double2 *v, const double *re, const double *im, int k, uint32_t t) {
+            for (int j = 0; j < 4; j++) {
+                x[j] = (uint64_t)__double_as_longlong(v[j].x);
+                y[j] = (uint64_t)__double_as_longlong(v[j].y);
+            }
+            T4::template swap_words<KLO>(x);
+            T4::template swap_words<KLO>(y);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-            const uint32_t e = skew(T4::word(k, t, j));
-            v[j] = double2{re[e], im[e]};
+            for (int j = 0; j < 4; j++) v[j] = double2{__longlong_as_double((long long)x[j]), __longlong_as_double((long long)y[j])};
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t e = skew(T4::word(FROM, t, j));
+                re[e] = v[j].x;
+                im[e] = v[j].y;
+            }
+            lds_barrier();
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const uint32_t e = skew(T4::word(TO, t, j));
+                v[j] = double2{re[e], im[e]};
+            }
         }
     }
     // the stages in order (INVERSE), values of block 0 -> values of the last block
@@ -150,9 +165,7 @@ struct FftTile {
             butterfly<INVERSE>(v[2], v[3], tw[K].b);
         }
         if constexpr (K + 1 < T4::kBlocks) {
-            put(v, re, im, K, t);
-            T4::template sync<K>();
-            get(v, re, im, K + 1, t);
+            move<K, K + 1>(v, re, im, t);
             down<K + 1>(v, tw, re, im, t);
         }
     }
@@ -166,9 +179,7 @@ struct FftTile {
         butterfly<INVERSE>(v[0], v[2], tw[K].a0);
         butterfly<INVERSE>(v[1], v[3], tw[K].a1);
         if constexpr (K > 0) {
-            put(v, re, im, K, t);
-            T4::template sync<K - 1>();
-            get(v, re, im, K - 1, t);
+            move<K, K - 1>(v, re, im, t);
             up<K - 1>(v, tw, re, im, t);
         }
     }

@@ -385,23 +385,28 @@ struct Tile4 {
     // From the layout of block KLO to that of block KLO + 1, or back: the register bits and the thread bits low - 1 and low - 2
     // change places.  Inside a wave that is done in registers (8 to 16 instructions for 4 words; through LDS 8 accesses
     // and about 300 cycles before the next butterfly starts).
+    static constexpr bool in_wave(int klo) { return B - 2 * klo - 2 <= 6; }
+    template <int KLO>
+    static __device__ __forceinline__ void swap_words(uint64_t *w) {
+        constexpr int LOW = B - 2 * KLO - 2;
+        swap_lane_bit<LOW - 1>(w[0], w[2]);
+        swap_lane_bit<LOW - 1>(w[1], w[3]);
+        swap_lane_bit<LOW - 2>(w[0], w[1]);
+        swap_lane_bit<LOW - 2>(w[2], w[3]);
+    }
     template <class A, int KLO, bool BACK>
     static __device__ __forceinline__ void exchange(typename A::V *v, uint64_t *lds, uint32_t t) {
-        constexpr int LOW = B - 2 * KLO - 2;
         uint64_t w[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) w[j] = A::to_word(v[j]);
-        if constexpr (LOW > 6) {
+        if constexpr (in_wave(KLO)) {
+            swap_words<KLO>(w);
+        } else {
 #pragma unroll
             for (int j = 0; j < 4; j++) lds[skew(word(BACK ? KLO + 1 : KLO, t, j))] = w[j];
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < 4; j++) w[j] = lds[skew(word(BACK ? KLO : KLO + 1, t, j))];
-        } else {
-            swap_lane_bit<LOW - 1>(w[0], w[2]);
-            swap_lane_bit<LOW - 1>(w[1], w[3]);
-            swap_lane_bit<LOW - 2>(w[0], w[1]);
-            swap_lane_bit<LOW - 2>(w[2], w[3]);
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = A::from_word(w[j]);
