@@ -11,8 +11,11 @@
 #include <cstdlib>
 #include <cstring>
 
+#include <type_traits>
+
 #include "kernels.h"
 #include "modarith.cuh"
+#include "ntt_common.cuh"
 
 namespace he {
 
@@ -683,6 +686,242 @@ __global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
     }
 }
 
+// Sums of one wave's terms of a hoisted inner product: both key polynomials, two coefficients per lane.
+// A prime below 2^50: exact (hi, lo) pairs of doubles, see hoist_inner_kernel.
+struct HoistSumsFp {
+    FpMod m;
+    double base, down, hi[4], lo[4], f[4];
+    FpTw wB;
+    uint32_t period, pending;
+    __device__ __forceinline__ HoistSumsFp(const double *consts, uint64_t q, uint32_t n_terms) : m{scalar(consts)[0], scalar(consts)[1]} {
+        const uint32_t qbits = 64 - __builtin_clzll(q), tbits = 32 - __builtin_clz(n_terms);
+        const bool one_go = 2 * qbits + tbits <= 100;
+        const uint32_t B = !one_go ? 103 : 2 * qbits + tbits < 60 ? 60 : 2 * qbits + tbits;
+        period = one_go ? n_terms : 8;
+        pending = 0;
+        base = __hiloint2double((int)((1023 + B) << 20), 0);
+        down = __hiloint2double((int)((1023 + 52 - B) << 20), 0);
+        const double cB = fp_reduce(__hiloint2double((int)((1023 + B - 52) << 20), 0), m);
+        wB = FpTw{cB, cB * m.qinv};
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            hi[i] = base;
+            lo[i] = f[i] = 0.0;
+        }
+    }
+    __device__ __forceinline__ void fold() {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            f[i] = fp_reduce(f[i] + fp_mulmod((hi[i] - base) * down, wB, m) + fp_reduce(lo[i], m), m);
+            hi[i] = base;
+            lo[i] = 0.0;
+        }
+        pending = 0;
+    }
+    // v: words of the two coefficients; k: the key polynomials' words, [polynomial][coefficient]
+    __device__ __forceinline__ void add(const uint64_t *v, const uint64_t (*k)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            const double x = fp_from_u64(v[c]);
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                const double w = fp_from_u64(k[r][c]), t = __builtin_fma(x, w, hi[2 * r + c]);
+                lo[2 * r + c] += __builtin_fma(x, w, -(t - hi[2 * r + c]));
+                hi[2 * r + c] = t;
+            }
+        }
+        if (++pending == period) fold();
+    }
+    __device__ __forceinline__ void finish(uint64_t (*o)[2]) {
+        if (pending) fold();
+#pragma unroll
+        for (int i = 0; i < 4; i++) o[i >> 1][i & 1] = fp_to_u64(fp_canonical(f[i], m));
+    }
+};
+
+// Any prime: sums of partial products (Lazy3)
+struct HoistSumsInt {
+    Lazy3 s[4], h[4];
+    uint64_t q, r0, r1;
+    uint32_t period, pending;
+    __device__ __forceinline__ HoistSumsInt(uint64_t q_, uint64_t r0_, uint64_t r1_) : q(q_), r0(r0_), r1(r1_) {
+        period = (q >> 60) ? 4 : 8;
+        pending = 0;
+#pragma unroll
+        for (int i = 0; i < 4; i++) s[i] = h[i] = Lazy3{0, 0, 0};
+    }
+    __device__ __forceinline__ void add(const uint64_t *v, const uint64_t (*k)[2]) {
+#pragma unroll
+        for (int c = 0; c < 2; c++) mac3x2(s[c], s[2 + c], split30(v[c]), split30(k[0][c]), split30(k[1][c]));
+        if (++pending == period) {
+#pragma unroll
+            for (int i = 0; i < 4; i++) spill3(h[i], s[i]);
+            pending = 0;
+        }
+    }
+    __device__ __forceinline__ void finish(uint64_t (*o)[2]) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const U128 a = total3(h[i], s[i]);
+            o[i >> 1][i & 1] = barrett128(a.lo, a.hi, q, r0, r1);
+        }
+    }
+};
+
+__device__ __forceinline__ Words2 load_pair(const uint64_t *p) { return *reinterpret_cast<const Words2 *>(p); }
+__device__ __forceinline__ Words2 stream_pair(const uint64_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const Words2 *>(p)); }
+
+// The two words that an automorphism brings to coefficients j and j + 1 (j even), src its gather index of j: odd elements
+// keep aligned pairs of the NTT order together, so they are one 16-byte access, in their order or turned round.
+__device__ __forceinline__ void turned(uint64_t *v, Words2 w, uint32_t src) {
+    v[0] = src & 1 ? w.y : w.x;
+    v[1] = src & 1 ? w.x : w.y;
+}
+
+// Terms [first, last) of limb t for the coefficients j, j + 1 of every lane; two terms are multiplied while the next two are
+// on their way.
+template <class Sums>
+__device__ __forceinline__ void hoist_terms(const HoistArgs &p, uint32_t t, uint32_t table, uint32_t j, uint32_t first, uint32_t last,
+                                            Sums &sums) {
+    constexpr uint32_t U = 2;
+    const uint32_t LK = p.L + p.K;
+    const uint64_t *y = p.y + ((size_t)t << p.log_n), *c1 = p.c0 + ((size_t)(p.L + t) << p.log_n);
+    const size_t key_off = ((size_t)table << p.log_n) + j, key_poly = (size_t)(p.size_q + p.K) << p.log_n;
+    const size_t digit = (size_t)LK << p.log_n;
+    const uint32_t own = (p.own_from_ct && t < p.L) ? t / p.K : 0xffffffffu;
+    uint32_t st = first / p.beta, d = first - st * p.beta, src = galois_index(j, p.elts[st], p.log_n);
+    Words2 k[2][U][2], w[2][U];
+    uint32_t turn[2][U];
+    uint32_t at = first;
+    auto fetch = [&](int b) {
+#pragma unroll
+        for (int u = 0; u < (int)U; u++) {
+            if (at >= last) break;
+            const uint64_t *key = p.evk.p[at] + key_off;
+            k[b][u][0] = stream_pair(key);
+            k[b][u][1] = stream_pair(key + key_poly);
+            w[b][u] = load_pair((d == own ? c1 : y + d * digit) + (src & ~1u));
+            turn[b][u] = src;
+            if (++d == p.beta) {
+                d = 0;
+                st++;
+                if (at + 1 < last) src = galois_index(j, p.elts[st], p.log_n);
+            }
+            at++;
+        }
+    };
+    auto take = [&](int b, uint32_t e) {
+#pragma unroll
+        for (int u = 0; u < (int)U; u++) {
+            if (e + u >= last) break;
+            uint64_t v[2], kk[2][2];
+            turned(v, w[b][u], turn[b][u]);
+#pragma unroll
+            for (int r = 0; r < 2; r++) {
+                kk[r][0] = k[b][u][r].x;
+                kk[r][1] = k[b][u][r].y;
+            }
+            sums.add(v, kk);
+        }
+    };
+    if (first >= last) return;
+    fetch(0);
+    for (uint32_t e = first;; e += 2 * U) {
+        if (e + U < last) fetch(1);
+        __builtin_amdgcn_sched_barrier(0);   // (the loads stay ahead of the products)
+        take(0, e);
+        if (e + U >= last) return;
+        if (e + 2 * U < last) fetch(0);
+        __builtin_amdgcn_sched_barrier(0);
+        take(1, e + U);
+        if (e + 2 * U >= last) return;
+    }
+}
+
+// Hoisted rotations of one ciphertext (hoist_inner_kernel's rows, same results).  Every key word is read once, so the kernel is
+// bound by that stream when there are many limbs and by the chain of a wave's terms when there are few.  A lane serves two
+// neighbouring coefficients with 16-byte accesses; an XCD takes a contiguous eighth of the (limb, block) sequence, so that
+// the words which the steps gather from a limb come from its own L2 after the first step, and the keys pass by without
+// staying there.  SPLIT = 4: the four waves of a workgroup deal the terms of one block out and add their sums in LDS.
+// Against one coefficient per lane, one term ahead, blocks dealt to the XCDs in turn: hoisting of 7 steps at N = 2^16,
+// L = 24, K = 8 303 -> 248 us (704 MB of keys, 5.5 TB/s in this kernel), of 15 steps at L = 2, K = 1 60 -> 52 us.
+template <int SPLIT>
+__global__ __launch_bounds__(kThreads) void hoist_one_kernel(HoistArgs p) {
+    constexpr uint32_t PER = 2 * kThreads / SPLIT;   // coefficients of a workgroup
+    __shared__ uint64_t part_lds[SPLIT > 1 ? SPLIT : 1][2][SPLIT > 1 ? PER : 1];
+    touch_arguments<sizeof(HoistArgs)>();
+    const uint32_t LK = p.L + p.K, log_b = p.log_n - (SPLIT == 1 ? 9 : 7), heavy = LK << log_b;
+    const uint32_t lane = threadIdx.x & 63, wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint32_t id = blockIdx.x;
+    auto contiguous = [](uint32_t i, uint32_t n) { return n % 8 == 0 ? (i & 7) * (n >> 3) + (i >> 3) : i; };
+    if (id >= heavy) {
+        // sums of the permuted c0, and the copy of c1
+        id = contiguous(id - heavy, gridDim.x - heavy);
+        const uint32_t t = id >> (p.log_n - 9), j = ((id & ((1u << (p.log_n - 9)) - 1)) << 9) + 2 * threadIdx.x;
+        const size_t o = ((size_t)t << p.log_n) + j;
+        Words2 *out = reinterpret_cast<Words2 *>(p.c0_out + o);
+        if (t >= p.L) {
+            if (!p.accumulate) *out = load_pair(p.c0 + o);
+            return;
+        }
+        const uint64_t q = scalar(p.moduli)[t];
+        const uint64_t *in = p.c0 + ((size_t)t << p.log_n);
+        Words2 acc = p.accumulate ? *out : p.with_self ? load_pair(in + j) : Words2{0, 0};
+#pragma unroll 4
+        for (uint32_t s = 0; s < p.n_steps; s++) {
+            const uint32_t g = galois_index(j, p.elts[s], p.log_n);
+            uint64_t v[2];
+            turned(v, load_pair(in + (g & ~1u)), g);
+            acc.x = add_mod(acc.x, v[0], q);
+            acc.y = add_mod(acc.y, v[1], q);
+        }
+        *out = acc;
+        return;
+    }
+    id = contiguous(id, heavy);
+    const uint32_t t = id >> log_b, base = (id & ((1u << log_b) - 1)) * PER, table = t < p.L ? t : p.size_q + (t - p.L);
+    const uint32_t j = base + (SPLIT == 1 ? 128 * wave : 0) + 2 * lane;
+    const uint32_t n_terms = p.n_steps * p.beta, share = (n_terms + SPLIT - 1) / SPLIT;
+    const uint32_t first = SPLIT == 1 ? 0 : wave * share, last = SPLIT == 1 || first + share > n_terms ? n_terms : first + share;
+    const uint64_t q = scalar(p.moduli)[table];
+    uint64_t o[2][2];
+    if (table < 64 && ((p.fp_mask >> table) & 1)) {
+        HoistSumsFp sums(p.fp_consts + 4 * (size_t)table, q, n_terms);
+        hoist_terms(p, t, table, j, first, last, sums);
+        sums.finish(o);
+    } else {
+        HoistSumsInt sums(q, scalar(p.barrett)[2 * table], scalar(p.barrett)[2 * table + 1]);
+        hoist_terms(p, t, table, j, first, last, sums);
+        sums.finish(o);
+    }
+    if constexpr (SPLIT > 1) {
+#pragma unroll
+        for (int r = 0; r < 2; r++)
+#pragma unroll
+            for (int c = 0; c < 2; c++) part_lds[wave][r][2 * lane + c] = o[r][c];
+        __syncthreads();
+        if (wave > 1) return;
+#pragma unroll
+        for (int c = 0; c < 2; c++) {
+            uint64_t v = part_lds[0][wave][2 * lane + c];
+#pragma unroll
+            for (int i = 1; i < SPLIT; i++) v = add_mod(v, part_lds[i][wave][2 * lane + c], q);
+            o[0][c] = v;
+        }
+    }
+#pragma unroll
+    for (int r = 0; r < (SPLIT > 1 ? 1 : 2); r++) {
+        Words2 *out = reinterpret_cast<Words2 *>(p.out + ((size_t)((SPLIT > 1 ? wave : (uint32_t)r) * LK + t) << p.log_n) + j);
+        Words2 v{o[r][0], o[r][1]};
+        if (p.accumulate) {
+            const Words2 old = *out;
+            v.x = add_mod(v.x, old.x, q);
+            v.y = add_mod(v.y, old.y, q);
+        }
+        *out = v;
+    }
+}
+
 // ---------------------------------------------------------------------------------------------------
 // samplers: ChaCha20 block function (RFC 8439 section 2.3), 64-bit block counter in words 12-13,
 // 64-bit stream id in words 14-15
@@ -1130,6 +1369,18 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
     // ... or inside the aligned stretches of 4,096 words (steps that are multiples of N / 8192)
     bool stretch_local = t.log_n >= 12;
     for (uint32_t i = 0; i < n_steps && stretch_local; i++) stretch_local = ((elts[i] - 1) & ((1u << (t.log_n - 11)) - 1)) == 0;
+    // One ciphertext: four waves share a block as long as that leaves at most four waves on a SIMD (hoisting split / unsplit:
+    // n = 2^12, 3 + 1 limbs, 7 steps of 2 digits 28.2 / 31.4 us; n = 2^15, 10 + 3 limbs, 5 steps of 4 digits 100.0 / 101.7 us;
+    // from 2^16 x 12 limbs on the unsplit form wins, 99.7 against 102.5 us, and 247.9 against 255.9 us at L = 24, K = 8)
+    const bool hoist_split = n_steps * beta >= 4 && ((uint64_t)(L + K) << (t.log_n - 7)) <= 4096;
+    if (items == 1 && t.log_n >= 9) {
+        const uint32_t light = (rows - (L + K)) << (t.log_n - 9);
+        if (hoist_split)
+            hipLaunchKernelGGL(hoist_one_kernel<4>, dim3(((L + K) << (t.log_n - 7)) + light), dim3(kThreads), 0, s, p);
+        else
+            hipLaunchKernelGGL(hoist_one_kernel<1>, dim3(((L + K) << (t.log_n - 9)) + light), dim3(kThreads), 0, s, p);
+        return hipGetLastError();
+    }
     const bool p_xcd_ok = !no_xcd && (nb * rows) % 8 == 0;
     auto launch = [&](auto kernel, uint32_t per) {
         p.groups = (items + per - 1) / per;
@@ -1145,10 +1396,8 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
     // 452 against 498 us for 15 steps of 45 items at N = 2^16); the block-local form keeps 4 (389 against 500 us).
     if (items >= 4 && (local || !p_xcd_ok)) {
         HE_HOIST(4);
-    } else if (items >= 2) {
-        HE_HOIST(2);
     } else {
-        HE_HOIST(1);
+        HE_HOIST(2);
     }
 #undef HE_HOIST
     return hipGetLastError();

@@ -118,3 +118,30 @@ def test_bounded_encoding_and_real_decoding(oracle, capi, chain, logn, slots, li
         assert (real.numpy()[0] == values).all() and (batch[k] == values).all(), k
         if limbs > 1 or k == 1:
             assert np.abs(values[:count] - z[0, k][:take]).max() < 2.0 ** -18, k
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,size_p,L,n_steps", [(9, 1, 4, 1), (9, 2, 3, 40), (12, 2, 4, 1), (12, 2, 3, 2), (13, 1, 5, 1), (14, 1, 4, 16),
+                                                   (16, 2, 4, 3)])
+def test_hoisting_of_one_ciphertext(oracle, capi, chain, logn, size_p, L, n_steps):
+    """he_hoisted_rotations with fewer, as many and more terms than the waves that share a block (3, 4, 5: one is left without),
+    in one launch and in several that add up, with and without the input added."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], size_p)
+    rng = np.random.default_rng(n_steps)
+    lib, h = capi.lib(), ctx.he_handle()
+    beta = -(-L // size_p)
+    host = [[rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(beta)] for _ in range(2)]
+    dev = [[DeviceArray(capi, host=d) for d in key] for key in host]
+    # elements of every residue modulo 4 and 8: neighbouring words keep their order or are turned round
+    elts = [(pow(5, 3 * k + 1, 2 * p.n) * (2 * p.n - 1 if k % 2 else 1)) % (2 * p.n) for k in range(n_steps)]
+    flat = capi.evk_array([dev[i % 2][d].ptr for i in range(n_steps) for d in range(beta)])
+    d_elts = (C.c_uint32 * n_steps)(*elts)
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, 1),))
+    ct = rand_limbs(p, rng, range(L), n_polys=2)
+    want = p.hoisting(ct, elts, [host[i % 2] for i in range(n_steps)])
+    din, dout = DeviceArray(capi, host=ct), DeviceArray(capi, shape=(2, L, p.n))
+    capi.check(lib.he_hoisted_rotations(h, L, din.ptr, flat, d_elts, n_steps, dout.ptr, ws.ptr, None))
+    assert (dout.numpy() == want).all()
+    capi.check(lib.he_hoisted_rotations_batch(h, L, 1, din.ptr, flat, d_elts, n_steps, 1, dout.ptr, ws.ptr, None))
+    assert (dout.numpy() == np.stack([p.add(want[i], ct[i]) for i in range(2)])).all()
+    assert (din.numpy() == ct).all()
