@@ -263,7 +263,7 @@ bool fp_for_level(const he_context *ctx, uint32_t L) {
 
 // base conversion fused with the rows pass of the forward transform that follows it (launch_bconv_rows)
 bool fuse_rows_ok(const he_context *ctx, const Level *lv, uint32_t L) {
-    return ctx->fuse_rows && !ctx->single_limb_digits && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16 && fp_for_level(ctx, L);
+    return ctx->fuse_rows && !ctx->single_limb_digits && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16;
 }
 
 int check_map(const he_context *ctx, uint32_t limbs, uint32_t first, uint32_t split, uint32_t tail) {
@@ -931,10 +931,12 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
                                     c + (size_t)d * n, (size_t)c_item_stride * n * sizeof(uint64_t), n * sizeof(uint64_t),
                                     items, hipMemcpyDeviceToDevice, S(s)));
     } else if (fused) {
-        BconvRows b{ws, out, c, lv->d_mats_fp, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
+        const int backend = backend_for_level(ctx, L);
+        BconvRows b{ws, out, c, fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
                     lv->beta, lv->modup_max_rows, copy_rows,
-                    items, (size_t)L * n, (size_t)lv->beta * LK * n, (size_t)c_item_stride * n, 0, lv->d_mx_up};
-        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, ctx->tune, S(s)));
+                    items, (size_t)L * n, (size_t)lv->beta * LK * n, (size_t)c_item_stride * n, 0, lv->d_mx_up,
+                    nullptr, lv->d_mats, nullptr, ctx->size_p};
+        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend, ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{ws, out, c, lv->d_mats, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
                      lv->beta, lv->modup_max_rows, copy_rows, lv->d_mats_fp, ctx->d_fp_consts,
@@ -1035,9 +1037,10 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     } else if (batched) {
         const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
         if (fused) {
-            BconvRows b{cx, ws, nullptr, ctx->d_phat_mod_q_fp, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
-                        items, (size_t)units * LK * n, (size_t)units * L * n, 0, 0};
-            HE_HIP(launch_bconv_rows(base_args(ctx, true), b, ctx->tune, S(s)));
+            BconvRows b{cx, ws, nullptr, fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
+                        items, (size_t)units * LK * n, (size_t)units * L * n, 0, 0, nullptr, nullptr,
+                        ctx->d_phat_mod_q, nullptr, K};
+            HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L, 0)), ctx->tune, S(s)));
         } else {
             BconvBatch b{cx, ws, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
                          fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_fp_consts,
@@ -1320,10 +1323,12 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     if (k1) {
     } else if (fused) {
         // with the prologue of (4) and the rows pass of its transform
-        BconvRows b{cx, delta, nullptr, ctx->d_phat_pinv_fp, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,
+        const bool fp = fp_for_level(ctx, L);
+        BconvRows b{cx, delta, nullptr, fp ? ctx->d_phat_pinv_fp : nullptr, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,
                     items, 2 * (size_t)LK * n, 2 * (size_t)L * n, 0, 1, ctx->d_mx_down,
-                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr};
-        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, ctx->tune, S(s)));
+                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr,
+                    ctx->d_phat_mod_q, ctx->d_pinv_mod_q, K};
+        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L - 1, 0), (int)L - 1), ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{cx, delta, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,
                      fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_fp_consts,

@@ -10,7 +10,7 @@ namespace he {
 // that select bit-identical alternates): the launchers read nothing from the environment themselves.
 struct Tuning {
     uint32_t cus = 256;              // compute units of the context's device
-    uint32_t fuse_rows_forced = 0;   // CAHEL_HIP_FUSE_ROWS: output limbs per workgroup of bconv_rows_fp_kernel, 0 = chosen per launch
+    uint32_t fuse_rows_forced = 0;   // CAHEL_HIP_FUSE_ROWS: output limbs per workgroup of the fused base conversions, 0 = chosen per launch
     uint32_t bconv_rows = 6;         // CAHEL_HIP_BCONV_ROWS: output rows per workgroup of the batched base conversion
     bool hoist_no_local = false;     // CAHEL_HIP_NO_LOCAL_HOIST=1
     bool hoist_no_xcd = false;       // CAHEL_HIP_NO_XCD_MAP=1
@@ -247,7 +247,7 @@ struct BconvBatch {
 };
 hipError_t launch_bconv_batched(const Tables &t, const BconvBatch &b, const Tuning &tune, hipStream_t s);
 
-// Base conversion fused with the rows pass of the forward transform of its output limbs (FP64 back end, N >= 2^12,
+// Base conversion fused with the rows pass of the forward transform of its output limbs (N >= 2^12,
 // n_in <= 8): the units of a BconvBatch, with the results left as the lazy words that the blocks pass continues on.
 struct BconvRows {
     const uint64_t *x_base;
@@ -275,10 +275,17 @@ struct BconvRows {
     // stores byte i of r = (t - sum_i x_i M[last][i]) mod q_last there, and the records of mx_tab multiply it by the
     // digits of 2^(8 i) mod q_r.
     const void *mx_last;
+    // levels with a prime from 2^50 on (mat_fp == nullptr): the matrix in integers at mat_off, and, mdr, P^-1 mod q_j (Shoup pairs)
+    const uint64_t *mat;
+    const uint64_t *w;
+    uint32_t max_in;             // the most input limbs of a unit, at most 8
 };
 constexpr uint32_t kMxRecord = 144;
 // `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
-hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, const Tuning &tune, hipStream_t s);
+// and `backend` says what the blocks pass that follows runs on
+hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s);
+hipError_t launch_bconv_rows4(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups,
+                              uint32_t rows_per, int backend, hipStream_t s);
 
 constexpr int kMaxDigits = 64;
 struct EvkPtrs {

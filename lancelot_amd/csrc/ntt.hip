@@ -10,11 +10,10 @@
 //                 tile of R rows x C columns in LDS; global accesses run along the columns (C consecutive words
 //                 per row).
 //   blocks pass : the last 8 stages stay inside one row (256 consecutive words), which a wave owns.
-// The passes themselves are in ntt_passes.hip.  The forward transform runs rows pass then blocks pass, the inverse
-// the other way round.  This file holds what replaces or fuses them: the whole-limb kernel of the small degrees, the base
-// conversions with the rows pass that follows, the inner product with the blocks pass before it, the tensor product
-// with the inverse blocks pass after it.  Fused kernels work on 8 or 16 words per thread; their LDS indices are skewed by
-// one word per 16 so that both the stride-16 and the stride-256 gathers of a wave hit distinct banks.
+// The forward transform runs rows pass then blocks pass, the inverse
+// the other way round.  The passes, and the inner product, the tensor product, encryption and decryption fused with the blocks pass,
+// are in ntt_passes.hip, base conversions fused with the rows pass in ntt_bconv.hip.  This file holds the whole-limb kernel of the
+// small degrees and the conversion on the matrix cores, and chooses between them.
 //
 // Two arithmetic back ends share this skeleton:
 //   integer : 64-bit Shoup/Harvey butterflies, any prime below 2^61 (~35 VALU instructions per butterfly);
@@ -160,77 +159,32 @@ inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_
     return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && n_jobs >= 64) || (a.log_n == 14 && forward && n_jobs >= 192);
 }
 
-// ---------------------------------------------------------------------------------------------------
-// Base conversion fused with the rows pass of the forward transform that follows it (FP64 back end, N >= 2^12).
-//
-// Both operate on the same set of coefficients: a tile of all 2^LD rows x C columns of the limb's (N / 256) x 256
-// view.  A workgroup of 256 threads owns a tile of 2048 coefficients (8 per thread) of one unit (a ModUp digit or a
-// ModDown polynomial) and a group of the unit's output limbs.  Every thread keeps its 8 coefficients of the unit's
-// (at most 8) input limbs in registers; for each output limb of the group it forms sum_i x_i M[r][i] for its
-// coefficients, which are exactly the 8 words of its first register block of the rows pass (rows 2^(LD-3) apart),
-// runs the first three stages on them, and the tile then crosses LDS between the remaining register blocks.  The
-// converted limbs never exist in coefficient form in memory: 2 limb transfers and one launch less per output limb
-// than conversion kernel + rows pass.  The groups of one tile re-read the same inputs (from L2: they run on one XCD).
-//
-// mdr (merged ModDown + rescale): the last matrix row belongs to the limb that the rescale drops; with
-// r = t - sum_i x_i M[last][i] mod q_last (t: the limb right before the unit's inputs), output limb j receives
-// sum_i x_i M[j][i] + (r mod q_j); the matrix carries the factor P^-1.
-// ---------------------------------------------------------------------------------------------------
 constexpr int kFuseLog = 11;
 constexpr uint32_t kFuseWords = 1u << kFuseLog;
-
-// LDS index of tile word e: 8 words of padding per 32 and 8 more per 256, so that the 32 lanes of a half-wave that
-// read the words {32 a + 8 j + c}, {256 u + 32 j + c'} or {256 u + 32 j + 8 w + c} of one register slot j hit distinct
-// 8-byte banks
-__device__ __forceinline__ uint32_t skew8(uint32_t e) { return e + ((e >> 5) << 3) + ((e >> 8) << 3); }
-constexpr uint32_t kFuseLds = kFuseWords + (kFuseWords >> 2) + (kFuseWords >> 5);
 
 struct BconvRowsK {
     BconvRows b;
     uint32_t compute_groups, copy_groups, rows_per;
 };
 
-// register block of LOGR stages on the groups of a tile that lives in LDS (tile index bits: [upper][LOGR bits][low_bits]);
-// P words per thread; twl: entries 0..255 of the limb's twiddle table, in LDS; LAST: the results go to global memory
-// (lazy signed doubles for the blocks pass), else back to LDS
-template <int LD, int P, int LOGR, bool LAST, bool SWZ = false>
-__device__ __forceinline__ void fuse_block(double *ld, const double *twl, uint32_t s0, FpMod m, uint64_t *dst, uint32_t col0) {
-    auto slot = [](uint32_t e) { return SWZ ? e ^ ((((e >> 5) ^ (e >> 8)) & 3u) << 3) : skew8(e); };
-    constexpr int LOGC = kFuseLog - LD;
-    constexpr uint32_t C = 1u << LOGC, T = kFuseWords / P;
-    constexpr int R = 1 << LOGR, PER = P >> LOGR;
-    const uint32_t low_bits = (uint32_t)(LD - LOGR + LOGC) - s0;
-    const uint32_t low_mask = (1u << low_bits) - 1;
-#pragma unroll
-    for (int gi = 0; gi < PER; gi++) {
-        const uint32_t g = threadIdx.x + T * gi;
-        const uint32_t upper = g >> low_bits;
-        const uint32_t base = (upper << (low_bits + LOGR)) | (g & low_mask);
-        double v[R];
-#pragma unroll
-        for (int j = 0; j < R; j++) v[j] = ld[slot(base + ((uint32_t)j << low_bits))];
-        fp_ct_block<LOGR, 2>(v, twl, (1u << s0) + upper, m);
-#pragma unroll
-        for (int j = 0; j < R; j++) {
-            const uint32_t e = base + ((uint32_t)j << low_bits);
-            if (LAST)
-                dst[(size_t)(e >> LOGC) * 256 + col0 + (e & (C - 1))] = (uint64_t)__double_as_longlong(v[j]);
-            else
-                ld[slot(e)] = v[j];
-        }
-    }
-}
+// see the matrix-core kernel below
+__device__ __forceinline__ uint32_t swz8(uint32_t e) { return e ^ ((((e >> 5) ^ (e >> 8)) & 3u) << 3); }
 
-// the stages S0 .. LD-1 of the rows pass, in register blocks of at most log2(P) stages with the tile in LDS between them
-template <int LD, int P, int S0>
-__device__ __forceinline__ void fuse_rest(double *ld, const double *twl, FpMod m, uint64_t *dst, uint32_t col0) {
-    constexpr int LOGP = P == 8 ? 3 : 2;
-    constexpr int LOGR = (LD - S0) < LOGP ? (LD - S0) : LOGP;
-    constexpr bool LAST = S0 + LOGR == LD;
-    fuse_block<LD, P, LOGR, LAST>(ld, twl, S0, m, dst, col0);
-    if constexpr (!LAST) {
-        lds_barrier();
-        fuse_rest<LD, P, S0 + LOGR>(ld, twl, m, dst, col0);
+// the last two stages of a tile that lives in LDS, 8 words per thread; twl: entries 0..255 of the limb's twiddle table, in LDS;
+// the results go to global memory as lazy signed doubles for the blocks pass
+__device__ __forceinline__ void fuse_last(const double *ld, const double *twl, FpMod m, uint64_t *dst, uint32_t col0) {
+#pragma unroll
+    for (int gi = 0; gi < 2; gi++) {
+        const uint32_t g = threadIdx.x + 256 * gi, upper = g >> 3, base = (upper << 5) | (g & 7);
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = ld[swz8(base + ((uint32_t)j << 3))];
+        fp_ct_block<2, 2>(v, twl, 64u + upper, m);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const uint32_t e = base + ((uint32_t)j << 3);
+            dst[(size_t)(e >> 3) * 256 + col0 + (e & 7)] = (uint64_t)__double_as_longlong(v[j]);
+        }
     }
 }
 
@@ -245,195 +199,9 @@ __device__ __forceinline__ double uniform_f64(double v) {
 // strides over the workgroup, whatever its size)
 constexpr uint32_t kFuseMaxRows = 24;
 
-// P = coefficients per thread.  8: 256 threads, two waves per SIMD.  (4, with 512 threads and four waves per SIMD,
-// compiles but measured 1.7 times slower at N = 2^16: the inputs' registers spill, and a tile needs twice the LDS
-// exchanges and barriers.)
-//
-// Thread -> coefficient mapping.  The thread's P words are rows row0 + i 2^(LD-3) of one column (the first register
-// block pairs exactly these).  At N = 2^16 (LD = 8: 256 rows x 8 columns) wave w takes row0 = w + 4 j, j = lane / 8:
-// the second register block (stages 3..5, rows that differ in bits 2..4) then exchanges words inside the wave only, so
-// the tile needs one workgroup barrier per output limb (before the last block) instead of three; the tile and the
-// twiddles are double / triple buffered so that the next limb's first block never waits for this limb's last one.
-// Other degrees use row0 = thread / C and a barrier after every block.
-template <int LD, int P>
-__global__ __launch_bounds__(kFuseWords / P) __attribute__((amdgpu_waves_per_eu(P == 8 ? 2 : 4)))
-void bconv_rows_fp_kernel(NttArgs a, BconvRowsK p) {
-    constexpr bool WAVE_B = LD == 8 && P == 8;
-    __shared__ double ld[WAVE_B ? 2 : 1][kFuseLds];
-    __shared__ double twl[3][256];
-    __shared__ double mrow[kFuseMaxRows][18];
-    __shared__ uint32_t mlimb[kFuseMaxRows], mtable[kFuseMaxRows];
-    static_assert(LD >= 4 && LD <= 8 && (P == 8 || P == 4), "N from 2^12 to 2^16");
-    constexpr int LOGC = kFuseLog - LD, LOGP = P == 8 ? 3 : 2;
-    constexpr uint32_t T = kFuseWords / P;
-    constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC, row_step = T >> LOGC;
-    const size_t n = (size_t)1 << a.log_n;
-
-    // consecutive logical ids (one XCD, one L2): the groups of one tile, which read the same inputs
-    uint32_t lb = logical_block();
-    const uint32_t groups = p.compute_groups + p.copy_groups;
-    const uint32_t grp = lb % groups;
-    lb /= groups;
-    const uint32_t tile = lb % tiles_per_limb, uidx = lb / tiles_per_limb;
-    const uint32_t item = uidx / p.b.n_units;
-    const BconvDesc d = p.b.descs[uidx - item * p.b.n_units];
-    const uint32_t col0 = tile << LOGC;
-    // word i of this thread: row row0 + i row_step, column col of the tile = tile word e0 + T i
-    const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const uint32_t row0 = WAVE_B ? wave + 4 * (lane >> 3) : threadIdx.x >> LOGC;
-    const uint32_t col = threadIdx.x & (C - 1);
-    const uint32_t e0 = (row0 << LOGC) + col;
-    const size_t g0 = (size_t)row0 * 256 + col0 + col;
-    constexpr size_t gstep = (size_t)row_step * 256;
-    uint64_t *out = p.b.out_base + item * p.b.out_item_stride + d.out_off;
-
-    if (grp >= p.compute_groups) {
-        // limbs that pass through unchanged (a digit's own limbs keep their NTT form)
-        const uint64_t *from = p.b.copy_base + item * p.b.copy_item_stride;
-        const uint32_t first = (grp - p.compute_groups) * p.rows_per;
-        for (uint32_t r = first; r < first + p.rows_per && r < d.copy_count; r++) {
-            const size_t limb = (size_t)(d.copy_first + r) << a.log_n;
-            uint64_t w[P];
-#pragma unroll
-            for (int i = 0; i < P; i++) w[i] = from[limb + g0 + gstep * i];
-#pragma unroll
-            for (int i = 0; i < P; i++) out[limb + g0 + gstep * i] = w[i];
-        }
-        return;
-    }
-    const uint32_t n_rows = p.b.mdr ? d.n_out - 1 : d.n_out;
-    const uint32_t r_begin = grp * p.rows_per;
-    const uint32_t r_end = r_begin + p.rows_per < n_rows ? r_begin + p.rows_per : n_rows;
-    if (r_begin >= n_rows) return;
-
-    // The constants of this group's output limbs (matrix row, modulus, output limb, table) go to LDS once, and are
-    // read back into scalar registers limb by limb: a scalar load per limb would stall the workgroup for a cache miss.
-    const double *mat = p.b.mat_fp + 2 * d.mat_off;
-    for (uint32_t w = threadIdx.x; w < (r_end - r_begin) * 18; w += T) {
-        const uint32_t rl = w / 18, c = w - rl * 18, r = r_begin + rl;
-        const uint32_t table = p.b.out_table[d.map_off + r];
-        // (the matrices are padded: 8 pairs can be fetched whatever the row's length)
-        mrow[rl][c] = c < 16 ? mat[2 * (size_t)r * d.n_in + c] : a.fp_consts[4 * (size_t)table + (c - 16)];
-        if (c == 0) {
-            mlimb[rl] = p.b.out_limb[d.map_off + r];
-            mtable[rl] = table;
-        }
-    }
-    // entries 1..255 of the first limb's table: every twiddle of the rows pass
-    double tw_cur = a.tw_fp[((size_t)p.b.out_table[d.map_off + r_begin] << a.log_n) + (threadIdx.x & 255)];
-
-    // the unit's inputs at this thread's P coefficients (limbs past n_in repeat the last one; their matrix entries
-    // are replaced by zero below), all loads in flight together
-    const uint64_t *x = p.b.x_base + item * p.b.x_item_stride + d.x_off;
-    double xv[8][P];
-#pragma unroll
-    for (int k = 0; k < 8; k++) {
-        const uint32_t kk = (uint32_t)k < d.n_in ? (uint32_t)k : d.n_in - 1;
-#pragma unroll
-        for (int i = 0; i < P; i++) xv[k][i] = fp_from_u64(x[((size_t)kk << a.log_n) + g0 + gstep * i]);
-    }
-
-    double rr[P];
-#pragma unroll
-    for (int i = 0; i < P; i++) rr[i] = 0.0;
-    if (p.b.mdr) {
-        // coefficients of the dropped limb of the ModDown result, canonical mod q_last
-        const uint32_t last = d.n_out - 1;
-        const FpMod ml = fp_ctx(a, p.b.out_table[d.map_off + last]).m;
-        const double *row = mat + 2 * (size_t)last * d.n_in;
-        const uint64_t *tsrc = x - n;
-#pragma unroll
-        for (int i = 0; i < P; i++) rr[i] = fp_from_u64(tsrc[g0 + gstep * i]);
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const bool on = (uint32_t)k < d.n_in;
-            const FpTw w{on ? row[2 * k] : 0.0, on ? row[2 * k + 1] : 0.0};
-#pragma unroll
-            for (int i = 0; i < P; i++) rr[i] -= fp_mulmod(xv[k][i], w, ml);
-        }
-#pragma unroll
-        for (int i = 0; i < P; i++) rr[i] = fp_canonical(rr[i], ml);
-    }
-    if (threadIdx.x < 256) twl[r_begin % 3][threadIdx.x] = tw_cur;
-    lds_barrier();
-
-    for (uint32_t r = r_begin; r < r_end; r++) {
-        const uint32_t rl = r - r_begin;
-        // the next output limb's twiddles travel while this one is computed
-        double tw_nxt = 0.0;
-        const bool more = r + 1 < r_end;
-        if (more) tw_nxt = a.tw_fp[((size_t)mtable[rl + 1] << a.log_n) + (threadIdx.x & 255)];
-        const FpMod mod{uniform_f64(mrow[rl][16]), uniform_f64(mrow[rl][17])};
-        const uint32_t limb = __builtin_amdgcn_readfirstlane(mlimb[rl]);
-        const double *tws = twl[r % 3];
-        double *tile_ld = ld[WAVE_B ? (r & 1) : 0];
-        // sum_k x_k M_k as an exact pair (hi, lo) before any reduction, four operations per term instead of the seven of
-        // a modular product and an addition.  hi runs in [2^103, 2^104), where doubles are the multiples of 2^51: the
-        // fused multiply-add t = fl(x w + hi) rounds the exact sum to such a multiple (eight products below 2^100 keep
-        // it under 2^104), t - hi is exact, x w - (t - hi) is the rounding error, an integer of at most 2^50 in
-        // magnitude that the second fused multiply-add returns exactly, and eight of those sum exactly (<= 2^53).
-        // The value is (hi - 2^103) + lo; it is reduced once per output word.
-        double hi[P], lo[P];
-#pragma unroll
-        for (int i = 0; i < P; i++) {
-            hi[i] = 0x1p103;
-            lo[i] = 0.0;
-        }
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            const double w = (uint32_t)k < d.n_in ? uniform_f64(mrow[rl][2 * k]) : 0.0;
-#pragma unroll
-            for (int i = 0; i < P; i++) {
-                const double t = __builtin_fma(xv[k][i], w, hi[i]);
-                const double step = t - hi[i];
-                lo[i] += __builtin_fma(xv[k][i], w, -step);
-                hi[i] = t;
-            }
-        }
-        // (hi - 2^103) / 2^51 is an integer below 2^52; times c = 2^51 mod m it is congruent to the high part.  The
-        // modular product takes it as it is: for |x| < 2^52 the quotient estimate is off by at most 1.5 |x| 2^-52 + 1,
-        // so |x c - k m| <= 2.5 m < 2^53 and every step stays exact.  With the rescale term (canonical for the dropped
-        // prime, below 2^50, added as it is) |v| <= 3 m + 2^50 <= 4 x 2^50: the bound that the register blocks of
-        // this pass start from (they reduce only what they do not multiply, see fp_ct_block).
-        const double c51 = fp_reduce(0x1p51, mod);
-        const FpTw w51{c51, c51 * mod.qinv};
-        double v[P];
-#pragma unroll
-        for (int i = 0; i < P; i++) {
-            v[i] = fp_mulmod((hi[i] - 0x1p103) * 0x1p-51, w51, mod) + fp_reduce(lo[i], mod);
-            if (p.b.mdr) v[i] += rr[i];
-        }
-        // the first log2(P) stages pair rows that differ in their top bits: this thread's own P words
-        fp_ct_block<LOGP, 2>(v, tws, 1u, mod);
-#pragma unroll
-        for (int i = 0; i < P; i++) tile_ld[skew8(e0 + T * i)] = v[i];
-        uint64_t *dst = out + ((size_t)limb << a.log_n);
-        if constexpr (WAVE_B) {
-            // stages 3..5 inside the wave: lane (u, col) takes rows 32 u + 4 j + wave, which lanes of this wave wrote
-            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-            const uint32_t u = lane >> 3;
-            const uint32_t base = ((32 * u + wave) << LOGC) + col;
-#pragma unroll
-            for (int j = 0; j < 8; j++) v[j] = tile_ld[skew8(base + ((uint32_t)(4 * j) << LOGC))];
-            fp_ct_block<3, 2>(v, tws, 8u + u, mod);
-#pragma unroll
-            for (int j = 0; j < 8; j++) tile_ld[skew8(base + ((uint32_t)(4 * j) << LOGC))] = v[j];
-            // the twiddles of the next limb become visible with the same barrier (their buffer was last read two
-            // limbs ago, and every wave has passed the barrier of the limb in between)
-            if (more) twl[(r + 1) % 3][threadIdx.x] = tw_nxt;
-            lds_barrier();
-            fuse_block<LD, P, 2, true>(tile_ld, tws, 6, mod, dst, col0);
-        } else {
-            lds_barrier();
-            fuse_rest<LD, P, LOGP>(tile_ld, tws, mod, dst, col0);
-            if (more && threadIdx.x < 256) twl[(r + 1) % 3][threadIdx.x] = tw_nxt;
-            lds_barrier();  // every read of this tile is done before the next output limb overwrites it
-        }
-    }
-}
-
 // ---------------------------------------------------------------------------------------------------
-// The same fusion at N = 2^16 with the matrix product of the conversion on the int8 matrix cores.
+// Base conversion fused with the rows pass of the transform that follows it (ntt_bconv.hip) at N = 2^16, with the matrix product of
+// the conversion on the int8 matrix cores.
 //
 // sum_i x_i M[r][i] mod q_r is a 64-term integer product per 7-bit digit of the constants M_ij = M[r][i] 2^(8 j) mod q_r,
 // over the bytes x_ij of the inputs as they lie in memory (BconvRows::mx_tab).  One v_mfma_i32_16x16x64_i8 forms it for 16
@@ -441,14 +209,14 @@ void bconv_rows_fp_kernel(NttArgs a, BconvRowsK p) {
 // (row rr, coefficient c) in lane 16 rr + c, and
 //     sum_e S_e 2^(7 e) = lo + 2^28 hi,   lo = S_0 + 2^7 S_1 + 2^14 S_2 + 2^21 S_3 < 2^43,  hi likewise,
 // becomes the lazy residue (hi x (2^28 mod q)) mod q + lo with one modular product: 13 FP64-rate operations and two
-// matrix instructions per word against 44 operations for the eight exact multiply-adds on the vector units.
+// matrix instructions per word against 44 operations for the eight exact multiply-adds on the vector units.  (ModUp of one operation
+// at L = 24, K = 8 takes 29.5 us either way, both kernels being short of waves; of eight 147 against 158 us.)
 //
-// Wave w of the workgroup owns the coefficients of rows w + 4 j + 32 i (j, i < 8) of the 256 x 8 tile, as in the kernel
-// above; lane (kg, c) keeps the words of input limbs 2 kg, 2 kg + 1 for coefficient c of each of 32 sets of 16
+// Wave w of the workgroup owns the coefficients of rows w + 4 j + 32 i (j, i < 8) of the 256 x 8 tile; lane (kg, c) keeps the words of input limbs 2 kg, 2 kg + 1 for coefficient c of each of 32 sets of 16
 // coefficients (set (g, i): (j, column) = (2 g + c / 8, c % 8), row w + 4 j + 32 i), which is at once the B operand of the
 // set.  Output rows go four at a time: lane (rr, c) receives row rr's words of every set, i.e. for each g the 8 words
 // i = 0..7 of one first register block, runs the block on them and stores them to row rr's tile in LDS.  The second block
-// (stages 3..5) stays inside the wave tile by tile, the third follows a workgroup barrier, as above.
+// (stages 3..5) stays inside the wave tile by tile, the third follows a workgroup barrier.
 //
 // LDS index of tile word e = (row << 3) | column: bits 4..3 are XORed with bits 6..5 and bits 9..8.  The accesses of
 // a half-wave vary the column and either bit 5 (first block), bits 9..8 (second) or bits 6..5 (third) with bits 4..3
@@ -457,7 +225,6 @@ void bconv_rows_fp_kernel(NttArgs a, BconvRowsK p) {
 // ---------------------------------------------------------------------------------------------------
 typedef int v4i __attribute__((ext_vector_type(4)));
 constexpr uint32_t kMxStride = kFuseWords + 16;
-__device__ __forceinline__ uint32_t swz8(uint32_t e) { return e ^ ((((e >> 5) ^ (e >> 8)) & 3u) << 3); }
 
 template <bool MDR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
@@ -694,7 +461,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
         for (uint32_t rr = 0; rr < nr; rr++) {
             const FpMod mod{uniform_f64(rconst[k & 1][rr][0]), uniform_f64(rconst[k & 1][rr][1])};
             const uint32_t limb = __builtin_amdgcn_readfirstlane(rlimb[k & 1][rr]);
-            fuse_block<8, 8, 2, true, true>(tiles + rr * kMxStride, twl[rr], 6, mod, out + ((size_t)limb << 16), col0);
+            fuse_last(tiles + rr * kMxStride, twl[rr], mod, out + ((size_t)limb << 16), col0);
         }
         if (more) {
             // entries 0..63 were last read by the second block, before the barrier above
@@ -707,8 +474,8 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
 
 }  // namespace
 
-hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, const Tuning &tune, hipStream_t s) {
-    if (a.log_n < 12 || a.log_n > 16 || !b.mat_fp || b.n_units == 0) return hipErrorInvalidValue;
+hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s) {
+    if (a.log_n < 12 || a.log_n > 16 || b.n_units == 0) return hipErrorInvalidValue;
     const uint32_t forced = tune.fuse_rows_forced <= kFuseMaxRows ? tune.fuse_rows_forced : 0;
     const uint32_t items = b.items ? b.items : 1;
     const int ld = (int)a.log_n - 8;
@@ -725,8 +492,8 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, const Tuning 
     // the matrix-core kernel (N = 2^16) takes the output rows four at a time
     // (merged ModDown + rescale: the matrix-core kernel first forms the rescale term for its whole tile, two rows' worth of
     // work that pays once a workgroup has many rows, i.e. once the launch fills the chip without splitting the rows:
-    // 98 against 114 us for 8 operations, 27.8 against 25.3 us for one)
-    const bool mx = ld == 8 && b.mx_tab && !tune.no_matrix_bconv &&
+    // 106 against 122 us for 8 operations, 27.8 against 25.4 us for one)
+    const bool mx = ld == 8 && b.mat_fp && b.mx_tab && !tune.no_matrix_bconv &&
                     (!b.mdr || (b.mx_last && (uint64_t)b.n_units * items * tiles >= (tune.cus ? tune.cus : 256)));
     const uint32_t step = mx ? 4 : 1;
     uint32_t target = mx ? (forced + 3) / 4 * 4 : forced;
@@ -755,14 +522,7 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, const Tuning 
             hipLaunchKernelGGL(bconv_rows_mx_kernel<false>, grid, dim3(256), 0, s, a, p);
         return hipGetLastError();
     }
-    switch (ld) {
-#define HE_CASE(LD) \
-    case LD: hipLaunchKernelGGL((bconv_rows_fp_kernel<LD, 8>), grid, dim3(kFuseWords / 8), 0, s, a, p); break;
-        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
-#undef HE_CASE
-        default: return hipErrorInvalidValue;
-    }
-    return hipGetLastError();
+    return launch_bconv_rows4(a, b, p.compute_groups, p.copy_groups, target, backend, s);
 }
 
 hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, hipStream_t s, bool rows_done) {

@@ -1,0 +1,288 @@
+// Base conversion fused with the rows pass of the forward transform that follows it, 4 words per thread, every back end.
+//
+// Both operate on the same set of coefficients: a tile of all N / 256 rows x C columns of a limb's (N / 256) x 256 view.  A workgroup
+// of 512 threads owns a tile of 2048 words of one unit (a ModUp digit or a ModDown polynomial) and a group of the unit's output limbs;
+// a thread keeps its 4 words of each of the (at most 8) input limbs in registers, and for every output limb of the group it
+// forms sum_i x_i M[r][i] and goes straight on with the rows pass (Tile4 of ntt_common.cuh): the converted limbs never
+// exist in coefficient form in memory.  The groups of one tile re-read the same inputs (from L2: they run on one XCD).
+//
+// mdr (merged ModDown + rescale): the last matrix row belongs to the limb that the rescale drops; with
+// r = t - P^-1 sum_i x_i M[last][i] mod q_last (t: the limb right before the unit's inputs), output limb j receives
+// P^-1 sum_i x_i M[j][i] + (r mod q_j).  (FP64: the matrix carries the factor P^-1.)
+//
+// What bounds it: instruction issue, about 380 operations per output word of 64 lanes with 8 input limbs, and the wait for the inputs
+// that every workgroup starts with; 4 words a thread leave room for four waves per SIMD with 8 input limbs in registers (124 of
+// 128; on integers two or three), where 8 words left two.  One product against a kernel with 8 words per thread (FP64 only):
+// n = 2^15, 10 of 12 limbs, K = 3 64.7 -> 55.8 us; n = 2^14, 8 limbs, K = 2 42.6 -> 38.4; a batch of 8, n = 2^15, 12 limbs, K = 4
+// 233 -> 219; L = 24, K = 8 the same 150 us.  Levels with a prime from 2^50 on against conversion kernel + rows pass: n = 2^15, 10 of
+// 12 limbs of 60 / 40 bits 77.5 -> 71.6 us; n = 2^13, 6 limbs, K = 2 45.4 -> 38.3; n = 2^16, 24 + 8 limbs 217 -> 204; a batch of 8,
+// n = 2^15, 12 limbs, K = 3 323 -> 277.
+#include <hip/hip_runtime.h>
+
+#include <type_traits>
+
+#include "kernels.h"
+#include "modarith.cuh"
+#include "ntt_common.cuh"
+
+namespace he {
+
+namespace {
+
+constexpr int kTileLog = 11;
+
+typedef const uint32_t __attribute__((address_space(4))) *ScalarU32;
+__device__ __forceinline__ ScalarU32 scalar(const uint32_t *p) { return (ScalarU32)(uintptr_t)p; }
+
+__device__ __forceinline__ BconvDesc load_desc(const BconvDesc *p) {
+    static_assert(sizeof(BconvDesc) % 8 == 0, "read as 8-byte words");
+    BconvDesc d;
+    uint64_t w[sizeof(BconvDesc) / 8];
+#pragma unroll
+    for (size_t i = 0; i < sizeof(BconvDesc) / 8; i++) w[i] = scalar(reinterpret_cast<const uint64_t *>(p))[i];
+    __builtin_memcpy(&d, w, sizeof(d));
+    return d;
+}
+
+// Conversion in FP64 (every prime of the level below 2^50)
+template <int NIN, bool MDR>
+struct ConvFp {
+    double x[NIN][4], rr[MDR ? 4 : 1];
+    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = fp_from_u64(w); }
+    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvRows &b, const BconvDesc &d, const uint64_t *t) {
+        const uint32_t last = d.n_out - 1;
+        const FpMod m = fp_ctx(a, scalar(b.out_table)[d.map_off + last]).m;
+        const ScalarF64 row = scalar(b.mat_fp) + 2 * (d.mat_off + (size_t)last * d.n_in);
+#pragma unroll
+        for (int j = 0; j < 4; j++) rr[j] = fp_from_u64(t[j]);
+#pragma unroll
+        for (int k = 0; k < NIN; k++) {
+            if ((uint32_t)k >= d.n_in) break;
+            const FpTw w{row[2 * k], row[2 * k + 1]};
+#pragma unroll
+            for (int j = 0; j < 4; j++) rr[j] -= fp_mulmod(x[k][j], w, m);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) rr[j] = fp_canonical(rr[j], m);
+    }
+    // The sum as an exact pair (hi, lo) before any reduction, four operations per term.  hi runs in [2^103, 2^104), where
+    // doubles are the multiples of 2^51: t = fl(x w + hi) rounds the exact sum to such a multiple (eight products below 2^100 keep
+    // it under 2^104), t - hi is exact, x w - (t - hi) is the rounding error, an integer of at most 2^50 in magnitude that the
+    // second fused multiply-add returns exactly, and eight of those sum exactly.  (hi - 2^103) / 2^51 is an integer below
+    // 2^52; times 2^51 mod m it is congruent to the high part, and the modular product takes it as it is.
+    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvRows &b, const BconvDesc &d, uint32_t r, uint32_t,
+                                            const FpArith &ar) const {
+        const ScalarF64 row = scalar(b.mat_fp) + 2 * (d.mat_off + (size_t)r * d.n_in);
+        double hi[4], lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            hi[j] = 0x1p103;
+            lo[j] = 0.0;
+        }
+        double w[NIN];
+#pragma unroll
+        for (int k = 0; k < NIN; k++) w[k] = row[2 * k];   // (the matrices are padded: 8 pairs can be read whatever the row's length)
+#pragma unroll
+        for (int k = 0; k < NIN; k++) {
+            if ((uint32_t)k >= d.n_in) break;
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                const double t = __builtin_fma(x[k][j], w[k], hi[j]);
+                lo[j] += __builtin_fma(x[k][j], w[k], -(t - hi[j]));
+                hi[j] = t;
+            }
+        }
+        const FpMod m = ar.m;
+        const double c51 = fp_reduce(0x1p51, m);
+        const FpTw w51{c51, c51 * m.qinv};
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            v[j] = fp_mulmod((hi[j] - 0x1p103) * 0x1p-51, w51, m) + fp_reduce(lo[j], m);   // below 3 m
+            if constexpr (MDR) v[j] += rr[j];
+        }
+        ar.reduce(v);   // (four stages without a reduction start from at most 1.27 q)
+    }
+};
+
+// Conversion in integers (any primes); the results go to the arithmetic of the output limb.
+template <int NIN, bool MDR>
+struct ConvInt {
+    Split30 x[NIN][4];
+    uint64_t rr[MDR ? 4 : 1];
+    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = split30(w); }
+    // sums of words j, j + 1 (the partial products are relieved every four terms: see Lazy3)
+    __device__ __forceinline__ void sum(uint64_t *o, int j, const uint64_t *row, uint32_t n_in, uint64_t q, uint64_t r0, uint64_t r1) const {
+        Lazy3 s0{0, 0, 0}, s1{0, 0, 0}, h0{0, 0, 0}, h1{0, 0, 0};
+#pragma unroll
+        for (int k = 0; k < NIN; k++) {
+            if ((uint32_t)k >= n_in) break;
+            mac3x2(s0, s1, split30(scalar(row)[k]), x[k][j], x[k][j + 1]);
+            if (k % 4 == 3 && k + 1 < NIN) {
+                spill3(h0, s0);
+                spill3(h1, s1);
+            }
+        }
+        const U128 a0 = total3(h0, s0), a1 = total3(h1, s1);
+        o[0] = barrett128(a0.lo, a0.hi, q, r0, r1);
+        o[1] = barrett128(a1.lo, a1.hi, q, r0, r1);
+    }
+    __device__ __forceinline__ void sums(uint64_t *o, const NttArgs &a, const BconvRows &b, const BconvDesc &d, uint32_t r, uint32_t table) const {
+        const uint64_t q = scalar(a.moduli)[table], r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
+        const uint64_t *row = b.mat + d.mat_off + (size_t)r * d.n_in;
+        sum(o, 0, row, d.n_in, q, r0, r1);
+        sum(o + 2, 2, row, d.n_in, q, r0, r1);
+    }
+    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvRows &b, const BconvDesc &d, const uint64_t *t) {
+        const uint32_t last = d.n_out - 1, table = scalar(b.out_table)[d.map_off + last];
+        const uint64_t q = scalar(a.moduli)[table];
+        const Shoup w = scalar_shoup(b.w, last);
+        uint64_t s[4];
+        sums(s, a, b, d, last, table);
+#pragma unroll
+        for (int j = 0; j < 4; j++) rr[j] = sub_mod(t[j], mul_shoup(s[j], w, q), q);
+    }
+    template <class A>
+    __device__ __forceinline__ void convert(typename A::V *v, const NttArgs &a, const BconvRows &b, const BconvDesc &d, uint32_t r,
+                                            uint32_t table, const A &) const {
+        uint64_t s[4];
+        sums(s, a, b, d, r, table);
+        if constexpr (MDR) {
+            const uint64_t q = scalar(a.moduli)[table], r1 = scalar(a.barrett)[2 * table + 1];
+            const Shoup w = scalar_shoup(b.w, r);
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] = add_mod(mul_shoup(s[j], w, q), barrett64(rr[j], q, r1), q);
+        }
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (std::is_same<A, FpArith>::value)
+                v[j] = fp_from_u64(s[j]);
+            else
+                v[j] = s[j];
+        }
+    }
+};
+
+// FP: the whole level is below 2^50; otherwise the conversion is done in integers and bit `table` of a.fp_mask says in which
+// arithmetic the limb is transformed
+template <int LD, bool FP, int NIN, bool MDR>
+__global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(FP || NIN <= 4 ? 4 : 2)))
+void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per) {
+    using T4 = Tile4<kTileLog, LD>;
+    constexpr int LOGC = kTileLog - LD, NB = T4::kBlocks;
+    constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
+    // (two tiles in turn: the barriers of one output limb say that the tile of the limb before is free again)
+    __shared__ uint64_t lds[2][(1 << kTileLog) + (1 << (kTileLog - 4))];
+    touch_arguments<sizeof(NttArgs) + sizeof(BconvRows)>();
+    const size_t n = (size_t)1 << a.log_n;
+    uint32_t lb = logical_block();
+    const uint32_t groups = compute_groups + copy_groups, grp = lb % groups;
+    lb /= groups;
+    const uint32_t col0 = (lb % tiles_per_limb) << LOGC, uidx = lb / tiles_per_limb, item = uidx / b.n_units;
+    const BconvDesc d = load_desc(b.descs + (uidx - item * b.n_units));
+    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    // word j of layout k: a scalar distance from the lane's first one
+    auto first = [&](int k) {
+        const uint32_t e = T4::word(k, t, 0);
+        return (e >> LOGC) * 256 + col0 + (e & (C - 1));
+    };
+    auto step = [](int k, int j) {
+        const uint32_t e = (uint32_t)j << (kTileLog - 2 * k - 2);
+        return (e >> LOGC) * 256 + (e & (C - 1));
+    };
+    const uint32_t in0 = first(0), out0 = first(NB - 1);
+    uint64_t *out = b.out_base + item * b.out_item_stride + d.out_off;
+    if (grp >= compute_groups) {
+        // limbs that pass through unchanged (a digit's own limbs keep their NTT form)
+        const uint64_t *from = b.copy_base + item * b.copy_item_stride;
+        const uint32_t c0 = (grp - compute_groups) * rows_per;
+        for (uint32_t r = c0; r < c0 + rows_per && r < d.copy_count; r++) {
+            const size_t limb = (size_t)(d.copy_first + r) << a.log_n;
+            uint64_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = (from + limb + step(0, j))[in0];
+#pragma unroll
+            for (int j = 0; j < 4; j++) (out + limb + step(0, j))[in0] = w[j];
+        }
+        return;
+    }
+    const uint32_t n_rows = MDR ? d.n_out - 1 : d.n_out, r_begin = grp * rows_per;
+    const uint32_t r_end = r_begin + rows_per < n_rows ? r_begin + rows_per : n_rows;
+    if (r_begin >= n_rows) return;
+    typename std::conditional<FP, ConvFp<NIN, MDR>, ConvInt<NIN, MDR>>::type conv;
+    const uint64_t *x = b.x_base + item * b.x_item_stride + d.x_off;
+    {
+        uint64_t w[NIN][4], tw[4];
+#pragma unroll
+        for (int k = 0; k < NIN; k++) {
+            const uint32_t kk = (uint32_t)k < d.n_in ? (uint32_t)k : d.n_in - 1;
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[k][j] = (x + ((size_t)kk << a.log_n) + step(0, j))[in0];
+        }
+        if constexpr (MDR) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) tw[j] = (x - n + step(0, j))[in0];
+        }
+#pragma unroll
+        for (int k = 0; k < NIN; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) conv.take(k, j, w[k][j]);
+        if constexpr (MDR) conv.dropped(a, b, d, tw);
+    }
+    for (uint32_t r = r_begin; r < r_end; r++) {
+        const uint32_t table = scalar(b.out_table)[d.map_off + r], limb = scalar(b.out_limb)[d.map_off + r];
+        uint64_t *dst = out + ((size_t)limb << a.log_n), *tile = lds[(r - r_begin) & 1];
+        auto row = [&](const auto &ar) {
+            using A = typename std::remove_cv<typename std::remove_reference<decltype(ar)>::type>::type;
+            typename A::V v[4];
+            typename A::Tw tw[NB];
+            T4::template load_tw<A, 0>(tw, ar, 1, t);
+            conv.convert(v, a, b, d, r, table, ar);
+            T4::template forward<A>(v, tw, ar, tile, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) (dst + step(NB - 1, j))[out0] = A::to_word(v[j]);
+        };
+        if constexpr (FP) {
+            row(fp_arith(a, table));
+        } else {
+            if ((a.fp_mask >> table) & 1)
+                row(fp_arith(a, table));
+            else
+                row(int_arith(a, table));
+        }
+    }
+}
+
+template <bool FP, int NIN, bool MDR>
+hipError_t launch_nin(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per,
+                      dim3 grid, hipStream_t s) {
+    switch (a.log_n - 8) {
+#define HE_CASE(LD)                                                                                                          \
+    case LD:                                                                                                                 \
+        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR>), grid, dim3(1 << (kTileLog - 2)), 0, s, a, b, compute_groups,   \
+                           copy_groups, rows_per);                                                                           \
+        break;
+        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+#undef HE_CASE
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+}  // namespace
+
+hipError_t launch_bconv_rows4(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per,
+                              int backend, hipStream_t s) {
+    const uint64_t wgs = (uint64_t)b.n_units * (b.items ? b.items : 1) * (1u << (a.log_n - kTileLog)) * (compute_groups + copy_groups);
+    if (a.log_n < 12 || a.log_n > 16 || b.max_in == 0 || b.max_in > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs);
+    NttArgs m = a;
+    if (!b.mat_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;
+#define HE_NIN(FP, MDR)                                                                              \
+    (b.max_in <= 4 ? launch_nin<FP, 4, MDR>(m, b, compute_groups, copy_groups, rows_per, grid, s)     \
+                   : launch_nin<FP, 8, MDR>(m, b, compute_groups, copy_groups, rows_per, grid, s))
+    if (b.mat_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
+    return b.mdr ? HE_NIN(false, true) : HE_NIN(false, false);
+#undef HE_NIN
+}
+
+}  // namespace he

@@ -10,7 +10,7 @@ namespace he {
 
 namespace {
 
-__device__ __forceinline__ uint32_t skew(uint32_t e) { return e + (e >> 4); }
+__host__ __device__ __forceinline__ constexpr uint32_t skew(uint32_t e) { return e + (e >> 4); }
 
 // read-only tables that every lane of a wave reads at one address: through the scalar cache
 typedef const double __attribute__((address_space(4))) *ScalarF64;
@@ -402,11 +402,16 @@ struct Tile4 {
         if constexpr (in_wave(KLO)) {
             swap_words<KLO>(w);
         } else {
+            // (bits low and low + 1 of a thread's first word are clear, and low >= 4: the words' slots lie a constant apart)
+            constexpr int FROM = BACK ? KLO + 1 : KLO, TO = BACK ? KLO : KLO + 1;
+            static_assert(B - 2 * KLO - 4 >= 4, "skew() adds to the words' distances");
+            uint64_t *from = lds + skew(word(FROM, t, 0));
+            const uint64_t *to = lds + skew(word(TO, t, 0));
 #pragma unroll
-            for (int j = 0; j < 4; j++) lds[skew(word(BACK ? KLO + 1 : KLO, t, j))] = w[j];
+            for (int j = 0; j < 4; j++) from[j * skew(1u << (B - 2 * FROM - 2))] = w[j];
             lds_barrier();
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = lds[skew(word(BACK ? KLO : KLO + 1, t, j))];
+            for (int j = 0; j < 4; j++) w[j] = to[j * skew(1u << (B - 2 * TO - 2))];
         }
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = A::from_word(w[j]);

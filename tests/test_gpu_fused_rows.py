@@ -1,5 +1,5 @@
-"""Base conversion fused with the rows pass of the forward transform (bconv_rows_fp_kernel, and bconv_rows_mx_kernel at
-N = 2^16: every prime below 2^50, N >= 2^12) against the oracle, through the C-ABI entry points that use it: he_modup (with the copy of a digit's own
+"""Base conversion fused with the rows pass of the forward transform (bconv_rows4_kernel, and bconv_rows_mx_kernel at
+N = 2^16 with every prime below 2^50) against the oracle, through the C-ABI entry points that use it: he_modup (with the copy of a digit's own
 limbs), he_moddown (1 to 6 polynomials, overwriting and adding), he_keyswitch, he_keyswitch_rescale (the merged
 ModDown + rescale prologue) and its batch form; every degree from 2^12 to 2^16, full and partial last digits, and
 the same calls with the fusion switched off by the environment."""

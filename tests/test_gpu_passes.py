@@ -145,3 +145,40 @@ def test_hoisting_of_one_ciphertext(oracle, capi, chain, logn, size_p, L, n_step
     capi.check(lib.he_hoisted_rotations_batch(h, L, 1, din.ptr, flat, d_elts, n_steps, 1, dout.ptr, ws.ptr, None))
     assert (dout.numpy() == np.stack([p.add(want[i], ct[i]) for i in range(2)])).all()
     assert (din.numpy() == ct).all()
+
+
+@pytest.mark.parametrize("logn,bits,size_p,levels", [
+    (12, [60, 40, 60, 40, 60, 40, 60, 60], 2, (6, 3)), (13, [60, 58, 60, 60, 55, 60, 60, 60, 60], 3, (6, 5)),
+    (14, [60, 45, 45, 45, 60, 60, 60, 60], 4, (4, 2)), (15, [60, 40, 40, 40, 40, 60, 60, 60, 60, 60], 5, (5, 4)),
+    (16, [60, 40, 60, 50, 60, 60], 2, (4, 3)), (16, [60] * 4 + [50] * 4 + [60] * 8, 8, (8,))])
+def test_conversion_fused_on_integers(oracle, capi, logn, bits, size_p, levels):
+    """ModUp, ModDown and the merged ModDown + rescale of levels with primes from 2^50 on, of up to 4 and up to 8 input limbs a
+    digit, with residues that make the largest sums, and of a batch."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    rng = np.random.default_rng(logn)
+    lib, h = capi.lib(), ctx.he_handle()
+    K, n, items = p.size_p, p.n, 3
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(p.size_q // K)]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    ptrs = capi.evk_array([d.ptr for d in dev])
+    for L in levels:
+        beta, tables = -(-L // K), [p.table_index(L, t) for t in range(L + K)]
+        dy, ws = DeviceArray(capi, shape=(beta, L + K, n)), DeviceArray(capi, shape=(2 * L, n))
+        coeff = np.stack([np.full(n, p.moduli[t] - 1, dtype=np.uint64) for t in range(L)])
+        for c in (rand_limbs(p, rng, range(L)), p.ntt_fwd(coeff, list(range(L)))):
+            dc = DeviceArray(capi, host=c)
+            capi.check(lib.he_modup(h, L, dc.ptr, dy.ptr, ws.ptr, None))
+            assert (dy.numpy() == p.modup(c)).all(), L
+        cx = np.stack([rand_limbs(p, rng, tables) for _ in range(2)])
+        dcx, dout, wsd = DeviceArray(capi, host=cx), DeviceArray(capi, shape=(2, L, n)), DeviceArray(capi, shape=(2, L, n))
+        capi.check(lib.he_moddown(h, L, dcx.ptr, dout.ptr, 2, 0, wsd.ptr, None))
+        assert (dout.numpy() == np.stack([p.moddown(x) for x in cx])).all(), L
+        c = rand_limbs(p, rng, range(L), n_polys=items)
+        ct = np.stack([rand_limbs(p, rng, range(L), n_polys=2) for _ in range(items)])
+        dc, dct, out = DeviceArray(capi, host=c), DeviceArray(capi, host=ct), DeviceArray(capi, shape=(items, 2, L - 1, n))
+        bws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+        capi.check(lib.he_keyswitch_rescale_batch(h, L, items, dc.ptr, L, ptrs, dct.ptr, out.ptr, 0, bws.ptr, None))
+        got = out.numpy()
+        for k in range(items):
+            ks = p.key_switch(c[k], host)
+            assert (got[k] == p.rescale(np.stack([p.add(ct[k][b], ks[b]) for b in range(2)]))).all(), (L, k)
