@@ -268,6 +268,17 @@ int he_keyswitch_rescale_batch(const he_context *ctx, uint32_t L, uint32_t items
 int he_pair_square_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32_t chunks,
                        const uint64_t *const *d_pairs, uint64_t *out01, uint64_t *out2, he_stream stream);
 
+/* out [items][size][L][N]: item k is the sum of the `count` ciphertexts ([size][L][N]) that row k of the DEVICE pointer table
+ * d_cts [items][count] names (add_inplace, src/evaluate.cu:118-165, once per term). */
+int he_sum_ciphertexts(const he_context *ctx, uint32_t L, uint32_t size, uint32_t items, uint32_t count,
+                       const uint64_t *const *d_cts, uint64_t *out, he_stream stream);
+
+/* out [items][3][L][N]: item k is the sum of the products (size-3 tensor products) of the `count` pairs of size-2 ciphertexts
+ * that row k of the DEVICE pointer table d_pairs [items][count][2] names: the multiply and add_inplace loop of the masked
+ * sum (byzantine_fl.py:371-429, lazy relinearisation) in one pass. */
+int he_multiply_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32_t count, const uint64_t *const *d_pairs,
+                    uint64_t *out, he_stream stream);
+
 /* out [2][L-1][N] = rescale(ct + KeySwitch(c)): he_keyswitch followed by he_rescale with the same limbs, in one
  * pass less over the data (ModDown and the rescale share one inverse and one forward transform: the NTT is linear).
  * ct [2][L][N] is only read.  workspace as for he_keyswitch.

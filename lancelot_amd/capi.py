@@ -66,6 +66,8 @@ SIGNATURES = {
     "he_hoisted_rotations_batch": (C.c_int, [vp, u32, u32, vp, C.POINTER(vp), C.POINTER(u32), u32, C.c_int, vp, vp, vp]),
     "he_keyswitch_rescale_batch": (C.c_int, [vp, u32, u32, vp, u32, C.POINTER(vp), vp, vp, u32, vp, vp]),
     "he_pair_square_sum": (C.c_int, [vp, u32, u32, u32, vp, vp, vp, vp]),
+    "he_sum_ciphertexts": (C.c_int, [vp, u32, u32, u32, u32, vp, vp, vp]),
+    "he_multiply_sum": (C.c_int, [vp, u32, u32, u32, vp, vp, vp]),
     "he_keyswitch_rescale": (C.c_int, [vp, u32, vp, C.POINTER(vp), vp, vp, u32, vp, vp]),
     "he_multiply_relin_rescale_workspace_words": (C.c_size_t, [vp, u32]),
     "he_multiply_relin_rescale": (C.c_int, [vp, u32, vp, vp, C.POINTER(vp), vp, vp, vp]),

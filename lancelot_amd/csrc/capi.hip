@@ -831,6 +831,24 @@ int he_pair_square_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32
     return HE_OK;
 }
 
+int he_sum_ciphertexts(const he_context *ctx, uint32_t L, uint32_t size, uint32_t items, uint32_t count,
+                       const uint64_t *const *d_cts, uint64_t *out, he_stream s) {
+    if (!ctx || !d_cts || !out || L == 0 || L > ctx->size_q || size == 0 || size > 16 || items == 0 || items > 4095 || count == 0)
+        return HE_E_INVALID_ARGUMENT;
+    if (ctx->log_n < 9) return HE_E_UNSUPPORTED;
+    HE_HIP(launch_sum(ctx->tables(), d_cts, out, L, size, items, count, S(s)));
+    return HE_OK;
+}
+
+int he_multiply_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32_t count, const uint64_t *const *d_pairs,
+                    uint64_t *out, he_stream s) {
+    if (!ctx || !d_pairs || !out || L == 0 || L > ctx->size_q || items == 0 || items > 16384 || count == 0)
+        return HE_E_INVALID_ARGUMENT;
+    if (ctx->log_n < 9) return HE_E_UNSUPPORTED;
+    HE_HIP(launch_multiply_sum(ctx->tables(), d_pairs, out, L, items, count, S(s)));
+    return HE_OK;
+}
+
 int he_galois_ntt(const he_context *ctx, const uint64_t *in, uint64_t *out, uint32_t total_limbs, uint32_t elt,
                   he_stream s) {
     if (!ctx || !in || !out || in == out || !(elt & 1) || elt >= (2u << ctx->log_n)) return HE_E_INVALID_ARGUMENT;

@@ -3,12 +3,116 @@
 // ciphertext per call; every item goes through the same arithmetic as the single-ciphertext functions, so its limbs
 // equal theirs.
 #include <cmath>
+#include <cstring>
 #include <stdexcept>
 
 #include "cahel.h"
+#include "staging.h"
 
 using cahel::check_status;
 using cahel::DeviceBuffer;
+
+// a table of device pointers, uploaded through page-locked memory without waiting
+static DeviceBuffer upload_table(const std::vector<const uint64_t *> &table, he_stream st) {
+    const std::size_t bytes = table.size() * sizeof(uint64_t);
+    DeviceBuffer d_table(table.size());
+    if (bytes > cahel::PinnedRing::kMaxBytes) {
+        check_status(he_memcpy_h2d(d_table.get(), table.data(), bytes, st), "upload");
+        return d_table;
+    }
+    cahel::PinnedRing &ring = cahel::PinnedRing::of_thread();
+    void *host = ring.take(bytes);
+    std::memcpy(host, table.data(), bytes);
+    const int status = he_memcpy_h2d_async(d_table.get(), host, bytes, st);
+    ring.fence(st);
+    check_status(status, "upload");
+    return d_table;
+}
+
+// ciphertext objects that are the consecutive slices of a batch (no copies), like `like` but for their size, limbs and scale
+static std::vector<CAHELGPUCiphertext> slices(DeviceBuffer batch, std::size_t items, std::size_t size, const CAHELGPUCiphertext &like,
+                                              double scale) {
+    std::vector<CAHELGPUCiphertext> out(items);
+    const std::size_t limbs = like.coeff_modulus_size(), n = like.poly_modulus_degree(), words = size * limbs * n;
+    auto shared = std::make_shared<DeviceBuffer>(std::move(batch));
+    for (std::size_t k = 0; k < items; k++) {
+        CAHELGPUCiphertext &ct = out[k];
+        ct.adopt(DeviceBuffer::slice(shared, k * words, words));
+        ct.size_ = size;
+        ct.coeff_modulus_size_ = limbs;
+        ct.poly_modulus_degree_ = n;
+        ct.chain_index_ = like.chain_index();
+        ct.parms_id_ = like.parms_id();
+        ct.scale_ = scale;
+        ct.is_ntt_form_ = true;
+        ct.is_asymmetric_ = like.is_asymmetric_;
+    }
+    return out;
+}
+
+// The sum of every row of ciphertexts (add_inplace term by term), all rows in one launch.
+std::vector<CAHELGPUCiphertext> sum_ciphertexts(const CAHELGPUContext &context,
+                                                const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows) {
+    if (rows.empty()) return {};
+    if (rows.size() > 4095) throw std::invalid_argument("too many sums");
+    if (rows[0].empty() || !rows[0][0]) throw std::invalid_argument("no ciphertexts");
+    const CAHELGPUCiphertext &first = *rows[0][0];
+    std::vector<const uint64_t *> table;
+    for (const auto &row : rows) {
+        if (row.size() != rows[0].size()) throw std::invalid_argument("rows differ in their number of ciphertexts");
+        for (const CAHELGPUCiphertext *ct : row) {
+            if (!ct || !ct->is_ntt_form()) throw std::invalid_argument("encrypted is not valid");
+            if (ct->parms_id() != first.parms_id() || ct->chain_index() != first.chain_index() || ct->size() != first.size())
+                throw std::invalid_argument("encrypted parameter mismatch");
+            if (ct->scale() != first.scale()) throw std::invalid_argument("scale mismatch");
+            table.push_back(ct->data());
+        }
+    }
+    he_stream st = context.stream();
+    const uint32_t size = (uint32_t)first.size(), L = (uint32_t)first.coeff_modulus_size(), items = (uint32_t)rows.size();
+    const DeviceBuffer d_table = upload_table(table, st);
+    DeviceBuffer out((std::size_t)items * size * L * context.poly_degree());
+    check_status(he_sum_ciphertexts(context.handle(), L, size, items, (uint32_t)rows[0].size(),
+                                    reinterpret_cast<const uint64_t *const *>(d_table.get()), out.get(), st),
+                 "he_sum_ciphertexts");
+    return slices(std::move(out), items, size, first, first.scale());
+}
+
+// For every row of ciphertexts the sum of its products with `factors` (multiply, add_inplace term by term; size 3, not
+// relinearised), all rows in one launch.
+std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
+                                             const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows,
+                                             const std::vector<const CAHELGPUCiphertext *> &factors) {
+    if (context.scheme() != cahel::scheme_type::ckks) throw std::logic_error("unsupported scheme");
+    if (rows.empty()) return {};
+    if (rows.size() > 16384) throw std::invalid_argument("too many sums");
+    if (rows[0].empty() || !rows[0][0] || factors.empty() || !factors[0]) throw std::invalid_argument("no ciphertexts");
+    const CAHELGPUCiphertext &first = *rows[0][0];
+    auto check = [&](const CAHELGPUCiphertext *ct, double scale) {
+        if (!ct || ct->size() != 2 || !ct->is_ntt_form()) throw std::invalid_argument("encrypted is not valid");
+        if (ct->parms_id() != first.parms_id() || ct->chain_index() != first.chain_index())
+            throw std::invalid_argument("encrypted parameter mismatch");
+        if (ct->scale() != scale) throw std::invalid_argument("scale mismatch");
+    };
+    for (const CAHELGPUCiphertext *f : factors) check(f, first.scale());
+    std::vector<const uint64_t *> table;
+    for (const auto &row : rows) {
+        if (row.size() != factors.size()) throw std::invalid_argument("rows differ in their number of ciphertexts");
+        for (std::size_t k = 0; k < row.size(); k++) {
+            check(row[k], first.scale());
+            table.push_back(row[k]->data());
+            table.push_back(factors[k]->data());
+        }
+    }
+    he_stream st = context.stream();
+    const uint32_t L = (uint32_t)first.coeff_modulus_size(), items = (uint32_t)rows.size();
+    const DeviceBuffer d_table = upload_table(table, st);
+    DeviceBuffer out((std::size_t)items * 3 * L * context.poly_degree());
+    check_status(he_multiply_sum(context.handle(), L, items, (uint32_t)factors.size(),
+                                 reinterpret_cast<const uint64_t *const *>(d_table.get()), out.get(), st),
+                 "he_multiply_sum");
+    return slices(std::move(out), items, 3, first, first.scale() * factors[0]->scale());
+}
 
 // For every (i, j) of `pairs`: acc = sum over chunks of (clients[j][c] - clients[i][c])^2, relinearised and rescaled,
 // then for every round acc += sum over the round's steps of rot(acc, step) (hoisted), as
@@ -57,8 +161,7 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
             table.push_back(clients[pr.second][c]->data());
             table.push_back(clients[pr.first][c]->data());
         }
-    DeviceBuffer d_table(table.size());
-    check_status(he_memcpy_h2d(d_table.get(), table.data(), table.size() * sizeof(uint64_t), st), "upload");
+    const DeviceBuffer d_table = upload_table(table, st);
     DeviceBuffer d01((std::size_t)items * 2 * L * n), d2((std::size_t)items * L * n);
     check_status(he_pair_square_sum(h, L, items, (uint32_t)chunks, reinterpret_cast<const uint64_t *const *>(d_table.get()),
                                     d01.get(), d2.get(), st),

@@ -337,6 +337,8 @@ PYBIND11_MODULE(pyCAHEL, m) {
     m.def("pair_square_distances", &pair_square_distances, py::arg("context"), py::arg("clients"), py::arg("pairs"),
           py::arg("relin_key"), py::arg("galois_key"), py::arg("rounds"), py::arg("scale") = 0.0, py::arg("drop_levels") = 0,
           nogil);
+    m.def("sum_ciphertexts", &sum_ciphertexts, py::arg("context"), py::arg("rows"), nogil);
+    m.def("multiply_sum", &multiply_sum, py::arg("context"), py::arg("rows"), py::arg("factors"), nogil);
     m.def("mod_switch_to", py::overload_cast<const CAHELGPUContext &, const CAHELGPUPlaintext &, CAHELGPUPlaintext &, std::size_t>(&mod_switch_to), nogil);
     m.def("mod_switch_to", py::overload_cast<const CAHELGPUContext &, const CAHELGPUCiphertext &, CAHELGPUCiphertext &, std::size_t>(&mod_switch_to), nogil);
     m.def("mod_switch_to_inplace", py::overload_cast<const CAHELGPUContext &, CAHELGPUPlaintext &, std::size_t>(&mod_switch_to_inplace), nogil);

@@ -484,6 +484,11 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
     const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
     const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
     const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels = 0);
+std::vector<CAHELGPUCiphertext> sum_ciphertexts(const CAHELGPUContext &context,
+                                                const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows);
+std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
+                                             const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows,
+                                             const std::vector<const CAHELGPUCiphertext *> &factors);
 void relinearize_rescale_inplace(const CAHELGPUContext &context, CAHELGPUCiphertext &encrypted,
                                  const CAHELGPURelinKey &relin_keys);
 void multiply_relin_rescale(const CAHELGPUContext &context, const CAHELGPUCiphertext &encrypted1,

@@ -23,6 +23,8 @@ namespace {
 
 constexpr int kThreads = 256;
 
+__device__ __forceinline__ Words2 load_pair(const uint64_t *p) { return *reinterpret_cast<const Words2 *>(p); }
+
 struct EwArgs {
     const uint64_t *a, *b, *c;
     uint64_t *out;
@@ -234,6 +236,69 @@ __global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(PairSquareArg
     out[idx] = d0;
     out[idx + poly] = d1;
     p.out2[(size_t)blockIdx.z * poly + idx] = d2;
+}
+
+// Sums of ciphertexts and of products of ciphertexts, each of `count` terms: what a row of a distance matrix or a masked sum of
+// updates is.  A call per term read and wrote the running sum each time (3 us of launch and latency a term at N = 2^16, two or
+// three limbs: 90 terms of ten row sums 290 us, 20 of two masked sums 110 us); here every term is read once, by all sums together.
+struct SumArgs {
+    const uint64_t *const *cts;   // device array [items][count], or [items][count][2] for products
+    uint64_t *out;
+    const uint64_t *moduli, *barrett;
+    uint32_t limbs, log_n, polys, count;
+};
+
+typedef const uint64_t *const __attribute__((address_space(4))) *ScalarPtr;
+__device__ __forceinline__ ScalarPtr scalar(const uint64_t *const *p) { return (ScalarPtr)(uintptr_t)p; }
+
+// grid: (N / 512, limbs, items * polys), two words per thread
+__global__ __launch_bounds__(kThreads) void sum_kernel(SumArgs p) {
+    const uint32_t limb = blockIdx.y, item = blockIdx.z / p.polys, poly = blockIdx.z - item * p.polys;
+    const size_t at = ((size_t)(poly * p.limbs + limb) << p.log_n) + 2 * (blockIdx.x * kThreads + threadIdx.x);
+    const uint64_t q = scalar(p.moduli)[limb];
+    const ScalarPtr ct = scalar(p.cts) + (size_t)item * p.count;
+    Words2 acc = load_pair(ct[0] + at);
+#pragma unroll 4
+    for (uint32_t k = 1; k < p.count; k++) {
+        const Words2 w = load_pair(ct[k] + at);
+        acc.x = add_mod(acc.x, w.x, q);
+        acc.y = add_mod(acc.y, w.y, q);
+    }
+    *reinterpret_cast<Words2 *>(p.out + (((size_t)item * p.polys * p.limbs) << p.log_n) + at) = acc;
+}
+
+// grid: (N / 512, limbs, items): (d0, d1, d2) = sum of (a0 b0, a0 b1 + a1 b0, a1 b1), residues below 2^61: the 128-bit sums
+// take 16 terms (32 products below 2^122 in d1) before they are reduced
+__global__ __launch_bounds__(kThreads) void multiply_sum_kernel(SumArgs p) {
+    const uint32_t limb = blockIdx.y;
+    const uint64_t q = scalar(p.moduli)[limb], r0 = scalar(p.barrett)[2 * limb], r1 = scalar(p.barrett)[2 * limb + 1];
+    const size_t poly = (size_t)p.limbs << p.log_n, at = ((size_t)limb << p.log_n) + 2 * (blockIdx.x * kThreads + threadIdx.x);
+    const ScalarPtr pair = scalar(p.cts) + (size_t)blockIdx.z * p.count * 2;
+    U128 s[3][2];
+#pragma unroll
+    for (int i = 0; i < 3; i++) s[i][0] = s[i][1] = U128{0, 0};
+    for (uint32_t k = 0; k < p.count; k++) {
+        const uint64_t *a = pair[2 * k] + at, *b = pair[2 * k + 1] + at;
+        const Words2 a0 = load_pair(a), a1 = load_pair(a + poly), b0 = load_pair(b), b1 = load_pair(b + poly);
+#pragma unroll
+        for (int j = 0; j < 2; j++) {
+            mac128(s[0][j], a0[j], b0[j]);
+            mac128(s[1][j], a0[j], b1[j]);
+            mac128(s[1][j], a1[j], b0[j]);
+            mac128(s[2][j], a1[j], b1[j]);
+        }
+        if (k % 16 == 15) {
+#pragma unroll
+            for (int i = 0; i < 3; i++)
+#pragma unroll
+                for (int j = 0; j < 2; j++) s[i][j] = U128{barrett128(s[i][j].lo, s[i][j].hi, q, r0, r1), 0};
+        }
+    }
+    uint64_t *out = p.out + (size_t)blockIdx.z * 3 * poly + at;
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        *reinterpret_cast<Words2 *>(out + i * poly) = Words2{barrett128(s[i][0].lo, s[i][0].hi, q, r0, r1),
+                                                             barrett128(s[i][1].lo, s[i][1].hi, q, r0, r1)};
 }
 
 // grid: (N / 256, total limbs)
@@ -768,7 +833,6 @@ struct HoistSumsInt {
     }
 };
 
-__device__ __forceinline__ Words2 load_pair(const uint64_t *p) { return *reinterpret_cast<const Words2 *>(p); }
 __device__ __forceinline__ Words2 stream_pair(const uint64_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const Words2 *>(p)); }
 
 // The two words that an automorphism brings to coefficients j and j + 1 (j even), src its gather index of j: odd elements
@@ -1167,6 +1231,20 @@ hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *const *pairs,
     if (items == 0 || items > 65535 || chunks == 0 || L == 0) return hipErrorInvalidValue;
     PairSquareArgs p{pairs, out01, out2, t.moduli, t.barrett, L, t.log_n, chunks};
     hipLaunchKernelGGL(pair_square_sum_kernel, dim3((1u << t.log_n) / kThreads, L, items), dim3(kThreads), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_sum(const Tables &t, const uint64_t *const *cts, uint64_t *out, uint32_t limbs, uint32_t polys, uint32_t items,
+                      uint32_t count, hipStream_t s) {
+    SumArgs p{cts, out, t.moduli, t.barrett, limbs, t.log_n, polys, count};
+    hipLaunchKernelGGL(sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), limbs, items * polys), dim3(kThreads), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_multiply_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out, uint32_t limbs, uint32_t items,
+                               uint32_t count, hipStream_t s) {
+    SumArgs p{pairs, out, t.moduli, t.barrett, limbs, t.log_n, 2, count};
+    hipLaunchKernelGGL(multiply_sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), limbs, items), dim3(kThreads), 0, s, p);
     return hipGetLastError();
 }
 

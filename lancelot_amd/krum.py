@@ -376,13 +376,22 @@ def decrypt_sort_mask(state: KrumState, enc):
         return total
 
     if state.config.batched:
-        totals = [row_sum(i) for i in range(n_clients)]
+        rows = [[ct for ct in row if ct is not None] for row in enc]
+        if len({len(row) for row in rows}) == 1 and rows[0]:
+            totals = c.sum_ciphertexts(ctx, rows)
+        else:
+            totals = [row_sum(i) for i in range(n_clients)]
         scores = list(state.sk.decrypt_decode_many(ctx, totals, state.slots, 1)[:, 0])
     else:
         scores = _map_lanes(state, list(range(n_clients)), lambda i: state.encoder.decode_array(
             ctx, state.sk.decrypt(ctx, row_sum(i)), 1)[0])
     order = np.argsort(np.asarray(scores), kind="stable")
-    zero, one = _encrypt_constant(state, 0.0), _encrypt_constant(state, 1.0)
+    if state.config.batched:
+        constants = np.zeros((2, state.slots))
+        constants[1] = 1.0
+        zero, one = state.encoder.encode_encrypt_many(ctx, state.pk, constants, state.config.scale)
+    else:
+        zero, one = _encrypt_constant(state, 0.0), _encrypt_constant(state, 1.0)
     mask = [[one if order[r] == k else zero for k in range(n_clients)] for r in range(n_clients)]
     _sync(c)
     state.timings["mask"] = state.timings.get("mask", 0.0) + time.perf_counter() - t0
@@ -396,6 +405,12 @@ def mul_mask_weight(state: KrumState, cts, mask_row):
     c, ctx = state.cahel, state.context
     t0 = time.perf_counter()
     n_chunks = len(cts[0])
+    if state.config.batched:
+        sums = c.multiply_sum(ctx, [[client[chunk] for client in cts[:len(mask_row)]] for chunk in range(n_chunks)], mask_row)
+        plain = [state.sk.decrypt(ctx, acc) for acc in sums]
+        out = [state.encoder.decode_array(ctx, p) for p in plain]
+        state.timings["mask_multiply"] = state.timings.get("mask_multiply", 0.0) + time.perf_counter() - t0
+        return np.concatenate(out)
     out = []
     prod = c.ciphertext(ctx)
     for chunk in range(n_chunks):

@@ -182,3 +182,35 @@ def test_conversion_fused_on_integers(oracle, capi, logn, bits, size_p, levels):
         for k in range(items):
             ks = p.key_switch(c[k], host)
             assert (got[k] == p.rescale(np.stack([p.add(ct[k][b], ks[b]) for b in range(2)]))).all(), (L, k)
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS) + ["largest"])
+@pytest.mark.parametrize("logn,L,items,count", [(9, 1, 1, 1), (10, 5, 3, 2), (13, 2, 2, 16), (12, 3, 1, 17), (16, 2, 2, 33)])
+def test_sums_of_ciphertexts_and_products(oracle, capi, chain, logn, L, items, count):
+    """he_sum_ciphertexts and he_multiply_sum around the 16 terms after which the products' sums are reduced, some of the words
+    the largest residues, some operands shared between the sums."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS.get(chain, [60] * 6), 1)
+    rng = np.random.default_rng(count)
+    lib, h = capi.lib(), ctx.he_handle()
+    n, kinds = p.n, min(3, count + 1)
+    top = np.array(p.moduli[:L], dtype=np.uint64)[:, None] - np.uint64(1)
+    cts = [rand_limbs(p, rng, range(L), n_polys=2) for _ in range(kinds)]
+    for ct in cts:
+        ct[:, :, :n // 2] = top
+    dev = [DeviceArray(capi, host=ct) for ct in cts]
+    pick = rng.integers(0, kinds, (items, count, 2))
+    table = DeviceArray(capi, host=np.array([[[dev[i].at(0) for i in pair] for pair in row] for row in pick], dtype=np.uint64))
+    first = DeviceArray(capi, host=np.array([[dev[pair[0]].at(0) for pair in row] for row in pick], dtype=np.uint64))
+    out, products = DeviceArray(capi, shape=(items, 2, L, n)), DeviceArray(capi, shape=(items, 3, L, n))
+    capi.check(lib.he_sum_ciphertexts(h, L, 2, items, count, first.ptr, out.ptr, None))
+    capi.check(lib.he_multiply_sum(h, L, items, count, table.ptr, products.ptr, None))
+    got, got3 = out.numpy(), products.numpy()
+    tensors = {(i, j): p.tensor(cts[i], cts[j]) for i, j in {tuple(x) for row in pick for x in row}}
+    for k in range(items):
+        want, want3 = cts[pick[k, 0, 0]], tensors[tuple(pick[k, 0])]
+        for i, j in pick[k, 1:]:
+            want = np.stack([p.add(want[r], cts[i][r]) for r in range(2)])
+            want3 = np.stack([p.add(want3[r], tensors[(i, j)][r]) for r in range(3)])
+        assert (got[k] == want).all() and (got3[k] == want3).all(), k
+    assert lib.he_sum_ciphertexts(h, L, 2, items, 0, first.ptr, out.ptr, None) == -1
+    assert lib.he_multiply_sum(h, 7, items, count, table.ptr, products.ptr, None) == -1
