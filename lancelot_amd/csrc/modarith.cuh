@@ -133,6 +133,54 @@ __device__ __forceinline__ U128 total3(const Lazy3 &h, const Lazy3 &s) {
     return U128{(uint64_t)t, (uint64_t)(t >> 64)};
 }
 
+// The same sum with three multiply-adds per product: a1 b0 + a0 b1 = a0 b0 + a1 b1 - (a1 - a0)(b1 - b0), the difference's product
+// summed with its sign.  Residues below 2^60: |a1 - a0| < 2^30, eight terms fit into 63 bits (and sixteen into ll and hh);
+// below 2^61: |a1 - a0| < 2^31, two terms.
+struct Split30d {
+    uint32_t lo, hi;
+    int32_t d;
+};
+
+__device__ __forceinline__ Split30d split30d(uint64_t a) {
+    const Split30 s = split30(a);
+    return Split30d{s.lo, s.hi, (int32_t)(s.hi - s.lo)};
+}
+
+struct Sum3 {
+    uint64_t ll, hh;
+    int64_t mm;
+};
+
+// one term for two sums that share the factor a (see mac3x2)
+__device__ __forceinline__ void mac_sum3x2(Sum3 &s, Sum3 &t, Split30d a, Split30d b, Split30d c) {
+    uint64_t carry;
+    asm("v_mad_u64_u32 %0, %6, %7, %10, %0\n\t"
+        "v_mad_u64_u32 %3, %6, %7, %13, %3\n\t"
+        "v_mad_u64_u32 %1, %6, %8, %11, %1\n\t"
+        "v_mad_u64_u32 %4, %6, %8, %14, %4\n\t"
+        "v_mad_i64_i32 %2, %6, %9, %12, %2\n\t"
+        "v_mad_i64_i32 %5, %6, %9, %15, %5"
+        : "+v"(s.ll), "+v"(s.hh), "+v"(s.mm), "+v"(t.ll), "+v"(t.hh), "+v"(t.mm), "=&s"(carry)
+        : "v"(a.lo), "v"(a.hi), "v"(a.d), "v"(b.lo), "v"(b.hi), "v"(b.d), "v"(c.lo), "v"(c.hi), "v"(c.d));
+}
+
+__device__ __forceinline__ void spill_sum3(Sum3 &h, Sum3 &s) {
+    h.ll += s.ll >> 32;
+    s.ll &= 0xffffffffu;
+    h.hh += s.hh >> 32;
+    s.hh &= 0xffffffffu;
+    h.mm += s.mm >> 32;
+    s.mm &= 0xffffffff;
+}
+
+__device__ __forceinline__ U128 total_sum3(const Sum3 &h, const Sum3 &s) {
+    typedef unsigned __int128 u128;
+    const u128 ll = (u128)s.ll + ((u128)h.ll << 32), hh = (u128)s.hh + ((u128)h.hh << 32);
+    const u128 mm = (u128)(__int128)s.mm + ((u128)(__int128)h.mm << 32);     // modulo 2^128; the difference below is not negative
+    const u128 t = ll + ((ll + hh - mm) << 30) + (hh << 60);
+    return U128{(uint64_t)t, (uint64_t)(t >> 64)};
+}
+
 // The butterflies' view of a modulus: q, 2q and their negatives modulo 2^64.  With the negatives at hand a Shoup
 // product is y w + hi (2^64 - q) and a conditional subtraction is x + (2^64 - 2q) followed by a select on the sign, i.e.
 // 64-bit additions (one instruction each) where subtractions would be borrow chains through VCC, which on this GPU need

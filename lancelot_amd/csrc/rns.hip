@@ -23,6 +23,14 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// word `at` of a limb whose address all lanes share: a scalar address and a 32-bit distance per lane (the empty statement keeps the
+// compiler from widening the distance outside a loop, which would cost a 64-bit addition per load)
+__device__ __forceinline__ const uint64_t *lane_word(const uint64_t *limb, uint32_t at) {
+    uint32_t bytes = at * 8u;
+    asm("" : "+v"(bytes));
+    return reinterpret_cast<const uint64_t *>(reinterpret_cast<const char *>(limb) + bytes);
+}
+
 __device__ __forceinline__ Words2 load_pair(const uint64_t *p) { return *reinterpret_cast<const Words2 *>(p); }
 
 struct EwArgs {
@@ -512,10 +520,17 @@ struct HoistArgs {
     int xcd_map;                    // workgroup order that keeps the sharers of a key block on one XCD
 };
 
+// The two words that an automorphism brings to coefficients j and j + 1 (j even), src its gather index of j: odd elements
+// keep aligned pairs of the NTT order together, so they are one 16-byte access, in their order or turned round.
+__device__ __forceinline__ void turned(uint64_t *v, Words2 w, uint32_t src) {
+    v[0] = src & 1 ? w.y : w.x;
+    v[1] = src & 1 ? w.x : w.y;
+}
+
 // Hoisted rotations in one launch: grid (N / 256, (L + K) + L [+ L], ceil(items / I)); a thread serves the same
 // coefficient of I consecutive items, so that a key word is loaded once for all of them.
 // rows t < L + K:  out[p][t] = sum_s sum_d sigma_s(y_d)[t] * evk_{s,d}[p][t]  (n_steps * beta <= 64 products, summed
-//                  lazily as partial products of factors split at bit 30, see Lazy3, and reduced once); the automorphism is the
+//                  lazily as partial products of factors split at bit 30, see Sum3, and reduced once); the automorphism is the
 //                  gather index of the load of y.  The kernel is bound by instruction issue (its multiply-adds).
 // rows L + K + t:  c0_out[t] = sum_s sigma_s(c0)[t]  (+ c0[t] with_self)
 // rows L + K + L + t (with_self only): c1 is copied to the output, so that the ModDown that follows adds onto
@@ -523,9 +538,11 @@ struct HoistArgs {
 // LOCAL: every step's Galois element is 1 modulo 2^(log_n - 7) (steps that are multiples of N / 512), so the
 // automorphism permutes inside each aligned block of 256 NTT-order words: a workgroup stages its block of every item
 // and digit in LDS once (I * beta <= kHoistLocalTiles) and gathers from there, instead of one global gather per step.
+// 45 ciphertexts of [60, 40 | 60] bits at N = 2^16, 15 steps: 331 -> 255 us block-local (three multiply-adds per
+// product instead of four, no register moves between terms, c0 from LDS, four waves per SIMD), 7 and 15 steps with gathers from memory 334 -> 320 us on average (four ciphertexts per thread there too).
 constexpr int kHoistLocalTiles = 16;
 template <int I, bool LOCAL>
-__global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void hoist_inner_kernel(HoistArgs p) {
     __shared__ uint64_t ybuf[LOCAL ? kHoistLocalTiles * kThreads : 1];
     const uint32_t LK = p.L + p.K;
     // Workgroup -> (block of 256 coefficients bx, row by, group of items bz).  The workgroups that share key words
@@ -567,70 +584,126 @@ __global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
                     p.c0_out[(item0 + it) * p.ct_item_stride + o] = p.c0[(item0 + it) * p.ct_item_stride + o];
             return;
         }
-        // the gathers of a step are independent of the running sums: one index per step for all items, and the
-        // loads of several steps in flight (a loop of one dependent load after the other ran longer than the rows
-        // that multiply)
         const uint32_t t = by - LK;
         const uint64_t q = p.moduli[t];
         const uint64_t *in = p.c0 + item0 * p.ct_item_stride + ((size_t)t << p.log_n);
-        uint64_t *c0_out = p.c0_out + item0 * p.ct_item_stride + o;
-        uint64_t acc[I];
+        uint64_t *c0_out = p.c0_out + item0 * p.ct_item_stride + ((size_t)t << p.log_n);
+        if constexpr (LOCAL) {
+            // every step permutes the block's words: they come from LDS, one index per step for all items
+            uint64_t acc[I];
 #pragma unroll
-        for (int it = 0; it < I; it++)
-            acc[it] = (uint32_t)it >= count ? 0 : p.accumulate ? c0_out[it * p.ct_item_stride] : p.with_self ? in[it * p.ct_item_stride + j] : 0;
+            for (int it = 0; it < I; it++) {
+                const uint64_t w = in[((uint32_t)it < count ? it : count - 1) * p.ct_item_stride + j];
+                ybuf[it * kThreads + threadIdx.x] = w;
+                acc[it] = p.accumulate ? c0_out[((uint32_t)it < count ? it : count - 1) * p.ct_item_stride + j] : p.with_self ? w : 0;
+            }
+            __syncthreads();
 #pragma unroll 4
-        for (uint32_t s = 0; s < p.n_steps; s++) {
-            const uint32_t g = galois_index(j, p.elts[s], p.log_n);
-            uint64_t w[I];
+            for (uint32_t s = 0; s < p.n_steps; s++) {
+                const uint32_t g = galois_index(j, p.elts[s], p.log_n) & (kThreads - 1);
 #pragma unroll
-            for (int it = 0; it < I; it++) w[it] = (uint32_t)it < count ? in[it * p.ct_item_stride + g] : 0;
+                for (int it = 0; it < I; it++) acc[it] = add_mod(acc[it], ybuf[it * kThreads + g], q);
+            }
 #pragma unroll
-            for (int it = 0; it < I; it++) acc[it] = add_mod(acc[it], w[it], q);
+            for (int it = 0; it < I; it++)
+                if ((uint32_t)it < count) c0_out[it * p.ct_item_stride + j] = acc[it];
+        } else {
+            // two neighbouring words per thread (see turned) of half the items; the gathers of a step are independent of the running
+            // sums, several steps' are in flight
+            constexpr int H = I / 2;
+            const uint32_t half = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / (kThreads / 2)) * H;
+            const uint32_t j2 = bx * kThreads + 2 * (threadIdx.x % (kThreads / 2));
+            const uint64_t *src[H];
+            Words2 acc[H];
+#pragma unroll
+            for (int it = 0; it < H; it++) {
+                const size_t at = (half + it < count ? half + it : count - 1) * p.ct_item_stride;
+                src[it] = in + at;
+                acc[it] = p.accumulate ? load_pair(c0_out + at + j2) : p.with_self ? load_pair(in + at + j2) : Words2{0, 0};
+            }
+#pragma unroll 4
+            for (uint32_t s = 0; s < p.n_steps; s++) {
+                const uint32_t g = galois_index(j2, p.elts[s], p.log_n);
+#pragma unroll
+                for (int it = 0; it < H; it++) {
+                    uint64_t v[2];
+                    turned(v, load_pair(lane_word(src[it], g & ~1u)), g);
+                    acc[it].x = add_mod(acc[it].x, v[0], q);
+                    acc[it].y = add_mod(acc[it].y, v[1], q);
+                }
+            }
+#pragma unroll
+            for (int it = 0; it < H; it++)
+                if (half + it < count) *reinterpret_cast<Words2 *>(c0_out + (half + it) * p.ct_item_stride + j2) = acc[it];
         }
-#pragma unroll
-        for (int it = 0; it < I; it++)
-            if ((uint32_t)it < count) c0_out[it * p.ct_item_stride] = acc[it];
         return;
     }
     const uint32_t t = by;
     const size_t y_item = (size_t)p.beta * LK << p.log_n;
     const uint64_t *y = p.y + item0 * y_item + ((size_t)t << p.log_n);
     const uint32_t table = t < p.L ? t : p.size_q + (t - p.L);
-    const size_t key_off = ((size_t)table << p.log_n) + j;
+    const size_t key_row = (size_t)table << p.log_n;
     const size_t key_poly = (size_t)(p.size_q + p.K) << p.log_n;
     const size_t digit = (size_t)LK << p.log_n;
     // the digit that owns limb t: its "lifted" limb is the input's c1 itself
     const uint32_t own = (p.own_from_ct && t < p.L) ? t / p.K : 0xffffffffu;
     const uint64_t *c1 = p.c0 + item0 * p.ct_item_stride + ((size_t)(p.L + t) << p.log_n);
-    auto word = [&](uint32_t d, int it, uint32_t at) {
-        return d == own ? c1[it * p.ct_item_stride + at] : y[it * y_item + d * digit + at];
-    };
     const uint32_t n_terms = p.n_steps * p.beta;
     if (LOCAL) {
         for (uint32_t d = 0; d < p.beta; d++)
 #pragma unroll
-            for (int it = 0; it < I; it++)
-                ybuf[(it * p.beta + d) * kThreads + threadIdx.x] = (uint32_t)it < count ? word(d, it, j) : 0;
+            for (int it = 0; it < I; it++) {
+                const uint32_t i = (uint32_t)it < count ? it : count - 1;
+                ybuf[(d * I + it) * kThreads + threadIdx.x] = *lane_word(d == own ? c1 + i * p.ct_item_stride : y + i * y_item + d * digit, j);
+            }
         __syncthreads();
     }
-    // term e = step e / beta, digit e mod beta; the operands of term e + 1 are requested before term e is
-    // multiplied, so that a wave does not wait for memory once per term
-    // (the gather index belongs to the step: it is formed for a step's first digit and kept for the others; the last
-    // iteration's repeated request is for the term just served)
-    uint32_t src = 0;
-    auto fetch = [&](uint32_t e, uint64_t &k0, uint64_t &k1, uint64_t(&v)[I]) {
-        const uint32_t st = e / p.beta, d = e - st * p.beta;
-        if (d == 0 || e == 0) src = galois_index(j, p.elts[st], p.log_n);
-        const uint64_t *k = p.evk.p[e];
-        k0 = k[key_off];
-        k1 = k[key_off + key_poly];
-#pragma unroll
-        for (int it = 0; it < I; it++)
-            v[it] = LOCAL ? ybuf[(it * p.beta + d) * kThreads + (src & (kThreads - 1))]
-                          : ((uint32_t)it < count ? word(d, it, src) : 0);
+    // The operands of one term are requested while another is multiplied, in two sets by turns, so that a wave neither waits for
+    // memory once per term nor moves a set; the gather index belongs to the step.  Every request is made on every path, past the end
+    // for the last term again: behind a branch that may skip loads the compiler waits for all of them.  (A thread's items past
+    // the last one read that one again.)
+    struct Term {
+        uint64_t k0, k1, v[I];
     };
-    uint64_t k0, k1, v[I];
-    fetch(0, k0, k1, v);
+    uint32_t st = 0, d = 0, next = 0, src = galois_index(j, p.elts[0], p.log_n);
+    const uint64_t *yd = y;
+    auto fetch = [&](Term &x) {
+        const uint64_t *k = p.evk.p[next] + key_row;
+        x.k0 = *lane_word(k, j);
+        x.k1 = *lane_word(k + key_poly, j);
+        const bool mine = d == own;
+        const uint64_t *w = mine ? c1 : yd;
+        const size_t stride = mine ? p.ct_item_stride : y_item;
+#pragma unroll
+        for (int it = 0; it < I; it++) {
+            x.v[it] = LOCAL ? ybuf[(d * I + it) * kThreads + (src & (kThreads - 1))] : *lane_word(w, src);
+            w += (uint32_t)it + 1 < count ? stride : 0;
+        }
+        const bool more = next + 1 < n_terms, wrap = more && d + 1 == p.beta;
+        next += more ? 1 : 0;
+        d = wrap ? 0 : d + (more ? 1 : 0);
+        yd = wrap ? y : yd + (more ? digit : 0);
+        if (wrap) src = galois_index(j, p.elts[++st], p.log_n);
+    };
+    auto terms = [&](auto &&take) {
+        Term x, z;
+        fetch(x);
+        uint32_t e = 0;
+        if (n_terms > 1) {
+            do {
+                fetch(z);
+                asm volatile("" ::: "memory");       // (a compiler barrier: without it the loads, whose values are first used in the
+                __builtin_amdgcn_sched_barrier(0);   //  next half, sink to the end of this one and every term waits for its operands)
+                take(e, x);
+                fetch(x);
+                asm volatile("" ::: "memory");
+                __builtin_amdgcn_sched_barrier(0);
+                take(e + 1, z);
+                e += 2;
+            } while (e + 1 < n_terms);
+        }
+        if (e < n_terms) take(e, x);
+    };
     const size_t o = ((size_t)t << p.log_n) + j;
     const size_t opoly = (size_t)LK << p.log_n;
     if (table < 64 && ((p.fp_mask >> table) & 1)) {
@@ -645,7 +718,7 @@ __global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
         const uint32_t tbits = 32 - __builtin_clz(n_terms);                        // n_terms < 2^tbits
         const bool one_go = 2 * qbits + tbits <= 100;
         const uint32_t B = !one_go ? 103 : 2 * qbits + tbits < 60 ? 60 : 2 * qbits + tbits;   // (any B up to 100 serves small primes)
-        const uint32_t period = one_go ? n_terms : 8;
+        const uint32_t fold_mask = one_go ? 0xffffffffu : 7u;
         const double base = __hiloint2double((int)((1023 + B) << 20), 0);
         const double down = __hiloint2double((int)((1023 + 52 - B) << 20), 0);     // 2^-(B-52)
         const double cB = fp_reduce(__hiloint2double((int)((1023 + B - 52) << 20), 0), m);
@@ -667,32 +740,20 @@ __global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
                 lo0[it] = lo1[it] = 0.0;
             }
         };
-        uint32_t pending = 0;
-        for (uint32_t e = 0; e < n_terms; e++) {
-            uint64_t nk0, nk1, nv[I];
-            fetch(e + 1 < n_terms ? e + 1 : e, nk0, nk1, nv);
-            asm volatile("" ::: "memory");       // (a compiler barrier: without it the loads, whose values are first used in the
-            __builtin_amdgcn_sched_barrier(0);   //  next iteration, sink to the end of this one and every term waits for its operands)
-            const double w0 = fp_from_u64(k0), w1 = fp_from_u64(k1);
+        terms([&](uint32_t e, const Term &x) {
+            const double w0 = fp_from_u64(x.k0), w1 = fp_from_u64(x.k1);
 #pragma unroll
             for (int it = 0; it < I; it++) {
-                const double x = fp_from_u64(v[it]);
-                const double t0 = __builtin_fma(x, w0, hi0[it]), t1 = __builtin_fma(x, w1, hi1[it]);
-                lo0[it] += __builtin_fma(x, w0, -(t0 - hi0[it]));
-                lo1[it] += __builtin_fma(x, w1, -(t1 - hi1[it]));
+                const double v = fp_from_u64(x.v[it]);
+                const double t0 = __builtin_fma(v, w0, hi0[it]), t1 = __builtin_fma(v, w1, hi1[it]);
+                lo0[it] += __builtin_fma(v, w0, -(t0 - hi0[it]));
+                lo1[it] += __builtin_fma(v, w1, -(t1 - hi1[it]));
                 hi0[it] = t0;
                 hi1[it] = t1;
             }
-            if (++pending == period) {
-                fold();
-                pending = 0;
-            }
-            k0 = nk0;
-            k1 = nk1;
-#pragma unroll
-            for (int it = 0; it < I; it++) v[it] = nv[it];
-        }
-        if (pending) fold();
+            if ((e & fold_mask) == fold_mask) fold();
+        });
+        fold();   // (what the last full eight terms left, possibly nothing)
 #pragma unroll
         for (int it = 0; it < I; it++) {
             if ((uint32_t)it >= count) break;
@@ -707,39 +768,29 @@ __global__ __launch_bounds__(kThreads) void hoist_inner_kernel(HoistArgs p) {
         }
         return;
     }
-    Lazy3 s0[I], s1[I], h0[I], h1[I];
-    // the words are relieved every 8 terms for a prime below 2^60, every 4 otherwise (see Lazy3)
-    const uint32_t spill_mask = (p.moduli[table] >> 60) ? 3u : 7u;
+    Sum3 s0[I], s1[I], h0[I], h1[I];
+    // the words are relieved every 8 terms for a prime below 2^60, every 2 otherwise (see Sum3)
+    const uint32_t spill_mask = (p.moduli[table] >> 60) ? 1u : 7u;
 #pragma unroll
-    for (int it = 0; it < I; it++) s0[it] = s1[it] = h0[it] = h1[it] = Lazy3{0, 0, 0};
-    for (uint32_t e = 0; e < n_terms; e++) {
-        uint64_t nk0, nk1, nv[I];
-        fetch(e + 1 < n_terms ? e + 1 : e, nk0, nk1, nv);
-        asm volatile("" ::: "memory");       // (a compiler barrier: without it the loads, whose values are first used in the
-            __builtin_amdgcn_sched_barrier(0);   //  next iteration, sink to the end of this one and every term waits for its operands)
-        const Split30 ks0 = split30(k0), ks1 = split30(k1);
+    for (int it = 0; it < I; it++) s0[it] = s1[it] = h0[it] = h1[it] = Sum3{0, 0, 0};
+    terms([&](uint32_t e, const Term &x) {
+        const Split30d ks0 = split30d(x.k0), ks1 = split30d(x.k1);
 #pragma unroll
-        for (int it = 0; it < I; it++) {
-            mac3x2(s0[it], s1[it], split30(v[it]), ks0, ks1);
-        }
+        for (int it = 0; it < I; it++) mac_sum3x2(s0[it], s1[it], split30d(x.v[it]), ks0, ks1);
         if ((e & spill_mask) == spill_mask) {
 #pragma unroll
             for (int it = 0; it < I; it++) {
-                spill3(h0[it], s0[it]);
-                spill3(h1[it], s1[it]);
+                spill_sum3(h0[it], s0[it]);
+                spill_sum3(h1[it], s1[it]);
             }
         }
-        k0 = nk0;
-        k1 = nk1;
-#pragma unroll
-        for (int it = 0; it < I; it++) v[it] = nv[it];
-    }
+    });
     const uint64_t q = p.moduli[table], r0 = p.barrett[2 * table], r1 = p.barrett[2 * table + 1];
 #pragma unroll
     for (int it = 0; it < I; it++) {
         if ((uint32_t)it >= count) break;
         uint64_t *out = p.out + (item0 + it) * ((size_t)2 * LK << p.log_n);
-        const U128 a0 = total3(h0[it], s0[it]), a1 = total3(h1[it], s1[it]);
+        const U128 a0 = total_sum3(h0[it], s0[it]), a1 = total_sum3(h1[it], s1[it]);
         uint64_t o0 = barrett128(a0.lo, a0.hi, q, r0, r1);
         uint64_t o1 = barrett128(a1.lo, a1.hi, q, r0, r1);
         if (p.accumulate) {
@@ -834,13 +885,6 @@ struct HoistSumsInt {
 };
 
 __device__ __forceinline__ Words2 stream_pair(const uint64_t *p) { return __builtin_nontemporal_load(reinterpret_cast<const Words2 *>(p)); }
-
-// The two words that an automorphism brings to coefficients j and j + 1 (j even), src its gather index of j: odd elements
-// keep aligned pairs of the NTT order together, so they are one 16-byte access, in their order or turned round.
-__device__ __forceinline__ void turned(uint64_t *v, Words2 w, uint32_t src) {
-    v[0] = src & 1 ? w.y : w.x;
-    v[1] = src & 1 ? w.x : w.y;
-}
 
 // Terms [first, last) of limb t for the coefficients j, j + 1 of every lane; two terms are multiplied while the next two are
 // on their way.
@@ -1470,9 +1514,7 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
     else launch(hoist_inner_kernel<I, false>, I)
     // (more items per thread read the keys less often but need more registers: 5, 6 and 8 items at 3, 2 and 2 waves per
     // SIMD measured 6 %, 5 to 20 % and 20 % slower than 4 items at 4 waves)
-    // With the keys shared through L2, gathers from memory are served better by twice the waves (2 items per thread:
-    // 452 against 498 us for 15 steps of 45 items at N = 2^16); the block-local form keeps 4 (389 against 500 us).
-    if (items >= 4 && (local || !p_xcd_ok)) {
+    if (items >= 4) {
         HE_HOIST(4);
     } else {
         HE_HOIST(2);

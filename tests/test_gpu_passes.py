@@ -214,3 +214,40 @@ def test_sums_of_ciphertexts_and_products(oracle, capi, chain, logn, L, items, c
         assert (got[k] == want).all() and (got3[k] == want3).all(), k
     assert lib.he_sum_ciphertexts(h, L, 2, items, 0, first.ptr, out.ptr, None) == -1
     assert lib.he_multiply_sum(h, 7, items, count, table.ptr, products.ptr, None) == -1
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("local", [False, True])
+@pytest.mark.parametrize("logn,size_p,L,n_steps,items", [(9, 1, 1, 1, 2), (10, 1, 3, 3, 3), (12, 2, 4, 4, 4), (11, 1, 4, 16, 5), (13, 1, 1, 17, 6),
+                                                         (16, 1, 2, 15, 5)])
+def test_hoisting_of_batches(oracle, capi, chain, local, logn, size_p, L, n_steps, items):
+    """he_hoisted_rotations_batch with odd and even counts of terms around the 8 after which the integer sums are relieved (up to
+    64 of them), with groups of two and of four ciphertexts and a rest, with keys that make the largest partial products and
+    differences (halves all ones or zero), steps inside aligned blocks and across them."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], size_p)
+    rng = np.random.default_rng(n_steps)
+    lib, h = capi.lib(), ctx.he_handle()
+    beta = -(-L // size_p)
+    host = [[rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(beta)] for _ in range(2)]
+    for key in host[0]:
+        for t in range(p.size_qp):
+            q, low = p.moduli[t], (1 << 30) - 1
+            key[:, t, :4] = [q - 1, low, (q - 1) & ~low, 0]
+            key[0, t, 4:p.n // 2] = min(low, q - 1)
+            key[1, t, 4:p.n // 2] = (q - 1) & ~low
+    dev = [[DeviceArray(capi, host=d) for d in key] for key in host]
+    unit = max(1, p.n // 512) if local else 1
+    elts = [pow(5, unit * (k + 1), 2 * p.n) for k in range(n_steps)]
+    flat = capi.evk_array([dev[i % 2][d].ptr for i in range(n_steps) for d in range(beta)])
+    d_elts = (C.c_uint32 * n_steps)(*elts)
+    wsb = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+    cts = np.stack([rand_limbs(p, rng, range(L), n_polys=2) for _ in range(items)])
+    din, dout = DeviceArray(capi, host=cts), DeviceArray(capi, shape=(items, 2, L, p.n))
+    want = [p.hoisting(ct, elts, [host[i % 2] for i in range(n_steps)]) for ct in cts]
+    for add_input in (0, 1):
+        capi.check(lib.he_hoisted_rotations_batch(h, L, items, din.ptr, flat, d_elts, n_steps, add_input, dout.ptr, wsb.ptr, None))
+        got = dout.numpy()
+        for k in range(items):
+            w = np.stack([p.add(want[k][b], cts[k][b]) for b in range(2)]) if add_input else want[k]
+            assert (got[k] == w).all(), (add_input, k)
+    assert (din.numpy() == cts).all()
