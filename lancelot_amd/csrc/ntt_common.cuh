@@ -217,12 +217,6 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
     }
 }
 
-// Orders the LDS accesses of one wave's lanes: the hardware runs them in program order, so only the compiler is held.
-__device__ __forceinline__ void wave_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-}
-
 // a of the lanes whose bit BIT is set and b of the lanes where it is not change places: the words' register bit becomes that
 // bit of the lane
 template <int BIT>
@@ -416,6 +410,7 @@ struct Tile4 {
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = A::from_word(w[j]);
     }
+    // (lds: only for exchanges across waves)
     template <class A, int K = 0>
     static __device__ __forceinline__ void forward(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
         ar.template ct<stages(K)>(v, tw[K]);

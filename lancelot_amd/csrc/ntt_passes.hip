@@ -2,9 +2,9 @@
 //
 // What bounds a pass is how many waves a SIMD has to switch between while loads, twiddle look-ups and LDS exchanges are on
 // their way, so a thread holds little: 4 words, its twiddles (at most 12, requested together with the words) and no more, 52
-// to 110 registers, 4 to 8 waves per SIMD.  The stages run as register blocks of two; the exchanges between them go through
-// LDS, and all of a blocks pass's, and all but the first (two for 2048-word tiles) of a rows pass's, stay inside one wave and
-// need no barrier.  Passes with 16 words per thread (radix-16 blocks, half the LDS exchanges, at most 2 waves per SIMD on
+// to 110 registers, 4 to 8 waves per SIMD.  The stages run as register blocks of two; the exchanges between them, all of
+// a blocks pass's and all but the first (two for 2048-word tiles) of a rows pass's, stay inside one wave and move words between its
+// lanes in registers; the others go through LDS.  Passes with 16 words per thread (radix-16 blocks, half the LDS exchanges, at most 2 waves per SIMD on
 // FP64 and 3 on integers), which this layout replaced, measured against it: 2 x 24 limbs at N = 2^16 30.0 against 27.3 us
 // (50 bits) and 43.5 against 37.5 us (60 bits), 8 x 24 limbs of 60 bits 139 against 112 us, 12 x 24 of 50 bits the same
 // 112 us (5.3 TB/s: the two trips through memory), 2 limbs at N = 2^13 9.8 against 8.1 us (50 bits) and 13 against 8.5 us
@@ -193,7 +193,7 @@ __device__ __forceinline__ BlockUnit block_unit(const NttArgs &a, uint32_t u) {
 // wave.  The next limb's words are requested before the current one's butterflies.
 template <bool FWD, bool EPI, bool LOOP, class A>
 __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &unit, Job job, const A &ar, uint64_t q, uint32_t blk,
-                                              uint32_t lane, uint64_t *lds) {
+                                              uint32_t lane) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t off = (size_t)blk * 256;
@@ -231,7 +231,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
                 ar.reduce(v);
-                T4::template forward<A>(v, tw, ar, lds, lane);
+                T4::template forward<A>(v, tw, ar, nullptr, lane);
                 if (EPI) {
                     // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
                     const double wd = fp_from_u64(e.w.w);
@@ -258,13 +258,13 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(x[j]);
-                T4::template inverse<A>(v, tw, ar, lds, lane);
+                T4::template inverse<A>(v, tw, ar, nullptr, lane);
             }
         } else {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = x[j];
             if (FWD) {
-                T4::template forward<A>(v, tw, ar, lds, lane);
+                T4::template forward<A>(v, tw, ar, nullptr, lane);
 #pragma unroll
                 for (int j = 0; j < 4; j++) x[j] = reduce_4q(v[j], q);
                 if (EPI) {
@@ -284,7 +284,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 }
                 store4(EPI ? e.dst : job.out + off + 4 * lane, x);
             } else {
-                T4::template inverse<A>(v, tw, ar, lds, lane);
+                T4::template inverse<A>(v, tw, ar, nullptr, lane);
             }
         }
         if (!FWD) {
@@ -294,13 +294,11 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
         }
         if (!more) break;
         job = next;
-        wave_sync();   // (the next limb's exchanges reuse the LDS words that this one's lanes have read)
     }
 }
 
 template <bool FWD, bool EPI, bool LOOP, int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a) {
-    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
     touch_arguments<sizeof(NttArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -309,9 +307,9 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a)
     const uint32_t blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, unit.job(0));
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane, lds_all[w]);
+    if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), scalar(a.moduli)[job.table], blk, lane, lds_all[w]);
+        if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), scalar(a.moduli)[job.table], blk, lane);
     }
 }
 
@@ -365,7 +363,7 @@ struct IntSums {
 // and waves 0 and 1 finish one polynomial each.
 template <int SPLIT, class A>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &x, uint32_t t, uint32_t table, uint32_t blk,
-                                            uint32_t item, uint32_t lane, const A &ar, uint64_t *lds, uint32_t part,
+                                            uint32_t item, uint32_t lane, const A &ar, uint32_t part,
                                             uint64_t *sums_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
@@ -436,13 +434,12 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         // again instead: n = 2^15, 10 of 12 limbs 71.5 -> 69.8 us.  One wave a block loses by it: L = 24, K = 8 153 against 156 us)
         if (SPLIT > 1 || d < x.beta) fetch(nx, d < x.beta ? d : now);
         ar.reduce(v);
-        T4::template forward<A>(v, tw, ar, lds, lane);
+        T4::template forward<A>(v, tw, ar, nullptr, lane);
         if constexpr (!FP) {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = reduce_4q(v[j], ar.m.q);
         }
         sums.add(v, k, ar);
-        wave_sync();   // (the next digit's exchanges reuse the LDS words that this one's lanes have read)
     }
     if constexpr (SPLIT > 1) {
 #pragma unroll
@@ -537,10 +534,9 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         }
         uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)r * LK * n + (size_t)t * n;
         if (invert) {
-            T4::template inverse<A>(v, tw, iar, lds, lane);
+            T4::template inverse<A>(v, tw, iar, nullptr, lane);
 #pragma unroll
             for (int j = 0; j < 4; j++) o[off + T4::word(0, lane, j)] = A::to_word(v[j]);
-            wave_sync();
         } else {
             uint64_t res[4];
 #pragma unroll
@@ -561,7 +557,6 @@ constexpr int kInnerWaves = 4;
 
 template <int BE, int SPLIT>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
-    __shared__ uint64_t lds_all[kInnerWaves][256 + 16];
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
     touch_arguments<sizeof(NttArgs) + sizeof(KsFuseArgs) - (kMaxDigits - 8) * sizeof(uint64_t *)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = (x.L + x.K) << lr;
@@ -591,9 +586,9 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
     const uint32_t t = pair >> lr, blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
-    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, fp_arith(a, table), lds_all[w], part, sums);
+    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, fp_arith(a, table), part, sums);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, int_arith(a, table), lds_all[w], part, sums);
+        if (!fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, int_arith(a, table), part, sums);
     }
 }
 
@@ -630,7 +625,7 @@ __device__ __forceinline__ void tensor4(const IntArith &ar, const NttArgs &a, ui
 // than tensor kernel + inverse transform.
 template <class A>
 __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse &x, const Job &job, const A &ar, uint32_t blk,
-                                             uint32_t lane, uint64_t *lds) {
+                                             uint32_t lane) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + 4 * lane;
@@ -669,23 +664,22 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
     store4(x.d01 + ct, o0);
     store4(x.d01 + ct + poly, o1);
     store4(x.d2 + job.poly * poly + job.limb * n + at, o2);
-    T4::template inverse<A>(d2, tw, ar, lds, lane);
+    T4::template inverse<A>(d2, tw, ar, nullptr, lane);
 #pragma unroll
     for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(d2[j]);
 }
 
 template <int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(NttArgs a, TensorFuse x) {
-    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
     touch_arguments<sizeof(NttArgs) + sizeof(TensorFuse)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane, lds_all[w]);
+    if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) tensor_block(a, x, job, int_arith(a, job.table), blk, lane, lds_all[w]);
+        if (!fp) tensor_block(a, x, job, int_arith(a, job.table), blk, lane);
     }
 }
 
@@ -708,7 +702,7 @@ __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t
 template <class A>
 __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t LK, uint32_t size_qp, uint32_t t,
                                               uint32_t table, uint32_t blk, uint32_t item, uint32_t items, uint32_t w, uint32_t lane,
-                                              const A &ar, uint64_t *lds, uint64_t *u_lds) {
+                                              const A &ar, uint64_t *u_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
@@ -724,7 +718,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
     ar.reduce(v);
-    T4::template forward<A>(v, tw, ar, lds, lane);
+    T4::template forward<A>(v, tw, ar, nullptr, lane);
     if (w == 0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) u[j] = canonical_word(v[j], ar);
@@ -752,7 +746,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
             else
                 v[j] = o[j];
         }
-        T4::template inverse<A>(v, tw, iar, lds, lane);
+        T4::template inverse<A>(v, tw, iar, nullptr, lane);
 #pragma unroll
         for (int j = 0; j < 4; j++) poly[off + T4::word(0, lane, j)] = A::to_word(v[j]);
     } else {
@@ -763,7 +757,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
 template <int BE>
 __global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
                                                              uint32_t items) {
-    __shared__ uint64_t lds_all[3][256 + 16], u_lds[256];
+    __shared__ uint64_t u_lds[256];
     touch_arguments<sizeof(NttArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -771,16 +765,16 @@ __global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const ui
     const uint32_t item = it / LK, t = it - item * LK, table = t < L ? t : size_q + (t - L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     if (BE != NTT_BACKEND_INT && fp)
-        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, fp_arith(a, table), lds_all[w], u_lds);
+        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, fp_arith(a, table), u_lds);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, int_arith(a, table), lds_all[w], u_lds);
+        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, int_arith(a, table), u_lds);
     }
 }
 
 // Decryption: the flooding noise's block through the last 8 stages, plus c0 + c1 s [+ c2 s^2].
 template <class A>
 __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArgs &d, const Job &job, uint32_t blk, uint32_t lane,
-                                              const A &ar, uint64_t *lds) {
+                                              const A &ar) {
     using T4 = Tile4<8, 8>;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane, poly = (size_t)a.map.limbs * n;
     const uint64_t q = scalar(a.moduli)[job.table], r0 = scalar(a.barrett)[2 * job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
@@ -802,7 +796,7 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
     ar.reduce(v);
-    T4::template forward<A>(v, tw, ar, lds, lane);
+    T4::template forward<A>(v, tw, ar, nullptr, lane);
     uint64_t o[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
@@ -814,16 +808,15 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
 
 template <int BE>
 __global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArgs a, DecryptArgs d) {
-    __shared__ uint64_t lds_all[kBlockWaves][256 + 16];
     touch_arguments<sizeof(NttArgs) + sizeof(DecryptArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) decrypt_block(a, d, job, blk, lane, fp_arith(a, job.table), lds_all[w]);
+    if (BE != NTT_BACKEND_INT && fp) decrypt_block(a, d, job, blk, lane, fp_arith(a, job.table));
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) decrypt_block(a, d, job, blk, lane, int_arith(a, job.table), lds_all[w]);
+        if (!fp) decrypt_block(a, d, job, blk, lane, int_arith(a, job.table));
     }
 }
 
