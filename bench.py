@@ -48,19 +48,18 @@ sys.path.insert(0, ROOT)
 LOG_N, SIZE_Q, SIZE_P, BITS, SCALE = 16, 24, 8, 50, 2.0 ** 40
 HBM_PEAK_GBS = 8000.0
 BLOCKS = 5
-# From profiles/hmult_relin_rescale_n65536_l24_k8.md (rocprofv3 --pmc runs of `bench.py --only step` and
-# `--only batch`), per operation: L2-miss traffic in limbs of 8 N bytes (FETCH_SIZE scaled by 2, WRITE_SIZE by 1: the
+# From profiles/hmult_relin_rescale_n65536_l24_k8.md (rocprofv3 --pmc runs of he_multiply_relin_rescale_batch
+# with 1 and 8 items), per operation: L2-miss traffic in limbs of 8 N bytes (FETCH_SIZE scaled by 2, WRITE_SIZE by 1: the
 # factors a copy of known size gives) and SQ_INSTS_VALU summed over the kernels.  Constants of the profile, not
 # measured in this run.
-PROFILE = {"single": {"traffic_limbs": 1117.7, "valu_wave_instr": 30.88e6,
-                      "kernels": "tensor_intt_blocks_fp, ntt_rows (inverse), bconv_rows_mx (ModUp, conversion on the int8 "
-                                 "matrix cores), ntt_blocks_fp_inner, ntt_blocks_fp + ntt_rows (inverse), bconv_rows_fp, "
-                                 "ntt_blocks_fp with the rescale epilogue"},
-           "batch": {"traffic_limbs": 896.1, "valu_wave_instr": 27.3e6,
-                     "kernels": "per call of 8 operations: tensor_fp, ntt_blocks_fp + ntt_rows (inverse), bconv_rows_mx, "
-                                "ntt_blocks_fp_inner (items of a tile on one XCD, key tile shared through L2), "
-                                "ntt_blocks_fp + ntt_rows (inverse), bconv_rows_mx, ntt_blocks_fp with the rescale "
-                                "epilogue"}}
+PROFILE = {"single": {"traffic_limbs": 1111.3, "valu_wave_instr": 34.92e6,
+                      "kernels": "tensor_intt_blocks, ntt_rows (inverse), bconv_rows_mx (ModUp, conversion on the int8 "
+                                 "matrix cores), ntt_inner (special limbs leave through the inverse blocks pass), ntt_rows "
+                                 "(inverse), bconv_rows4, ntt_blocks with the rescale epilogue"},
+           "batch": {"traffic_limbs": 844.8, "valu_wave_instr": 30.57e6,
+                     "kernels": "per call of 8 operations: tensor_intt_blocks, ntt_rows (inverse), bconv_rows_mx, "
+                                "ntt_inner (items of a block on one XCD, key words shared through L2), ntt_rows "
+                                "(inverse), bconv_rows_mx, ntt_blocks with the rescale epilogue"}}
 
 
 def issue_rates(capi):

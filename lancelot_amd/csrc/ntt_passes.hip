@@ -26,7 +26,7 @@ namespace {
 // SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first; it leaves the
 // coefficients where the forward pass takes them from.
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
-template <int LD, bool FWD, int BE, bool SRC_INTT, int B>
+template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B>
 __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
     using T4 = Tile4<B, LD>;
     constexpr int LOGC = B - LD, NB = T4::kBlocks;
@@ -82,7 +82,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
                 const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
-            } else if (rows_input_fp(v, a, job, c, [&](int j) { return glob(0, j); })) {
+            } else if (rows_input_fp<MDR>(v, a, job, c, [&](int j) { return glob(0, j); })) {
                 ar.reduce(v);
             }
             T4::template forward<FpArith>(v, tw, ar, lds, t);
@@ -113,7 +113,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
             } else {
-                rows_input_int(v, a, job, q, [&](int j) { return glob(0, j); });
+                rows_input_int<MDR>(v, a, job, q, [&](int j) { return glob(0, j); });
             }
             T4::template forward<IntArith>(v, tw, ar, lds, t);
             // lazy values in [0, 4q) go to the blocks pass
@@ -823,13 +823,13 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArg
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
-template <bool FWD, int BE, bool SRC_INTT = false>
+template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false>
 hipError_t launch_rows(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
     const uint32_t ld = a.log_n - 8;
     const bool large = ((uint64_t)n_jobs << a.log_n) >= ((uint64_t)32 << 16);
     const uint32_t b = ld < 4 ? 8 : (large || ld > 8) ? 11 : 10;
     const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
-#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, B>), grid, block, 0, s, a)
+#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B>), grid, block, 0, s, a)
 #define HE_CASE(LD)         \
     case LD:                \
         if (large)          \
@@ -870,6 +870,10 @@ hipError_t launch_ntt_rows(const NttArgs &a, uint32_t n_jobs, bool forward, int 
         b.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
         return launch_rows<true, NTT_BACKEND_MIXED, true>(b, n_jobs, s);
     }
+    if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE)
+        return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED, false, true>(a, n_jobs, s)
+               : backend                    ? launch_rows<true, NTT_BACKEND_FP, false, true>(a, n_jobs, s)
+                                            : launch_rows<true, NTT_BACKEND_INT, false, true>(a, n_jobs, s);
     if (forward)
         return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED>(a, n_jobs, s)
                : backend                    ? launch_rows<true, NTT_BACKEND_FP>(a, n_jobs, s)
