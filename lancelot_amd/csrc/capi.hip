@@ -833,7 +833,7 @@ int he_pair_square_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32
 
 int he_sum_ciphertexts(const he_context *ctx, uint32_t L, uint32_t size, uint32_t items, uint32_t count,
                        const uint64_t *const *d_cts, uint64_t *out, he_stream s) {
-    if (!ctx || !d_cts || !out || L == 0 || L > ctx->size_q || size == 0 || size > 16 || items == 0 || items > 4095 || count == 0)
+    if (!ctx || !d_cts || !out || L == 0 || L > ctx->size_q || size == 0 || size > 16 || items == 0 || items > 16384 || count == 0)
         return HE_E_INVALID_ARGUMENT;
     if (ctx->log_n < 9) return HE_E_UNSUPPORTED;
     HE_HIP(launch_sum(ctx->tables(), d_cts, out, L, size, items, count, S(s)));

@@ -2,6 +2,7 @@
 // one of them neither fills the GPU nor amortises a kernel launch).  Not in the reference, which evaluates one
 // ciphertext per call; every item goes through the same arithmetic as the single-ciphertext functions, so its limbs
 // equal theirs.
+#include <algorithm>
 #include <cmath>
 #include <cstring>
 #include <stdexcept>
@@ -50,11 +51,12 @@ static std::vector<CAHELGPUCiphertext> slices(DeviceBuffer batch, std::size_t it
     return out;
 }
 
-// The sum of every row of ciphertexts (add_inplace term by term), all rows in one launch.
+constexpr std::size_t kRowsPerCall = 16384;   // what he_sum_ciphertexts and he_multiply_sum take at once
+
+// The sum of every row of ciphertexts (add_inplace term by term), all rows in one launch (up to kRowsPerCall).
 std::vector<CAHELGPUCiphertext> sum_ciphertexts(const CAHELGPUContext &context,
                                                 const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows) {
     if (rows.empty()) return {};
-    if (rows.size() > 4095) throw std::invalid_argument("too many sums");
     if (rows[0].empty() || !rows[0][0]) throw std::invalid_argument("no ciphertexts");
     const CAHELGPUCiphertext &first = *rows[0][0];
     std::vector<const uint64_t *> table;
@@ -69,23 +71,24 @@ std::vector<CAHELGPUCiphertext> sum_ciphertexts(const CAHELGPUContext &context,
         }
     }
     he_stream st = context.stream();
-    const uint32_t size = (uint32_t)first.size(), L = (uint32_t)first.coeff_modulus_size(), items = (uint32_t)rows.size();
+    const uint32_t size = (uint32_t)first.size(), L = (uint32_t)first.coeff_modulus_size(), count = (uint32_t)rows[0].size();
+    const std::size_t items = rows.size(), words = (std::size_t)size * L * context.poly_degree();
     const DeviceBuffer d_table = upload_table(table, st);
-    DeviceBuffer out((std::size_t)items * size * L * context.poly_degree());
-    check_status(he_sum_ciphertexts(context.handle(), L, size, items, (uint32_t)rows[0].size(),
-                                    reinterpret_cast<const uint64_t *const *>(d_table.get()), out.get(), st),
-                 "he_sum_ciphertexts");
+    DeviceBuffer out(items * words);
+    for (std::size_t k = 0; k < items; k += kRowsPerCall)
+        check_status(he_sum_ciphertexts(context.handle(), L, size, (uint32_t)std::min(kRowsPerCall, items - k), count,
+                                        reinterpret_cast<const uint64_t *const *>(d_table.get()) + k * count, out.get() + k * words, st),
+                     "he_sum_ciphertexts");
     return slices(std::move(out), items, size, first, first.scale());
 }
 
 // For every row of ciphertexts the sum of its products with `factors` (multiply, add_inplace term by term; size 3, not
-// relinearised), all rows in one launch.
+// relinearised), all rows in one launch (up to kRowsPerCall).
 std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
                                              const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows,
                                              const std::vector<const CAHELGPUCiphertext *> &factors) {
     if (context.scheme() != cahel::scheme_type::ckks) throw std::logic_error("unsupported scheme");
     if (rows.empty()) return {};
-    if (rows.size() > 16384) throw std::invalid_argument("too many sums");
     if (rows[0].empty() || !rows[0][0] || factors.empty() || !factors[0]) throw std::invalid_argument("no ciphertexts");
     const CAHELGPUCiphertext &first = *rows[0][0];
     auto check = [&](const CAHELGPUCiphertext *ct, double scale) {
@@ -105,12 +108,14 @@ std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
         }
     }
     he_stream st = context.stream();
-    const uint32_t L = (uint32_t)first.coeff_modulus_size(), items = (uint32_t)rows.size();
+    const uint32_t L = (uint32_t)first.coeff_modulus_size(), count = (uint32_t)factors.size();
+    const std::size_t items = rows.size(), words = 3 * (std::size_t)L * context.poly_degree();
     const DeviceBuffer d_table = upload_table(table, st);
-    DeviceBuffer out((std::size_t)items * 3 * L * context.poly_degree());
-    check_status(he_multiply_sum(context.handle(), L, items, (uint32_t)factors.size(),
-                                 reinterpret_cast<const uint64_t *const *>(d_table.get()), out.get(), st),
-                 "he_multiply_sum");
+    DeviceBuffer out(items * words);
+    for (std::size_t k = 0; k < items; k += kRowsPerCall)
+        check_status(he_multiply_sum(context.handle(), L, (uint32_t)std::min(kRowsPerCall, items - k), count,
+                                     reinterpret_cast<const uint64_t *const *>(d_table.get()) + k * 2 * count, out.get() + k * words, st),
+                     "he_multiply_sum");
     return slices(std::move(out), items, 3, first, first.scale() * factors[0]->scale());
 }
 

@@ -199,7 +199,7 @@ hipError_t launch_tensor_mxn(const Tables &t, const uint64_t *ct1, uint32_t s1, 
 // (out01 [items][2][L][N], out2 [items][L][N]) = sum over chunks of (a - b)^2 for the pairs of ciphertexts in the
 // device pointer table pairs [items][chunks][2]
 // sums of `count` ciphertexts, and of `count` products of two size-2 ciphertexts: tables of device pointers in device memory,
-// N >= 512, items * polys <= 65535
+// N >= 512
 hipError_t launch_sum(const Tables &t, const uint64_t *const *cts, uint64_t *out, uint32_t limbs, uint32_t polys, uint32_t items,
                       uint32_t count, hipStream_t s);
 hipError_t launch_multiply_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out, uint32_t limbs, uint32_t items,

@@ -1308,9 +1308,15 @@ hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *const *pairs,
 
 hipError_t launch_sum(const Tables &t, const uint64_t *const *cts, uint64_t *out, uint32_t limbs, uint32_t polys, uint32_t items,
                       uint32_t count, hipStream_t s) {
-    SumArgs p{cts, out, t.moduli, t.barrett, limbs, t.log_n, polys, count};
-    hipLaunchKernelGGL(sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), limbs, items * polys), dim3(kThreads), 0, s, p);
-    return hipGetLastError();
+    // (one launch holds 65535 polynomials: more rows take several)
+    const uint32_t per_launch = 65535u / polys;
+    for (uint32_t first = 0; first < items; first += per_launch) {
+        const uint32_t rows = items - first < per_launch ? items - first : per_launch;
+        SumArgs p{cts + (size_t)first * count, out + ((size_t)first * polys * limbs << t.log_n), t.moduli, t.barrett, limbs, t.log_n, polys, count};
+        hipLaunchKernelGGL(sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), limbs, rows * polys), dim3(kThreads), 0, s, p);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_multiply_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out, uint32_t limbs, uint32_t items,
