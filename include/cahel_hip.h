@@ -371,7 +371,8 @@ int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const u
 
 /* plain [limbs][N] = c0 + c1 s (+ c2 s^2) + e for ct [size][limbs][N] of 2 or 3 polynomials, e the discrete Gaussian that
  * he_sample (kind 3) draws from the same stream: the noise's samples stay bytes, and the sums are formed by its transform's last
- * pass.  sk: s in NTT form, s^2 sk_stride words behind it.  cdt: DEVICE, at most 127 entries (HE_E_UNSUPPORTED beyond).
+ * pass.  limbs: those of a data level, or size_q + size_p (a ciphertext at the key level).  sk: s in NTT form, s^2 sk_stride words
+ * behind it.  cdt: DEVICE, at most 127 entries (HE_E_UNSUPPORTED beyond).
  * workspace: N / 8 words.  Replaces ckks_decrypt (src/secretkey.cu:594-654). */
 int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t size, uint32_t limbs, const uint64_t *sk, size_t sk_stride,
                      const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain,

@@ -1625,7 +1625,7 @@ int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const u
 int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t size, uint32_t limbs, const uint64_t *sk, size_t sk_stride,
                      const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain,
                      uint64_t *ws, he_stream s) {
-    if (!ctx || !ct || !sk || !key || !cdt || !plain || !ws || limbs == 0 || limbs > ctx->size_q || size < 2) return HE_E_INVALID_ARGUMENT;
+    if (!ctx || !ct || !sk || !key || !cdt || !plain || !ws || limbs == 0 || limbs > ctx->size_qp || size < 2) return HE_E_INVALID_ARGUMENT;
     if (size > 3 || cdt_len == 0 || cdt_len >= 128) return HE_E_UNSUPPORTED;
     return decrypt_flood_impl(ctx, DecryptArgs{ct, nullptr, sk, sk_stride, size}, limbs, 1, key, stream_id, cdt, cdt_len, plain, ws, s);
 }

@@ -1,4 +1,7 @@
-"""Calls at the ends of what the entry points take: more rows of sums than one launch or one call of the C-ABI holds."""
+"""Calls at the ends of what the entry points take: more rows of sums than one launch or one call of the C-ABI holds, decryption at
+the key level."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -61,3 +64,35 @@ def test_any_number_of_rows(oracle, rows):
     for k in sorted({0, 1, 4094, 4095, rows - 3, rows - 2, rows - 1}):
         assert (sums[k].to_numpy() == want_sum[which[k]]).all(), k
         assert (products[k].to_numpy() == want_mul[which[k]]).all(), k
+
+
+@pytest.mark.parametrize("logn,bits,size_p", [(9, [50, 49, 50], 1), (12, [60, 40, 40, 50, 60, 60], 2), (13, [60, 58, 60], 1)])
+def test_decryption_at_the_key_level(oracle, capi, logn, bits, size_p):
+    """A ciphertext over all primes, the special ones among them: encrypted and decrypted through pyCAHEL, and he_decrypt_flood of 2 and
+    3 polynomials."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    sk, pk = keys_for(cahel, parms, ctx)
+    enc = cahel.ckks_encoder(ctx)
+    plain = enc.encode_to(ctx, np.linspace(-1, 1, p.n // 2), 0, 2.0 ** 30)
+    ct = pk.encrypt_asymmetric(ctx, plain)
+    assert ct.chain_index() == 0 and ct.coeff_modulus_size() == p.size_qp
+    got = sk.decrypt(ctx, ct)
+    assert got.chain_index() == 0
+    # the difference of the decryption and the plaintext: encryption's and flooding's noise, the same small integers modulo every prime
+    diff = p.ntt_inv(np.ascontiguousarray(p.sub(got.to_numpy(), plain.to_numpy())))
+    signed = [np.where(d > np.uint64(q // 2), d.astype(np.int64) - q, d.astype(np.int64)) for d, q in zip(diff, p.moduli)]
+    assert all((s == signed[0]).all() for s in signed) and 0 < np.abs(signed[0]).max() < 2 ** 20
+    lib, h, rng = capi.lib(), ctx.he_handle(), np.random.default_rng(logn)
+    key, cdt = oracle.chacha_key(3), oracle.gauss_cdt()
+    kp = key.ctypes.data_as(C.POINTER(C.c_uint32))
+    for limbs in (p.size_q, p.size_qp):
+        ct3, s = (rand_limbs(p, rng, range(limbs), n_polys=k) for k in (3, 2))
+        dct, dsk, dcdt = DeviceArray(capi, host=ct3), DeviceArray(capi, host=s), DeviceArray(capi, host=cdt)
+        out, noise = DeviceArray(capi, shape=(limbs, p.n)), DeviceArray(capi, shape=(p.n // 8,))
+        e = p.ntt_fwd(p.sample_gauss(key, 5, limbs, cdt))
+        for size in (2, 3):
+            capi.check(lib.he_decrypt_flood(h, dct.ptr, size, limbs, dsk.ptr, limbs * p.n, kp, 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None))
+            want = p.mul_add(ct3[1], s[0], ct3[0])
+            want = p.mul_add(ct3[2], s[1], want) if size == 3 else want
+            assert (out.numpy() == p.add(want, e)).all(), (limbs, size)
+    assert lib.he_decrypt_flood(h, dct.ptr, 2, p.size_qp + 1, dsk.ptr, 0, kp, 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None) == -1
