@@ -90,6 +90,10 @@ enum : int {
     NTT_PRO_ROUND = 11,
 };
 
+// Workgroups that a launch may have: a grid of 2^32 threads and more is not refused by the runtime, which starts what is left of
+// the count modulo 2^32.
+inline constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads < 0x7fffffffu ? 0xffffffffu / threads : 0x7fffffffu; }
+
 struct NttArgs {
     const uint64_t *in;   // limb (poly, i) at in + (poly * in_poly_stride + i) * N
     uint64_t *out;
@@ -109,6 +113,7 @@ struct NttArgs {
     uint32_t items;           // list mode: the whole list is applied to `items` buffers (0 = 1) ...
     size_t item_stride;       // ... that lie item_stride words apart
     uint32_t batch, n_polys;  // filled in by the launcher
+    uint32_t first_job;       // ... where a rows pass of too many jobs for one launch goes on
     uint32_t log_n;
     LimbMap map;
     int pro_mode;

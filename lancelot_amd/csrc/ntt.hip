@@ -513,7 +513,7 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     BconvRowsK p{b, (rows + target - 1) / target, 0, target};
     p.copy_groups = b.copy_base ? (b.max_copy + target - 1) / target : 0;
     const uint64_t wgs = (uint64_t)b.n_units * items * tiles * (p.compute_groups + p.copy_groups);
-    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    if (wgs > most_workgroups(256)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs);
     if (mx) {
         if (b.mdr)

@@ -273,7 +273,8 @@ hipError_t launch_nin(const NttArgs &a, const BconvRows &b, uint32_t compute_gro
 hipError_t launch_bconv_rows4(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per,
                               int backend, hipStream_t s) {
     const uint64_t wgs = (uint64_t)b.n_units * (b.items ? b.items : 1) * (1u << (a.log_n - kTileLog)) * (compute_groups + copy_groups);
-    if (a.log_n < 12 || a.log_n > 16 || b.max_in == 0 || b.max_in > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    if (a.log_n < 12 || a.log_n > 16 || b.max_in == 0 || b.max_in > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
+        return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs);
     NttArgs m = a;
     if (!b.mat_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;

@@ -34,7 +34,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
     __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
     touch_arguments<sizeof(NttArgs)>();
     const uint32_t lb = logical_block();
-    const Job job = decode_job(a, lb / tiles_per_limb);
+    const Job job = decode_job(a, a.first_job + lb / tiles_per_limb);
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     auto glob = [&](int k, int j) {
@@ -756,13 +756,13 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
 
 template <int BE>
 __global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
-                                                             uint32_t items) {
+                                                             uint32_t items, uint32_t first_item) {
     __shared__ uint64_t u_lds[256];
     touch_arguments<sizeof(NttArgs)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = logical_block(), blk = id & ((1u << lr) - 1), it = id >> lr;
-    const uint32_t item = it / LK, t = it - item * LK, table = t < L ? t : size_q + (t - L);
+    const uint32_t of_launch = it / LK, item = first_item + of_launch, t = it - of_launch * LK, table = t < L ? t : size_q + (t - L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     if (BE != NTT_BACKEND_INT && fp)
         encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, fp_arith(a, table), u_lds);
@@ -824,10 +824,17 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArg
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
 template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false>
-hipError_t launch_rows(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
+hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
     const uint32_t ld = a.log_n - 8;
     const bool large = ((uint64_t)n_jobs << a.log_n) >= ((uint64_t)32 << 16);
     const uint32_t b = ld < 4 ? 8 : (large || ld > 8) ? 11 : 10;
+    // (from 2^34 words on, 137 GB, one launch does not hold the threads)
+    const uint32_t per_launch = most_workgroups(1u << (b - 2)) >> (a.log_n - b);
+    while (n_jobs > per_launch) {
+        if (hipError_t e = launch_rows<FWD, BE, SRC_INTT, MDR>(a, per_launch, s)) return e;
+        a.first_job += per_launch;
+        n_jobs -= per_launch;
+    }
     const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
 #define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B>), grid, block, 0, s, a)
 #define HE_CASE(LD)         \
@@ -900,7 +907,9 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     a.batch = (repeats + split - 1) / split;
     if (a.batch < 4 && !a.groups) a.batch = 1;
     a.n_polys = n_polys;
-    const dim3 grid(kinds * ((repeats + a.batch - 1) / a.batch) * (blocks / kBlockWaves)), block(64 * kBlockWaves);
+    const uint64_t wgs = (uint64_t)kinds * ((repeats + a.batch - 1) / a.batch) * (blocks / kBlockWaves);
+    if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
 #define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
     do {                                                                                                                \
         if (backend == NTT_BACKEND_MIXED)                                                                               \
@@ -940,7 +949,7 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
     // blocks) 64.4 / 64.3 / 64.5; from 3072 blocks on nothing is gained, at 8192 four waves lose 5 %.
     const int split = items > 1 || x.beta < 2 ? 1 : x.beta > 2 && pairs <= 512 ? 4 : pairs <= 2048 ? 2 : 1;
     const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs * split + kInnerWaves - 1) / kInnerWaves;
-    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    if (wgs > most_workgroups(64 * kInnerWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kInnerWaves);
 #define HE_INNER(SPLIT)                                                                                           \
     do {                                                                                                          \
@@ -964,7 +973,7 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
 hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s) {
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0 || items == 0) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
-    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
@@ -978,22 +987,26 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint
 hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
                                  int backend, hipStream_t s) {
     if (a.log_n < 9 || a.log_n > 17 || items == 0) return hipErrorInvalidValue;
-    const uint64_t wgs = (uint64_t)(L + K) * items << (a.log_n - 8);
-    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)wgs), block(192);
-    if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, pk, L, K, size_q, items);
-    else if (backend)
-        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, pk, L, K, size_q, items);
-    else
-        hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, pk, L, K, size_q, items);
-    return hipGetLastError();
+    const dim3 block(192);
+    const uint32_t wgs_per_item = (L + K) << (a.log_n - 8), per_launch = most_workgroups(block.x) / wgs_per_item;
+    if (per_launch == 0) return hipErrorInvalidValue;
+    for (uint32_t first = 0; first < items; first += per_launch) {
+        const dim3 grid((items - first < per_launch ? items - first : per_launch) * wgs_per_item);
+        if (backend == NTT_BACKEND_MIXED)
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+        else if (backend)
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+        else
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t launch_decrypt_blocks(const NttArgs &a, const DecryptArgs &d, uint32_t items, int backend, hipStream_t s) {
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || items == 0 || d.size < 2 || d.size > 3) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)a.map.limbs * items << (a.log_n - 8)) / kBlockWaves;
-    if (wgs > 0x7fffffffu) return hipErrorInvalidValue;
+    if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, d);

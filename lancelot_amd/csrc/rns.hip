@@ -1541,20 +1541,17 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
     auto launch = [&](auto kernel, uint32_t per) {
         p.groups = (items + per - 1) / per;
         p.xcd_map = p_xcd_ok && p.groups > 1 ? (local || no_contig || !stretch_local || nb < 128 || (nb >> 4) % 8 != 0 ? 1 : 2) : 0;
-        hipLaunchKernelGGL(kernel, dim3(nb * rows * p.groups), dim3(kThreads), 0, s, p);
+        const uint64_t wgs = (uint64_t)nb * rows * p.groups;
+        if (wgs > most_workgroups(kThreads)) return hipErrorInvalidValue;
+        hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(kThreads), 0, s, p);
+        return hipGetLastError();
     };
-#define HE_HOIST(I) \
-    if (local) launch(hoist_inner_kernel<I, true>, I); \
-    else launch(hoist_inner_kernel<I, false>, I)
+#define HE_HOIST(I) return local ? launch(hoist_inner_kernel<I, true>, I) : launch(hoist_inner_kernel<I, false>, I)
     // (more items per thread read the keys less often but need more registers: 5, 6 and 8 items at 3, 2 and 2 waves per
     // SIMD measured 6 %, 5 to 20 % and 20 % slower than 4 items at 4 waves)
-    if (items >= 4) {
-        HE_HOIST(4);
-    } else {
-        HE_HOIST(2);
-    }
+    if (items >= 4) HE_HOIST(4);
+    HE_HOIST(2);
 #undef HE_HOIST
-    return hipGetLastError();
 }
 
 hipError_t launch_sample(const Tables &t, int kind, ChaChaKey key, uint64_t stream_id, uint64_t *out, LimbMap map,

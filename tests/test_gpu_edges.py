@@ -1,5 +1,5 @@
 """Calls at the ends of what the entry points take: more rows of sums than one launch or one call of the C-ABI holds, decryption at
-the key level."""
+the key level, batches of more threads than a launch has."""
 import ctypes as C
 
 import numpy as np
@@ -96,3 +96,59 @@ def test_decryption_at_the_key_level(oracle, capi, logn, bits, size_p):
             want = p.mul_add(ct3[2], s[1], want) if size == 3 else want
             assert (out.numpy() == p.add(want, e)).all(), (limbs, size)
     assert lib.he_decrypt_flood(h, dct.ptr, 2, p.size_qp + 1, dsk.ptr, 0, kp, 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None) == -1
+
+
+def allocate(capi, words):
+    """words of device memory, zero; skips where the card has no room for them."""
+    ptr = C.c_void_p()
+    if capi.lib().he_malloc(C.byref(ptr), 8 * words) != 0:
+        pytest.skip("not enough free device memory")
+    capi.check(capi.lib().he_memset_zero(ptr.value, 8 * words, None))
+    return ptr.value
+
+
+@pytest.mark.parametrize("bits", [[50, 50], [60, 60], [60, 40, 60]])
+def test_transforms_of_more_words_than_a_launch_holds(oracle, capi, bits):
+    """2^34 words (137 GB) and some: a thread of the rows pass takes four, and a launch has fewer than 2^32 threads."""
+    cahel, parms, ctx, p = make_pair(oracle, 16, bits, 1)
+    lib, h, n, limbs = capi.lib(), ctx.he_handle(), p.n, len(bits) - 1
+    polys, rng = ((1 << 18) + 8) // limbs, np.random.default_rng(limbs)
+    data = allocate(capi, polys * limbs * n)
+    try:
+        last = 0xffffffff // 512 // 32 // limbs      # the first launch's last polynomial
+        xs = {k: rand_limbs(p, rng, range(limbs)) for k in (0, 8, last - 1, last, last + 1, polys - 1)}
+        at = lambda k: data + 8 * k * limbs * n
+        for k, x in xs.items():
+            capi.check(lib.he_memcpy_h2d(at(k), x.ctypes.data, x.nbytes, None))
+        for transform, want in ((lib.he_ntt_forward, {k: p.ntt_fwd(x.copy()) for k, x in xs.items()}), (lib.he_ntt_inverse, xs)):
+            capi.check(transform(h, data, polys, limbs, limbs, 0, limbs, 0, None))
+            got = np.empty((limbs, n), dtype=np.uint64)
+            for k in xs:
+                capi.check(lib.he_memcpy_d2h(got.ctypes.data, at(k), got.nbytes, None))
+                assert (got == want[k]).all(), k
+    finally:
+        lib.he_free(data)
+
+
+def test_encryptions_of_more_words_than_a_launch_holds(oracle, capi):
+    """he_encrypt_batch of 8192 items over 11 limbs of 2^16 words (193 GB): its passes have more than 2^32 threads."""
+    cahel, parms, ctx, p = make_pair(oracle, 16, [50] * 16, 8)
+    lib, h, n, L, items = capi.lib(), ctx.he_handle(), p.n, 3, 8192
+    pk = DeviceArray(capi, host=rand_limbs(p, np.random.default_rng(1), range(p.size_qp), n_polys=2))
+    kp = oracle.chacha_key(3).ctypes.data_as(C.POINTER(C.c_uint32))
+    cts = allocate(capi, items * 2 * L * n)
+    try:
+        ws = allocate(capi, lib.he_encrypt_batch_workspace_words(h, L, items))
+        try:
+            capi.check(lib.he_encrypt_batch(h, L, items, pk.ptr, kp, 7, cts, ws, None))
+            zero, one = DeviceArray(capi, host=np.zeros((L, n), dtype=np.uint64)), DeviceArray(capi, shape=(2, L, n))
+            got = np.empty((2, L, n), dtype=np.uint64)
+            first = 0xffffffff // 192 // (11 * 256)    # the items of the first launch
+            for k in (0, first // 2, first - 1, first, items - 1):
+                capi.check(lib.he_encrypt(h, L, zero.ptr, pk.ptr, kp, 7 + 3 * k, one.ptr, ws, None))
+                capi.check(lib.he_memcpy_d2h(got.ctypes.data, cts + 16 * k * L * n, got.nbytes, None))
+                assert (got == one.numpy()).all(), k
+        finally:
+            lib.he_free(ws)
+    finally:
+        lib.he_free(cts)
