@@ -285,7 +285,7 @@ PYBIND11_MODULE(pyCAHEL, m) {
         .def("scale", [](const CAHELGPUPlaintext &p) { return p.scale(); })
         .def("data_ptr", [](const CAHELGPUPlaintext &p) { return reinterpret_cast<std::uintptr_t>(p.data()); })
         .def("to_numpy", [](const CAHELGPUPlaintext &p) {
-            return to_host(p.data(), {(py::ssize_t)p.coeff_modulus_size(), (py::ssize_t)p.poly_modulus_degree()});
+            return to_host(p.lane_data(), {(py::ssize_t)p.coeff_modulus_size(), (py::ssize_t)p.poly_modulus_degree()});
         });
 
     py::class_<CAHELGPUCiphertext>(m, "ciphertext")

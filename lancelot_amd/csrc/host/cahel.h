@@ -98,6 +98,7 @@ public:
     // the shared owner of the block, or null for a plain buffer
     const std::shared_ptr<DeviceBuffer> &owner() const { return parent_; }
     uint64_t *get() const { return ptr_; }
+    int lane() const { return lane_; }
     std::size_t words() const { return words_; }
     static void trim_pool();  // return every cached block to the driver
 
@@ -112,7 +113,8 @@ private:
 // lanes 1 .. lane_count() are non-blocking streams.  Every evaluator, encoder and key function enqueues on the
 // current lane, and temporaries are recycled per lane, so independent ciphertext pipelines given different lanes
 // overlap on the GPU.  An object produced on one lane may be used on another only after synchronize_lanes(); it
-// may be dropped there (its storage returns to the producing lane after the dropping lane has drained).
+// may be dropped there (its storage returns to the producing lane after the dropping lane has drained).  An encoding, which
+// enqueues like the others, may be used on any lane at once: a plaintext waits for its encoding where another lane reads it.
 he_stream current_stream();
 int current_lane();
 int lane_count();
@@ -195,13 +197,36 @@ private:
     std::vector<uint64_t> psi_host_, ipsi_host_;
 };
 
+// An encoding that its lane may still be working on (the reference's encode ends in a blocking copy, so its plaintexts are always
+// there).
+struct EncodingInFlight {
+    explicit EncodingInFlight(int lane) : lane(lane) {}
+    const int lane;
+    std::atomic<bool> done{false};   // somebody has waited for it
+};
+
 // include/plaintext.h: CKKS plaintext = one polynomial over the limbs of its chain index, NTT form.
 class CAHELGPUPlaintext {
 public:
     CAHELGPUPlaintext() = default;
     explicit CAHELGPUPlaintext(const CAHELGPUContext &) {}
+    CAHELGPUPlaintext(const CAHELGPUPlaintext &o) { *this = o; }
+    CAHELGPUPlaintext &operator=(const CAHELGPUPlaintext &o);
+    CAHELGPUPlaintext(CAHELGPUPlaintext &&) noexcept = default;
+    CAHELGPUPlaintext &operator=(CAHELGPUPlaintext &&) noexcept = default;
     void resize(std::size_t coeff_modulus_size, std::size_t poly_modulus_degree);
-    uint64_t *data() const { return data_.get(); }
+    // the words, with no encoding left to run: for any stream, and for the host
+    uint64_t *data() const {
+        if (encoding_) await(true);
+        return data_.get();
+    }
+    // the words for work that is enqueued on the current lane
+    uint64_t *lane_data() const {
+        if (encoding_) await(false);
+        return data_.get();
+    }
+    // marks the words as those of an encoding that the current lane works on
+    void encoding_enqueued() { encoding_ = std::make_shared<EncodingInFlight>(cahel::current_lane()); }
     std::size_t &chain_index() { return chain_index_; }
     std::size_t chain_index() const { return chain_index_; }
     double &scale() { return scale_; }
@@ -220,6 +245,10 @@ public:
     double scale_ = 1.0;
     bool is_ntt_form_ = true;
     cahel::parms_id_type parms_id_ = cahel::parms_id_zero;
+
+private:
+    void await(bool on_every_lane) const;
+    std::shared_ptr<EncodingInFlight> encoding_;
 };
 
 // A relinearize_inplace that has not run yet: the ciphertext still holds the three polynomials of the product and

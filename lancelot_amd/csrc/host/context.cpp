@@ -244,6 +244,28 @@ std::vector<uint32_t> get_elts_from_steps(const std::vector<int> &steps, std::si
 // ---------------------------------------------------------------------------------------------------
 // containers
 // ---------------------------------------------------------------------------------------------------
+void CAHELGPUPlaintext::await(bool on_every_lane) const {
+    EncodingInFlight &e = *encoding_;
+    if (e.done.load(std::memory_order_acquire) || (!on_every_lane && e.lane == g_lane)) return;
+    check_status(he_stream_synchronize(g_lane_streams[e.lane]), "synchronisation failed");
+    e.done.store(true, std::memory_order_release);
+}
+
+CAHELGPUPlaintext &CAHELGPUPlaintext::operator=(const CAHELGPUPlaintext &o) {
+    if (this == &o) return *this;
+    (void)lane_data();   // (the block may be written again)
+    (void)o.lane_data();
+    data_ = o.data_;
+    encoding_.reset();
+    chain_index_ = o.chain_index_;
+    coeff_modulus_size_ = o.coeff_modulus_size_;
+    poly_modulus_degree_ = o.poly_modulus_degree_;
+    scale_ = o.scale_;
+    is_ntt_form_ = o.is_ntt_form_;
+    parms_id_ = o.parms_id_;
+    return *this;
+}
+
 void CAHELGPUPlaintext::resize(std::size_t coeff_modulus_size, std::size_t poly_modulus_degree) {
     const std::size_t words = coeff_modulus_size * poly_modulus_degree;
     if (words != data_.words()) data_.allocate(words);

@@ -154,6 +154,8 @@ void CAHELGPUCKKSEncoder::encode_complex(const CAHELGPUContext &context, const d
         throw std::invalid_argument("scale out of bounds");
     const std::size_t ss = message_slots(count);
     const uint32_t limbs = (uint32_t)context.limbs_at(chain_index);
+    // (a block of another lane goes back there: an encoding's block belongs to the lane that writes it)
+    if (destination.data_.get() && destination.data_.lane() != current_lane()) destination.data_.release();
     destination.resize(limbs, n);
     he_context *h = context.handle();
     he_stream st = context.stream();
@@ -165,11 +167,12 @@ void CAHELGPUCKKSEncoder::encode_complex(const CAHELGPUContext &context, const d
     if (im) sum += copy_sum(host_im, im, count);
     if (surely_small(sum, scale, ss, total_bits)) {
         const int status = he_ckks_encode_bounded(h, host_re, host_im, (uint32_t)count, (uint32_t)ss, scale, limbs, 1, count,
-                                                  destination.data(), limbs, ws.get(), st);
+                                                  destination.data_.get(), limbs, ws.get(), st);
         ring.fence(st);
+        destination.encoding_enqueued();
         check_status(status, "he_ckks_encode_bounded");
     } else {
-        const int status = he_ckks_encode(h, host_re, host_im, (uint32_t)count, (uint32_t)ss, scale, limbs, destination.data(),
+        const int status = he_ckks_encode(h, host_re, host_im, (uint32_t)count, (uint32_t)ss, scale, limbs, destination.data_.get(),
                                           ws.get(), st);
         ring.fence(st);
         check_status(status, "he_ckks_encode");
@@ -198,7 +201,7 @@ void CAHELGPUCKKSEncoder::decode_values(const CAHELGPUContext &context, const CA
     he_context *h = context.handle();
     DeviceBuffer ws(he_ckks_workspace_words(h, limbs));
     DeviceBuffer out(2 * ss);
-    check_status(he_ckks_decode(h, plain.data(), limbs, (uint32_t)ss, plain.scale(),
+    check_status(he_ckks_decode(h, plain.lane_data(), limbs, (uint32_t)ss, plain.scale(),
                                 reinterpret_cast<double *>(out.get()), ws.get(), context.stream()),
                  "he_ckks_decode");
     v.resize(2 * count);
@@ -220,7 +223,7 @@ void CAHELGPUCKKSEncoder::decode_complex(const CAHELGPUContext &context, const C
 
 std::size_t CAHELGPUCKKSEncoder::decode_count(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count) {
     if (!plain.is_ntt_form()) throw std::invalid_argument("plain is not in NTT form");
-    if (plain.coeff_modulus_size() == 0 || !plain.data()) throw std::invalid_argument("plain is empty");
+    if (plain.coeff_modulus_size() == 0 || !plain.data_.get()) throw std::invalid_argument("plain is empty");
     const int total_bits = context.total_coeff_modulus_bit_count(plain.chain_index());
     if (plain.scale() <= 0 || (static_cast<int>(std::log2(plain.scale())) >= total_bits))
         throw std::invalid_argument("scale out of bounds");
@@ -236,7 +239,7 @@ void CAHELGPUCKKSEncoder::decode_real(const CAHELGPUContext &context, const CAHE
     const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
     DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)sparse_slots_));
     double *host = static_cast<double *>(PinnedRing::of_thread().take(count * sizeof(double)));
-    check_status(he_ckks_decode_real(h, plain.data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
+    check_status(he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
                                      context.stream()),
                  "he_ckks_decode_real");
     check_status(he_stream_synchronize(context.stream()), "synchronisation failed");

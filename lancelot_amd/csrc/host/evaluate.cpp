@@ -100,7 +100,7 @@ static void check_plain(const CAHELGPUCiphertext &encrypted, const CAHELGPUPlain
 
 void add_plain_inplace(const CAHELGPUContext &context, CAHELGPUCiphertext &encrypted, const CAHELGPUPlaintext &plain) {
     check_plain(encrypted, plain, true);
-    check_status(he_add(context.handle(), encrypted.data(), plain.data(), encrypted.data(), 1,
+    check_status(he_add(context.handle(), encrypted.data(), plain.lane_data(), encrypted.data(), 1,
                         (uint32_t)encrypted.coeff_modulus_size(), 0, context.stream()),
                  "he_add");
 }
@@ -113,7 +113,7 @@ void add_plain(const CAHELGPUContext &context, CAHELGPUCiphertext &encrypted, co
 
 void sub_plain_inplace(const CAHELGPUContext &context, CAHELGPUCiphertext &encrypted, const CAHELGPUPlaintext &plain) {
     check_plain(encrypted, plain, true);
-    check_status(he_sub(context.handle(), encrypted.data(), plain.data(), encrypted.data(), 1,
+    check_status(he_sub(context.handle(), encrypted.data(), plain.lane_data(), encrypted.data(), 1,
                         (uint32_t)encrypted.coeff_modulus_size(), 0, context.stream()),
                  "he_sub");
 }
@@ -130,7 +130,7 @@ void multiply_plain_inplace(const CAHELGPUContext &context, CAHELGPUCiphertext &
     const uint32_t limbs = (uint32_t)encrypted.coeff_modulus_size();
     for (std::size_t i = 0; i < encrypted.size(); i++) {
         uint64_t *ci = encrypted.data() + i * limbs * n;
-        check_status(he_multiply(context.handle(), ci, plain.data(), ci, 1, limbs, 0, context.stream()), "he_multiply");
+        check_status(he_multiply(context.handle(), ci, plain.lane_data(), ci, 1, limbs, 0, context.stream()), "he_multiply");
     }
     encrypted.scale() *= plain.scale();
     if (!scale_within_bounds(context, encrypted.scale(), encrypted.chain_index()))
@@ -366,7 +366,7 @@ void mod_switch_to_next(const CAHELGPUContext &context, const CAHELGPUPlaintext 
     if (!scale_within_bounds(context, plain.scale(), next)) throw std::invalid_argument("scale out of bounds");
     // dropping the last limb of a single polynomial keeps the leading words in place
     DeviceBuffer fresh(next_limbs * n);
-    check_status(he_memcpy_d2d(fresh.get(), plain.data(), next_limbs * n * sizeof(uint64_t), context.stream()), "copy");
+    check_status(he_memcpy_d2d(fresh.get(), plain.lane_data(), next_limbs * n * sizeof(uint64_t), context.stream()), "copy");
     const double scale = plain.scale();
     destination.data_ = std::move(fresh);
     destination.coeff_modulus_size_ = next_limbs;

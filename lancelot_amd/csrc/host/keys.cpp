@@ -150,7 +150,7 @@ void CAHELGPUSecretKey::encrypt_symmetric(const CAHELGPUContext &context, const 
     if (!plain.is_ntt_form()) throw std::invalid_argument("CKKS plain must be in NTT form");
     encrypt_zero_symmetric(context, cipher, plain.chain_index());
     const uint32_t limbs = (uint32_t)context.limbs_at(plain.chain_index());
-    check_status(he_add(context.handle(), cipher.data(), plain.data(), cipher.data(), 1, limbs, 0, context.stream()), "he_add");
+    check_status(he_add(context.handle(), cipher.data(), plain.lane_data(), cipher.data(), 1, limbs, 0, context.stream()), "he_add");
     cipher.scale() = plain.scale();
 }
 
@@ -176,14 +176,14 @@ void CAHELGPUPublicKey::encrypt_asymmetric(const CAHELGPUContext &context, const
             check_status(he_multiply_add(h, u.get(), pk_.data() + (std::size_t)i * QP * n, ci, ci, 1, limbs, 0, 0, st),
                          "he_multiply_add");
         }
-        check_status(he_add(h, cipher.data(), plain.data(), cipher.data(), 1, limbs, 0, st), "he_add");
+        check_status(he_add(h, cipher.data(), plain.lane_data(), cipher.data(), 1, limbs, 0, st), "he_add");
     } else {
         // encrypt over Ql u P, then divide by P (ModDown) onto the L limbs of the plaintext's level: the batched
         // pipeline with one item (u, e0, e1 from the next three stream ids; the division adds onto the plaintext)
         const uint32_t L = (uint32_t)context.limbs_at(chain);
         cipher.resize(context, chain, 2);
         DeviceBuffer ws(he_encrypt_batch_workspace_words(h, L, 1));
-        check_status(he_encrypt(h, L, plain.data(), pk_.data(), context.prng_key(), context.next_stream(3), cipher.data(),
+        check_status(he_encrypt(h, L, plain.lane_data(), pk_.data(), context.prng_key(), context.next_stream(3), cipher.data(),
                                 ws.get(), st),
                      "he_encrypt");
     }
@@ -207,20 +207,20 @@ void CAHELGPUSecretKey::decrypt(const CAHELGPUContext &context, const CAHELGPUCi
     if (noise_flooding_ && needed <= 2) {
         DeviceBuffer noise(n / 8);
         check_status(he_decrypt_flood(h, cipher.data(), (uint32_t)cipher.size(), limbs, sk_powers_.get(), sk_poly, context.prng_key(),
-                                      context.next_stream(), context.gauss_cdt(), context.gauss_cdt_len(), plain.data(), noise.get(),
+                                      context.next_stream(), context.gauss_cdt(), context.gauss_cdt_len(), plain.lane_data(), noise.get(),
                                       st),
                      "he_decrypt_flood");
     } else {
         // c0 + c1 s (+ c2 s^2 ...): the first product reads c0 directly
         for (std::size_t i = 1; i <= needed; i++)
             check_status(he_multiply_add(h, cipher.data() + i * poly, sk_powers_.get() + (i - 1) * sk_poly,
-                                         i == 1 ? cipher.data() : plain.data(), plain.data(), 1, limbs, 0, 0, st),
+                                         i == 1 ? cipher.data() : plain.lane_data(), plain.lane_data(), 1, limbs, 0, 0, st),
                          "he_multiply_add");
         if (noise_flooding_) {
             DeviceBuffer noise(poly);
             sample(context, 3, noise.get(), limbs, limbs, 0);
             check_status(he_ntt_forward(h, noise.get(), 1, limbs, limbs, 0, limbs, 0, st), "he_ntt_forward");
-            check_status(he_add(h, plain.data(), noise.get(), plain.data(), 1, limbs, 0, st), "he_add");
+            check_status(he_add(h, plain.lane_data(), noise.get(), plain.lane_data(), 1, limbs, 0, st), "he_add");
         }
     }
     plain.chain_index() = cipher.chain_index();

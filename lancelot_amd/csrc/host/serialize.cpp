@@ -134,7 +134,7 @@ void CAHELGPUPlaintext::save(std::ostream &stream) const {
         put<uint64_t>(stream, chain_index_);
         put<uint64_t>(stream, poly_modulus_degree_);
         put<double>(stream, scale_);
-        put_device_words(stream, data(), coeff_modulus_size_ * poly_modulus_degree_);
+        put_device_words(stream, lane_data(), coeff_modulus_size_ * poly_modulus_degree_);
     });
 }
 

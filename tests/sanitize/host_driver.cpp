@@ -1,4 +1,5 @@
-// Runs the CPU-only parts of the host layer (number theory, BLAKE2b, table construction, record save / load) under
+// Runs the CPU-only parts of the host layer (number theory, BLAKE2b, table construction, record save / load, what waits for an
+// encoding) under
 // AddressSanitizer + UndefinedBehaviorSanitizer, against the host-memory mock of the device ABI (mock_device.cpp).
 // Ends with a bounded, seeded loop that feeds damaged and random records to every load() entry: a parser may refuse
 // a record (any std::exception), it may not crash or touch memory it does not own.  Exit code 0 = clean.
@@ -176,6 +177,67 @@ int main(int argc, char **argv) {
         three.pending_ = std::make_shared<PendingKeySwitch>();   // overwritten as a whole: nothing runs
         three.adopt(DeviceBuffer(2 * L2 * n));
         REQUIRE(!three.has_pending_key_switch());
+    }
+
+    // ---- encodings that nothing has waited for: used at once on other lanes, through data(), copied, written again ----
+    {
+        CAHELGPUCKKSEncoder encoder(context);
+        std::vector<double> values(n / 2), others(n / 2);
+        for (std::size_t i = 0; i < n / 2; i++) {
+            values[i] = 1.0 + 0.001 * (double)i;
+            others[i] = -values[i];
+        }
+        const std::size_t L1 = context.limbs_at(1), bytes = n / 2 * sizeof(double);
+        auto holds = [&](const uint64_t *words, const std::vector<double> &v) {
+            for (std::size_t l = 0; l < L1; l++)
+                if (std::memcmp(words + l * n, v.data(), bytes) != 0) return false;
+            return true;
+        };
+        auto stale = [&](CAHELGPUPlaintext &p) {   // what the block holds before the encoding runs
+            set_lane(0);
+            p.resize(L1, n);
+            std::memset(p.data_.get(), 0x77, p.data_.words() * 8);
+        };
+        CAHELGPUPlaintext p(context);
+        stale(p);
+        encoder.encode(context, values, 1099511627776.0, p);
+        REQUIRE(!holds(p.data_.get(), values));        // (the mock's device has not run it)
+        (void)p.lane_data();
+        REQUIRE(!holds(p.data_.get(), values));        // on its own lane nobody waits
+        set_lane(2);
+        REQUIRE(holds(p.lane_data(), values));         // another lane
+        stale(p);
+        encoder.encode(context, values, 1099511627776.0, p);
+        REQUIRE(holds(p.data(), values));              // data(): any stream
+        stale(p);
+        encoder.encode(context, values, 1099511627776.0, p);
+        CAHELGPUPlaintext moved = std::move(p);
+        set_lane(1);
+        CAHELGPUPlaintext copy = moved;                // a copy made on another lane
+        REQUIRE(holds(copy.data(), values));
+        CAHELGPUPlaintext record(context);
+        stale(moved);
+        encoder.encode(context, values, 1099511627776.0, moved);
+        set_lane(3);
+        const std::string bytes_of = saved(moved);     // a record written on another lane
+        std::istringstream is(bytes_of, std::ios::binary);
+        record.load(context, is);
+        REQUIRE(holds(record.data(), values));
+        stale(moved);
+        encoder.encode(context, values, 1099511627776.0, moved);
+        const uint64_t *block = moved.data_.get();
+        set_lane(4);
+        encoder.encode(context, others, 1099511627776.0, moved);   // encoded again on another lane: in a block of that lane
+        REQUIRE(moved.data_.get() != block && moved.data_.lane() == 4);
+        set_lane(0);
+        REQUIRE(holds(moved.lane_data(), others));
+        stale(p);
+        encoder.encode(context, others, 1099511627776.0, p);
+        set_lane(5);
+        p = copy;                                      // assigned to while its encoding runs: what is assigned stays
+        synchronize_lanes();
+        REQUIRE(holds(p.data_.get(), values));
+        set_lane(0);
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused

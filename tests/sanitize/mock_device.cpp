@@ -1,15 +1,30 @@
 // Host-memory stand-in for the C-ABI entry points that the host layer's table construction, record parsing and
 // containers call (he_malloc .. he_context_destroy, and he_keyswitch for a deferred relinearisation), so that those
 // CPU code paths can run under AddressSanitizer and UndefinedBehaviorSanitizer without a GPU.  Test infrastructure: "device" memory is malloc'ed host memory, copies
-// are memcpy, a context is an opaque token.  Nothing here computes.
+// are memcpy, a context is an opaque token.  Nothing here computes.  Streams are queues: an encoding that nothing waits for writes its
+// plaintext when its stream is next used or waited for, as late as a device may.
 #include <cstdlib>
 #include <cstring>
+#include <functional>
+#include <map>
+#include <vector>
 
 #include "cahel_hip.h"
 
 struct he_context {
     uint32_t log_n, size_q, size_p;
 };
+
+namespace {
+
+std::map<he_stream, std::vector<std::function<void()>>> queues;
+
+void run(he_stream stream) {
+    for (auto &work : queues[stream]) work();
+    queues[stream].clear();
+}
+
+}  // namespace
 
 extern "C" {
 
@@ -26,28 +41,58 @@ int he_free(void *dev_ptr) {
     return HE_OK;
 }
 
-int he_memcpy_h2d(void *dst, const void *src, size_t bytes, he_stream) {
+int he_memcpy_h2d(void *dst, const void *src, size_t bytes, he_stream stream) {
+    run(stream);
     if (bytes) std::memcpy(dst, src, bytes);
     return HE_OK;
 }
 
-int he_memcpy_d2h(void *dst, const void *src, size_t bytes, he_stream) {
+int he_memcpy_d2h(void *dst, const void *src, size_t bytes, he_stream stream) {
+    run(stream);
     if (bytes) std::memcpy(dst, src, bytes);
     return HE_OK;
 }
 
-int he_memcpy_d2d(void *dst, const void *src, size_t bytes, he_stream) {
+int he_memcpy_d2d(void *dst, const void *src, size_t bytes, he_stream stream) {
+    run(stream);
     if (bytes) std::memmove(dst, src, bytes);
     return HE_OK;
 }
 
 int he_stream_create(he_stream *stream) {
     if (!stream) return HE_E_INVALID_ARGUMENT;
-    *stream = nullptr;
+    static char tokens[64];
+    static int used = 0;
+    *stream = &tokens[used++ % 64];
     return HE_OK;
 }
 
-int he_stream_synchronize(he_stream) { return HE_OK; }
+int he_stream_synchronize(he_stream stream) {
+    run(stream);
+    return HE_OK;
+}
+
+int he_host_malloc(void **host_ptr, size_t bytes) { return he_malloc(host_ptr, bytes); }
+int he_host_free(void *host_ptr) { return he_free(host_ptr); }
+int he_memcpy_h2d_async(void *dst, const void *src, size_t bytes, he_stream stream) { return he_memcpy_h2d(dst, src, bytes, stream); }
+
+// an event knows the stream it was recorded on
+int he_event_create(he_event *event) {
+    *event = new he_stream(nullptr);
+    return HE_OK;
+}
+int he_event_destroy(he_event event) {
+    delete static_cast<he_stream *>(event);
+    return HE_OK;
+}
+int he_event_record(he_event event, he_stream stream) {
+    *static_cast<he_stream *>(event) = stream;
+    return HE_OK;
+}
+int he_event_synchronize(he_event event) {
+    run(*static_cast<he_stream *>(event));
+    return HE_OK;
+}
 
 int he_context_create(const he_context_desc *d, he_context **out) {
     if (!d || !out || !d->moduli || !d->barrett || !d->psi || !d->ipsi_div2) return HE_E_INVALID_ARGUMENT;
@@ -84,6 +129,37 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
 int he_context_destroy(he_context *ctx) {
     delete ctx;
     return HE_OK;
+}
+
+// "Encodes" later: the bits of value i as word i of every limb, zeros behind them.
+int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t, double, uint32_t limbs,
+                           uint32_t items, size_t, uint64_t *out, uint32_t, uint64_t *ws, he_stream stream) {
+    if (!ctx || !re || im || !out || !ws || items != 1) return HE_E_INVALID_ARGUMENT;
+    const size_t n = (size_t)1 << ctx->log_n;
+    queues[stream].push_back([=] {
+        std::memset(out, 0, limbs * n * sizeof(uint64_t));
+        for (uint32_t l = 0; l < limbs; l++) std::memcpy(out + l * n, re, count * sizeof(double));
+    });
+    return HE_OK;
+}
+
+size_t he_ckks_encode_batch_workspace_words(const he_context *, uint32_t items) { return 8 * (size_t)items; }
+
+// (what encoder.cpp refers to besides; not called)
+int he_ckks_encode(const he_context *, const double *, const double *, uint32_t, uint32_t, double, uint32_t, uint64_t *, uint64_t *,
+                   he_stream) { return HE_E_UNSUPPORTED; }
+int he_ckks_encode_batch(const he_context *, const double *, const double *, uint32_t, uint32_t, double, uint32_t, uint32_t, size_t,
+                         uint64_t *, uint32_t, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
+size_t he_encrypt_batch_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
+int he_encrypt_batch(const he_context *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, uint64_t *,
+                     he_stream) { return HE_E_UNSUPPORTED; }
+size_t he_ckks_workspace_words(const he_context *, uint32_t) { return 0; }
+int he_ckks_decode(const he_context *, const uint64_t *, uint32_t, uint32_t, double, double *, uint64_t *, he_stream) {
+    return HE_E_UNSUPPORTED;
+}
+size_t he_ckks_decode_real_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
+int he_ckks_decode_real(const he_context *, const uint64_t *, uint32_t, uint32_t, double, double *, uint32_t, uint64_t *, he_stream) {
+    return HE_E_UNSUPPORTED;
 }
 
 size_t he_keyswitch_workspace_words(const he_context *ctx, uint32_t L) { return ctx ? (size_t)L << ctx->log_n : 0; }

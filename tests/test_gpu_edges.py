@@ -1,5 +1,5 @@
 """Calls at the ends of what the entry points take: more rows of sums than one launch or one call of the C-ABI holds, decryption at
-the key level, batches of more threads than a launch has."""
+the key level, batches of more threads than a launch has, plaintexts used on another lane while their encoding runs."""
 import ctypes as C
 
 import numpy as np
@@ -23,6 +23,35 @@ def keys_for(cahel, parms, ctx):
     pk = cahel.public_key(ctx)
     sk.gen_publickey(ctx, pk)
     return sk, pk
+
+
+def test_encodings_used_on_other_lanes_at_once(oracle, capi):
+    """encode returns while its lane works: what another lane, another stream or a copy reads is the whole plaintext."""
+    cahel, parms, ctx, p = make_pair(oracle, 16, [60, 40, 40, 60], 1)
+    sk, pk = keys_for(cahel, parms, ctx)
+    sk.set_noise_flooding(False)
+    enc, rng, lib = cahel.ckks_encoder(ctx), np.random.default_rng(3), capi.lib()
+    z = rng.uniform(-1, 1, (6, p.n // 2))
+    want = [enc.encode(ctx, row, 2.0 ** 40).to_numpy() for row in z]
+    cahel._synchronize()
+    other = C.c_void_p()
+    capi.check(lib.he_stream_create(C.byref(other)))
+    try:
+        for turn, lane in enumerate([1, 2, 0, 3]):
+            cahel._set_lane(0)
+            plains = [enc.encode(ctx, row, 2.0 ** 40) for row in z]
+            words = np.empty_like(want[5])
+            capi.check(lib.he_memcpy_d2h(words.ctypes.data, plains[5].data_ptr(), words.nbytes, other))
+            cahel._set_lane(lane)
+            got = plains[4].to_numpy()
+            cts = [pk.encrypt_asymmetric(ctx, plain) for plain in plains[:4]]
+            back = [enc.decode_array(ctx, sk.decrypt(ctx, ct)) for ct in cts]
+            assert (words == want[5]).all() and (got == want[4]).all(), (turn, lane)
+            assert all(np.abs(b - row).max() < 1e-5 for b, row in zip(back, z)), (turn, lane)
+            cahel._synchronize()
+    finally:
+        cahel._set_lane(0)
+        lib.he_stream_destroy(other)
 
 
 @pytest.mark.parametrize("size,items", [(2, 16384), (4, 16384), (16, 4095), (16, 4096)])
