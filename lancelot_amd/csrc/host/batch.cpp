@@ -107,6 +107,10 @@ std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
             table.push_back(factors[k]->data());
         }
     }
+    // (multiply's condition on the product)
+    const double scale = first.scale() * factors[0]->scale();
+    if (scale <= 0 || static_cast<int>(std::log2(scale)) >= context.total_coeff_modulus_bit_count(first.chain_index()))
+        throw std::invalid_argument("scale out of bounds");
     he_stream st = context.stream();
     const uint32_t L = (uint32_t)first.coeff_modulus_size(), count = (uint32_t)factors.size();
     const std::size_t items = rows.size(), words = 3 * (std::size_t)L * context.poly_degree();
@@ -116,7 +120,7 @@ std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
         check_status(he_multiply_sum(context.handle(), L, (uint32_t)std::min(kRowsPerCall, items - k), count,
                                      reinterpret_cast<const uint64_t *const *>(d_table.get()) + k * 2 * count, out.get() + k * words, st),
                      "he_multiply_sum");
-    return slices(std::move(out), items, 3, first, first.scale() * factors[0]->scale());
+    return slices(std::move(out), items, 3, first, scale);
 }
 
 // For every (i, j) of `pairs`: acc = sum over chunks of (clients[j][c] - clients[i][c])^2, relinearised and rescaled,

@@ -25,6 +25,22 @@ def keys_for(cahel, parms, ctx):
     return sk, pk
 
 
+def test_products_refuse_the_scales_that_multiply_refuses(oracle):
+    """90 bits of modulus at this level: a product of scale 2^89 is one, of scale 2^90 none."""
+    cahel, parms, ctx, p = make_pair(oracle, 9, [50, 40, 50], 1)
+    sk, pk = keys_for(cahel, parms, ctx)
+    ct = pk.encrypt_asymmetric(ctx, cahel.ckks_encoder(ctx).encode(ctx, np.ones(p.n // 2), 2.0 ** 20))
+    for log_scale in (44.5, 45.0, 60.0):
+        ct.set_scale(2.0 ** log_scale)
+        calls = [lambda: cahel.multiply(ctx, ct, ct, cahel.ciphertext(ctx)), lambda: cahel.multiply_sum(ctx, [[ct, ct]], [ct, ct])]
+        for call in calls:
+            if log_scale < 45:
+                call()
+            else:
+                with pytest.raises(ValueError, match="scale out of bounds"):
+                    call()
+
+
 def test_encodings_used_on_other_lanes_at_once(oracle, capi):
     """encode returns while its lane works: what another lane, another stream or a copy reads is the whole plaintext."""
     cahel, parms, ctx, p = make_pair(oracle, 16, [60, 40, 40, 60], 1)
