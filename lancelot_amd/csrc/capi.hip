@@ -1489,9 +1489,8 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
     // (the complex scratch of an item is `slots` values = at most N words: the items are packed `slots` apart)
     // (the rounding kernel writes the residues itself: the coefficients never exist as an array of doubles)
-    const Tables tab = ctx->tables();
-    HE_HIP(launch_ckks_encode(ft, re, im, count, slots, scale, v, nullptr, ws, items, value_stride, S(s), &tab, out, limbs,
-                              (size_t)out_poly_stride * n));
+    HE_HIP(launch_ckks_encode(ft, ctx->tables(), re, im, count, slots, scale, v, ws, items, value_stride, out, limbs,
+                              (size_t)out_poly_stride * n, S(s)));
     return he_ntt_forward(ctx, out, items, out_poly_stride, limbs, 0, limbs, 0, s);
 }
 

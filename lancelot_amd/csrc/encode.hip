@@ -238,11 +238,9 @@ __global__ __launch_bounds__(64 * kFftWaves) void cfft_blocks_kernel(double2 *v,
                                                                      FftTarget dst) {
     using F = FftTile<INVERSE, 8, 8>;
     using T4 = typename F::T4;
-    __shared__ double re_all[kFftWaves][256 + 16], im_all[kFftWaves][256 + 16];
     const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63, item = blockIdx.y;
     const uint32_t blk = blockIdx.x * kFftWaves + w;
     if (blk >= 1u << (log_slots - 8)) return;   // (256 slots: one block)
-    double *re = re_all[w], *im = im_all[w];
     v += ((size_t)item << log_slots) + (size_t)blk * 256;
     auto pos = [&](int k, int j) { return T4::word(k, lane, j); };   // (the twiddles depend on the position inside the block)
     double2 x[4];
@@ -258,14 +256,14 @@ __global__ __launch_bounds__(64 * kFftWaves) void cfft_blocks_kernel(double2 *v,
             for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
         }
         F::load_tw(tw, t, log_slots, log_slots - 8, pos);
-        F::down(x, tw, re, im, lane);
+        F::down(x, tw, nullptr, nullptr, lane);   // (every exchange stays inside the wave)
 #pragma unroll
         for (int j = 0; j < 4; j++) v[pos(3, j)] = x[j];
     } else {
 #pragma unroll
         for (int j = 0; j < 4; j++) x[j] = v[pos(3, j)];
         F::load_tw(tw, t, log_slots, log_slots - 8, pos);
-        F::up(x, tw, re, im, lane);
+        F::up(x, tw, nullptr, nullptr, lane);
         if (dst.re && log_slots == 8) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
@@ -297,10 +295,9 @@ __device__ __forceinline__ void block_max_to(unsigned long long *dst, unsigned l
     }
 }
 
-// Where the rounded coefficients go: as doubles to coeffs [items][N], or (out given) as residues of the first `limbs`
-// primes to out [items][limbs][N], items out_item_stride words apart.
+// Where the rounded coefficients go: as residues of the first `limbs` primes to out [items][limbs][N], items out_item_stride words
+// apart.
 struct RoundSink {
-    double *coeffs;
     uint64_t *out;
     const uint64_t *moduli, *barrett;
     uint32_t limbs;
@@ -320,7 +317,6 @@ __global__ __launch_bounds__(kThreads) void encode_round_kernel(const double2 *v
                                                                 unsigned long long *max_bits) {
     const uint32_t c = blockIdx.x * kThreads + threadIdx.x;
     v += (size_t)blockIdx.y << log_slots;
-    double *coeffs = sink.coeffs + (size_t)blockIdx.y * 2 * half;
     max_bits += blockIdx.y;
     const bool imag = c >= half;
     const uint32_t k = imag ? c - half : c;
@@ -330,13 +326,8 @@ __global__ __launch_bounds__(kThreads) void encode_round_kernel(const double2 *v
         const double2 z = v[__brev(i) >> (32 - log_slots)];
         val = round((imag ? z.y : z.x) * fix);
     }
-    if (sink.out) {
-        uint64_t *o = sink.out + blockIdx.y * sink.out_item_stride + c;
-        for (uint32_t l = 0; l < sink.limbs; l++)
-            o[(size_t)l * 2 * half] = real_residue(val, sink.moduli[l], sink.barrett[2 * l + 1]);
-    } else {
-        coeffs[c] = val;
-    }
+    uint64_t *o = sink.out + blockIdx.y * sink.out_item_stride + c;
+    for (uint32_t l = 0; l < sink.limbs; l++) o[(size_t)l * 2 * half] = real_residue(val, sink.moduli[l], sink.barrett[2 * l + 1]);
     block_max_to(max_bits, (unsigned long long)__double_as_longlong(fabs(val)));
 }
 
@@ -351,7 +342,6 @@ __global__ __launch_bounds__(kThreads) void encode_round_tiled_kernel(const doub
     __shared__ double2 tile[16][17];
     const uint32_t x = threadIdx.x & 15, y = threadIdx.x >> 4, mid = blockIdx.x, mid_bits = log_slots - 8;
     v += (size_t)blockIdx.y << log_slots;
-    double *coeffs = sink.coeffs + (size_t)blockIdx.y * 2 * half;
     max_bits += blockIdx.y;
     const uint32_t rmid = mid_bits ? __brev(mid) >> (32 - mid_bits) : 0;
     const uint32_t brev4_y = __brev(y) >> 28;
@@ -360,16 +350,11 @@ __global__ __launch_bounds__(kThreads) void encode_round_tiled_kernel(const doub
     const double2 z = tile[x][y];
     const uint32_t i = (brev4_y << (log_slots - 4)) | (mid << 4) | x;
     const double re = round(z.x * fix), im = round(z.y * fix);
-    if (sink.out) {
-        uint64_t *o = sink.out + blockIdx.y * sink.out_item_stride + i;
-        for (uint32_t l = 0; l < sink.limbs; l++) {
-            const uint64_t q = sink.moduli[l], r1 = sink.barrett[2 * l + 1];
-            o[(size_t)l * 2 * half] = real_residue(re, q, r1);
-            o[(size_t)l * 2 * half + half] = real_residue(im, q, r1);
-        }
-    } else {
-        coeffs[i] = re;
-        coeffs[half + i] = im;
+    uint64_t *o = sink.out + blockIdx.y * sink.out_item_stride + i;
+    for (uint32_t l = 0; l < sink.limbs; l++) {
+        const uint64_t q = sink.moduli[l], r1 = sink.barrett[2 * l + 1];
+        o[(size_t)l * 2 * half] = real_residue(re, q, r1);
+        o[(size_t)l * 2 * half + half] = real_residue(im, q, r1);
     }
     const double big = fabs(re) > fabs(im) ? fabs(re) : fabs(im);
     block_max_to(max_bits, (unsigned long long)__double_as_longlong(big));
@@ -551,16 +536,15 @@ __global__ __launch_bounds__(kThreads) void take_slots_kernel(const double2 *v, 
 
 }  // namespace
 
-hipError_t launch_ckks_encode(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
-                              double scale, double2 *v, double *coeffs, uint64_t *max_bits, uint32_t items,
-                              size_t value_stride, hipStream_t s, const Tables *tab, uint64_t *out, uint32_t limbs,
-                              size_t out_item_stride) {
+hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const double *re, const double *im, uint32_t count,
+                              uint32_t slots, double scale, double2 *v, uint64_t *max_bits, uint32_t items, size_t value_stride,
+                              uint64_t *out, uint32_t limbs, size_t out_item_stride, hipStream_t s) {
     const uint32_t n = 1u << t.log_n, log_slots = 31 - __builtin_clz(slots);
-    if (items == 0 || items > 65535 || (out ? (!tab || limbs == 0) : !coeffs)) return hipErrorInvalidValue;
+    if (items == 0 || items > 65535 || !out || limbs == 0) return hipErrorInvalidValue;
     unsigned long long *maxima = reinterpret_cast<unsigned long long *>(max_bits);
     hipError_t e = run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, maxima}, FftTarget{nullptr, 0, 0});
     if (e != hipSuccess) return e;
-    const RoundSink sink{coeffs, out, out ? tab->moduli : nullptr, out ? tab->barrett : nullptr, limbs, out_item_stride};
+    const RoundSink sink{out, tab.moduli, tab.barrett, limbs, out_item_stride};
     if (slots == n / 2 && log_slots >= 8)
         hipLaunchKernelGGL(encode_round_tiled_kernel, dim3(slots / kThreads, items), dim3(kThreads), 0, s, v, log_slots, n / 2,
                            scale / (double)slots, sink, maxima);

@@ -198,17 +198,17 @@ hipError_t launch_scalar_mul_add(const Tables &t, const uint64_t *a, const uint6
 hipError_t launch_tensor(const Tables &t, const uint64_t *ct1, const uint64_t *ct2, uint64_t *out, uint32_t L,
                          bool square, hipStream_t s, const double *fp_consts = nullptr, uint32_t items = 1,
                          uint64_t *out2 = nullptr);
-// ct1 [s1][L][N] x ct2 [s2][L][N] -> out [s1 + s2 - 1][L][N], 1 <= s1, s2 <= 3
+// ct1 [s1][L][N] x ct2 [s2][L][N] -> out [s1 + s2 - 1][L][N], 1 <= s1, s2 <= 16
 hipError_t launch_tensor_mxn(const Tables &t, const uint64_t *ct1, uint32_t s1, const uint64_t *ct2, uint32_t s2,
                              uint64_t *out, uint32_t L, hipStream_t s);
-// (out01 [items][2][L][N], out2 [items][L][N]) = sum over chunks of (a - b)^2 for the pairs of ciphertexts in the
-// device pointer table pairs [items][chunks][2]
 // sums of `count` ciphertexts, and of `count` products of two size-2 ciphertexts: tables of device pointers in device memory,
 // N >= 512
 hipError_t launch_sum(const Tables &t, const uint64_t *const *cts, uint64_t *out, uint32_t limbs, uint32_t polys, uint32_t items,
                       uint32_t count, hipStream_t s);
 hipError_t launch_multiply_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out, uint32_t limbs, uint32_t items,
                                uint32_t count, hipStream_t s);
+// (out01 [items][2][L][N], out2 [items][L][N]) = sum over chunks of (a - b)^2 for the pairs of ciphertexts in the
+// device pointer table pairs [items][chunks][2]
 hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out01, uint64_t *out2,
                                   uint32_t L, uint32_t items, uint32_t chunks, hipStream_t s);
 hipError_t launch_galois(const Tables &t, const uint64_t *in, uint64_t *out, uint32_t total_limbs, uint32_t elt,
@@ -410,14 +410,12 @@ struct FftTables {
     const double2 *ksi;
     uint32_t log_n;
 };
-// values (count <= slots, zero padded) -> rounded real coefficients [N]; *max_bits receives the bit pattern of the
-// largest |coefficient| (a non-negative double).  v: scratch of `slots` complex values.  With `out` the coefficients
-// leave as residues of the first `limbs` primes of `tab` instead (out [items][limbs][N], items out_item_stride words
-// apart) and coeffs is not written.
-hipError_t launch_ckks_encode(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
-                              double scale, double2 *v, double *coeffs, uint64_t *max_bits, uint32_t items,
-                              size_t value_stride, hipStream_t s, const Tables *tab = nullptr, uint64_t *out = nullptr,
-                              uint32_t limbs = 0, size_t out_item_stride = 0);
+// values (count <= slots, zero padded) -> rounded coefficients as residues of the first `limbs` primes of `tab` (out
+// [items][limbs][N], items out_item_stride words apart); max_bits[item] receives the bit pattern of the largest |coefficient| (a
+// non-negative double).  v: scratch of `slots` complex values per item.
+hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const double *re, const double *im, uint32_t count,
+                              uint32_t slots, double scale, double2 *v, uint64_t *max_bits, uint32_t items, size_t value_stride,
+                              uint64_t *out, uint32_t limbs, size_t out_item_stride, hipStream_t s);
 // Only the transform: the slot vectors stay in v [items][slots] for NTT_PRO_ROUND.  re / im may be page-locked host memory.
 hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
                                    double2 *v, uint32_t items, size_t value_stride, hipStream_t s);

@@ -253,43 +253,6 @@ __device__ __forceinline__ uint32_t galois_index(uint32_t i, uint32_t elt, uint3
     return __brev(raw) >> (32 - log_n);
 }
 
-// R = 2^LOGR point decimation-in-time block: LOGR consecutive forward stages on register values.
-// v[j] are the elements whose index differs in the LOGR bits that these stages pair, most significant
-// first; idx = 2^s0 + (group number at the first stage s0); twiddle of local stage l, sub-block b is
-// table[(idx << l) + b].
-template <int LOGR>
-__device__ __forceinline__ void ct_block(uint64_t *v, const uint64_t *table, uint32_t idx, uint64_t q) {
-    constexpr int R = 1 << LOGR;
-    const IntMod m = int_mod(q);
-#pragma unroll
-    for (int l = 0; l < LOGR; l++) {
-        const int half = R >> (l + 1);
-#pragma unroll
-        for (int b = 0; b < (1 << l); b++) {
-            Shoup tw = load_shoup(table, ((size_t)idx << l) + b);
-#pragma unroll
-            for (int j = 0; j < half; j++) ct_butterfly(v[2 * b * half + j], v[2 * b * half + j + half], tw, m);
-        }
-    }
-}
-
-// The mirror image: the same LOGR stages in inverse order with Gentleman-Sande butterflies.
-template <int LOGR>
-__device__ __forceinline__ void gs_block(uint64_t *v, const uint64_t *table, uint32_t idx, uint64_t q) {
-    constexpr int R = 1 << LOGR;
-    const IntMod m = int_mod(q);
-#pragma unroll
-    for (int l = LOGR - 1; l >= 0; l--) {
-        const int half = R >> (l + 1);
-#pragma unroll
-        for (int b = 0; b < (1 << l); b++) {
-            Shoup tw = load_shoup(table, ((size_t)idx << l) + b);
-#pragma unroll
-            for (int j = 0; j < half; j++) gs_butterfly(v[2 * b * half + j], v[2 * b * half + j + half], tw, m);
-        }
-    }
-}
-
 }  // namespace he
 
 // ---------------------------------------------------------------------------------------------------
@@ -351,7 +314,9 @@ __device__ __forceinline__ FpTw load_fptw(const double *table, size_t idx, FpMod
     return FpTw{w, w * m.qinv};
 }
 
-// Forward block on lazy signed doubles.  REDUCE_FIRST = 1 brings every input back to |v| <= q/2; from there
+// Forward block: LOGR consecutive forward stages on 2^LOGR lazy signed doubles.  v[j] are the elements whose index differs in the
+// LOGR bits that these stages pair, most significant first; idx = 2^s0 + (group number at the first stage s0); twiddle of local
+// stage l, sub-block b is table[(idx << l) + b].  REDUCE_FIRST = 1 brings every input back to |v| <= q/2; from there
 // (or from canonical inputs) the bound grows by 1.375 b + 0.5 per stage: 5.3 q after four stages, 7.1 q from
 // canonical inputs, always below 8 q < 2^53.
 // REDUCE_FIRST = 2 reduces only the inputs that the first stage adds and subtracts; those that it multiplies go into
@@ -405,73 +370,6 @@ __device__ __forceinline__ void fp_gs_block(double *v, const double *table, uint
                 const double x = v[2 * b * half + j], y = v[2 * b * half + j + half];
                 v[2 * b * half + j] = x + y;
                 v[2 * b * half + j + half] = fp_mulmod(x - y, tw, m);
-            }
-        }
-        if (LOGR >= 4 && l > 0 && ((LOGR - l) & 1) == 0) {
-#pragma unroll
-            for (int b = 0; b < (1 << l); b++)
-#pragma unroll
-                for (int j = 0; j < half; j++) v[2 * b * half + j] = fp_reduce(v[2 * b * half + j], m);
-        }
-    }
-}
-
-// The same blocks with the 2^LOGR - 1 twiddles already in registers (tw[2^l - 1 + b] for stage l, sub-block b):
-// a workgroup that transforms several limbs of one modulus loads them once.
-template <int LOGR>
-__device__ __forceinline__ void fp_load_block_tw(double *tw, const double *table, uint32_t idx) {
-#pragma unroll
-    for (int l = 0; l < LOGR; l++)
-#pragma unroll
-        for (int b = 0; b < (1 << l); b++) tw[(1 << l) - 1 + b] = table[((size_t)idx << l) + b];
-}
-
-template <int LOGR, bool REDUCE_FIRST>
-__device__ __forceinline__ void fp_ct_block_tw(double *v, const double *tw, FpMod m) {
-    constexpr int R = 1 << LOGR;
-    if (REDUCE_FIRST) {
-#pragma unroll
-        for (int j = 0; j < R; j++) v[j] = fp_reduce(v[j], m);
-    }
-#pragma unroll
-    for (int l = 0; l < LOGR; l++) {
-        const int half = R >> (l + 1);
-#pragma unroll
-        for (int b = 0; b < (1 << l); b++) {
-            double w = tw[(1 << l) - 1 + b];
-            asm volatile("" : "+v"(w));  // keeps w * qinv out of the caller's loop-invariant registers
-            const FpTw t{w, w * m.qinv};
-#pragma unroll
-            for (int j = 0; j < half; j++) {
-                const double x = v[2 * b * half + j];
-                const double p = fp_mulmod(v[2 * b * half + j + half], t, m);
-                v[2 * b * half + j] = x + p;
-                v[2 * b * half + j + half] = x - p;
-            }
-        }
-    }
-}
-
-template <int LOGR, bool REDUCE_FIRST>
-__device__ __forceinline__ void fp_gs_block_tw(double *v, const double *tw, FpMod m) {
-    constexpr int R = 1 << LOGR;
-    if (REDUCE_FIRST) {
-#pragma unroll
-        for (int j = 0; j < R; j++) v[j] = fp_reduce(v[j], m);
-    }
-#pragma unroll
-    for (int l = LOGR - 1; l >= 0; l--) {
-        const int half = R >> (l + 1);
-#pragma unroll
-        for (int b = 0; b < (1 << l); b++) {
-            double w = tw[(1 << l) - 1 + b];
-            asm volatile("" : "+v"(w));  // keeps w * qinv out of the caller's loop-invariant registers
-            const FpTw t{w, w * m.qinv};
-#pragma unroll
-            for (int j = 0; j < half; j++) {
-                const double x = v[2 * b * half + j], y = v[2 * b * half + j + half];
-                v[2 * b * half + j] = x + y;
-                v[2 * b * half + j + half] = fp_mulmod(x - y, t, m);
             }
         }
         if (LOGR >= 4 && l > 0 && ((LOGR - l) & 1) == 0) {
