@@ -1,10 +1,13 @@
 """Calls at the ends of what the entry points take: more rows of sums than one launch or one call of the C-ABI holds, decryption at
-the key level, batches of more threads than a launch has, plaintexts used on another lane while their encoding runs."""
+the key level, batches of more threads than a launch has, plaintexts used on another lane while their encoding runs, buffers that are aligned to one
+word only."""
 import ctypes as C
 
 import numpy as np
 import pytest
 
+import test_gpu_fused_rows as fused_rows
+import test_gpu_passes as passes
 from gpu_util import DeviceArray, make_pair, rand_limbs
 
 pytestmark = pytest.mark.gpu
@@ -197,3 +200,48 @@ def test_encryptions_of_more_words_than_a_launch_holds(oracle, capi):
             lib.he_free(ws)
     finally:
         lib.he_free(cts)
+
+
+class OddArray(DeviceArray):
+    """A device buffer that starts 8 bytes behind a 16-byte boundary."""
+
+    def __init__(self, capi, shape=None, host=None, dtype=np.uint64):
+        host = None if host is None else np.ascontiguousarray(host)
+        self.capi = capi
+        self.shape, self.dtype = (tuple(shape), np.dtype(dtype)) if host is None else (host.shape, host.dtype)
+        self.nbytes = int(np.prod(self.shape)) * self.dtype.itemsize
+        self.base = C.c_void_p()
+        capi.check(capi.lib().he_malloc(C.byref(self.base), self.nbytes + 16), "he_malloc")
+        self.ptr = self.base.value + 8
+        assert self.ptr % 16 == 8
+        if host is not None:
+            capi.check(capi.lib().he_memcpy_h2d(self.ptr, host.ctypes.data, self.nbytes, None), "h2d")
+
+    def free(self):
+        if self.ptr:
+            self.capi.lib().he_free(self.base.value)
+            self.ptr = None
+
+
+@pytest.mark.parametrize("chain", ["fp", "int", "mixed"])
+def test_buffers_aligned_to_one_word(oracle, capi, monkeypatch, chain):
+    """The header asks for 8-byte alignment; the passes and what is fused with them move 16 bytes at a time."""
+    monkeypatch.setattr(passes, "DeviceArray", OddArray)
+    passes.test_batched_transforms(oracle, capi, chain, 15, 5, 30)
+    passes.test_batched_transforms(oracle, capi, chain, 12, 3, 2)
+    passes.test_encrypt_and_decrypt(oracle, capi, chain, 13, 2, 3)
+    passes.test_bounded_encoding_and_real_decoding(oracle, capi, chain, 13, 4096, 3)
+    passes.test_hoisting_of_one_ciphertext(oracle, capi, chain, 12, 2, 4, 3)
+    passes.test_hoisting_of_one_ciphertext(oracle, capi, chain, 16, 2, 4, 3)
+    for local in (False, True):
+        passes.test_hoisting_of_batches(oracle, capi, chain, local, 12, 2, 4, 4, 5)
+    passes.test_sums_of_ciphertexts_and_products(oracle, capi, chain, 13, 2, 2, 17)
+
+
+@pytest.mark.parametrize("case", [c for c in fused_rows.CASES if c[0] in (12, 14)] + [(16, [50] * 6, 2, (4,))])
+def test_key_switches_of_buffers_aligned_to_one_word(oracle, capi, monkeypatch, case):
+    monkeypatch.setattr(fused_rows, "DeviceArray", OddArray)
+    fused_rows.test_entry_points_with_fused_conversion(oracle, capi, monkeypatch, *case, "0")
+    fused_rows.test_multiply_relin_rescale_entry_point(oracle, capi, monkeypatch, *case, "0")
+    for inner in ("fused", "fp_kernel"):
+        fused_rows.test_multiply_relin_rescale_batch_equals_single_calls(oracle, capi, monkeypatch, *case[:3], case[3][0], 3, inner)
