@@ -464,7 +464,7 @@ def test_c5_pair_distances_against_the_oracle():
 @pytest.mark.parametrize("no_fuse", ["0", "1"])
 def test_largest_degree_entry_points_bit_exact(oracle, monkeypatch, bits, size_p, L, no_fuse):
     """N = 2^17, the largest degree of the reference's parameter tables (include/util/hestdparms.h): the rows pass has
-    512 rows there (a register block of five stages), the base conversions run as kernels of their own.  he_keyswitch,
+    512 rows there (nine stages), the base conversions run as kernels of their own.  he_keyswitch,
     he_keyswitch_rescale, he_multiply_relin_rescale, he_rotate and he_hoisted_rotations against the oracle, every
     limb, on the FP64 and the mixed back end, with the inner product inside the forward transform and as a kernel of
     its own, with a partial last digit."""

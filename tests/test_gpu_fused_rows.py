@@ -95,7 +95,7 @@ def test_entry_points_with_fused_conversion(oracle, capi, monkeypatch, logn, bit
                 dct, dout = DeviceArray(capi, host=ct), DeviceArray(capi, shape=(2, L - 1, n))
                 capi.check(lib.he_keyswitch_rescale(h, L, dc.ptr, ptrs, dct.ptr, dout.ptr, elt, kws.ptr, None))
                 assert (dout.numpy() == p.rescale(want)).all(), ("keyswitch_rescale", L, elt)
-        # the batch form over three inputs (separate kernels for the inner product, same conversions)
+        # the batch form over several inputs
         if L >= 2:
             items = 4 if logn == 16 else 3   # (four items: the merged ModDown + rescale then takes the matrix-core kernel at N = 2^16)
             c3 = rand_limbs(p, rng, range(L), n_polys=items)
@@ -113,9 +113,8 @@ def test_entry_points_with_fused_conversion(oracle, capi, monkeypatch, logn, bit
 @pytest.mark.parametrize("no_fused", ["0", "1"])
 @pytest.mark.parametrize("logn,bits,size_p,levels", CASES + [(11, [45, 40, 40, 50], 1, (3, 2)), (12, [60, 40, 50, 45, 30, 59, 60, 60], 2, (6, 3))])
 def test_multiply_relin_rescale_entry_point(oracle, capi, monkeypatch, logn, bits, size_p, levels, no_fused):
-    """he_multiply_relin_rescale (tensor product formed inside the key switch's first pass when every prime is below
-    2^50; tensor kernel + key switch otherwise or when switched off) against the oracle's tensor, relinearize and
-    rescale; a product of two ciphertexts and a square."""
+    """he_multiply_relin_rescale (tensor product formed inside the key switch's first pass; tensor kernel + key switch when
+    switched off) against the oracle's tensor, relinearize and rescale; a product of two ciphertexts and a square."""
     monkeypatch.setenv("CAHEL_HIP_NO_FUSED_TENSOR", no_fused)
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(200 + logn)
@@ -153,10 +152,10 @@ def test_multiply_relin_rescale_entry_point(oracle, capi, monkeypatch, logn, bit
                                                        (12, [50, 49, 48, 50, 47, 50, 50, 50], 2, 6, 7)])
 @pytest.mark.parametrize("inner", ["fused", "fp_kernel"])
 def test_multiply_relin_rescale_batch_equals_single_calls(oracle, capi, monkeypatch, logn, bits, size_p, L, items, inner):
-    """The batch entry point against the oracle item by item.  With every prime below 2^50 its inner product runs
-    inside the blocks pass of ModUp's forward transform, the items of one tile next to each other on one XCD
-    ("fused"); switched off, it is the FP64 kernel that shares key words among up to 8 items (groups of 2, 4 and 8,
-    full and partial); with larger primes (the second parameter set) the integer kernel."""
+    """The batch entry point against the oracle item by item.  Its inner product runs inside the blocks pass of ModUp's forward
+    transform, the items of one block next to each other on one XCD ("fused"); switched off, it is, with every prime below
+    2^50, the FP64 kernel that shares key words among up to 8 items (groups of 2, 4 and 8, full and partial), with larger
+    primes (the second parameter set) the integer kernel."""
     monkeypatch.setenv("CAHEL_HIP_NO_BATCH_FUSED_KS", "0" if inner == "fused" else "1")
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(300 + logn)

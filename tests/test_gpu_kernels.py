@@ -185,7 +185,7 @@ def test_mixed_back_end_agrees_with_the_integer_one(oracle, capi, monkeypatch, l
                                                  (14, [50, 49, 48, 50, 47, 50, 50, 50, 50], 3, 5),
                                                  (11, [45, 40, 40, 50], 1, 3), (9, [40, 40, 45, 45], 2, 2)])
 def test_fused_and_separate_key_switch_agree(oracle, capi, monkeypatch, logn, bits, size_p, L):
-    """he_keyswitch with the inner product inside the forward NTT (the default for primes below 2^50) and, forced
+    """he_keyswitch with the inner product inside the forward NTT (the default) and, forced
     by the environment, with the separate kernels: both equal the oracle, with and without a Galois element, with a
     partial last digit (L = 3 over two special primes, L = 5 over three), and at the smallest degree."""
     for no_fuse in ("0", "1"):
@@ -304,7 +304,7 @@ def test_hoisted_rotations_entry_point(oracle, capi, logn, bits, size_p, L, n_st
 def test_hoisted_rotations_with_block_local_steps(oracle, capi, monkeypatch, logn, bits, size_p, L, items, no_local):
     """Steps that are multiples of N / 512 (Galois elements 1 modulo 2^(log N - 7)) permute the NTT order inside
     aligned blocks of 256 words; the batch kernel then gathers from a copy of the block in LDS.  Against the oracle
-    item by item, with that path on and switched off, for groups of 8 + 1, 2 + 1 and 2 items."""
+    item by item, with that path on and switched off, for groups of 4, 4 and a rest of one, of 2 and one, and of 2 items."""
     monkeypatch.setenv("CAHEL_HIP_NO_LOCAL_HOIST", no_local)
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(17)
@@ -335,8 +335,8 @@ def test_hoisted_rotations_with_block_local_steps(oracle, capi, monkeypatch, log
 @pytest.mark.parametrize("bits,L", [([60, 60, 60, 60, 60], 4), ([50, 49, 50, 50, 50], 4), ([60, 40, 60, 40, 60], 4)])
 def test_hoisted_rotations_largest_residues(oracle, capi, bits, L, local):
     """Every residue of the inputs and of the keys is q - 1 and the launch has the most products it accepts (16 steps x
-    4 digits = 64 per output word): the lazy sums of the hoisting kernel (three 64-bit words relieved every 8 terms for
-    the 60-bit primes, the exact FP64 pair for those below 2^50) and its final 128-bit reduction at their bounds.
+    4 digits = 64 per output word): the lazy sums of the hoisting kernel (two 64-bit words and a signed one, relieved every 8
+    terms for the 60-bit primes, the exact FP64 pair for those below 2^50) and its final 128-bit reduction at their bounds.
     5 items: a group of 4 and a remainder.  Against the oracle, item by item."""
     logn, size_p, items, n_steps = 11, 1, 5, 16
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
@@ -738,7 +738,7 @@ def test_keyswitch_benchmark_shape(full, capi):
 
 @pytest.mark.parametrize("no_fp", ["0", "1"])
 def test_rows_pass_on_registers_at_benchmark_shape(oracle, capi, monkeypatch, no_fp):
-    """N = 2^16 with enough limbs for full tiles: the rows pass keeps its outer half on registers.  Both back ends
+    """N = 2^16 with enough limbs for tiles of 2048 words in the rows pass.  Both back ends
     (FP64, and the integer one forced by the environment) against the oracle: plain forward and inverse transforms,
     the rescale (prologue that broadcasts the last limb) and key switch + rescale (prologue of the merged ModDown +
     rescale, inverse transform with a scaling epilogue)."""
