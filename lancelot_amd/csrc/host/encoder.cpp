@@ -238,10 +238,12 @@ void CAHELGPUCKKSEncoder::decode_real(const CAHELGPUContext &context, const CAHE
     he_context *h = context.handle();
     const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
     DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)sparse_slots_));
-    double *host = static_cast<double *>(PinnedRing::of_thread().take(count * sizeof(double)));
-    check_status(he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
-                                     context.stream()),
-                 "he_ckks_decode_real");
+    PinnedRing &ring = PinnedRing::of_thread();
+    double *host = static_cast<double *>(ring.take(count * sizeof(double)));
+    const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
+                                           context.stream());
+    if (status != HE_OK) ring.fence(context.stream());   // (what was launched before the failure may still write the block)
+    check_status(status, "he_ckks_decode_real");
     check_status(he_stream_synchronize(context.stream()), "synchronisation failed");
     std::memcpy(destination, host, count * sizeof(double));
 }

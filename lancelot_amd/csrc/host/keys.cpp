@@ -255,7 +255,7 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
     const uint64_t **table = static_cast<const uint64_t **>(ring.take(items * sizeof(uint64_t)));
     for (uint32_t k = 0; k < items; k++) table[k] = ciphers[k]->data();
     DeviceBuffer d_table(items);
-    const int status = he_memcpy_h2d_async(d_table.get(), table, items * sizeof(uint64_t), st);
+    int status = he_memcpy_h2d_async(d_table.get(), table, items * sizeof(uint64_t), st);
     ring.fence(st);
     check_status(status, "upload");
     const std::size_t bytes = (std::size_t)items * count * sizeof(double);
@@ -264,12 +264,12 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
     if (!staged) d_out.allocate((std::size_t)items * count);
     double *out = staged ? static_cast<double *>(ring.take(bytes)) : reinterpret_cast<double *>(d_out.get());
     // flooding noise: the stream ids that `items` calls of decrypt would draw
-    check_status(he_decrypt_decode_real_batch(h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs,
-                                              sk_powers_.get(), noise_flooding_ ? context.prng_key() : nullptr,
-                                              noise_flooding_ ? context.next_stream(items) : 0, context.gauss_cdt(),
-                                              context.gauss_cdt_len(), (uint32_t)slots, first.scale(), (uint32_t)count, out,
-                                              ws.get(), st),
-                 "he_decrypt_decode_real_batch");
+    status = he_decrypt_decode_real_batch(h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs, sk_powers_.get(),
+                                          noise_flooding_ ? context.prng_key() : nullptr,
+                                          noise_flooding_ ? context.next_stream(items) : 0, context.gauss_cdt(),
+                                          context.gauss_cdt_len(), (uint32_t)slots, first.scale(), (uint32_t)count, out, ws.get(), st);
+    if (status != HE_OK && staged) ring.fence(st);   // (what was launched before the failure may still write the block)
+    check_status(status, "he_decrypt_decode_real_batch");
     if (staged) {
         check_status(he_stream_synchronize(st), "synchronisation failed");
         std::memcpy(destination, out, bytes);

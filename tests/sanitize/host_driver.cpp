@@ -12,6 +12,7 @@
 #include <vector>
 
 #include "cahel.h"
+#include "staging.h"
 
 using namespace cahel;
 
@@ -238,6 +239,17 @@ int main(int argc, char **argv) {
         synchronize_lanes();
         REQUIRE(holds(p.data_.get(), values));
         set_lane(0);
+        // a decoding that fails behind its first launches: their writes come before the staging block is handed out again
+        PinnedRing &ring = PinnedRing::of_thread();
+        for (int i = 0; i < PinnedRing::kBlocks; i++) (void)ring.take(bytes);   // (nothing is left of the encodings above)
+        REQUIRE(refuses([&] { encoder.decode_real(context, p, n / 2, others.data()); }));
+        std::vector<double *> blocks;
+        for (int i = 0; i < PinnedRing::kBlocks; i++) {
+            blocks.push_back(static_cast<double *>(ring.take(bytes)));
+            std::memcpy(blocks.back(), values.data(), bytes);
+        }
+        synchronize_lanes();
+        for (double *b : blocks) REQUIRE(std::memcmp(b, values.data(), bytes) == 0);
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused
