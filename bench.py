@@ -5,7 +5,7 @@
 
 One "step" is one homomorphic multiplication with relinearisation and rescale (tensor product -> hybrid key
 switch with dnum = 3 digits -> rescale) of two fresh ciphertexts at N = 2^16, L = 24 data limbs and 8 special
-limbs of 50 bits, scale 2^40 (BASELINE.json configs[2]), on buffers that are resident in HBM before the timed region
+limbs of 50 bits, scale 2^40, on buffers that are resident in HBM before the timed region
 starts.  Every figure is the median of BLOCKS timed blocks of K steps each, after W warm-up steps.  Prints ONE JSON
 line.
 
@@ -26,11 +26,11 @@ Extra objects on the line:
                 has to move (the key once per launch)
   ntt           config "batched forward + inverse NTT, 24 limbs x 2 polynomials": GB/s of limb data
   rotate        one rotation with key switch; rotate-and-sum over 15 steps
-  krum          the encrypted Krum round at its real shape, with the CPU checker's time for the same evaluate phase,
+  krum          the encrypted Krum round at its real shape, with the CPU oracle's time for the same evaluate phase,
                 and the distance phase driven call for call as lancelot-main-GPU's byzantine_fl.py does
                 (`reference_call_sequence`: 55 pairs, operands encoded and encrypted again for every pair)
-  cpu_baseline  the CPU checker (oracle/, OpenMP) on the same HMult+relin+rescale workload, bounded sample; and at
-                BASELINE.json configs[0] (N = 2^14, 4 + 1 primes)
+  cpu_baseline  the CPU oracle (oracle/, OpenMP) on the same HMult+relin+rescale workload, bounded sample; and at
+                the small product (N = 2^14, 4 + 1 primes)
 """
 import argparse
 import ctypes as C
@@ -121,7 +121,7 @@ class Buf:
 
 
 def cpu_hmult(log_n, size_q, size_p, seconds_budget):
-    """HMult + relinearise + rescale on the CPU checker (random residues): (ops/s, iterations, threads)."""
+    """HMult + relinearise + rescale on the CPU oracle (random residues): (ops/s, iterations, threads)."""
     from oracle import ckks_oracle as O
     n = 1 << log_n
     mods = O.coeff_modulus_create(n, [BITS] * (size_q + size_p))
@@ -161,7 +161,7 @@ def cpu_baseline():
                       "oracle/ckks_oracle.c with OpenMP" % iters,
             "ms_per_op": 1e3 / v,
             "config_c1": {"value": v1, "unit": "HMult+relin+rescale ops/s", "cores": threads,
-                          "workload": "BASELINE.json configs[0]: N=2^14, 4 limbs of 50 bits + 1 special prime",
+                          "workload": "N=2^14, 4 limbs of 50 bits + 1 special prime",
                           "sample": "%d iterations" % iters1, "ms_per_op": 1e3 / v1}}
 
 
@@ -205,14 +205,14 @@ def gpu_c1(capi, cahel, timer, steps=400):
     got = np.empty((2, L - 1, n), dtype=np.uint64)
     capi.check(lib.he_memcpy_d2h(got.ctypes.data, bres.at((B - 1) * 2 * (L - 1) * n), got.nbytes, None))
     err = float(np.max(np.abs(np.array(enc.decode(ctx, sk.decrypt(ctx, prod))) - x * y)))
-    return {"workload": "BASELINE.json configs[0]: HMult+relinearize+rescale, N=2^14, 4 limbs of 50 bits + 1 special prime",
+    return {"workload": "HMult+relinearize+rescale, N=2^14, 4 limbs of 50 bits + 1 special prime",
             "single_stream": {"ms_per_step": single, "ops_per_s": 1e3 / single},
             "batch": {"ms_per_step": batch, "ops_per_s": 1e3 / batch, "ops_per_call": B},
             "batch_equals_single": bool((got == prod.to_numpy()).all()), "decrypt_max_abs_err_vs_xy": err}
 
 
 def krum_cpu_evaluate(updates, pairs_sampled=2):
-    """The evaluate phase of the Krum round on the CPU checker: per pair sub, square and add over the chunks,
+    """The evaluate phase of the Krum round on the CPU oracle: per pair sub, square and add over the chunks,
     relinearise, rescale, and the slot sum as 15 rotations (each a key switch) + additions, with Lancelot's
     parameters; `pairs_sampled` pairs are timed and the figure is scaled to the 45 pairs of the round."""
     from oracle import ckks_oracle as O
@@ -248,7 +248,7 @@ def krum_cpu_evaluate(updates, pairs_sampled=2):
             r = np.stack([p.add(r[k], rot[k]) for k in range(2)])
     per_pair = (time.time() - t0) / pairs_sampled
     return {"evaluate_s": per_pair * 45, "sample": "%d of the 45 pairs timed (%.3f s each) on oracle/ckks_oracle.c, "
-            "%d threads; rotations one key switch each (the checker has no hoisting)"
+            "%d threads; rotations one key switch each (the oracle has no hoisting)"
             % (pairs_sampled, per_pair, int(os.environ.get("OMP_NUM_THREADS", os.cpu_count() or 1)))}
 
 
@@ -316,7 +316,7 @@ def main():
                          "hardware queues of a process)")
     ap.add_argument("--batch", type=int, default=8, help="operations per he_multiply_relin_rescale_batch call")
     ap.add_argument("--batch-streams", type=int, default=2, help="streams that the batch calls are dealt to")
-    ap.add_argument("--no-krum", action="store_true", help="skip the encrypted Krum round (BASELINE.json configs[4])")
+    ap.add_argument("--no-krum", action="store_true", help="skip the encrypted Krum round of 10 clients")
     ap.add_argument("--only", choices=["all", "step", "batch", "batch_streams", "rotate", "ntt", "krum", "krum_reference", "probe"], default="all",
                     help="step / batch / rotate / ntt: run just that workload on the null stream (for rocprofv3); "
                          "batch_streams: the batch calls dealt to --batch-streams streams, as `value` issues them; "
@@ -628,7 +628,7 @@ def main():
                   "calls of %d operations for `batch` and %d such calls for `batch_streams` (`value`), whatever --steps says"
                   % (BLOCKS, W, K_steps, calls, B, bs_calls),
         "config": {"workload": "HMult+relinearize+rescale, N=2^16, L=24 limbs of 50 bits, K=8, dnum=3, scale 2^40, "
-                               "two fresh ciphertexts of 32768 uniform[-1,1] slots (BASELINE.json configs[2]); "
+                               "two fresh ciphertexts of 32768 uniform[-1,1] slots; "
                                "independent operations, the best of %d streams of single calls, batches of %d per "
                                "call on one stream, and such batches dealt to %d streams"
                                % (args.lanes, B, len(batch_lanes)),

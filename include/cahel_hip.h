@@ -290,7 +290,8 @@ int he_keyswitch_rescale(const he_context *ctx, uint32_t L, const uint64_t *c, c
 
 /* out [2][L-1][N] = rescale(relinearize(ct1 * ct2)) for two size-2 ciphertexts ct1, ct2 [2][L][N] (ct2 == ct1
  * squares): he_tensor, he_keyswitch and he_rescale with the same limbs in one call; the tensor product is formed by the
- * first pass of the key switch's inverse transform (its third polynomial is not read back for it).  workspace: he_multiply_relin_rescale_workspace_words words.
+ * first pass of the key switch's inverse transform (its third polynomial is not read back for it).
+ * workspace: he_multiply_relin_rescale_workspace_words words.
  * Replaces the sequence multiply (src/evaluate.cu:447-501: tensor_prod_2x2_rns_poly), relinearize_inplace
  * (src/eval_key_switch.cu:80-216) and rescale_to_next (src/evaluate.cu:2058-2085). */
 size_t he_multiply_relin_rescale_workspace_words(const he_context *ctx, uint32_t L);

@@ -388,7 +388,7 @@ hipError_t launch_decrypt_blocks(const NttArgs &a, const DecryptArgs &d, uint32_
 hipError_t launch_decompose_real(const Tables &t, const double *coeffs, uint64_t *out, uint32_t limbs, uint32_t first,
                                  uint32_t items, size_t out_item_stride, hipStream_t s);
 
-// samplers (ChaCha20 block function keyed by key[8]; distributions as in the CPU checker)
+// samplers (ChaCha20 block function keyed by key[8]; distributions as in the CPU oracle)
 enum : int { SAMPLE_TERNARY = 0, SAMPLE_ERROR = 1, SAMPLE_UNIFORM = 2, SAMPLE_GAUSS = 3 };
 struct ChaChaKey {
     uint32_t k[8];

@@ -2,7 +2,7 @@
 //
 // All routines work on residues of primes below 2^61.  "lazy" values live in [0, 2q) or [0, 4q) and
 // never leave a kernel: every store to HBM that a caller can observe is the canonical residue, which
-// is what makes limb-for-limb comparison with the CPU checker meaningful.
+// is what makes limb-for-limb comparison with the CPU oracle meaningful.
 //
 // Semantics follow cahel-main/include/uintmodmath.cuh (Shoup :226-245, Barrett :112-218) and
 // cahel-main/src/ntt/butterfly.cuh:10-43 (Harvey butterflies); the code is written for the CDNA4

@@ -1,6 +1,6 @@
 // Batched negacyclic NTT / inverse NTT over RNS limbs for gfx950.
 //
-// Mathematics (what the CPU checker and the reference compute; cahel-main/src/ntt/fntt_2d.cu:8-246,
+// Mathematics (what the CPU oracle and the reference compute; cahel-main/src/ntt/fntt_2d.cu:8-246,
 // src/ntt/intt_2d.cu:8-198, src/ntt/butterfly.cuh): forward = log2(N) Cooley-Tukey stages m = 1, 2, ..., N/2
 // with twiddle psi^bitrev(m+k) for group k, output in bit-reversed order, canonical residues; inverse =
 // the Gentleman-Sande stages in the opposite order including the factor 1/N.

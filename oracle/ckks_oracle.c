@@ -1,7 +1,7 @@
 /*
  * CPU restatement of the CKKS integer hot path of CAHEL (reference tree: cahel-main/).
  *
- * TEST INFRASTRUCTURE ONLY.  This file is the checker the GPU library is compared against; it is
+ * TEST INFRASTRUCTURE ONLY.  This file is the oracle the GPU library is compared against; it is
  * loaded by tests/, by the smoke check and by the benchmark's cpu_baseline leg.  The product never
  * links, imports or calls it.
  *

@@ -1,4 +1,4 @@
-"""CPU checker for the CKKS hot path of CAHEL (reference tree: cahel-main/).
+"""CPU oracle for the CKKS hot path of CAHEL (reference tree: cahel-main/).
 
 TEST INFRASTRUCTURE ONLY: imported by tests/, by the smoke check and by the benchmark's
 cpu_baseline leg.  The product (lancelot_amd/) never imports it.

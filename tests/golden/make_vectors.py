@@ -1,7 +1,7 @@
 """Writes tests/golden/ckks_n512.npz: inputs and expected outputs of every stage of the hot path on one small
-parameter set (N = 512, four data primes of 40-50 bits, two special primes), computed with the CPU checker in
-oracle/.  The checker itself is pinned by the reference's known-answer tests and by closed forms
-(tests/test_oracle_*.py); these vectors freeze its answers so that neither the checker nor the HIP path can drift
+parameter set (N = 512, four data primes of 40-50 bits, two special primes), computed with the CPU oracle in
+oracle/.  The oracle itself is pinned by the reference's known-answer tests and by closed forms
+(tests/test_oracle_*.py); these vectors freeze its answers so that neither the oracle nor the HIP path can drift
 unnoticed.  Run from the repository root:  python tests/golden/make_vectors.py
 """
 import os

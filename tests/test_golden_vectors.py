@@ -1,5 +1,5 @@
-"""The committed vectors of tests/golden/ckks_n512.npz (written by tests/golden/make_vectors.py with the CPU checker):
-the checker must still reproduce them (CPU), and the HIP path must reproduce them through the C-ABI (GPU)."""
+"""The committed vectors of tests/golden/ckks_n512.npz (written by tests/golden/make_vectors.py with the CPU oracle):
+the oracle must still reproduce them (CPU), and the HIP path must reproduce them through the C-ABI (GPU)."""
 import os
 
 import numpy as np

@@ -1,6 +1,6 @@
 """AddressSanitizer + UndefinedBehaviorSanitizer over the code that runs on the CPU (no GPU needed):
 
-* oracle/ckks_oracle.c: a sanitizer build of the checker is loaded by a child interpreter (sanitizer runtime
+* oracle/ckks_oracle.c: a sanitizer build of the oracle is loaded by a child interpreter (sanitizer runtime
   preloaded) that runs the oracle's own pinning tests against it;
 * the host layer's number theory, table construction, record parsing and encodings in flight (hostmath.cpp, context.cpp,
   serialize.cpp, encoder.cpp):
@@ -34,7 +34,7 @@ def test_oracle_under_asan_ubsan(tmp_path):
     env["CKKS_ORACLE_LIB"] = os.path.join(ROOT, "oracle", "libckks_oracle_san.so")
     # the runtime has to come first among the preloaded libraries; whatever is preloaded already stays
     env["LD_PRELOAD"] = ":".join([asan] + [p for p in env.get("LD_PRELOAD", "").split(":") if p])
-    # the interpreter itself is not instrumented: its allocations at exit are not leaks of the checker
+    # the interpreter itself is not instrumented: its allocations at exit are not leaks of the oracle
     env["ASAN_OPTIONS"] = "detect_leaks=0:abort_on_error=1"
     env["UBSAN_OPTIONS"] = "print_stacktrace=1:halt_on_error=1"
     env["OMP_NUM_THREADS"] = "2"
