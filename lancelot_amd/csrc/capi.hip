@@ -96,8 +96,7 @@ struct he_context {
     bool fuse_tensor = true;     // environment CAHEL_HIP_NO_FUSED_TENSOR=1: he_multiply_relin_rescale as tensor kernel + key switch
     bool single_limb_digits = false;  // K = 1 (environment CAHEL_HIP_NO_REDUCE_IN_NTT=1: keep the conversion kernels)
     bool batch_fused_inner = true;  // environment CAHEL_HIP_NO_BATCH_FUSED_KS=1: a batch's inner product as a kernel of its own
-    uint32_t *d_rot_group = nullptr;     // encoder: 5^j mod 2N
-    double2 *d_ksi = nullptr;            // encoder: e^{2 pi i k / 2N}, k <= 2N
+    double2 *d_fft_forward = nullptr, *d_fft_inverse = nullptr;   // encoder: see FftTables
     uint64_t *d_garner_inv = nullptr;    // decoder: [size_q][size_q], q_j^-1 mod q_i for j < i
     std::vector<uint64_t> h_moduli;
     std::vector<uint8_t> fp_ok;  // per table: prime below 2^50
@@ -113,6 +112,7 @@ struct he_context {
 
     int32_t *d_mx_down = nullptr, *d_mx_last = nullptr;   // the P -> Ql matrix (times P^-1) for the int8 matrix cores
     Tables tables() const { return Tables{d_moduli, d_barrett, log_n}; }
+    FftTables fft() const { return FftTables{d_fft_forward, d_fft_inverse, log_n}; }
     size_t n() const { return (size_t)1 << log_n; }
 };
 
@@ -447,19 +447,24 @@ int he_context_create(const he_context_desc *d, he_context **out) {
         if (!rc) rc = upload(ctx, &ctx->d_phat_mod_q, d->phat_mod_q, (size_t)d->size_q * d->size_p);
     }
     if (!rc) {
-        // encoder tables (cahel-main/src/ckks.cu:34-102): rotation group and the 2N-th roots of unity
+        // encoder tables (cahel-main/src/ckks.cu:34-102): the 2N-th roots of unity, and from them every stage's twiddles in
+        // the order of the rotation group 5^j
         const size_t m = 2 * n;
-        std::vector<uint32_t> rot(n / 2);
-        uint32_t pos = 1;
-        for (size_t i = 0; i < n / 2; i++) {
-            rot[i] = pos;
-            pos = (uint32_t)(((uint64_t)pos * 5) & (m - 1));
-        }
         std::vector<double2> ksi(m + 1);
         const double pi = 3.14159265358979323846264338327950288;
         for (size_t k = 0; k <= m; k++) {
             const double angle = 2.0 * pi * (double)k / (double)m;
             ksi[k] = double2{std::cos(angle), std::sin(angle)};
+        }
+        std::vector<double2> fft_forward(n / 2), fft_inverse(n / 2);
+        for (size_t half = 1; half < n / 2; half <<= 1) {
+            const size_t lenq = 8 * half, gap = m / lenq;
+            size_t r = 1;
+            for (size_t j = 0; j < half; j++) {
+                fft_forward[half + j] = ksi[r * gap];
+                fft_inverse[half + j] = ksi[(lenq - r) * gap];
+                r = 5 * r & (lenq - 1);
+            }
         }
         // Garner constants of the data primes
         const size_t sq = d->size_q;
@@ -474,8 +479,8 @@ int he_context_create(const he_context_desc *d, he_context **out) {
                 }
                 ginv[i * sq + j] = (uint64_t)acc;
             }
-        rc = upload(ctx, &ctx->d_rot_group, rot.data(), rot.size());
-        if (!rc) rc = upload(ctx, &ctx->d_ksi, ksi.data(), ksi.size());
+        rc = upload(ctx, &ctx->d_fft_forward, fft_forward.data(), fft_forward.size());
+        if (!rc) rc = upload(ctx, &ctx->d_fft_inverse, fft_inverse.data(), fft_inverse.size());
         if (!rc) rc = upload(ctx, &ctx->d_garner_inv, ginv.data(), ginv.size());
     }
     if (!rc) {
@@ -1486,7 +1491,7 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     const size_t n = ctx->n();
     const size_t head = ((size_t)items + 7) & ~(size_t)7;
     double2 *v = reinterpret_cast<double2 *>(ws + head);
-    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    const FftTables ft = ctx->fft();
     // (the complex scratch of an item is `slots` values = at most N words: the items are packed `slots` apart)
     // (the rounding kernel writes the residues itself: the coefficients never exist as an array of doubles)
     HE_HIP(launch_ckks_encode(ft, ctx->tables(), re, im, count, slots, scale, v, ws, items, value_stride, out, limbs,
@@ -1504,7 +1509,7 @@ int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double
         (items > 1 && value_stride < count))
         return HE_E_INVALID_ARGUMENT;
     double2 *v = reinterpret_cast<double2 *>(ws + (((size_t)items + 7) & ~(size_t)7));
-    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    const FftTables ft = ctx->fft();
     HE_HIP(launch_ckks_fft_inverse(ft, re, im, count, slots, v, items, value_stride, S(s)));
     // rounding and residues happen where the transform reads its input
     NttArgs a = base_args(ctx, true);
@@ -1569,7 +1574,7 @@ int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
 int decode_real_impl(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t items, uint32_t slots, double scale,
                      uint64_t *coeff, double2 *v, double *out, uint32_t count, he_stream s) {
-    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    const FftTables ft = ctx->fft();
     NttArgs inv = base_args(ctx, false);
     inv.in = plain;
     inv.out = coeff;
@@ -1674,7 +1679,7 @@ int he_ckks_decode(const he_context *ctx, const uint64_t *plain, uint32_t limbs,
     inv.in_poly_stride = inv.out_poly_stride = limbs;
     inv.map = plain_map(limbs);
     HE_HIP(launch_ntt_inverse(inv, 1, backend_for(ctx, inv.map), S(s)));
-    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    const FftTables ft = ctx->fft();
     HE_HIP(launch_ckks_decode(ft, ctx->tables(), ws, limbs, slots, scale, ctx->d_garner_inv, ctx->size_q,
                               reinterpret_cast<double2 *>(out), 1, S(s)));
     return HE_OK;
@@ -1698,7 +1703,7 @@ int he_decrypt_decode_batch(const he_context *ctx, const uint64_t *const *d_cts,
     double2 *v = reinterpret_cast<double2 *>(ws + (size_t)items * limbs * n);
     HE_HIP(launch_decrypt_gather(ctx->tables(), d_cts, sk, noise, plain, limbs, items, S(s)));
     if (int rc = he_ntt_inverse(ctx, plain, items, limbs, limbs, 0, limbs, 0, s)) return rc;
-    const FftTables ft{ctx->d_rot_group, ctx->d_ksi, ctx->log_n};
+    const FftTables ft = ctx->fft();
     HE_HIP(launch_ckks_decode(ft, ctx->tables(), plain, limbs, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, S(s)));
     HE_HIP(launch_take_slots(v, slots, items, count, reinterpret_cast<double2 *>(out), S(s)));
     return HE_OK;

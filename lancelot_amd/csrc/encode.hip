@@ -21,12 +21,12 @@ __device__ __forceinline__ double2 cmul(double2 a, double2 w) {
     return double2{a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x};
 }
 
-// twiddle of butterfly j in a stage of span len: e^{+-2 pi i (5^j mod 4 len) / (4 len)}
+// twiddle of butterfly j < len / 2 in a stage of span len: e^{+-2 pi i (5^j mod 4 len) / (4 len)}; a stage's twiddles lie one
+// after the other (looked up as root[group[j]], two dependent loads of which the second gathers, the two passes of one
+// encoding of 32,768 values took 3 us longer)
 template <bool INVERSE>
 __device__ __forceinline__ double2 stage_twiddle(const FftTables &t, uint32_t len, uint32_t j) {
-    const uint32_t lenq = len << 2, gap = (2u << t.log_n) / lenq;
-    const uint32_t r = t.rot_group[j] & (lenq - 1);
-    return t.ksi[(INVERSE ? lenq - r : r) * gap];
+    return (INVERSE ? t.inverse : t.forward)[(len >> 1) + j];
 }
 
 // INVERSE (encode): decimation in frequency,  (a, b) -> (a + b, (a - b) w)
@@ -102,13 +102,14 @@ __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t
     }
 }
 
-// A transform of 2^s >= 256 values as two passes, like the number-theoretic one: the vector is 2^(s - 8) rows x 256 columns;
-// the rows pass holds the stages of span above 256 (a workgroup owns all rows of a few columns), the blocks pass the 8 stages
-// inside 256 consecutive values (a wave owns one block).  A thread holds 4 values in register blocks of two stages (Tile4's
-// layout); its 12 twiddles, each a look-up behind a look-up, are fetched together with the values.  Every butterfly has the
-// operands and the twiddle that a launch per stage would give it, so the results do not depend on the split.  (One
-// workgroup per 2048 values and one thread per 16 wide ones, which this replaced, left most of the chip idle: 12.4 + 10.1 us
-// on the way in, 7.2 + 4.1 us on the way out at 32,768 slots.)
+// A transform of 2^s >= 256 values as two passes, like the number-theoretic one: the vector is 2^(s - 10) rows x 1024 columns (x 256
+// below 1024 values); the rows pass holds the stages whose span is more than a row (a workgroup owns all rows of a few columns),
+// the blocks pass the 10 (8) stages inside one row.  A thread holds 4 values in register blocks of two stages (Tile4's
+// layout) and fetches its twiddles together with the values.  Every butterfly has the operands and the twiddle that a launch per
+// stage would give it, so the results do not depend on the split.
+// Why rows of 1024: the rows pass reads an encoding's values from, and writes a decoding's to, page-locked host memory, in segments as long
+// as a tile is wide.  A tile of 1024 values has 32 columns at 32,768 values, 256 bytes a segment; with rows of 256 columns it
+// had 8, and 256 KB read in segments of 64 bytes take 15.0 us over PCIe (128 bytes 8.7, 256 bytes and more 7.0; written 7.1, 6.3, 6.0).
 // Stage sigma of the inverse direction (the forward runs them backwards) pairs index bit s - 1 - sigma; a value's twiddle
 // is chosen by the bits below it.
 template <bool INVERSE, int B, int LD>
@@ -185,8 +186,8 @@ struct FftTile {
     }
 };
 
-// blockIdx.x = tile of 2^(B - LD) columns, blockIdx.y = item
-template <bool INVERSE, int B, int LD>
+// blockIdx.x = tile of 2^(B - LD) columns, blockIdx.y = item; LR = log2(columns of the vector)
+template <bool INVERSE, int B, int LD, int LR>
 __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, FftTables t, uint32_t log_slots, FftSource src,
                                                                  FftTarget dst) {
     using F = FftTile<INVERSE, B, LD>;
@@ -197,7 +198,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, Fft
     v += (size_t)item << log_slots;
     auto pos = [&](int k, int j) {
         const uint32_t e = T4::word(k, tid, j);
-        return ((e >> LOGC) << 8) + col0 + (e & ((1u << LOGC) - 1));
+        return ((e >> LOGC) << LR) + col0 + (e & ((1u << LOGC) - 1));
     };
     double2 x[4];
     typename F::Tw tw[NB];
@@ -230,41 +231,44 @@ __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, Fft
     }
 }
 
-constexpr int kFftWaves = 2;   // 256-value blocks of a workgroup
+// Blocks of 2^B values: a wave of a workgroup of two (B = 8), or a workgroup (B = 10).  blockIdx.y = item
+template <int B>
+constexpr uint32_t kFftBlocks = B == 8 ? 2 : 1;   // of a workgroup
 
-// blockIdx.y = item
-template <bool INVERSE>
-__global__ __launch_bounds__(64 * kFftWaves) void cfft_blocks_kernel(double2 *v, FftTables t, uint32_t log_slots, FftSource src,
-                                                                     FftTarget dst) {
-    using F = FftTile<INVERSE, 8, 8>;
+template <bool INVERSE, int B>
+__global__ __launch_bounds__((1 << (B - 2)) * kFftBlocks<B>) void cfft_blocks_kernel(double2 *v, FftTables t, uint32_t log_slots,
+                                                                                    FftSource src, FftTarget dst) {
+    using F = FftTile<INVERSE, B, B>;
     using T4 = typename F::T4;
-    const uint32_t w = threadIdx.x >> 6, lane = threadIdx.x & 63, item = blockIdx.y;
-    const uint32_t blk = blockIdx.x * kFftWaves + w;
-    if (blk >= 1u << (log_slots - 8)) return;   // (256 slots: one block)
-    v += ((size_t)item << log_slots) + (size_t)blk * 256;
-    auto pos = [&](int k, int j) { return T4::word(k, lane, j); };   // (the twiddles depend on the position inside the block)
+    constexpr int LAST = T4::kBlocks - 1, WORDS = T4::in_wave(0) ? 1 : (1 << B) + (1 << (B - 4));
+    __shared__ double re[WORDS], im[WORDS];
+    const uint32_t w = threadIdx.x >> (B - 2), tid = threadIdx.x & ((1u << (B - 2)) - 1), item = blockIdx.y;
+    const uint32_t blk = blockIdx.x * kFftBlocks<B> + w;
+    if (kFftBlocks<B> > 1 && blk >= 1u << (log_slots - B)) return;   // (256 slots: one block)
+    v += ((size_t)item << log_slots) + ((size_t)blk << B);
+    auto pos = [&](int k, int j) { return T4::word(k, tid, j); };   // (the twiddles depend on the position inside the block)
     double2 x[4];
-    typename F::Tw tw[4];
+    typename F::Tw tw[LAST + 1];
     if (INVERSE) {
         if (src.re) {
             // (only when the whole vector is this one block: otherwise the rows pass has run before)
-            if (src.max_bits && lane == 0) src.max_bits[item] = 0;
+            if (src.max_bits && tid == 0) src.max_bits[item] = 0;
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = source_value(src, item, pos(0, j));
         } else {
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
         }
-        F::load_tw(tw, t, log_slots, log_slots - 8, pos);
-        F::down(x, tw, nullptr, nullptr, lane);   // (every exchange stays inside the wave)
+        F::load_tw(tw, t, log_slots, log_slots - B, pos);
+        F::down(x, tw, re, im, tid);
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[pos(3, j)] = x[j];
+        for (int j = 0; j < 4; j++) v[pos(LAST, j)] = x[j];
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = v[pos(3, j)];
-        F::load_tw(tw, t, log_slots, log_slots - 8, pos);
-        F::up(x, tw, nullptr, nullptr, lane);
-        if (dst.re && log_slots == 8) {
+        for (int j = 0; j < 4; j++) x[j] = v[pos(LAST, j)];
+        F::load_tw(tw, t, log_slots, log_slots - B, pos);
+        F::up(x, tw, re, im, tid);
+        if (dst.re && log_slots == B) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
                 if (pos(0, j) < dst.count) dst.re[item * dst.value_stride + pos(0, j)] = x[j].x;
@@ -503,22 +507,35 @@ hipError_t run_fft(double2 *v, uint32_t slots, uint32_t items, const FftTables &
         hipLaunchKernelGGL(cfft_lds_kernel<INVERSE>, dim3(1, items), dim3(kThreads), 0, s, v, slots, t, slots, src, dst);
         return hipGetLastError();
     }
-    const uint32_t ld = log_slots - 8;
+    const uint32_t lr = log_slots >= 10 ? 10 : 8, ld = log_slots - lr;
     const FftSource none{nullptr, nullptr, 0, 0, nullptr};
     auto rows = [&]() {
-        // tiles of 1024 values (8 columns at 32,768 slots)
-#define HE_CASE(LD, B) \
-    case LD: hipLaunchKernelGGL((cfft_rows_kernel<INVERSE, B, LD>), dim3(256u >> (B - LD), items), dim3(1u << (B - 2)), 0, s, v, t, log_slots, src, dst); break;
-        switch (ld) {
-            HE_CASE(1, 8) HE_CASE(2, 10) HE_CASE(3, 10) HE_CASE(4, 10) HE_CASE(5, 10) HE_CASE(6, 10) HE_CASE(7, 10) HE_CASE(8, 10)
-            default: return hipErrorInvalidValue;
+        // tiles of 1024 values (256 of the 512)
+#define HE_CASE(LD, B, LR)                                                                                                              \
+    case LD:                                                                                                                            \
+        hipLaunchKernelGGL((cfft_rows_kernel<INVERSE, B, LD, LR>), dim3((1u << LR) >> (B - LD), items), dim3(1u << (B - 2)), 0, s, v, t, \
+                           log_slots, src, dst);                                                                                        \
+        break;
+        if (lr == 8) {
+            switch (ld) {
+                HE_CASE(1, 8, 8)
+                default: return hipErrorInvalidValue;
+            }
+        } else {
+            switch (ld) {
+                HE_CASE(1, 10, 10) HE_CASE(2, 10, 10) HE_CASE(3, 10, 10) HE_CASE(4, 10, 10) HE_CASE(5, 10, 10) HE_CASE(6, 10, 10)
+                default: return hipErrorInvalidValue;
+            }
         }
 #undef HE_CASE
         return hipGetLastError();
     };
     auto blocks = [&]() {
-        hipLaunchKernelGGL(cfft_blocks_kernel<INVERSE>, dim3(((1u << ld) + kFftWaves - 1) / kFftWaves, items), dim3(64 * kFftWaves), 0, s, v, t,
-                           log_slots, ld ? none : src, dst);
+        if (lr == 8)
+            hipLaunchKernelGGL((cfft_blocks_kernel<INVERSE, 8>), dim3(1, items), dim3(64 * kFftBlocks<8>), 0, s, v, t, log_slots,
+                               ld ? none : src, dst);
+        else
+            hipLaunchKernelGGL((cfft_blocks_kernel<INVERSE, 10>), dim3(1u << ld, items), dim3(256), 0, s, v, t, log_slots, ld ? none : src, dst);
         return hipGetLastError();
     };
     if (INVERSE && ld)

@@ -404,10 +404,10 @@ hipError_t launch_sample_encrypt(uint32_t log_n, ChaChaKey key, uint64_t stream_
 hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, const uint64_t *cdt,
                                      uint32_t cdt_len, uint32_t items, hipStream_t s);
 
-// CKKS encoder tables: 5^j mod 2N for j < N/2 and e^{2 pi i k / 2N} for k <= 2N.
+// CKKS encoder twiddles: entry len / 2 + j (2 <= len <= N/2, j < len / 2) is e^{2 pi i r / (4 len)}, r = 5^j mod 4 len, of the decoding's
+// stage of span len, and e^{2 pi i (4 len - r) / (4 len)} of the encoding's.
 struct FftTables {
-    const uint32_t *rot_group;
-    const double2 *ksi;
+    const double2 *forward, *inverse;
     uint32_t log_n;
 };
 // values (count <= slots, zero padded) -> rounded coefficients as residues of the first `limbs` primes of `tab` (out

@@ -80,6 +80,33 @@ def test_encrypt_and_decrypt(oracle, capi, chain, logn, size_p, L):
     assert lib.he_decrypt_flood(h, dct3.ptr, 2, L, dsk.ptr, L * n, kp, 5, dcdt.ptr, 128, out.ptr, noise.ptr, None) != 0
 
 
+@pytest.mark.parametrize("slots", [128, 256, 512, 1024, 2048])
+def test_slot_transform_at_the_edges_of_its_rows(oracle, capi, slots):
+    """Encoding and decoding where the special FFT changes its shape: inside LDS, one block of 256, two of them, one block of
+    1024, two of them.  Coefficients within one unit of the oracle's (the rounding of a sum that falls on the middle), values
+    within 2^-20: 12 stages in double precision and a rounding to 2^-41 per coefficient stay far below."""
+    cahel, parms, ctx, p = make_pair(oracle, 12, CHAINS["mixed"], 1)
+    lib, h = capi.lib(), ctx.he_handle()
+    rng = np.random.default_rng(slots)
+    limbs, n, count, scale = 2, p.n, slots - 3, 2.0 ** 40
+    z = rng.uniform(-1, 1, count) + 1j * rng.uniform(-1, 1, count)
+    o_enc = oracle.Encoder(p)
+    re, im = DeviceArray(capi, host=np.ascontiguousarray(z.real)), DeviceArray(capi, host=np.ascontiguousarray(z.imag))
+    ws, out = DeviceArray(capi, shape=(lib.he_ckks_workspace_words(h, limbs),)), DeviceArray(capi, shape=(limbs, n))
+    capi.check(lib.he_ckks_encode(h, re.ptr, im.ptr, count, slots, scale, limbs, out.ptr, ws.ptr, None))
+    got = out.numpy()
+    got_coeff, want_coeff = p.ntt_inv(got.copy()), p.ntt_inv(o_enc.encode(z, scale, limbs, slots))
+    for i in range(limbs):
+        q = p.moduli[i]
+        d = (got_coeff[i].astype(np.int64) - want_coeff[i].astype(np.int64)) % q
+        assert np.minimum(d, q - d).max() <= 1, i
+    dec = DeviceArray(capi, shape=(slots, 2), dtype=np.float64)
+    capi.check(lib.he_ckks_decode(h, out.ptr, limbs, slots, scale, dec.ptr, ws.ptr, None))
+    values = dec.numpy() @ np.array([1, 1j])
+    assert np.abs(values - o_enc.decode(got, scale, slots)).max() < 2.0 ** -20
+    assert np.abs(values[:count] - z).max() < 2.0 ** -20 and np.abs(values[count:]).max() < 2.0 ** -20
+
+
 @pytest.mark.parametrize("chain", sorted(CHAINS))
 @pytest.mark.parametrize("logn,slots,limbs", [(12, 2, 1), (12, 2048, 5), (13, 128, 2), (13, 4096, 3), (14, 512, 4), (15, 16384, 2),
                                               (16, 32768, 4), (17, 65536, 2)])
