@@ -134,28 +134,125 @@ __global__ __launch_bounds__((1 << LOGN) / 16) void ntt_limb_fp_kernel(NttArgs a
     }
 }
 
+// The same for N = 2^10 and 2^12 with 4 words a thread (N / 4 threads), on every back end.  What bounds a transform of this size is the
+// chain of one workgroup: with 16 words a thread N / 1024 waves a SIMD go through blocks of four stages, each behind a fetch of its 15
+// twiddles and a trip of all its words through LDS; here all twiddles are requested together with the words, and only the
+// exchanges of more than 256 words (two at 2^12) go through LDS, the others stay in a wave's registers (Tile4).
+// Six limbs of 50 bits, forward and inverse: 2^10 4.35 -> 3.76 and 4.76 -> 3.90 us, 2^12 5.36 -> 5.11 and 5.85 -> 5.36; of 60 bits
+// at 2^10, against rows pass and blocks pass, 6.6 -> 3.8 us.
+template <int LOGN, bool FWD, int BE>
+__global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(NttArgs a) {
+    using T4 = Tile4<LOGN, LOGN>;
+    constexpr int NB = T4::kBlocks;
+    __shared__ uint64_t lds[(1 << LOGN) + (1 << (LOGN - 4))];
+    touch_arguments<sizeof(NttArgs)>();
+    const Job job = decode_job(a, blockIdx.x);
+    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    uint64_t x[4];
+    // (the forward direction starts from the layout of block 0, words N / 4 apart, and ends with four neighbouring words a thread; the
+    // inverse the other way round)
+    if (FWD) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = job.in[T4::word(0, t, j)];
+    } else {
+        load4(x, job.in + 4 * t);
+    }
+    if (BE != NTT_BACKEND_INT && fp) {
+        const FpArith ar = fp_arith(a, job.table);
+        FpArith::Tw tw[NB];
+        T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = fp_from_u64(x[j]);
+        if (FWD) {
+            T4::template forward<FpArith>(v, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(v[j], ar.m));
+        } else {
+            const FpTw scale = inverse_scale(a, job, ar.m);
+            T4::template inverse<FpArith>(v, tw, ar, lds, t);
+#pragma unroll
+            for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, ar.m), ar.m));
+        }
+    }
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) {
+            const IntArith ar = int_arith(a, job.table);
+            const uint64_t q = scalar(a.moduli)[job.table];
+            IntArith::Tw tw[NB];
+            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+            if (FWD) {
+                T4::template forward<IntArith>(x, tw, ar, lds, t);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[j] = reduce_4q(x[j], q);
+            } else {
+                Shoup w{0, 0};
+                if (a.epi_mode == NTT_EPI_MUL) w = scalar_shoup(a.w, job.limb);
+                T4::template inverse<IntArith>(x, tw, ar, lds, t);
+#pragma unroll
+                for (int j = 0; j < 4; j++) x[j] = a.epi_mode == NTT_EPI_MUL ? mul_shoup(x[j], w, q) : reduce_2q(x[j], q);
+            }
+        }
+    }
+    if (FWD) {
+        store4(job.out + 4 * t, x);
+    } else {
+#pragma unroll
+        for (int j = 0; j < 4; j++) job.out[T4::word(0, t, j)] = x[j];
+    }
+}
+
+// 4 words a thread or 16 (FP64) at 2^12: 16 waves a limb shorten its chain, 4 issue fewer instructions, which counts once every CU has
+// a limb of its own (6 limbs 5.11 against 5.36 us, 96 5.74 against 5.93, 960 16.6 against 14.8).
+inline bool limb4(const NttArgs &a, int backend, uint32_t n_jobs) {
+    return a.log_n == 10 || (a.log_n == 12 && (backend != NTT_BACKEND_FP || n_jobs <= 256));
+}
+
 template <bool FWD>
-hipError_t launch_limb_fp(const NttArgs &a, uint32_t n_jobs, hipStream_t s) {
+hipError_t launch_limb(const NttArgs &a, uint32_t n_jobs, int backend, hipStream_t s) {
+    if (n_jobs > most_workgroups((1u << a.log_n) / 4)) return hipErrorInvalidValue;
+    if (limb4(a, backend, n_jobs)) {
+#define HE_LIMB4(LOGN)                                                                                                                  \
+    do {                                                                                                                                \
+        const dim3 block((1u << LOGN) / 4);                                                                                             \
+        if (backend == NTT_BACKEND_MIXED)                                                                                               \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_MIXED>), dim3(n_jobs), block, 0, s, a);                         \
+        else if (backend)                                                                                                               \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_FP>), dim3(n_jobs), block, 0, s, a);                            \
+        else                                                                                                                            \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_INT>), dim3(n_jobs), block, 0, s, a);                           \
+    } while (0)
+        if (a.log_n == 10)
+            HE_LIMB4(10);
+        else
+            HE_LIMB4(12);
+#undef HE_LIMB4
+        return hipGetLastError();
+    }
     switch (a.log_n) {
 #define HE_CASE(LOGN) \
     case LOGN: hipLaunchKernelGGL((ntt_limb_fp_kernel<LOGN, FWD>), dim3(n_jobs), dim3((1u << LOGN) / 16), 0, s, a); break;
-        HE_CASE(9) HE_CASE(10) HE_CASE(11) HE_CASE(12) HE_CASE(13) HE_CASE(14)
+        HE_CASE(9) HE_CASE(11) HE_CASE(12) HE_CASE(13) HE_CASE(14)
 #undef HE_CASE
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
 }
 
-// The launches that the whole-limb kernel covers and wins.  A limb is one workgroup on one CU: up to N = 2^12 that is
-// faster than two launches whatever the number of limbs (5.5 against 8.5 us); a limb of 2^13 or 2^14 words takes one CU
+// The launches that a whole-limb kernel covers and wins.  A limb is one workgroup on one CU: up to N = 2^12 that is
+// faster on FP64 than two launches whatever the number of limbs; a limb of 2^13 or 2^14 words takes one CU
 // longer than two launches of a few limbs take, so there the kernel pays only when the launch has enough limbs to occupy
 // the chip: from 64 limbs on at 2^13 (192 limbs 10.7 against 13.8 us, 576 limbs 25.6 against 33.3 us), from 192 on in the
 // forward direction at 2^14 (19.4 against 25.1 us, 576 limbs 55.7 against 59.9 us; its inverse, whose first blocks wait for the whole
-// limb, takes 28.4 against 25.4 us and 82 against 56 us).  a.one_pass = 2 forces it (tests).
+// limb, takes 28.4 against 25.4 us and 82 against 56 us).  Integers take 2.5 times the instructions: one launch at 2^10
+// always, at 2^12 once there is a limb for every CU (6 limbs 7.2 against 6.8 us, inverse 7.9 against 6.9; 96 limbs 7.6 against 8.4 and 8.3 against
+// 8.2; 960 limbs 24.2 against 30.7 and 26.8 against 33.2).  a.one_pass = 2 forces it (tests).
 inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_jobs) {
-    if (!a.one_pass || backend != NTT_BACKEND_FP || a.log_n > 14 || a.jobs || a.pro_mode != NTT_PLAIN || a.in_galois ||
+    if (!a.one_pass || a.log_n > 14 || a.jobs || a.pro_mode != NTT_PLAIN || a.in_galois ||
         !(a.epi_mode == NTT_PLAIN || (!forward && a.epi_mode == NTT_EPI_MUL)))
         return false;
+    if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || n_jobs >= 256));
     return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && n_jobs >= 64) || (a.log_n == 14 && forward && n_jobs >= 192);
 }
 
@@ -529,7 +626,7 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
     if (a.log_n < 9 || a.log_n > 17 || backend < NTT_BACKEND_INT || backend > NTT_BACKEND_MIXED) return hipErrorInvalidValue;
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
-    if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb_fp<true>(a, n_jobs, s);
+    if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb<true>(a, n_jobs, backend, s);
     const hipError_t e = rows_done ? hipSuccess : launch_ntt_rows(a, n_jobs, true, backend, s);
     return e != hipSuccess ? e : launch_ntt_blocks(a, n_polys, true, backend, s);
 }
@@ -539,7 +636,7 @@ hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, h
     if (a.log_n < 9 || a.log_n > 17 || backend < NTT_BACKEND_INT || backend > NTT_BACKEND_MIXED) return hipErrorInvalidValue;
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
-    if (!blocks_done && !rows_skipped && one_pass_ok(a, backend, false, n_jobs)) return launch_limb_fp<false>(a, n_jobs, s);
+    if (!blocks_done && !rows_skipped && one_pass_ok(a, backend, false, n_jobs)) return launch_limb<false>(a, n_jobs, backend, s);
     const hipError_t e = blocks_done ? hipSuccess : launch_ntt_blocks(a, n_polys, false, backend, s);
     if (e != hipSuccess || rows_skipped) return e;
     NttArgs rows = a;

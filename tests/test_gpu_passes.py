@@ -37,6 +37,27 @@ def test_batched_transforms(oracle, capi, chain, logn, limbs, polys):
 
 
 @pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,limbs,polys", [(10, 1, 1), (10, 5, 3), (12, 1, 1), (12, 5, 51), (12, 5, 52)])
+@pytest.mark.parametrize("one_pass", ["default", "forced"])
+def test_whole_limb_transforms(oracle, capi, monkeypatch, chain, logn, limbs, polys, one_pass):
+    """A limb of 2^10 or 2^12 words in one workgroup, on both sides of the number of limbs (255 and 260) at which the kernel
+    changes."""
+    monkeypatch.setenv("CAHEL_HIP_FORCE_ONE_PASS", "1" if one_pass == "forced" else "0")
+    cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], 1)
+    lib, h = capi.lib(), ctx.he_handle()
+    x = rand_limbs(p, np.random.default_rng(polys), range(limbs), n_polys=polys)
+    x[0, 0, :4] = [0, 1, p.moduli[0] - 1, p.moduli[0] - 2]
+    x[polys - 1, limbs - 1, :] = p.moduli[limbs - 1] - 1
+    d = DeviceArray(capi, host=x)
+    capi.check(lib.he_ntt_forward(h, d.ptr, polys, limbs, limbs, 0, limbs, 0, None))
+    got = d.numpy()
+    for k in sorted({0, polys // 2, polys - 1}):
+        assert (got[k] == p.ntt_fwd(x[k].copy())).all(), k
+    capi.check(lib.he_ntt_inverse(h, d.ptr, polys, limbs, limbs, 0, limbs, 0, None))
+    assert (d.numpy() == x).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
 @pytest.mark.parametrize("logn,size_p,L", [(12, 1, 5), (13, 2, 3), (14, 1, 1), (15, 2, 4), (16, 1, 2)])
 def test_encrypt_and_decrypt(oracle, capi, chain, logn, size_p, L):
     """he_encrypt of a plaintext elsewhere, he_encrypt_batch of three in place, he_decrypt_flood of 2 and 3 polynomials."""
