@@ -470,7 +470,7 @@ __global__ __launch_bounds__(256) void decode_rows_compose_kernel(NttArgs a, uin
             const FpArith ar = fp_arith(a, job.table);
             FpArith::Tw tw[NB];
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-            const FpTw scale = inverse_scale(a, job, ar.m);
+            const double scale = inverse_scale(a, job, ar.m);
             double w[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) w[j] = FpArith::from_word(x[j]);

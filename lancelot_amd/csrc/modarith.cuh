@@ -263,19 +263,17 @@ __device__ __forceinline__ uint32_t galois_index(uint32_t i, uint32_t elt, uint3
 // in a double; residues are signed and lazy (|v| < 2^53).  All steps below are exact integer
 // computations, so the canonical result equals the integer path's bit for bit.
 //
-//   x * w = h + l exactly (h = fl(x w), l = fma(x, w, -h)); k = rint(x * winv), winv ~ w/q with
-//   relative error at most 2^-52, differs from x w / q by at most 1/2 + 1.5 |x| 2^-52; h - k q and
-//   (h - k q) + l are integers below 2^53 in magnitude, hence exact; the result is congruent to x w
-//   with |r| <= (1/2 + 1.5 |x| 2^-52) q, i.e. (1/2 + 0.375 b) q for |x| <= b q, q < 2^50.
+//   x * w = h + l exactly (h = fl(x w), l = fma(x, w, -h)); k = rint(fl(h fl(1/q))), three roundings from
+//   x w / q, differs from it by at most 1/2 + 1.5 |x w / q| 2^-52; h - k q and (h - k q) + l are integers
+//   below 2^53 in magnitude, hence exact; the result is congruent to x w with
+//   |r| <= (1/2 + 1.5 |x| 2^-52) q for |w| <= q, i.e. (1/2 + 0.375 b) q for |x| <= b q, q < 2^50.
+//   (With the quotient from a second operand fl(w fl(1/q)) beside w the bound is the same, and a twiddle or a key word
+//   costs one multiplication more.)
 // ---------------------------------------------------------------------------------------------------
 namespace he {
 
 struct FpMod {
     double q, qinv;
-};
-
-struct FpTw {
-    double w, winv;
 };
 
 // canonical residue (< 2^52) <-> exact double, through the exponent-bias trick
@@ -287,10 +285,10 @@ __device__ __forceinline__ uint64_t fp_to_u64(double c) {  // 0 <= c < 2^52, int
     return (uint64_t)__double_as_longlong(c + 4503599627370496.0) & 0x000FFFFFFFFFFFFFull;
 }
 
-__device__ __forceinline__ double fp_mulmod(double x, FpTw t, FpMod m) {
-    const double k = __builtin_rint(x * t.winv);
-    const double h = x * t.w;
-    const double l = __builtin_fma(x, t.w, -h);
+__device__ __forceinline__ double fp_mulmod(double x, double w, FpMod m) {
+    const double h = x * w;
+    const double l = __builtin_fma(x, w, -h);
+    const double k = __builtin_rint(h * m.qinv);
     return __builtin_fma(-k, m.q, h) + l;
 }
 
@@ -304,14 +302,6 @@ __device__ __forceinline__ double fp_reduce(double v, FpMod m) {
 __device__ __forceinline__ double fp_canonical(double v, FpMod m) {
     const double c = fp_reduce(v, m);
     return c < 0.0 ? c + m.q : c;
-}
-
-// Twiddle tables hold w only (8 bytes per entry: the tables are as large as the data they transform, so
-// their size is HBM traffic); the quotient estimate w * fl(1/q) has relative error 2^-52, which with the
-// rounding of x * winv puts k within 1/2 + 1.5 |x| 2^-52 of x w / q.
-__device__ __forceinline__ FpTw load_fptw(const double *table, size_t idx, FpMod m) {
-    const double w = table[idx];
-    return FpTw{w, w * m.qinv};
 }
 
 // Forward block: LOGR consecutive forward stages on 2^LOGR lazy signed doubles.  v[j] are the elements whose index differs in the
@@ -337,7 +327,7 @@ __device__ __forceinline__ void fp_ct_block(double *v, const double *table, uint
         const int half = R >> (l + 1);
 #pragma unroll
         for (int b = 0; b < (1 << l); b++) {
-            const FpTw tw = load_fptw(table, ((size_t)idx << l) + b, m);
+            const double tw = table[((size_t)idx << l) + b];
 #pragma unroll
             for (int j = 0; j < half; j++) {
                 const double x = v[2 * b * half + j];
@@ -364,7 +354,7 @@ __device__ __forceinline__ void fp_gs_block(double *v, const double *table, uint
         const int half = R >> (l + 1);
 #pragma unroll
         for (int b = 0; b < (1 << l); b++) {
-            const FpTw tw = load_fptw(table, ((size_t)idx << l) + b, m);
+            const double tw = table[((size_t)idx << l) + b];
 #pragma unroll
             for (int j = 0; j < half; j++) {
                 const double x = v[2 * b * half + j], y = v[2 * b * half + j + half];

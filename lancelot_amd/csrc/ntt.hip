@@ -128,7 +128,7 @@ __global__ __launch_bounds__((1 << LOGN) / 16) void ntt_limb_fp_kernel(NttArgs a
             }
         }
         // block 0: base = t, low = log2(T): the coalesced store pattern
-        const FpTw scale = inverse_scale(a, job, m);
+        const double scale = inverse_scale(a, job, m);
 #pragma unroll
         for (int j = 0; j < 16; j++) job.out[t + T * j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, m), m));
     }
@@ -170,7 +170,7 @@ __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(NttArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(v[j], ar.m));
         } else {
-            const FpTw scale = inverse_scale(a, job, ar.m);
+            const double scale = inverse_scale(a, job, ar.m);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
 #pragma unroll
             for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, ar.m), ar.m));
@@ -415,7 +415,6 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
         const double *loff = reinterpret_cast<const double *>(lrec + 128);
         const double off = loff[0];
         const double c28 = fp_reduce(0x1p28, ml);
-        const FpTw w28{c28, c28 * ml.qinv};
         const uint64_t *tl = reinterpret_cast<const uint64_t *>(tiles);
 #pragma unroll
         for (int g = 0; g < 4; g++) {
@@ -431,7 +430,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
                 const double ld = __builtin_fma((double)l23, 16384.0, (double)l01) + off;
                 const double hd = __builtin_fma((double)h23, 16384.0, (double)h01);
                 const double t = fp_from_u64(tl[e + ((uint32_t)(32 * i) << LOGC)]);
-                const uint64_t r = fp_to_u64(fp_canonical(t - (fp_mulmod(hd, w28, ml) + ld), ml));
+                const uint64_t r = fp_to_u64(fp_canonical(t - (fp_mulmod(hd, c28, ml) + ld), ml));
                 const uint32_t b0 = (uint32_t)(r >> (16 * kg)) & 0xffu, b1 = (uint32_t)(r >> (16 * kg + 8)) & 0xffu;
                 // (in place: as a new value in the source, the compiler keeps the old and the new operand beside each other,
                 // 32 times four registers)
@@ -478,7 +477,6 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
             const FpMod mod{rconst[k & 1][kg][0], rconst[k & 1][kg][1]};
             const double off = rconst[k & 1][kg][2];
             const double c28 = fp_reduce(0x1p28, mod);
-            const FpTw w28{c28, c28 * mod.qinv};
             const double *tws = twl[kg];
             double *tile_ld = tiles + kg * kMxStride;
 #pragma unroll
@@ -506,7 +504,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
                     const double ld = __builtin_fma((double)l23, 16384.0, (double)l01) + off;
                     const double hd = __builtin_fma((double)h23, 16384.0, (double)h01);
                     // |v| <= (1/2 + 2^-8) q + 2^44 + q: within the 4 x 2^50 that the register blocks of this pass start from
-                    v[i] = fp_mulmod(hd, w28, mod) + ld;
+                    v[i] = fp_mulmod(hd, c28, mod) + ld;
                 }
                 fp_ct_block<3, 2>(v, tws, 1u, mod);
                 // word i is 32 i rows further: bits 10..8 of the tile index, of which the slot takes bits 9..8 into bits 4..3

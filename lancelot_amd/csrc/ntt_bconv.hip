@@ -58,7 +58,7 @@ struct ConvFp {
 #pragma unroll
         for (int k = 0; k < NIN; k++) {
             if ((uint32_t)k >= d.n_in) break;
-            const FpTw w{row[2 * k], row[2 * k + 1]};
+            const double w = row[2 * k];
 #pragma unroll
             for (int j = 0; j < 4; j++) rr[j] -= fp_mulmod(x[k][j], w, m);
         }
@@ -94,10 +94,9 @@ struct ConvFp {
         }
         const FpMod m = ar.m;
         const double c51 = fp_reduce(0x1p51, m);
-        const FpTw w51{c51, c51 * m.qinv};
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            v[j] = fp_mulmod((hi[j] - 0x1p103) * 0x1p-51, w51, m) + fp_reduce(lo[j], m);   // below 3 m
+            v[j] = fp_mulmod((hi[j] - 0x1p103) * 0x1p-51, c51, m) + fp_reduce(lo[j], m);   // below 3 m
             if constexpr (MDR) v[j] += rr[j];
         }
         ar.reduce(v);   // (four stages without a reduction start from at most 1.27 q)

@@ -105,13 +105,12 @@ __device__ __forceinline__ FpCtx fp_ctx(const NttArgs &a, uint32_t table) {
     return FpCtx{FpMod{c[0], c[1]}, a.tw_fp + ((size_t)table << a.log_n)};
 }
 
-// (N^-1 [* w]) as an FP twiddle for the last multiplication of the inverse transform
-__device__ __forceinline__ FpTw inverse_scale(const NttArgs &a, const Job &job, FpMod m) {
+// (N^-1 [* w]) for the last multiplication of the inverse transform
+__device__ __forceinline__ double inverse_scale(const NttArgs &a, const Job &job, FpMod m) {
     const ScalarF64 c = scalar(a.fp_consts) + 4 * (size_t)job.table;
-    FpTw ninv{c[2], c[3]};
+    const double ninv = c[2];
     if (a.epi_mode != NTT_EPI_MUL) return ninv;
-    const double w = fp_canonical(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
-    return FpTw{w, w * m.qinv};
+    return fp_canonical(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
 }
 
 // coefficient at `at` of polynomial job.poly of an encoding, rounded (NTT_PRO_ROUND)
@@ -134,8 +133,7 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
         const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
         const FpMod ml = fp_ctx(a, a.pro_last).m;
-        const double wd = fp_from_u64(scalar(a.pro_w)[2 * job.limb]), wl = fp_from_u64(scalar(a.pro_w)[2 * a.pro_last]);
-        const FpTw w{wd, wd * c.m.qinv}, wlast{wl, wl * ml.qinv};
+        const double w = fp_from_u64(scalar(a.pro_w)[2 * job.limb]), wlast = fp_from_u64(scalar(a.pro_w)[2 * a.pro_last]);
         const uint64_t qj = scalar(a.moduli)[job.table], rj = scalar(a.barrett)[2 * job.table + 1];
         const uint64_t qlast = scalar(a.moduli)[a.pro_last], rlast = scalar(a.barrett)[2 * a.pro_last + 1];
 #pragma unroll
@@ -322,16 +320,14 @@ struct FpArith {
         return t;
     }
     __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
-        asm volatile("" : "+v"(w));   // keeps w * qinv out of the registers that a loop over limbs holds
-        const double t = fp_mulmod(y, FpTw{w, w * m.qinv}, m);
+        const double t = fp_mulmod(y, w, m);
         y = x - t;
         x = x + t;
     }
     __device__ __forceinline__ void gs1(V &x, V &y, double w) const {
-        asm volatile("" : "+v"(w));
         const double d = x - y;
         x = x + y;
-        y = fp_mulmod(d, FpTw{w, w * m.qinv}, m);
+        y = fp_mulmod(d, w, m);
     }
     template <int ST>
     __device__ __forceinline__ void ct(V *v, const Tw &t) const {

@@ -54,7 +54,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
             ar.reduce(v);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
             const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
-            const FpTw ninv{cc[2], cc[3]};
+            const double ninv = cc[2];
 #pragma unroll
             for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
         } else {
@@ -93,7 +93,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(job.in[glob(NB - 1, j)]);
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-            const FpTw scale = inverse_scale(a, job, c.m);
+            const double scale = inverse_scale(a, job, c.m);
             ar.reduce(v);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
 #pragma unroll
@@ -234,11 +234,9 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
                 if (EPI) {
                     // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
-                    const double wd = fp_from_u64(e.w.w);
-                    const FpTw ew{wd, wd * m.qinv};
+                    const double ew = fp_from_u64(e.w.w);
                     if (e.fma) {
-                        const double pd = fp_from_u64(e.pro_w.w);
-                        const FpTw pw{pd, pd * m.qinv};
+                        const double pw = fp_from_u64(e.pro_w.w);
 #pragma unroll
                         for (int j = 0; j < 4; j++) {
                             const double lhs = fp_mulmod(fp_from_u64(e.a[j]), pw, m) + fp_from_u64(e.b[j]);
@@ -329,7 +327,7 @@ struct FpSums {
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const double w = fp_from_u64(k[r][j]);
-                s[r][j] += fp_mulmod(v[j], FpTw{w, w * ar.m.qinv}, ar.m);
+                s[r][j] += fp_mulmod(v[j], w, ar.m);
             }
         if (++pending == 2) {
             pending = 0;
@@ -502,12 +500,12 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
             if (add && r == 0) {
                 const double pd = fp_from_u64(add_w.w);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] += fp_mulmod(fp_from_u64(c0[j]), FpTw{pd, pd * m.qinv}, m);
+                for (int j = 0; j < 4; j++) v[j] += fp_mulmod(fp_from_u64(c0[j]), pd, m);
             }
             if (fold) {
                 const double wd = fp_from_u64(fold_w.w);
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], FpTw{wd, wd * m.qinv}, m) + fp_from_u64(cl[j]);
+                for (int j = 0; j < 4; j++) v[j] = fp_mulmod(v[j], wd, m) + fp_from_u64(cl[j]);
             }
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = fp_canonical(v[j], m);
@@ -599,10 +597,10 @@ __device__ __forceinline__ void tensor4(const FpArith &ar, const NttArgs &, uint
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         const double x0 = fp_from_u64(a0[j]), x1 = fp_from_u64(a1[j]), y0 = fp_from_u64(b0[j]), y1 = fp_from_u64(b1[j]);
-        d0[j] = fp_canonical(fp_mulmod(x0, FpTw{y0, y0 * m.qinv}, m), m);
-        d2[j] = fp_canonical(fp_mulmod(x1, FpTw{y1, y1 * m.qinv}, m), m);
+        d0[j] = fp_canonical(fp_mulmod(x0, y0, m), m);
+        d2[j] = fp_canonical(fp_mulmod(x1, y1, m), m);
         // Karatsuba: both factors are below 2 q, the product is reduced to |r| <= 2 q, the difference stays below 4 q
-        const double sy = y0 + y1, mm = fp_mulmod(x0 + x1, FpTw{sy, sy * m.qinv}, m);
+        const double sy = y0 + y1, mm = fp_mulmod(x0 + x1, sy, m);
         d1[j] = fp_canonical(mm - d0[j] - d2[j], m);
     }
 }
@@ -690,7 +688,7 @@ __device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &a
 // v + x * y mod q for canonical words x, y and v as the forward stages have left it; canonical
 __device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y, const FpArith &ar, uint64_t, uint64_t) {
     const double w = fp_from_u64(y);
-    return fp_to_u64(fp_canonical(v + fp_mulmod(fp_from_u64(x), FpTw{w, w * ar.m.qinv}, ar.m), ar.m));
+    return fp_to_u64(fp_canonical(v + fp_mulmod(fp_from_u64(x), w, ar.m), ar.m));
 }
 __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t y, const IntArith &ar, uint64_t r0, uint64_t r1) {
     return add_mod(reduce_4q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);

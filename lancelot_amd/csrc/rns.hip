@@ -137,16 +137,16 @@ __global__ __launch_bounds__(kThreads) void tensor_fp_kernel(TensorArgs p, const
     const double a0 = fp_from_u64(ct1[idx]), a1 = fp_from_u64(ct1[idx + poly]);
     double d0, d1, d2;
     if (SQUARE) {
-        d0 = fp_canonical(fp_mulmod(a0, FpTw{a0, a0 * m.qinv}, m), m);
-        d2 = fp_canonical(fp_mulmod(a1, FpTw{a1, a1 * m.qinv}, m), m);
-        const double mm = fp_mulmod(a0, FpTw{a1, a1 * m.qinv}, m);
+        d0 = fp_canonical(fp_mulmod(a0, a0, m), m);
+        d2 = fp_canonical(fp_mulmod(a1, a1, m), m);
+        const double mm = fp_mulmod(a0, a1, m);
         d1 = fp_canonical(mm + mm, m);
     } else {
         const double b0 = fp_from_u64(ct2[idx]), b1 = fp_from_u64(ct2[idx + poly]);
-        d0 = fp_canonical(fp_mulmod(a0, FpTw{b0, b0 * m.qinv}, m), m);
-        d2 = fp_canonical(fp_mulmod(a1, FpTw{b1, b1 * m.qinv}, m), m);
+        d0 = fp_canonical(fp_mulmod(a0, b0, m), m);
+        d2 = fp_canonical(fp_mulmod(a1, b1, m), m);
         const double sb = b0 + b1;
-        const double mm = fp_mulmod(a0 + a1, FpTw{sb, sb * m.qinv}, m);
+        const double mm = fp_mulmod(a0 + a1, sb, m);
         d1 = fp_canonical(mm - d0 - d2, m);
     }
     out[idx] = fp_to_u64(d0);
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(kThreads) void bconv_batched_fp_kernel(BconvBatchK 
         double acc = 0.0;
 #pragma unroll
         for (int i = 0; i < kBatchIn; i++)
-            if ((uint32_t)i < d.n_in) acc += fp_mulmod(xv[i], FpTw{m[2 * i], m[2 * i + 1]}, mod);
+            if ((uint32_t)i < d.n_in) acc += fp_mulmod(xv[i], m[2 * i], mod);
         out[((size_t)p.b.out_limb[d.map_off + row] << p.log_n) + j] = fp_to_u64(fp_canonical(acc, mod));
     }
 }
@@ -722,7 +722,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         const double base = __hiloint2double((int)((1023 + B) << 20), 0);
         const double down = __hiloint2double((int)((1023 + 52 - B) << 20), 0);     // 2^-(B-52)
         const double cB = fp_reduce(__hiloint2double((int)((1023 + B - 52) << 20), 0), m);
-        const FpTw wB{cB, cB * m.qinv};
         double hi0[I], lo0[I], hi1[I], lo1[I], f0[I], f1[I];
 #pragma unroll
         for (int it = 0; it < I; it++) {
@@ -734,8 +733,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         auto fold = [&]() {
 #pragma unroll
             for (int it = 0; it < I; it++) {
-                f0[it] = fp_reduce(f0[it] + fp_mulmod((hi0[it] - base) * down, wB, m) + fp_reduce(lo0[it], m), m);
-                f1[it] = fp_reduce(f1[it] + fp_mulmod((hi1[it] - base) * down, wB, m) + fp_reduce(lo1[it], m), m);
+                f0[it] = fp_reduce(f0[it] + fp_mulmod((hi0[it] - base) * down, cB, m) + fp_reduce(lo0[it], m), m);
+                f1[it] = fp_reduce(f1[it] + fp_mulmod((hi1[it] - base) * down, cB, m) + fp_reduce(lo1[it], m), m);
                 hi0[it] = hi1[it] = base;
                 lo0[it] = lo1[it] = 0.0;
             }
@@ -807,7 +806,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
 struct HoistSumsFp {
     FpMod m;
     double base, down, hi[4], lo[4], f[4];
-    FpTw wB;
+    double cB;
     uint32_t period, pending;
     __device__ __forceinline__ HoistSumsFp(const double *consts, uint64_t q, uint32_t n_terms) : m{scalar(consts)[0], scalar(consts)[1]} {
         const uint32_t qbits = 64 - __builtin_clzll(q), tbits = 32 - __builtin_clz(n_terms);
@@ -817,8 +816,7 @@ struct HoistSumsFp {
         pending = 0;
         base = __hiloint2double((int)((1023 + B) << 20), 0);
         down = __hiloint2double((int)((1023 + 52 - B) << 20), 0);
-        const double cB = fp_reduce(__hiloint2double((int)((1023 + B - 52) << 20), 0), m);
-        wB = FpTw{cB, cB * m.qinv};
+        cB = fp_reduce(__hiloint2double((int)((1023 + B - 52) << 20), 0), m);
 #pragma unroll
         for (int i = 0; i < 4; i++) {
             hi[i] = base;
@@ -828,7 +826,7 @@ struct HoistSumsFp {
     __device__ __forceinline__ void fold() {
 #pragma unroll
         for (int i = 0; i < 4; i++) {
-            f[i] = fp_reduce(f[i] + fp_mulmod((hi[i] - base) * down, wB, m) + fp_reduce(lo[i], m), m);
+            f[i] = fp_reduce(f[i] + fp_mulmod((hi[i] - base) * down, cB, m) + fp_reduce(lo[i], m), m);
             hi[i] = base;
             lo[i] = 0.0;
         }
@@ -1421,7 +1419,6 @@ __global__ __launch_bounds__(kThreads) void inner_product_fp_kernel(InnerFpArgs 
         const ulonglong2 k0 = *reinterpret_cast<const ulonglong2 *>(k + key_off);
         const ulonglong2 k1 = *reinterpret_cast<const ulonglong2 *>(k + key_off + key_poly);
         const double w00 = fp_from_u64(k0.x), w01 = fp_from_u64(k0.y), w10 = fp_from_u64(k1.x), w11 = fp_from_u64(k1.y);
-        const FpTw t00{w00, w00 * m.qinv}, t01{w01, w01 * m.qinv}, t10{w10, w10 * m.qinv}, t11{w11, w11 * m.qinv};
         const bool is_own = d == own_digit;
         const uint64_t *src = is_own ? p.own + ((size_t)t << p.log_n) + j : p.y + (((size_t)d * LK + t) << p.log_n) + j;
         const size_t stride = is_own ? p.own_item_stride : p.y_item_stride;
@@ -1430,10 +1427,10 @@ __global__ __launch_bounds__(kThreads) void inner_product_fp_kernel(InnerFpArgs 
             const uint32_t item = item0 + i < p.items ? item0 + i : p.items - 1;
             const ulonglong2 v = *reinterpret_cast<const ulonglong2 *>(src + item * stride);
             const double y0 = fp_from_u64(v.x), y1 = fp_from_u64(v.y);
-            acc[i][0] += fp_mulmod(y0, t00, m);
-            acc[i][1] += fp_mulmod(y1, t01, m);
-            acc[i][2] += fp_mulmod(y0, t10, m);
-            acc[i][3] += fp_mulmod(y1, t11, m);
+            acc[i][0] += fp_mulmod(y0, w00, m);
+            acc[i][1] += fp_mulmod(y1, w01, m);
+            acc[i][2] += fp_mulmod(y0, w10, m);
+            acc[i][3] += fp_mulmod(y1, w11, m);
         }
         if ((d & 7) == 7) {
 #pragma unroll
@@ -1444,8 +1441,7 @@ __global__ __launch_bounds__(kThreads) void inner_product_fp_kernel(InnerFpArgs 
     const size_t o = ((size_t)t << p.log_n) + j;
     const size_t opoly = (size_t)LK << p.log_n;
     const bool fold = p.fold_ct && t == p.L - 1;
-    const double wd = fold ? fp_from_u64(p.fold_w[0]) : 0.0;
-    const FpTw fw{wd, wd * m.qinv};
+    const double fw = fold ? fp_from_u64(p.fold_w[0]) : 0.0;
 #pragma unroll
     for (int i = 0; i < I; i++) {
         if (item0 + i >= p.items) break;
