@@ -268,6 +268,20 @@ int he_keyswitch_rescale_batch(const he_context *ctx, uint32_t L, uint32_t items
 int he_pair_square_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32_t chunks,
                        const uint64_t *const *d_pairs, uint64_t *out01, uint64_t *out2, he_stream stream);
 
+/* Two sums of squares per item: first + X^(N/2) second, for the two halves of row k of the DEVICE pointer table d_pairs
+ * [items][2][count][2] (a null first entry of the second half: no second).  X^(N/2) multiplies every slot by i, so messages with real
+ * slots travel as the real and imaginary parts of one ciphertext.  Otherwise as he_pair_square_sum. */
+int he_pair_square_sum_packed(const he_context *ctx, uint32_t L, uint32_t items, uint32_t count, const uint64_t *const *d_pairs,
+                              uint64_t *out01, uint64_t *out2, he_stream stream);
+
+/* Row sums of the squared distances: for client i of the DEVICE pointer table d_cts [clients][chunks] the sum over all clients j and
+ * all chunks of (x_i - x_j)^2, word for word what he_pair_square_sum and he_sum_ciphertexts give, two clients per item as above:
+ * item k = client 2 k + X^(N/2) client 2 k + 1, ceil(clients / 2) items (decrypt-sort-mask's scores, byzantine_fl.py:327-353).
+ * workspace: he_row_square_sums_workspace_words words. */
+size_t he_row_square_sums_workspace_words(const he_context *ctx, uint32_t L, uint32_t chunks);
+int he_row_square_sums_packed(const he_context *ctx, uint32_t L, uint32_t clients, uint32_t chunks, const uint64_t *const *d_cts,
+                              uint64_t *out01, uint64_t *out2, uint64_t *workspace, he_stream stream);
+
 /* out [items][size][L][N]: item k is the sum of the `count` ciphertexts ([size][L][N]) that row k of the DEVICE pointer table
  * d_cts [items][count] names (add_inplace, src/evaluate.cu:118-165, once per term). */
 int he_sum_ciphertexts(const he_context *ctx, uint32_t L, uint32_t size, uint32_t items, uint32_t count,
@@ -391,6 +405,12 @@ int he_decrypt_decode_real_batch(const he_context *ctx, const uint64_t *const *d
                                  const uint64_t *sk, const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt,
                                  uint32_t cdt_len, uint32_t slots, double scale, uint32_t count, double *out,
                                  uint64_t *workspace, he_stream stream);
+
+/* The same with both parts of every value: out [items][count] (re, im). */
+int he_decrypt_decode_flood_batch(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs,
+                                  const uint64_t *sk, const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt,
+                                  uint32_t cdt_len, uint32_t slots, double scale, uint32_t count, double *out,
+                                  uint64_t *workspace, he_stream stream);
 
 /* Decryption and decoding of `items` size-2 ciphertexts in one launch per stage: for the ciphertexts [2][limbs][N]
  * named by the DEVICE pointer table d_cts, m = c0 + c1 s (+ noise [items][limbs][N] in NTT form, or NULL), inverse

@@ -66,6 +66,9 @@ SIGNATURES = {
     "he_hoisted_rotations_batch": (C.c_int, [vp, u32, u32, vp, C.POINTER(vp), C.POINTER(u32), u32, C.c_int, vp, vp, vp]),
     "he_keyswitch_rescale_batch": (C.c_int, [vp, u32, u32, vp, u32, C.POINTER(vp), vp, vp, u32, vp, vp]),
     "he_pair_square_sum": (C.c_int, [vp, u32, u32, u32, vp, vp, vp, vp]),
+    "he_pair_square_sum_packed": (C.c_int, [vp, u32, u32, u32, vp, vp, vp, vp]),
+    "he_row_square_sums_workspace_words": (C.c_size_t, [vp, u32, u32]),
+    "he_row_square_sums_packed": (C.c_int, [vp, u32, u32, u32, vp, vp, vp, vp, vp]),
     "he_sum_ciphertexts": (C.c_int, [vp, u32, u32, u32, u32, vp, vp, vp]),
     "he_multiply_sum": (C.c_int, [vp, u32, u32, u32, vp, vp, vp]),
     "he_keyswitch_rescale": (C.c_int, [vp, u32, vp, C.POINTER(vp), vp, vp, u32, vp, vp]),
@@ -88,6 +91,8 @@ SIGNATURES = {
     "he_decrypt_decode_real_workspace_words": (C.c_size_t, [vp, u32, u32, u32]),
     "he_decrypt_decode_real_batch": (C.c_int, [vp, vp, u32, u32, vp, C.POINTER(u32), u64, vp, u32, u32, C.c_double, u32, vp, vp,
                                                vp]),
+    "he_decrypt_decode_flood_batch": (C.c_int, [vp, vp, u32, u32, vp, C.POINTER(u32), u64, vp, u32, u32, C.c_double, u32, vp, vp,
+                                                vp]),
     "he_encrypt_batch_workspace_words": (C.c_size_t, [vp, u32, u32]),
     "he_encrypt_batch": (C.c_int, [vp, u32, u32, vp, C.POINTER(u32), u64, vp, vp, vp]),
     "he_sample_batch": (C.c_int, [vp, C.c_int, C.POINTER(u32), u64, vp, u32, u32, u32, u32, vp, u32, u32, vp]),

@@ -832,7 +832,27 @@ int he_pair_square_sum(const he_context *ctx, uint32_t L, uint32_t items, uint32
                        const uint64_t *const *d_pairs, uint64_t *out01, uint64_t *out2, he_stream s) {
     if (!ctx || !d_pairs || !out01 || !out2 || L == 0 || L > ctx->size_q || items == 0 || items > 16384 || chunks == 0)
         return HE_E_INVALID_ARGUMENT;
-    HE_HIP(launch_pair_square_sum(ctx->tables(), d_pairs, out01, out2, L, items, chunks, S(s)));
+    HE_HIP(launch_pair_square_sum(ctx->tables(), ctx->d_psi, d_pairs, out01, out2, L, items, 1, chunks, S(s)));
+    return HE_OK;
+}
+
+int he_pair_square_sum_packed(const he_context *ctx, uint32_t L, uint32_t items, uint32_t count, const uint64_t *const *d_pairs,
+                              uint64_t *out01, uint64_t *out2, he_stream s) {
+    if (!ctx || !d_pairs || !out01 || !out2 || L == 0 || L > ctx->size_q || items == 0 || items > 16384 || count == 0)
+        return HE_E_INVALID_ARGUMENT;
+    HE_HIP(launch_pair_square_sum(ctx->tables(), ctx->d_psi, d_pairs, out01, out2, L, items, 2, count, S(s)));
+    return HE_OK;
+}
+
+size_t he_row_square_sums_workspace_words(const he_context *ctx, uint32_t L, uint32_t chunks) {
+    return ctx ? (2 * (size_t)chunks + 3) * L * ctx->n() : 0;
+}
+
+int he_row_square_sums_packed(const he_context *ctx, uint32_t L, uint32_t clients, uint32_t chunks, const uint64_t *const *d_cts,
+                              uint64_t *out01, uint64_t *out2, uint64_t *ws, he_stream s) {
+    if (!ctx || !d_cts || !out01 || !out2 || !ws || L == 0 || L > ctx->size_q || clients == 0 || clients > 32768 || chunks == 0)
+        return HE_E_INVALID_ARGUMENT;
+    HE_HIP(launch_row_square_sums(ctx->tables(), ctx->d_psi, d_cts, out01, out2, ws, L, clients, chunks, S(s)));
     return HE_OK;
 }
 
@@ -1572,8 +1592,9 @@ int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
+// (both: (re, im) pairs)
 int decode_real_impl(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t items, uint32_t slots, double scale,
-                     uint64_t *coeff, double2 *v, double *out, uint32_t count, he_stream s) {
+                     uint64_t *coeff, double2 *v, double *out, uint32_t count, bool both, he_stream s) {
     const FftTables ft = ctx->fft();
     NttArgs inv = base_args(ctx, false);
     inv.in = plain;
@@ -1584,12 +1605,12 @@ int decode_real_impl(const he_context *ctx, const uint64_t *plain, uint32_t limb
     if (limbs <= 4 && ctx->log_n >= 12 && ctx->log_n <= 16 && ctx->size_qp <= 64) {
         HE_HIP(launch_ntt_blocks(inv, items, false, backend, S(s)));
         inv.in = coeff;
-        HE_HIP(launch_ckks_decode_real(ft, inv, backend, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, out, count, S(s)));
+        HE_HIP(launch_ckks_decode_real(ft, inv, backend, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, out, count, both, S(s)));
         return HE_OK;
     }
     HE_HIP(launch_ntt_inverse(inv, items, backend, S(s)));
     HE_HIP(launch_ckks_compose(ft, ctx->tables(), coeff, limbs, slots, scale, ctx->d_garner_inv, ctx->size_q, v, items, S(s)));
-    HE_HIP(launch_ckks_fft_real(ft, slots, v, items, out, count, S(s)));
+    HE_HIP(launch_ckks_fft_real(ft, slots, v, items, out, count, both, S(s)));
     return HE_OK;
 }
 
@@ -1609,6 +1630,25 @@ int decrypt_flood_impl(const he_context *ctx, const DecryptArgs &d, uint32_t lim
     HE_HIP(launch_ntt_rows(a, items * limbs, true, backend, S(s)));
     HE_HIP(launch_decrypt_blocks(a, d, items, backend, S(s)));
     return HE_OK;
+}
+
+// out [items][count] real parts, or [items][count][2] (both)
+int decrypt_decode_impl(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs, const uint64_t *sk,
+                        const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t slots, double scale,
+                        uint32_t count, bool both, double *out, uint64_t *ws, he_stream s) {
+    if (!ctx || !d_cts || !sk || !out || !ws || items == 0 || items > 16384 || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
+    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0) || count == 0 || count > slots || (key && !cdt))
+        return HE_E_INVALID_ARGUMENT;
+    if (key && (cdt_len == 0 || cdt_len >= 128)) return HE_E_UNSUPPORTED;
+    const size_t n = ctx->n();
+    uint64_t *plain = ws, *v = ws + (size_t)items * limbs * n, *noise = v + 2 * (size_t)items * slots;
+    if (key) {
+        if (int rc = decrypt_flood_impl(ctx, DecryptArgs{nullptr, d_cts, sk, 0, 2}, limbs, items, key, stream_id, cdt, cdt_len, plain, noise, s))
+            return rc;
+    } else {
+        HE_HIP(launch_decrypt_gather(ctx->tables(), d_cts, sk, nullptr, plain, limbs, items, S(s)));
+    }
+    return decode_real_impl(ctx, plain, limbs, items, slots, scale, plain, reinterpret_cast<double2 *>(v), out, count, both, s);
 }
 
 }  // namespace
@@ -1643,7 +1683,8 @@ int he_ckks_decode_real(const he_context *ctx, const uint64_t *plain, uint32_t l
                         uint32_t count, uint64_t *ws, he_stream s) {
     if (!ctx || !plain || !out || !ws || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0) || count == 0 || count > slots) return HE_E_INVALID_ARGUMENT;
-    return decode_real_impl(ctx, plain, limbs, 1, slots, scale, ws, reinterpret_cast<double2 *>(ws + (size_t)limbs * ctx->n()), out, count, s);
+    return decode_real_impl(ctx, plain, limbs, 1, slots, scale, ws, reinterpret_cast<double2 *>(ws + (size_t)limbs * ctx->n()), out, count, false,
+                            s);
 }
 
 size_t he_decrypt_decode_real_workspace_words(const he_context *ctx, uint32_t limbs, uint32_t slots, uint32_t items) {
@@ -1654,20 +1695,15 @@ size_t he_decrypt_decode_real_workspace_words(const he_context *ctx, uint32_t li
 int he_decrypt_decode_real_batch(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs, const uint64_t *sk,
                                  const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t slots,
                                  double scale, uint32_t count, double *out, uint64_t *ws, he_stream s) {
-    if (!ctx || !d_cts || !sk || !out || !ws || items == 0 || items > 16384 || limbs == 0 || limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
-    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || !(scale > 0) || count == 0 || count > slots || (key && !cdt))
-        return HE_E_INVALID_ARGUMENT;
-    if (key && (cdt_len == 0 || cdt_len >= 128)) return HE_E_UNSUPPORTED;
-    const size_t n = ctx->n();
-    uint64_t *plain = ws, *v = ws + (size_t)items * limbs * n, *noise = v + 2 * (size_t)items * slots;
-    if (key) {
-        if (int rc = decrypt_flood_impl(ctx, DecryptArgs{nullptr, d_cts, sk, 0, 2}, limbs, items, key, stream_id, cdt, cdt_len, plain, noise, s))
-            return rc;
-    } else {
-        HE_HIP(launch_decrypt_gather(ctx->tables(), d_cts, sk, nullptr, plain, limbs, items, S(s)));
-    }
-    return decode_real_impl(ctx, plain, limbs, items, slots, scale, plain, reinterpret_cast<double2 *>(v), out, count, s);
+    return decrypt_decode_impl(ctx, d_cts, items, limbs, sk, key, stream_id, cdt, cdt_len, slots, scale, count, false, out, ws, s);
 }
+
+int he_decrypt_decode_flood_batch(const he_context *ctx, const uint64_t *const *d_cts, uint32_t items, uint32_t limbs, const uint64_t *sk,
+                                  const uint32_t key[8], uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t slots,
+                                  double scale, uint32_t count, double *out, uint64_t *ws, he_stream s) {
+    return decrypt_decode_impl(ctx, d_cts, items, limbs, sk, key, stream_id, cdt, cdt_len, slots, scale, count, true, out, ws, s);
+}
+
 
 int he_ckks_decode(const he_context *ctx, const uint64_t *plain, uint32_t limbs, uint32_t slots, double scale,
                    double *out, uint64_t *ws, he_stream s) {

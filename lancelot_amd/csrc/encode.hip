@@ -61,12 +61,21 @@ __device__ __forceinline__ double2 source_value(const FftSource &src, uint32_t i
     return double2{src.re[at], src.im ? src.im[at] : 0.0};
 }
 
-// Where a decoding ends: with `re` the real parts of the first `count` values of every item, packed, instead of the vector.
+// Where a decoding ends: with `re` the real parts of the first `count` values of every item, or both parts, packed, instead of the
+// vector.
 struct FftTarget {
     double *re;
     uint32_t count;
-    size_t value_stride;   // doubles between the items' values
+    bool both;
 };
+
+__device__ __forceinline__ void store_value(const FftTarget &dst, uint32_t item, uint32_t i, double2 v) {
+    const size_t at = (size_t)item * dst.count + i;
+    if (dst.both)
+        reinterpret_cast<double2 *>(dst.re)[at] = v;
+    else
+        dst.re[at] = v.x;
+}
 
 constexpr uint32_t kSmallSlots = 256;   // below this the small kernel runs
 
@@ -96,7 +105,7 @@ __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t
         __syncthreads();
     }
     if (!INVERSE && dst.re) {
-        for (uint32_t i = threadIdx.x; i < dst.count; i += kThreads) dst.re[blockIdx.y * dst.value_stride + i] = s[i].x;
+        for (uint32_t i = threadIdx.x; i < dst.count; i += kThreads) store_value(dst, blockIdx.y, i, s[i]);
     } else {
         for (uint32_t i = threadIdx.x; i < tile; i += kThreads) g[i] = s[i];
     }
@@ -223,7 +232,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, Fft
         if (dst.re) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (pos(0, j) < dst.count) dst.re[item * dst.value_stride + pos(0, j)] = x[j].x;
+                if (pos(0, j) < dst.count) store_value(dst, item, pos(0, j), x[j]);
         } else {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
@@ -271,7 +280,7 @@ __global__ __launch_bounds__((1 << (B - 2)) * kFftBlocks<B>) void cfft_blocks_ke
         if (dst.re && log_slots == B) {
 #pragma unroll
             for (int j = 0; j < 4; j++)
-                if (pos(0, j) < dst.count) dst.re[item * dst.value_stride + pos(0, j)] = x[j].x;
+                if (pos(0, j) < dst.count) store_value(dst, item, pos(0, j), x[j]);
         } else {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
@@ -559,7 +568,7 @@ hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const doubl
     const uint32_t n = 1u << t.log_n, log_slots = 31 - __builtin_clz(slots);
     if (items == 0 || items > 65535 || !out || limbs == 0) return hipErrorInvalidValue;
     unsigned long long *maxima = reinterpret_cast<unsigned long long *>(max_bits);
-    hipError_t e = run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, maxima}, FftTarget{nullptr, 0, 0});
+    hipError_t e = run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, maxima}, FftTarget{nullptr, 0, false});
     if (e != hipSuccess) return e;
     const RoundSink sink{out, tab.moduli, tab.barrett, limbs, out_item_stride};
     if (slots == n / 2 && log_slots >= 8)
@@ -574,13 +583,13 @@ hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const doubl
 hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
                                    double2 *v, uint32_t items, size_t value_stride, hipStream_t s) {
     if (items == 0 || items > 65535 || !re) return hipErrorInvalidValue;
-    return run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, nullptr}, FftTarget{nullptr, 0, 0});
+    return run_fft<true>(v, slots, items, t, s, FftSource{re, im, count, value_stride, nullptr}, FftTarget{nullptr, 0, false});
 }
 
 hipError_t launch_ckks_fft_real(const FftTables &t, uint32_t slots, double2 *v, uint32_t items, double *re, uint32_t count,
-                                hipStream_t s) {
+                                bool both, hipStream_t s) {
     if (items == 0 || items > 65535 || !re || count == 0 || count > slots) return hipErrorInvalidValue;
-    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{re, count, count});
+    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{re, count, both});
 }
 
 hipError_t launch_ckks_compose(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs,
@@ -607,12 +616,12 @@ hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint6
                               uint32_t slots, double scale, const uint64_t *garner_inv, uint32_t garner_stride,
                               double2 *v, uint32_t items, hipStream_t s) {
     if (hipError_t e = launch_ckks_compose(t, tab, res, limbs, slots, scale, garner_inv, garner_stride, v, items, s)) return e;
-    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{nullptr, 0, 0});
+    return run_fft<false>(v, slots, items, t, s, FftSource{nullptr, nullptr, 0, 0, nullptr}, FftTarget{nullptr, 0, false});
 }
 
 hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int backend, uint32_t slots, double scale,
                                    const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items, double *re,
-                                   uint32_t count, hipStream_t s) {
+                                   uint32_t count, bool both, hipStream_t s) {
     const uint32_t limbs = inv.map.limbs, log_slots = 31 - __builtin_clz(slots);
     if (inv.log_n < 12 || inv.log_n > 16 || inv.jobs || limbs == 0 || limbs > 4 || items == 0 || items > 65535) return hipErrorInvalidValue;
     NttArgs a = inv;   // (the mask stands for the launch's back end)
@@ -636,7 +645,7 @@ hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int b
 #undef HE_CASE
 #undef HE_LIMBS
     if (hipError_t e = hipGetLastError()) return e;
-    return launch_ckks_fft_real(t, slots, v, items, re, count, s);
+    return launch_ckks_fft_real(t, slots, v, items, re, count, both, s);
 }
 
 hipError_t launch_take_slots(const double2 *v, uint32_t slots, uint32_t items, uint32_t count, double2 *out, hipStream_t s) {

@@ -123,20 +123,14 @@ std::vector<CAHELGPUCiphertext> multiply_sum(const CAHELGPUContext &context,
     return slices(std::move(out), items, 3, first, scale);
 }
 
-// For every (i, j) of `pairs`: acc = sum over chunks of (clients[j][c] - clients[i][c])^2, relinearised and rescaled,
-// then for every round acc += sum over the round's steps of rot(acc, step) (hoisted), as
-// GPU_compute_pair_distance does per pair (lancelot-main-GPU/utils/byzantine_fl.py:173-321) -- here with one
-// launch per stage for all pairs.  scale > 0 overrides the scale after the rescale (the reference's set_scale).
-// drop_levels > 0 switches the rescaled ciphertexts down by that many further limbs without scaling
-// (mod_switch_to_next) before the slot sum, whose key switches then run over fewer limbs.
-std::vector<CAHELGPUCiphertext> pair_square_distances(
-    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
-    const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
-    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels) {
+namespace {
+
+using Clients = std::vector<std::vector<const CAHELGPUCiphertext *>>;
+
+// What the distances of `clients` and the key switches after them need; throws what the calls one by one would.
+void check_clients(const CAHELGPUContext &context, const Clients &clients, const CAHELGPURelinKey &rlk, const CAHELGPUGaloisKey &glk) {
     if (context.scheme() != cahel::scheme_type::ckks) throw std::logic_error("unsupported scheme");
     if (clients.empty() || clients[0].empty()) throw std::invalid_argument("no ciphertexts");
-    if (pairs.empty()) return {};
-    if (pairs.size() > 16384) throw std::invalid_argument("too many pairs");
     const CAHELGPUCiphertext &first = *clients[0][0];
     const std::size_t chunks = clients[0].size();
     for (const auto &client : clients) {
@@ -148,35 +142,36 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
             if (ct->scale() != first.scale()) throw std::invalid_argument("scale mismatch");
         }
     }
-    for (const auto &pr : pairs)
-        if (pr.first >= clients.size() || pr.second >= clients.size()) throw std::invalid_argument("pair out of range");
     if (rlk.parms_id() != context.key_parms_id() || glk.parms_id() != context.key_parms_id())
         throw std::invalid_argument("keys are not valid for encryption parameters");
     if (!context.using_keyswitching()) throw std::logic_error("keyswitching is not supported by the context");
     const std::size_t chain = first.chain_index();
     if (chain == 0) throw std::invalid_argument("key switching needs a data-level ciphertext");
     if (chain == context.max_chain_index()) throw std::invalid_argument("end of modulus switching chain reached");
+}
 
+// the chunks of both clients of a pair, side by side
+void push_pair(std::vector<const uint64_t *> &table, const Clients &clients, const std::pair<std::size_t, std::size_t> &pr) {
+    for (std::size_t c = 0; c < clients[0].size(); c++) {
+        table.push_back(clients[pr.second][c]->data());
+        table.push_back(clients[pr.first][c]->data());
+    }
+}
+
+// Squared distances (d01 [items][2][L][N], d2 [items][L][N], like products of `first` with itself) relinearised and rescaled, then for
+// every round acc += sum over the round's steps of rot(acc, step) (hoisted).  scale > 0 overrides the scale after the rescale
+// (the reference's set_scale).  drop_levels > 0 switches the rescaled ciphertexts down by that many further limbs without
+// scaling (mod_switch_to_next) before the slot sum, whose key switches then run over fewer limbs.
+std::vector<CAHELGPUCiphertext> sum_of_slots(const CAHELGPUContext &context, const CAHELGPUCiphertext &first, const DeviceBuffer &d01,
+                                             const DeviceBuffer &d2, uint32_t items, const CAHELGPURelinKey &rlk,
+                                             const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale,
+                                             std::size_t drop_levels) {
     he_context *h = context.handle();
     he_stream st = context.stream();
-    const std::size_t n = context.poly_degree(), K = context.size_p();
-    const uint32_t L = (uint32_t)first.coeff_modulus_size(), items = (uint32_t)pairs.size();
+    const std::size_t n = context.poly_degree(), K = context.size_p(), chain = first.chain_index();
+    const uint32_t L = (uint32_t)first.coeff_modulus_size();
 
-    // (1) squared differences, summed over the chunks, as size-3 ciphertexts (lazy relinearisation)
-    std::vector<const uint64_t *> table;
-    table.reserve((std::size_t)items * chunks * 2);
-    for (const auto &pr : pairs)
-        for (std::size_t c = 0; c < chunks; c++) {
-            table.push_back(clients[pr.second][c]->data());
-            table.push_back(clients[pr.first][c]->data());
-        }
-    const DeviceBuffer d_table = upload_table(table, st);
-    DeviceBuffer d01((std::size_t)items * 2 * L * n), d2((std::size_t)items * L * n);
-    check_status(he_pair_square_sum(h, L, items, (uint32_t)chunks, reinterpret_cast<const uint64_t *const *>(d_table.get()),
-                                    d01.get(), d2.get(), st),
-                 "he_pair_square_sum");
-
-    // (2) relinearise + rescale
+    // (1) relinearise + rescale
     auto rl = rlk.key_ptrs();
     if (rl.size() < (L + K - 1) / K) throw std::invalid_argument("key_poly_num != 2");
     DeviceBuffer ws(he_keyswitch_batch_workspace_words(h, L, items));
@@ -186,7 +181,7 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
     double out_scale = first.scale() * first.scale() / static_cast<double>(context.key_modulus()[L - 1].value());
     if (scale > 0) out_scale = scale;
 
-    // (2b) optional: drop limbs without scaling, the leading limbs of every polynomial move to a denser batch
+    // (2) optional: drop limbs without scaling, the leading limbs of every polynomial move to a denser batch
     uint32_t L1 = L - 1;
     std::size_t out_chain = chain + 1;
     if (drop_levels) {
@@ -224,7 +219,7 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
         std::swap(acc, next);
     }
 
-    // (4) one ciphertext object per pair, each a slice of the batch (no copies)
+    // (4) one ciphertext object per item, each a slice of the batch (no copies)
     std::vector<CAHELGPUCiphertext> out(items);
     const std::size_t words = 2 * (std::size_t)L1 * n;
     auto shared = std::make_shared<DeviceBuffer>(std::move(acc));
@@ -241,4 +236,79 @@ std::vector<CAHELGPUCiphertext> pair_square_distances(
         ct.is_asymmetric_ = first.is_asymmetric_;
     }
     return out;
+}
+
+std::vector<CAHELGPUCiphertext> square_distances(const CAHELGPUContext &context, const Clients &clients,
+                                                 const std::vector<std::pair<std::size_t, std::size_t>> &pairs,
+                                                 const CAHELGPURelinKey &rlk, const CAHELGPUGaloisKey &glk,
+                                                 const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels,
+                                                 bool packed) {
+    if (context.scheme() != cahel::scheme_type::ckks) throw std::logic_error("unsupported scheme");
+    if (clients.empty() || clients[0].empty()) throw std::invalid_argument("no ciphertexts");
+    if (pairs.empty()) return {};
+    if (pairs.size() > 16384) throw std::invalid_argument("too many pairs");
+    check_clients(context, clients, rlk, glk);
+    for (const auto &pr : pairs)
+        if (pr.first >= clients.size() || pr.second >= clients.size()) throw std::invalid_argument("pair out of range");
+    const CAHELGPUCiphertext &first = *clients[0][0];
+    const std::size_t n = context.poly_degree(), chunks = clients[0].size(), items = packed ? (pairs.size() + 1) / 2 : pairs.size();
+    const uint32_t L = (uint32_t)first.coeff_modulus_size();
+    he_stream st = context.stream();
+    std::vector<const uint64_t *> table;
+    table.reserve(2 * chunks * (pairs.size() + 1));
+    for (const auto &pr : pairs) push_pair(table, clients, pr);
+    if (packed && pairs.size() % 2) table.insert(table.end(), 2 * chunks, nullptr);
+    const DeviceBuffer d_table = upload_table(table, st);
+    DeviceBuffer d01(items * 2 * L * n), d2(items * L * n);
+    check_status((packed ? he_pair_square_sum_packed : he_pair_square_sum)(context.handle(), L, (uint32_t)items, (uint32_t)chunks,
+                                                                           reinterpret_cast<const uint64_t *const *>(d_table.get()),
+                                                                           d01.get(), d2.get(), st),
+                 "he_pair_square_sum");
+    return sum_of_slots(context, first, d01, d2, (uint32_t)items, rlk, glk, rounds, scale, drop_levels);
+}
+
+}  // namespace
+
+// For every (i, j) of `pairs`: the sum over chunks of (clients[j][c] - clients[i][c])^2 and its slot sum, as
+// GPU_compute_pair_distance does per pair (lancelot-main-GPU/utils/byzantine_fl.py:173-321) -- here with one
+// launch per stage for all pairs.
+std::vector<CAHELGPUCiphertext> pair_square_distances(
+    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
+    const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
+    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels) {
+    return square_distances(context, clients, pairs, rlk, glk, rounds, scale, drop_levels, false);
+}
+
+// The same, two pairs per ciphertext: item k holds pair 2 k in the real and pair 2 k + 1 in the imaginary parts of its slots
+// (the messages' slots are real), half the key switches.
+std::vector<CAHELGPUCiphertext> packed_pair_distances(
+    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
+    const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
+    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels) {
+    return square_distances(context, clients, pairs, rlk, glk, rounds, scale, drop_levels, true);
+}
+
+// Every client's sum of squared distances to all others (its score), client 2 k in the real and client 2 k + 1 in the imaginary parts
+// of item k: relinearisation, rescale and slot sum are linear, so the scores go through them instead of all pairs.
+std::vector<CAHELGPUCiphertext> packed_distance_scores(
+    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients, const CAHELGPURelinKey &rlk,
+    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels) {
+    check_clients(context, clients, rlk, glk);
+    if (clients.size() > 32768) throw std::invalid_argument("too many clients");
+    const CAHELGPUCiphertext &first = *clients[0][0];
+    const std::size_t n = context.poly_degree(), items = (clients.size() + 1) / 2;
+    const uint32_t L = (uint32_t)first.coeff_modulus_size(), chunks = (uint32_t)clients[0].size();
+    he_stream st = context.stream();
+    std::vector<const uint64_t *> table;
+    for (const auto &client : clients)
+        for (const CAHELGPUCiphertext *ct : client) table.push_back(ct->data());
+    const DeviceBuffer d_table = upload_table(table, st);
+    DeviceBuffer d01(items * 2 * L * n), d2(items * L * n);
+    {
+        DeviceBuffer ws(he_row_square_sums_workspace_words(context.handle(), L, chunks));
+        check_status(he_row_square_sums_packed(context.handle(), L, (uint32_t)clients.size(), chunks,
+                                               reinterpret_cast<const uint64_t *const *>(d_table.get()), d01.get(), d2.get(), ws.get(), st),
+                     "he_row_square_sums_packed");
+    }
+    return sum_of_slots(context, first, d01, d2, (uint32_t)items, rlk, glk, rounds, scale, drop_levels);
 }

@@ -3,6 +3,7 @@
 // with an underscore, and the accessor methods on context / plaintext / ciphertext / keys, are additions used
 // by the test-suite and the benchmark (seeding, raw device pointers, host copies); they do not exist in the
 // reference and nothing in Lancelot calls them.
+#include <complex>
 #include <fstream>
 #include <sstream>
 
@@ -167,6 +168,19 @@ PYBIND11_MODULE(pyCAHEL, m) {
                  {
                      py::gil_scoped_release release;
                      k.decrypt_decode_many(c, cts, slots, count, values);
+                 }
+                 return a;
+             },
+             py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count") = 1)
+        .def("decrypt_decode_complex_many",
+             [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, const std::vector<const CAHELGPUCiphertext *> &cts,
+                std::size_t slots, std::size_t count) {
+                 py::array_t<std::complex<double>> a(
+                     {(py::ssize_t)cts.size(), (py::ssize_t)(count > slots || slots > c.poly_degree() ? 0 : count)});
+                 double *values = reinterpret_cast<double *>(a.mutable_data());
+                 {
+                     py::gil_scoped_release release;
+                     k.decrypt_decode_many(c, cts, slots, count, values, true);
                  }
                  return a;
              },
@@ -337,6 +351,11 @@ PYBIND11_MODULE(pyCAHEL, m) {
     m.def("pair_square_distances", &pair_square_distances, py::arg("context"), py::arg("clients"), py::arg("pairs"),
           py::arg("relin_key"), py::arg("galois_key"), py::arg("rounds"), py::arg("scale") = 0.0, py::arg("drop_levels") = 0,
           nogil);
+    m.def("packed_pair_distances", &packed_pair_distances, py::arg("context"), py::arg("clients"), py::arg("pairs"),
+          py::arg("relin_key"), py::arg("galois_key"), py::arg("rounds"), py::arg("scale") = 0.0, py::arg("drop_levels") = 0,
+          nogil);
+    m.def("packed_distance_scores", &packed_distance_scores, py::arg("context"), py::arg("clients"), py::arg("relin_key"),
+          py::arg("galois_key"), py::arg("rounds"), py::arg("scale") = 0.0, py::arg("drop_levels") = 0, nogil);
     m.def("sum_ciphertexts", &sum_ciphertexts, py::arg("context"), py::arg("rows"), nogil);
     m.def("multiply_sum", &multiply_sum, py::arg("context"), py::arg("rows"), py::arg("factors"), nogil);
     m.def("mod_switch_to", py::overload_cast<const CAHELGPUContext &, const CAHELGPUPlaintext &, CAHELGPUPlaintext &, std::size_t>(&mod_switch_to), nogil);

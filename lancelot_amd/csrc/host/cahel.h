@@ -393,8 +393,9 @@ public:
     // Real parts of the first `count` slots of every ciphertext, [items][count] row-major: decrypt + decode of all of
     // them with one launch per stage (not in the reference).  All ciphertexts: size 2, one level, one scale;
     // `slots` = the encoder's slot count.
+    // both: (re, im) pairs, [items][count][2].
     void decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
-                             std::size_t slots, std::size_t count, double *destination);
+                             std::size_t slots, std::size_t count, double *destination, bool both = false);
     std::vector<double> decrypt_decode_many(const CAHELGPUContext &context,
                                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots,
                                             std::size_t count) {
@@ -512,6 +513,13 @@ void relinearize_inplace(const CAHELGPUContext &context, CAHELGPUCiphertext &enc
 std::vector<CAHELGPUCiphertext> pair_square_distances(
     const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
     const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
+    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels = 0);
+std::vector<CAHELGPUCiphertext> packed_pair_distances(
+    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients,
+    const std::vector<std::pair<std::size_t, std::size_t>> &pairs, const CAHELGPURelinKey &rlk,
+    const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels = 0);
+std::vector<CAHELGPUCiphertext> packed_distance_scores(
+    const CAHELGPUContext &context, const std::vector<std::vector<const CAHELGPUCiphertext *>> &clients, const CAHELGPURelinKey &rlk,
     const CAHELGPUGaloisKey &glk, const std::vector<std::vector<int>> &rounds, double scale, std::size_t drop_levels = 0);
 std::vector<CAHELGPUCiphertext> sum_ciphertexts(const CAHELGPUContext &context,
                                                 const std::vector<std::vector<const CAHELGPUCiphertext *>> &rows);

@@ -230,7 +230,7 @@ void CAHELGPUSecretKey::decrypt(const CAHELGPUContext &context, const CAHELGPUCi
 }
 
 void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
-                                            std::size_t slots, std::size_t count, double *destination) {
+                                            std::size_t slots, std::size_t count, double *destination, bool both) {
     if (!gen_flag_) throw std::logic_error("secret key has not been generated");
     if (ciphers.empty()) return;
     if (ciphers.size() > 16384) throw std::invalid_argument("too many ciphertexts");
@@ -258,18 +258,18 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
     int status = he_memcpy_h2d_async(d_table.get(), table, items * sizeof(uint64_t), st);
     ring.fence(st);
     check_status(status, "upload");
-    const std::size_t bytes = (std::size_t)items * count * sizeof(double);
+    const std::size_t words = (std::size_t)items * count * (both ? 2 : 1), bytes = words * sizeof(double);
     const bool staged = bytes <= PinnedRing::kMaxBytes;
     DeviceBuffer ws(he_decrypt_decode_real_workspace_words(h, limbs, (uint32_t)slots, items)), d_out;
-    if (!staged) d_out.allocate((std::size_t)items * count);
+    if (!staged) d_out.allocate(words);
     double *out = staged ? static_cast<double *>(ring.take(bytes)) : reinterpret_cast<double *>(d_out.get());
     // flooding noise: the stream ids that `items` calls of decrypt would draw
-    status = he_decrypt_decode_real_batch(h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs, sk_powers_.get(),
-                                          noise_flooding_ ? context.prng_key() : nullptr,
-                                          noise_flooding_ ? context.next_stream(items) : 0, context.gauss_cdt(),
-                                          context.gauss_cdt_len(), (uint32_t)slots, first.scale(), (uint32_t)count, out, ws.get(), st);
+    status = (both ? he_decrypt_decode_flood_batch : he_decrypt_decode_real_batch)(
+        h, reinterpret_cast<const uint64_t *const *>(d_table.get()), items, limbs, sk_powers_.get(),
+        noise_flooding_ ? context.prng_key() : nullptr, noise_flooding_ ? context.next_stream(items) : 0, context.gauss_cdt(),
+        context.gauss_cdt_len(), (uint32_t)slots, first.scale(), (uint32_t)count, out, ws.get(), st);
     if (status != HE_OK && staged) ring.fence(st);   // (what was launched before the failure may still write the block)
-    check_status(status, "he_decrypt_decode_real_batch");
+    check_status(status, "he_decrypt_decode_batch");
     if (staged) {
         check_status(he_stream_synchronize(st), "synchronisation failed");
         std::memcpy(destination, out, bytes);

@@ -207,10 +207,14 @@ hipError_t launch_sum(const Tables &t, const uint64_t *const *cts, uint64_t *out
                       uint32_t count, hipStream_t s);
 hipError_t launch_multiply_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out, uint32_t limbs, uint32_t items,
                                uint32_t count, hipStream_t s);
-// (out01 [items][2][L][N], out2 [items][L][N]) = sum over chunks of (a - b)^2 for the pairs of ciphertexts in the
-// device pointer table pairs [items][chunks][2]
-hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out01, uint64_t *out2,
-                                  uint32_t L, uint32_t items, uint32_t chunks, hipStream_t s);
+// (out01 [items][2][L][N], out2 [items][L][N]) = sum of (a - b)^2 for the pairs of ciphertexts in the device pointer table pairs
+// [items][parts][count][2], the second part's sum (null: none) times X^(N/2); psi: the forward twiddles, N >= 512
+hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *psi, const uint64_t *const *pairs, uint64_t *out01, uint64_t *out2,
+                                  uint32_t L, uint32_t items, uint32_t parts, uint32_t count, hipStream_t s);
+// the same for the sum of a client's squared distances to all others: device pointer table cts [clients][chunks], two clients per item,
+// sums: (2 chunks + 3) L N words of scratch
+hipError_t launch_row_square_sums(const Tables &t, const uint64_t *psi, const uint64_t *const *cts, uint64_t *out01, uint64_t *out2,
+                                  uint64_t *sums, uint32_t L, uint32_t clients, uint32_t chunks, hipStream_t s);
 hipError_t launch_galois(const Tables &t, const uint64_t *in, uint64_t *out, uint32_t total_limbs, uint32_t elt,
                          hipStream_t s);
 
@@ -428,13 +432,13 @@ hipError_t launch_ckks_decode(const FftTables &t, const Tables &tab, const uint6
 // The same from plaintexts in NTT form that have been through their inverse blocks pass (inv: the inverse transform's
 // arguments, map = the limbs, in = the lazy words), real parts of the first `count` values only, to re [items][count] (device
 // or page-locked host memory): the inverse rows pass of all limbs and the composition are one kernel.  2^12 <= N <= 2^16,
-// at most 4 limbs.
+// at most 4 limbs.  both: (re, im) pairs [items][count][2] instead.
 hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int backend, uint32_t slots, double scale,
                                    const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items, double *re,
-                                   uint32_t count, hipStream_t s);
-// the forward transform of v and the real parts of the first `count` values, for the other cases
+                                   uint32_t count, bool both, hipStream_t s);
+// the forward transform of v and the real parts of (or both parts) the first `count` values, for the other cases
 hipError_t launch_ckks_fft_real(const FftTables &t, uint32_t slots, double2 *v, uint32_t items, double *re, uint32_t count,
-                                hipStream_t s);
+                                bool both, hipStream_t s);
 // only the composition of launch_ckks_decode
 hipError_t launch_ckks_compose(const FftTables &t, const Tables &tab, const uint64_t *res, uint32_t limbs, uint32_t slots,
                                double scale, const uint64_t *garner_inv, uint32_t garner_stride, double2 *v, uint32_t items,

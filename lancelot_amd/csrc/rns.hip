@@ -214,38 +214,6 @@ __global__ __launch_bounds__(kThreads) void decrypt_gather_kernel(const uint64_t
     out[o] = v;
 }
 
-struct PairSquareArgs {
-    const uint64_t *const *pairs;   // device array [items][chunks][2] of ciphertext pointers, each [2][L][N]
-    uint64_t *out01, *out2;         // [items][2][L][N] (d0, d1) and [items][L][N] (d2)
-    const uint64_t *moduli, *barrett;
-    uint32_t L, log_n, chunks;
-};
-
-// grid: (N / 256, L, items).  (d0, d1 | d2)[item] = sum over chunks of (a - b)^2 as a size-3 ciphertext, for the pair
-// (a, b) of every chunk: the subtraction, the tensor square and the accumulation of the lazily relinearised
-// squared distance in one pass over the inputs.  d2, the key-switch input, goes to a buffer of its own so that
-// (d0, d1) is a dense batch of size-2 ciphertexts.
-__global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(PairSquareArgs p) {
-    const uint32_t limb = blockIdx.y;
-    const uint64_t q = p.moduli[limb], r0 = p.barrett[2 * limb], r1 = p.barrett[2 * limb + 1];
-    const size_t poly = (size_t)p.L << p.log_n;
-    const size_t idx = ((size_t)limb << p.log_n) + blockIdx.x * kThreads + threadIdx.x;
-    const uint64_t *const *pair = p.pairs + (size_t)blockIdx.z * p.chunks * 2;
-    uint64_t d0 = 0, d1 = 0, d2 = 0;
-    for (uint32_t c = 0; c < p.chunks; c++) {
-        const uint64_t *a = pair[2 * c], *b = pair[2 * c + 1];
-        const uint64_t x0 = sub_mod(a[idx], b[idx], q), x1 = sub_mod(a[idx + poly], b[idx + poly], q);
-        d0 = add_mod(d0, mul_mod(x0, x0, q, r0, r1), q);
-        d2 = add_mod(d2, mul_mod(x1, x1, q, r0, r1), q);
-        const uint64_t m = mul_mod(x0, x1, q, r0, r1);
-        d1 = add_mod(d1, add_mod(m, m, q), q);
-    }
-    uint64_t *out = p.out01 + (size_t)blockIdx.z * 2 * poly;
-    out[idx] = d0;
-    out[idx + poly] = d1;
-    p.out2[(size_t)blockIdx.z * poly + idx] = d2;
-}
-
 // Sums of ciphertexts and of products of ciphertexts, each of `count` terms: what a row of a distance matrix or a masked sum of
 // updates is.  A call per term read and wrote the running sum each time (3 us of launch and latency a term at N = 2^16, two or
 // three limbs: 90 terms of ten row sums 290 us, 20 of two masked sums 110 us); here every term is read once, by all sums together.
@@ -307,6 +275,171 @@ __global__ __launch_bounds__(kThreads) void multiply_sum_kernel(SumArgs p) {
     for (int i = 0; i < 3; i++)
         *reinterpret_cast<Words2 *>(out + i * poly) = Words2{barrett128(s[i][0].lo, s[i][0].hi, q, r0, r1),
                                                              barrett128(s[i][1].lo, s[i][1].hi, q, r0, r1)};
+}
+
+// Squared distances for Krum, as size-3 ciphertexts (lazy relinearisation) whose third polynomial, the key switch's input, has a
+// buffer of its own, so that (d0, d1) is a dense batch of size-2 ciphertexts.
+// Two distances can share a ciphertext: the squared differences of real messages have real slots, and X^(N/2) multiplies every slot by
+// i, so that out = first + X^(N/2) second carries one sum in the real and one in the imaginary parts through relinearisation,
+// rescale and slot sum (all of them linear and compatible with i), at half the work per distance.
+struct SquareSumArgs {
+    const uint64_t *const *table;   // device table of ciphertexts [2][L][N]
+    uint64_t *sums;                 // row_square_kernel: what client_sums_kernel has left
+    uint64_t *out01, *out2;         // [items][2][L][N] (d0, d1) and [items][L][N] (d2)
+    const uint64_t *moduli, *barrett, *psi;
+    uint32_t L, log_n, count, parts;
+};
+
+// sums of products below 2^122, two words a thread: 64 of them fit into 128 bits
+struct SquareSums {
+    U128 s[3][2];
+    uint64_t q, r0, r1;
+    __device__ __forceinline__ SquareSums(const SquareSumArgs &p, uint32_t limb)
+        : q(scalar(p.moduli)[limb]), r0(scalar(p.barrett)[2 * limb]), r1(scalar(p.barrett)[2 * limb + 1]) {
+#pragma unroll
+        for (int i = 0; i < 3; i++) s[i][0] = s[i][1] = U128{0, 0};
+    }
+    __device__ __forceinline__ uint64_t reduced(int i, int j) const { return barrett128(s[i][j].lo, s[i][j].hi, q, r0, r1); }
+    // after term k, the number of products a term adds to one sum being at most two
+    __device__ __forceinline__ void relieve(uint32_t k) {
+        if (k % 16 != 15) return;
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < 2; j++) s[i][j] = U128{reduced(i, j), 0};
+    }
+    // d gains the sums, as they are or times X^(N/2): psi^(N/2) at the words of the NTT order's first half, its negative at
+    // those of the second
+    __device__ __forceinline__ void add_to(Words2 *d, const SquareSumArgs &p, uint32_t limb, bool imaginary, bool upper) const {
+        const Shoup w = scalar_shoup(p.psi, ((size_t)limb << p.log_n) + 1);
+#pragma unroll
+        for (int i = 0; i < 3; i++) {
+            uint64_t v[2];
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                v[j] = reduced(i, j);
+                if (!imaginary) continue;
+                v[j] = mul_shoup(v[j], w, q);
+                if (upper) v[j] = neg_mod(v[j], q);
+            }
+            d[i].x = add_mod(d[i].x, v[0], q);
+            d[i].y = add_mod(d[i].y, v[1], q);
+        }
+    }
+};
+
+__device__ __forceinline__ void store_squares(const SquareSumArgs &p, uint32_t item, size_t at, const Words2 *d) {
+    const size_t poly = (size_t)p.L << p.log_n;
+    uint64_t *out = p.out01 + (size_t)item * 2 * poly + at;
+    *reinterpret_cast<Words2 *>(out) = d[0];
+    *reinterpret_cast<Words2 *>(out + poly) = d[1];
+    *reinterpret_cast<Words2 *>(p.out2 + (size_t)item * poly + at) = d[2];
+}
+
+// grid: (N / 512, L, items).  Item = sum of (a - b)^2 over the `count` pairs of its row of the table [items][parts][count][2], plus X^(N/2) times that over its second
+// part's (null: no second part): the subtraction, the tensor square and the accumulation in one pass over the inputs.
+// What bounds it: integer multiplies, about 1000 instructions a thread (45 pairs of two chunks, three limbs of 2^16 words, two pairs an item
+// 85 us: one reduction per sum and half the outputs buy what the reductions of X^(N/2) cost; 90 us with a reduction per term and a
+// pair an item.  An order of workgroups in which the items that share a ciphertext meet on one XCD: the same 85).
+__global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(SquareSumArgs p) {
+    const uint32_t limb = blockIdx.y, j2 = 2 * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
+    const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + j2;
+    Words2 d[3] = {Words2{0, 0}, Words2{0, 0}, Words2{0, 0}};
+    for (uint32_t part = 0; part < p.parts; part++) {
+        const ScalarPtr pair = scalar(p.table) + ((size_t)item * p.parts + part) * p.count * 2;
+        if (part && !pair[0]) break;
+        SquareSums sums(p, limb);
+        const uint64_t q = sums.q;
+#pragma unroll 2
+        for (uint32_t k = 0; k < p.count; k++) {
+            const uint64_t *a = pair[2 * k] + at, *b = pair[2 * k + 1] + at;
+            const Words2 a0 = load_pair(a), a1 = load_pair(a + poly), b0 = load_pair(b), b1 = load_pair(b + poly);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                const uint64_t x0 = sub_mod(a0[j], b0[j], q), x1 = sub_mod(a1[j], b1[j], q);
+                mac128(sums.s[0][j], x0, x0);
+                mac128(sums.s[1][j], x0, add_mod(x1, x1, q));
+                mac128(sums.s[2][j], x1, x1);
+            }
+            sums.relieve(k);
+        }
+        sums.add_to(d, p, limb, part != 0, j2 >> (p.log_n - 1));
+    }
+    store_squares(p, item, at, d);
+}
+
+// The sum of a client's squared distances to all others, sum_j (x_i - x_j)^2 = x_i (n x_i - 2 S) + T with S = sum x_j and
+// T = sum x_j^2, word for word the same modulo q and n products instead of n (n - 1): client_sums_kernel leaves S of every chunk
+// [chunks][2][L][N] and T [3][L][N] (over all chunks), row_square_kernel forms two clients' sums per item.
+// 10 clients of two chunks: 22 + 37 us.
+// table [clients][chunks], count = clients, parts = chunks.  grid: (N / 512, L)
+__global__ __launch_bounds__(kThreads) void client_sums_kernel(SquareSumArgs p) {
+    const uint32_t limb = blockIdx.y;
+    const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + 2 * (blockIdx.x * kThreads + threadIdx.x);
+    SquareSums squares(p, limb);
+    const uint64_t q = squares.q;
+    for (uint32_t c = 0, term = 0; c < p.parts; c++) {
+        Words2 s0{0, 0}, s1{0, 0};
+#pragma unroll 4
+        for (uint32_t k = 0; k < p.count; k++, term++) {
+            const uint64_t *ct = scalar(p.table)[(size_t)k * p.parts + c] + at;
+            const Words2 x0 = load_pair(ct), x1 = load_pair(ct + poly);
+            s0 = Words2{add_mod(s0.x, x0.x, q), add_mod(s0.y, x0.y, q)};
+            s1 = Words2{add_mod(s1.x, x1.x, q), add_mod(s1.y, x1.y, q)};
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                mac128(squares.s[0][j], x0[j], x0[j]);
+                mac128(squares.s[1][j], x0[j], add_mod(x1[j], x1[j], q));
+                mac128(squares.s[2][j], x1[j], x1[j]);
+            }
+            squares.relieve(term);
+        }
+        uint64_t *out = p.sums + (size_t)c * 2 * poly + at;
+        *reinterpret_cast<Words2 *>(out) = s0;
+        *reinterpret_cast<Words2 *>(out + poly) = s1;
+    }
+#pragma unroll
+    for (int i = 0; i < 3; i++)
+        *reinterpret_cast<Words2 *>(p.sums + ((size_t)2 * p.parts + i) * poly + at) = Words2{squares.reduced(i, 0), squares.reduced(i, 1)};
+}
+
+// grid: (N / 512, L, items): item k holds client 2 k, and client 2 k + 1 (if there is one) times X^(N/2)
+__global__ __launch_bounds__(kThreads) void row_square_kernel(SquareSumArgs p) {
+    const uint32_t limb = blockIdx.y, j2 = 2 * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
+    const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + j2;
+    Words2 d[3] = {Words2{0, 0}, Words2{0, 0}, Words2{0, 0}};
+    for (uint32_t part = 0; part < 2; part++) {
+        const uint32_t client = 2 * item + part;
+        if (client >= p.count) break;
+        SquareSums sums(p, limb);
+        const uint64_t q = sums.q;
+        for (int i = 0; i < 3; i++) {
+            const Words2 t = load_pair(p.sums + ((size_t)2 * p.parts + i) * poly + at);
+            sums.s[i][0] = U128{t.x, 0};
+            sums.s[i][1] = U128{t.y, 0};
+        }
+#pragma unroll 2
+        for (uint32_t c = 0; c < p.parts; c++) {
+            const uint64_t *ct = scalar(p.table)[(size_t)client * p.parts + c] + at, *s = p.sums + (size_t)c * 2 * poly + at;
+            const Words2 x0 = load_pair(ct), x1 = load_pair(ct + poly), s0 = load_pair(s), s1 = load_pair(s + poly);
+#pragma unroll
+            for (int j = 0; j < 2; j++) {
+                // n x - 2 S
+                auto spread = [&](uint64_t x, uint64_t sum) {
+                    const uint64_t nx = mul_mod(x, p.count, q, sums.r0, sums.r1);
+                    return sub_mod(sub_mod(nx, sum, q), sum, q);
+                };
+                const uint64_t y0 = spread(x0[j], s0[j]), y1 = spread(x1[j], s1[j]);
+                mac128(sums.s[0][j], x0[j], y0);
+                mac128(sums.s[1][j], x0[j], y1);
+                mac128(sums.s[1][j], x1[j], y0);
+                mac128(sums.s[2][j], x1[j], y1);
+            }
+            sums.relieve(c);
+        }
+        sums.add_to(d, p, limb, part != 0, j2 >> (p.log_n - 1));
+    }
+    store_squares(p, item, at, d);
 }
 
 // grid: (N / 256, total limbs)
@@ -1296,11 +1429,22 @@ hipError_t launch_tensor_mxn(const Tables &t, const uint64_t *ct1, uint32_t s1, 
     return hipGetLastError();
 }
 
-hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *const *pairs, uint64_t *out01, uint64_t *out2,
-                                  uint32_t L, uint32_t items, uint32_t chunks, hipStream_t s) {
-    if (items == 0 || items > 65535 || chunks == 0 || L == 0) return hipErrorInvalidValue;
-    PairSquareArgs p{pairs, out01, out2, t.moduli, t.barrett, L, t.log_n, chunks};
-    hipLaunchKernelGGL(pair_square_sum_kernel, dim3((1u << t.log_n) / kThreads, L, items), dim3(kThreads), 0, s, p);
+hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *psi, const uint64_t *const *pairs, uint64_t *out01, uint64_t *out2,
+                                  uint32_t L, uint32_t items, uint32_t parts, uint32_t count, hipStream_t s) {
+    if (items == 0 || items > 65535 || count == 0 || L == 0 || parts == 0 || parts > 2) return hipErrorInvalidValue;
+    SquareSumArgs p{pairs, nullptr, out01, out2, t.moduli, t.barrett, psi, L, t.log_n, count, parts};
+    hipLaunchKernelGGL(pair_square_sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), L, items), dim3(kThreads), 0, s, p);
+    return hipGetLastError();
+}
+
+hipError_t launch_row_square_sums(const Tables &t, const uint64_t *psi, const uint64_t *const *cts, uint64_t *out01, uint64_t *out2,
+                                  uint64_t *sums, uint32_t L, uint32_t clients, uint32_t chunks, hipStream_t s) {
+    if (clients == 0 || clients > 2 * 65535 || chunks == 0 || L == 0) return hipErrorInvalidValue;
+    SquareSumArgs p{cts, sums, out01, out2, t.moduli, t.barrett, psi, L, t.log_n, clients, chunks};
+    const uint32_t wgs = (1u << t.log_n) / (2 * kThreads);
+    hipLaunchKernelGGL(client_sums_kernel, dim3(wgs, L), dim3(kThreads), 0, s, p);
+    if (hipError_t e = hipGetLastError()) return e;
+    hipLaunchKernelGGL(row_square_kernel, dim3(wgs, L, (clients + 1) / 2), dim3(kThreads), 0, s, p);
     return hipGetLastError();
 }
 

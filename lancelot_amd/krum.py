@@ -307,6 +307,10 @@ def _map_lanes(state: KrumState, items, fn):
     return out
 
 
+def _rounds(state: KrumState):
+    return rotate_sum_plan(int(math.log2(state.slots)), state.config)
+
+
 def all_pair_distances(state: KrumState, cts, enc):
     """enc[i][j] = enc[j][i] = pair_distance(i, j) for every i < j.  The pairs are independent, and at Lancelot's
     sizes (three or four limbs) one of them neither fills the GPU nor keeps one host thread's launch rate busy, so
@@ -315,8 +319,7 @@ def all_pair_distances(state: KrumState, cts, enc):
     pairs = [(i, j) for i in range(n_clients) for j in range(i + 1, n_clients)]
     if state.config.batched:
         c = state.cahel
-        rounds = rotate_sum_plan(int(math.log2(state.slots)), state.config)
-        out = c.pair_square_distances(state.context, cts, pairs, state.rlk, state.glk, rounds, state.config.scale,
+        out = c.pair_square_distances(state.context, cts, pairs, state.rlk, state.glk, _rounds(state), state.config.scale,
                                       state.config.sum_drop_levels)
         _sync(c)
     else:
@@ -348,6 +351,33 @@ def distance_matrix(state: KrumState, updates):
         dist[i, j] = dist[j, i] = value
     state.timings["decrypt"] += time.perf_counter() - t0
     return dist, enc
+
+
+def _unpacked(state: KrumState, cts, count: int):
+    """Slot 0 of `count` results that travel two to a ciphertext, in its real and its imaginary part."""
+    values = state.sk.decrypt_decode_complex_many(state.context, cts, state.slots, 1)[:, 0]
+    return np.stack([values.real, values.imag], axis=1).reshape(-1)[:count]
+
+
+def _packed_distance_matrix(state: KrumState, updates):
+    """distance_matrix's numbers without its ciphertexts: the squared differences have real slots, so two pairs share a ciphertext
+    through relinearisation, rescale, slot sum and decryption."""
+    c = state.cahel
+    cts = encrypt_updates(state, split_updates(updates, state.slots))
+    n_clients = len(updates)
+    pairs = [(i, j) for i in range(n_clients) for j in range(i + 1, n_clients)]
+    t0 = time.perf_counter()
+    packed = c.packed_pair_distances(state.context, cts, pairs, state.rlk, state.glk, _rounds(state), state.config.scale,
+                                     state.config.sum_drop_levels)
+    _sync(c)
+    t1 = time.perf_counter()
+    state.timings["evaluate"] += t1 - t0
+    dist = np.zeros((n_clients, n_clients))
+    if pairs:
+        for (i, j), value in zip(pairs, _unpacked(state, packed, len(pairs))):
+            dist[i, j] = dist[j, i] = value
+    state.timings["decrypt"] += time.perf_counter() - t1
+    return dist
 
 
 def _encrypt_constant(state: KrumState, value: float):
@@ -385,17 +415,23 @@ def decrypt_sort_mask(state: KrumState, enc):
     else:
         scores = _map_lanes(state, list(range(n_clients)), lambda i: state.encoder.decode_array(
             ctx, state.sk.decrypt(ctx, row_sum(i)), 1)[0])
+    mask, order = _mask(state, scores)
+    _sync(c)
+    state.timings["mask"] = state.timings.get("mask", 0.0) + time.perf_counter() - t0
+    return mask, order, np.asarray(scores)
+
+
+def _mask(state: KrumState, scores):
+    """The clients by ascending score, and the one-hot mask ciphertexts of that order."""
+    n_clients = len(scores)
     order = np.argsort(np.asarray(scores), kind="stable")
     if state.config.batched:
         constants = np.zeros((2, state.slots))
         constants[1] = 1.0
-        zero, one = state.encoder.encode_encrypt_many(ctx, state.pk, constants, state.config.scale)
+        zero, one = state.encoder.encode_encrypt_many(state.context, state.pk, constants, state.config.scale)
     else:
         zero, one = _encrypt_constant(state, 0.0), _encrypt_constant(state, 1.0)
-    mask = [[one if order[r] == k else zero for k in range(n_clients)] for r in range(n_clients)]
-    _sync(c)
-    state.timings["mask"] = state.timings.get("mask", 0.0) + time.perf_counter() - t0
-    return mask, order, np.asarray(scores)
+    return [[one if order[r] == k else zero for k in range(n_clients)] for r in range(n_clients)], order
 
 
 def mul_mask_weight(state: KrumState, cts, mask_row):
@@ -450,7 +486,7 @@ def gpu_krum(updates, config: KrumConfig | None = None, state: KrumState | None 
     for k in state.timings:
         state.timings[k] = 0.0
     t0 = time.perf_counter()
-    dist, _ = distance_matrix(state, updates)
+    dist = _packed_distance_matrix(state, updates) if state.config.batched else distance_matrix(state, updates)[0]
     total = time.perf_counter() - t0
     timings = dict(state.timings, total=total)
     return krum_select(dist), dist, timings
@@ -459,7 +495,8 @@ def gpu_krum(updates, config: KrumConfig | None = None, state: KrumState | None 
 def gpu_krum_aggregate(updates, config: KrumConfig | None = None, state: KrumState | None = None):
     """The full round of the reference's driver: encrypted distances, decrypt-sort-mask, and the masked sum of
     the encrypted updates, which is the update of the chosen client (byzantine_fl.py:517-525 followed by
-    :327-429).  Returns (chosen client index, aggregated weights of len(updates[0]), timings in seconds)."""
+    :327-429).  Batched, the encrypted distances are summed by rows before they are relinearised: relinearisation, rescale and slot sum are
+    linear, and only the row sums are decrypted.  Returns (chosen client index, aggregated weights of len(updates[0]), timings in seconds)."""
     state = state or gpu_init(config)
     for k in list(state.timings):
         state.timings[k] = 0.0
@@ -467,11 +504,20 @@ def gpu_krum_aggregate(updates, config: KrumConfig | None = None, state: KrumSta
     chunks = split_updates(updates, state.slots)
     cts = encrypt_updates(state, chunks)
     n_clients = len(updates)
-    enc = [[None] * n_clients for _ in range(n_clients)]
     t1 = time.perf_counter()
-    all_pair_distances(state, cts, enc)
-    state.timings["evaluate"] += time.perf_counter() - t1
-    mask, order, _ = decrypt_sort_mask(state, enc)
+    if state.config.batched and n_clients > 1:
+        packed = state.cahel.packed_distance_scores(state.context, cts, state.rlk, state.glk, _rounds(state), state.config.scale,
+                                                    state.config.sum_drop_levels)
+        _sync(state.cahel)
+        t2 = time.perf_counter()
+        state.timings["evaluate"] += t2 - t1
+        mask, order = _mask(state, _unpacked(state, packed, n_clients))
+        state.timings["mask"] = state.timings.get("mask", 0.0) + time.perf_counter() - t2
+    else:
+        enc = [[None] * n_clients for _ in range(n_clients)]
+        all_pair_distances(state, cts, enc)
+        state.timings["evaluate"] += time.perf_counter() - t1
+        mask, order, _ = decrypt_sort_mask(state, enc)
     weights = mul_mask_weight(state, cts, mask[0])
     total = time.perf_counter() - t0
     length = len(np.asarray(updates[0]).reshape(-1))
