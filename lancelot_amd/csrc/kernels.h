@@ -367,6 +367,7 @@ struct KsFuseArgs {
     // other, so that the key tile is read from memory by the first and from that XCD's L2 by the others.
     uint32_t items;
     size_t own_item_stride, fold_item_stride;
+    uint32_t ordered, order[16];   // filled in by the launcher: with `ordered`, byte i of order is the limb that stands in i's place
     EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form (last: of its lines a launch reads the first ones)
 };
 hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s);

@@ -21,6 +21,37 @@ namespace he {
 
 namespace {
 
+// The inverse rows pass of the source limb's tile: lazy words of the last block's layout become canonical coefficients in the first
+// block's.  (Behind the request of the forward twiddles: the exchanges' compiler barriers would hold that back until the inverse
+// pass has ended.)
+template <class T4>
+__device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a, const Job &job, uint64_t *lds, uint32_t t) {
+    constexpr int NB = T4::kBlocks;
+    const uint32_t st = job.src_table;
+    if ((a.pro_src_fp_mask >> st) & 1) {
+        const FpArith ar{fp_ctx(a, st).m, a.pro_itw_fp + ((size_t)st << a.log_n)};
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(s[j]);
+        FpArith::Tw tw[NB];
+        T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+        ar.reduce(v);
+        T4::template inverse<FpArith>(v, tw, ar, lds, t);
+        const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
+        const double ninv = cc[2];
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
+    } else {
+        const uint64_t q = scalar(a.moduli)[st];
+        const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
+        IntArith::Tw tw[NB];
+        T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+        T4::template inverse<IntArith>(s, tw, ar, lds, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) s[j] = reduce_2q(s[j], q);
+    }
+}
+
 // Rows pass.  The thread index is (wave, lane), the wave the same scalar in all its lanes, so that the twiddles of the
 // first two blocks come through scalar loads.
 // SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first; it leaves the
@@ -43,32 +74,8 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
     };
     uint64_t s[4];   // canonical coefficients of the source limb
     if constexpr (SRC_INTT) {
-        const uint32_t st = job.src_table;
-        if ((a.pro_src_fp_mask >> st) & 1) {
-            const FpArith ar{fp_ctx(a, st).m, a.pro_itw_fp + ((size_t)st << a.log_n)};
-            double v[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(job.src[glob(NB - 1, j)]);
-            FpArith::Tw tw[NB];
-            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-            ar.reduce(v);
-            T4::template inverse<FpArith>(v, tw, ar, lds, t);
-            const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
-            const double ninv = cc[2];
-#pragma unroll
-            for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
-        } else {
-            const uint64_t q = scalar(a.moduli)[st];
-            const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
-            uint64_t v[4];
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = job.src[glob(NB - 1, j)];
-            IntArith::Tw tw[NB];
-            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
-            T4::template inverse<IntArith>(v, tw, ar, lds, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) s[j] = reduce_2q(v[j], q);
-        }
+        for (int j = 0; j < 4; j++) s[j] = job.src[glob(NB - 1, j)];
     }
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) {
@@ -79,6 +86,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
         if (FWD) {
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) {
+                source_words<T4>(s, a, job, lds, t);
                 const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
@@ -109,6 +117,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
         if (FWD) {
             T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) {
+                source_words<T4>(s, a, job, lds, t);
                 const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
@@ -399,6 +408,34 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     if (add) add_w = scalar_shoup(x.p_mod_q, t);
     if (fold) fold_w = scalar_shoup(x.fold_w, 0);
     const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
+    // (the words of a limb that ModDown transforms back go through the inverse blocks pass before they leave the wave)
+    const bool invert = t >= x.inv_first;
+    A iar = ar;
+    if constexpr (FP)
+        iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
+    else
+        iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
+    typename A::Tw itw[SPLIT > 1 ? 4 : 1];
+    uint64_t c0[4], cl[4];
+    auto fetch_addends = [&](uint32_t r) {
+        if (add && r == 0) {
+            const uint64_t *src = x.add_c0 + (size_t)t * n;
+            if (x.own_galois) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+            } else {
+                load4(c0, src + at);
+            }
+        }
+        if (fold) load4(cl, x.fold_ct + item * x.fold_item_stride + ((size_t)r * x.L + t) * n + at);
+    };
+    if constexpr (SPLIT > 1) {
+        // (what the two waves that finish need after the sums have met is requested before the digits)
+        if (part < 2) {
+            if (invert) T4::template load_tw<A, 0>(itw, iar, (1u << (a.log_n - 8)) + blk, lane);
+            fetch_addends(part);
+        }
+    }
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = x.own + item * x.own_item_stride + (size_t)t * n;
@@ -456,35 +493,17 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         lds_barrier();
         if (part > 1) return;
     }
-    // (the words of a limb that ModDown transforms back go through the inverse blocks pass before they leave the wave)
-    const bool invert = t >= x.inv_first;
-    A iar = ar;
-    if (invert) {
-        if constexpr (FP)
-            iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
-        else
-            iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
-        T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
-    }
+    if (SPLIT == 1 && invert) T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         if (SPLIT > 1 && (uint32_t)r != part) continue;
         typename A::V v[4];
-        uint64_t c0[4], cl[4], parts[SPLIT][4];
+        uint64_t parts[SPLIT][4];
         if constexpr (SPLIT > 1) {
 #pragma unroll
             for (int i = 0; i < SPLIT; i++) load4(parts[i], sums_lds + (2 * i + r) * 256 + 4 * lane);
         }
-        if (add && r == 0) {
-            const uint64_t *src = x.add_c0 + (size_t)t * n;
-            if (x.own_galois) {
-#pragma unroll
-                for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
-            } else {
-                load4(c0, src + at);
-            }
-        }
-        if (fold) load4(cl, x.fold_ct + item * x.fold_item_stride + ((size_t)r * x.L + t) * n + at);
+        if (SPLIT == 1) fetch_addends(r);
         if constexpr (FP) {
             const FpMod m = ar.m;
 #pragma unroll
@@ -532,7 +551,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         }
         uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)r * LK * n + (size_t)t * n;
         if (invert) {
-            T4::template inverse<A>(v, tw, iar, nullptr, lane);
+            T4::template inverse<A>(v, SPLIT > 1 ? itw : tw, iar, nullptr, lane);
 #pragma unroll
             for (int j = 0; j < 4; j++) o[off + T4::word(0, lane, j)] = A::to_word(v[j]);
         } else {
@@ -581,7 +600,14 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
         if (SPLIT == 1 && pair >= pairs) return;
         pair = pairs - 1 - pair;
     }
-    const uint32_t t = pair >> lr, blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
+    uint32_t t = pair >> lr;
+    if (BE == NTT_BACKEND_MIXED && x.ordered) {
+        typedef const uint32_t __attribute__((address_space(4))) *Order;
+        const Order order = (Order)((const char __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr() +
+                                    sizeof(NttArgs) + offsetof(KsFuseArgs, order));
+        t = (order[t >> 2] >> (8 * (t & 3))) & 0xff;
+    }
+    const uint32_t blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
     if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, fp_arith(a, table), part, sums);
@@ -935,7 +961,8 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     return hipGetLastError();
 }
 
-hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s) {
+hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x_, int backend, hipStream_t s) {
+    KsFuseArgs x = x_;
     if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
     const uint32_t items = x.items ? x.items : 1;
     if (items > 1 && (x.own_galois || x.add_c0)) return hipErrorInvalidValue;
@@ -949,6 +976,19 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
     const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs * split + kInnerWaves - 1) / kInnerWaves;
     if (wgs > most_workgroups(64 * kInnerWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kInnerWaves);
+    // Mixed back end, more than a workgroup for every CU: the launch walks its limbs from the last to the first, so the integer
+    // limbs, whose waves issue three times the instructions, take the last places and a CU's second workgroup is one of the short
+    // ones (a rotation on [60, 40, 40, 60], two limbs of 2^16 words: 30.4 -> 29.1 us, in this kernel 9.8 -> 8.5)
+    x.ordered = backend == NTT_BACKEND_MIXED && items == 1 && wgs > 256 && x.L + x.K <= 64;
+    if (x.ordered) {
+        uint32_t at = x.L + x.K;
+        for (int fp = 0; fp < 2; fp++)
+            for (uint32_t t = x.L + x.K; t-- > 0;)
+                if ((int)((a.fp_mask >> (t < x.L ? t : x.size_q + (t - x.L))) & 1) == fp) {
+                    at--;
+                    x.order[at >> 2] |= t << (8 * (at & 3));
+                }
+    }
 #define HE_INNER(SPLIT)                                                                                           \
     do {                                                                                                          \
         if (backend == NTT_BACKEND_MIXED)                                                                         \

@@ -299,3 +299,27 @@ def test_hoisting_of_batches(oracle, capi, chain, local, logn, size_p, L, n_step
             w = np.stack([p.add(want[k][b], cts[k][b]) for b in range(2)]) if add_input else want[k]
             assert (got[k] == w).all(), (add_input, k)
     assert (din.numpy() == cts).all()
+
+
+@pytest.mark.parametrize("logn,bits,size_p,L", [(16, [60, 40, 40, 60], 1, 2), (16, [60, 40, 40, 60], 1, 3), (15, [40, 60, 50, 45, 30, 59, 60, 50], 2, 5),
+                                                (15, [60, 40, 50, 45, 30, 59, 60, 60], 2, 4), (14, [60, 40, 50, 45, 30, 59, 60, 60], 2, 6)])
+def test_key_switch_of_a_mixed_chain(oracle, capi, logn, bits, size_p, L):
+    """Rotation and key switch + rescale where the inner product takes its limbs in an order of their own (more than one workgroup for
+    every CU) and where it does not."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    rng = np.random.default_rng(logn + L)
+    lib, h = capi.lib(), ctx.he_handle()
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(p.size_q // p.size_p)]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    keys = capi.evk_array([d.ptr for d in dev])
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_workspace_words(h, L),))
+    ct, c = rand_limbs(p, rng, range(L), n_polys=2), rand_limbs(p, rng, range(L))
+    dct, dc = DeviceArray(capi, host=ct), DeviceArray(capi, host=c)
+    out, elt = DeviceArray(capi, shape=(2, L, p.n)), 25
+    capi.check(lib.he_rotate(h, L, dct.ptr, keys, out.ptr, elt, ws.ptr, None))
+    ks = p.key_switch(p.galois_ntt(ct[1], elt), host)
+    assert (out.numpy() == np.stack([p.add(p.galois_ntt(ct[0], elt), ks[0]), ks[1]])).all()
+    low = DeviceArray(capi, shape=(2, L - 1, p.n))
+    capi.check(lib.he_keyswitch_rescale(h, L, dc.ptr, keys, dct.ptr, low.ptr, 0, ws.ptr, None))
+    ks = p.key_switch(c, host)
+    assert (low.numpy() == p.rescale(np.stack([p.add(ct[b], ks[b]) for b in range(2)]))).all()
