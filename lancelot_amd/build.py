@@ -25,7 +25,9 @@ LIB = os.path.join(PKG, "libcahel_hip.so")
 PROBE_LIB = os.path.join(PKG, "libcahel_probe.so")
 
 HIP_FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-Wall", "-Wno-unused-function", "-ffp-contract=off",
-             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
+             "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+             # the first scalar arguments of a kernel arrive in registers (NttHead in csrc/kernels.h)
+             "-mllvm", "-amdgpu-kernarg-preload-count=14"]
 
 
 def _run(cmd):

@@ -169,16 +169,28 @@ void mx_record(std::vector<int32_t> &tab, uint32_t rows, uint32_t n_in, int term
 }
 
 template <typename T>
-int upload(he_context *ctx, T **dst, const T *src, size_t count) {
-    if (count == 0) {
-        *dst = nullptr;
-        return HE_OK;
-    }
+int reserve(he_context *ctx, T **dst, size_t count) {
     void *p = nullptr;
     HE_HIP(hipMalloc(&p, count * sizeof(T)));
     ctx->owned.push_back(p);
-    HE_HIP(hipMemcpy(p, src, count * sizeof(T), hipMemcpyHostToDevice));
     *dst = static_cast<T *>(p);
+    return HE_OK;
+}
+
+template <typename T>
+int put(T *dst, const T *src, size_t count) {
+    HE_HIP(hipMemcpy(dst, src, count * sizeof(T), hipMemcpyHostToDevice));
+    return HE_OK;
+}
+
+template <typename T>
+int upload(he_context *ctx, T **dst, const T *src, size_t count) {
+    *dst = nullptr;
+    if (count == 0) return HE_OK;
+    T *p = nullptr;
+    if (int rc = reserve(ctx, &p, count)) return rc;
+    if (int rc = put(p, src, count)) return rc;
+    *dst = p;
     return HE_OK;
 }
 
@@ -195,6 +207,7 @@ NttArgs base_args(const he_context *ctx, bool forward) {
     NttArgs a;
     memset(&a, 0, sizeof(a));
     a.tw = forward ? ctx->d_psi : ctx->d_ipsi;
+    a.size_qp = ctx->size_qp;
     a.tw_fp = forward ? ctx->d_psi_fp : ctx->d_ipsi_fp;
     a.fp_consts = ctx->d_fp_consts;
     a.moduli = ctx->d_moduli;
@@ -435,13 +448,27 @@ int he_context_create(const he_context_desc *d, he_context **out) {
         uint64_t *unused = nullptr;
         rc = static_scratch(&unused);
     }
-    if (!rc) rc = upload(ctx, &ctx->d_moduli, d->moduli, qp);
-    if (!rc) rc = upload(ctx, &ctx->d_barrett, d->barrett, 2 * qp);
-    if (!rc) rc = upload(ctx, &ctx->d_psi, d->psi, 2 * qp * n);
-    if (!rc) rc = upload(ctx, &ctx->d_ipsi, d->ipsi_div2, 2 * qp * n);
+    // the block of each direction (NttArgs::tw): twiddles of both back ends, then the primes' constants
+    if (!rc) rc = reserve(ctx, &ctx->d_psi, (3 * n + 7) * qp + 4 * (size_t)d->size_q);
+    if (!rc) rc = reserve(ctx, &ctx->d_ipsi, (3 * n + 7) * qp);
+    if (!rc) {
+        ctx->d_psi_fp = reinterpret_cast<double *>(ctx->d_psi + 2 * qp * n);
+        ctx->d_ipsi_fp = reinterpret_cast<double *>(ctx->d_ipsi + 2 * qp * n);
+        ctx->d_fp_consts = ctx->d_psi_fp + qp * n;
+        ctx->d_moduli = reinterpret_cast<uint64_t *>(ctx->d_fp_consts + 4 * qp);
+        ctx->d_barrett = ctx->d_moduli + qp;
+        rc = put(ctx->d_psi, d->psi, 2 * qp * n);
+        if (!rc) rc = put(ctx->d_ipsi, d->ipsi_div2, 2 * qp * n);
+        for (uint64_t *moduli : {ctx->d_moduli, reinterpret_cast<uint64_t *>(ctx->d_ipsi_fp + qp * n) + 4 * qp}) {
+            if (!rc) rc = put(moduli, d->moduli, qp);
+            if (!rc) rc = put(moduli + qp, d->barrett, 2 * qp);
+        }
+    }
     if (!rc && d->size_p) {
-        rc = upload(ctx, &ctx->d_p_mod_q, d->p_mod_q, 2 * (size_t)d->size_q);
-        if (!rc) rc = upload(ctx, &ctx->d_pinv_mod_q, d->pinv_mod_q, 2 * (size_t)d->size_q);
+        ctx->d_p_mod_q = ctx->d_barrett + 2 * qp;
+        ctx->d_pinv_mod_q = ctx->d_p_mod_q + 2 * (size_t)d->size_q;
+        rc = put(ctx->d_p_mod_q, d->p_mod_q, 2 * (size_t)d->size_q);
+        if (!rc) rc = put(ctx->d_pinv_mod_q, d->pinv_mod_q, 2 * (size_t)d->size_q);
         if (!rc) rc = upload(ctx, &ctx->d_phat_inv, d->phat_inv_mod_p, 2 * (size_t)d->size_p);
         ctx->h_phat_inv.assign(d->phat_inv_mod_p, d->phat_inv_mod_p + 2 * (size_t)d->size_p);
         if (!rc) rc = upload(ctx, &ctx->d_phat_mod_q, d->phat_mod_q, (size_t)d->size_q * d->size_p);
@@ -573,9 +600,10 @@ int he_context_create(const he_context_desc *d, he_context **out) {
                 if (!rc) rc = upload(ctx, &ctx->d_mx_last, single.data(), single.size());
             }
         }
-        if (!rc) rc = upload(ctx, &ctx->d_psi_fp, psi_fp.data(), psi_fp.size());
-        if (!rc) rc = upload(ctx, &ctx->d_ipsi_fp, ipsi_fp.data(), ipsi_fp.size());
-        if (!rc) rc = upload(ctx, &ctx->d_fp_consts, consts.data(), consts.size());
+        if (!rc) rc = put(ctx->d_psi_fp, psi_fp.data(), psi_fp.size());
+        if (!rc) rc = put(ctx->d_ipsi_fp, ipsi_fp.data(), ipsi_fp.size());
+        if (!rc) rc = put(ctx->d_fp_consts, consts.data(), consts.size());
+        if (!rc) rc = put(ctx->d_ipsi_fp + qp * n, consts.data(), consts.size());
     }
     if (!rc) {
         std::vector<uint32_t> iota(qp);
@@ -998,7 +1026,11 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     NttArgs fwd = base_args(ctx, true);
     fwd.in = out;
     fwd.out = out;
+    fwd.map = LimbMap{LK, 0, L, ctx->size_q};
     fwd.jobs = lv->d_modup_jobs;
+    fwd.listed = 1;
+    fwd.digit_limbs = ctx->size_p;
+    fwd.digits = lv->beta;
     fwd.n_jobs = lv->n_modup_jobs;
     fwd.groups = lv->d_modup_groups;
     fwd.n_groups = lv->n_modup_groups;
@@ -1008,7 +1040,6 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
         fwd.pro_mode = NTT_PRO_SOURCE_REDUCE;
         fwd.pro_src = ws;
         fwd.pro_item_stride = (size_t)L * n;
-        fwd.pro_lk = LK;
         if (source_intt) set_source_intt(ctx, fwd, inv_backend);
     }
     if (lazy) {
@@ -1206,7 +1237,6 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         x.own = src;
         x.own_galois = galois_elt;
         x.add_c0 = add_c0;
-        x.p_mod_q = ctx->d_p_mod_q;
         x.out = cx;
         x.L = L;
         x.K = ctx->size_p;
@@ -1214,7 +1244,6 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         x.size_qp = ctx->size_qp;
         x.beta = lv->beta;
         x.fold_ct = fold_ct;
-        x.fold_w = fold_w;
         x.inv_first = fold_ct ? L - 1 : L;
         x.items = items;
         x.own_item_stride = (size_t)c_item_stride * n;

@@ -69,7 +69,7 @@ enum : int {
     // forward prologue: input value = source limb mod q by integer Barrett reduction (the source may be any 64-bit
     // residue, also where the limb itself runs on the FP64 back end).  Map mode: the source of polynomial p is
     // pro_src + p * pro_poly_stride * N.  List mode: the source of job (data_limb, table) of item i is limb
-    // data_limb / pro_lk of pro_src + i * pro_item_stride: the base conversion of digits of one limb each (K = 1),
+    // data_limb / (L + K) of pro_src + i * pro_item_stride: the base conversion of digits of one limb each (K = 1),
     // whose matrix is all ones, done where the forward transform of the converted limb reads its input
     NTT_PRO_SOURCE_REDUCE = 8,
     // the same with the source limb still in the middle of its inverse transform: pro_src holds the words that the
@@ -77,7 +77,7 @@ enum : int {
     // rows pass on its tile of the source (the two passes work on the same rows x columns tile), without the round trip
     // of the coefficients through memory and without a launch.  Every job repeats its source's inverse rows pass, so
     // this is for launches of a few limbs, which are bound by the latency of one workgroup (ntt_source_intt_ok).
-    // Source of a job as for NTT_PRO_SOURCE_REDUCE; its prime is table data_limb / pro_lk in list mode, pro_src_table
+    // Source of a job as for NTT_PRO_SOURCE_REDUCE; its prime is table data_limb / (L + K) in list mode, pro_src_table
     // in map mode; bit t of pro_src_fp_mask says whether the blocks pass of table t ran on the FP64 back end.  The
     // inverse transform's scaling must be N^-1 alone (digits of one limb each).
     NTT_PRO_SOURCE_INTT_REDUCE = 9,
@@ -99,15 +99,22 @@ struct NttArgs {
     uint64_t *out;
     uint32_t in_poly_stride;
     uint32_t out_poly_stride;
-    const uint64_t *tw;       // [tables][N][2] (operand, Shoup quotient)
-    const double *tw_fp;      // [tables][N] twiddles as exact doubles for the FP64 back end (primes below 2^50)
-    const double *fp_consts;  // [tables][4]: q, 1/q, N^-1 mod q, (N^-1 mod q)/q
+    // One block per direction, with everything that a pass reads about its primes: [tables][N][2] (operand, Shoup quotient), then
+    // [tables][N] twiddles as exact doubles for the FP64 back end (primes below 2^50), [tables][4] of q, 1/q, N^-1 mod q and
+    // (N^-1 mod q)/q as doubles, [tables] moduli, [tables][2] Barrett ratios; forward also [size_q][2] Shoup pairs of P mod q and
+    // [size_q][2] of P^-1 mod q
+    const uint64_t *tw;
+    uint32_t size_qp;         // tables
+    const double *tw_fp;      // (into the block; set where a kernel starts)
+    const double *fp_consts;
     uint64_t fp_mask;         // bit t: table t has a prime below 2^50 (read by the mixed back end only)
     int one_pass;             // N <= 2^14, FP64 back end, plain transforms: one kernel with the limb resident in LDS
     const uint64_t *moduli;   // [tables]
     const uint64_t *barrett;  // [tables][2]
-    const LimbJob *jobs;      // explicit list (then in/out limbs are absolute, no prologue/epilogue)
-    uint32_t n_jobs;
+    const LimbJob *jobs;      // explicit list: the converted limbs of a ModUp, digit by digit, ascending (then in/out limbs are
+                              // absolute, no prologue/epilogue; map describes Ql u P)
+    uint32_t listed;          // (jobs is there)
+    uint32_t n_jobs, digit_limbs, digits;   // ... of so many digits of so many limbs (the last one may have fewer)
     const LimbGroup *groups;  // partition of `jobs` into runs with one table each, or nullptr
     uint32_t n_groups;
     uint32_t items;           // list mode: the whole list is applied to `items` buffers (0 = 1) ...
@@ -121,13 +128,12 @@ struct NttArgs {
     const uint64_t *pro_src;  // [poly][pro_poly_stride limbs], the first limb of each poly is the source
     uint32_t pro_poly_stride;
     size_t pro_item_stride;   // NTT_PRO_SOURCE_REDUCE in list mode: words between the sources of consecutive items
-    uint32_t pro_lk;          // ... and limbs per digit of the list's buffer (L + K)
     uint32_t pro_src_table;   // NTT_PRO_SOURCE_INTT_REDUCE in map mode: table of the source limb
     double pro_fix;           // NTT_PRO_ROUND: scale / slots
     uint32_t pro_log_slots;
     uint64_t pro_src_fp_mask; // NTT_PRO_SOURCE_INTT_REDUCE: tables whose inverse blocks pass left FP64 lazy words
-    const uint64_t *pro_itw;  // ... and the inverse transform's twiddle tables (laid out like tw and tw_fp)
-    const double *pro_itw_fp;
+    const uint64_t *pro_itw;  // ... and the inverse transform's block (laid out like tw)
+    const double *pro_itw_fp; // (into that block; set where a kernel starts)
     const uint64_t *epi_a;    // limb (poly, i) like `out`, with its own poly stride
     uint32_t epi_a_poly_stride;
     const uint64_t *epi_b;
@@ -145,6 +151,35 @@ struct NttArgs {
     uint64_t *epi_dst;        // destination of the forward epilogues
     uint32_t epi_dst_poly_stride;
 };
+
+// The arguments of a pass are few: a launch with more than 112 bytes of them costs the host 0.6 us more (3.3 against 2.7), and a
+// kernel waits for them.  NttHead is what it needs before it can ask for its first words, scalars in front of the others:
+// 14 registers that are loaded before a wave starts (the rest, lines of memory that no cache holds, arrives 700 to 1900 cycles
+// later; a launch of a few limbs takes 8,000 to 15,000 in all).  Behind it comes what the pass's mode needs, 56 bytes.
+struct NttHead {
+    const uint64_t *in;
+    uint64_t *out;
+    const uint64_t *tables;   // NttArgs::tw
+    uint64_t fp_mask;
+    uint32_t h0, h1, h2, h3, h4, h5;
+};
+#define HE_HEAD_PARAMS                                                                                                        \
+    const uint64_t *h_in, uint64_t *h_out, const uint64_t *h_tables, uint64_t h_fp_mask, uint32_t h0, uint32_t h1, uint32_t h2, \
+        uint32_t h3, uint32_t h4, uint32_t h5
+#define HE_HEAD_NAMES h_in, h_out, h_tables, h_fp_mask, h0, h1, h2, h3, h4, h5
+#define HE_HEAD_ARGS(h) h.in, h.out, h.tables, h.fp_mask, h.h0, h.h1, h.h2, h.h3, h.h4, h.h5
+
+// (limbs, tables and digits are at most 256; wgs: the launch's workgroups; extra: whatever else the kernel needs early)
+inline NttHead ntt_head(const NttArgs &a, uint32_t wgs, uint32_t extra) {
+    NttHead h{a.in, a.out, a.tw, a.fp_mask, 0, 0, 0, 0, wgs, extra};
+    const bool whole = a.map.split >= a.map.limbs;   // (then the caller's split and tail_first are any numbers)
+    const uint32_t split = whole ? a.map.limbs : a.map.split, tail = whole ? 0 : a.map.tail_first;
+    h.h0 = a.log_n | (a.jobs ? 1u << 5 : 0) | a.map.limbs << 6 | (a.size_qp - 1) << 24;
+    h.h1 = a.jobs ? a.n_jobs : a.in_poly_stride;
+    h.h2 = a.jobs ? (a.digit_limbs | a.digits << 16) : a.out_poly_stride;
+    h.h3 = a.map.first | split << 9 | tail << 18 | (uint32_t)a.pro_mode << 27;
+    return h;
+}
 
 // Forward transform: phase 1 (strided rows) then phase 2 (contiguous 256-blocks).  `a.in`/`a.out` and the
 // prologue describe phase 1's input; phase 2 runs in place on a.out unless an epilogue redirects it.
@@ -177,6 +212,7 @@ struct TensorFuse {
     uint64_t *d2;                // [L][N]: d2 in NTT form
     uint32_t L;
     int square;                  // ct2 is ignored, (d0, d1, d2) = (a0^2, 2 a0 a1, a1^2)
+    uint32_t wgs;                // filled in by the launcher
 };
 hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s);
 
@@ -351,13 +387,12 @@ struct KsFuseArgs {
     // optional (a rotation): out[0][t] += P * sigma(add_c0)[t] on the data limbs, with the same sigma; the ModDown that
     // follows divides by P, so the rotated c0 arrives in the result without a pass of its own
     const uint64_t *add_c0;   // [L][N], NTT form
-    const uint64_t *p_mod_q;  // [size_q][2] Shoup pairs of P mod q_i
     uint64_t *out;        // [2][L+K][N]
     uint32_t L, K, size_q, size_qp, beta;
     // optional: limb L-1 of the result becomes out * fold_w + fold_ct[k][L-1] (what the merged ModDown + rescale
-    // transforms back to coefficients); fold_ct = nullptr leaves the inner product as it is
+    // transforms back to coefficients), fold_w = P^-1 mod q_{L-1}; nullptr leaves the inner product as it is.  Not together with
+    // add_c0.
     const uint64_t *fold_ct;  // [2][L][N]
-    const uint64_t *fold_w;   // Shoup pair of P^-1 mod q_{L-1}
     // limbs t >= inv_first leave as the lazy words of their inverse blocks pass (what ModDown transforms back; the launch's
     // NttArgs::pro_itw / pro_itw_fp hold the inverse tables); L + K: none
     uint32_t inv_first;
@@ -367,8 +402,7 @@ struct KsFuseArgs {
     // other, so that the key tile is read from memory by the first and from that XCD's L2 by the others.
     uint32_t items;
     size_t own_item_stride, fold_item_stride;
-    uint32_t ordered, order[16];   // filled in by the launcher: with `ordered`, byte i of order is the limb that stands in i's place
-    EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form (last: of its lines a launch reads the first ones)
+    EvkPtrs evk;          // per digit: [2][size_qp][N], NTT form
 };
 hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, hipStream_t s);
 

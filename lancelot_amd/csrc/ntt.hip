@@ -141,11 +141,14 @@ __global__ __launch_bounds__((1 << LOGN) / 16) void ntt_limb_fp_kernel(NttArgs a
 // Six limbs of 50 bits, forward and inverse: 2^10 4.35 -> 3.76 and 4.76 -> 3.90 us, 2^12 5.36 -> 5.11 and 5.85 -> 5.36; of 60 bits
 // at 2^10, against rows pass and blocks pass, 6.6 -> 3.8 us.
 template <int LOGN, bool FWD, int BE>
-__global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(NttArgs a) {
+__global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARAMS, const uint64_t *w) {
     using T4 = Tile4<LOGN, LOGN>;
     constexpr int NB = T4::kBlocks;
     __shared__ uint64_t lds[(1 << LOGN) + (1 << (LOGN - 4))];
-    touch_arguments<sizeof(NttArgs)>();
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    a.w = w;
+    a.epi_mode = h5;
     const Job job = decode_job(a, blockIdx.x);
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
@@ -213,15 +216,16 @@ template <bool FWD>
 hipError_t launch_limb(const NttArgs &a, uint32_t n_jobs, int backend, hipStream_t s) {
     if (n_jobs > most_workgroups((1u << a.log_n) / 4)) return hipErrorInvalidValue;
     if (limb4(a, backend, n_jobs)) {
+        const NttHead head = ntt_head(a, n_jobs, (uint32_t)a.epi_mode);
 #define HE_LIMB4(LOGN)                                                                                                                  \
     do {                                                                                                                                \
         const dim3 block((1u << LOGN) / 4);                                                                                             \
         if (backend == NTT_BACKEND_MIXED)                                                                                               \
-            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_MIXED>), dim3(n_jobs), block, 0, s, a);                         \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_MIXED>), dim3(n_jobs), block, 0, s, HE_HEAD_ARGS(head), a.w);                         \
         else if (backend)                                                                                                               \
-            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_FP>), dim3(n_jobs), block, 0, s, a);                            \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_FP>), dim3(n_jobs), block, 0, s, HE_HEAD_ARGS(head), a.w);                            \
         else                                                                                                                            \
-            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_INT>), dim3(n_jobs), block, 0, s, a);                           \
+            hipLaunchKernelGGL((ntt_limb4_kernel<LOGN, FWD, NTT_BACKEND_INT>), dim3(n_jobs), block, 0, s, HE_HEAD_ARGS(head), a.w);                           \
     } while (0)
         if (a.log_n == 10)
             HE_LIMB4(10);
@@ -261,7 +265,7 @@ constexpr uint32_t kFuseWords = 1u << kFuseLog;
 
 struct BconvRowsK {
     BconvRows b;
-    uint32_t compute_groups, copy_groups, rows_per;
+    uint32_t compute_groups, copy_groups, rows_per, wgs;
 };
 
 // see the matrix-core kernel below
@@ -334,7 +338,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
     constexpr int LOGC = 3;
     constexpr uint32_t tiles_per_limb = 32;
 
-    uint32_t lb = logical_block();
+    uint32_t lb = logical_block(p.wgs);
     const uint32_t groups = p.compute_groups + p.copy_groups;
     const uint32_t grp = lb % groups;
     lb /= groups;
@@ -605,11 +609,12 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
             }
         }
     }
-    BconvRowsK p{b, (rows + target - 1) / target, 0, target};
+    BconvRowsK p{b, (rows + target - 1) / target, 0, target, 0};
     p.copy_groups = b.copy_base ? (b.max_copy + target - 1) / target : 0;
     const uint64_t wgs = (uint64_t)b.n_units * items * tiles * (p.compute_groups + p.copy_groups);
     if (wgs > most_workgroups(256)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs);
+    p.wgs = (uint32_t)wgs;
     if (mx) {
         if (b.mdr)
             hipLaunchKernelGGL(bconv_rows_mx_kernel<true>, grid, dim3(256), 0, s, a, p);

@@ -165,7 +165,7 @@ struct ConvInt {
 // arithmetic the limb is transformed
 template <int LD, bool FP, int NIN, bool MDR>
 __global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(FP || NIN <= 4 ? 4 : 2)))
-void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per) {
+void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per, uint32_t wgs) {
     using T4 = Tile4<kTileLog, LD>;
     constexpr int LOGC = kTileLog - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
@@ -173,7 +173,7 @@ void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_
     __shared__ uint64_t lds[2][(1 << kTileLog) + (1 << (kTileLog - 4))];
     touch_arguments<sizeof(NttArgs) + sizeof(BconvRows)>();
     const size_t n = (size_t)1 << a.log_n;
-    uint32_t lb = logical_block();
+    uint32_t lb = logical_block(wgs);
     const uint32_t groups = compute_groups + copy_groups, grp = lb % groups;
     lb /= groups;
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC, uidx = lb / tiles_per_limb, item = uidx / b.n_units;
@@ -258,7 +258,7 @@ hipError_t launch_nin(const NttArgs &a, const BconvRows &b, uint32_t compute_gro
 #define HE_CASE(LD)                                                                                                          \
     case LD:                                                                                                                 \
         hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR>), grid, dim3(1 << (kTileLog - 2)), 0, s, a, b, compute_groups,   \
-                           copy_groups, rows_per);                                                                           \
+                           copy_groups, rows_per, grid.x);                                                                           \
         break;
         HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
 #undef HE_CASE

@@ -42,10 +42,44 @@ __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(
 
 // Workgroups are dealt round-robin to the 8 XCDs; give every XCD a contiguous range of logical ids so
 // that the tiles of one limb (which share a twiddle table) meet in one L2.
-__device__ __forceinline__ uint32_t logical_block() {
-    uint32_t b = blockIdx.x, n = gridDim.x;
+// n: workgroups of the launch
+__device__ __forceinline__ uint32_t logical_block(uint32_t n) {
+    const uint32_t b = blockIdx.x;
     if (n % 8 == 0) return (b % 8) * (n / 8) + b / 8;
     return b;
+}
+
+// the pointers into a direction's block (NttArgs::tw)
+__device__ __forceinline__ const double *block_fp(const uint64_t *block, uint32_t qp, uint32_t log_n) {
+    return reinterpret_cast<const double *>(block + ((size_t)(2 * qp) << log_n));
+}
+
+// the fields that came as scalar arguments
+__device__ __forceinline__ void set_head(NttArgs &a, HE_HEAD_PARAMS) {
+    const uint32_t qp = (h0 >> 24) + 1;
+    a.in = h_in;
+    a.out = h_out;
+    a.tw = h_tables;
+    a.fp_mask = h_fp_mask;
+    a.log_n = h0 & 31;
+    a.size_qp = qp;
+    a.tw_fp = block_fp(h_tables, qp, a.log_n);
+    a.fp_consts = a.tw_fp + ((size_t)qp << a.log_n);
+    a.moduli = reinterpret_cast<const uint64_t *>(a.fp_consts + 4 * qp);
+    a.barrett = a.moduli + qp;
+    a.map = LimbMap{(h0 >> 6) & 0x3ff, h3 & 0x1ff, (h3 >> 9) & 0x1ff, (h3 >> 18) & 0x1ff};
+    a.pro_mode = h3 >> 27;
+    a.listed = (h0 >> 5) & 1;
+    a.in_poly_stride = a.n_jobs = h1;
+    a.out_poly_stride = h2;
+    a.digit_limbs = h2 & 0xffff;
+    a.digits = h2 >> 16;
+    a.batch = a.first_job = h5;
+}
+
+__device__ __forceinline__ void set_inverse_block(NttArgs &a, const uint64_t *block) {
+    a.pro_itw = block;
+    a.pro_itw_fp = block_fp(block, a.size_qp, a.log_n);
 }
 
 struct Job {
@@ -58,29 +92,55 @@ struct Job {
     uint32_t src_table;    // NTT_PRO_SOURCE_INTT_REDUCE: its prime
 };
 
+// LOOKUP (blocks pass): entries of the list as it is stored, ordered by their primes
+template <bool SRC = false, bool LOOKUP = false>
 __device__ __forceinline__ Job decode_job(const NttArgs &a, uint32_t job) {
     Job j;
     const size_t n = (size_t)1 << a.log_n;
-    if (a.jobs) {
+    if (LOOKUP && a.listed) {
         // job = item * n_jobs + entry of the list
         const uint32_t item = job / a.n_jobs;
-        LimbJob lj = a.jobs[job - item * a.n_jobs];
-        j.in = a.in + item * a.item_stride + (size_t)lj.data_limb * n;
+        const LimbJob lj = a.jobs[job - item * a.n_jobs];
+        j.in = nullptr;
         j.out = a.out + item * a.item_stride + (size_t)lj.data_limb * n;
         j.table = lj.table;
         j.poly = 0;
         j.limb = 0;
+        j.src = nullptr;
+        j.src_table = 0;
+    } else if (a.listed) {
+        // job = item * n_jobs + entry of the list, which is worked out (looked up, the entry was a second trip to memory in front of the
+        // words)
+        const uint32_t item = job / a.n_jobs, r = job - item * a.n_jobs, per = a.map.limbs - a.digit_limbs;
+        uint32_t d = r / per;
+        d = d < a.digits ? d : a.digits - 1;
+        const uint32_t own0 = d * a.digit_limbs, t0 = r - d * per;
+        const uint32_t own = own0 + a.digit_limbs < a.map.split ? a.digit_limbs : a.map.split - own0;
+        const uint32_t t = t0 < own0 ? t0 : t0 + own, data_limb = d * a.map.limbs + t;
         const bool sourced = a.pro_mode == NTT_PRO_SOURCE_REDUCE || a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE;
-        j.src_table = sourced ? lj.data_limb / a.pro_lk : 0;
-        j.src = sourced ? a.pro_src + item * a.pro_item_stride + (size_t)j.src_table * n : nullptr;
+        j.in = sourced ? nullptr : a.in + (size_t)data_limb * n;
+        j.out = a.out + (size_t)data_limb * n;
+        j.table = map_table(a.map, t);
+        j.poly = 0;
+        j.limb = 0;
+        j.src_table = sourced ? d : 0;
+        j.src = sourced ? a.in + (size_t)d * n : nullptr;
+        if (item) {
+            if (sourced)
+                j.src += item * a.pro_item_stride;
+            else
+                j.in += item * a.item_stride;
+            j.out += item * a.item_stride;
+        }
     } else {
         j.poly = job / a.map.limbs;
         j.limb = job % a.map.limbs;
         j.in = a.in ? a.in + ((size_t)j.poly * a.in_poly_stride + j.limb) * n : nullptr;
         j.out = a.out + ((size_t)j.poly * a.out_poly_stride + j.limb) * n;
         j.table = map_table(a.map, j.limb);
-        j.src = a.pro_src + ((size_t)j.poly * a.pro_poly_stride << a.log_n);
-        j.src_table = a.pro_src_table;
+        // (rows pass: a prologue that has one source limb for every limb of a polynomial finds it, and its stride, in place of the input)
+        j.src = a.in + ((size_t)j.poly * a.in_poly_stride << a.log_n);
+        j.src_table = SRC ? a.pro_src_table : 0;
     }
     return j;
 }
@@ -115,11 +175,11 @@ __device__ __forceinline__ double inverse_scale(const NttArgs &a, const Job &job
 
 // coefficient at `at` of polynomial job.poly of an encoding, rounded (NTT_PRO_ROUND)
 __device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Job &job, uint32_t at) {
-    const uint32_t half = 1u << (a.log_n - 1), log_gap = a.log_n - 1 - a.pro_log_slots;
+    const uint32_t log_slots = a.in_poly_stride, half = 1u << (a.log_n - 1), log_gap = a.log_n - 1 - log_slots;
     const uint32_t k = at & (half - 1);
     if (k & ((1u << log_gap) - 1)) return 0.0;
-    const double *v = reinterpret_cast<const double *>(a.pro_src) + ((size_t)job.poly << (a.pro_log_slots + 1));
-    const uint32_t slot = __brev(k >> log_gap) >> (32 - a.pro_log_slots);
+    const double *v = reinterpret_cast<const double *>(a.in) + ((size_t)job.poly << (log_slots + 1));
+    const uint32_t slot = __brev(k >> log_gap) >> (32 - log_slots);
     return round(v[2 * slot + (at >= half ? 1 : 0)] * a.pro_fix);
 }
 
@@ -149,7 +209,7 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
     }
     if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE) {
         // one source limb for every limb: it may exceed this limb's prime, so reduce first
-        const uint64_t *src = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
+        const uint64_t *src = job.src;
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(src[glob(j)]);
         return true;
@@ -159,7 +219,7 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(barrett64(job.src[glob(j)], q, r1));
     } else if (a.pro_mode == NTT_PRO_SMALL) {
-        const int8_t *src = reinterpret_cast<const int8_t *>(a.pro_src) + ((size_t)job.poly << a.log_n);
+        const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = (double)src[glob(j)];
     } else if (a.pro_mode == NTT_PRO_ROUND) {
@@ -193,11 +253,11 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
         }
     } else if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE || a.pro_mode == NTT_PRO_SOURCE_REDUCE) {
         const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
-        const uint64_t *src = a.pro_mode == NTT_PRO_SOURCE_REDUCE ? job.src : a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
+        const uint64_t *src = job.src;
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = barrett64(src[glob(j)], q, r1);
     } else if (a.pro_mode == NTT_PRO_SMALL) {
-        const int8_t *src = reinterpret_cast<const int8_t *>(a.pro_src) + ((size_t)job.poly << a.log_n);
+        const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll
         for (int j = 0; j < W; j++) {
             const int64_t x = src[glob(j)];

@@ -11,6 +11,7 @@
 // (60 bits).
 #include <hip/hip_runtime.h>
 
+#include <cstring>
 #include <type_traits>
 
 #include "kernels.h"
@@ -20,6 +21,56 @@
 namespace he {
 
 namespace {
+
+// What a rows pass's mode needs behind NttHead.
+struct RowsExtra {
+    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_INTT_REDUCE: pro_itw; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2, pro_w
+    uint64_t u0, u1, mask;          // list: item_stride, pro_item_stride; NTT_PRO_ROUND: pro_fix; NTT_PRO_MODDOWN_RESCALE: strides, pro_last and pro_k1
+    uint32_t w0;                    // inverse: epi_mode; NTT_PRO_SOURCE_INTT_REDUCE in map mode: pro_src_table
+};
+
+RowsExtra rows_extra(const NttArgs &a, bool fwd) {
+    RowsExtra e{nullptr, nullptr, nullptr, a.item_stride, a.pro_item_stride, a.pro_src_fp_mask, 0};
+    if (!fwd) {
+        e.p0 = a.w;
+        e.w0 = (uint32_t)a.epi_mode;
+    } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
+        e.p0 = a.pro_itw;
+        e.w0 = a.pro_src_table;
+    } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
+        e.p0 = a.pro_src;
+        e.p1 = a.pro_src2;
+        e.p2 = a.pro_w;
+        e.u0 = a.pro_poly_stride | (uint64_t)a.pro2_poly_stride << 32;
+        e.u1 = a.pro_last | (uint64_t)a.pro_k1 << 32;
+    } else if (a.pro_mode == NTT_PRO_ROUND) {
+        memcpy(&e.u0, &a.pro_fix, sizeof(e.u0));
+    }
+    return e;
+}
+
+template <bool FWD, bool SRC_INTT, bool MDR>
+__device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
+    a.epi_mode = FWD ? NTT_PLAIN : (int)e.w0;
+    a.w = FWD ? nullptr : e.p0;
+    a.item_stride = e.u0;
+    a.pro_item_stride = e.u1;
+    a.pro_fix = __longlong_as_double((long long)e.u0);
+    if constexpr (SRC_INTT) {
+        set_inverse_block(a, e.p0);
+        a.pro_src_fp_mask = e.mask;
+        a.pro_src_table = e.w0;
+    }
+    if constexpr (MDR) {
+        a.pro_src = e.p0;
+        a.pro_src2 = e.p1;
+        a.pro_w = e.p2;
+        a.pro_poly_stride = (uint32_t)e.u0;
+        a.pro2_poly_stride = (uint32_t)(e.u0 >> 32);
+        a.pro_last = (uint32_t)e.u1;
+        a.pro_k1 = (int)(e.u1 >> 32);
+    }
+}
 
 // The inverse rows pass of the source limb's tile: lazy words of the last block's layout become canonical coefficients in the first
 // block's.  (Behind the request of the forward twiddles: the exchanges' compiler barriers would hold that back until the inverse
@@ -58,14 +109,16 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
 // coefficients where the forward pass takes them from.
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
 template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B>
-__global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
+__global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, RowsExtra x) {
+    NttArgs a;
     using T4 = Tile4<B, LD>;
     constexpr int LOGC = B - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
     __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
-    touch_arguments<sizeof(NttArgs)>();
-    const uint32_t lb = logical_block();
-    const Job job = decode_job(a, a.first_job + lb / tiles_per_limb);
+    set_head(a, HE_HEAD_NAMES);
+    set_extra<FWD, SRC_INTT, MDR>(a, x);
+    const uint32_t lb = logical_block(h4);
+    const Job job = decode_job<SRC_INTT>(a, a.first_job + lb / tiles_per_limb);
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     auto glob = [&](int k, int j) {
@@ -148,6 +201,38 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(NttArgs a) {
 
 constexpr int kBlockWaves = 2;   // 256-word blocks of a workgroup, one per wave
 
+// What a blocks pass's mode needs behind NttHead: the operands of an epilogue, or the list.
+struct BlocksExtra {
+    const void *p0, *p1, *p2, *p3, *p4;   // epi_a, epi_b, epi_dst, w, pro_w; or jobs, groups, item_stride
+    uint32_t u0, u1, u2, n_polys;         // strides of epi_a and epi_b, of epi_dst and epi_mode, epi_b_mask; or n_groups, items; in_galois
+};
+
+BlocksExtra blocks_extra(const NttArgs &a, bool fwd) {
+    if (a.jobs) return BlocksExtra{a.jobs, a.groups, reinterpret_cast<const void *>(a.item_stride), nullptr, nullptr, a.n_groups, a.items, 0, a.n_polys};
+    return BlocksExtra{a.epi_a, a.epi_b, a.epi_dst, a.w, a.pro_w, a.epi_a_poly_stride | a.epi_b_poly_stride << 16,
+                       a.epi_dst_poly_stride | (uint32_t)a.epi_mode << 16, fwd ? a.epi_b_mask : a.in_galois, a.n_polys};
+}
+
+__device__ __forceinline__ void set_extra(NttArgs &a, const BlocksExtra &e, bool fwd) {
+    a.n_polys = e.n_polys;
+    a.in_galois = fwd ? 0 : e.u2;
+    a.jobs = static_cast<const LimbJob *>(e.p0);
+    a.groups = static_cast<const LimbGroup *>(e.p1);
+    a.item_stride = reinterpret_cast<size_t>(e.p2);
+    a.n_groups = e.u0;
+    a.items = e.u1;
+    a.epi_a = static_cast<const uint64_t *>(e.p0);
+    a.epi_b = static_cast<const uint64_t *>(e.p1);
+    a.epi_dst = static_cast<uint64_t *>(const_cast<void *>(e.p2));
+    a.w = static_cast<const uint64_t *>(e.p3);
+    a.pro_w = static_cast<const uint64_t *>(e.p4);
+    a.epi_a_poly_stride = e.u0 & 0xffff;
+    a.epi_b_poly_stride = e.u0 >> 16;
+    a.epi_dst_poly_stride = e.u1 & 0xffff;
+    a.epi_mode = e.u1 >> 16;
+    a.epi_b_mask = e.u2;
+}
+
 // Operands of a fused forward epilogue at the lane's four consecutive words, and its constants
 struct EpiOperands {
     bool fma, add;
@@ -178,7 +263,7 @@ struct BlockUnit {
 };
 
 __device__ __forceinline__ BlockUnit block_unit(const NttArgs &a, uint32_t u) {
-    if (a.jobs) {
+    if (a.listed) {
         const uint32_t items = a.items ? a.items : 1;
         uint32_t first, per, chunk;
         if (a.groups) {
@@ -230,7 +315,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
         if (FWD && EPI) e = load_epilogue(a, job, off + 4 * lane);
         Job next = job;
         if (more) {
-            next = decode_job(a, unit.job(b + 1));
+            next = decode_job<false, true>(a, unit.job(b + 1));
             fetch(nx, next);
         }
         typename A::V v[4];
@@ -305,14 +390,16 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
 }
 
 template <bool FWD, bool EPI, bool LOOP, int BE>
-__global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(NttArgs a) {
-    touch_arguments<sizeof(NttArgs)>();
+__global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PARAMS, BlocksExtra x) {
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    set_extra(a, x, FWD);
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block() * kBlockWaves + w;   // (a limb has an even number of blocks)
+    const uint32_t id = logical_block(h4) * kBlockWaves + w;   // (a limb has an even number of blocks)
     const BlockUnit unit = block_unit(a, id >> lr);
     const uint32_t blk = id & ((1u << lr) - 1);
-    const Job job = decode_job(a, unit.job(0));
+    const Job job = decode_job<false, true>(a, unit.job(0));
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane);
     if constexpr (BE != NTT_BACKEND_FP) {
@@ -360,6 +447,29 @@ struct IntSums {
     }
 };
 
+// What the inner product needs behind NttHead: up to three digits of one item, or any number of both.
+struct InnerFew {
+    static constexpr uint32_t kDigits = 3;
+    const uint64_t *itw, *addend;   // the inverse direction's block; add_c0 or fold_ct
+    uint64_t *out;
+    uint32_t own_galois, inv_first;  // inv_first: bit 16: addend is add_c0, bit 17: it is fold_ct
+    const uint64_t *evk[kDigits];
+    __device__ __forceinline__ size_t item_stride() const { return 0; }
+    __device__ __forceinline__ size_t own_item_stride() const { return 0; }
+    __device__ __forceinline__ size_t fold_item_stride() const { return 0; }
+};
+struct InnerMany {
+    static constexpr uint32_t kDigits = kMaxDigits;
+    const uint64_t *itw, *addend;
+    uint64_t *out;
+    uint32_t own_galois, inv_first;
+    size_t strides[3];
+    const uint64_t *evk[kDigits];
+    __device__ __forceinline__ size_t item_stride() const { return strides[0]; }
+    __device__ __forceinline__ size_t own_item_stride() const { return strides[1]; }
+    __device__ __forceinline__ size_t fold_item_stride() const { return strides[2]; }
+};
+
 // Blocks pass of ModUp's forward transform fused with the key-switch inner product: a wave owns one block of 256 words of limb t of
 // Ql u P, takes it through the last 8 stages for every digit in turn and multiplies it by both key polynomials; the digit
 // that owns limb t contributes the input itself.  The transformed limbs never reach memory, and the limbs of the sum that
@@ -368,16 +478,17 @@ struct IntSums {
 // FP64 kernel from 96 registers to 120).
 // SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
 // and waves 0 and 1 finish one polynomial each.
-template <int SPLIT, class A>
-__device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &x, uint32_t t, uint32_t table, uint32_t blk,
-                                            uint32_t item, uint32_t lane, const A &ar, uint32_t part,
+template <int SPLIT, class A, class X>
+__device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32_t L, uint32_t LK, uint32_t beta, uint32_t t,
+                                            uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
                                             uint64_t *sums_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
-    const uint32_t LK = x.L + x.K, own = t < x.L ? t / x.K : 0xffffffffu;
-    const uint64_t *lazy = a.out + item * a.item_stride + (size_t)t * n + off;   // words left by the rows pass, digit 0
-    const size_t digit_stride = (size_t)LK * n, key_off = (size_t)table * n + at, key_poly = (size_t)x.size_qp * n;
+    const uint32_t own = t < L ? t / (LK - L) : 0xffffffffu;
+    const uint64_t *lazy = a.out + (size_t)t * n + off;   // words left by the rows pass, digit 0
+    if (item) lazy += item * x.item_stride();
+    const size_t digit_stride = (size_t)LK * n, key_off = (size_t)table * n + at, key_poly = (size_t)a.size_qp * n;
     // the digits to transform: all but the own one, the own one counting as the first for the deal
     auto skip_own = [&](uint32_t d) { return d == own ? d + 1 : d; };
     auto next_digit = [&](uint32_t d) {
@@ -390,8 +501,8 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
     };
     auto keys = [&](uint64_t (*k)[4], uint32_t d) {
-        load4(k[0], x.evk.p[d] + key_off);
-        load4(k[1], x.evk.p[d] + key_poly + key_off);
+        load4(k[0], x.evk[d] + key_off);
+        load4(k[1], x.evk[d] + key_poly + key_off);
     };
     typename A::Tw tw[4];
     uint64_t nx[4];
@@ -400,16 +511,17 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         const uint32_t skip = own == 0xffffffffu ? part : (part + SPLIT - 1) % SPLIT;
         for (uint32_t i = 0; i < skip; i++) d = skip_own(d + 1);
     }
-    if (d < x.beta) fetch(nx, d);
+    if (d < beta) fetch(nx, d);
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
-    const bool add = x.add_c0 && t < x.L;                 // polynomial 0 gains P sigma(c0) (a rotation)
-    const bool fold = x.fold_ct && t == x.L - 1;
+    const bool add = (x.inv_first >> 16 & 1) && t < L;                 // polynomial 0 gains P sigma(c0) (a rotation)
+    const bool fold = (x.inv_first >> 17 & 1) && t == L - 1;
     Shoup add_w{0, 0}, fold_w{0, 0};
-    if (add) add_w = scalar_shoup(x.p_mod_q, t);
-    if (fold) fold_w = scalar_shoup(x.fold_w, 0);
+    const uint64_t *p_mod_q = a.barrett + 2 * a.size_qp;   // and P^-1 behind it (NttArgs::tw)
+    if (add) add_w = scalar_shoup(p_mod_q, t);
+    if (fold) fold_w = scalar_shoup(p_mod_q, a.map.tail_first + t);
     const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
     // (the words of a limb that ModDown transforms back go through the inverse blocks pass before they leave the wave)
-    const bool invert = t >= x.inv_first;
+    const bool invert = t >= (x.inv_first & 0xffff);
     A iar = ar;
     if constexpr (FP)
         iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
@@ -419,7 +531,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     uint64_t c0[4], cl[4];
     auto fetch_addends = [&](uint32_t r) {
         if (add && r == 0) {
-            const uint64_t *src = x.add_c0 + (size_t)t * n;
+            const uint64_t *src = x.addend + (size_t)t * n;
             if (x.own_galois) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
@@ -427,7 +539,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
                 load4(c0, src + at);
             }
         }
-        if (fold) load4(cl, x.fold_ct + item * x.fold_item_stride + ((size_t)r * x.L + t) * n + at);
+        if (fold) load4(cl, x.addend + item * x.fold_item_stride() + ((size_t)r * L + t) * n + at);
     };
     if constexpr (SPLIT > 1) {
         // (what the two waves that finish need after the sums have met is requested before the digits)
@@ -438,7 +550,8 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
     }
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
-        const uint64_t *src = x.own + item * x.own_item_stride + (size_t)t * n;
+        const uint64_t *src = a.in + (size_t)t * n;
+        if (item) src += item * x.own_item_stride();
         uint64_t c[4], k[2][4];
         keys(k, own);
         if (x.own_galois) {
@@ -457,7 +570,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         }
         sums.add(v, k, ar);
     }
-    while (d < x.beta) {
+    while (d < beta) {
         uint64_t k[2][4];
         keys(k, d);
         typename A::V v[4];
@@ -467,7 +580,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
         d = next_digit(d);
         // (behind a branch that may skip these loads the compiler waits for them with the keys; short chains fetch their last digit
         // again instead: n = 2^15, 10 of 12 limbs 71.5 -> 69.8 us.  One wave a block loses by it: L = 24, K = 8 153 against 156 us)
-        if (SPLIT > 1 || d < x.beta) fetch(nx, d < x.beta ? d : now);
+        if (SPLIT > 1 || d < beta) fetch(nx, d < beta ? d : now);
         ar.reduce(v);
         T4::template forward<A>(v, tw, ar, nullptr, lane);
         if constexpr (!FP) {
@@ -572,15 +685,18 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const KsFuseArgs &
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
 constexpr int kInnerWaves = 4;
 
-template <int BE, int SPLIT>
-__global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, KsFuseArgs x) {
+template <int BE, int SPLIT, class X>
+__global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PARAMS, X x) {
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
-    touch_arguments<sizeof(NttArgs) + sizeof(KsFuseArgs) - (kMaxDigits - 8) * sizeof(uint64_t *)>();
-    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = (x.L + x.K) << lr;
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    set_inverse_block(a, x.itw);
+    const uint32_t LK = a.map.limbs, L = a.map.split, items = h5 >> 8;
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, pairs = LK << lr;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), part = w % SPLIT;
     uint32_t pair, item = 0;
-    if (SPLIT == 1 && x.items > 1) {
-        const uint32_t groups = (x.items + kInnerWaves - 1) / kInnerWaves, id = blockIdx.x;
+    if (SPLIT == 1 && items > 1) {
+        const uint32_t groups = (items + kInnerWaves - 1) / kInnerWaves, id = blockIdx.x;
         uint32_t g;
         if (pairs % 8 == 0) {
             // hardware id -> XCD id & 7; inside an XCD the groups of one pair are consecutive
@@ -592,7 +708,7 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
             pair = id - g * pairs;
         }
         item = g * kInnerWaves + w;
-        if (item >= x.items) return;
+        if (item >= items) return;
     } else {
         // last limb first: the special limbs have one digit more to transform than the others
         // (a limb has an even number of blocks: with SPLIT > 1 no wave is left over, and a workgroup's blocks share their limb)
@@ -601,18 +717,13 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(NttArgs a, 
         pair = pairs - 1 - pair;
     }
     uint32_t t = pair >> lr;
-    if (BE == NTT_BACKEND_MIXED && x.ordered) {
-        typedef const uint32_t __attribute__((address_space(4))) *Order;
-        const Order order = (Order)((const char __attribute__((address_space(4))) *)__builtin_amdgcn_kernarg_segment_ptr() +
-                                    sizeof(NttArgs) + offsetof(KsFuseArgs, order));
-        t = (order[t >> 2] >> (8 * (t & 3))) & 0xff;
-    }
-    const uint32_t blk = pair & ((1u << lr) - 1), table = t < x.L ? t : x.size_q + (t - x.L);
+    if (BE == NTT_BACKEND_MIXED && LK <= 16) t = (uint32_t)((((uint64_t)h2 << 32) | h1) >> (4 * t)) & 15;
+    const uint32_t blk = pair & ((1u << lr) - 1), table = map_table(a.map, t);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
-    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, fp_arith(a, table), part, sums);
+    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, fp_arith(a, table), part, sums);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) inner_block<SPLIT>(a, x, t, table, blk, item, lane, int_arith(a, table), part, sums);
+        if (!fp) inner_block<SPLIT>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, int_arith(a, table), part, sums);
     }
 }
 
@@ -698,7 +809,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(Nt
     touch_arguments<sizeof(NttArgs) + sizeof(TensorFuse)>();
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const uint32_t id = logical_block(x.wgs) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane);
@@ -779,19 +890,21 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
 }
 
 template <int BE>
-__global__ __launch_bounds__(192) void encrypt_blocks_kernel(NttArgs a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q,
-                                                             uint32_t items, uint32_t first_item) {
+__global__ __launch_bounds__(192) void encrypt_blocks_kernel(HE_HEAD_PARAMS, const uint64_t *itw) {
     __shared__ uint64_t u_lds[256];
-    touch_arguments<sizeof(NttArgs)>();
-    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = L + K;
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    set_inverse_block(a, itw);
+    const uint64_t *pk = a.in;
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = a.map.limbs, L = a.map.split, items = h1, first_item = h5;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block(), blk = id & ((1u << lr) - 1), it = id >> lr;
-    const uint32_t of_launch = it / LK, item = first_item + of_launch, t = it - of_launch * LK, table = t < L ? t : size_q + (t - L);
+    const uint32_t id = logical_block(h4), blk = id & ((1u << lr) - 1), it = id >> lr;
+    const uint32_t of_launch = it / LK, item = first_item + of_launch, t = it - of_launch * LK, table = map_table(a.map, t);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     if (BE != NTT_BACKEND_INT && fp)
-        encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, fp_arith(a, table), u_lds);
+        encrypt_block(a, pk, L, LK, a.size_qp, t, table, blk, item, items, w, lane, fp_arith(a, table), u_lds);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) encrypt_block(a, pk, L, LK, size_q + K, t, table, blk, item, items, w, lane, int_arith(a, table), u_lds);
+        if (!fp) encrypt_block(a, pk, L, LK, a.size_qp, t, table, blk, item, items, w, lane, int_arith(a, table), u_lds);
     }
 }
 
@@ -802,7 +915,7 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
     using T4 = Tile4<8, 8>;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane, poly = (size_t)a.map.limbs * n;
     const uint64_t q = scalar(a.moduli)[job.table], r0 = scalar(a.barrett)[2 * job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
-    const uint64_t *ct = (d.cts ? d.cts[job.poly] : d.ct) + job.limb * n + at;
+    const uint64_t *ct = (a.in ? a.in : d.cts[job.poly]) + job.limb * n + at;
     const uint64_t *sk = d.sk + job.limb * n + at;
     uint64_t x[4], c0[4], c1[4], s1[4], c2[4], s2[4];
 #pragma unroll
@@ -831,11 +944,12 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
 }
 
 template <int BE>
-__global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(NttArgs a, DecryptArgs d) {
-    touch_arguments<sizeof(NttArgs) + sizeof(DecryptArgs)>();
+__global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(HE_HEAD_PARAMS, DecryptArgs d) {
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block() * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const uint32_t id = logical_block(h4) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) decrypt_block(a, d, job, blk, lane, fp_arith(a, job.table));
@@ -860,7 +974,9 @@ hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
         n_jobs -= per_launch;
     }
     const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
-#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B>), grid, block, 0, s, a)
+    const NttHead head = ntt_head(a, grid.x, a.first_job);
+    const RowsExtra extra = rows_extra(a, FWD);
+#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B>), grid, block, 0, s, HE_HEAD_ARGS(head), extra)
 #define HE_CASE(LD)         \
     case LD:                \
         if (large)          \
@@ -892,14 +1008,19 @@ bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
     return log_n >= 12 && log_n <= 16 && n_tables <= 64 && ((uint64_t)n_jobs << log_n) <= ((uint64_t)16 << 16);
 }
 
-hipError_t launch_ntt_rows(const NttArgs &a, uint32_t n_jobs, bool forward, int backend, hipStream_t s) {
-    if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
+hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, int backend, hipStream_t s) {
+    if (args.log_n < 9 || args.log_n > 17) return hipErrorInvalidValue;
+    NttArgs a = args;
+    if (forward && a.pro_mode != NTT_PLAIN && a.pro_mode != NTT_PRO_MODDOWN_RESCALE) {
+        // the source in place of the input, which these prologues do not read (see Job::src and rows_input_fp)
+        a.in = a.pro_src;
+        a.in_poly_stride = a.pro_mode == NTT_PRO_ROUND ? a.pro_log_slots : a.pro_poly_stride;
+    }
     if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
         // one instantiation per degree, which follows fp_mask limb by limb: the mask stands for the launch's back end here
         if (!forward || !a.pro_itw || (a.pro_src_fp_mask && !a.pro_itw_fp)) return hipErrorInvalidValue;
-        NttArgs b = a;
-        b.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
-        return launch_rows<true, NTT_BACKEND_MIXED, true>(b, n_jobs, s);
+        a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+        return launch_rows<true, NTT_BACKEND_MIXED, true>(a, n_jobs, s);
     }
     if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE)
         return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED, false, true>(a, n_jobs, s)
@@ -934,14 +1055,16 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     const uint64_t wgs = (uint64_t)kinds * ((repeats + a.batch - 1) / a.batch) * (blocks / kBlockWaves);
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    const NttHead head = ntt_head(a, grid.x, a.batch);
+    const BlocksExtra extra = blocks_extra(a, forward);
 #define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
     do {                                                                                                                \
         if (backend == NTT_BACKEND_MIXED)                                                                               \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_MIXED>), grid, block, 0, s, a);    \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_MIXED>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
         else if (backend)                                                                                               \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_FP>), grid, block, 0, s, a);       \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_FP>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
         else                                                                                                            \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT>), grid, block, 0, s, a);      \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
     } while (0)
     const bool epi = forward && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || a.epi_mode == NTT_EPI_FMA_SUB_MUL);
     const bool loop = a.batch > 1 || a.groups;
@@ -961,9 +1084,9 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     return hipGetLastError();
 }
 
-hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x_, int backend, hipStream_t s) {
-    KsFuseArgs x = x_;
-    if (a.log_n < 9 || a.log_n > 17) return hipErrorInvalidValue;
+hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backend, hipStream_t s) {
+    NttArgs a = args;
+    if (a.log_n < 9 || a.log_n > 17 || x.items > 0xffffff || x.beta > 255) return hipErrorInvalidValue;
     const uint32_t items = x.items ? x.items : 1;
     if (items > 1 && (x.own_galois || x.add_c0)) return hipErrorInvalidValue;
     const uint64_t pairs = (uint64_t)(x.L + x.K) << (a.log_n - 8);
@@ -976,27 +1099,43 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x_, int backend,
     const uint64_t wgs = items > 1 ? pairs * ((items + kInnerWaves - 1) / kInnerWaves) : (pairs * split + kInnerWaves - 1) / kInnerWaves;
     if (wgs > most_workgroups(64 * kInnerWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kInnerWaves);
-    // Mixed back end, more than a workgroup for every CU: the launch walks its limbs from the last to the first, so the integer
-    // limbs, whose waves issue three times the instructions, take the last places and a CU's second workgroup is one of the short
-    // ones (a rotation on [60, 40, 40, 60], two limbs of 2^16 words: 30.4 -> 29.1 us, in this kernel 9.8 -> 8.5)
-    x.ordered = backend == NTT_BACKEND_MIXED && items == 1 && wgs > 256 && x.L + x.K <= 64;
-    if (x.ordered) {
+    a.in = x.own;
+    a.map = LimbMap{x.L + x.K, 0, x.L, x.size_q};
+    if (x.add_c0 && x.fold_ct) return hipErrorInvalidValue;
+    NttHead head = ntt_head(a, (uint32_t)wgs, x.beta | items << 8);
+    if (backend == NTT_BACKEND_MIXED && x.L + x.K <= 16) {
+        // The launch walks its limbs from the last to the first.  With more than one workgroup for every CU the integer
+        // limbs, whose waves issue three times the instructions, take the last places, so that a CU's second workgroup is one of the short
+        // ones (a rotation on [60, 40, 40, 60], two limbs of 2^16 words: 30.4 -> 29.1 us, in this kernel 9.8 -> 8.5)
+        const bool reorder = items == 1 && wgs > 256;
+        uint64_t order = 0;
         uint32_t at = x.L + x.K;
         for (int fp = 0; fp < 2; fp++)
             for (uint32_t t = x.L + x.K; t-- > 0;)
-                if ((int)((a.fp_mask >> (t < x.L ? t : x.size_q + (t - x.L))) & 1) == fp) {
-                    at--;
-                    x.order[at >> 2] |= t << (8 * (at & 3));
-                }
+                if (reorder ? (int)((a.fp_mask >> map_table(a.map, t)) & 1) == fp : fp == 0) order |= (uint64_t)t << (4 * --at);
+        head.h1 = (uint32_t)order;
+        head.h2 = (uint32_t)(order >> 32);
     }
-#define HE_INNER(SPLIT)                                                                                           \
-    do {                                                                                                          \
-        if (backend == NTT_BACKEND_MIXED)                                                                         \
-            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_MIXED, SPLIT>), grid, block, 0, s, a, x);            \
-        else if (backend)                                                                                         \
-            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_FP, SPLIT>), grid, block, 0, s, a, x);               \
-        else                                                                                                      \
-            hipLaunchKernelGGL((ntt_inner_kernel<NTT_BACKEND_INT, SPLIT>), grid, block, 0, s, a, x);              \
+    const uint64_t *addend = x.add_c0 ? x.add_c0 : x.fold_ct;
+    const uint32_t inv_first = x.inv_first | (x.add_c0 ? 1u << 16 : 0) | (x.fold_ct ? 1u << 17 : 0);
+    InnerFew few{a.pro_itw, addend, x.out, x.own_galois, inv_first, {x.evk.p[0], x.evk.p[1], x.evk.p[2]}};
+    InnerMany many{a.pro_itw, addend, x.out, x.own_galois, inv_first, {a.item_stride, x.own_item_stride, x.fold_item_stride}, {}};
+    memcpy(many.evk, x.evk.p, sizeof(many.evk));
+#define HE_INNER_BE(BE, SPLIT)                                                                                                    \
+    do {                                                                                                                          \
+        if (items == 1 && x.beta <= InnerFew::kDigits)                                                                            \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, InnerFew>), grid, block, 0, s, HE_HEAD_ARGS(head), few);               \
+        else                                                                                                                      \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, InnerMany>), grid, block, 0, s, HE_HEAD_ARGS(head), many);             \
+    } while (0)
+#define HE_INNER(SPLIT)                                  \
+    do {                                                 \
+        if (backend == NTT_BACKEND_MIXED)                \
+            HE_INNER_BE(NTT_BACKEND_MIXED, SPLIT);       \
+        else if (backend)                                \
+            HE_INNER_BE(NTT_BACKEND_FP, SPLIT);          \
+        else                                             \
+            HE_INNER_BE(NTT_BACKEND_INT, SPLIT);         \
     } while (0)
     if (split == 4)
         HE_INNER(4);
@@ -1005,13 +1144,16 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x_, int backend,
     else
         HE_INNER(1);
 #undef HE_INNER
+#undef HE_INNER_BE
     return hipGetLastError();
 }
 
-hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s) {
+hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &fuse, uint32_t items, int backend, hipStream_t s) {
+    TensorFuse x = fuse;
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0 || items == 0) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
+    x.wgs = (uint32_t)wgs;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
@@ -1022,36 +1164,44 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint
     return hipGetLastError();
 }
 
-hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
+hipError_t launch_encrypt_blocks(const NttArgs &args, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
                                  int backend, hipStream_t s) {
+    NttArgs a = args;
     if (a.log_n < 9 || a.log_n > 17 || items == 0) return hipErrorInvalidValue;
+    a.in = pk;
+    a.in_poly_stride = items;
+    a.map = LimbMap{L + K, 0, L, size_q};
     const dim3 block(192);
     const uint32_t wgs_per_item = (L + K) << (a.log_n - 8), per_launch = most_workgroups(block.x) / wgs_per_item;
     if (per_launch == 0) return hipErrorInvalidValue;
     for (uint32_t first = 0; first < items; first += per_launch) {
         const dim3 grid((items - first < per_launch ? items - first : per_launch) * wgs_per_item);
+        const NttHead head = ntt_head(a, grid.x, first);
         if (backend == NTT_BACKEND_MIXED)
-            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);
         else if (backend)
-            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);
         else
-            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, pk, L, K, size_q, items, first);
+            hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);
         if (hipError_t e = hipGetLastError()) return e;
     }
     return hipSuccess;
 }
 
-hipError_t launch_decrypt_blocks(const NttArgs &a, const DecryptArgs &d, uint32_t items, int backend, hipStream_t s) {
+hipError_t launch_decrypt_blocks(const NttArgs &args, const DecryptArgs &d, uint32_t items, int backend, hipStream_t s) {
+    NttArgs a = args;
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || items == 0 || d.size < 2 || d.size > 3) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)a.map.limbs * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    a.in = d.ct;
+    const NttHead head = ntt_head(a, grid.x, 0);
     if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, d);
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), d);
     else if (backend)
-        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, d);
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(head), d);
     else
-        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, d);
+        hipLaunchKernelGGL(decrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(head), d);
     return hipGetLastError();
 }
 

@@ -323,3 +323,33 @@ def test_key_switch_of_a_mixed_chain(oracle, capi, logn, bits, size_p, L):
     capi.check(lib.he_keyswitch_rescale(h, L, dc.ptr, keys, dct.ptr, low.ptr, 0, ws.ptr, None))
     ks = p.key_switch(c, host)
     assert (low.numpy() == p.rescale(np.stack([p.add(ct[b], ks[b]) for b in range(2)]))).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("size_p,L", [(1, 2), (1, 3), (1, 4), (1, 5), (2, 2), (2, 3), (2, 4)])
+def test_key_switches_of_few_and_of_many_digits(oracle, capi, chain, size_p, L):
+    """The inner product takes its keys' addresses in one form up to three digits of one ciphertext and in another beyond; the converted
+    limbs of a digit (the last one may have fewer) are worked out.  A map of one run may have anything as its second run."""
+    cahel, parms, ctx, p = make_pair(oracle, 13, CHAINS[chain], size_p)
+    rng = np.random.default_rng(16 * size_p + L)
+    lib, h = capi.lib(), ctx.he_handle()
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(-(-p.size_q // p.size_p))]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    keys = capi.evk_array([d.ptr for d in dev])
+    for items in (1, 2):
+        cs = np.stack([rand_limbs(p, rng, range(L)) for _ in range(items)])
+        cts = np.stack([rand_limbs(p, rng, range(L), n_polys=2) for _ in range(items)])
+        dc, dct = DeviceArray(capi, host=cs), DeviceArray(capi, host=cts)
+        low = DeviceArray(capi, shape=(items, 2, L - 1, p.n))
+        ws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+        capi.check(lib.he_keyswitch_rescale_batch(h, L, items, dc.ptr, L, keys, dct.ptr, low.ptr, 0, ws.ptr, None))
+        got = low.numpy()
+        for k in range(items):
+            ks = p.key_switch(cs[k], host)
+            assert (got[k] == p.rescale(np.stack([p.add(cts[k][b], ks[b]) for b in range(2)]))).all(), (items, k)
+    x = rand_limbs(p, rng, range(L))
+    d = DeviceArray(capi, host=x)
+    capi.check(lib.he_ntt_forward(h, d.ptr, 1, L, L, 0, L, 0xfffffff7, None))
+    assert (d.numpy() == p.ntt_fwd(x.copy())).all()
+    capi.check(lib.he_ntt_inverse(h, d.ptr, 1, L, L, 0, L, 0xfffffff7, None))
+    assert (d.numpy() == x).all()
