@@ -1648,15 +1648,19 @@ int decrypt_flood_impl(const he_context *ctx, const DecryptArgs &d, uint32_t lim
                        const uint64_t *cdt, uint32_t cdt_len, uint64_t *plain, uint64_t *noise, he_stream s) {
     ChaChaKey k;
     memcpy(k.k, key, sizeof(k.k));
-    HE_HIP(launch_sample_gauss_small(ctx->log_n, k, stream_id, reinterpret_cast<int8_t *>(noise), cdt, cdt_len, items, S(s)));
     NttArgs a = base_args(ctx, true);
     a.out = plain;
     a.out_poly_stride = limbs;
     a.map = plain_map(limbs);
-    a.pro_mode = NTT_PRO_SMALL;
-    a.pro_src = noise;
     const int backend = backend_for(ctx, a.map);
-    HE_HIP(launch_ntt_rows(a, items * limbs, true, backend, S(s)));
+    if (flood_rows_ok(ctx->log_n, limbs, items)) {
+        HE_HIP(launch_flood_rows(a, k, stream_id, cdt, cdt_len, items, backend, S(s)));
+    } else {
+        HE_HIP(launch_sample_gauss_small(ctx->log_n, k, stream_id, reinterpret_cast<int8_t *>(noise), cdt, cdt_len, items, S(s)));
+        a.pro_mode = NTT_PRO_SMALL;
+        a.pro_src = noise;
+        HE_HIP(launch_ntt_rows(a, items * limbs, true, backend, S(s)));
+    }
     HE_HIP(launch_decrypt_blocks(a, d, items, backend, S(s)));
     return HE_OK;
 }

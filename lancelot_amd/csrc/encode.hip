@@ -451,61 +451,94 @@ __global__ __launch_bounds__(kThreads) void decode_compose_kernel(const uint64_t
     slot[imag ? 1 : 0] = compose<LIMBS>(d, limbs, inv_scale, moduli, barrett, garner_inv, garner_stride);
 }
 
-// The inverse rows pass of all limbs of a plaintext and the composition in one kernel: a workgroup takes one tile of every
-// limb in turn through the pass, which leaves rows r, r + R/4 (real parts of two values) and r + R/2, r + 3R/4 (their
-// imaginary parts) of one column in each thread, and composes them.  The two values go to neighbouring positions of the
-// slot vector.  Full and sparse packing; blockIdx.y = item.
+// The inverse rows pass of all limbs of a plaintext and the composition in one kernel: a workgroup takes one tile of every limb
+// through the pass, a limb to each group of four waves, which leaves rows r, r + R/4 (real parts of two values) and r + R/2, r + 3R/4
+// (their imaginary parts) of one column in each thread; the groups exchange their words, and the first two compose one of the two
+// values each, which go to neighbouring positions of the slot vector.  Full and sparse packing; blockIdx.y = item.
+// Bound by the chain from the words' arrival to the composed value: the launch has one tile for every fourth CU.  One group that took
+// limb after limb, 7.2 us for 2 limbs of 2^16 words, now 6.2; a decryption to host values of 4 limbs with 2^12 values 49 -> 43.5 us
+// (1.6 us of it the sampling, see flood_rows_kernel).
 template <int LD, int LIMBS>
-__global__ __launch_bounds__(256) void decode_rows_compose_kernel(NttArgs a, uint32_t log_slots, double inv_scale,
-                                                                  const uint64_t *garner_inv, uint32_t garner_stride, double2 *v) {
+__global__ __launch_bounds__(256 * LIMBS) void decode_rows_compose_kernel(HE_HEAD_PARAMS, double2 *v, const uint64_t *garner_inv,
+                                                                          double inv_scale, uint32_t log_slots, uint32_t garner_stride) {
     constexpr int B = 10, LOGC = B - LD;
     using T4 = Tile4<B, LD>;
     constexpr int NB = T4::kBlocks;
-    __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
-    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    __shared__ uint64_t tiles[LIMBS][(1 << B) + (1 << (B - 4))];
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    a.epi_mode = NTT_PLAIN;
+    const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6), group = wave >> 2;
+    const uint32_t t = ((wave & 3) << 6) | (threadIdx.x & 63);
     const uint32_t col0 = blockIdx.x << LOGC, item = blockIdx.y;
     auto glob = [&](int k, int j) {
         const uint32_t e = T4::word(k, t, j);
         return (size_t)(e >> LOGC) * 256 + col0 + (e & ((1u << LOGC) - 1));
     };
-    uint64_t d[4][LIMBS];
+    uint64_t *lds = tiles[group];
+    const Job job = decode_job(a, item * LIMBS + group);
+    uint64_t x[4];
 #pragma unroll
-    for (int l = 0; l < LIMBS; l++) {
-        const Job job = decode_job(a, item * LIMBS + l);
-        uint64_t x[4];
+    for (int j = 0; j < 4; j++) x[j] = job.in[glob(NB - 1, j)];
+    // (the composition's constants, requested with the words: behind the exchange they were another trip to memory)
+    uint64_t moduli[LIMBS], barrett[2 * LIMBS], garner[LIMBS * LIMBS];
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = job.in[glob(NB - 1, j)];
-        if ((a.fp_mask >> job.table) & 1) {
-            const FpArith ar = fp_arith(a, job.table);
-            FpArith::Tw tw[NB];
-            T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-            const double scale = inverse_scale(a, job, ar.m);
-            double w[4];
+    for (int i = 0; i < LIMBS; i++) {
+        moduli[i] = scalar(a.moduli)[i];
+        barrett[2 * i] = scalar(a.barrett)[2 * i];
+        barrett[2 * i + 1] = scalar(a.barrett)[2 * i + 1];
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = FpArith::from_word(x[j]);
-            ar.reduce(w);
-            T4::template inverse<FpArith>(w, tw, ar, lds, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) d[j][l] = fp_to_u64(fp_canonical(fp_mulmod(w[j], scale, ar.m), ar.m));
-        } else {
-            const IntArith ar = int_arith(a, job.table);
-            IntArith::Tw tw[NB];
-            T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
-            T4::template inverse<IntArith>(x, tw, ar, lds, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) d[j][l] = reduce_2q(x[j], ar.m.q);
-        }
-        lds_barrier();   // (the next limb's tile overwrites this one's)
+        for (int j = 0; j < i; j++) garner[i * LIMBS + j] = scalar(garner_inv)[(size_t)i * garner_stride + j];
     }
-    double val[4];
 #pragma unroll
-    for (int j = 0; j < 4; j++) val[j] = compose<LIMBS>(d[j], LIMBS, inv_scale, a.moduli, a.barrett, garner_inv, garner_stride);
+    for (int i = 0; i < LIMBS; i++) {
+        asm volatile("" ::"s"(moduli[i]), "s"(barrett[2 * i]), "s"(barrett[2 * i + 1]));
+#pragma unroll
+        for (int j = 0; j < i; j++) asm volatile("" ::"s"(garner[i * LIMBS + j]));
+    }
+    if ((a.fp_mask >> job.table) & 1) {
+        const FpArith ar = fp_arith(a, job.table);
+        FpArith::Tw tw[NB];
+        T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+        const double scale = inverse_scale(a, job, ar.m);
+        double w[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = FpArith::from_word(x[j]);
+        ar.reduce(w);
+        T4::template inverse<FpArith>(w, tw, ar, lds, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(fp_mulmod(w[j], scale, ar.m), ar.m));
+    } else {
+        const IntArith ar = int_arith(a, job.table);
+        IntArith::Tw tw[NB];
+        T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+        T4::template inverse<IntArith>(x, tw, ar, lds, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = reduce_2q(x[j], ar.m.q);
+    }
+    uint64_t d[2][LIMBS];
+    if constexpr (LIMBS > 1) {
+        lds_barrier();   // (the other waves of the group have read the tile)
+#pragma unroll
+        for (int j = 0; j < 4; j++) lds[256 * j + t] = x[j];
+        lds_barrier();
+    }
     const uint32_t log_gap = a.log_n - 1 - log_slots;
     v += (size_t)item << log_slots;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        const uint32_t k = (uint32_t)glob(0, j);   // (below N / 2)
-        if ((k & ((1u << log_gap) - 1)) == 0) v[__brev(k >> log_gap) >> (32 - log_slots)] = double2{val[j], val[j + 2]};
+    for (int pair = 0; pair < (LIMBS > 1 ? 1 : 2); pair++) {
+        const uint32_t j = LIMBS > 1 ? group : pair;
+        if (j >= 2) return;
+#pragma unroll
+        for (int l = 0; l < LIMBS; l++) {
+            d[0][l] = LIMBS > 1 ? tiles[l][256 * j + t] : x[pair];
+            d[1][l] = LIMBS > 1 ? tiles[l][256 * (j + 2) + t] : x[pair + 2];
+        }
+        double2 val;
+        val.x = compose<LIMBS>(d[0], LIMBS, inv_scale, moduli, barrett, garner, LIMBS);
+        val.y = compose<LIMBS>(d[1], LIMBS, inv_scale, moduli, barrett, garner, LIMBS);
+        const uint32_t k = (uint32_t)glob(0, (int)j);   // (below N / 2)
+        if ((k & ((1u << log_gap) - 1)) == 0) v[__brev(k >> log_gap) >> (32 - log_slots)] = val;
     }
 }
 
@@ -627,8 +660,10 @@ hipError_t launch_ckks_decode_real(const FftTables &t, const NttArgs &inv, int b
     NttArgs a = inv;   // (the mask stands for the launch's back end)
     a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : inv.fp_mask);
     const dim3 grid(1u << (a.log_n - 10), items);
+    const NttHead h = ntt_head(a, 0, 0);
 #define HE_LIMBS(LD, L)                                                                                                            \
-    hipLaunchKernelGGL((decode_rows_compose_kernel<LD, L>), grid, dim3(256), 0, s, a, log_slots, 1.0 / scale, garner_inv, garner_stride, v)
+    hipLaunchKernelGGL((decode_rows_compose_kernel<LD, L>), grid, dim3(256 * L), 0, s, HE_HEAD_ARGS(h), v, garner_inv, 1.0 / scale,    \
+                       log_slots, garner_stride)
 #define HE_CASE(LD)                         \
     case LD:                                \
         switch (limbs) {                    \

@@ -442,6 +442,11 @@ hipError_t launch_sample_encrypt(uint32_t log_n, ChaChaKey key, uint64_t stream_
 // ... or the discrete Gaussian by the cumulative table cdt (at most 128 entries), item k from stream_id + k
 hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t stream_id, int8_t *out, const uint64_t *cdt,
                                      uint32_t cdt_len, uint32_t items, hipStream_t s);
+// ... or that polynomial's residues, with the rows pass of their forward transform done: limb l of item k at a.out (a: map mode,
+// dense).  flood_rows_ok: whether that is the faster way.
+bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items);
+hipError_t launch_flood_rows(const NttArgs &a, ChaChaKey key, uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t items,
+                             int backend, hipStream_t s);
 
 // CKKS encoder twiddles: entry len / 2 + j (2 <= len <= N/2, j < len / 2) is e^{2 pi i r / (4 len)}, r = 5^j mod 4 len, of the decoding's
 // stage of span len, and e^{2 pi i (4 len - r) / (4 len)} of the encoding's.

@@ -14,6 +14,7 @@
 #include <cstring>
 #include <type_traits>
 
+#include "chacha.cuh"
 #include "kernels.h"
 #include "modarith.cuh"
 #include "ntt_common.cuh"
@@ -958,6 +959,76 @@ __global__ __launch_bounds__(64 * kBlockWaves) void decrypt_blocks_kernel(HE_HEA
     }
 }
 
+// What the noise's rows pass needs behind NttHead.
+struct FloodExtra {
+    ChaChaKey key;
+    uint64_t stream;
+    const uint64_t *cdt;
+    uint32_t cdt_len;
+};
+
+// The rows pass of a small Gaussian polynomial that is sampled on the spot: a thread makes four neighbouring coefficients of its tile
+// (half of its ChaCha block), a byte each in LDS.  Every limb's workgroups sample anew, on CUs that a launch of a few limbs leaves
+// idle, which costs less than a sampler's launch and the bytes' way through memory: decryption of two limbs of
+// 2^16 coefficients 10.7 -> 8.9 us.
+template <int LD>
+__global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodExtra f) {
+    using T4 = Tile4<10, LD>;
+    constexpr int LOGC = 10 - LD, NB = T4::kBlocks;
+    constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
+    __shared__ uint64_t lds[(1 << 10) + (1 << 6)], cdt[kSmallCdt];
+    __shared__ uint32_t noise[256];
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    const uint32_t lb = logical_block(h4);
+    const Job job = decode_job(a, lb / tiles_per_limb);
+    const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
+    const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
+    if (t < kSmallCdt) cdt[t] = padded_cdt(f.cdt, f.cdt_len, t);
+    auto glob = [&](int k, int j) {
+        const uint32_t e = T4::word(k, t, j);
+        return (size_t)(e >> LOGC) * 256 + col0 + (e & (C - 1));
+    };
+    auto sample = [&]() {
+        const uint32_t at = ((4 * t) >> LOGC) * 256 + col0 + ((4 * t) & (C - 1));
+        uint32_t w[16];
+        chacha20_block(f.key, at >> 3, f.stream + job.poly, w);
+        const bool upper = at & 4;
+#pragma unroll
+        for (int e = 0; e < 8; e++) w[e] = upper ? w[8 + e] : w[e];
+        lds_barrier();   // cdt
+        gauss_bytes<4>(noise + t, w, cdt);
+        lds_barrier();
+    };
+    auto value = [&](int j) { return (int)reinterpret_cast<const int8_t *>(noise)[T4::word(0, t, j)]; };
+    if ((a.fp_mask >> job.table) & 1) {
+        const FpArith ar = fp_arith(a, job.table);
+        FpArith::Tw tw[NB];
+        T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+        sample();
+        double v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = (double)value(j);
+        T4::template forward<FpArith>(v, tw, ar, lds, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = FpArith::to_word(v[j]);
+    } else {
+        const IntArith ar = int_arith(a, job.table);
+        IntArith::Tw tw[NB];
+        T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+        sample();
+        uint64_t v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int64_t x = value(j);
+            v[j] = (uint64_t)x + (x < 0 ? ar.m.q : 0);
+        }
+        T4::template forward<IntArith>(v, tw, ar, lds, t);
+#pragma unroll
+        for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = v[j];
+    }
+}
+
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
@@ -1033,6 +1104,30 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
     return backend == NTT_BACKEND_MIXED ? launch_rows<false, NTT_BACKEND_MIXED>(a, n_jobs, s)
            : backend                    ? launch_rows<false, NTT_BACKEND_FP>(a, n_jobs, s)
                                         : launch_rows<false, NTT_BACKEND_INT>(a, n_jobs, s);
+}
+
+// one workgroup for every CU: 4 limbs of 2^16 coefficients 11.5 -> 9.9 us with the blocks pass behind them, 16 of 2^14 10.6 -> 9.4; half as
+// many workgroups more and the sampling is no longer hidden (6 of 2^16: 12.4 -> 12.5 us, 24 of 2^14: 11.5 -> 12.0)
+bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items) {
+    return log_n >= 12 && log_n <= 16 && limbs <= 64 && ((uint64_t)items * limbs << log_n) <= (1u << 18);
+}
+
+hipError_t launch_flood_rows(const NttArgs &args, ChaChaKey key, uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t items,
+                             int backend, hipStream_t s) {
+    const uint32_t n_jobs = items * args.map.limbs;
+    if (items == 0 || items > 65535 || args.jobs || cdt_len == 0 || cdt_len >= kSmallCdt || !flood_rows_ok(args.log_n, args.map.limbs, items)) return hipErrorInvalidValue;
+    NttArgs a = args;
+    a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+    const dim3 grid(n_jobs << (a.log_n - 10));
+    const NttHead head = ntt_head(a, grid.x, 0);
+    const FloodExtra f{key, stream_id, cdt, cdt_len};
+    switch (a.log_n - 8) {
+#define HE_CASE(LD) case LD: hipLaunchKernelGGL(flood_rows_kernel<LD>, grid, dim3(256), 0, s, HE_HEAD_ARGS(head), f); break;
+        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+#undef HE_CASE
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
 }
 
 // Limbs of one prime in turn on one wave, which reads its twiddles once: saves up to a third of the traffic (FP64; half of it

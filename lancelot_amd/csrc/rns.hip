@@ -13,6 +13,7 @@
 
 #include <type_traits>
 
+#include "chacha.cuh"
 #include "kernels.h"
 #include "modarith.cuh"
 #include "ntt_common.cuh"
@@ -1161,33 +1162,6 @@ __global__ __launch_bounds__(kThreads) void hoist_one_kernel(HoistArgs p) {
     }
 }
 
-// ---------------------------------------------------------------------------------------------------
-// samplers: ChaCha20 block function (RFC 8439 section 2.3), 64-bit block counter in words 12-13,
-// 64-bit stream id in words 14-15
-// ---------------------------------------------------------------------------------------------------
-__device__ __forceinline__ uint32_t rotl32(uint32_t v, int c) { return (v << c) | (v >> (32 - c)); }
-
-#define HE_QR(a, b, c, d) \
-    a += b; d ^= a; d = rotl32(d, 16); \
-    c += d; b ^= c; b = rotl32(b, 12); \
-    a += b; d ^= a; d = rotl32(d, 8);  \
-    c += d; b ^= c; b = rotl32(b, 7);
-
-__device__ void chacha20_block(const ChaChaKey &key, uint64_t counter, uint64_t stream, uint32_t *out) {
-    uint32_t s[16] = {0x61707865u, 0x3320646eu, 0x79622d32u, 0x6b206574u,
-                      key.k[0], key.k[1], key.k[2], key.k[3], key.k[4], key.k[5], key.k[6], key.k[7],
-                      (uint32_t)counter, (uint32_t)(counter >> 32), (uint32_t)stream, (uint32_t)(stream >> 32)};
-    uint32_t x[16];
-#pragma unroll
-    for (int i = 0; i < 16; i++) x[i] = s[i];
-    for (int i = 0; i < 10; i++) {
-        HE_QR(x[0], x[4], x[8], x[12]) HE_QR(x[1], x[5], x[9], x[13]) HE_QR(x[2], x[6], x[10], x[14]) HE_QR(x[3], x[7], x[11], x[15])
-        HE_QR(x[0], x[5], x[10], x[15]) HE_QR(x[1], x[6], x[11], x[12]) HE_QR(x[2], x[7], x[8], x[13]) HE_QR(x[3], x[4], x[9], x[14])
-    }
-#pragma unroll
-    for (int i = 0; i < 16; i++) out[i] = x[i] + s[i];
-}
-
 struct SampleArgs {
     uint64_t *out;
     const uint64_t *moduli, *barrett;
@@ -1304,7 +1278,6 @@ struct SmallArgs {
     uint32_t log_n, cdt_len, items;
 };
 constexpr int kSmallThreads = 64;
-constexpr uint32_t kSmallCdt = 128;
 
 template <int KIND>
 __device__ __forceinline__ void sample_bytes(const SmallArgs &p, uint64_t stream, int8_t *out) {
@@ -1334,36 +1307,17 @@ __global__ __launch_bounds__(kSmallThreads) void sample_encrypt_kernel(SmallArgs
     }
 }
 
-// blockIdx.y = item.  The table is padded to 128 entries that nothing reaches, so that the eight searches of a thread take the same
-// seven steps together, their LDS reads behind one another instead of each search after the one before (bound by that chain:
-// one polynomial of 2^16 coefficients 7.9 -> 5.1 us, a decryption to host values 56.8 -> 53.6 us).
+// blockIdx.y = item.  Bound by the chain of a search: see gauss_bytes.
 __global__ __launch_bounds__(kSmallThreads) void sample_gauss_small_kernel(SmallArgs p) {
     __shared__ uint64_t cdt[kSmallCdt];
-    for (uint32_t i = threadIdx.x; i < kSmallCdt; i += kSmallThreads) cdt[i] = i < p.cdt_len ? p.cdt[i] : ~(uint64_t)0;
+    for (uint32_t i = threadIdx.x; i < kSmallCdt; i += kSmallThreads) cdt[i] = padded_cdt(p.cdt, p.cdt_len, i);
     const uint32_t b = blockIdx.x * kSmallThreads + threadIdx.x;
     uint32_t w[16];
     chacha20_block(p.key, b, p.stream + blockIdx.y, w);
     __syncthreads();
     if (b >= (1u << p.log_n) / 8) return;
-    uint64_t u[8];
-    uint32_t mag[8];
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        u[e] = (((uint64_t)w[2 * e + 1] << 32) | w[2 * e]) & 0x7FFFFFFFFFFFFFFFull;
-        mag[e] = 0;
-    }
-    // the number of entries that are not above u (the table ascends)
-#pragma unroll
-    for (uint32_t step = kSmallCdt / 2; step; step >>= 1) {
-#pragma unroll
-        for (int e = 0; e < 8; e++) mag[e] += u[e] >= cdt[mag[e] + step - 1] ? step : 0;
-    }
-    uint32_t o[2] = {0, 0};
-#pragma unroll
-    for (int e = 0; e < 8; e++) {
-        const uint32_t v = w[2 * e + 1] >> 31 ? 0u - mag[e] : mag[e];
-        o[e / 4] |= (v & 255) << (8 * (e % 4));
-    }
+    uint32_t o[2];
+    gauss_bytes<8>(o, w, cdt);
     uint32_t *dst = reinterpret_cast<uint32_t *>(p.out + ((size_t)blockIdx.y << p.log_n) + 8 * (size_t)b);
     dst[0] = o[0];
     dst[1] = o[1];

@@ -353,3 +353,19 @@ def test_key_switches_of_few_and_of_many_digits(oracle, capi, chain, size_p, L):
     assert (d.numpy() == p.ntt_fwd(x.copy())).all()
     capi.check(lib.he_ntt_inverse(h, d.ptr, 1, L, L, 0, L, 0xfffffff7, None))
     assert (d.numpy() == x).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,limbs", [(11, 2), (12, 1), (12, 63), (13, 32), (13, 33), (14, 16), (14, 17), (15, 3), (16, 4), (16, 5)])
+def test_decryption_where_the_noise_has_a_launch_of_its_own_and_where_not(oracle, capi, chain, logn, limbs):
+    """Up to 2^18 coefficients the rows pass samples what it transforms."""
+    bits = (CHAINS[chain] * 11)[:limbs + 1]
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, 1)
+    lib, h, rng = capi.lib(), ctx.he_handle(), np.random.default_rng(logn + limbs)
+    key, cdt = oracle.chacha_key(3), oracle.gauss_cdt()
+    kp = key.ctypes.data_as(C.POINTER(C.c_uint32))
+    ct, s = rand_limbs(p, rng, range(limbs), n_polys=2), rand_limbs(p, rng, range(limbs))
+    dct, dsk, dcdt = DeviceArray(capi, host=ct), DeviceArray(capi, host=s), DeviceArray(capi, host=cdt)
+    out, noise = DeviceArray(capi, shape=(limbs, p.n)), DeviceArray(capi, shape=(p.n // 8,))
+    capi.check(lib.he_decrypt_flood(h, dct.ptr, 2, limbs, dsk.ptr, limbs * p.n, kp, 2 ** 40 + 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None))
+    assert (out.numpy() == p.add(p.mul_add(ct[1], s, ct[0]), p.ntt_fwd(p.sample_gauss(key, 2 ** 40 + 5, limbs, cdt)))).all()
