@@ -644,7 +644,7 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
         lv.beta = beta;
         rc = upload(ctx, &lv.d_part_hat_inv, d->part_hat_inv, 2 * (size_t)L);
         if (rc) return rc;
-        size_t mat_words = 0;
+        std::vector<uint64_t> mats;   // one after the other, digit d's at d K L (BconvUnit)
         std::vector<LimbJob> jobs;
         lv.digits.resize(beta);
         for (uint32_t dg = 0; dg < beta; dg++) {
@@ -652,8 +652,9 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
             g.start = dg * K;
             g.size = (g.start + K <= L) ? K : L - g.start;
             g.n_out = L + K - g.size;
-            g.mat_off = d->digit_mat_off[dg];
-            mat_words = g.mat_off + (size_t)g.n_out * g.size;
+            g.mat_off = mats.size();
+            const uint64_t *mat = d->digit_mats + d->digit_mat_off[dg];
+            mats.insert(mats.end(), mat, mat + (size_t)g.n_out * g.size);
             std::vector<uint32_t> limb(g.n_out), table(g.n_out);
             for (uint32_t r = 0; r < g.n_out; r++) {
                 limb[r] = r < g.start ? r : r + g.size;
@@ -664,7 +665,8 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
             if (!rc) rc = upload(ctx, &g.d_out_table, table.data(), g.n_out);
             if (rc) return rc;
         }
-        rc = upload(ctx, &lv.d_mats, d->digit_mats, mat_words);
+        const size_t mat_words = mats.size();
+        rc = upload(ctx, &lv.d_mats, mats.data(), mat_words);
         if (rc) return rc;
         if (K <= 8) {
             const size_t n = ctx->n();
@@ -712,8 +714,8 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
                         const double m = (double)ctx->h_moduli[table_of(ctx, L, lim)];
                         for (uint32_t i = 0; i < g.size; i++) {
                             const size_t idx = g.mat_off + (size_t)r * g.size + i;
-                            mfp[2 * idx] = (double)d->digit_mats[idx];
-                            mfp[2 * idx + 1] = (double)d->digit_mats[idx] / m;
+                            mfp[2 * idx] = (double)mats[idx];
+                            mfp[2 * idx + 1] = (double)mats[idx] / m;
                         }
                     }
                 }
@@ -727,7 +729,7 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
                         up[dg].mx_off = (uint32_t)(tab.size() / (4 * kMxRecord));
                         for (uint32_t r0 = 0; r0 < g.n_out; r0 += 4)
                             mx_record(tab, g.n_out - r0, g.size, 0,
-                                      [&](uint32_t rr, uint32_t i) { return d->digit_mats[g.mat_off + (size_t)(r0 + rr) * g.size + i]; },
+                                      [&](uint32_t rr, uint32_t i) { return mats[g.mat_off + (size_t)(r0 + rr) * g.size + i]; },
                                       [&](uint32_t rr) {
                                           const uint32_t r = r0 + rr;
                                           return ctx->h_moduli[table_of(ctx, L, r < g.start ? r : r + g.size)];
@@ -1003,10 +1005,8 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
                                     items, hipMemcpyDeviceToDevice, S(s)));
     } else if (fused) {
         const int backend = backend_for_level(ctx, L);
-        BconvRows b{ws, out, c, fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
-                    lv->beta, lv->modup_max_rows, copy_rows,
-                    items, (size_t)L * n, (size_t)lv->beta * LK * n, (size_t)c_item_stride * n, 0, lv->d_mx_up,
-                    nullptr, lv->d_mats, nullptr, ctx->size_p};
+        BconvRows b{ws, out, skip_own ? nullptr : c, (size_t)c_item_stride * n, LimbMap{LK, 0, L, ctx->size_q}, ctx->size_p, lv->beta, items, 1,
+                    fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr};
         HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend, ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{ws, out, c, lv->d_mats, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
@@ -1111,9 +1111,8 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     } else if (batched) {
         const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
         if (fused) {
-            BconvRows b{cx, ws, nullptr, fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
-                        items, (size_t)units * LK * n, (size_t)units * L * n, 0, 0, nullptr, nullptr,
-                        ctx->d_phat_mod_q, nullptr, K};
+            BconvRows b{cx, ws, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, units, items, 0,
+                        fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr};
             HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L, 0)), ctx->tune, S(s)));
         } else {
             BconvBatch b{cx, ws, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
@@ -1396,10 +1395,9 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     } else if (fused) {
         // with the prologue of (4) and the rows pass of its transform
         const bool fp = fp_for_level(ctx, L);
-        BconvRows b{cx, delta, nullptr, fp ? ctx->d_phat_pinv_fp : nullptr, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,
-                    items, 2 * (size_t)LK * n, 2 * (size_t)L * n, 0, 1, ctx->d_mx_down,
-                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr,
-                    ctx->d_phat_mod_q, ctx->d_pinv_mod_q, K};
+        BconvRows b{cx, delta, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, 2, items, 0,
+                    fp ? ctx->d_phat_pinv_fp : nullptr, 1, ctx->d_mx_down,
+                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q};
         HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L - 1, 0), (int)L - 1), ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{cx, delta, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,

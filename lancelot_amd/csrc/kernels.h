@@ -212,7 +212,6 @@ struct TensorFuse {
     uint64_t *d2;                // [L][N]: d2 in NTT form
     uint32_t L;
     int square;                  // ct2 is ignored, (d0, d1, d2) = (a0^2, 2 a0 a1, a1^2)
-    uint32_t wgs;                // filled in by the launcher
 };
 hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s);
 
@@ -298,19 +297,20 @@ struct BconvBatch {
 };
 hipError_t launch_bconv_batched(const Tables &t, const BconvBatch &b, const Tuning &tune, hipStream_t s);
 
-// Base conversion fused with the rows pass of the forward transform of its output limbs (N >= 2^12,
-// n_in <= 8): the units of a BconvBatch, with the results left as the lazy words that the blocks pass continues on.
+// Base conversion fused with the rows pass of the forward transform of its output limbs (N >= 2^12, at most 8 special primes), with the
+// results left as the lazy words that the blocks pass continues on.
+// ModUp: unit = digit d of an item, in [items][L][N] its limbs d K ... (the last digit may have fewer), out [items][units][L + K][N] every
+// limb of Ql u P but its own, which are copied from copy_base (or left out); matrices one after the other.
+// ModDown (up = 0): unit = polynomial, in [items][units][L + K][N] its special limbs, out [items][units][L][N]; one matrix.
 struct BconvRows {
-    const uint64_t *x_base;
-    uint64_t *out_base;
-    const uint64_t *copy_base;   // limbs copied unchanged (descs' copy_first / copy_count), or nullptr
-    const double *mat_fp;        // (M, M/m) pairs at 2 * mat_off
-    const uint32_t *out_limb;
-    const uint32_t *out_table;
-    const BconvDesc *descs;      // device memory
-    uint32_t n_units, max_rows, max_copy;
-    uint32_t items;              // 0 = 1
-    size_t x_item_stride, out_item_stride, copy_item_stride;
+    const uint64_t *in;
+    uint64_t *out;
+    const uint64_t *copy_base;   // limbs copied unchanged (item k: copy_item_stride words further), or nullptr
+    size_t copy_item_stride;
+    LimbMap map;                 // Ql u P
+    uint32_t K, units, items;
+    int up;
+    const double *mat_fp;        // (M, M/m) pairs
     // merged ModDown + rescale: the last row of every unit's matrix is the limb that is dropped; the other output
     // limbs receive sum_i x_i M[j][i] + ((t - sum_i x_i M[last][i] mod q_last) mod q_j), t = the limb before x
     int mdr;
@@ -326,17 +326,23 @@ struct BconvRows {
     // stores byte i of r = (t - sum_i x_i M[last][i]) mod q_last there, and the records of mx_tab multiply it by the
     // digits of 2^(8 i) mod q_r.
     const void *mx_last;
-    // levels with a prime from 2^50 on (mat_fp == nullptr): the matrix in integers at mat_off, and, mdr, P^-1 mod q_j (Shoup pairs)
+    // levels with a prime from 2^50 on (mat_fp == nullptr): the matrix in integers, and, mdr, P^-1 mod q_j (Shoup pairs)
     const uint64_t *mat;
     const uint64_t *w;
-    uint32_t max_in;             // the most input limbs of a unit, at most 8
+};
+// What its kernels take: NttHead with in and out, h1 = units | K << 16, h2 = workgroups of a tile that compute | that copy << 16,
+// h5 = rows of one, and pro_mode 1 for ModUp; behind it
+struct BconvExtra {
+    const void *mat;             // mat_fp, mat or mx_tab
+    const void *w;               // w or mx_last
+    const uint64_t *copy_base;
+    size_t copy_item_stride;
 };
 constexpr uint32_t kMxRecord = 144;
 // `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
 // and `backend` says what the blocks pass that follows runs on
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s);
-hipError_t launch_bconv_rows4(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups,
-                              uint32_t rows_per, int backend, hipStream_t s);
+hipError_t launch_bconv_rows4(const NttHead &h, const BconvRows &b, hipStream_t s);
 
 constexpr int kMaxDigits = 64;
 struct EvkPtrs {

@@ -263,10 +263,6 @@ inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_
 constexpr int kFuseLog = 11;
 constexpr uint32_t kFuseWords = 1u << kFuseLog;
 
-struct BconvRowsK {
-    BconvRows b;
-    uint32_t compute_groups, copy_groups, rows_per, wgs;
-};
 
 // see the matrix-core kernel below
 __device__ __forceinline__ uint32_t swz8(uint32_t e) { return e ^ ((((e >> 5) ^ (e >> 8)) & 3u) << 3); }
@@ -329,7 +325,7 @@ constexpr uint32_t kMxStride = kFuseWords + 16;
 
 template <bool MDR>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2)))
-void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
+void bconv_rows_mx_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     __shared__ double tiles[4 * kMxStride];
     __shared__ double twl[4][256];
     __shared__ double rconst[2][4][4];         // per group parity and row: q, 1/q, the constant that the digit sums lack
@@ -338,23 +334,23 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
     constexpr int LOGC = 3;
     constexpr uint32_t tiles_per_limb = 32;
 
-    uint32_t lb = logical_block(p.wgs);
-    const uint32_t groups = p.compute_groups + p.copy_groups;
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    uint32_t lb = logical_block(h4);
+    const uint32_t compute_groups = h2 & 0xffff, groups = compute_groups + (h2 >> 16), rows_per = h5;
     const uint32_t grp = lb % groups;
     lb /= groups;
-    const uint32_t tile = lb % tiles_per_limb, uidx = lb / tiles_per_limb;
-    const uint32_t item = uidx / p.b.n_units;
-    const BconvDesc d = p.b.descs[uidx - item * p.b.n_units];
-    const uint32_t col0 = tile << LOGC;
+    const BconvUnit d = bconv_unit(a, h1 & 0xffff, h1 >> 16, lb / tiles_per_limb);
+    const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
     const uint32_t lane = threadIdx.x & 63, wave = threadIdx.x >> 6, kg = lane >> 4, cn = lane & 15;
-    uint64_t *out = p.b.out_base + item * p.b.out_item_stride + d.out_off;
+    uint64_t *out = d.out;
 
-    if (grp >= p.compute_groups) {
+    if (grp >= compute_groups) {
         // limbs that pass through unchanged (a digit's own limbs keep their NTT form)
-        const uint64_t *from = p.b.copy_base + item * p.b.copy_item_stride;
-        const uint32_t first = (grp - p.compute_groups) * p.rows_per;
+        const uint64_t *from = b.copy_base + d.item * b.copy_item_stride;
+        const uint32_t first = (grp - compute_groups) * rows_per;
         const size_t g0 = (size_t)(threadIdx.x >> LOGC) * 256 + col0 + (threadIdx.x & 7);
-        for (uint32_t r = first; r < first + p.rows_per && r < d.copy_count; r++) {
+        for (uint32_t r = first; r < first + rows_per && r < d.n_in; r++) {
             const size_t limb = (size_t)(d.copy_first + r) << 16;
             uint64_t w[8];
 #pragma unroll
@@ -365,17 +361,17 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
         return;
     }
     const uint32_t n_rows = MDR ? d.n_out - 1 : d.n_out;
-    const uint32_t r_begin = grp * p.rows_per;
-    const uint32_t r_end = r_begin + p.rows_per < n_rows ? r_begin + p.rows_per : n_rows;
+    const uint32_t r_begin = grp * rows_per;
+    const uint32_t r_end = r_begin + rows_per < n_rows ? r_begin + rows_per : n_rows;
     if (r_begin >= n_rows) return;
 
     // the tables of this workgroup's rows (rows past the end repeat the last one; they are computed and not stored)
     if (threadIdx.x < kFuseMaxRows + 4) {
         const uint32_t r = r_begin + threadIdx.x < r_end ? r_begin + threadIdx.x : r_end - 1;
-        rtable[threadIdx.x] = p.b.out_table[d.map_off + r];
+        rtable[threadIdx.x] = map_table(a.map, d.limb(r));
     }
     // the inputs: bytes 0..6 as signed numbers (x - 128), byte 7 (zero: the residues are below 2^50) stays zero
-    const uint64_t *x = p.b.x_base + item * p.b.x_item_stride + d.x_off;
+    const uint64_t *x = d.in;
     const uint32_t l0 = 2 * kg < d.n_in ? 2 * kg : d.n_in - 1, l1 = 2 * kg + 1 < d.n_in ? 2 * kg + 1 : d.n_in - 1;
     // (a uniform base and 32-bit byte offsets: one address register per load in flight instead of two)
     const char *xbytes = reinterpret_cast<const char *>(x);
@@ -412,9 +408,9 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
             for (int i = 0; i < 8; i++) tl[threadIdx.x + 256 * i] = tw[i];   // tile word (row << 3) | column
         }
         lds_barrier();
-        const uint32_t ltable = p.b.out_table[d.map_off + d.n_out - 1];
+        const uint32_t ltable = map_table(a.map, d.n_out - 1);
         const FpMod ml{a.fp_consts[4 * (size_t)ltable], a.fp_consts[4 * (size_t)ltable + 1]};
-        const v4i *lrec = reinterpret_cast<const v4i *>(p.b.mx_last);
+        const v4i *lrec = static_cast<const v4i *>(b.w);
         const v4i la = lrec[lane], lh = lrec[64 + lane];
         const double *loff = reinterpret_cast<const double *>(lrec + 128);
         const double off = loff[0];
@@ -444,7 +440,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
         }
         lds_barrier();   // the tiles are free again
     }
-    const v4i *rec = reinterpret_cast<const v4i *>(p.b.mx_tab) + ((size_t)d.mx_off + (r_begin >> 2)) * kMxRecord;
+    const v4i *rec = static_cast<const v4i *>(b.mat) + ((size_t)d.mx_off + (r_begin >> 2)) * kMxRecord;
     lds_barrier();   // rtable
 
     // Twiddles: entries 1..63 of a row's table serve the first two blocks, 64..255 the third.  Thread t fetches entry
@@ -462,7 +458,7 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
         if (threadIdx.x >= 16 && threadIdx.x < 20) {
             const uint32_t rr = threadIdx.x - 16;
             const uint32_t r = r_begin + 4 * k + rr < r_end ? r_begin + 4 * k + rr : r_end - 1;
-            rlimb[k & 1][rr] = p.b.out_limb[d.map_off + r];
+            rlimb[k & 1][rr] = d.limb(r);
         }
     };
     twl[trow][tcol] = low_part(0);
@@ -574,12 +570,14 @@ void bconv_rows_mx_kernel(NttArgs a, BconvRowsK p) {
 }  // namespace
 
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s) {
-    if (a.log_n < 12 || a.log_n > 16 || b.n_units == 0) return hipErrorInvalidValue;
+    if (a.log_n < 12 || a.log_n > 16 || b.units == 0 || b.K == 0 || b.K > 8) return hipErrorInvalidValue;
     const uint32_t forced = tune.fuse_rows_forced <= kFuseMaxRows ? tune.fuse_rows_forced : 0;
     const uint32_t items = b.items ? b.items : 1;
     const int ld = (int)a.log_n - 8;
     const uint32_t tiles = 256u >> (kFuseLog - ld);
-    const uint32_t rows = b.mdr ? b.max_rows - 1 : b.max_rows;
+    // (the most of a unit: ModUp, the last digit's)
+    const uint32_t L = b.map.split, last = L % b.K ? L % b.K : b.K;
+    const uint32_t rows = b.up ? b.map.limbs - last : b.mdr ? L - 1 : L;
     if (rows == 0) return hipErrorInvalidValue;
     // Output limbs per workgroup.  The kernel is bound by instruction issue, so a CU's time is the number of workgroups
     // it is dealt times a workgroup's work: r rows plus about 1.5 rows' worth of fetching and converting its 8 x 8 block
@@ -593,14 +591,14 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     // work that pays once a workgroup has many rows, i.e. once the launch fills the chip without splitting the rows:
     // 106 against 122 us for 8 operations, 27.8 against 25.4 us for one)
     const bool mx = ld == 8 && b.mat_fp && b.mx_tab && !tune.no_matrix_bconv &&
-                    (!b.mdr || (b.mx_last && (uint64_t)b.n_units * items * tiles >= (tune.cus ? tune.cus : 256)));
+                    (!b.mdr || (b.mx_last && (uint64_t)b.units * items * tiles >= (tune.cus ? tune.cus : 256)));
     const uint32_t step = mx ? 4 : 1;
     uint32_t target = mx ? (forced + 3) / 4 * 4 : forced;
     if (!target) {
         const uint32_t cus = tune.cus ? tune.cus : 256;
         uint64_t best = ~0ull;
         for (uint32_t r = step; r <= kFuseMaxRows && r < rows + step; r += step) {
-            const uint64_t wgs = (uint64_t)b.n_units * items * tiles * ((rows + r - 1) / r);
+            const uint64_t wgs = (uint64_t)b.units * items * tiles * ((rows + r - 1) / r);
             const uint64_t per_cu = (wgs + cus - 1) / cus;
             const uint64_t cost = (per_cu < 2 ? 2 : per_cu) * (2 * r + 3);
             if (cost < best) {
@@ -609,20 +607,27 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
             }
         }
     }
-    BconvRowsK p{b, (rows + target - 1) / target, 0, target, 0};
-    p.copy_groups = b.copy_base ? (b.max_copy + target - 1) / target : 0;
-    const uint64_t wgs = (uint64_t)b.n_units * items * tiles * (p.compute_groups + p.copy_groups);
+    const uint32_t compute_groups = (rows + target - 1) / target, copy_groups = b.copy_base ? ((L < b.K ? L : b.K) + target - 1) / target : 0;
+    const uint64_t wgs = (uint64_t)b.units * items * tiles * (compute_groups + copy_groups);
     if (wgs > most_workgroups(256)) return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)wgs);
-    p.wgs = (uint32_t)wgs;
+    NttArgs m = a;
+    m.in = b.in;
+    m.out = b.out;
+    m.map = b.map;
+    m.pro_mode = b.up;
+    if (!b.mat_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;
+    NttHead h = ntt_head(m, (uint32_t)wgs, target);
+    h.h1 = b.units | b.K << 16;
+    h.h2 = compute_groups | copy_groups << 16;
     if (mx) {
+        const BconvExtra x{b.mx_tab, b.mx_last, b.copy_base, b.copy_item_stride};
         if (b.mdr)
-            hipLaunchKernelGGL(bconv_rows_mx_kernel<true>, grid, dim3(256), 0, s, a, p);
+            hipLaunchKernelGGL(bconv_rows_mx_kernel<true>, dim3(h.h4), dim3(256), 0, s, HE_HEAD_ARGS(h), x);
         else
-            hipLaunchKernelGGL(bconv_rows_mx_kernel<false>, grid, dim3(256), 0, s, a, p);
+            hipLaunchKernelGGL(bconv_rows_mx_kernel<false>, dim3(h.h4), dim3(256), 0, s, HE_HEAD_ARGS(h), x);
         return hipGetLastError();
     }
-    return launch_bconv_rows4(a, b, p.compute_groups, p.copy_groups, target, backend, s);
+    return launch_bconv_rows4(h, b, s);
 }
 
 hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, hipStream_t s, bool rows_done) {

@@ -17,6 +17,9 @@
 // 233 -> 219; L = 24, K = 8 the same 150 us.  Levels with a prime from 2^50 on against conversion kernel + rows pass: n = 2^15, 10 of
 // 12 limbs of 60 / 40 bits 77.5 -> 71.6 us; n = 2^13, 6 limbs, K = 2 45.4 -> 38.3; n = 2^16, 24 + 8 limbs 217 -> 204; a batch of 8,
 // n = 2^15, 12 limbs, K = 3 323 -> 277.
+// The unit, its rows and their primes are worked out from a few scalars (BconvUnit): looked up in the arguments, a description and two
+// lists, one behind the other, they cost 1.2 us a product (n = 2^15, 10 of 12 limbs of 60 / 40 bits 67.4 -> 66.1 us; n = 2^13, 6
+// limbs, K = 2 36.2 -> 35.1; n = 2^16, 24 + 8 limbs 141.8 -> 139.8).
 #include <hip/hip_runtime.h>
 
 #include <type_traits>
@@ -31,28 +34,15 @@ namespace {
 
 constexpr int kTileLog = 11;
 
-typedef const uint32_t __attribute__((address_space(4))) *ScalarU32;
-__device__ __forceinline__ ScalarU32 scalar(const uint32_t *p) { return (ScalarU32)(uintptr_t)p; }
-
-__device__ __forceinline__ BconvDesc load_desc(const BconvDesc *p) {
-    static_assert(sizeof(BconvDesc) % 8 == 0, "read as 8-byte words");
-    BconvDesc d;
-    uint64_t w[sizeof(BconvDesc) / 8];
-#pragma unroll
-    for (size_t i = 0; i < sizeof(BconvDesc) / 8; i++) w[i] = scalar(reinterpret_cast<const uint64_t *>(p))[i];
-    __builtin_memcpy(&d, w, sizeof(d));
-    return d;
-}
-
 // Conversion in FP64 (every prime of the level below 2^50)
 template <int NIN, bool MDR>
 struct ConvFp {
     double x[NIN][4], rr[MDR ? 4 : 1];
     __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = fp_from_u64(w); }
-    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvRows &b, const BconvDesc &d, const uint64_t *t) {
+    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
         const uint32_t last = d.n_out - 1;
-        const FpMod m = fp_ctx(a, scalar(b.out_table)[d.map_off + last]).m;
-        const ScalarF64 row = scalar(b.mat_fp) + 2 * (d.mat_off + (size_t)last * d.n_in);
+        const FpMod m = fp_ctx(a, map_table(a.map, last)).m;
+        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + 2 * (d.mat_off + (size_t)last * d.n_in);
 #pragma unroll
         for (int j = 0; j < 4; j++) rr[j] = fp_from_u64(t[j]);
 #pragma unroll
@@ -70,9 +60,9 @@ struct ConvFp {
     // it under 2^104), t - hi is exact, x w - (t - hi) is the rounding error, an integer of at most 2^50 in magnitude that the
     // second fused multiply-add returns exactly, and eight of those sum exactly.  (hi - 2^103) / 2^51 is an integer below
     // 2^52; times 2^51 mod m it is congruent to the high part, and the modular product takes it as it is.
-    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvRows &b, const BconvDesc &d, uint32_t r, uint32_t,
+    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t,
                                             const FpArith &ar) const {
-        const ScalarF64 row = scalar(b.mat_fp) + 2 * (d.mat_off + (size_t)r * d.n_in);
+        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + 2 * (d.mat_off + (size_t)r * d.n_in);
         double hi[4], lo[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -125,29 +115,29 @@ struct ConvInt {
         o[0] = barrett128(a0.lo, a0.hi, q, r0, r1);
         o[1] = barrett128(a1.lo, a1.hi, q, r0, r1);
     }
-    __device__ __forceinline__ void sums(uint64_t *o, const NttArgs &a, const BconvRows &b, const BconvDesc &d, uint32_t r, uint32_t table) const {
+    __device__ __forceinline__ void sums(uint64_t *o, const NttArgs &a, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t table) const {
         const uint64_t q = scalar(a.moduli)[table], r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
-        const uint64_t *row = b.mat + d.mat_off + (size_t)r * d.n_in;
+        const uint64_t *row = static_cast<const uint64_t *>(b.mat) + d.mat_off + (size_t)r * d.n_in;
         sum(o, 0, row, d.n_in, q, r0, r1);
         sum(o + 2, 2, row, d.n_in, q, r0, r1);
     }
-    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvRows &b, const BconvDesc &d, const uint64_t *t) {
-        const uint32_t last = d.n_out - 1, table = scalar(b.out_table)[d.map_off + last];
+    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
+        const uint32_t last = d.n_out - 1, table = map_table(a.map, last);
         const uint64_t q = scalar(a.moduli)[table];
-        const Shoup w = scalar_shoup(b.w, last);
+        const Shoup w = scalar_shoup(static_cast<const uint64_t *>(b.w), last);
         uint64_t s[4];
         sums(s, a, b, d, last, table);
 #pragma unroll
         for (int j = 0; j < 4; j++) rr[j] = sub_mod(t[j], mul_shoup(s[j], w, q), q);
     }
     template <class A>
-    __device__ __forceinline__ void convert(typename A::V *v, const NttArgs &a, const BconvRows &b, const BconvDesc &d, uint32_t r,
+    __device__ __forceinline__ void convert(typename A::V *v, const NttArgs &a, const BconvExtra &b, const BconvUnit &d, uint32_t r,
                                             uint32_t table, const A &) const {
         uint64_t s[4];
         sums(s, a, b, d, r, table);
         if constexpr (MDR) {
             const uint64_t q = scalar(a.moduli)[table], r1 = scalar(a.barrett)[2 * table + 1];
-            const Shoup w = scalar_shoup(b.w, r);
+            const Shoup w = scalar_shoup(static_cast<const uint64_t *>(b.w), r);
 #pragma unroll
             for (int j = 0; j < 4; j++) s[j] = add_mod(mul_shoup(s[j], w, q), barrett64(rr[j], q, r1), q);
         }
@@ -165,19 +155,20 @@ struct ConvInt {
 // arithmetic the limb is transformed
 template <int LD, bool FP, int NIN, bool MDR>
 __global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(FP || NIN <= 4 ? 4 : 2)))
-void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per, uint32_t wgs) {
+void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     using T4 = Tile4<kTileLog, LD>;
     constexpr int LOGC = kTileLog - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
     // (two tiles in turn: the barriers of one output limb say that the tile of the limb before is free again)
     __shared__ uint64_t lds[2][(1 << kTileLog) + (1 << (kTileLog - 4))];
-    touch_arguments<sizeof(NttArgs) + sizeof(BconvRows)>();
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
     const size_t n = (size_t)1 << a.log_n;
-    uint32_t lb = logical_block(wgs);
-    const uint32_t groups = compute_groups + copy_groups, grp = lb % groups;
+    uint32_t lb = logical_block(h4);
+    const uint32_t compute_groups = h2 & 0xffff, groups = compute_groups + (h2 >> 16), grp = lb % groups, rows_per = h5;
     lb /= groups;
-    const uint32_t col0 = (lb % tiles_per_limb) << LOGC, uidx = lb / tiles_per_limb, item = uidx / b.n_units;
-    const BconvDesc d = load_desc(b.descs + (uidx - item * b.n_units));
+    const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
+    const BconvUnit d = bconv_unit(a, h1 & 0xffff, h1 >> 16, lb / tiles_per_limb);
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     // word j of layout k: a scalar distance from the lane's first one
     auto first = [&](int k) {
@@ -189,18 +180,17 @@ void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_
         return (e >> LOGC) * 256 + (e & (C - 1));
     };
     const uint32_t in0 = first(0), out0 = first(NB - 1);
-    uint64_t *out = b.out_base + item * b.out_item_stride + d.out_off;
     if (grp >= compute_groups) {
         // limbs that pass through unchanged (a digit's own limbs keep their NTT form)
-        const uint64_t *from = b.copy_base + item * b.copy_item_stride;
+        const uint64_t *from = b.copy_base + d.item * b.copy_item_stride;
         const uint32_t c0 = (grp - compute_groups) * rows_per;
-        for (uint32_t r = c0; r < c0 + rows_per && r < d.copy_count; r++) {
+        for (uint32_t r = c0; r < c0 + rows_per && r < d.n_in; r++) {
             const size_t limb = (size_t)(d.copy_first + r) << a.log_n;
             uint64_t w[4];
 #pragma unroll
             for (int j = 0; j < 4; j++) w[j] = (from + limb + step(0, j))[in0];
 #pragma unroll
-            for (int j = 0; j < 4; j++) (out + limb + step(0, j))[in0] = w[j];
+            for (int j = 0; j < 4; j++) (d.out + limb + step(0, j))[in0] = w[j];
         }
         return;
     }
@@ -208,7 +198,7 @@ void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_
     const uint32_t r_end = r_begin + rows_per < n_rows ? r_begin + rows_per : n_rows;
     if (r_begin >= n_rows) return;
     typename std::conditional<FP, ConvFp<NIN, MDR>, ConvInt<NIN, MDR>>::type conv;
-    const uint64_t *x = b.x_base + item * b.x_item_stride + d.x_off;
+    const uint64_t *x = d.in;
     {
         uint64_t w[NIN][4], tw[4];
 #pragma unroll
@@ -228,8 +218,8 @@ void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_
         if constexpr (MDR) conv.dropped(a, b, d, tw);
     }
     for (uint32_t r = r_begin; r < r_end; r++) {
-        const uint32_t table = scalar(b.out_table)[d.map_off + r], limb = scalar(b.out_limb)[d.map_off + r];
-        uint64_t *dst = out + ((size_t)limb << a.log_n), *tile = lds[(r - r_begin) & 1];
+        const uint32_t limb = d.limb(r), table = map_table(a.map, limb);
+        uint64_t *dst = d.out + ((size_t)limb << a.log_n), *tile = lds[(r - r_begin) & 1];
         auto row = [&](const auto &ar) {
             using A = typename std::remove_cv<typename std::remove_reference<decltype(ar)>::type>::type;
             typename A::V v[4];
@@ -252,13 +242,11 @@ void bconv_rows4_kernel(NttArgs a, BconvRows b, uint32_t compute_groups, uint32_
 }
 
 template <bool FP, int NIN, bool MDR>
-hipError_t launch_nin(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per,
-                      dim3 grid, hipStream_t s) {
-    switch (a.log_n - 8) {
-#define HE_CASE(LD)                                                                                                          \
-    case LD:                                                                                                                 \
-        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR>), grid, dim3(1 << (kTileLog - 2)), 0, s, a, b, compute_groups,   \
-                           copy_groups, rows_per, grid.x);                                                                           \
+hipError_t launch_nin(const NttHead &h, uint32_t log_n, const BconvExtra &b, hipStream_t s) {
+    switch (log_n - 8) {
+#define HE_CASE(LD)                                                                                                              \
+    case LD:                                                                                                                     \
+        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR>), dim3(h.h4), dim3(1 << (kTileLog - 2)), 0, s, HE_HEAD_ARGS(h), b); \
         break;
         HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
 #undef HE_CASE
@@ -269,17 +257,15 @@ hipError_t launch_nin(const NttArgs &a, const BconvRows &b, uint32_t compute_gro
 
 }  // namespace
 
-hipError_t launch_bconv_rows4(const NttArgs &a, const BconvRows &b, uint32_t compute_groups, uint32_t copy_groups, uint32_t rows_per,
-                              int backend, hipStream_t s) {
-    const uint64_t wgs = (uint64_t)b.n_units * (b.items ? b.items : 1) * (1u << (a.log_n - kTileLog)) * (compute_groups + copy_groups);
-    if (a.log_n < 12 || a.log_n > 16 || b.max_in == 0 || b.max_in > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
+hipError_t launch_bconv_rows4(const NttHead &head, const BconvRows &b, hipStream_t s) {
+    NttHead h = head;
+    const uint32_t log_n = h.h0 & 31, groups = (h.h2 & 0xffff) + (h.h2 >> 16);
+    const uint64_t wgs = (uint64_t)b.units * (b.items ? b.items : 1) * (1u << (log_n - kTileLog)) * groups;
+    if (log_n < 12 || log_n > 16 || b.K == 0 || b.K > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
         return hipErrorInvalidValue;
-    const dim3 grid((uint32_t)wgs);
-    NttArgs m = a;
-    if (!b.mat_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;
-#define HE_NIN(FP, MDR)                                                                              \
-    (b.max_in <= 4 ? launch_nin<FP, 4, MDR>(m, b, compute_groups, copy_groups, rows_per, grid, s)     \
-                   : launch_nin<FP, 8, MDR>(m, b, compute_groups, copy_groups, rows_per, grid, s))
+    h.h4 = (uint32_t)wgs;
+    const BconvExtra x{b.mat_fp ? static_cast<const void *>(b.mat_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride};
+#define HE_NIN(FP, MDR) (b.K <= 4 ? launch_nin<FP, 4, MDR>(h, log_n, x, s) : launch_nin<FP, 8, MDR>(h, log_n, x, s))
     if (b.mat_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
     return b.mdr ? HE_NIN(false, true) : HE_NIN(false, false);
 #undef HE_NIN

@@ -82,6 +82,43 @@ __device__ __forceinline__ void set_inverse_block(NttArgs &a, const uint64_t *bl
     a.pro_itw_fp = block_fp(block, a.size_qp, a.log_n);
 }
 
+// A unit of a fused base conversion (BconvRows), worked out from the workgroup's number: looked up, it was a trip to memory before the
+// one for the words.
+struct BconvUnit {
+    uint32_t item, copy_first, n_in, n_out;   // (copy_first: the first of a digit's own limbs)
+    const uint64_t *in;
+    uint64_t *out;
+    size_t mat_off;
+    uint32_t mx_off;
+    bool up;
+    __device__ __forceinline__ uint32_t limb(uint32_t row) const { return up && row >= copy_first ? row + n_in : row; }
+};
+
+__device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units, uint32_t K, uint32_t index) {
+    const uint32_t L = a.map.split, LK = a.map.limbs;
+    BconvUnit u;
+    u.up = a.pro_mode;
+    u.item = index / units;
+    u.copy_first = u.mx_off = 0;
+    u.mat_off = 0;
+    u.n_in = K;
+    u.n_out = L;
+    if (u.up) {
+        const uint32_t d = index - u.item * units;
+        u.copy_first = d * K;
+        u.n_in = u.copy_first + K < L ? K : L - u.copy_first;
+        u.n_out = LK - u.n_in;
+        u.mat_off = (size_t)u.copy_first * (LK - K);
+        u.mx_off = d * ((LK - K + 3) / 4);
+        u.in = a.in + (((size_t)u.item * L + u.copy_first) << a.log_n);
+        u.out = a.out + ((size_t)index * LK << a.log_n);
+    } else {
+        u.in = a.in + (((size_t)index * LK + L) << a.log_n);
+        u.out = a.out + ((size_t)index * L << a.log_n);
+    }
+    return u;
+}
+
 struct Job {
     const uint64_t *in;
     uint64_t *out;

@@ -806,11 +806,13 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
 }
 
 template <int BE>
-__global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(NttArgs a, TensorFuse x) {
-    touch_arguments<sizeof(NttArgs) + sizeof(TensorFuse)>();
+__global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(HE_HEAD_PARAMS, const uint64_t *ct2, uint64_t *d01, uint64_t *d2) {
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    const TensorFuse x{h_in, ct2, d01, d2, a.map.limbs, (int)h5};
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block(x.wgs) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const uint32_t id = logical_block(h4) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane);
@@ -1243,19 +1245,20 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     return hipGetLastError();
 }
 
-hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &fuse, uint32_t items, int backend, hipStream_t s) {
-    TensorFuse x = fuse;
+hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, uint32_t items, int backend, hipStream_t s) {
+    NttArgs a = args;
+    a.in = x.ct1;
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs != x.L || x.L == 0 || items == 0) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
-    x.wgs = (uint32_t)wgs;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    const NttHead h = ntt_head(a, grid.x, x.square ? 1 : 0);
     if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, a, x);
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
     else if (backend)
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, a, x);
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
     else
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, a, x);
+        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
     return hipGetLastError();
 }
 
