@@ -1385,7 +1385,9 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     inv.map = LimbMap{K + 1, L - 1, 1, ctx->size_q};
     inv.epi_mode = NTT_EPI_MUL;
     inv.w = lv->d_mdr_w;
-    HE_HIP(launch_ntt_inverse(inv, polys, inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map), S(s), inverted));
+    const int inv_backend = inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map);
+    const bool source_intt = ctx->single_limb_digits && !ctx->tune.no_source_intt && ntt_two_sources_ok(ctx->log_n, polys * (L - 1), ctx->size_qp);
+    HE_HIP(launch_ntt_inverse(inv, polys, inv_backend, S(s), inverted, source_intt));
     // (3) delta = P -> Ql conversion of the special limbs
     const bool fused = fuse_rows_ok(ctx, lv, L);
     // one special prime: the conversion is the reduction of its coefficients modulo every q_j, which the prologue of (4)
@@ -1427,6 +1429,13 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
         fwd.pro_src2 = cx + (size_t)L * n;
         fwd.pro2_poly_stride = LK;
         fwd.pro_k1 = 1;
+        if (source_intt) {
+            // (the rest of (2), where the prologue reads its sources)
+            fwd.pro_src_fp_mask = fp_mask_of(ctx, inv_backend);
+            fwd.pro_src_table = ctx->size_q;
+            fwd.pro_itw = ctx->d_ipsi;
+            fwd.pro_itw_fp = ctx->d_ipsi_fp;
+        }
     }
     fwd.epi_mode = NTT_EPI_FMA_SUB_MUL;
     fwd.epi_a = cx;

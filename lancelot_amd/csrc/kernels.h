@@ -202,6 +202,8 @@ hipError_t launch_ntt_rows(const NttArgs &a, uint32_t n_jobs, bool forward, int 
 hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int backend, hipStream_t s);
 // whether a forward launch of n_jobs limbs may take NTT_PRO_SOURCE_INTT_REDUCE
 bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables);
+// ... and one with NTT_PRO_MODDOWN_RESCALE and one special prime (pro_k1) the inverse rows passes of its two sources (pro_itw)
+bool ntt_two_sources_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables);
 
 // Tensor product of two size-2 ciphertexts fused with the blocks pass of the inverse transform of its third polynomial, for
 // `items` products (operands and d01 [items][2][L][N], d2 [items][L][N]).  `a`: inverse base arguments with map = the L data

@@ -224,8 +224,10 @@ __device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Jo
 // doubles; returns whether they have to be reduced before the first stage (else they are canonical).
 // MDR: the launch's mode is NTT_PRO_MODDOWN_RESCALE (a template argument: its operands cost the other modes registers, 90 instead of
 // 64 for the mixed rows pass; encryption 69.1 -> 68.6 us, a Krum round of 10 clients 4.30 -> 4.23 ms)
-template <bool MDR, int W, typename Glob>
-__device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, const Job &job, const FpCtx &c, Glob glob) {
+// GIVEN: its two sources are in ts and ds already.
+template <bool MDR, bool GIVEN, int W, typename Glob>
+__device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, const Job &job, const FpCtx &c, Glob glob, const uint64_t *ts,
+                                              const uint64_t *given_ds) {
     if constexpr (MDR) {
         const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
         const uint64_t *dsrc = a.pro_src2 + ((size_t)job.poly * a.pro2_poly_stride << a.log_n);
@@ -235,11 +237,11 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t qlast = scalar(a.moduli)[a.pro_last], rlast = scalar(a.barrett)[2 * a.pro_last + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) {
-            const uint64_t ds = dsrc[glob(j)];
-            const uint64_t dl = a.pro_k1 ? barrett64(ds, qlast, rlast) : ds;
-            const uint64_t dj = a.pro_k1 ? barrett64(ds, qj, rj) : job.in[glob(j)];
+            const uint64_t ds = GIVEN ? given_ds[j] : dsrc[glob(j)], t = GIVEN ? ts[j] : tsrc[glob(j)];
+            const uint64_t dl = GIVEN || a.pro_k1 ? barrett64(ds, qlast, rlast) : ds;
+            const uint64_t dj = GIVEN || a.pro_k1 ? barrett64(ds, qj, rj) : job.in[glob(j)];
             // coefficient of the dropped limb of the ModDown result, canonical mod q_last
-            const double r = fp_canonical(fp_from_u64(tsrc[glob(j)]) - fp_mulmod(fp_from_u64(dl), wlast, ml), ml);
+            const double r = fp_canonical(fp_from_u64(t) - fp_mulmod(fp_from_u64(dl), wlast, ml), ml);
             v[j] = fp_mulmod(fp_from_u64(dj), w, c.m) + fp_reduce(r, c.m);
         }
         return true;
@@ -271,8 +273,9 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
 }
 
 // The same on the integer back end: residues below q.
-template <bool MDR, int W, typename Glob>
-__device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &a, const Job &job, uint64_t q, Glob glob) {
+template <bool MDR, bool GIVEN, int W, typename Glob>
+__device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &a, const Job &job, uint64_t q, Glob glob, const uint64_t *ts,
+                                               const uint64_t *given_ds) {
     if constexpr (MDR) {
         const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
         const uint64_t *tsrc = a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n);
@@ -282,10 +285,10 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
         const uint64_t rlast = scalar(a.barrett)[2 * a.pro_last + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) {
-            const uint64_t ds = dsrc[glob(j)];
-            const uint64_t dl = a.pro_k1 ? barrett64(ds, ql, rlast) : ds;
-            const uint64_t dj = a.pro_k1 ? barrett64(ds, q, r1) : job.in[glob(j)];
-            const uint64_t r = sub_mod(tsrc[glob(j)], mul_shoup(dl, wlast, ql), ql);
+            const uint64_t ds = GIVEN ? given_ds[j] : dsrc[glob(j)], t = GIVEN ? ts[j] : tsrc[glob(j)];
+            const uint64_t dl = GIVEN || a.pro_k1 ? barrett64(ds, ql, rlast) : ds;
+            const uint64_t dj = GIVEN || a.pro_k1 ? barrett64(ds, q, r1) : job.in[glob(j)];
+            const uint64_t r = sub_mod(t, mul_shoup(dl, wlast, ql), ql);
             v[j] = add_mod(mul_shoup(dj, w, q), barrett64(r, q, r1), q);
         }
     } else if (a.pro_mode == NTT_PRO_BROADCAST_REDUCE || a.pro_mode == NTT_PRO_SOURCE_REDUCE) {

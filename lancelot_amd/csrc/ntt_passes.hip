@@ -25,7 +25,7 @@ namespace {
 
 // What a rows pass's mode needs behind NttHead.
 struct RowsExtra {
-    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_INTT_REDUCE: pro_itw; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2, pro_w
+    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_INTT_REDUCE: pro_itw; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2 (or pro_itw), pro_w
     uint64_t u0, u1, mask;          // list: item_stride, pro_item_stride; NTT_PRO_ROUND: pro_fix; NTT_PRO_MODDOWN_RESCALE: strides, pro_last and pro_k1
     uint32_t w0;                    // inverse: epi_mode; NTT_PRO_SOURCE_INTT_REDUCE in map mode: pro_src_table
 };
@@ -37,6 +37,13 @@ RowsExtra rows_extra(const NttArgs &a, bool fwd) {
         e.w0 = (uint32_t)a.epi_mode;
     } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
         e.p0 = a.pro_itw;
+        e.w0 = a.pro_src_table;
+    } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE && a.pro_itw) {
+        e.p0 = a.pro_src;
+        e.p1 = a.pro_itw;
+        e.p2 = a.pro_w;
+        e.u0 = a.pro_poly_stride;
+        e.u1 = a.pro_last;
         e.w0 = a.pro_src_table;
     } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE) {
         e.p0 = a.pro_src;
@@ -58,11 +65,19 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
     a.pro_item_stride = e.u1;
     a.pro_fix = __longlong_as_double((long long)e.u0);
     if constexpr (SRC_INTT) {
-        set_inverse_block(a, e.p0);
+        set_inverse_block(a, MDR ? e.p1 : e.p0);
         a.pro_src_fp_mask = e.mask;
         a.pro_src_table = e.w0;
     }
-    if constexpr (MDR) {
+    if constexpr (MDR && SRC_INTT) {
+        // (the special limb lies behind the dropped one)
+        a.pro_src = e.p0;
+        a.pro_src2 = e.p0 + ((size_t)1 << a.log_n);
+        a.pro_w = e.p2;
+        a.pro_poly_stride = a.pro2_poly_stride = (uint32_t)e.u0;
+        a.pro_last = (uint32_t)e.u1;
+        a.pro_k1 = 1;
+    } else if constexpr (MDR) {
         a.pro_src = e.p0;
         a.pro_src2 = e.p1;
         a.pro_w = e.p2;
@@ -73,13 +88,12 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
     }
 }
 
-// The inverse rows pass of the source limb's tile: lazy words of the last block's layout become canonical coefficients in the first
+// The inverse rows pass of a source limb's tile: lazy words of the last block's layout become canonical coefficients in the first
 // block's.  (Behind the request of the forward twiddles: the exchanges' compiler barriers would hold that back until the inverse
 // pass has ended.)
 template <class T4>
-__device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a, const Job &job, uint64_t *lds, uint32_t t) {
+__device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a, uint32_t st, uint64_t *lds, uint32_t t) {
     constexpr int NB = T4::kBlocks;
-    const uint32_t st = job.src_table;
     if ((a.pro_src_fp_mask >> st) & 1) {
         const FpArith ar{fp_ctx(a, st).m, a.pro_itw_fp + ((size_t)st << a.log_n)};
         double v[4];
@@ -107,7 +121,8 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
 // Rows pass.  The thread index is (wave, lane), the wave the same scalar in all its lanes, so that the twiddles of the
 // first two blocks come through scalar loads.
 // SRC_INTT (forward, NTT_PRO_SOURCE_INTT_REDUCE): the inverse rows pass of the source limb's tile runs first; it leaves the
-// coefficients where the forward pass takes them from.
+// coefficients where the forward pass takes them from.  With MDR (one special prime) those of the dropped limb and of the special
+// one behind it, which every output limb's workgroup transforms anew: a launch less, and CUs that were idle (see ntt_two_sources_ok).
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
 template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B>
 __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, RowsExtra x) {
@@ -115,22 +130,31 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
     using T4 = Tile4<B, LD>;
     constexpr int LOGC = B - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
-    __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))];
+    __shared__ uint64_t lds[(1 << B) + (1 << (B - 4))], lds2[SRC_INTT && MDR ? (1 << B) + (1 << (B - 4)) : 1];
     set_head(a, HE_HEAD_NAMES);
     set_extra<FWD, SRC_INTT, MDR>(a, x);
     const uint32_t lb = logical_block(h4);
-    const Job job = decode_job<SRC_INTT>(a, a.first_job + lb / tiles_per_limb);
+    const Job job = decode_job<SRC_INTT && !MDR>(a, a.first_job + lb / tiles_per_limb);
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     auto glob = [&](int k, int j) {
         const uint32_t e = T4::word(k, t, j);
         return (size_t)(e >> LOGC) * 256 + col0 + (e & (C - 1));
     };
-    uint64_t s[4];   // canonical coefficients of the source limb
+    uint64_t s[4], s2[4];   // canonical coefficients of the source limbs
     if constexpr (SRC_INTT) {
+        const uint64_t *src = MDR ? a.pro_src + ((size_t)job.poly * a.pro_poly_stride << a.log_n) : job.src;
 #pragma unroll
-        for (int j = 0; j < 4; j++) s[j] = job.src[glob(NB - 1, j)];
+        for (int j = 0; j < 4; j++) s[j] = src[glob(NB - 1, j)];
+        if constexpr (MDR) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) s2[j] = (src + ((size_t)1 << a.log_n))[glob(NB - 1, j)];
+        }
     }
+    auto sources = [&]() {
+        source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t);
+        if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t);
+    };
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) {
         const FpCtx c = fp_ctx(a, job.table);
@@ -139,12 +163,12 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
         FpArith::Tw tw[NB];
         if (FWD) {
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-            if constexpr (SRC_INTT) {
-                source_words<T4>(s, a, job, lds, t);
+            if constexpr (SRC_INTT) sources();
+            if constexpr (SRC_INTT && !MDR) {
                 const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
-            } else if (rows_input_fp<MDR>(v, a, job, c, [&](int j) { return glob(0, j); })) {
+            } else if (rows_input_fp<MDR, SRC_INTT>(v, a, job, c, [&](int j) { return glob(0, j); }, s, s2)) {
                 ar.reduce(v);
             }
             T4::template forward<FpArith>(v, tw, ar, lds, t);
@@ -170,13 +194,13 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
         IntArith::Tw tw[NB];
         if (FWD) {
             T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
-            if constexpr (SRC_INTT) {
-                source_words<T4>(s, a, job, lds, t);
+            if constexpr (SRC_INTT) sources();
+            if constexpr (SRC_INTT && !MDR) {
                 const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
             } else {
-                rows_input_int<MDR>(v, a, job, q, [&](int j) { return glob(0, j); });
+                rows_input_int<MDR, SRC_INTT>(v, a, job, q, [&](int j) { return glob(0, j); }, s, s2);
             }
             T4::template forward<IntArith>(v, tw, ar, lds, t);
             // lazy values in [0, 4q) go to the blocks pass
@@ -1081,6 +1105,14 @@ bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
     return log_n >= 12 && log_n <= 16 && n_tables <= 64 && ((uint64_t)n_jobs << log_n) <= ((uint64_t)16 << 16);
 }
 
+// ModDown + rescale with one special prime: two inverse rows passes in front of every output limb's, which pay as long as the launch is
+// small.  n limbs in all, us of a multiplication with a launch for them -> without (50 bits / 60 bits): n = 2^12, L = 2 26.0 -> 21.9 /
+// 27.2 -> 25.0; 2^14, L = 4 26.1 -> 23.0 / 31.4 -> 28.7; 2^15, L = 8 47.1 -> 45.7 / 62.8 -> 61.8; 2^16, L = 4 39.9 -> 38.5 / 54.7 ->
+// 54.9, L = 6 55.7 -> 55.0 / 72.9 -> 76.1.
+bool ntt_two_sources_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
+    return ntt_source_intt_ok(log_n, n_jobs, n_tables) && ((uint64_t)n_jobs << log_n) <= ((uint64_t)7 << 16);
+}
+
 hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, int backend, hipStream_t s) {
     if (args.log_n < 9 || args.log_n > 17) return hipErrorInvalidValue;
     NttArgs a = args;
@@ -1094,6 +1126,11 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
         if (!forward || !a.pro_itw || (a.pro_src_fp_mask && !a.pro_itw_fp)) return hipErrorInvalidValue;
         a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
         return launch_rows<true, NTT_BACKEND_MIXED, true>(a, n_jobs, s);
+    }
+    if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE && a.pro_itw) {
+        if (!a.pro_k1 || a.pro_poly_stride != a.pro2_poly_stride || a.pro_src2 != a.pro_src + ((size_t)1 << a.log_n)) return hipErrorInvalidValue;
+        a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+        return launch_rows<true, NTT_BACKEND_MIXED, true, true>(a, n_jobs, s);
     }
     if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE)
         return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED, false, true>(a, n_jobs, s)

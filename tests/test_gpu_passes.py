@@ -369,3 +369,25 @@ def test_decryption_where_the_noise_has_a_launch_of_its_own_and_where_not(oracle
     out, noise = DeviceArray(capi, shape=(limbs, p.n)), DeviceArray(capi, shape=(p.n // 8,))
     capi.check(lib.he_decrypt_flood(h, dct.ptr, 2, limbs, dsk.ptr, limbs * p.n, kp, 2 ** 40 + 5, dcdt.ptr, len(cdt), out.ptr, noise.ptr, None))
     assert (out.numpy() == p.add(p.mul_add(ct[1], s, ct[0]), p.ntt_fwd(p.sample_gauss(key, 2 ** 40 + 5, limbs, cdt)))).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,L,items", [(11, 3, 1), (12, 2, 1), (13, 5, 3), (14, 4, 8), (14, 4, 10), (15, 8, 1), (15, 9, 1), (16, 4, 1), (16, 5, 1)])
+def test_key_switch_and_rescale_of_few_limbs(oracle, capi, chain, logn, L, items):
+    """One special prime: up to 7 * 2^16 output words the forward pass starts with the inverse passes of the dropped and the special limb."""
+    bits = (CHAINS[chain] * 2)[:L + 1]
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, 1)
+    rng = np.random.default_rng(logn + L)
+    lib, h = capi.lib(), ctx.he_handle()
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(2)]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    keys = capi.evk_array([dev[d % 2].ptr for d in range(p.size_q)])
+    cs, cts = rand_limbs(p, rng, range(L), n_polys=items), rand_limbs(p, rng, range(L), n_polys=2 * items).reshape(items, 2, L, p.n)
+    cs[0, :, 0], cts[0, 0, :, 0] = [q - 1 for q in p.moduli[:L]], [q - 1 for q in p.moduli[:L]]
+    dc, dct, low = DeviceArray(capi, host=cs), DeviceArray(capi, host=cts), DeviceArray(capi, shape=(items, 2, L - 1, p.n))
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+    capi.check(lib.he_keyswitch_rescale_batch(h, L, items, dc.ptr, L, keys, dct.ptr, low.ptr, 0, ws.ptr, None))
+    got = low.numpy()
+    for k in sorted({0, items - 1}):
+        ks = p.key_switch(cs[k], [host[d % 2] for d in range(p.size_q)])
+        assert (got[k] == p.rescale(np.stack([p.add(cts[k][b], ks[b]) for b in range(2)]))).all(), k
