@@ -1,6 +1,6 @@
 // Device-side 64-bit modular arithmetic for gfx950 (wave64, VALU integer multiplies).
 //
-// All routines work on residues of primes below 2^61.  "lazy" values live in [0, 2q) or [0, 4q) and
+// All routines work on residues of primes below 2^61.  "lazy" values live in [0, 3q) or [0, 6q) and
 // never leave a kernel: every store to HBM that a caller can observe is the canonical residue, which
 // is what makes limb-for-limb comparison with the CPU oracle meaningful.
 //
@@ -181,13 +181,13 @@ __device__ __forceinline__ U128 total_sum3(const Sum3 &h, const Sum3 &s) {
     return U128{(uint64_t)t, (uint64_t)(t >> 64)};
 }
 
-// The butterflies' view of a modulus: q, 2q and their negatives modulo 2^64.  With the negatives at hand a Shoup
-// product is y w + hi (2^64 - q) and a conditional subtraction is x + (2^64 - 2q) followed by a select on the sign, i.e.
+// The butterflies' view of a modulus: q, 3q, 4q and their negatives modulo 2^64.  With the negatives at hand a Shoup
+// product is y w + hi (2^64 - q) and a conditional subtraction is x + (2^64 - 3q) followed by a select on the sign, i.e.
 // 64-bit additions (one instruction each) where subtractions would be borrow chains through VCC, which on this GPU need
 // two idle issue slots between producer and consumer.  The negatives pass through an empty asm statement so that the
 // compiler does not fold them back into subtractions: 37 -> 31 instructions per butterfly.
 struct IntMod {
-    uint64_t q, q2, nq, nq2;
+    uint64_t q, q3, q4, nq, nq3, nq4;
 };
 
 // (q is the same in every lane of a wave: a workgroup works on one limb; read from lane 0 so that the constants are
@@ -195,50 +195,65 @@ struct IntMod {
 __device__ __forceinline__ IntMod int_mod(uint64_t q_any_lane) {
     const uint32_t q_hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(q_any_lane >> 32));
     const uint32_t q_lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)q_any_lane);   // (the builtin returns int)
-    const uint64_t q = ((uint64_t)q_hi << 32) | q_lo;
+    const uint64_t q = ((uint64_t)q_hi << 32) | q_lo, q3 = 3 * q, q4 = 4 * q;
     // (as 32-bit scalars)
     uint32_t a0 = (uint32_t)(0 - q), a1 = (uint32_t)((0 - q) >> 32);
-    uint32_t b0 = (uint32_t)(0 - (q << 1)), b1 = (uint32_t)((0 - (q << 1)) >> 32);
-    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(b0), "+s"(b1));
-    return IntMod{q, q << 1, ((uint64_t)a1 << 32) | a0, ((uint64_t)b1 << 32) | b0};
+    uint32_t b0 = (uint32_t)(0 - q3), b1 = (uint32_t)((0 - q3) >> 32);
+    uint32_t c0 = (uint32_t)(0 - q4), c1 = (uint32_t)((0 - q4) >> 32);
+    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(b0), "+s"(b1), "+s"(c0), "+s"(c1));
+    return IntMod{q, q3, q4, ((uint64_t)a1 << 32) | a0, ((uint64_t)b1 << 32) | b0, ((uint64_t)c1 << 32) | c0};
 }
 
-// y w mod q up to one subtraction of q, in [0, 2q), for any 64-bit y
+// floor(a b / 2^64) or one less: the product of the lower halves, below 2^64, is left out
+__device__ __forceinline__ uint64_t mulhi64_low(uint64_t a, uint64_t b) {
+    const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32), b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
+    const uint64_t t = (uint64_t)a0 * b1, u = (uint64_t)a1 * b0 + (uint32_t)t;
+    return (uint64_t)a1 * b1 + (t >> 32) + (u >> 32);
+}
+
+// y w mod q up to two subtractions of q, in [0, 3q), for any 64-bit y
 __device__ __forceinline__ uint64_t mul_shoup_lazy(uint64_t y, Shoup s, const IntMod &m) {
-    return y * s.w + mulhi64(y, s.wq) * m.nq;
+    return y * s.w + mulhi64_low(y, s.wq) * m.nq;
 }
 
-// v - 2q if that is not negative, else v (v below 2^63)
-__device__ __forceinline__ uint64_t reduce_once_2q(uint64_t v, const IntMod &m) {
-    const uint64_t d = v + m.nq2;
+// v - k q if that is not negative, else v; nkq = 2^64 - k q (v below 6q: the difference fits 63 bits)
+__device__ __forceinline__ uint64_t reduce_once(uint64_t v, uint64_t nkq) {
+    const uint64_t d = v + nkq;
     return (int64_t)d < 0 ? v : d;
 }
 
-// Cooley-Tukey butterfly, inputs in [0, 4q), outputs in [0, 4q).
+// Cooley-Tukey butterfly, inputs in [0, 6q), outputs in [0, 6q): below 2^64 for q < 2^61.  (The range is what the shorter product
+// costs: a reduction more per word at the end of a transform, against one of ten multiplications and a link of the
+// chain per butterfly: multiplication with 4 limbs of 2^16 words and 60 bits 56.5 -> 54.8 us, 10 of 12 limbs of 2^15 with 60 and
+// 40 bits 65.8 -> 65.0, a transform of 2 x 24 limbs back 33.4 -> 33.0.)
 __device__ __forceinline__ void ct_butterfly(uint64_t &x, uint64_t &y, Shoup tw, const IntMod &m) {
     const uint64_t t = mul_shoup_lazy(y, tw, m);
-    const uint64_t xr = reduce_once_2q(x, m);
-    y = (xr + m.q2) - t;
+    const uint64_t xr = reduce_once(x, m.nq3);
+    y = (xr + m.q3) - t;
     x = xr + t;
 }
 
 // Gentleman-Sande butterfly with the division by two folded in (the inverse twiddles are stored
-// pre-halved), inputs in [0, 2q), outputs in [0, 2q).
+// pre-halved), inputs in [0, 3q), outputs in [0, 3q): the sum is below 6q, 4q once reduced, 2.5q once halved; the difference below
+// 7q (2^64 for q < 2^61).  4q, not 3q: both have the parity of x + y, so that the sum's halving does not wait for its reduction.
 __device__ __forceinline__ void gs_butterfly(uint64_t &x, uint64_t &y, Shoup tw, const IntMod &m) {
-    const uint64_t d = x + m.q2 - y;
-    uint64_t s = reduce_once_2q(x + y, m);
+    const uint64_t d = x + m.q4 - y;
+    uint64_t s = reduce_once(x + y, m.nq4);
     s += (d & 1) ? m.q : 0;
     x = s >> 1;
     y = mul_shoup_lazy(d, tw, m);
 }
 
-__device__ __forceinline__ uint64_t reduce_4q(uint64_t v, uint64_t q) {
-    uint64_t q2 = q << 1;
+__device__ __forceinline__ uint64_t reduce_3q(uint64_t v, uint64_t q) {
+    const uint64_t q2 = q << 1;
     v = v >= q2 ? v - q2 : v;
     return v >= q ? v - q : v;
 }
 
-__device__ __forceinline__ uint64_t reduce_2q(uint64_t v, uint64_t q) { return v >= q ? v - q : v; }
+__device__ __forceinline__ uint64_t reduce_6q(uint64_t v, uint64_t q) {
+    const uint64_t q3 = 3 * q;
+    return reduce_3q(v >= q3 ? v - q3 : v, q);
+}
 
 __device__ __forceinline__ Shoup load_shoup(const uint64_t *table, size_t idx) {
     const ulonglong2 v = reinterpret_cast<const ulonglong2 *>(table)[idx];

@@ -114,7 +114,7 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
         T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
         T4::template inverse<IntArith>(s, tw, ar, lds, t);
 #pragma unroll
-        for (int j = 0; j < 4; j++) s[j] = reduce_2q(s[j], q);
+        for (int j = 0; j < 4; j++) s[j] = reduce_3q(s[j], q);
     }
 }
 
@@ -203,7 +203,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 rows_input_int<MDR, SRC_INTT>(v, a, job, q, [&](int j) { return glob(0, j); }, s, s2);
             }
             T4::template forward<IntArith>(v, tw, ar, lds, t);
-            // lazy values in [0, 4q) go to the blocks pass
+            // lazy values in [0, 6q) go to the blocks pass
 #pragma unroll
             for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = v[j];
         } else {
@@ -218,7 +218,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 for (int j = 0; j < 4; j++) job.out[glob(0, j)] = mul_shoup(v[j], w, q);
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = reduce_2q(v[j], q);
+                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = reduce_3q(v[j], q);
             }
         }
     }
@@ -383,7 +383,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             if (FWD) {
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
 #pragma unroll
-                for (int j = 0; j < 4; j++) x[j] = reduce_4q(v[j], q);
+                for (int j = 0; j < 4; j++) x[j] = reduce_6q(v[j], q);
                 if (EPI) {
                     const Shoup ew = e.w;
                     if (e.fma) {
@@ -405,7 +405,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             }
         }
         if (!FWD) {
-            // lazy words (signed doubles, or integers in [0, 2q)) go to the rows pass
+            // lazy words (signed doubles, or integers in [0, 3q)) go to the rows pass
 #pragma unroll
             for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(v[j]);
         }
@@ -610,7 +610,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         T4::template forward<A>(v, tw, ar, nullptr, lane);
         if constexpr (!FP) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = reduce_4q(v[j], ar.m.q);
+            for (int j = 0; j < 4; j++) v[j] = reduce_6q(v[j], ar.m.q);
         }
         sums.add(v, k, ar);
     }
@@ -847,7 +847,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(HE
 
 // a word that the forward stages have left (lazy) as a canonical residue, and a canonical word as the arithmetic's value
 __device__ __forceinline__ uint64_t canonical_word(double v, const FpArith &ar) { return fp_to_u64(fp_canonical(v, ar.m)); }
-__device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &ar) { return reduce_4q(v, ar.m.q); }
+__device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &ar) { return reduce_6q(v, ar.m.q); }
 
 // v + x * y mod q for canonical words x, y and v as the forward stages have left it; canonical
 __device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y, const FpArith &ar, uint64_t, uint64_t) {
@@ -855,7 +855,7 @@ __device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y
     return fp_to_u64(fp_canonical(v + fp_mulmod(fp_from_u64(x), w, ar.m), ar.m));
 }
 __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t y, const IntArith &ar, uint64_t r0, uint64_t r1) {
-    return add_mod(reduce_4q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
+    return add_mod(reduce_6q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
 }
 
 // Encryption: three waves take their block of u, e0 and e1 of one limb through the last 8 stages; the transformed u stays in
