@@ -579,28 +579,31 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     const uint32_t L = b.map.split, last = L % b.K ? L % b.K : b.K;
     const uint32_t rows = b.up ? b.map.limbs - last : b.mdr ? L - 1 : L;
     if (rows == 0) return hipErrorInvalidValue;
-    // Output limbs per workgroup.  The kernel is bound by instruction issue, so a CU's time is the number of workgroups
-    // it is dealt times a workgroup's work: r rows plus about 1.5 rows' worth of fetching and converting its 8 x 8 block
-    // of inputs and setting up.  Few rows per workgroup pay that overhead often, many leave CUs with one workgroup more
-    // than others; the count that minimises ceil(workgroups / CUs) x (r + 1.5) matches the measured order at N = 2^16
-    // (one operation: 3 and 6 equal, 4 and 8 slower; 8 operations: 207, 179, 168 us at 3, 8, 12 rows).  A CU with a
-    // single workgroup has one wave per SIMD and nothing to cover its waits with (ModDown of one operation: 24.2 us in
-    // 256 workgroups of 6 rows against 22.5 us in 512 of 3), so fewer than two per CU count as two.
-    // the matrix-core kernel (N = 2^16) takes the output rows four at a time
-    // (merged ModDown + rescale: the matrix-core kernel first forms the rescale term for its whole tile, two rows' worth of
-    // work that pays once a workgroup has many rows, i.e. once the launch fills the chip without splitting the rows:
-    // 106 against 122 us for 8 operations, 27.8 against 25.4 us for one)
-    const bool mx = ld == 8 && b.mat_fp && b.mx_tab && !tune.no_matrix_bconv &&
-                    (!b.mdr || (b.mx_last && (uint64_t)b.units * items * tiles >= (tune.cus ? tune.cus : 256)));
+    // The matrix-core kernel (N = 2^16) multiplies 8 input limbs deep whatever there are, takes the output rows four at a time and two
+    // workgroups to a CU: it pays from five limbs on, and once the tiles alone give every CU a workgroup.  us with it / without, all of
+    // a multiplication: K = 8, L = 24: one 140.0 / 139.0, two 241.5 / 241.4, three 338.8 / 340.6, four 422 / 436, eight 805 / 840;
+    // K = 6, L = 30: one 203.0 / 201.2; K = 4, L = 12: one 80.8 / 74.4, two 129.7 / 124.4, eight 410 / 403.  (Merged ModDown +
+    // rescale, K = 8: eight 106 / 122 us.)
+    const uint32_t cus = tune.cus ? tune.cus : 256;
+    const bool mx = ld == 8 && b.mat_fp && b.mx_tab && !tune.no_matrix_bconv && b.K > 4 && (!b.mdr || b.mx_last) &&
+                    (uint64_t)b.units * items * tiles >= cus;
+    // Output limbs per workgroup.  The kernel is bound by instruction issue, so a CU's time is the number of workgroups it is dealt
+    // times a workgroup's work: r rows plus the fetching of the inputs and setting up, one row's worth and a half with 4 waves and a
+    // tile of 8 words per thread, half a row's with 8 waves and 4 words.  Few rows per workgroup pay that often, many leave
+    // CUs with one workgroup more than others.  A CU with a single workgroup has fewer waves to cover its waits with: as much as two
+    // take (4 waves), 15 % (8 waves, 25 % on integers: n = 2^14, 12 limbs of 60 bits, K = 4, one row 49.5 us, two
+    // 50.0).  Measured at n = 2^16 (8 waves), us with 1, 2, 3, 4, 5, 6, 8 rows a workgroup: K = 8, 24 rows
+    // for 96 tiles 37.5, 36.0, 30.5, 34.1, 30.9, 33.2, 38.4; K = 8, 23 rows for 64 tiles 33.3, 28.8, 24.4, 26.8, 30.5, 24.7, 28.4;
+    // K = 4, 12 rows for 96 tiles 16.7, 16.2, 15.8, 18.1, -, 17.0; K = 4, 11 rows for 64 tiles 13.3, 12.5, 11.4, 12.4, -, 16.0.
     const uint32_t step = mx ? 4 : 1;
     uint32_t target = mx ? (forced + 3) / 4 * 4 : forced;
     if (!target) {
-        const uint32_t cus = tune.cus ? tune.cus : 256;
         uint64_t best = ~0ull;
+        const uint32_t single = b.mat_fp ? 23 : 25;
         for (uint32_t r = step; r <= kFuseMaxRows && r < rows + step; r += step) {
             const uint64_t wgs = (uint64_t)b.units * items * tiles * ((rows + r - 1) / r);
             const uint64_t per_cu = (wgs + cus - 1) / cus;
-            const uint64_t cost = (per_cu < 2 ? 2 : per_cu) * (2 * r + 3);
+            const uint64_t cost = mx ? (per_cu < 2 ? 2 : per_cu) * (2 * r + 3) : (per_cu < 2 ? single : 20 * per_cu) * (2 * r + 1);
             if (cost < best) {
                 best = cost;
                 target = r;

@@ -391,3 +391,29 @@ def test_key_switch_and_rescale_of_few_limbs(oracle, capi, chain, logn, L, items
     for k in sorted({0, items - 1}):
         ks = p.key_switch(cs[k], [host[d % 2] for d in range(p.size_q)])
         assert (got[k] == p.rescale(np.stack([p.add(cts[k][b], ks[b]) for b in range(2)]))).all(), k
+
+
+@pytest.mark.parametrize("size_p,L,items", [(4, 4, 8), (5, 10, 3), (5, 10, 4), (6, 12, 4), (8, 8, 8)])
+def test_conversions_on_both_sides_of_the_matrix_kernel(oracle, capi, size_p, L, items):
+    """Key switch + rescale at n = 2^16, primes below 2^50: from five special primes and 256 tiles on the conversions run on the matrix
+    cores."""
+    cahel, parms, ctx, p = make_pair(oracle, 16, [50] * (L + size_p), size_p)
+    rng = np.random.default_rng(size_p + items)
+    lib, h = capi.lib(), ctx.he_handle()
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(2)]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    beta = L // size_p
+    keys = capi.evk_array([dev[d % 2].ptr for d in range(beta)])
+    one, ct1 = rand_limbs(p, rng, range(L), n_polys=2), rand_limbs(p, rng, range(L), n_polys=2)
+    one[0, :, :2] = np.array([[q - 1, 0] for q in p.moduli[:L]], dtype=np.uint64)
+    cs, cts = np.stack([one[k % 2] for k in range(items)]), np.stack([ct1] * items)
+    dc, dct, low = DeviceArray(capi, host=cs), DeviceArray(capi, host=cts), DeviceArray(capi, shape=(items, 2, L - 1, p.n))
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+    capi.check(lib.he_keyswitch_rescale_batch(h, L, items, dc.ptr, L, keys, dct.ptr, low.ptr, 0, ws.ptr, None))
+    got = low.numpy()
+    want = []
+    for k in range(2):
+        ks = p.key_switch(one[k], [host[d % 2] for d in range(beta)])
+        want.append(p.rescale(np.stack([p.add(ct1[b], ks[b]) for b in range(2)])))
+    for k in range(items):
+        assert (got[k] == want[k % 2]).all(), k
