@@ -306,8 +306,8 @@ constexpr uint32_t kFuseMaxRows = 24;
 // (row rr, coefficient c) in lane 16 rr + c, and
 //     sum_e S_e 2^(7 e) = lo + 2^28 hi,   lo = S_0 + 2^7 S_1 + 2^14 S_2 + 2^21 S_3 < 2^43,  hi likewise,
 // becomes the lazy residue (hi x (2^28 mod q)) mod q + lo with one modular product: 13 FP64-rate operations and two
-// matrix instructions per word against 44 operations for the eight exact multiply-adds on the vector units.  (ModUp of one operation
-// at L = 24, K = 8 takes 29.5 us either way, both kernels being short of waves; of eight 147 against 158 us.)
+// matrix instructions per word against 44 operations for the eight exact multiply-adds on the vector units.  (When it runs: see
+// launch_bconv_rows.)
 //
 // Wave w of the workgroup owns the coefficients of rows w + 4 j + 32 i (j, i < 8) of the 256 x 8 tile; lane (kg, c) keeps the words of input limbs 2 kg, 2 kg + 1 for coefficient c of each of 32 sets of 16
 // coefficients (set (g, i): (j, column) = (2 g + c / 8, c % 8), row w + 4 j + 32 i), which is at once the B operand of the
