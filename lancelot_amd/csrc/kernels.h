@@ -114,6 +114,7 @@ struct NttArgs {
     const LimbJob *jobs;      // explicit list: the converted limbs of a ModUp, digit by digit, ascending (then in/out limbs are
                               // absolute, no prologue/epilogue; map describes Ql u P)
     uint32_t listed;          // (jobs is there)
+    uint32_t spread;          // filled in by the launcher: an eighth of every limb to an XCD (limb_block)
     uint32_t n_jobs, digit_limbs, digits;   // ... of so many digits of so many limbs (the last one may have fewer)
     const LimbGroup *groups;  // partition of `jobs` into runs with one table each, or nullptr
     uint32_t n_groups;
@@ -174,7 +175,7 @@ inline NttHead ntt_head(const NttArgs &a, uint32_t wgs, uint32_t extra) {
     NttHead h{a.in, a.out, a.tw, a.fp_mask, 0, 0, 0, 0, wgs, extra};
     const bool whole = a.map.split >= a.map.limbs;   // (then the caller's split and tail_first are any numbers)
     const uint32_t split = whole ? a.map.limbs : a.map.split, tail = whole ? 0 : a.map.tail_first;
-    h.h0 = a.log_n | (a.jobs ? 1u << 5 : 0) | a.map.limbs << 6 | (a.size_qp - 1) << 24;
+    h.h0 = a.log_n | (a.jobs ? 1u << 5 : 0) | a.map.limbs << 6 | (a.spread ? 1u << 16 : 0) | (a.size_qp - 1) << 24;
     h.h1 = a.jobs ? a.n_jobs : a.in_poly_stride;
     h.h2 = a.jobs ? (a.digit_limbs | a.digits << 16) : a.out_poly_stride;
     h.h3 = a.map.first | split << 9 | tail << 18 | (uint32_t)a.pro_mode << 27;

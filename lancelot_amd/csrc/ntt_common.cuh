@@ -49,6 +49,13 @@ __device__ __forceinline__ uint32_t logical_block(uint32_t n) {
     return b;
 }
 
+// The same for a launch of limbs of 2^log_tiles workgroups each, where NttArgs::spread says so: an XCD gets the same eighth of every limb.
+__device__ __forceinline__ uint32_t limb_block(uint32_t n, uint32_t log_tiles, uint32_t h0) {
+    if (log_tiles < 3 || !(h0 >> 16 & 1)) return logical_block(n);
+    const uint32_t b = blockIdx.x, k = b >> 3, log_per = log_tiles - 3;
+    return (k >> log_per << log_tiles) | (b & 7) << log_per | (k & ((1u << log_per) - 1));
+}
+
 // the pointers into a direction's block (NttArgs::tw)
 __device__ __forceinline__ const double *block_fp(const uint64_t *block, uint32_t qp, uint32_t log_n) {
     return reinterpret_cast<const double *>(block + ((size_t)(2 * qp) << log_n));

@@ -421,7 +421,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
     set_extra(a, x, FWD);
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block(h4) * kBlockWaves + w;   // (a limb has an even number of blocks)
+    const uint32_t id = (EPI ? limb_block(h4, lr - 1, h0) : logical_block(h4)) * kBlockWaves + w;   // (a limb has an even number of blocks)
     const BlockUnit unit = block_unit(a, id >> lr);
     const uint32_t blk = id & ((1u << lr) - 1);
     const Job job = decode_job<false, true>(a, unit.job(0));
@@ -836,7 +836,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(HE
     const TensorFuse x{h_in, ct2, d01, d2, a.map.limbs, (int)h5};
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block(h4) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane);
@@ -925,7 +925,7 @@ __global__ __launch_bounds__(192) void encrypt_blocks_kernel(HE_HEAD_PARAMS, con
     const uint64_t *pk = a.in;
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = a.map.limbs, L = a.map.split, items = h1, first_item = h5;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t id = logical_block(h4), blk = id & ((1u << lr) - 1), it = id >> lr;
+    const uint32_t id = limb_block(h4, lr, h0), blk = id & ((1u << lr) - 1), it = id >> lr;
     const uint32_t of_launch = it / LK, item = first_item + of_launch, t = it - of_launch * LK, table = map_table(a.map, t);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     if (BE != NTT_BACKEND_INT && fp)
@@ -1054,6 +1054,15 @@ __global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodEx
         for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = v[j];
     }
 }
+
+// Which launches deal every limb's workgroups to all XCDs (limb_block).  Otherwise an XCD has a contiguous range of the launch, which
+// the passes need that go over the same words one after the other: they meet them in the XCD's L2 (2 x 6 limbs of 2^16 words 10.8 us, dealt
+// out 13.1).  But with few limbs of both arithmetics, two XCDs have all the work of a 60-bit limb and two that of a 40-bit one.  It
+// pays where that work is most: in encryption's blocks pass and in the blocks passes with an
+// epilogue from three workgroups per CU on (both: encryption of 3 limbs of 2^16 words 56.0 -> 53.1 us, of 10 of 2^15 62.2 -> 57.1; the
+// epilogue alone: multiplication with 10 limbs of 2^15 64.0 -> 63.2, rotation with 5 limbs of 2^16 49.6 -> 48.4; with 2 limbs of 2^16, 512
+// workgroups, 27.6 -> 27.8).
+bool spread_ok(int backend, uint64_t n_jobs, uint64_t wgs, uint64_t least) { return backend == NTT_BACKEND_MIXED && n_jobs <= 32 && wgs >= least; }
 
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
@@ -1189,6 +1198,8 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     const uint64_t wgs = (uint64_t)kinds * ((repeats + a.batch - 1) / a.batch) * (blocks / kBlockWaves);
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    const bool epi = forward && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || a.epi_mode == NTT_EPI_FMA_SUB_MUL);
+    a.spread = epi && spread_ok(backend, (uint64_t)kinds * repeats, wgs, 768);
     const NttHead head = ntt_head(a, grid.x, a.batch);
     const BlocksExtra extra = blocks_extra(a, forward);
 #define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
@@ -1200,7 +1211,6 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
         else                                                                                                            \
             hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
     } while (0)
-    const bool epi = forward && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || a.epi_mode == NTT_EPI_FMA_SUB_MUL);
     const bool loop = a.batch > 1 || a.groups;
     if (epi && loop)
         HE_LAUNCH(true, true, true);
@@ -1289,6 +1299,8 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, u
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    // (a limb's twiddles serve all items: dealt out, an XCD keeps its eighth of all of them; 8 x 24 limbs 792 -> 785 us of a product)
+    a.spread = items > 1;
     const NttHead h = ntt_head(a, grid.x, x.square ? 1 : 0);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
@@ -1311,6 +1323,7 @@ hipError_t launch_encrypt_blocks(const NttArgs &args, const uint64_t *pk, uint32
     if (per_launch == 0) return hipErrorInvalidValue;
     for (uint32_t first = 0; first < items; first += per_launch) {
         const dim3 grid((items - first < per_launch ? items - first : per_launch) * wgs_per_item);
+        a.spread = spread_ok(backend, (uint64_t)items * (L + K), grid.x, 256);
         const NttHead head = ntt_head(a, grid.x, first);
         if (backend == NTT_BACKEND_MIXED)
             hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);

@@ -417,3 +417,22 @@ def test_conversions_on_both_sides_of_the_matrix_kernel(oracle, capi, size_p, L,
         want.append(p.rescale(np.stack([p.add(ct1[b], ks[b]) for b in range(2)])))
     for k in range(items):
         assert (got[k] == want[k % 2]).all(), k
+
+
+@pytest.mark.parametrize("logn,bits,size_p", [(13, [60, 40, 40, 50, 60, 60], 2), (14, [60, 40, 40, 60], 1), (15, [40, 60, 60, 40, 60], 1)])
+def test_encryption_of_a_mixed_chain(oracle, capi, logn, bits, size_p):
+    """Encryption's blocks pass deals the limbs' workgroups to all XCDs from 256 workgroups on (L + K limbs of N / 256)."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    key = oracle.chacha_key(3)
+    kp = key.ctypes.data_as(C.POINTER(C.c_uint32))
+    rng = np.random.default_rng(logn)
+    pk, plain = rand_limbs(p, rng, range(p.size_qp), n_polys=2), rand_limbs(p, rng, range(p.size_q))
+    dpk, dplain, dct = DeviceArray(capi, host=pk), DeviceArray(capi, host=plain), DeviceArray(capi, shape=(2, p.size_q, n))
+    ws = DeviceArray(capi, shape=(lib.he_encrypt_batch_workspace_words(h, p.size_q, 1),))
+    capi.check(lib.he_encrypt(h, p.size_q, dplain.ptr, dpk.ptr, kp, 11, dct.ptr, ws.ptr, None))
+    got, u = dct.numpy(), p.ntt_fwd(p.sample_ternary(key, 11, p.size_qp))
+    for i in range(2):
+        e = p.ntt_fwd(p.sample_error(key, 12 + i, p.size_qp))
+        want = p.moddown(np.ascontiguousarray(p.mul_add(u, pk[i], e)))
+        assert (got[i] == (p.add(want, plain) if i == 0 else want)).all(), i
