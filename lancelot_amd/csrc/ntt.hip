@@ -213,9 +213,8 @@ inline bool limb4(const NttArgs &a, int backend, uint32_t n_jobs) {
 }
 
 template <bool FWD>
-hipError_t launch_limb(const NttArgs &a, uint32_t n_jobs, int backend, hipStream_t s) {
-    if (n_jobs > most_workgroups((1u << a.log_n) / 4)) return hipErrorInvalidValue;
-    if (limb4(a, backend, n_jobs)) {
+hipError_t launch_limbs(const NttArgs &a, uint32_t n_jobs, bool four, int backend, hipStream_t s) {
+    if (four) {
         const NttHead head = ntt_head(a, n_jobs, (uint32_t)a.epi_mode);
 #define HE_LIMB4(LOGN)                                                                                                                  \
     do {                                                                                                                                \
@@ -242,6 +241,22 @@ hipError_t launch_limb(const NttArgs &a, uint32_t n_jobs, int backend, hipStream
         default: return hipErrorInvalidValue;
     }
     return hipGetLastError();
+}
+
+// With 4 words a thread one launch does not hold the threads from 2^34 words (137 GB) on: whole polynomials, as many as it holds, go
+// into each of several.
+template <bool FWD>
+hipError_t launch_limb(NttArgs a, uint32_t n_polys, int backend, hipStream_t s) {
+    const bool four = limb4(a, backend, n_polys * a.map.limbs);
+    const uint32_t per_launch = most_workgroups((1u << a.log_n) / (four ? 4 : 16)) / a.map.limbs;
+    for (;;) {
+        const uint32_t polys = n_polys < per_launch ? n_polys : per_launch;
+        if (hipError_t e = launch_limbs<FWD>(a, polys * a.map.limbs, four, backend, s)) return e;
+        n_polys -= polys;
+        if (n_polys == 0) return hipSuccess;
+        a.in += (size_t)polys * a.in_poly_stride << a.log_n;
+        a.out += (size_t)polys * a.out_poly_stride << a.log_n;
+    }
 }
 
 // The launches that a whole-limb kernel covers and wins.  A limb is one workgroup on one CU: up to N = 2^12 that is
@@ -637,7 +652,7 @@ hipError_t launch_ntt_forward(const NttArgs &a, uint32_t n_polys, int backend, h
     if (a.log_n < 9 || a.log_n > 17 || backend < NTT_BACKEND_INT || backend > NTT_BACKEND_MIXED) return hipErrorInvalidValue;
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
-    if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb<true>(a, n_jobs, backend, s);
+    if (!rows_done && one_pass_ok(a, backend, true, n_jobs)) return launch_limb<true>(a, n_polys, backend, s);
     const hipError_t e = rows_done ? hipSuccess : launch_ntt_rows(a, n_jobs, true, backend, s);
     return e != hipSuccess ? e : launch_ntt_blocks(a, n_polys, true, backend, s);
 }
@@ -647,7 +662,7 @@ hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, h
     if (a.log_n < 9 || a.log_n > 17 || backend < NTT_BACKEND_INT || backend > NTT_BACKEND_MIXED) return hipErrorInvalidValue;
     const uint32_t n_jobs = a.jobs ? a.n_jobs * (a.items ? a.items : 1) : n_polys * a.map.limbs;
     if (n_jobs == 0) return hipSuccess;
-    if (!blocks_done && !rows_skipped && one_pass_ok(a, backend, false, n_jobs)) return launch_limb<false>(a, n_jobs, backend, s);
+    if (!blocks_done && !rows_skipped && one_pass_ok(a, backend, false, n_jobs)) return launch_limb<false>(a, n_polys, backend, s);
     const hipError_t e = blocks_done ? hipSuccess : launch_ntt_blocks(a, n_polys, false, backend, s);
     if (e != hipSuccess || rows_skipped) return e;
     NttArgs rows = a;

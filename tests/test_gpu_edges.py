@@ -155,15 +155,17 @@ def allocate(capi, words):
     return ptr.value
 
 
-@pytest.mark.parametrize("bits", [[50, 50], [60, 60], [60, 40, 60]])
-def test_transforms_of_more_words_than_a_launch_holds(oracle, capi, bits):
-    """2^34 words (137 GB) and some: a thread of the rows pass takes four, and a launch has fewer than 2^32 threads."""
-    cahel, parms, ctx, p = make_pair(oracle, 16, bits, 1)
+@pytest.mark.parametrize("logn,bits", [(16, [50, 50]), (16, [60, 60]), (16, [60, 40, 60]), (10, [50, 50]), (10, [60, 40, 60]),
+                                       (12, [50, 50]), (12, [60, 60]), (12, [60, 40, 60])])
+def test_transforms_of_more_words_than_a_launch_holds(oracle, capi, logn, bits):
+    """2^34 words (137 GB) and some: a thread of the rows pass, or of a whole limb of 2^10 or 2^12 words, takes four (16 at 2^12, 50
+    bits), and a launch has fewer than 2^32 threads."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, 1)
     lib, h, n, limbs = capi.lib(), ctx.he_handle(), p.n, len(bits) - 1
-    polys, rng = ((1 << 18) + 8) // limbs, np.random.default_rng(limbs)
+    polys, rng = ((1 << (34 - logn)) + 8) // limbs, np.random.default_rng(limbs)
     data = allocate(capi, polys * limbs * n)
     try:
-        last = 0xffffffff // 512 // 32 // limbs      # the first launch's last polynomial
+        last = 0xffffffff // (n // 4) // limbs       # the polynomials of the first launch
         xs = {k: rand_limbs(p, rng, range(limbs)) for k in (0, 8, last - 1, last, last + 1, polys - 1)}
         at = lambda k: data + 8 * k * limbs * n
         for k, x in xs.items():
