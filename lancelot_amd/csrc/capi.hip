@@ -449,7 +449,7 @@ int he_context_create(const he_context_desc *d, he_context **out) {
         rc = static_scratch(&unused);
     }
     // the block of each direction (NttArgs::tw): twiddles of both back ends, then the primes' constants
-    if (!rc) rc = reserve(ctx, &ctx->d_psi, (3 * n + 7) * qp + 4 * (size_t)d->size_q);
+    if (!rc) rc = reserve(ctx, &ctx->d_psi, (3 * n + 5) * qp + p_constants_from_barrett(ctx->size_qp) + 4 * (size_t)d->size_q);
     if (!rc) rc = reserve(ctx, &ctx->d_ipsi, (3 * n + 7) * qp);
     if (!rc) {
         ctx->d_psi_fp = reinterpret_cast<double *>(ctx->d_psi + 2 * qp * n);
@@ -465,7 +465,7 @@ int he_context_create(const he_context_desc *d, he_context **out) {
         }
     }
     if (!rc && d->size_p) {
-        ctx->d_p_mod_q = ctx->d_barrett + 2 * qp;
+        ctx->d_p_mod_q = ctx->d_barrett + p_constants_from_barrett(ctx->size_qp);
         ctx->d_pinv_mod_q = ctx->d_p_mod_q + 2 * (size_t)d->size_q;
         rc = put(ctx->d_p_mod_q, d->p_mod_q, 2 * (size_t)d->size_q);
         if (!rc) rc = put(ctx->d_pinv_mod_q, d->pinv_mod_q, 2 * (size_t)d->size_q);

@@ -94,6 +94,10 @@ enum : int {
 // the count modulo 2^32.
 inline constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads < 0x7fffffffu ? 0xffffffffu / threads : 0x7fffffffu; }
 
+// Where the Shoup pairs of P mod q lie in a block (NttArgs::tw), in words from the Barrett ratios, which start (3 N + 5) x tables words
+// into it: behind the ratios, on an even word, since load_shoup reads a pair as one 16-byte word.
+__host__ __device__ constexpr uint32_t p_constants_from_barrett(uint32_t tables) { return 2 * tables + (tables & 1); }
+
 struct NttArgs {
     const uint64_t *in;   // limb (poly, i) at in + (poly * in_poly_stride + i) * N
     uint64_t *out;
@@ -101,8 +105,8 @@ struct NttArgs {
     uint32_t out_poly_stride;
     // One block per direction, with everything that a pass reads about its primes: [tables][N][2] (operand, Shoup quotient), then
     // [tables][N] twiddles as exact doubles for the FP64 back end (primes below 2^50), [tables][4] of q, 1/q, N^-1 mod q and
-    // (N^-1 mod q)/q as doubles, [tables] moduli, [tables][2] Barrett ratios; forward also [size_q][2] Shoup pairs of P mod q and
-    // [size_q][2] of P^-1 mod q
+    // (N^-1 mod q)/q as doubles, [tables] moduli, [tables][2] Barrett ratios; forward also, from p_constants_from_barrett words behind
+    // the start of the ratios on, [size_q][2] Shoup pairs of P mod q and [size_q][2] of P^-1 mod q
     const uint64_t *tw;
     uint32_t size_qp;         // tables
     const double *tw_fp;      // (into the block; set where a kernel starts)

@@ -541,7 +541,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
     const bool add = (x.inv_first >> 16 & 1) && t < L;                 // polynomial 0 gains P sigma(c0) (a rotation)
     const bool fold = (x.inv_first >> 17 & 1) && t == L - 1;
     Shoup add_w{0, 0}, fold_w{0, 0};
-    const uint64_t *p_mod_q = a.barrett + 2 * a.size_qp;   // and P^-1 behind it (NttArgs::tw)
+    const uint64_t *p_mod_q = a.barrett + p_constants_from_barrett(a.size_qp);   // and P^-1 behind it (NttArgs::tw)
     if (add) add_w = scalar_shoup(p_mod_q, t);
     if (fold) fold_w = scalar_shoup(p_mod_q, a.map.tail_first + t);
     const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];

@@ -302,10 +302,11 @@ def test_hoisting_of_batches(oracle, capi, chain, local, logn, size_p, L, n_step
 
 
 @pytest.mark.parametrize("logn,bits,size_p,L", [(16, [60, 40, 40, 60], 1, 2), (16, [60, 40, 40, 60], 1, 3), (15, [40, 60, 50, 45, 30, 59, 60, 50], 2, 5),
-                                                (15, [60, 40, 50, 45, 30, 59, 60, 60], 2, 4), (14, [60, 40, 50, 45, 30, 59, 60, 60], 2, 6)])
+                                                (15, [60, 40, 50, 45, 30, 59, 60, 60], 2, 4), (14, [60, 40, 50, 45, 30, 59, 60, 60], 2, 6),
+                                                (12, [60, 40, 60], 1, 2), (13, [60, 40, 50, 45, 60], 1, 3)])
 def test_key_switch_of_a_mixed_chain(oracle, capi, logn, bits, size_p, L):
     """Rotation and key switch + rescale where the inner product takes its limbs in an order of their own (more than one workgroup for
-    every CU) and where it does not."""
+    every CU) and where it does not, with even and odd numbers of primes (behind an odd one the constants of P lie a word further)."""
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(logn + L)
     lib, h = capi.lib(), ctx.he_handle()

@@ -2,6 +2,7 @@
 number theory agrees with the reference's known answers and with the oracle.  No GPU calls."""
 import os
 import re
+import subprocess
 
 import numpy as np
 import pytest
@@ -241,3 +242,24 @@ def test_bench_refuses_more_than_one_gpu():
                        timeout=120)
     assert r.returncode != 0
     assert "one GPU" in (r.stdout + r.stderr)
+
+
+def test_shoup_pairs_lie_on_even_words(tmp_path):
+    """The kernels read a Shoup pair as one 16-byte word: those of P, behind the Barrett ratios of a context's table block, begin an even
+    number of words into it for every number of primes, behind the last ratio."""
+    source = tmp_path / "layout.cpp"
+    source.write_text("""
+#include "kernels.h"
+int main() {
+    for (unsigned log_n = 9; log_n <= 17; log_n++)
+        for (unsigned tables = 1; tables <= 256; tables++) {
+            const unsigned long barrett = ((3ul << log_n) + 5) * tables, at = barrett + he::p_constants_from_barrett(tables);
+            if (at % 2 || at < barrett + 2 * tables || at > barrett + 2 * tables + 1) return 1;
+        }
+    return 0;
+}
+""")
+    exe = str(tmp_path / "layout")
+    subprocess.check_call(["g++", "-std=c++17", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include", "-I",
+                           os.path.join(ROOT, "lancelot_amd", "csrc"), str(source), "-o", exe])
+    assert subprocess.run([exe]).returncode == 0
