@@ -279,10 +279,13 @@ bool fuse_rows_ok(const he_context *ctx, const Level *lv, uint32_t L) {
     return ctx->fuse_rows && !ctx->single_limb_digits && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16;
 }
 
+// whether `count` limbs from `first` on are among the first `size` (a sum of the two could wrap around)
+bool in_range(uint32_t first, uint32_t count, uint32_t size) { return count <= size && first <= size - count; }
+
 int check_map(const he_context *ctx, uint32_t limbs, uint32_t first, uint32_t split, uint32_t tail) {
     if (split > limbs) return HE_E_INVALID_ARGUMENT;
-    if (first + split > ctx->size_qp) return HE_E_INVALID_ARGUMENT;
-    if (limbs > split && tail + (limbs - split) > ctx->size_qp) return HE_E_INVALID_ARGUMENT;
+    if (!in_range(first, split, ctx->size_qp)) return HE_E_INVALID_ARGUMENT;
+    if (limbs > split && !in_range(tail, limbs - split, ctx->size_qp)) return HE_E_INVALID_ARGUMENT;
     return HE_OK;
 }
 
@@ -796,7 +799,7 @@ int he_ntt_inverse(const he_context *ctx, uint64_t *data, uint32_t n_polys, uint
 static int elementwise(const he_context *ctx, int op, const uint64_t *a, const uint64_t *b, const uint64_t *c,
                        uint64_t *out, uint32_t n_polys, uint32_t limbs, uint32_t first, he_stream s) {
     if (!ctx || !a || !out || (op != EW_NEG && !b)) return HE_E_INVALID_ARGUMENT;
-    if (first + limbs > ctx->size_qp) return HE_E_INVALID_ARGUMENT;
+    if (!in_range(first, limbs, ctx->size_qp)) return HE_E_INVALID_ARGUMENT;
     HE_HIP(launch_elementwise(ctx->tables(), op, a, b, c, out, n_polys, plain_map(limbs, first), S(s)));
     return HE_OK;
 }
@@ -829,7 +832,7 @@ int he_multiply_add(const he_context *ctx, const uint64_t *a, const uint64_t *b,
 
 int he_add_p_multiple(const he_context *ctx, const uint64_t *a, const uint64_t *b, uint64_t *out, uint32_t first_limb,
                       uint32_t limbs, he_stream s) {
-    if (!ctx || !a || !b || !out || ctx->size_p == 0 || first_limb + limbs > ctx->size_q) return HE_E_INVALID_ARGUMENT;
+    if (!ctx || !a || !b || !out || ctx->size_p == 0 || !in_range(first_limb, limbs, ctx->size_q)) return HE_E_INVALID_ARGUMENT;
     HE_HIP(launch_scalar_mul_add(ctx->tables(), a, b, out, ctx->d_p_mod_q, first_limb, limbs, S(s)));
     return HE_OK;
 }
@@ -1515,7 +1518,7 @@ int he_keyswitch_rescale(const he_context *ctx, uint32_t L, const uint64_t *c, c
 
 int he_decompose_real(const he_context *ctx, const double *coeffs, uint64_t *out, uint32_t limbs, uint32_t first,
                       he_stream s) {
-    if (!ctx || !coeffs || !out || first + limbs > ctx->size_qp) return HE_E_INVALID_ARGUMENT;
+    if (!ctx || !coeffs || !out || !in_range(first, limbs, ctx->size_qp)) return HE_E_INVALID_ARGUMENT;
     HE_HIP(launch_decompose_real(ctx->tables(), coeffs, out, limbs, first, 1, 0, S(s)));
     return HE_OK;
 }

@@ -204,6 +204,23 @@ def test_encryptions_of_more_words_than_a_launch_holds(oracle, capi):
         lib.he_free(cts)
 
 
+@pytest.mark.parametrize("first,count", [(4, 1), (3, 2), (0, 5), (2 ** 32 - 1, 1), (2 ** 32 - 1, 4), (2 ** 32 - 2, 3), (2, 2 ** 32 - 1)])
+def test_limbs_past_the_last_prime_are_refused(oracle, capi, first, count):
+    """Runs of limbs that end behind the last of four primes, and runs whose end is beyond 2^32: refused before anything is launched."""
+    cahel, parms, ctx, p = make_pair(oracle, 9, [50, 40, 40, 50], 1)
+    lib, h = capi.lib(), ctx.he_handle()
+    a, b, out = (DeviceArray(capi, host=np.zeros((8, p.n), dtype=np.uint64)) for _ in range(3))
+    kp = oracle.chacha_key(3).ctypes.data_as(C.POINTER(C.c_uint32))
+    calls = [lib.he_add(h, a.ptr, b.ptr, out.ptr, 1, count, first, None), lib.he_negate(h, a.ptr, out.ptr, 1, count, first, None),
+             lib.he_multiply_add(h, a.ptr, b.ptr, a.ptr, out.ptr, 1, count, first, 0, None),
+             lib.he_add_p_multiple(h, a.ptr, b.ptr, out.ptr, first, count, None), lib.he_decompose_real(h, a.ptr, out.ptr, count, first, None)]
+    for transform in (lib.he_ntt_forward, lib.he_ntt_inverse):
+        calls.append(transform(h, out.ptr, 1, count, count, first, count, 0, None))
+        calls.append(transform(h, out.ptr, 1, count, count, 0, 0, first, None))
+    calls.append(lib.he_sample(h, 0, kp, 1, out.ptr, count, first, count, 0, None, 0, None))
+    assert calls == [-1] * len(calls)
+
+
 class OddArray(DeviceArray):
     """A device buffer that starts 8 bytes behind a 16-byte boundary."""
 
