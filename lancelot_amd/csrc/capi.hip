@@ -42,7 +42,7 @@ struct Level {
     uint32_t *d_modup_limb = nullptr, *d_modup_table = nullptr;
     uint32_t modup_max_rows = 0, modup_max_copy = 0;
     bool batched = false;
-    double *d_mats_fp = nullptr;         // (M, M/m) pairs of the digit matrices, when every prime is below 2^50
+    double *d_mats_fp = nullptr;         // the digit matrices as doubles, when every prime is below 2^50
     int32_t *d_mx_up = nullptr;          // the same matrices as 7-bit digits for the int8 matrix cores (N = 2^16)
 };
 
@@ -90,7 +90,7 @@ struct he_context {
     uint32_t *d_iota = nullptr;  // 0, 1, 2, ...: row -> limb/table map of the P -> Ql conversion
     std::vector<uint64_t> h_phat_inv;    // host copy of d_phat_inv
     double *d_psi_fp = nullptr, *d_ipsi_fp = nullptr, *d_fp_consts = nullptr;  // FP64 back end tables
-    double *d_phat_mod_q_fp = nullptr;   // (M, M/q_j) pairs of the P -> Ql matrix
+    double *d_phat_mod_q_fp = nullptr;   // the P -> Ql matrix as doubles
     double *d_phat_pinv_fp = nullptr;    // the same matrix times P^-1 mod q_j (merged ModDown + rescale, fused kernel)
     bool fuse_rows = true;       // environment CAHEL_HIP_NO_FUSED_BCONV=1: conversion kernel, then the rows pass
     bool fuse_tensor = true;     // environment CAHEL_HIP_NO_FUSED_TENSOR=1: he_multiply_relin_rescale as tensor kernel + key switch
@@ -566,25 +566,18 @@ int he_context_create(const he_context_desc *d, he_context **out) {
             consts[4 * t] = qd;
             consts[4 * t + 1] = 1.0 / qd;
             consts[4 * t + 2] = (double)ninv;
-            consts[4 * t + 3] = (double)ninv / qd;
         }
         if (d->size_p) {
-            // (16 doubles of padding: the fused conversion kernel fetches 8 pairs per row whatever the row's length)
-            std::vector<double> pfp(2 * (size_t)d->size_q * d->size_p + 16, 0.0);
-            for (size_t jq = 0; jq < d->size_q; jq++)
-                for (size_t k = 0; k < d->size_p; k++) {
-                    pfp[2 * (jq * d->size_p + k)] = (double)d->phat_mod_q[jq * d->size_p + k];
-                    pfp[2 * (jq * d->size_p + k) + 1] = (double)d->phat_mod_q[jq * d->size_p + k] / (double)d->moduli[jq];
-                }
+            // (8 doubles of padding: the fused conversion kernel fetches 8 entries per row whatever the row's length)
+            const size_t entries = (size_t)d->size_q * d->size_p;
+            std::vector<double> pfp(entries + 8, 0.0);
+            for (size_t i = 0; i < entries; i++) pfp[i] = (double)d->phat_mod_q[i];
             rc = upload(ctx, &ctx->d_phat_mod_q_fp, pfp.data(), pfp.size());
             // (P / p_k) P^-1 mod q_j: delta_j P^-1 straight from the conversion
-            for (size_t jq = 0; jq < d->size_q; jq++)
-                for (size_t k = 0; k < d->size_p; k++) {
-                    const uint64_t q = d->moduli[jq];
-                    const uint64_t v = (uint64_t)((unsigned __int128)d->phat_mod_q[jq * d->size_p + k] * d->pinv_mod_q[2 * jq] % q);
-                    pfp[2 * (jq * d->size_p + k)] = (double)v;
-                    pfp[2 * (jq * d->size_p + k) + 1] = (double)v / (double)q;
-                }
+            for (size_t i = 0; i < entries; i++) {
+                const size_t jq = i / d->size_p;
+                pfp[i] = (double)(uint64_t)((unsigned __int128)d->phat_mod_q[i] * d->pinv_mod_q[2 * jq] % d->moduli[jq]);
+            }
             if (!rc) rc = upload(ctx, &ctx->d_phat_pinv_fp, pfp.data(), pfp.size());
             if (!rc && d->log_n == 16 && d->size_p <= 8) {
                 // the same matrix for the int8 matrix cores: rows in groups of four with the bytes of the rescale term,
@@ -709,19 +702,8 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
             if (rc) return rc;
             lv.batched = true;
             if (fp_for_level(ctx, L)) {
-                std::vector<double> mfp(2 * mat_words + 16, 0.0);   // padded as the P -> Ql matrix is
-                for (uint32_t dg = 0; dg < beta; dg++) {
-                    const Digit &g = lv.digits[dg];
-                    for (uint32_t r = 0; r < g.n_out; r++) {
-                        const uint32_t lim = r < g.start ? r : r + g.size;
-                        const double m = (double)ctx->h_moduli[table_of(ctx, L, lim)];
-                        for (uint32_t i = 0; i < g.size; i++) {
-                            const size_t idx = g.mat_off + (size_t)r * g.size + i;
-                            mfp[2 * idx] = (double)mats[idx];
-                            mfp[2 * idx + 1] = (double)mats[idx] / m;
-                        }
-                    }
-                }
+                std::vector<double> mfp(mat_words + 8, 0.0);   // padded as the P -> Ql matrix is
+                for (size_t i = 0; i < mat_words; i++) mfp[i] = (double)mats[i];
                 rc = upload(ctx, &lv.d_mats_fp, mfp.data(), mfp.size());
                 if (rc) return rc;
                 if (ctx->log_n == 16) {
@@ -729,7 +711,6 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
                     std::vector<int32_t> tab;
                     for (uint32_t dg = 0; dg < beta; dg++) {
                         const Digit &g = lv.digits[dg];
-                        up[dg].mx_off = (uint32_t)(tab.size() / (4 * kMxRecord));
                         for (uint32_t r0 = 0; r0 < g.n_out; r0 += 4)
                             mx_record(tab, g.n_out - r0, g.size, 0,
                                       [&](uint32_t rr, uint32_t i) { return mats[g.mat_off + (size_t)(r0 + rr) * g.size + i]; },

@@ -104,8 +104,8 @@ struct NttArgs {
     uint32_t in_poly_stride;
     uint32_t out_poly_stride;
     // One block per direction, with everything that a pass reads about its primes: [tables][N][2] (operand, Shoup quotient), then
-    // [tables][N] twiddles as exact doubles for the FP64 back end (primes below 2^50), [tables][4] of q, 1/q, N^-1 mod q and
-    // (N^-1 mod q)/q as doubles, [tables] moduli, [tables][2] Barrett ratios; forward also, from p_constants_from_barrett words behind
+    // [tables][N] twiddles as exact doubles for the FP64 back end (primes below 2^50), [tables][4] of q, 1/q, N^-1 mod q as
+    // doubles and a zero, [tables] moduli, [tables][2] Barrett ratios; forward also, from p_constants_from_barrett words behind
     // the start of the ratios on, [size_q][2] Shoup pairs of P mod q and [size_q][2] of P^-1 mod q
     const uint64_t *tw;
     uint32_t size_qp;         // tables
@@ -282,7 +282,6 @@ struct BconvDesc {
     uint32_t map_off;    // offset into out_limb / out_table
     uint32_t n_in, n_out;
     uint32_t copy_first, copy_count;  // limbs copied from copy_base (same limb index in the unit's output)
-    uint32_t mx_off;     // first record of this unit in BconvRows::mx_tab (one record per four output rows)
 };
 struct BconvBatch {
     const uint64_t *x_base;
@@ -295,8 +294,8 @@ struct BconvBatch {
     uint32_t n_units, max_rows, max_copy;
     // the same units applied to `items` inputs (0 = 1): item k reads x_base + k * x_item_stride (and copy_base + k *
     // copy_item_stride) and writes out_base + k * out_item_stride (strides in words)
-    // FP64 back end (all primes involved below 2^50): the matrix as (M, M/m) pairs at the same offsets * 2,
-    // per-table constants as in NttArgs::fp_consts; null selects the integer kernel
+    // FP64 back end (all primes involved below 2^50): the matrix as doubles, per-table constants as in NttArgs::fp_consts; null
+    // selects the integer kernel
     const double *mat_fp;
     const double *fp_consts;
     uint32_t items;
@@ -317,7 +316,7 @@ struct BconvRows {
     LimbMap map;                 // Ql u P
     uint32_t K, units, items;
     int up;
-    const double *mat_fp;        // (M, M/m) pairs
+    const double *mat_fp;        // behind the last row 8 more that may be read
     // merged ModDown + rescale: the last row of every unit's matrix is the limb that is dropped; the other output
     // limbs receive sum_i x_i M[j][i] + ((t - sum_i x_i M[last][i] mod q_last) mod q_j), t = the limb before x
     int mdr;

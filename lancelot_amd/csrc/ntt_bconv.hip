@@ -42,13 +42,13 @@ struct ConvFp {
     __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
         const uint32_t last = d.n_out - 1;
         const FpMod m = fp_ctx(a, map_table(a.map, last)).m;
-        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + 2 * (d.mat_off + (size_t)last * d.n_in);
+        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + d.mat_off + (size_t)last * d.n_in;
 #pragma unroll
         for (int j = 0; j < 4; j++) rr[j] = fp_from_u64(t[j]);
 #pragma unroll
         for (int k = 0; k < NIN; k++) {
             if ((uint32_t)k >= d.n_in) break;
-            const double w = row[2 * k];
+            const double w = row[k];
 #pragma unroll
             for (int j = 0; j < 4; j++) rr[j] -= fp_mulmod(x[k][j], w, m);
         }
@@ -62,7 +62,7 @@ struct ConvFp {
     // 2^52; times 2^51 mod m it is congruent to the high part, and the modular product takes it as it is.
     __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t,
                                             const FpArith &ar) const {
-        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + 2 * (d.mat_off + (size_t)r * d.n_in);
+        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + d.mat_off + (size_t)r * d.n_in;
         double hi[4], lo[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
@@ -71,7 +71,7 @@ struct ConvFp {
         }
         double w[NIN];
 #pragma unroll
-        for (int k = 0; k < NIN; k++) w[k] = row[2 * k];   // (the matrices are padded: 8 pairs can be read whatever the row's length)
+        for (int k = 0; k < NIN; k++) w[k] = row[k];   // (the matrices are padded: 8 entries can be read whatever the row's length)
 #pragma unroll
         for (int k = 0; k < NIN; k++) {
             if ((uint32_t)k >= d.n_in) break;

@@ -537,8 +537,8 @@ __global__ __launch_bounds__(kThreads) void bconv_batched_kernel(BconvBatchK p) 
     }
 }
 
-// FP64 variant: every product is reduced on the fly to |r| <= 0.75 m, so the sum of up to 8 terms stays an
-// exact integer below 6 m < 2^53; one canonicalisation per output.
+// FP64 variant: every product is reduced on the fly to |r| <= 0.875 m (fp_mulmod, words below 2^50), so the sum of up to 8 terms stays
+// an exact integer of at most 7 m < 2^53; one canonicalisation per output.
 __global__ __launch_bounds__(kThreads) void bconv_batched_fp_kernel(BconvBatchK p) {
     const uint32_t item = blockIdx.z / p.b.n_units;
     const BconvDesc d = p.b.descs[blockIdx.z - item * p.b.n_units];
@@ -559,15 +559,15 @@ __global__ __launch_bounds__(kThreads) void bconv_batched_fp_kernel(BconvBatchK 
     double xv[kBatchIn];
 #pragma unroll
     for (int i = 0; i < kBatchIn; i++) xv[i] = (uint32_t)i < d.n_in ? fp_from_u64(x[((size_t)i << p.log_n) + j]) : 0.0;
-    const double *mat = p.b.mat_fp + 2 * d.mat_off;
+    const double *mat = p.b.mat_fp + d.mat_off;
     for (uint32_t row = row0; row < row0 + p.rows_per && row < d.n_out; row++) {
-        const double *m = mat + 2 * (size_t)row * d.n_in;
+        const double *m = mat + (size_t)row * d.n_in;
         const uint32_t t = p.b.out_table[d.map_off + row];
         const FpMod mod{p.b.fp_consts[4 * t], p.b.fp_consts[4 * t + 1]};
         double acc = 0.0;
 #pragma unroll
         for (int i = 0; i < kBatchIn; i++)
-            if ((uint32_t)i < d.n_in) acc += fp_mulmod(xv[i], m[2 * i], mod);
+            if ((uint32_t)i < d.n_in) acc += fp_mulmod(xv[i], m[i], mod);
         out[((size_t)p.b.out_limb[d.map_off + row] << p.log_n) + j] = fp_to_u64(fp_canonical(acc, mod));
     }
 }
