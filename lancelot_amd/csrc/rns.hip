@@ -291,14 +291,38 @@ struct SquareSumArgs {
     uint32_t L, log_n, count, parts;
 };
 
-// sums of products below 2^122, two words a thread: 64 of them fit into 128 bits
+// W neighbouring words of a thread
+template <int W>
+__device__ __forceinline__ void load_words(uint64_t (&v)[W], const uint64_t *p) {
+    static_assert(W == 1 || W == 2, "8 or 16 bytes");
+    if constexpr (W == 1) {
+        v[0] = *p;
+    } else {
+        const Words2 w = load_pair(p);
+        v[0] = w.x;
+        v[1] = w.y;
+    }
+}
+
+template <int W>
+__device__ __forceinline__ void store_words(uint64_t *p, const uint64_t (&v)[W]) {
+    if constexpr (W == 1)
+        *p = v[0];
+    else
+        *reinterpret_cast<Words2 *>(p) = Words2{v[0], v[1]};
+}
+
+// sums of products below 2^122, W words a thread: 64 of them fit into 128 bits
+template <int W>
 struct SquareSums {
-    U128 s[3][2];
+    U128 s[3][W];
     uint64_t q, r0, r1;
     __device__ __forceinline__ SquareSums(const SquareSumArgs &p, uint32_t limb)
         : q(scalar(p.moduli)[limb]), r0(scalar(p.barrett)[2 * limb]), r1(scalar(p.barrett)[2 * limb + 1]) {
 #pragma unroll
-        for (int i = 0; i < 3; i++) s[i][0] = s[i][1] = U128{0, 0};
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < W; j++) s[i][j] = U128{0, 0};
     }
     __device__ __forceinline__ uint64_t reduced(int i, int j) const { return barrett128(s[i][j].lo, s[i][j].hi, q, r0, r1); }
     // after term k, the number of products a term adds to one sum being at most two
@@ -307,56 +331,66 @@ struct SquareSums {
 #pragma unroll
         for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) s[i][j] = U128{reduced(i, j), 0};
+            for (int j = 0; j < W; j++) s[i][j] = U128{reduced(i, j), 0};
     }
-    // d gains the sums, as they are or times X^(N/2): psi^(N/2) at the words of the NTT order's first half, its negative at
-    // those of the second
-    __device__ __forceinline__ void add_to(Words2 *d, const SquareSumArgs &p, uint32_t limb, bool imaginary, bool upper) const {
-        const Shoup w = scalar_shoup(p.psi, ((size_t)limb << p.log_n) + 1);
+    // the first part's sums
+    __device__ __forceinline__ void real_part(uint64_t (&d)[3][W]) const {
 #pragma unroll
-        for (int i = 0; i < 3; i++) {
-            uint64_t v[2];
+        for (int i = 0; i < 3; i++)
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
-                v[j] = reduced(i, j);
-                if (!imaginary) continue;
-                v[j] = mul_shoup(v[j], w, q);
-                if (upper) v[j] = neg_mod(v[j], q);
+            for (int j = 0; j < W; j++) d[i][j] = reduced(i, j);
+    }
+    // d gains the second part's times X^(N/2): w = psi^(N/2) at the words of the NTT order's first half, its negative at those of the
+    // second
+    __device__ __forceinline__ void add_imaginary_part(uint64_t (&d)[3][W], Shoup w, bool upper) const {
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+#pragma unroll
+            for (int j = 0; j < W; j++) {
+                const uint64_t v = mul_shoup(reduced(i, j), w, q);
+                d[i][j] = add_mod(d[i][j], upper ? neg_mod(v, q) : v, q);
             }
-            d[i].x = add_mod(d[i].x, v[0], q);
-            d[i].y = add_mod(d[i].y, v[1], q);
-        }
     }
 };
 
-__device__ __forceinline__ void store_squares(const SquareSumArgs &p, uint32_t item, size_t at, const Words2 *d) {
+// psi^(N/2), which X^(N/2) is at half of the words
+__device__ __forceinline__ Shoup half_root(const SquareSumArgs &p, uint32_t limb) { return scalar_shoup(p.psi, ((size_t)limb << p.log_n) + 1); }
+
+template <int W>
+__device__ __forceinline__ void store_squares(const SquareSumArgs &p, uint32_t item, size_t at, const uint64_t (&d)[3][W]) {
     const size_t poly = (size_t)p.L << p.log_n;
     uint64_t *out = p.out01 + (size_t)item * 2 * poly + at;
-    *reinterpret_cast<Words2 *>(out) = d[0];
-    *reinterpret_cast<Words2 *>(out + poly) = d[1];
-    *reinterpret_cast<Words2 *>(p.out2 + (size_t)item * poly + at) = d[2];
+    store_words(out, d[0]);
+    store_words(out + poly, d[1]);
+    store_words(p.out2 + (size_t)item * poly + at, d[2]);
 }
 
-// grid: (N / 512, L, items).  Item = sum of (a - b)^2 over the `count` pairs of its row of the table [items][parts][count][2], plus X^(N/2) times that over its second
-// part's (null: no second part): the subtraction, the tensor square and the accumulation in one pass over the inputs.
+// grid: (N / (256 W), L, items).  Item = sum of (a - b)^2 over the `count` pairs of its row of the table [items][PARTS][count][2], plus
+// X^(N/2) times that over its second part's (null: no second part): the subtraction, the tensor square and the accumulation in one
+// pass over the inputs.
 // What bounds it: integer multiplies, about 1000 instructions a thread (45 pairs of two chunks, three limbs of 2^16 words, two pairs an item
 // 85 us: one reduction per sum and half the outputs buy what the reductions of X^(N/2) cost; 90 us with a reduction per term and a
 // pair an item.  An order of workgroups in which the items that share a ciphertext meet on one XCD: the same 85).
+template <int PARTS, int W>
 __global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(SquareSumArgs p) {
-    const uint32_t limb = blockIdx.y, j2 = 2 * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
-    const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + j2;
-    Words2 d[3] = {Words2{0, 0}, Words2{0, 0}, Words2{0, 0}};
-    for (uint32_t part = 0; part < p.parts; part++) {
-        const ScalarPtr pair = scalar(p.table) + ((size_t)item * p.parts + part) * p.count * 2;
+    const uint32_t limb = blockIdx.y, word = W * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
+    const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + word;
+    uint64_t d[3][W];
+    for (int part = 0; part < PARTS; part++) {
+        const ScalarPtr pair = scalar(p.table) + ((size_t)item * PARTS + part) * p.count * 2;
         if (part && !pair[0]) break;
-        SquareSums sums(p, limb);
+        SquareSums<W> sums(p, limb);
         const uint64_t q = sums.q;
 #pragma unroll 2
         for (uint32_t k = 0; k < p.count; k++) {
             const uint64_t *a = pair[2 * k] + at, *b = pair[2 * k + 1] + at;
-            const Words2 a0 = load_pair(a), a1 = load_pair(a + poly), b0 = load_pair(b), b1 = load_pair(b + poly);
+            uint64_t a0[W], a1[W], b0[W], b1[W];
+            load_words(a0, a);
+            load_words(a1, a + poly);
+            load_words(b0, b);
+            load_words(b1, b + poly);
 #pragma unroll
-            for (int j = 0; j < 2; j++) {
+            for (int j = 0; j < W; j++) {
                 const uint64_t x0 = sub_mod(a0[j], b0[j], q), x1 = sub_mod(a1[j], b1[j], q);
                 mac128(sums.s[0][j], x0, x0);
                 mac128(sums.s[1][j], x0, add_mod(x1, x1, q));
@@ -364,7 +398,10 @@ __global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(SquareSumArgs
             }
             sums.relieve(k);
         }
-        sums.add_to(d, p, limb, part != 0, j2 >> (p.log_n - 1));
+        if (part == 0)
+            sums.real_part(d);
+        else
+            sums.add_imaginary_part(d, half_root(p, limb), word >> (p.log_n - 1));
     }
     store_squares(p, item, at, d);
 }
@@ -377,7 +414,7 @@ __global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(SquareSumArgs
 __global__ __launch_bounds__(kThreads) void client_sums_kernel(SquareSumArgs p) {
     const uint32_t limb = blockIdx.y;
     const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + 2 * (blockIdx.x * kThreads + threadIdx.x);
-    SquareSums squares(p, limb);
+    SquareSums<2> squares(p, limb);
     const uint64_t q = squares.q;
     for (uint32_t c = 0, term = 0; c < p.parts; c++) {
         Words2 s0{0, 0}, s1{0, 0};
@@ -408,11 +445,11 @@ __global__ __launch_bounds__(kThreads) void client_sums_kernel(SquareSumArgs p) 
 __global__ __launch_bounds__(kThreads) void row_square_kernel(SquareSumArgs p) {
     const uint32_t limb = blockIdx.y, j2 = 2 * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
     const size_t poly = (size_t)p.L << p.log_n, at = ((size_t)limb << p.log_n) + j2;
-    Words2 d[3] = {Words2{0, 0}, Words2{0, 0}, Words2{0, 0}};
+    uint64_t d[3][2];
     for (uint32_t part = 0; part < 2; part++) {
         const uint32_t client = 2 * item + part;
         if (client >= p.count) break;
-        SquareSums sums(p, limb);
+        SquareSums<2> sums(p, limb);
         const uint64_t q = sums.q;
         for (int i = 0; i < 3; i++) {
             const Words2 t = load_pair(p.sums + ((size_t)2 * p.parts + i) * poly + at);
@@ -438,7 +475,10 @@ __global__ __launch_bounds__(kThreads) void row_square_kernel(SquareSumArgs p) {
             }
             sums.relieve(c);
         }
-        sums.add_to(d, p, limb, part != 0, j2 >> (p.log_n - 1));
+        if (part == 0)
+            sums.real_part(d);
+        else
+            sums.add_imaginary_part(d, half_root(p, limb), j2 >> (p.log_n - 1));
     }
     store_squares(p, item, at, d);
 }
@@ -1387,7 +1427,18 @@ hipError_t launch_pair_square_sum(const Tables &t, const uint64_t *psi, const ui
                                   uint32_t L, uint32_t items, uint32_t parts, uint32_t count, hipStream_t s) {
     if (items == 0 || items > 65535 || count == 0 || L == 0 || parts == 0 || parts > 2) return hipErrorInvalidValue;
     SquareSumArgs p{pairs, nullptr, out01, out2, t.moduli, t.barrett, psi, L, t.log_n, count, parts};
-    hipLaunchKernelGGL(pair_square_sum_kernel, dim3((1u << t.log_n) / (2 * kThreads), L, items), dim3(kThreads), 0, s, p);
+    // One part: while the launch is small its time is the chain of a thread, with one word half as long as with two; once the operands
+    // fill the caches 16-byte accesses win.  us of one word a thread / two, two terms an item: 3 limbs of 2^12 words 2.62 / 3.28, 6 of 2^16
+    // 5.66 / 5.91, 16 of 2^16 10.38 / 10.97, 24 of 2^16 15.8 / 16.2, 32 of 2^16 26.0 / 25.0, 160 of 2^16 152 / 132; ten terms, 10 of 2^15
+    // 23.2 / 19.7.
+    const uint32_t blocks = (1u << t.log_n) / kThreads;
+    const bool one_word = (uint64_t)count * items * L << t.log_n <= (uint64_t)48 << 16;
+    if (parts == 2)
+        hipLaunchKernelGGL((pair_square_sum_kernel<2, 2>), dim3(blocks / 2, L, items), dim3(kThreads), 0, s, p);
+    else if (one_word)
+        hipLaunchKernelGGL((pair_square_sum_kernel<1, 1>), dim3(blocks, L, items), dim3(kThreads), 0, s, p);
+    else
+        hipLaunchKernelGGL((pair_square_sum_kernel<1, 2>), dim3(blocks / 2, L, items), dim3(kThreads), 0, s, p);
     return hipGetLastError();
 }
 

@@ -69,6 +69,26 @@ def test_pairs_of_square_sums(oracle, capi, logn, bits, L, pairs, chunks):
     assert lib.he_pair_square_sum_packed(h, L, items, 0, dtab.ptr, d01.ptr, d2.ptr, None) == -1
 
 
+@pytest.mark.parametrize("items,chunks", [(1, 1), (3, 17), (16, 32), (16, 33)])
+def test_square_sums_with_one_and_with_two_words_a_thread(oracle, capi, items, chunks):
+    """he_pair_square_sum; up to 48 * 2^16 words a side, 512 terms of three limbs of 2^11, a thread takes one word, beyond two."""
+    cahel, parms, ctx, p = make_pair(oracle, 11, [60, 60, 30, 60], 1)
+    rng = np.random.default_rng(items + chunks)
+    lib, h, L = capi.lib(), ctx.he_handle(), 3
+    host = [rand_limbs(p, rng, range(L), n_polys=2) for _ in range(3)]
+    host[0][:], host[1][:] = 0, np.array([p.moduli[i] - 1 for i in range(L)], dtype=np.uint64)[None, :, None]
+    cts = [DeviceArray(capi, host=x) for x in host]
+    which = rng.integers(0, 3, (items, chunks, 2))
+    which[0, 0] = [1, 0]
+    table = DeviceArray(capi, host=np.array([c.ptr for c in cts], dtype=np.uint64)[which])
+    d01, d2 = DeviceArray(capi, shape=(items, 2, L, p.n)), DeviceArray(capi, shape=(items, 1, L, p.n))
+    capi.check(lib.he_pair_square_sum(h, L, items, chunks, table.ptr, d01.ptr, d2.ptr, None))
+    got = np.concatenate([d01.numpy(), d2.numpy()], axis=1)
+    squares = {(a, b): _square(p, host[a], host[b]) for a in range(3) for b in range(3)}
+    for k in range(items):
+        assert (got[k] == _total(p, [squares[tuple(pair)] for pair in which[k]])).all(), k
+
+
 @pytest.mark.parametrize("logn,bits,L", [(9, [60, 40, 40, 60], 3), (11, [60, 60, 30, 60], 3)])
 @pytest.mark.parametrize("clients,chunks", [(1, 1), (2, 1), (3, 2), (5, 4), (17, 1), (2, 17)])
 def test_row_sums_of_squares(oracle, capi, logn, bits, L, clients, chunks):
