@@ -216,6 +216,7 @@ NttArgs base_args(const he_context *ctx, bool forward) {
     a.epi_b_mask = 0xffffffffu;
     a.fp_mask = ctx->fp_mask;
     a.one_pass = ctx->one_pass;
+    a.cus = ctx->tune.cus;
     return a;
 }
 
@@ -1066,8 +1067,9 @@ namespace {
 // add_mask: which polynomials of `out` are added onto (bit p set) instead of overwritten
 // (addend: where the words to add come from, limb stride addend_stride between polynomials; nullptr: out itself)
 // inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
+// deal: see NttArgs
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
-                 uint64_t *ws, he_stream s, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0) {
+                 uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     const int accumulate = add_mask != 0;
     const size_t n = ctx->n();
@@ -1120,6 +1122,7 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     fwd.epi_b = addend ? addend : out;
     fwd.epi_b_poly_stride = addend ? addend_stride : L;
     fwd.epi_b_mask = add_mask;
+    fwd.deal = deal;
     fwd.w = ctx->d_pinv_mod_q;
     fwd.epi_dst = out;
     fwd.epi_dst_poly_stride = L;
@@ -1142,7 +1145,7 @@ extern "C" {
 
 int he_moddown(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, int accumulate,
                uint64_t *ws, he_stream s) {
-    return moddown_impl(ctx, L, cx, out, n_polys, accumulate ? 0xffffffffu : 0u, ws, s);
+    return moddown_impl(ctx, L, cx, out, n_polys, accumulate ? 0xffffffffu : 0u, ws, s, NTT_DEAL_NEVER);
 }
 
 size_t he_keyswitch_workspace_words(const he_context *ctx, uint32_t L) {
@@ -1276,7 +1279,7 @@ int he_keyswitch(const he_context *ctx, uint32_t L, const uint64_t *c, const uin
     const KsWorkspace w = ks_workspace(ctx, lv, L, 1, ws);
     bool inverted = false;
     if (int rc = ks_accumulate(ctx, lv, L, c, L, 1, evk, galois_elt, nullptr, ws, s, &inverted)) return rc;
-    return moddown_impl(ctx, L, w.cx, ct, 2, 0xffffffffu, w.tmp, s, inverted);
+    return moddown_impl(ctx, L, w.cx, ct, 2, 0xffffffffu, w.tmp, s, NTT_DEAL_ALWAYS, inverted);
 }
 
 int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const uint64_t *const *evk, uint64_t *ct_out,
@@ -1292,7 +1295,7 @@ int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const ui
     bool inverted = false;
     if (int rc = ks_accumulate(ctx, lv, L, ct_in + (size_t)L * n, L, 1, evk, galois_elt, nullptr, ws, s, &inverted, ct_in)) return rc;
     // out0 = sigma(c0) + ks0 (the inner product carries P sigma(c0)), out1 = ks1
-    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s, inverted);
+    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s, NTT_DEAL_ALWAYS, inverted);
 }
 
 int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *ct_in,
@@ -1323,7 +1326,7 @@ int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items
                                   2 * (size_t)L * n, S(s), ctx->use_fp ? ctx->d_fp_consts : nullptr, ctx->fp_mask, skip_own));
     }
     // out0 = [c0 +] sum sigma(c0) + ModDown(cx0), out1 = [c1 +] ModDown(cx1)
-    return moddown_impl(ctx, L, w.cx, ct_out, 2 * items, add_input ? 0xffffffffu : 0x55555555u, w.tmp, s);
+    return moddown_impl(ctx, L, w.cx, ct_out, 2 * items, add_input ? 0xffffffffu : 0x55555555u, w.tmp, s, NTT_DEAL_LONG);
 }
 
 int he_hoisted_rotations(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const uint64_t *const *evk,
@@ -1421,6 +1424,7 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
             fwd.pro_itw_fp = ctx->d_ipsi_fp;
         }
     }
+    fwd.deal = NTT_DEAL_ALWAYS;
     fwd.epi_mode = NTT_EPI_FMA_SUB_MUL;
     fwd.epi_a = cx;
     fwd.epi_a_poly_stride = LK;
@@ -1608,7 +1612,8 @@ int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64
     HE_HIP(launch_ntt_rows(a, 3 * items * LK, true, backend, S(s)));
     HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
     // divide by P onto the plaintexts
-    return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s, true, plain, plain ? L : 0);
+    return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
+                        plain ? L : 0);
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
@@ -1644,7 +1649,7 @@ int decrypt_flood_impl(const he_context *ctx, const DecryptArgs &d, uint32_t lim
     a.out_poly_stride = limbs;
     a.map = plain_map(limbs);
     const int backend = backend_for(ctx, a.map);
-    if (flood_rows_ok(ctx->log_n, limbs, items)) {
+    if (flood_rows_ok(ctx->log_n, limbs, items, ctx->tune.cus)) {
         HE_HIP(launch_flood_rows(a, k, stream_id, cdt, cdt_len, items, backend, S(s)));
     } else {
         HE_HIP(launch_sample_gauss_small(ctx->log_n, k, stream_id, reinterpret_cast<int8_t *>(noise), cdt, cdt_len, items, S(s)));

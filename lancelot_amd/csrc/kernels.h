@@ -90,6 +90,9 @@ enum : int {
     NTT_PRO_ROUND = 11,
 };
 
+// NttArgs::deal
+enum : uint32_t { NTT_DEAL_NEVER = 0, NTT_DEAL_LONG = 1 /* limbs of 2^15 words and more */, NTT_DEAL_ALWAYS = 2 };
+
 // Workgroups that a launch may have: a grid of 2^32 threads and more is not refused by the runtime, which starts what is left of
 // the count modulo 2^32.
 inline constexpr uint32_t most_workgroups(uint32_t threads) { return 0xffffffffu / threads < 0x7fffffffu ? 0xffffffffu / threads : 0x7fffffffu; }
@@ -119,6 +122,8 @@ struct NttArgs {
                               // absolute, no prologue/epilogue; map describes Ql u P)
     uint32_t listed;          // (jobs is there)
     uint32_t spread;          // filled in by the launcher: an eighth of every limb to an XCD (limb_block)
+    uint32_t deal;            // NTT_DEAL_*: whether a forward epilogue's launch may do that
+    uint32_t cus;             // compute units (Tuning::cus)
     uint32_t n_jobs, digit_limbs, digits;   // ... of so many digits of so many limbs (the last one may have fewer)
     const LimbGroup *groups;  // partition of `jobs` into runs with one table each, or nullptr
     uint32_t n_groups;
@@ -456,7 +461,7 @@ hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t str
                                      uint32_t cdt_len, uint32_t items, hipStream_t s);
 // ... or that polynomial's residues, with the rows pass of their forward transform done: limb l of item k at a.out (a: map mode,
 // dense).  flood_rows_ok: whether that is the faster way.
-bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items);
+bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items, uint32_t cus);
 hipError_t launch_flood_rows(const NttArgs &a, ChaChaKey key, uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t items,
                              int backend, hipStream_t s);
 

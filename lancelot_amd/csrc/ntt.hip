@@ -209,7 +209,7 @@ __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARA
 // 4 words a thread or 16 (FP64) at 2^12: 16 waves a limb shorten its chain, 4 issue fewer instructions, which counts once every CU has
 // a limb of its own (6 limbs 5.11 against 5.36 us, 96 5.74 against 5.93, 960 16.6 against 14.8).
 inline bool limb4(const NttArgs &a, int backend, uint32_t n_jobs) {
-    return a.log_n == 10 || (a.log_n == 12 && (backend != NTT_BACKEND_FP || n_jobs <= 256));
+    return a.log_n == 10 || (a.log_n == 12 && (backend != NTT_BACKEND_FP || n_jobs <= a.cus));
 }
 
 template <bool FWD>
@@ -271,7 +271,7 @@ inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_
     if (!a.one_pass || a.log_n > 14 || a.jobs || a.pro_mode != NTT_PLAIN || a.in_galois ||
         !(a.epi_mode == NTT_PLAIN || (!forward && a.epi_mode == NTT_EPI_MUL)))
         return false;
-    if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || n_jobs >= 256));
+    if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || n_jobs >= a.cus));
     return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && n_jobs >= 64) || (a.log_n == 14 && forward && n_jobs >= 192);
 }
 

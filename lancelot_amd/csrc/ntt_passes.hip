@@ -1057,12 +1057,31 @@ __global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodEx
 
 // Which launches deal every limb's workgroups to all XCDs (limb_block).  Otherwise an XCD has a contiguous range of the launch, which
 // the passes need that go over the same words one after the other: they meet them in the XCD's L2 (2 x 6 limbs of 2^16 words 10.8 us, dealt
-// out 13.1).  But with few limbs of both arithmetics, two XCDs have all the work of a 60-bit limb and two that of a 40-bit one.  It
-// pays where that work is most: in encryption's blocks pass and in the blocks passes with an
-// epilogue from three workgroups per CU on (both: encryption of 3 limbs of 2^16 words 56.0 -> 53.1 us, of 10 of 2^15 62.2 -> 57.1; the
-// epilogue alone: multiplication with 10 limbs of 2^15 64.0 -> 63.2, rotation with 5 limbs of 2^16 49.6 -> 48.4; with 2 limbs of 2^16, 512
-// workgroups, 27.6 -> 27.8).
-bool spread_ok(int backend, uint64_t n_jobs, uint64_t wgs, uint64_t least) { return backend == NTT_BACKEND_MIXED && n_jobs <= 32 && wgs >= least; }
+// out 13.1).  But with few limbs of both arithmetics, two XCDs have all the work of a 60-bit limb and two that of a 40-bit one.
+//
+// Encryption's blocks pass: up to four items, of which an XCD's range is half of one or less; a range over more evens itself out.
+// Together / dealt, us of an encryption on 60 + 40 .. + 60 bits, L + K limbs x items: 2^16, 3 + 1 x 1 32.4 / 29.2, x 2 48.1 / 44.0, x 4
+// 64.4 / 63.5, x 6 81.3 / 83.0, x 20 210 / 211, 20 + 4 x 1 96.9 / 84.2, x 4 254 / 240; 2^15, 10 + 2 x 1 43.3 / 38.2, x 4 82.5 / 80.9.  Short
+// limbs need more workgroups: 2^14, 12 + 4 x 1 35.0 / 31.1, 3 + 1 x 2 23.4 / 24.1, x 3 27.1 / 29.1, x 6 33.6 / 38.5, 12 + 4 x 2 47.3 / 45.4, x 4
+// 62.2 / 61.6; 2^13, 8 + 1 x 1 (288 workgroups) 20.1 / 21.0, 10 + 2 x 1 (384) 27.1 / 26.0, 3 + 1 x 8 26.0 / 29.8.
+bool spread_encryption(const NttArgs &a, int backend, uint32_t items, uint64_t wgs) {
+    if (backend != NTT_BACKEND_MIXED || items > 4) return false;
+    const uint64_t halves = a.log_n >= 15 || items == 1 ? 3 : items == 2 ? 6 : 24;   // workgroups for every two CUs
+    return 2 * wgs >= halves * a.cus;
+}
+
+// A blocks pass with an epilogue, where its caller asks for it (NttArgs::deal) and from three workgroups per CU on.  Behind an inner
+// product, which leaves an operand that no order of this launch finds in its XCD's L2: multiplication with 10 + 2 limbs of 2^15 words
+// 61.1 / 60.6, 20 + 4 of 2^14 61.9 / 61.2, eight of 10 + 2 of 2^16 446 / 438, rotation with 5 + 1 limbs of 2^16 49.2 / 47.8, 12 + 4 of 2^14
+// 41.2 / 40.1; with 2 + 1 of 2^16 (512 workgroups) 27.6 / 27.9.  Behind other passes only long limbs gain, and a single ciphertext's
+// encryption: encryption with 3 + 1 limbs of 2^16 words -4.7 %, 10 + 2 of 2^15 -6.2 %, hoisting of four ciphertexts, 4 + 2 limbs of 2^15
+// -1.5 %, but encryption of four, 8 + 1 limbs of 2^14 + 7.4 %, hoisting of eight, 5 + 1 of 2^13 + 3.2 %.  ModDown and rescale alone find their
+// operands where the passes before them have left them, rescale of 12 + 4 limbs of 2^16 22.3 / 24.2, ModDown of 8 + 1 20.9 / 22.4, and gain
+// while a ciphertext has no more limbs than there are XCDs: rescale of 4 + 2 16.0 / 15.5, ModDown of 3 + 1 15.9 / 15.5.
+bool spread_epilogue(const NttArgs &a, int backend, uint32_t limbs, uint32_t polys, uint64_t wgs) {
+    if (backend != NTT_BACKEND_MIXED || wgs < 3 * (uint64_t)a.cus) return false;
+    return a.deal == NTT_DEAL_ALWAYS || (a.deal == NTT_DEAL_LONG && a.log_n >= 15) || (polys <= 2 && limbs * polys <= 8);
+}
 
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
@@ -1156,14 +1175,14 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
 
 // one workgroup for every CU: 4 limbs of 2^16 coefficients 11.5 -> 9.9 us with the blocks pass behind them, 16 of 2^14 10.6 -> 9.4; half as
 // many workgroups more and the sampling is no longer hidden (6 of 2^16: 12.4 -> 12.5 us, 24 of 2^14: 11.5 -> 12.0)
-bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items) {
-    return log_n >= 12 && log_n <= 16 && limbs <= 64 && ((uint64_t)items * limbs << log_n) <= (1u << 18);
+bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items, uint32_t cus) {
+    return log_n >= 12 && log_n <= 16 && limbs <= 64 && ((uint64_t)items * limbs << (log_n - 10)) <= cus;
 }
 
 hipError_t launch_flood_rows(const NttArgs &args, ChaChaKey key, uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t items,
                              int backend, hipStream_t s) {
     const uint32_t n_jobs = items * args.map.limbs;
-    if (items == 0 || items > 65535 || args.jobs || cdt_len == 0 || cdt_len >= kSmallCdt || !flood_rows_ok(args.log_n, args.map.limbs, items)) return hipErrorInvalidValue;
+    if (items == 0 || items > 65535 || args.jobs || cdt_len == 0 || cdt_len >= kSmallCdt || !flood_rows_ok(args.log_n, args.map.limbs, items, args.cus)) return hipErrorInvalidValue;
     NttArgs a = args;
     a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
     const dim3 grid(n_jobs << (a.log_n - 10));
@@ -1199,7 +1218,7 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
     const bool epi = forward && (a.epi_mode == NTT_EPI_SUB_MUL || a.epi_mode == NTT_EPI_SUB_MUL_ADD || a.epi_mode == NTT_EPI_FMA_SUB_MUL);
-    a.spread = epi && spread_ok(backend, (uint64_t)kinds * repeats, wgs, 768);
+    a.spread = epi && spread_epilogue(a, backend, kinds, repeats, wgs);
     const NttHead head = ntt_head(a, grid.x, a.batch);
     const BlocksExtra extra = blocks_extra(a, forward);
 #define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
@@ -1251,7 +1270,7 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
         // The launch walks its limbs from the last to the first.  With more than one workgroup for every CU the integer
         // limbs, whose waves issue three times the instructions, take the last places, so that a CU's second workgroup is one of the short
         // ones (a rotation on [60, 40, 40, 60], two limbs of 2^16 words: 30.4 -> 29.1 us, in this kernel 9.8 -> 8.5)
-        const bool reorder = items == 1 && wgs > 256;
+        const bool reorder = items == 1 && wgs > a.cus;
         uint64_t order = 0;
         uint32_t at = x.L + x.K;
         for (int fp = 0; fp < 2; fp++)
@@ -1299,8 +1318,11 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, u
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
-    // (a limb's twiddles serve all items: dealt out, an XCD keeps its eighth of all of them; 8 x 24 limbs 792 -> 785 us of a product)
-    a.spread = items > 1;
+    // A limb's twiddles serve all items: dealt out, an XCD keeps its eighth of all of them.  It pays once the operands do not fit into the
+    // L2s, where the launch before has left them otherwise: from 6 * 2^16 words a polynomial on, 10 * 2^16 with limbs of 2^14 and less
+    // (products of a batch, us together / dealt: 8 x 24 limbs of 2^16 782 / 772, 2 x 3 of 2^16 43.2 / 42.6, 20 x 3 of 2^15 122 / 118, 2 x 3 of
+    // 2^15 32.4 / 32.7, 8 x 10 of 2^13 62.5 / 61.9; 8 x 3 of 2^14 39.5 / 41.1, 8 x 8 of 2^12 58.7 / 61.6).
+    a.spread = items > 1 && ((uint64_t)x.L * items << a.log_n) >= (uint64_t)(a.log_n >= 15 ? 6 : 10) << 16;
     const NttHead h = ntt_head(a, grid.x, x.square ? 1 : 0);
     if (backend == NTT_BACKEND_MIXED)
         hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
@@ -1323,7 +1345,7 @@ hipError_t launch_encrypt_blocks(const NttArgs &args, const uint64_t *pk, uint32
     if (per_launch == 0) return hipErrorInvalidValue;
     for (uint32_t first = 0; first < items; first += per_launch) {
         const dim3 grid((items - first < per_launch ? items - first : per_launch) * wgs_per_item);
-        a.spread = spread_ok(backend, (uint64_t)items * (L + K), grid.x, 256);
+        a.spread = spread_encryption(a, backend, items, grid.x);
         const NttHead head = ntt_head(a, grid.x, first);
         if (backend == NTT_BACKEND_MIXED)
             hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);

@@ -303,10 +303,12 @@ def test_hoisting_of_batches(oracle, capi, chain, local, logn, size_p, L, n_step
 
 @pytest.mark.parametrize("logn,bits,size_p,L", [(16, [60, 40, 40, 60], 1, 2), (16, [60, 40, 40, 60], 1, 3), (15, [40, 60, 50, 45, 30, 59, 60, 50], 2, 5),
                                                 (15, [60, 40, 50, 45, 30, 59, 60, 60], 2, 4), (14, [60, 40, 50, 45, 30, 59, 60, 60], 2, 6),
-                                                (12, [60, 40, 60], 1, 2), (13, [60, 40, 50, 45, 60], 1, 3)])
+                                                (12, [60, 40, 60], 1, 2), (13, [60, 40, 50, 45, 60], 1, 3),
+                                                (13, [60] + [40] * 23 + [60] * 8, 8, 24), (14, [60] + [40] * 15 + [60] * 4, 4, 15)])
 def test_key_switch_of_a_mixed_chain(oracle, capi, logn, bits, size_p, L):
     """Rotation and key switch + rescale where the inner product takes its limbs in an order of their own (more than one workgroup for
-    every CU) and where it does not, with even and odd numbers of primes (behind an odd one the constants of P lie a word further)."""
+    every CU) and where it does not, with even and odd numbers of primes (behind an odd one the constants of P lie a word further), with an epilogue's workgroups dealt to all
+    XCDs (768 and more) and not."""
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(logn + L)
     lib, h = capi.lib(), ctx.he_handle()
@@ -420,20 +422,63 @@ def test_conversions_on_both_sides_of_the_matrix_kernel(oracle, capi, size_p, L,
         assert (got[k] == want[k % 2]).all(), k
 
 
-@pytest.mark.parametrize("logn,bits,size_p", [(13, [60, 40, 40, 50, 60, 60], 2), (14, [60, 40, 40, 60], 1), (15, [40, 60, 60, 40, 60], 1)])
-def test_encryption_of_a_mixed_chain(oracle, capi, logn, bits, size_p):
-    """Encryption's blocks pass deals the limbs' workgroups to all XCDs from 256 workgroups on (L + K limbs of N / 256)."""
+@pytest.mark.parametrize("logn,L,size_p,items", [(14, 3, 1, 1), (13, 8, 1, 1), (13, 10, 2, 1), (14, 3, 1, 2), (14, 4, 2, 2), (12, 24, 8, 2), (14, 8, 1, 4),
+                                                 (14, 10, 2, 4), (15, 2, 1, 4), (15, 2, 1, 5), (15, 10, 2, 2)])
+def test_encryption_of_a_mixed_chain(oracle, capi, logn, L, size_p, items):
+    """Encryption's blocks pass deals the limbs' workgroups to all XCDs for up to four items, from 3 workgroups for two CUs on, with limbs
+    of 2^14 words and less from 3 a CU for two items and from 12 for more; its ModDown from 3 a CU on for one item or limbs of 2^15."""
+    bits = [60] + [40] * (L - 1) + [60] * size_p
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     lib, h, n = capi.lib(), ctx.he_handle(), p.n
     key = oracle.chacha_key(3)
     kp = key.ctypes.data_as(C.POINTER(C.c_uint32))
-    rng = np.random.default_rng(logn)
-    pk, plain = rand_limbs(p, rng, range(p.size_qp), n_polys=2), rand_limbs(p, rng, range(p.size_q))
-    dpk, dplain, dct = DeviceArray(capi, host=pk), DeviceArray(capi, host=plain), DeviceArray(capi, shape=(2, p.size_q, n))
-    ws = DeviceArray(capi, shape=(lib.he_encrypt_batch_workspace_words(h, p.size_q, 1),))
-    capi.check(lib.he_encrypt(h, p.size_q, dplain.ptr, dpk.ptr, kp, 11, dct.ptr, ws.ptr, None))
-    got, u = dct.numpy(), p.ntt_fwd(p.sample_ternary(key, 11, p.size_qp))
-    for i in range(2):
-        e = p.ntt_fwd(p.sample_error(key, 12 + i, p.size_qp))
-        want = p.moddown(np.ascontiguousarray(p.mul_add(u, pk[i], e)))
-        assert (got[i] == (p.add(want, plain) if i == 0 else want)).all(), i
+    rng = np.random.default_rng(logn + L)
+    pk, plain = rand_limbs(p, rng, range(p.size_qp), n_polys=2), rand_limbs(p, rng, range(p.size_q), n_polys=items)
+    cts = np.zeros((items, 2, L, n), dtype=np.uint64)
+    cts[:, 0] = plain
+    dpk, dcts = DeviceArray(capi, host=pk), DeviceArray(capi, host=cts)
+    ws = DeviceArray(capi, shape=(lib.he_encrypt_batch_workspace_words(h, L, items),))
+    capi.check(lib.he_encrypt_batch(h, L, items, dpk.ptr, kp, 11, dcts.ptr, ws.ptr, None))
+    got = dcts.numpy()
+    for k in sorted({0, items - 1}):
+        u = p.ntt_fwd(p.sample_ternary(key, 11 + 3 * k, p.size_qp))
+        for i in range(2):
+            e = p.ntt_fwd(p.sample_error(key, 12 + 3 * k + i, p.size_qp))
+            want = p.moddown(np.ascontiguousarray(p.mul_add(u, pk[i], e)))
+            assert (got[k, i] == (p.add(want, plain[k]) if i == 0 else want)).all(), (k, i)
+
+
+@pytest.mark.parametrize("logn,L,polys", [(16, 3, 2), (16, 4, 2), (16, 5, 2), (16, 3, 4), (15, 6, 4)])
+def test_moddown_and_rescale_of_a_mixed_chain(oracle, capi, logn, L, polys):
+    """Their epilogue's workgroups, 768 and more, go to all XCDs for up to eight limbs of two polynomials."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, [60] + [40] * (L - 1) + [60], 1)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    cx = rand_limbs(p, np.random.default_rng(L + polys), range(L + 1), n_polys=polys)
+    dcx, dct, ws = DeviceArray(capi, host=cx), DeviceArray(capi, host=cx[:, :L]), DeviceArray(capi, shape=(polys, L, n))
+    down, low = DeviceArray(capi, shape=(polys, L, n)), DeviceArray(capi, shape=(polys, L - 1, n))
+    capi.check(lib.he_moddown(h, L, dcx.ptr, down.ptr, polys, 0, ws.ptr, None))
+    capi.check(lib.he_rescale(h, dct.ptr, low.ptr, polys, L, ws.ptr, None))
+    assert (down.numpy() == np.stack([p.moddown(x) for x in cx])).all()
+    assert (low.numpy() == p.rescale(np.ascontiguousarray(cx[:, :L]))).all()
+
+
+@pytest.mark.parametrize("chain", sorted(CHAINS))
+@pytest.mark.parametrize("logn,L,items", [(12, 8, 19), (12, 8, 20), (13, 5, 16), (15, 2, 5), (15, 2, 6)])
+def test_products_on_both_sides_of_the_dealt_tensor_product(oracle, capi, chain, logn, L, items):
+    """A batch's tensor product deals its workgroups to all XCDs from 10 * 2^16 words a polynomial on, from 6 * 2^16 with limbs of 2^15."""
+    bits = (CHAINS[chain] * 2)[:L + 1]
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, 1)
+    rng = np.random.default_rng(logn + items)
+    lib, h = capi.lib(), ctx.he_handle()
+    host = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(2)]
+    dev = [DeviceArray(capi, host=k) for k in host]
+    keys = capi.evk_array([dev[d % 2].ptr for d in range(L)])
+    a, b = (rand_limbs(p, rng, range(L), n_polys=2 * items).reshape(items, 2, L, p.n) for _ in range(2))
+    da, db, out = DeviceArray(capi, host=a), DeviceArray(capi, host=b), DeviceArray(capi, shape=(items, 2, L - 1, p.n))
+    ws = DeviceArray(capi, shape=(lib.he_multiply_relin_rescale_batch_workspace_words(h, L, items),))
+    capi.check(lib.he_multiply_relin_rescale_batch(h, L, items, da.ptr, db.ptr, keys, out.ptr, ws.ptr, None))
+    got = out.numpy()
+    for k in (0, items // 2, items - 1):
+        d = p.tensor(a[k], b[k])
+        ks = p.key_switch(d[2], [host[j % 2] for j in range(L)])
+        assert (got[k] == p.rescale(np.stack([p.add(d[i], ks[i]) for i in range(2)]))).all(), k
