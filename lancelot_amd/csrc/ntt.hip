@@ -16,7 +16,7 @@
 // small degrees and the conversion on the matrix cores, and chooses between them.
 //
 // Two arithmetic back ends share this skeleton:
-//   integer : 64-bit Shoup/Harvey butterflies, any prime below 2^61 (~35 VALU instructions per butterfly);
+//   integer : 64-bit Shoup/Harvey butterflies, any prime below 2^61 (25 VALU instructions per butterfly, 31 back);
 //             inverse twiddles are pre-halved so that 1/N comes for free
 //   FP64    : exact integer arithmetic in doubles for primes below 2^50 (8 full-rate operations per
 //             butterfly, see modarith.cuh); values between the two passes are lazy signed doubles stored
@@ -138,8 +138,8 @@ __global__ __launch_bounds__((1 << LOGN) / 16) void ntt_limb_fp_kernel(NttArgs a
 // chain of one workgroup: with 16 words a thread N / 1024 waves a SIMD go through blocks of four stages, each behind a fetch of its 15
 // twiddles and a trip of all its words through LDS; here all twiddles are requested together with the words, and only the
 // exchanges of more than 256 words (two at 2^12) go through LDS, the others stay in a wave's registers (Tile4).
-// Six limbs of 50 bits, forward and inverse: 2^10 4.35 -> 3.76 and 4.76 -> 3.90 us, 2^12 5.36 -> 5.11 and 5.85 -> 5.36; of 60 bits
-// at 2^10, against rows pass and blocks pass, 6.6 -> 3.8 us.
+// Six limbs of 50 bits, forward and inverse, the GPU's time of calls in a row: 2^10 4.39 -> 2.32 and 4.91 -> 2.48 us, 2^12 5.37 -> 4.67 and
+// 5.95 -> 4.76; of 60 bits at 2^10, against rows pass and blocks pass, 5.66 -> 3.14 and 5.76 -> 3.46.
 template <int LOGN, bool FWD, int BE>
 __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARAMS, const uint64_t *w) {
     using T4 = Tile4<LOGN, LOGN>;
@@ -207,7 +207,8 @@ __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARA
 }
 
 // 4 words a thread or 16 (FP64) at 2^12: 16 waves a limb shorten its chain, 4 issue fewer instructions, which counts once every CU has
-// a limb of its own (6 limbs 5.11 against 5.36 us, 96 5.74 against 5.93, 960 16.6 against 14.8).
+// a limb of its own (forward / inverse, us: 6 limbs 4.67 / 4.76 against 5.37 / 5.95, 192 5.64 / 5.67 against 6.18 / 6.72, 576 12.8 / 12.9 against
+// 11.9 / 13.4, 960 16.1 / 16.7 against 14.9 / 16.8).
 inline bool limb4(const NttArgs &a, int backend, uint32_t n_jobs) {
     return a.log_n == 10 || (a.log_n == 12 && (backend != NTT_BACKEND_FP || n_jobs <= a.cus));
 }
@@ -259,20 +260,22 @@ hipError_t launch_limb(NttArgs a, uint32_t n_polys, int backend, hipStream_t s) 
     }
 }
 
-// The launches that a whole-limb kernel covers and wins.  A limb is one workgroup on one CU: up to N = 2^12 that is
-// faster on FP64 than two launches whatever the number of limbs; a limb of 2^13 or 2^14 words takes one CU
-// longer than two launches of a few limbs take, so there the kernel pays only when the launch has enough limbs to occupy
-// the chip: from 64 limbs on at 2^13 (192 limbs 10.7 against 13.8 us, 576 limbs 25.6 against 33.3 us), from 192 on in the
-// forward direction at 2^14 (19.4 against 25.1 us, 576 limbs 55.7 against 59.9 us; its inverse, whose first blocks wait for the whole
-// limb, takes 28.4 against 25.4 us and 82 against 56 us).  Integers take 2.5 times the instructions: one launch at 2^10
-// always, at 2^12 once there is a limb for every CU (6 limbs 7.2 against 6.8 us, inverse 7.9 against 6.9; 96 limbs 7.6 against 8.4 and 8.3 against
-// 8.2; 960 limbs 24.2 against 30.7 and 26.8 against 33.2).  a.one_pass = 2 forces it (tests).
+// The launches that a whole-limb kernel covers and wins; us of one launch against rows pass and blocks pass, forward / inverse.  A limb
+// is one workgroup on one CU.  Up to N = 2^12 that is faster on FP64 whatever the number of limbs, or as fast and one launch for the
+// host instead of two (2^12, 6 limbs 4.67 / 4.76 against 5.46 / 5.14, 960 14.9 / 16.8 against 21.2 / 22.3; 2^9, 96 limbs 5.0 / 5.6 against 4.6 /
+// 4.7, 960 5.2 / 5.8 against 6.2 / 6.0).  A limb of 2^13 or 2^14 words takes one CU longer than two launches of a few limbs take: at 2^13 the
+// kernel pays from a limb for every second CU on (96 limbs 9.2 / 10.8 against 8.1 / 8.3, 129 9.5 / 11.1 against 10.2 / 10.6, 192 9.9 / 11.4 against
+// 12.1 / 12.3, 960 32.5 / 38.1 against 50.2 / 49.7), at 2^14 from 192 limbs on in the forward direction (129 limbs 16.0 against 15.9, 192 17.1
+// against 19.0, 960 71.4 against 84.4; its inverse, whose first blocks wait for the whole limb, takes 18.7 against 16.7 with 129 and 63.3
+// against 54.1 with 576).  Integers take 2.5 times the instructions: one launch at 2^10 always, at 2^12 from five limbs for every
+// eight CUs on (6 limbs 7.0 / 7.3 against 6.2 / 6.3, 128 7.6 / 7.9 against 7.5 / 7.6, 192 8.0 / 8.2 against 9.9 / 10.3, 960 24.4 / 25.6 against 29.1 /
+// 31.5; 60 and 40 bits, 128 limbs 7.4 / 7.7 against 6.9 / 7.1, 160 7.6 / 7.9 against 7.8 / 7.8).  a.one_pass = 2 forces it (tests).
 inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_jobs) {
     if (!a.one_pass || a.log_n > 14 || a.jobs || a.pro_mode != NTT_PLAIN || a.in_galois ||
         !(a.epi_mode == NTT_PLAIN || (!forward && a.epi_mode == NTT_EPI_MUL)))
         return false;
-    if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || n_jobs >= a.cus));
-    return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && n_jobs >= 64) || (a.log_n == 14 && forward && n_jobs >= 192);
+    if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || 8 * (uint64_t)n_jobs >= 5 * (uint64_t)a.cus));
+    return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && 2 * (uint64_t)n_jobs >= a.cus) || (a.log_n == 14 && forward && n_jobs >= 192);
 }
 
 constexpr int kFuseLog = 11;

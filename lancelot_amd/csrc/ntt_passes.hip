@@ -1134,9 +1134,12 @@ bool ntt_source_intt_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
 }
 
 // ModDown + rescale with one special prime: two inverse rows passes in front of every output limb's, which pay as long as the launch is
-// small.  n limbs in all, us of a multiplication with a launch for them -> without (50 bits / 60 bits): n = 2^12, L = 2 26.0 -> 21.9 /
-// 27.2 -> 25.0; 2^14, L = 4 26.1 -> 23.0 / 31.4 -> 28.7; 2^15, L = 8 47.1 -> 45.7 / 62.8 -> 61.8; 2^16, L = 4 39.9 -> 38.5 / 54.7 ->
-// 54.9, L = 6 55.7 -> 55.0 / 72.9 -> 76.1.
+// small: every limb repeats them, on CUs that are idle otherwise.  The line is where integers, with 2.5 times the instructions, cease to
+// gain.  Multiplication with a launch for them -> without, by n_jobs limbs of 2^16 words.  60 bits, the GPU's time, us: 0.1 (n = 2^12, L =
+// 2) 27.9 -> 25.7, 1.5 (2^14, 4) 32.8 -> 30.6, 3.5 (2^14, 8) 46.9 -> 44.5, 4 (2^15, 5) 46.7 -> 45.6; back to back: 6 (2^15, 7) 56.5 -> 55.5, 6 (2^16,
+// 4) 54.2 -> 54.0, 7 (2^15, 8) 61.7 -> 61.9, 8 (2^16, 5) 62.5 -> 63.5, 10 (2^16, 6) 72.0 -> 75.1.  50 bits: 0.1 22.6 -> 20.1, 1.5 26.2 -> 24.0,
+// 4 (2^15, 5) 35.6 -> 33.6, 7 48.6 -> 47.5, 8 48.9 -> 47.5, 10 56.4 -> 55.7, 14 71.0 -> 72.0; 60 and 40 bits: 7 54.1 -> 53.0, 8 57.7 -> 56.2, 10
+// 63.3 -> 64.3.  (With primes below 2^50 it would pay to 10.)
 bool ntt_two_sources_ok(uint32_t log_n, uint32_t n_jobs, uint32_t n_tables) {
     return ntt_source_intt_ok(log_n, n_jobs, n_tables) && ((uint64_t)n_jobs << log_n) <= ((uint64_t)7 << 16);
 }

@@ -37,11 +37,12 @@ def test_batched_transforms(oracle, capi, chain, logn, limbs, polys):
 
 
 @pytest.mark.parametrize("chain", sorted(CHAINS))
-@pytest.mark.parametrize("logn,limbs,polys", [(10, 1, 1), (10, 5, 3), (12, 1, 1), (12, 5, 51), (12, 5, 52)])
+@pytest.mark.parametrize("logn,limbs,polys", [(10, 1, 1), (10, 5, 3), (12, 1, 1), (12, 3, 53), (12, 5, 32), (12, 5, 51), (12, 5, 52), (13, 5, 25),
+                                              (13, 4, 32)])
 @pytest.mark.parametrize("one_pass", ["default", "forced"])
 def test_whole_limb_transforms(oracle, capi, monkeypatch, chain, logn, limbs, polys, one_pass):
-    """A limb of 2^10 or 2^12 words in one workgroup, on both sides of the number of limbs (255 and 260) at which the kernel
-    changes."""
+    """A limb of 2^10, 2^12 or 2^13 words in one workgroup, on both sides of the numbers of limbs at which it begins to run at 2^12
+    (integers, 159 and 160) and 2^13 (125 and 128) and at which the kernel changes at 2^12 (255 and 260)."""
     monkeypatch.setenv("CAHEL_HIP_FORCE_ONE_PASS", "1" if one_pass == "forced" else "0")
     cahel, parms, ctx, p = make_pair(oracle, logn, CHAINS[chain], 1)
     lib, h = capi.lib(), ctx.he_handle()
