@@ -17,6 +17,16 @@ namespace {
 
 constexpr int kThreads = 256;
 
+// A value of a vector or a result, which are only 8-byte aligned for certain, as one 16-byte access
+typedef double Value2 __attribute__((ext_vector_type(2), aligned(8)));
+
+__device__ __forceinline__ double2 get(const double2 *v) {
+    const Value2 x = *reinterpret_cast<const Value2 *>(v);
+    return double2{x.x, x.y};
+}
+
+__device__ __forceinline__ void put(double2 *v, double2 x) { *reinterpret_cast<Value2 *>(v) = Value2{x.x, x.y}; }
+
 __device__ __forceinline__ double2 cmul(double2 a, double2 w) {
     return double2{a.x * w.x - a.y * w.y, a.x * w.y + a.y * w.x};
 }
@@ -72,7 +82,7 @@ struct FftTarget {
 __device__ __forceinline__ void store_value(const FftTarget &dst, uint32_t item, uint32_t i, double2 v) {
     const size_t at = (size_t)item * dst.count + i;
     if (dst.both)
-        reinterpret_cast<double2 *>(dst.re)[at] = v;
+        put(reinterpret_cast<double2 *>(dst.re) + at, v);
     else
         dst.re[at] = v.x;
 }
@@ -89,7 +99,7 @@ __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t
         if (threadIdx.x == 0 && src.max_bits) src.max_bits[blockIdx.y] = 0;
         for (uint32_t i = threadIdx.x; i < tile; i += kThreads) s[i] = source_value(src, blockIdx.y, i);
     } else {
-        for (uint32_t i = threadIdx.x; i < tile; i += kThreads) s[i] = g[i];
+        for (uint32_t i = threadIdx.x; i < tile; i += kThreads) s[i] = get(g + i);
     }
     __syncthreads();
     for (uint32_t k = 2; k <= tile; k <<= 1) {
@@ -107,7 +117,7 @@ __global__ __launch_bounds__(kThreads) void cfft_lds_kernel(double2 *v, uint32_t
     if (!INVERSE && dst.re) {
         for (uint32_t i = threadIdx.x; i < dst.count; i += kThreads) store_value(dst, blockIdx.y, i, s[i]);
     } else {
-        for (uint32_t i = threadIdx.x; i < tile; i += kThreads) g[i] = s[i];
+        for (uint32_t i = threadIdx.x; i < tile; i += kThreads) put(g + i, s[i]);
     }
 }
 
@@ -218,15 +228,15 @@ __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, Fft
             for (int j = 0; j < 4; j++) x[j] = source_value(src, item, pos(0, j));
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
+            for (int j = 0; j < 4; j++) x[j] = get(v + pos(0, j));
         }
         F::load_tw(tw, t, log_slots, 0, pos);
         F::down(x, tw, re, im, tid);
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[pos(NB - 1, j)] = x[j];
+        for (int j = 0; j < 4; j++) put(v + pos(NB - 1, j), x[j]);
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = v[pos(NB - 1, j)];
+        for (int j = 0; j < 4; j++) x[j] = get(v + pos(NB - 1, j));
         F::load_tw(tw, t, log_slots, 0, pos);
         F::up(x, tw, re, im, tid);
         if (dst.re) {
@@ -235,7 +245,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void cfft_rows_kernel(double2 *v, Fft
                 if (pos(0, j) < dst.count) store_value(dst, item, pos(0, j), x[j]);
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
+            for (int j = 0; j < 4; j++) put(v + pos(0, j), x[j]);
         }
     }
 }
@@ -266,15 +276,15 @@ __global__ __launch_bounds__((1 << (B - 2)) * kFftBlocks<B>) void cfft_blocks_ke
             for (int j = 0; j < 4; j++) x[j] = source_value(src, item, pos(0, j));
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = v[pos(0, j)];
+            for (int j = 0; j < 4; j++) x[j] = get(v + pos(0, j));
         }
         F::load_tw(tw, t, log_slots, log_slots - B, pos);
         F::down(x, tw, re, im, tid);
 #pragma unroll
-        for (int j = 0; j < 4; j++) v[pos(LAST, j)] = x[j];
+        for (int j = 0; j < 4; j++) put(v + pos(LAST, j), x[j]);
     } else {
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = v[pos(LAST, j)];
+        for (int j = 0; j < 4; j++) x[j] = get(v + pos(LAST, j));
         F::load_tw(tw, t, log_slots, log_slots - B, pos);
         F::up(x, tw, re, im, tid);
         if (dst.re && log_slots == B) {
@@ -283,7 +293,7 @@ __global__ __launch_bounds__((1 << (B - 2)) * kFftBlocks<B>) void cfft_blocks_ke
                 if (pos(0, j) < dst.count) store_value(dst, item, pos(0, j), x[j]);
         } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[pos(0, j)] = x[j];
+            for (int j = 0; j < 4; j++) put(v + pos(0, j), x[j]);
         }
     }
 }
@@ -336,7 +346,7 @@ __global__ __launch_bounds__(kThreads) void encode_round_kernel(const double2 *v
     double val = 0.0;
     if (k % gap == 0) {
         const uint32_t i = k / gap;
-        const double2 z = v[__brev(i) >> (32 - log_slots)];
+        const double2 z = get(v + (__brev(i) >> (32 - log_slots)));
         val = round((imag ? z.y : z.x) * fix);
     }
     uint64_t *o = sink.out + blockIdx.y * sink.out_item_stride + c;
@@ -358,7 +368,7 @@ __global__ __launch_bounds__(kThreads) void encode_round_tiled_kernel(const doub
     max_bits += blockIdx.y;
     const uint32_t rmid = mid_bits ? __brev(mid) >> (32 - mid_bits) : 0;
     const uint32_t brev4_y = __brev(y) >> 28;
-    tile[y][x] = v[(brev4_y << (log_slots - 4)) | (rmid << 4) | x];
+    tile[y][x] = get(v + ((brev4_y << (log_slots - 4)) | (rmid << 4) | x));
     __syncthreads();
     const double2 z = tile[x][y];
     const uint32_t i = (brev4_y << (log_slots - 4)) | (mid << 4) | x;
@@ -538,7 +548,7 @@ __global__ __launch_bounds__(256 * LIMBS) void decode_rows_compose_kernel(HE_HEA
         val.x = compose<LIMBS>(d[0], LIMBS, inv_scale, moduli, barrett, garner, LIMBS);
         val.y = compose<LIMBS>(d[1], LIMBS, inv_scale, moduli, barrett, garner, LIMBS);
         const uint32_t k = (uint32_t)glob(0, (int)j);   // (below N / 2)
-        if ((k & ((1u << log_gap) - 1)) == 0) v[__brev(k >> log_gap) >> (32 - log_slots)] = val;
+        if ((k & ((1u << log_gap) - 1)) == 0) put(v + (__brev(k >> log_gap) >> (32 - log_slots)), val);
     }
 }
 
@@ -590,7 +600,7 @@ hipError_t run_fft(double2 *v, uint32_t slots, uint32_t items, const FftTables &
 // out[item][i] = v[item][i] for i < count: the leading slots of every item, packed
 __global__ __launch_bounds__(kThreads) void take_slots_kernel(const double2 *v, uint32_t slots, uint32_t count, double2 *out) {
     const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-    if (i < count) out[(size_t)blockIdx.y * count + i] = v[(size_t)blockIdx.y * slots + i];
+    if (i < count) put(out + (size_t)blockIdx.y * count + i, get(v + (size_t)blockIdx.y * slots + i));
 }
 
 }  // namespace
