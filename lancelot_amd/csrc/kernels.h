@@ -115,7 +115,7 @@ struct NttArgs {
     const double *tw_fp;      // (into the block; set where a kernel starts)
     const double *fp_consts;
     uint64_t fp_mask;         // bit t: table t has a prime below 2^50 (read by the mixed back end only)
-    int one_pass;             // N <= 2^14, FP64 back end, plain transforms: one kernel with the limb resident in LDS
+    int one_pass;             // plain transforms of limbs that LDS holds in one launch: 0 never, 1 by one_pass_ok, 2 wherever a kernel is there
     const uint64_t *moduli;   // [tables]
     const uint64_t *barrett;  // [tables][2]
     const LimbJob *jobs;      // explicit list: the converted limbs of a ModUp, digit by digit, ascending (then in/out limbs are

@@ -265,9 +265,9 @@ hipError_t launch_limb(NttArgs a, uint32_t n_polys, int backend, hipStream_t s) 
 // host instead of two (2^12, 6 limbs 4.67 / 4.76 against 5.46 / 5.14, 960 14.9 / 16.8 against 21.2 / 22.3; 2^9, 96 limbs 5.0 / 5.6 against 4.6 /
 // 4.7, 960 5.2 / 5.8 against 6.2 / 6.0).  A limb of 2^13 or 2^14 words takes one CU longer than two launches of a few limbs take: at 2^13 the
 // kernel pays from a limb for every second CU on (96 limbs 9.2 / 10.8 against 8.1 / 8.3, 129 9.5 / 11.1 against 10.2 / 10.6, 192 9.9 / 11.4 against
-// 12.1 / 12.3, 960 32.5 / 38.1 against 50.2 / 49.7), at 2^14 from 192 limbs on in the forward direction (129 limbs 16.0 against 15.9, 192 17.1
-// against 19.0, 960 71.4 against 84.4; its inverse, whose first blocks wait for the whole limb, takes 18.7 against 16.7 with 129 and 63.3
-// against 54.1 with 576).  Integers take 2.5 times the instructions: one launch at 2^10 always, at 2^12 from five limbs for every
+// 12.1 / 12.3, 960 32.5 / 38.1 against 50.2 / 49.7), at 2^14 from three limbs for every four CUs on in the forward direction (129 limbs 16.0
+// against 15.9, 192 17.1 against 19.0, 960 71.4 against 84.4; its inverse, whose first blocks wait for the whole limb, takes 18.7 against 16.7
+// with 129 and 63.3 against 54.1 with 576).  Integers take 2.5 times the instructions: one launch at 2^10 always, at 2^12 from five limbs for every
 // eight CUs on (6 limbs 7.0 / 7.3 against 6.2 / 6.3, 128 7.6 / 7.9 against 7.5 / 7.6, 192 8.0 / 8.2 against 9.9 / 10.3, 960 24.4 / 25.6 against 29.1 /
 // 31.5; 60 and 40 bits, 128 limbs 7.4 / 7.7 against 6.9 / 7.1, 160 7.6 / 7.9 against 7.8 / 7.8).  a.one_pass = 2 forces it (tests).
 inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_jobs) {
@@ -275,7 +275,7 @@ inline bool one_pass_ok(const NttArgs &a, int backend, bool forward, uint32_t n_
         !(a.epi_mode == NTT_PLAIN || (!forward && a.epi_mode == NTT_EPI_MUL)))
         return false;
     if (backend != NTT_BACKEND_FP) return a.log_n == 10 || (a.log_n == 12 && (a.one_pass == 2 || 8 * (uint64_t)n_jobs >= 5 * (uint64_t)a.cus));
-    return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && 2 * (uint64_t)n_jobs >= a.cus) || (a.log_n == 14 && forward && n_jobs >= 192);
+    return a.one_pass == 2 || a.log_n <= 12 || (a.log_n == 13 && 2 * (uint64_t)n_jobs >= a.cus) || (a.log_n == 14 && forward && 4 * (uint64_t)n_jobs >= 3 * (uint64_t)a.cus);
 }
 
 constexpr int kFuseLog = 11;

@@ -368,9 +368,10 @@ __device__ __forceinline__ void store_squares(const SquareSumArgs &p, uint32_t i
 // grid: (N / (256 W), L, items).  Item = sum of (a - b)^2 over the `count` pairs of its row of the table [items][PARTS][count][2], plus
 // X^(N/2) times that over its second part's (null: no second part): the subtraction, the tensor square and the accumulation in one
 // pass over the inputs.
-// What bounds it: integer multiplies, about 1000 instructions a thread (45 pairs of two chunks, three limbs of 2^16 words, two pairs an item
-// 85 us: one reduction per sum and half the outputs buy what the reductions of X^(N/2) cost; 90 us with a reduction per term and a
-// pair an item.  An order of workgroups in which the items that share a ciphertext meet on one XCD: the same 85).
+// What bounds it: integer multiplies, about 1000 instructions a thread, and close behind them its traffic (45 pairs of two chunks, three
+// limbs of 2^16 words, two pairs an item: 81 us for 407 MB, 5.0 TB/s; one reduction per sum and half the outputs buy what the reductions
+// of X^(N/2) cost: 90 us with a reduction per term and a pair an item.  An order of workgroups in which the items that share a ciphertext
+// meet on one XCD: the same).
 template <int PARTS, int W>
 __global__ __launch_bounds__(kThreads) void pair_square_sum_kernel(SquareSumArgs p) {
     const uint32_t limb = blockIdx.y, word = W * (blockIdx.x * kThreads + threadIdx.x), item = blockIdx.z;
