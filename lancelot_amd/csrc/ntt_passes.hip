@@ -258,7 +258,7 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const BlocksExtra &e, bool
     a.epi_b_mask = e.u2;
 }
 
-// Operands of a fused forward epilogue at the lane's four consecutive words, and its constants
+// Operands of a fused forward epilogue at the lane's two pairs of words, and its constants
 struct EpiOperands {
     bool fma, add;
     uint64_t a[4], b[4];
@@ -272,8 +272,8 @@ __device__ __forceinline__ EpiOperands load_epilogue(const NttArgs &a, const Job
     o.add = o.fma || (a.epi_mode == NTT_EPI_SUB_MUL_ADD && ((a.epi_b_mask >> (job.poly & 31)) & 1));
     const size_t n = (size_t)1 << a.log_n, at = off + (size_t)job.limb * n;
     o.dst = a.epi_dst + (size_t)job.poly * a.epi_dst_poly_stride * n + at;
-    load4(o.a, a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + at);
-    if (o.add) load4(o.b, a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + at);
+    load_pairs(o.a, a.epi_a + (size_t)job.poly * a.epi_a_poly_stride * n + at);
+    if (o.add) load_pairs(o.b, a.epi_b + (size_t)job.poly * a.epi_b_poly_stride * n + at);
     o.w = scalar_shoup(a.w, job.limb);
     o.pro_w = Shoup{0, 0};
     if (o.fma) o.pro_w = scalar_shoup(a.pro_w, job.limb);
@@ -323,9 +323,9 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             for (int i = 0; i < 4; i++) x[i] = j.out[off + T4::word(0, lane, i)];
         } else if (a.in_galois) {
 #pragma unroll
-            for (int i = 0; i < 4; i++) x[i] = j.in[galois_index((uint32_t)off + 4 * lane + i, a.in_galois, a.log_n)];
+            for (int i = 0; i < 4; i++) x[i] = j.in[galois_index((uint32_t)off + pair_lane(lane) + pair_word(i), a.in_galois, a.log_n)];
         } else {
-            load4(x, j.in + off + 4 * lane);
+            load_pairs(x, j.in + off + pair_lane(lane));
         }
     };
     uint64_t x[4], nx[4];
@@ -337,7 +337,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
         for (int j = 0; j < 4; j++) x[j] = nx[j];
         const bool more = LOOP && b + 1 < unit.count;
         EpiOperands e;
-        if (FWD && EPI) e = load_epilogue(a, job, off + 4 * lane);
+        if (FWD && EPI) e = load_epilogue(a, job, off + pair_lane(lane));
         Job next = job;
         if (more) {
             next = decode_job<false, true>(a, unit.job(b + 1));
@@ -351,6 +351,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
                 ar.reduce(v);
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
+                turn_pairs(v);
                 if (EPI) {
                     // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
                     const double ew = fp_from_u64(e.w.w);
@@ -371,10 +372,11 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 }
 #pragma unroll
                 for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(v[j], m));
-                store4(EPI ? e.dst : job.out + off + 4 * lane, x);
+                store_pairs(EPI ? e.dst : job.out + off + pair_lane(lane), x);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(x[j]);
+                turn_pairs(v);
                 T4::template inverse<A>(v, tw, ar, nullptr, lane);
             }
         } else {
@@ -382,6 +384,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             for (int j = 0; j < 4; j++) v[j] = x[j];
             if (FWD) {
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
+                turn_pairs(v);
 #pragma unroll
                 for (int j = 0; j < 4; j++) x[j] = reduce_6q(v[j], q);
                 if (EPI) {
@@ -399,8 +402,9 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                         }
                     }
                 }
-                store4(EPI ? e.dst : job.out + off + 4 * lane, x);
+                store_pairs(EPI ? e.dst : job.out + off + pair_lane(lane), x);
             } else {
+                turn_pairs(v);
                 T4::template inverse<A>(v, tw, ar, nullptr, lane);
             }
         }
@@ -509,7 +513,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
                                             uint64_t *sums_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
-    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     const uint32_t own = t < L ? t / (LK - L) : 0xffffffffu;
     const uint64_t *lazy = a.out + (size_t)t * n + off;   // words left by the rows pass, digit 0
     if (item) lazy += item * x.item_stride();
@@ -526,8 +530,8 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
     };
     auto keys = [&](uint64_t (*k)[4], uint32_t d) {
-        load4(k[0], x.evk[d] + key_off);
-        load4(k[1], x.evk[d] + key_poly + key_off);
+        load_pairs(k[0], x.evk[d] + key_off);
+        load_pairs(k[1], x.evk[d] + key_poly + key_off);
     };
     typename A::Tw tw[4];
     uint64_t nx[4];
@@ -559,12 +563,12 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
             const uint64_t *src = x.addend + (size_t)t * n;
             if (x.own_galois) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+                for (int j = 0; j < 4; j++) c0[j] = src[galois_index((uint32_t)at + pair_word(j), x.own_galois, a.log_n)];
             } else {
-                load4(c0, src + at);
+                load_pairs(c0, src + at);
             }
         }
-        if (fold) load4(cl, x.addend + item * x.fold_item_stride() + ((size_t)r * L + t) * n + at);
+        if (fold) load_pairs(cl, x.addend + item * x.fold_item_stride() + ((size_t)r * L + t) * n + at);
     };
     if constexpr (SPLIT > 1) {
         // (what the two waves that finish need after the sums have met is requested before the digits)
@@ -581,9 +585,9 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         keys(k, own);
         if (x.own_galois) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) c[j] = src[galois_index((uint32_t)at + j, x.own_galois, a.log_n)];
+            for (int j = 0; j < 4; j++) c[j] = src[galois_index((uint32_t)at + pair_word(j), x.own_galois, a.log_n)];
         } else {
-            load4(c, src + at);
+            load_pairs(c, src + at);
         }
         typename A::V v[4];
 #pragma unroll
@@ -608,6 +612,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         if (SPLIT > 1 || d < beta) fetch(nx, d < beta ? d : now);
         ar.reduce(v);
         T4::template forward<A>(v, tw, ar, nullptr, lane);
+        turn_pairs(v);
         if constexpr (!FP) {
 #pragma unroll
             for (int j = 0; j < 4; j++) v[j] = reduce_6q(v[j], ar.m.q);
@@ -626,7 +631,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
                 else
                     w[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, ar.m.q, r0, r1);
             }
-            store4(sums_lds + (2 * part + r) * 256 + 4 * lane, w);
+            store_pairs(sums_lds + (2 * part + r) * 256 + pair_lane(lane), w);
         }
         lds_barrier();
         if (part > 1) return;
@@ -639,7 +644,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         uint64_t parts[SPLIT][4];
         if constexpr (SPLIT > 1) {
 #pragma unroll
-            for (int i = 0; i < SPLIT; i++) load4(parts[i], sums_lds + (2 * i + r) * 256 + 4 * lane);
+            for (int i = 0; i < SPLIT; i++) load_pairs(parts[i], sums_lds + (2 * i + r) * 256 + pair_lane(lane));
         }
         if (SPLIT == 1) fetch_addends(r);
         if constexpr (FP) {
@@ -689,6 +694,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         }
         uint64_t *o = x.out + item * (2 * (size_t)LK * n) + (size_t)r * LK * n + (size_t)t * n;
         if (invert) {
+            turn_pairs(v);
             T4::template inverse<A>(v, SPLIT > 1 ? itw : tw, iar, nullptr, lane);
 #pragma unroll
             for (int j = 0; j < 4; j++) o[off + T4::word(0, lane, j)] = A::to_word(v[j]);
@@ -701,7 +707,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
                 else
                     res[j] = v[j];
             }
-            store4(o + at, res);
+            store_pairs(o + at, res);
         }
     }
 }
@@ -788,14 +794,14 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
                                              uint32_t lane) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
-    const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     const size_t ct = 2 * job.poly * poly + job.limb * n + at;
     uint64_t a0[4], a1[4], b0[4], b1[4];
-    load4(a0, x.ct1 + ct);
-    load4(a1, x.ct1 + ct + poly);
+    load_pairs(a0, x.ct1 + ct);
+    load_pairs(a1, x.ct1 + ct + poly);
     if (!x.square) {
-        load4(b0, x.ct2 + ct);
-        load4(b1, x.ct2 + ct + poly);
+        load_pairs(b0, x.ct2 + ct);
+        load_pairs(b1, x.ct2 + ct + poly);
     }
     typename A::Tw tw[4];
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
@@ -821,9 +827,10 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
             o2[j] = d2[j];
         }
     }
-    store4(x.d01 + ct, o0);
-    store4(x.d01 + ct + poly, o1);
-    store4(x.d2 + job.poly * poly + job.limb * n + at, o2);
+    store_pairs(x.d01 + ct, o0);
+    store_pairs(x.d01 + ct + poly, o1);
+    store_pairs(x.d2 + job.poly * poly + job.limb * n + at, o2);
+    turn_pairs(d2);
     T4::template inverse<A>(d2, tw, ar, nullptr, lane);
 #pragma unroll
     for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(d2[j]);
@@ -867,7 +874,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
                                               const A &ar, uint64_t *u_lds) {
     using T4 = Tile4<8, 8>;
     constexpr bool FP = std::is_same<A, FpArith>::value;
-    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     uint64_t *poly = a.out + ((size_t)(w == 0 ? item : items + 2 * item + w - 1) * LK + t) * n;
     const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
     uint64_t x[4], k[4], u[4];
@@ -875,16 +882,17 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
     for (int j = 0; j < 4; j++) x[j] = poly[off + T4::word(0, lane, j)];
     typename A::Tw tw[4];
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
-    if (w) load4(k, pk + ((size_t)(w - 1) * size_qp + table) * n + at);
+    if (w) load_pairs(k, pk + ((size_t)(w - 1) * size_qp + table) * n + at);
     typename A::V v[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
     ar.reduce(v);
     T4::template forward<A>(v, tw, ar, nullptr, lane);
+    turn_pairs(v);
     if (w == 0) {
 #pragma unroll
         for (int j = 0; j < 4; j++) u[j] = canonical_word(v[j], ar);
-        store4(u_lds + 4 * lane, u);
+        store_pairs(u_lds + pair_lane(lane), u);
     }
     A iar = ar;
     if (w && t >= L) {
@@ -896,7 +904,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
     }
     lds_barrier();
     if (w == 0) return;
-    load4(u, u_lds + 4 * lane);
+    load_pairs(u, u_lds + pair_lane(lane));
     uint64_t o[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) o[j] = add_product(v[j], u[j], k[j], ar, r0, r1);
@@ -908,11 +916,12 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
             else
                 v[j] = o[j];
         }
+        turn_pairs(v);
         T4::template inverse<A>(v, tw, iar, nullptr, lane);
 #pragma unroll
         for (int j = 0; j < 4; j++) poly[off + T4::word(0, lane, j)] = A::to_word(v[j]);
     } else {
-        store4(poly + at, o);
+        store_pairs(poly + at, o);
     }
 }
 
@@ -940,7 +949,7 @@ template <class A>
 __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArgs &d, const Job &job, uint32_t blk, uint32_t lane,
                                               const A &ar) {
     using T4 = Tile4<8, 8>;
-    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + 4 * lane, poly = (size_t)a.map.limbs * n;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane), poly = (size_t)a.map.limbs * n;
     const uint64_t q = scalar(a.moduli)[job.table], r0 = scalar(a.barrett)[2 * job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
     const uint64_t *ct = (a.in ? a.in : d.cts[job.poly]) + job.limb * n + at;
     const uint64_t *sk = d.sk + job.limb * n + at;
@@ -949,25 +958,26 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
     for (int j = 0; j < 4; j++) x[j] = job.out[off + T4::word(0, lane, j)];
     typename A::Tw tw[4];
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
-    load4(c0, ct);
-    load4(c1, ct + poly);
-    load4(s1, sk);
+    load_pairs(c0, ct);
+    load_pairs(c1, ct + poly);
+    load_pairs(s1, sk);
     if (d.size > 2) {
-        load4(c2, ct + 2 * poly);
-        load4(s2, sk + d.sk_stride);
+        load_pairs(c2, ct + 2 * poly);
+        load_pairs(s2, sk + d.sk_stride);
     }
     typename A::V v[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
     ar.reduce(v);
     T4::template forward<A>(v, tw, ar, nullptr, lane);
+    turn_pairs(v);
     uint64_t o[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         o[j] = add_mod(add_product(v[j], c1[j], s1[j], ar, r0, r1), c0[j], q);
         if (d.size > 2) o[j] = add_mod(o[j], mul_mod(c2[j], s2[j], q, r0, r1), q);
     }
-    store4(job.out + at, o);
+    store_pairs(job.out + at, o);
 }
 
 template <int BE>
