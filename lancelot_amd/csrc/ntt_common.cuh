@@ -580,6 +580,16 @@ __device__ __forceinline__ void load_pairs(uint64_t *v, const uint64_t *p) {
     v[3] = b.y;
 }
 
+// the same for words that are read once: they pass by without pushing others out of the caches
+__device__ __forceinline__ void stream_pairs(uint64_t *v, const uint64_t *p) {
+    const Words2 a = __builtin_nontemporal_load(reinterpret_cast<const Words2 *>(p));
+    const Words2 b = __builtin_nontemporal_load(reinterpret_cast<const Words2 *>(p + pair_word(2)));
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
 __device__ __forceinline__ void store_pairs(uint64_t *p, const uint64_t *v) {
     reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
     reinterpret_cast<Words2 *>(p + pair_word(2))[0] = Words2{v[2], v[3]};

@@ -507,7 +507,8 @@ struct InnerMany {
 // FP64 kernel from 96 registers to 120).
 // SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
 // and waves 0 and 1 finish one polynomial each.
-template <int SPLIT, class A, class X>
+// STREAM: the key words pass by the caches (launch_ntt_inner says when).
+template <int SPLIT, bool STREAM, class A, class X>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32_t L, uint32_t LK, uint32_t beta, uint32_t t,
                                             uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
                                             uint64_t *sums_lds) {
@@ -530,8 +531,13 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
     };
     auto keys = [&](uint64_t (*k)[4], uint32_t d) {
-        load_pairs(k[0], x.evk[d] + key_off);
-        load_pairs(k[1], x.evk[d] + key_poly + key_off);
+        if constexpr (STREAM) {
+            stream_pairs(k[0], x.evk[d] + key_off);
+            stream_pairs(k[1], x.evk[d] + key_poly + key_off);
+        } else {
+            load_pairs(k[0], x.evk[d] + key_off);
+            load_pairs(k[1], x.evk[d] + key_poly + key_off);
+        }
     };
     typename A::Tw tw[4];
     uint64_t nx[4];
@@ -716,7 +722,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
 constexpr int kInnerWaves = 4;
 
-template <int BE, int SPLIT, class X>
+template <int BE, int SPLIT, bool STREAM, class X>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PARAMS, X x) {
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
     NttArgs a;
@@ -752,9 +758,9 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PAR
     const uint32_t blk = pair & ((1u << lr) - 1), table = map_table(a.map, t);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
-    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, fp_arith(a, table), part, sums);
+    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, fp_arith(a, table), part, sums);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) inner_block<SPLIT>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, int_arith(a, table), part, sums);
+        if (!fp) inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, int_arith(a, table), part, sums);
     }
 }
 
@@ -1297,28 +1303,38 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     InnerFew few{a.pro_itw, addend, x.out, x.own_galois, inv_first, {x.evk.p[0], x.evk.p[1], x.evk.p[2]}};
     InnerMany many{a.pro_itw, addend, x.out, x.own_galois, inv_first, {a.item_stride, x.own_item_stride, x.fold_item_stride}, {}};
     memcpy(many.evk, x.evk.p, sizeof(many.evk));
-#define HE_INNER_BE(BE, SPLIT)                                                                                                    \
+    // Key words that pass by the caches leave them to the other operands, which the kernels around this one wrote or will read; but a
+    // key that would have stayed there for the next call comes from memory then.  So the line is where a key switch's words (key, digits,
+    // their sum, input and result) come near the 256 MiB of the last-level cache: 400 limbs of 2^16 words.  Rotations, us with keys kept /
+    // passing by (n = 2^16, L + K limbs, so many limbs in all): 16 + 4 (344) 82.6 / 83.7, 10 + 1 (392) 80.0 / 81.7, 20 + 8 (388) 104.8 /
+    // 104.9, 22 + 8 (414) 110.6 / 109.1, 18 + 4 (446) 104.7 / 103.7, 24 + 8 (448) 115.0 / 112.8, 12 + 1 (542) 105.6 / 104.9, 24 + 4 (656)
+    // 140.5 / 131.8, 14 + 1 (720) 132.7 / 125.4; 60 / 40 bits 10 + 1 87.7 / 89.7, 22 + 8 154.4 / 152.1, 24 + 4 167.8 / 161.4.  A batch's
+    // waves share their keys in a CU's cache: eight products 791 / 856.
+    const bool stream = items == 1 && (((3 * (uint64_t)x.beta + 2) * (x.L + x.K) + 4 * (uint64_t)x.L) << a.log_n) >= (uint64_t)400 << 16;
+#define HE_INNER_BE(BE, SPLIT, STREAM)                                                                                             \
     do {                                                                                                                          \
         if (items == 1 && x.beta <= InnerFew::kDigits)                                                                            \
-            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, InnerFew>), grid, block, 0, s, HE_HEAD_ARGS(head), few);               \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, InnerFew>), grid, block, 0, s, HE_HEAD_ARGS(head), few);       \
         else                                                                                                                      \
-            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, InnerMany>), grid, block, 0, s, HE_HEAD_ARGS(head), many);             \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, InnerMany>), grid, block, 0, s, HE_HEAD_ARGS(head), many);     \
     } while (0)
-#define HE_INNER(SPLIT)                                  \
-    do {                                                 \
-        if (backend == NTT_BACKEND_MIXED)                \
-            HE_INNER_BE(NTT_BACKEND_MIXED, SPLIT);       \
-        else if (backend)                                \
-            HE_INNER_BE(NTT_BACKEND_FP, SPLIT);          \
-        else                                             \
-            HE_INNER_BE(NTT_BACKEND_INT, SPLIT);         \
+#define HE_INNER(SPLIT, STREAM)                                  \
+    do {                                                         \
+        if (backend == NTT_BACKEND_MIXED)                        \
+            HE_INNER_BE(NTT_BACKEND_MIXED, SPLIT, STREAM);       \
+        else if (backend)                                        \
+            HE_INNER_BE(NTT_BACKEND_FP, SPLIT, STREAM);          \
+        else                                                     \
+            HE_INNER_BE(NTT_BACKEND_INT, SPLIT, STREAM);         \
     } while (0)
     if (split == 4)
-        HE_INNER(4);
+        HE_INNER(4, false);
     else if (split == 2)
-        HE_INNER(2);
+        HE_INNER(2, false);
+    else if (stream)
+        HE_INNER(1, true);
     else
-        HE_INNER(1);
+        HE_INNER(1, false);
 #undef HE_INNER
 #undef HE_INNER_BE
     return hipGetLastError();
