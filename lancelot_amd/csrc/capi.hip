@@ -280,6 +280,15 @@ bool fuse_rows_ok(const he_context *ctx, const Level *lv, uint32_t L) {
     return ctx->fuse_rows && !ctx->single_limb_digits && lv && lv->batched && ctx->log_n >= 12 && ctx->log_n <= 16;
 }
 
+// The inverse transform inv leaves the inputs of b tiled, `limbs` limbs a polynomial from `tiles` on, if that is the better form for both.
+void use_tiles(const he_context *ctx, NttArgs &inv, int inv_backend, BconvRows &b, uint64_t *tiles, uint32_t limbs) {
+    if (!bconv_wants_tiles(inv, inv_backend, b, ctx->tune)) return;
+    inv.tiles = tiles;
+    inv.tiles_poly_stride = limbs;
+    b.in = tiles;
+    b.tiled = 1;
+}
+
 // whether `count` limbs from `first` on are among the first `size` (a sum of the two could wrap around)
 bool in_range(uint32_t first, uint32_t count, uint32_t size) { return count <= size && first <= size - count; }
 
@@ -948,10 +957,10 @@ namespace {
 // in_galois != 0 (one item, skip_own): the input is sigma(c), X -> X^in_galois, gathered by the inverse blocks pass
 // lazy: the forward transform of the converted limbs stops after its rows pass (launch_ntt_inner goes on from there); the
 // digits' own limbs are not copied.  tin: c is the third polynomial of a tensor product that has not been formed yet; the
-// inverse blocks pass forms it (FP64 back end).
+// inverse blocks pass forms it (FP64 back end).  tiles: items * L limbs of scratch, for inputs of the fused conversion in its own order
 int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_item_stride, uint32_t items,
                uint64_t *out, uint64_t *ws, he_stream s, bool skip_own = false, uint32_t in_galois = 0, bool lazy = false,
-               const TensorFuse *tin = nullptr) {
+               const TensorFuse *tin = nullptr, uint64_t *tiles = nullptr) {
     if (!ctx || !c || !out || !ws || ctx->size_p == 0 || items == 0 || c_item_stride < L) return HE_E_INVALID_ARGUMENT;
     const Level *lv = level_of(ctx, L);
     if (!lv) return HE_E_LEVEL_NOT_SET;
@@ -980,6 +989,9 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     // ... and a small launch finishes the inverse transform there as well
     const int inv_backend = backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, lv->n_modup_jobs * items);
+    BconvRows conv{ws, out, skip_own ? nullptr : c, (size_t)c_item_stride * n, LimbMap{LK, 0, L, ctx->size_q}, ctx->size_p, lv->beta, items, 1,
+                   fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr, 0};
+    if (fused && tiles) use_tiles(ctx, inv, inv_backend, conv, tiles, L);
     if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, items, inv_backend, S(s)));
     HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), tin != nullptr, source_intt));
     const uint32_t copy_rows = skip_own ? 0 : lv->modup_max_copy;
@@ -990,9 +1002,7 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
                                     items, hipMemcpyDeviceToDevice, S(s)));
     } else if (fused) {
         const int backend = backend_for_level(ctx, L);
-        BconvRows b{ws, out, skip_own ? nullptr : c, (size_t)c_item_stride * n, LimbMap{LK, 0, L, ctx->size_q}, ctx->size_p, lv->beta, items, 1,
-                    fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr};
-        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend, ctx->tune, S(s)));
+        HE_HIP(launch_bconv_rows(base_args(ctx, true), conv, backend, ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{ws, out, c, lv->d_mats, lv->d_modup_limb, lv->d_modup_table, lv->d_modup_descs,
                      lv->beta, lv->modup_max_rows, copy_rows, lv->d_mats_fp, ctx->d_fp_consts,
@@ -1067,9 +1077,10 @@ namespace {
 // add_mask: which polynomials of `out` are added onto (bit p set) instead of overwritten
 // (addend: where the words to add come from, limb stride addend_stride between polynomials; nullptr: out itself)
 // inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
-// deal: see NttArgs
+// deal: see NttArgs; scratch: as many limbs that nothing else needs (inputs of the fused conversion in its own order)
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
-                 uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0) {
+                 uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0,
+                 uint64_t *scratch = nullptr, size_t scratch_limbs = 0) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     const int accumulate = add_mask != 0;
     const size_t n = ctx->n();
@@ -1092,14 +1103,15 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     // ... and a small launch finishes the special limb's inverse transform there as well
     const int inv_backend = inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, n_polys * L);
+    const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
+    BconvRows conv{cx, ws, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, units, items, 0,
+                   fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr, 0};
+    if (fused && (size_t)n_polys * K <= scratch_limbs) use_tiles(ctx, inv, inv_backend, conv, scratch, K);
     HE_HIP(launch_ntt_inverse(inv, n_polys, inv_backend, S(s), inverted, source_intt));
     if (reduce_in_ntt) {
     } else if (batched) {
-        const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
         if (fused) {
-            BconvRows b{cx, ws, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, units, items, 0,
-                        fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr};
-            HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L, 0)), ctx->tune, S(s)));
+            HE_HIP(launch_bconv_rows(base_args(ctx, true), conv, backend_for(ctx, plain_map(L, 0)), ctx->tune, S(s)));
         } else {
             BconvBatch b{cx, ws, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, units, L, 0,
                          fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_fp_consts,
@@ -1178,6 +1190,9 @@ KsWorkspace ks_workspace(const he_context *ctx, const Level *lv, uint32_t L, uin
     return w;
 }
 
+// what is free of y once the inner product has read it
+size_t digit_limbs(const he_context *ctx, const Level *lv, uint32_t L, uint32_t items) { return (size_t)items * lv->beta * (L + ctx->size_p); }
+
 // ModUp and inner product of a key switch over `items` inputs (item k at c + k * c_item_stride * N): ws -> cx.
 // fold_ct != nullptr: limb L-1 of cx becomes cx * P^-1 + fold_ct (see KsFuseArgs); fold_ct holds [items][2][L][N].
 // add_c0 != nullptr (a rotation, items = 1): polynomial 0 of cx gains P sigma(add_c0) on its data limbs, sigma =
@@ -1211,7 +1226,7 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         // fused with the inner product: the transformed digits are never written (216 limb transfers less at L = 24, K = 8)
         for (uint32_t d = 0; d < lv->beta; d++)
             if (!evk[d]) return HE_E_INVALID_ARGUMENT;
-        if (int rc = modup_impl(ctx, L, src, items == 1 ? L : c_item_stride, items, y, tmp, s, true, galois_elt, true, tin)) return rc;
+        if (int rc = modup_impl(ctx, L, src, items == 1 ? L : c_item_stride, items, y, tmp, s, true, galois_elt, true, tin, tmp + (size_t)items * L * n)) return rc;
         NttArgs fwd = base_args(ctx, true);
         fwd.out = y;
         fwd.item_stride = (size_t)lv->beta * (L + ctx->size_p) * n;
@@ -1247,7 +1262,8 @@ int ks_accumulate(const he_context *ctx, const Level *lv, uint32_t L, const uint
         // (batched levels: neither kernel needs the copy of a digit's own limbs into y)
         const bool skip_own = fp_batch || lv->batched;
         const uint32_t src_stride = (galois_elt && !gather) ? L : c_item_stride;
-        if (int rc = modup_impl(ctx, L, src, src_stride, items, y, tmp, s, skip_own, gather ? galois_elt : 0)) return rc;
+        if (int rc = modup_impl(ctx, L, src, src_stride, items, y, tmp, s, skip_own, gather ? galois_elt : 0, false, nullptr,
+                                src == c ? tmp + (size_t)items * L * n : nullptr)) return rc;
         EvkPtrs ptrs;
         memset(&ptrs, 0, sizeof(ptrs));
         for (uint32_t d = 0; d < lv->beta; d++) {
@@ -1279,7 +1295,7 @@ int he_keyswitch(const he_context *ctx, uint32_t L, const uint64_t *c, const uin
     const KsWorkspace w = ks_workspace(ctx, lv, L, 1, ws);
     bool inverted = false;
     if (int rc = ks_accumulate(ctx, lv, L, c, L, 1, evk, galois_elt, nullptr, ws, s, &inverted)) return rc;
-    return moddown_impl(ctx, L, w.cx, ct, 2, 0xffffffffu, w.tmp, s, NTT_DEAL_ALWAYS, inverted);
+    return moddown_impl(ctx, L, w.cx, ct, 2, 0xffffffffu, w.tmp, s, NTT_DEAL_ALWAYS, inverted, nullptr, 0, w.y, digit_limbs(ctx, lv, L, 1));
 }
 
 int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const uint64_t *const *evk, uint64_t *ct_out,
@@ -1295,7 +1311,7 @@ int he_rotate(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const ui
     bool inverted = false;
     if (int rc = ks_accumulate(ctx, lv, L, ct_in + (size_t)L * n, L, 1, evk, galois_elt, nullptr, ws, s, &inverted, ct_in)) return rc;
     // out0 = sigma(c0) + ks0 (the inner product carries P sigma(c0)), out1 = ks1
-    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s, NTT_DEAL_ALWAYS, inverted);
+    return moddown_impl(ctx, L, w.cx, ct_out, 2, 0u, w.tmp, s, NTT_DEAL_ALWAYS, inverted, nullptr, 0, w.y, digit_limbs(ctx, lv, L, 1));
 }
 
 int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *ct_in,
@@ -1316,7 +1332,8 @@ int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items
     const KsWorkspace w = ks_workspace(ctx, lv, L, items, ws);
     // (the digits' own limbs are not copied into y: the kernel reads them from c1 where they are)
     const bool skip_own = lv->batched;
-    if (int rc = modup_impl(ctx, L, ct_in + (size_t)L * n, 2 * L, items, w.y, w.tmp, s, skip_own)) return rc;
+    if (int rc = modup_impl(ctx, L, ct_in + (size_t)L * n, 2 * L, items, w.y, w.tmp, s, skip_own, 0, false, nullptr,
+                            w.tmp + (size_t)items * L * n)) return rc;
     // as many steps per launch as the 128-bit accumulator and the pointer table allow
     const uint32_t per_launch = (uint32_t)kMaxDigits / lv->beta;
     for (uint32_t first = 0; first < n_steps; first += per_launch) {
@@ -1326,7 +1343,8 @@ int he_hoisted_rotations_batch(const he_context *ctx, uint32_t L, uint32_t items
                                   2 * (size_t)L * n, S(s), ctx->use_fp ? ctx->d_fp_consts : nullptr, ctx->fp_mask, skip_own));
     }
     // out0 = [c0 +] sum sigma(c0) + ModDown(cx0), out1 = [c1 +] ModDown(cx1)
-    return moddown_impl(ctx, L, w.cx, ct_out, 2 * items, add_input ? 0xffffffffu : 0x55555555u, w.tmp, s, NTT_DEAL_LONG);
+    return moddown_impl(ctx, L, w.cx, ct_out, 2 * items, add_input ? 0xffffffffu : 0x55555555u, w.tmp, s, NTT_DEAL_LONG, false, nullptr, 0,
+                        w.y, digit_limbs(ctx, lv, L, items));
 }
 
 int he_hoisted_rotations(const he_context *ctx, uint32_t L, const uint64_t *ct_in, const uint64_t *const *evk,
@@ -1374,20 +1392,20 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     inv.w = lv->d_mdr_w;
     const int inv_backend = inverted ? backend_for_level(ctx, L) : backend_for(ctx, inv.map);
     const bool source_intt = ctx->single_limb_digits && !ctx->tune.no_source_intt && ntt_two_sources_ok(ctx->log_n, polys * (L - 1), ctx->size_qp);
-    HE_HIP(launch_ntt_inverse(inv, polys, inv_backend, S(s), inverted, source_intt));
     // (3) delta = P -> Ql conversion of the special limbs
     const bool fused = fuse_rows_ok(ctx, lv, L);
+    BconvRows conv{cx, delta, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, 2, items, 0,
+                   fp_for_level(ctx, L) ? ctx->d_phat_pinv_fp : nullptr, 1, ctx->d_mx_down,
+                   ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q, 0};
+    if (fused && (size_t)polys * (K + 1) <= digit_limbs(ctx, lv, L, items)) use_tiles(ctx, inv, inv_backend, conv, w.y, K + 1);
+    HE_HIP(launch_ntt_inverse(inv, polys, inv_backend, S(s), inverted, source_intt));
     // one special prime: the conversion is the reduction of its coefficients modulo every q_j, which the prologue of (4)
     // does where it reads them (no conversion kernel, no delta in memory before the transform)
     const bool k1 = ctx->single_limb_digits && !fused;
     if (k1) {
     } else if (fused) {
         // with the prologue of (4) and the rows pass of its transform
-        const bool fp = fp_for_level(ctx, L);
-        BconvRows b{cx, delta, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, 2, items, 0,
-                    fp ? ctx->d_phat_pinv_fp : nullptr, 1, ctx->d_mx_down,
-                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q};
-        HE_HIP(launch_bconv_rows(base_args(ctx, true), b, backend_for(ctx, plain_map(L - 1, 0), (int)L - 1), ctx->tune, S(s)));
+        HE_HIP(launch_bconv_rows(base_args(ctx, true), conv, backend_for(ctx, plain_map(L - 1, 0), (int)L - 1), ctx->tune, S(s)));
     } else if (lv->batched) {
         BconvBatch b{cx, delta, nullptr, ctx->d_phat_mod_q, ctx->d_iota, ctx->d_iota, lv->d_moddown_descs, 2, L, 0,
                      fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, ctx->d_fp_consts,
@@ -1613,7 +1631,7 @@ int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64
     HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
     // divide by P onto the plaintexts
     return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
-                        plain ? L : 0);
+                        plain ? L : 0, u, (size_t)items * LK);
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts

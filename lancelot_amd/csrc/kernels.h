@@ -149,6 +149,9 @@ struct NttArgs {
     const uint64_t *epi_b;
     uint32_t epi_b_poly_stride;
     uint32_t epi_b_mask;      // NTT_EPI_SUB_MUL_ADD: bit (poly mod 32) set = that polynomial has an addend
+    uint64_t *tiles;          // inverse transform, rows pass, N = 2^16: the coefficients leave in the order in which a fused base conversion
+                              // reads them (conversion_word), on the FP64 back end as doubles, limb (poly, i) at tiles + (poly * tiles_poly_stride + i) * N
+    uint32_t tiles_poly_stride;
     uint32_t in_galois;       // inverse transform, map mode: the input is sigma(in), gathered by the blocks pass
     const uint64_t *pro_w;    // [limbs][2] Shoup constants of the scaling prologue / epilogue, indexed like w
     const uint64_t *pro_src2; // NTT_PRO_MODDOWN_RESCALE: second source, limb (poly) at pro_src2 + poly * pro2_poly_stride * N
@@ -340,6 +343,9 @@ struct BconvRows {
     // levels with a prime from 2^50 on (mat_fp == nullptr): the matrix in integers, and, mdr, P^-1 mod q_j (Shoup pairs)
     const uint64_t *mat;
     const uint64_t *w;
+    // N = 2^16: the input limbs are in the order of conversion_word, as doubles with mat_fp (not for the matrix kernel); ModDown: in [items][units]
+    // [K][N], mdr: [K + 1][N] with t's limb in front
+    int tiled;
 };
 // What its kernels take: NttHead with in and out, h1 = units | K << 16, h2 = workgroups of a tile that compute | that copy << 16,
 // h5 = rows of one, and pro_mode 1 for ModUp; behind it
@@ -352,6 +358,9 @@ struct BconvExtra {
 constexpr uint32_t kMxRecord = 144;
 // `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
 // and `backend` says what the blocks pass that follows runs on
+// whether `inv`, the inverse transform that ends in b's inputs, should leave them tiled (in a buffer of their own: its last pass is in
+// place otherwise)
+bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune);
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s);
 hipError_t launch_bconv_rows4(const NttHead &h, const BconvRows &b, hipStream_t s);
 

@@ -587,6 +587,26 @@ void bconv_rows_mx_kernel(HE_HEAD_PARAMS, BconvExtra b) {
 
 }  // namespace
 
+// The matrix-core kernel (N = 2^16) multiplies 8 input limbs deep whatever there are, takes the output rows four at a time and two
+// workgroups to a CU: it pays from five limbs on, and once the tiles alone give every CU a workgroup.  us with it / without, all of
+// a multiplication: K = 8, L = 24: one 140.0 / 139.0, two 241.5 / 241.4, three 338.8 / 340.6, four 422 / 436, eight 805 / 840;
+// K = 6, L = 30: one 203.0 / 201.2; K = 4, L = 12: one 80.8 / 74.4, two 129.7 / 124.4, eight 410 / 403.  (Merged ModDown +
+// rescale, K = 8: eight 106 / 122 us.)
+static bool bconv_on_matrix_cores(uint32_t log_n, const BconvRows &b, const Tuning &tune) {
+    return log_n == 16 && b.mat_fp && b.mx_tab && !b.tiled && !tune.no_matrix_bconv && b.K > 4 && (!b.mdr || b.mx_last) &&
+           ((uint64_t)b.units * (b.items ? b.items : 1) << (log_n - kFuseLog)) >= (tune.cus ? tune.cus : 256);
+}
+
+// Tiled inputs (conversion_word): what a workgroup of the vector kernel fetches first, 64 KB to 144 KB, lay in segments of 64 bytes at N = 2^16,
+// which took 10 us of a launch's 28 with all workgroups at it.  The rows pass before it needs a buffer to leave them in, whose lines no cache
+// holds yet; that costs what is gained while there are few limbs.  us natural / tiled, n = 2^16, L + K limbs: rotation 24 + 8 113.1 / 108.8, 16 + 8
+// 78.4 / 75.1, 8 + 8 50.9 / 49.1, 10 + 3 65.7 / 64.7, 16 + 2 107 / 105; product 24 + 8 136.9 / 132.1, 16 + 8 94.6 / 90.5, 8 + 2 59.8 / 58.3, 4 + 2
+// 39.7 / 40.5; hoisting 24 + 8 238.6 / 235.6, 4 + 2 49.3 / 51.0; 60 / 40 bits: rotation 24 + 8 157.3 / 153.2, 8 + 2 65.2 / 63.3, 4 + 2 42.6 /
+// 42.8, product 24 + 8 189 / 187, 4 + 2 50.5 / 51.6.  At 2^15 the segments are whole lines already: rotation 24 + 8 68.0 / 67.3, 10 + 3 43.7 / 44.6.
+bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune) {
+    return inv.log_n == 16 && b.map.limbs >= 10 && !bconv_on_matrix_cores(inv.log_n, b, tune) && (b.mat_fp != nullptr) == (inv_backend == NTT_BACKEND_FP);
+}
+
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s) {
     if (a.log_n < 12 || a.log_n > 16 || b.units == 0 || b.K == 0 || b.K > 8) return hipErrorInvalidValue;
     const uint32_t forced = tune.fuse_rows_forced <= kFuseMaxRows ? tune.fuse_rows_forced : 0;
@@ -597,14 +617,8 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     const uint32_t L = b.map.split, last = L % b.K ? L % b.K : b.K;
     const uint32_t rows = b.up ? b.map.limbs - last : b.mdr ? L - 1 : L;
     if (rows == 0) return hipErrorInvalidValue;
-    // The matrix-core kernel (N = 2^16) multiplies 8 input limbs deep whatever there are, takes the output rows four at a time and two
-    // workgroups to a CU: it pays from five limbs on, and once the tiles alone give every CU a workgroup.  us with it / without, all of
-    // a multiplication: K = 8, L = 24: one 140.0 / 139.0, two 241.5 / 241.4, three 338.8 / 340.6, four 422 / 436, eight 805 / 840;
-    // K = 6, L = 30: one 203.0 / 201.2; K = 4, L = 12: one 80.8 / 74.4, two 129.7 / 124.4, eight 410 / 403.  (Merged ModDown +
-    // rescale, K = 8: eight 106 / 122 us.)
     const uint32_t cus = tune.cus ? tune.cus : 256;
-    const bool mx = ld == 8 && b.mat_fp && b.mx_tab && !tune.no_matrix_bconv && b.K > 4 && (!b.mdr || b.mx_last) &&
-                    (uint64_t)b.units * items * tiles >= cus;
+    const bool mx = bconv_on_matrix_cores(a.log_n, b, tune);
     // Output limbs per workgroup.  The kernel is bound by instruction issue, so a CU's time is the number of workgroups it is dealt
     // times a workgroup's work: r rows plus the fetching of the inputs and setting up, one row's worth and a half with 4 waves and a
     // tile of 8 words per thread, half a row's with 8 waves and 4 words.  Few rows per workgroup pay that often, many leave
@@ -671,6 +685,10 @@ hipError_t launch_ntt_inverse(const NttArgs &a, uint32_t n_polys, int backend, h
     NttArgs rows = a;
     rows.in = a.out;  // the rows pass continues in place on the output buffer
     rows.in_poly_stride = a.out_poly_stride;
+    if (a.tiles) {
+        rows.out = a.tiles;
+        rows.out_poly_stride = a.tiles_poly_stride;
+    }
     return launch_ntt_rows(rows, n_jobs, false, backend, s);
 }
 

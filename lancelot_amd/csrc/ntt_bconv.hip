@@ -35,16 +35,18 @@ namespace {
 constexpr int kTileLog = 11;
 
 // Conversion in FP64 (every prime of the level below 2^50)
-template <int NIN, bool MDR>
+template <int NIN, bool MDR, bool TILED>
 struct ConvFp {
     double x[NIN][4], rr[MDR ? 4 : 1];
-    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = fp_from_u64(w); }
+    // (tiled words are doubles)
+    static __device__ __forceinline__ double value(uint64_t w) { return TILED ? FpArith::from_word(w) : fp_from_u64(w); }
+    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = value(w); }
     __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
         const uint32_t last = d.n_out - 1;
         const FpMod m = fp_ctx(a, map_table(a.map, last)).m;
         const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + d.mat_off + (size_t)last * d.n_in;
 #pragma unroll
-        for (int j = 0; j < 4; j++) rr[j] = fp_from_u64(t[j]);
+        for (int j = 0; j < 4; j++) rr[j] = value(t[j]);
 #pragma unroll
         for (int k = 0; k < NIN; k++) {
             if ((uint32_t)k >= d.n_in) break;
@@ -153,7 +155,8 @@ struct ConvInt {
 
 // FP: the whole level is below 2^50; otherwise the conversion is done in integers and bit `table` of a.fp_mask says in which
 // arithmetic the limb is transformed
-template <int LD, bool FP, int NIN, bool MDR>
+// TILED: the input limbs are in the order of conversion_word (BconvRows::tiled)
+template <int LD, bool FP, int NIN, bool MDR, bool TILED>
 __global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(FP || NIN <= 4 ? 4 : 2)))
 void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     using T4 = Tile4<kTileLog, LD>;
@@ -168,7 +171,8 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     const uint32_t compute_groups = h2 & 0xffff, groups = compute_groups + (h2 >> 16), grp = lb % groups, rows_per = h5;
     lb /= groups;
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
-    const BconvUnit d = bconv_unit(a, h1 & 0xffff, h1 >> 16, lb / tiles_per_limb);
+    const uint32_t K = h1 >> 16;
+    const BconvUnit d = bconv_unit(a, h1 & 0xffff, K, lb / tiles_per_limb, TILED ? K + (MDR ? 1 : 0) : 0);
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
     // word j of layout k: a scalar distance from the lane's first one
     auto first = [&](int k) {
@@ -197,19 +201,26 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     const uint32_t n_rows = MDR ? d.n_out - 1 : d.n_out, r_begin = grp * rows_per;
     const uint32_t r_end = r_begin + rows_per < n_rows ? r_begin + rows_per : n_rows;
     if (r_begin >= n_rows) return;
-    typename std::conditional<FP, ConvFp<NIN, MDR>, ConvInt<NIN, MDR>>::type conv;
+    typename std::conditional<FP, ConvFp<NIN, MDR, TILED>, ConvInt<NIN, MDR>>::type conv;
     const uint64_t *x = d.in;
     {
         uint64_t w[NIN][4], tw[4];
+        if constexpr (TILED) {
+            const uint32_t at = conversion_word<kTileLog, LD>(col0 >> LOGC, t);
 #pragma unroll
-        for (int k = 0; k < NIN; k++) {
-            const uint32_t kk = (uint32_t)k < d.n_in ? (uint32_t)k : d.n_in - 1;
+            for (int k = 0; k < NIN; k++) load_tiled(w[k], x + ((size_t)((uint32_t)k < d.n_in ? (uint32_t)k : d.n_in - 1) << a.log_n) + at);
+            if constexpr (MDR) load_tiled(tw, x - n + at);
+        } else {
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[k][j] = (x + ((size_t)kk << a.log_n) + step(0, j))[in0];
-        }
-        if constexpr (MDR) {
+            for (int k = 0; k < NIN; k++) {
+                const uint32_t kk = (uint32_t)k < d.n_in ? (uint32_t)k : d.n_in - 1;
 #pragma unroll
-            for (int j = 0; j < 4; j++) tw[j] = (x - n + step(0, j))[in0];
+                for (int j = 0; j < 4; j++) w[k][j] = (x + ((size_t)kk << a.log_n) + step(0, j))[in0];
+            }
+            if constexpr (MDR) {
+#pragma unroll
+                for (int j = 0; j < 4; j++) tw[j] = (x - n + step(0, j))[in0];
+            }
         }
 #pragma unroll
         for (int k = 0; k < NIN; k++)
@@ -241,17 +252,24 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     }
 }
 
-template <bool FP, int NIN, bool MDR>
+template <bool FP, int NIN, bool MDR, bool TILED>
 hipError_t launch_nin(const NttHead &h, uint32_t log_n, const BconvExtra &b, hipStream_t s) {
-    switch (log_n - 8) {
 #define HE_CASE(LD)                                                                                                              \
     case LD:                                                                                                                     \
-        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR>), dim3(h.h4), dim3(1 << (kTileLog - 2)), 0, s, HE_HEAD_ARGS(h), b); \
+        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR, TILED>), dim3(h.h4), dim3(1 << (kTileLog - 2)), 0, s, HE_HEAD_ARGS(h), b); \
         break;
-        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
-#undef HE_CASE
-        default: return hipErrorInvalidValue;
+    if constexpr (TILED) {
+        switch (log_n - 8) {
+            HE_CASE(8)
+            default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (log_n - 8) {
+            HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+            default: return hipErrorInvalidValue;
+        }
     }
+#undef HE_CASE
     return hipGetLastError();
 }
 
@@ -265,10 +283,12 @@ hipError_t launch_bconv_rows4(const NttHead &head, const BconvRows &b, hipStream
         return hipErrorInvalidValue;
     h.h4 = (uint32_t)wgs;
     const BconvExtra x{b.mat_fp ? static_cast<const void *>(b.mat_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride};
-#define HE_NIN(FP, MDR) (b.K <= 4 ? launch_nin<FP, 4, MDR>(h, log_n, x, s) : launch_nin<FP, 8, MDR>(h, log_n, x, s))
+#define HE_TILED(FP, NIN, MDR) (b.tiled ? launch_nin<FP, NIN, MDR, true>(h, log_n, x, s) : launch_nin<FP, NIN, MDR, false>(h, log_n, x, s))
+#define HE_NIN(FP, MDR) (b.K <= 4 ? HE_TILED(FP, 4, MDR) : HE_TILED(FP, 8, MDR))
     if (b.mat_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
     return b.mdr ? HE_NIN(false, true) : HE_NIN(false, false);
 #undef HE_NIN
+#undef HE_TILED
 }
 
 }  // namespace he

@@ -101,7 +101,8 @@ struct BconvUnit {
     __device__ __forceinline__ uint32_t limb(uint32_t row) const { return up && row >= copy_first ? row + n_in : row; }
 };
 
-__device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units, uint32_t K, uint32_t index) {
+// packed: limbs of a ModDown polynomial where its inputs are tiled (BconvRows::tiled), 0: they are part of the sum's L + K
+__device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units, uint32_t K, uint32_t index, uint32_t packed = 0) {
     const uint32_t L = a.map.split, LK = a.map.limbs;
     BconvUnit u;
     u.up = a.pro_mode;
@@ -120,7 +121,7 @@ __device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units
         u.in = a.in + (((size_t)u.item * L + u.copy_first) << a.log_n);
         u.out = a.out + ((size_t)index * LK << a.log_n);
     } else {
-        u.in = a.in + (((size_t)index * LK + L) << a.log_n);
+        u.in = a.in + ((packed ? (size_t)index * packed + (packed - K) : (size_t)index * LK + L) << a.log_n);
         u.out = a.out + ((size_t)index * L << a.log_n);
     }
     return u;
@@ -536,6 +537,23 @@ struct Tile4 {
     }
 };
 
+// Where the words of thread t of a tile of 2^B words lie in a limb between the inverse rows pass and a fused base conversion (a rows
+// pass ends, and the conversion begins, with the words t + j 2^(B - 2) of the tile in thread t): words j = 0, 1 from here on, words 2, 3
+// from 512 words further on.  Half a tile of 2048 words (a tile of 1024) lies together, so that every access is one of 16 bytes a lane
+// over whole lines, and a workgroup's accesses go to all channels of its L2.  (As [row][column] a tile of 2048 words at N = 2^16 is 256
+// segments of 64 bytes, 2 KiB apart: a quarter of the channels.)
+template <int B, int LD>
+__device__ __forceinline__ uint32_t conversion_word(uint32_t tile, uint32_t t) {
+    if constexpr (B == 10) {
+        return (tile << 10) + 2 * t;
+    } else {
+        static_assert(B == 11, "tiles of the passes from 2^12 words on");
+        constexpr int LOGH = 10 - LD;   // columns of half a tile, log2
+        const uint32_t u = ((t >> (LOGH + 1)) << LOGH) | (t & ((1u << LOGH) - 1));
+        return (tile << 11) + ((t >> LOGH & 1) << 10) + 2 * u;
+    }
+}
+
 __device__ __forceinline__ IntArith int_arith(const NttArgs &a, uint32_t table) {
     const IntCtx c = int_ctx(a, table);
     return IntArith{int_mod(c.q), c.tw};
@@ -561,6 +579,19 @@ __device__ __forceinline__ void load4(uint64_t *v, const uint64_t *p) {
 __device__ __forceinline__ void store4(uint64_t *p, const uint64_t *v) {
     reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
     reinterpret_cast<Words2 *>(p)[1] = Words2{v[2], v[3]};
+}
+
+__device__ __forceinline__ void load_tiled(uint64_t *v, const uint64_t *p) {
+    const Words2 a = reinterpret_cast<const Words2 *>(p)[0], b = reinterpret_cast<const Words2 *>(p + 512)[0];
+    v[0] = a.x;
+    v[1] = a.y;
+    v[2] = b.x;
+    v[3] = b.y;
+}
+
+__device__ __forceinline__ void store_tiled(uint64_t *p, const uint64_t *v) {
+    reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
+    reinterpret_cast<Words2 *>(p + 512)[0] = Words2{v[2], v[3]};
 }
 
 // A wave's block of 256 words in memory: a lane's words are not the four neighbours 4 lane .. 4 lane + 3 of the last register block

@@ -124,7 +124,8 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
 // coefficients where the forward pass takes them from.  With MDR (one special prime) those of the dropped limb and of the special
 // one behind it, which every output limb's workgroup transforms anew: a launch less, and CUs that were idle (see ntt_two_sources_ok).
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
-template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B>
+// TILES (inverse): the coefficients leave where a fused conversion looks for them (conversion_word), on the FP64 back end as doubles.
+template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B, bool TILES>
 __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, RowsExtra x) {
     NttArgs a;
     using T4 = Tile4<B, LD>;
@@ -155,6 +156,15 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
         source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t);
         if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t);
     };
+    // the last words of an inverse pass: to their places in the limb, or where a conversion looks for them
+    auto leave = [&](const uint64_t *w) {
+        if constexpr (TILES) {
+            store_tiled(job.out + conversion_word<B, LD>(lb % tiles_per_limb, t), w);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 4; j++) job.out[glob(0, j)] = w[j];
+        }
+    };
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
     if (BE != NTT_BACKEND_INT && fp) {
         const FpCtx c = fp_ctx(a, job.table);
@@ -183,7 +193,11 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             ar.reduce(v);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
 #pragma unroll
-            for (int j = 0; j < 4; j++) job.out[glob(0, j)] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, c.m), c.m));
+            for (int j = 0; j < 4; j++) v[j] = fp_canonical(fp_mulmod(v[j], scale, c.m), c.m);
+            uint64_t w[4];
+#pragma unroll
+            for (int j = 0; j < 4; j++) w[j] = TILES && BE == NTT_BACKEND_FP ? FpArith::to_word(v[j]) : fp_to_u64(v[j]);
+            leave(w);
         }
         return;
     }
@@ -215,11 +229,12 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             T4::template inverse<IntArith>(v, tw, ar, lds, t);
             if (a.epi_mode == NTT_EPI_MUL) {
 #pragma unroll
-                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = mul_shoup(v[j], w, q);
+                for (int j = 0; j < 4; j++) v[j] = mul_shoup(v[j], w, q);
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; j++) job.out[glob(0, j)] = reduce_3q(v[j], q);
+                for (int j = 0; j < 4; j++) v[j] = reduce_3q(v[j], q);
             }
+            leave(v);
         }
     }
 }
@@ -1102,7 +1117,7 @@ bool spread_epilogue(const NttArgs &a, int backend, uint32_t limbs, uint32_t pol
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
-template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false>
+template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false, bool TILES = false>
 hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
     const uint32_t ld = a.log_n - 8;
     const bool large = ((uint64_t)n_jobs << a.log_n) >= ((uint64_t)32 << 16);
@@ -1110,14 +1125,14 @@ hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
     // (from 2^34 words on, 137 GB, one launch does not hold the threads)
     const uint32_t per_launch = most_workgroups(1u << (b - 2)) >> (a.log_n - b);
     while (n_jobs > per_launch) {
-        if (hipError_t e = launch_rows<FWD, BE, SRC_INTT, MDR>(a, per_launch, s)) return e;
+        if (hipError_t e = launch_rows<FWD, BE, SRC_INTT, MDR, TILES>(a, per_launch, s)) return e;
         a.first_job += per_launch;
         n_jobs -= per_launch;
     }
     const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
     const NttHead head = ntt_head(a, grid.x, a.first_job);
     const RowsExtra extra = rows_extra(a, FWD);
-#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B>), grid, block, 0, s, HE_HEAD_ARGS(head), extra)
+#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B, TILES>), grid, block, 0, s, HE_HEAD_ARGS(head), extra)
 #define HE_CASE(LD)         \
     case LD:                \
         if (large)          \
@@ -1125,7 +1140,7 @@ hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
         else                \
             HE_ROWS(LD, 10); \
         break;
-    if constexpr (!SRC_INTT) {
+    if constexpr (!SRC_INTT && !TILES) {
         switch (ld) {
             case 1: HE_ROWS(1, 8); return hipGetLastError();
             case 2: HE_ROWS(2, 8); return hipGetLastError();
@@ -1134,9 +1149,16 @@ hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
             default: break;
         }
     }
-    switch (ld) {
-        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
-        default: return hipErrorInvalidValue;
+    if constexpr (TILES) {
+        switch (ld) {
+            HE_CASE(8)
+            default: return hipErrorInvalidValue;
+        }
+    } else {
+        switch (ld) {
+            HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+            default: return hipErrorInvalidValue;
+        }
     }
 #undef HE_CASE
 #undef HE_ROWS
@@ -1187,6 +1209,10 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
         return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED>(a, n_jobs, s)
                : backend                    ? launch_rows<true, NTT_BACKEND_FP>(a, n_jobs, s)
                                             : launch_rows<true, NTT_BACKEND_INT>(a, n_jobs, s);
+    if (a.tiles)
+        return backend == NTT_BACKEND_MIXED ? launch_rows<false, NTT_BACKEND_MIXED, false, false, true>(a, n_jobs, s)
+               : backend                    ? launch_rows<false, NTT_BACKEND_FP, false, false, true>(a, n_jobs, s)
+                                            : launch_rows<false, NTT_BACKEND_INT, false, false, true>(a, n_jobs, s);
     return backend == NTT_BACKEND_MIXED ? launch_rows<false, NTT_BACKEND_MIXED>(a, n_jobs, s)
            : backend                    ? launch_rows<false, NTT_BACKEND_FP>(a, n_jobs, s)
                                         : launch_rows<false, NTT_BACKEND_INT>(a, n_jobs, s);
