@@ -43,6 +43,7 @@ struct Level {
     uint32_t modup_max_rows = 0, modup_max_copy = 0;
     bool batched = false;
     double *d_mats_fp = nullptr;         // the digit matrices as doubles, when every prime is below 2^50
+    double *d_rows_up = nullptr;         // ... and as the fused kernel reads them (BconvRows::rows_fp)
     int32_t *d_mx_up = nullptr;          // the same matrices as 7-bit digits for the int8 matrix cores (N = 2^16)
 };
 
@@ -91,7 +92,8 @@ struct he_context {
     std::vector<uint64_t> h_phat_inv;    // host copy of d_phat_inv
     double *d_psi_fp = nullptr, *d_ipsi_fp = nullptr, *d_fp_consts = nullptr;  // FP64 back end tables
     double *d_phat_mod_q_fp = nullptr;   // the P -> Ql matrix as doubles
-    double *d_phat_pinv_fp = nullptr;    // the same matrix times P^-1 mod q_j (merged ModDown + rescale, fused kernel)
+    double *d_rows_down = nullptr, *d_rows_mdr = nullptr;   // ... as the fused kernel reads it (BconvRows::rows_fp), and times P^-1 mod q_j (merged
+                                                            // ModDown + rescale)
     bool fuse_rows = true;       // environment CAHEL_HIP_NO_FUSED_BCONV=1: conversion kernel, then the rows pass
     bool fuse_tensor = true;     // environment CAHEL_HIP_NO_FUSED_TENSOR=1: he_multiply_relin_rescale as tensor kernel + key switch
     bool single_limb_digits = false;  // K = 1 (environment CAHEL_HIP_NO_REDUCE_IN_NTT=1: keep the conversion kernels)
@@ -123,6 +125,22 @@ namespace {
         hipError_t _e = (expr);               \
         if (_e != hipSuccess) return (int)_e; \
     } while (0)
+
+// the representative of w in (-q/2, q/2): what multiplies a value v is half as large that way, and the quotient of the modular product off
+// by at most 0.19 |v| 2^-50 instead of 0.38
+double centred(uint64_t w, uint64_t q) { return w > q / 2 ? -(double)(q - w) : (double)w; }
+
+// One row of BconvRows::rows_fp
+template <class Entry>
+void conversion_row(std::vector<double> &rows, uint32_t n_in, uint64_t q, Entry entry) {
+    uint64_t shift = 0;
+    for (uint32_t i = 0; i < 8; i++) {
+        rows.push_back(i < n_in ? centred(entry(i), q) : 0.0);
+        if (i < n_in) shift = (uint64_t)((shift + ((unsigned __int128)entry(i) << 49)) % q);
+    }
+    rows.push_back(centred(shift, q));
+    rows.push_back(centred((uint64_t)((1ull << 50) % q), q) * 0x1p-50);
+}
 
 // One record of BconvRows::mx_tab: up to four rows of a conversion matrix with at most 8 columns as 7-bit digits of
 // M[r][i] 2^(8 j) mod q_r, laid out as the A operands of v_mfma_i32_16x16x64_i8, and the constant that undoes the shift of
@@ -569,26 +587,32 @@ int he_context_create(const he_context_desc *d, he_context **out) {
                 const uint64_t w = d->psi[2 * (t * n + i)];
                 uint64_t iw = 2 * d->ipsi_div2[2 * (t * n + i)];
                 if (iw >= q) iw -= q;
-                psi_fp[t * n + i] = (double)w;
-                ipsi_fp[t * n + i] = (double)iw;
+                psi_fp[t * n + i] = centred(w, q);
+                ipsi_fp[t * n + i] = centred(iw, q);
             }
             const uint64_t ninv = q - (q - 1) / n;  // q = 1 mod 2N, so N * (q - (q-1)/N) = 1 mod q
             consts[4 * t] = qd;
             consts[4 * t + 1] = 1.0 / qd;
-            consts[4 * t + 2] = (double)ninv;
+            consts[4 * t + 2] = centred(ninv, q);
         }
         if (d->size_p) {
-            // (8 doubles of padding: the fused conversion kernel fetches 8 entries per row whatever the row's length)
             const size_t entries = (size_t)d->size_q * d->size_p;
-            std::vector<double> pfp(entries + 8, 0.0);
+            std::vector<double> pfp(entries);
             for (size_t i = 0; i < entries; i++) pfp[i] = (double)d->phat_mod_q[i];
             rc = upload(ctx, &ctx->d_phat_mod_q_fp, pfp.data(), pfp.size());
-            // (P / p_k) P^-1 mod q_j: delta_j P^-1 straight from the conversion
-            for (size_t i = 0; i < entries; i++) {
-                const size_t jq = i / d->size_p;
-                pfp[i] = (double)(uint64_t)((unsigned __int128)d->phat_mod_q[i] * d->pinv_mod_q[2 * jq] % d->moduli[jq]);
+            if (!rc && d->size_p <= 8) {
+                std::vector<double> down, mdr;
+                for (uint32_t jq = 0; jq < d->size_q; jq++) {
+                    const uint64_t q = d->moduli[jq];
+                    auto entry = [&](uint32_t k) { return d->phat_mod_q[(size_t)jq * d->size_p + k]; };
+                    conversion_row(down, d->size_p, q, entry);
+                    // (P / p_k) P^-1 mod q_j: delta_j P^-1 straight from the conversion
+                    conversion_row(mdr, d->size_p, q,
+                                   [&](uint32_t k) { return (uint64_t)((unsigned __int128)entry(k) * d->pinv_mod_q[2 * jq] % q); });
+                }
+                rc = upload(ctx, &ctx->d_rows_down, down.data(), down.size());
+                if (!rc) rc = upload(ctx, &ctx->d_rows_mdr, mdr.data(), mdr.size());
             }
-            if (!rc) rc = upload(ctx, &ctx->d_phat_pinv_fp, pfp.data(), pfp.size());
             if (!rc && d->log_n == 16 && d->size_p <= 8) {
                 // the same matrix for the int8 matrix cores: rows in groups of four with the bytes of the rescale term,
                 // and every row alone (the row of the limb that a level drops)
@@ -712,9 +736,17 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
             if (rc) return rc;
             lv.batched = true;
             if (fp_for_level(ctx, L)) {
-                std::vector<double> mfp(mat_words + 8, 0.0);   // padded as the P -> Ql matrix is
+                std::vector<double> mfp(mat_words), rows;
                 for (size_t i = 0; i < mat_words; i++) mfp[i] = (double)mats[i];
                 rc = upload(ctx, &lv.d_mats_fp, mfp.data(), mfp.size());
+                if (rc) return rc;
+                for (uint32_t dg = 0; dg < beta; dg++) {
+                    const Digit &g = lv.digits[dg];
+                    for (uint32_t r = 0; r < g.n_out; r++)
+                        conversion_row(rows, g.size, ctx->h_moduli[table_of(ctx, L, r < g.start ? r : r + g.size)],
+                                       [&](uint32_t i) { return mats[g.mat_off + (size_t)r * g.size + i]; });
+                }
+                rc = upload(ctx, &lv.d_rows_up, rows.data(), rows.size());
                 if (rc) return rc;
                 if (ctx->log_n == 16) {
                     // the digit matrices for the int8 matrix cores (BconvRows::mx_tab), one record per four output rows
@@ -990,7 +1022,7 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     const int inv_backend = backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, lv->n_modup_jobs * items);
     BconvRows conv{ws, out, skip_own ? nullptr : c, (size_t)c_item_stride * n, LimbMap{LK, 0, L, ctx->size_q}, ctx->size_p, lv->beta, items, 1,
-                   fp_for_level(ctx, L) ? lv->d_mats_fp : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr, 0};
+                   fp_for_level(ctx, L) ? lv->d_rows_up : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr, 0};
     if (fused && tiles) use_tiles(ctx, inv, inv_backend, conv, tiles, L);
     if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, items, inv_backend, S(s)));
     HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), tin != nullptr, source_intt));
@@ -1105,7 +1137,7 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, n_polys * L);
     const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
     BconvRows conv{cx, ws, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, units, items, 0,
-                   fp_for_level(ctx, L) ? ctx->d_phat_mod_q_fp : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr, 0};
+                   fp_for_level(ctx, L) ? ctx->d_rows_down : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr, 0};
     if (fused && (size_t)n_polys * K <= scratch_limbs) use_tiles(ctx, inv, inv_backend, conv, scratch, K);
     HE_HIP(launch_ntt_inverse(inv, n_polys, inv_backend, S(s), inverted, source_intt));
     if (reduce_in_ntt) {
@@ -1395,7 +1427,7 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     // (3) delta = P -> Ql conversion of the special limbs
     const bool fused = fuse_rows_ok(ctx, lv, L);
     BconvRows conv{cx, delta, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, 2, items, 0,
-                   fp_for_level(ctx, L) ? ctx->d_phat_pinv_fp : nullptr, 1, ctx->d_mx_down,
+                   fp_for_level(ctx, L) ? ctx->d_rows_mdr : nullptr, 1, ctx->d_mx_down,
                    ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q, 0};
     if (fused && (size_t)polys * (K + 1) <= digit_limbs(ctx, lv, L, items)) use_tiles(ctx, inv, inv_backend, conv, w.y, K + 1);
     HE_HIP(launch_ntt_inverse(inv, polys, inv_backend, S(s), inverted, source_intt));

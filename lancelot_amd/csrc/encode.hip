@@ -514,10 +514,8 @@ __global__ __launch_bounds__(256 * LIMBS) void decode_rows_compose_kernel(HE_HEA
         double w[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) w[j] = FpArith::from_word(x[j]);
-        ar.reduce(w);
         T4::template inverse<FpArith>(w, tw, ar, lds, t);
-#pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(fp_mulmod(w[j], scale, ar.m), ar.m));
+        ar.template scale<T4::stages(0)>(x, w, scale);
     } else {
         const IntArith ar = int_arith(a, job.table);
         IntArith::Tw tw[NB];

@@ -150,7 +150,7 @@ struct NttArgs {
     uint32_t epi_b_poly_stride;
     uint32_t epi_b_mask;      // NTT_EPI_SUB_MUL_ADD: bit (poly mod 32) set = that polynomial has an addend
     uint64_t *tiles;          // inverse transform, rows pass, N = 2^16: the coefficients leave in the order in which a fused base conversion
-                              // reads them (conversion_word), on the FP64 back end as doubles, limb (poly, i) at tiles + (poly * tiles_poly_stride + i) * N
+                              // reads them (conversion_word), on the FP64 back end as doubles less 2^49, limb (poly, i) at tiles + (poly * tiles_poly_stride + i) * N
     uint32_t tiles_poly_stride;
     uint32_t in_galois;       // inverse transform, map mode: the input is sigma(in), gathered by the blocks pass
     const uint64_t *pro_w;    // [limbs][2] Shoup constants of the scaling prologue / epilogue, indexed like w
@@ -324,7 +324,10 @@ struct BconvRows {
     LimbMap map;                 // Ql u P
     uint32_t K, units, items;
     int up;
-    const double *mat_fp;        // behind the last row 8 more that may be read
+    // Levels whose primes are all below 2^50: a row of kConversionRow doubles per output limb, digit after digit: 8 entries of the matrix
+    // row, each in (-q/2, q/2), zeros behind the last; 2^49 times their sum mod q (the kernel multiplies x - 2^49); 2^50 mod q, times 2^-50.
+    // Otherwise nullptr.
+    const double *rows_fp;
     // merged ModDown + rescale: the last row of every unit's matrix is the limb that is dropped; the other output
     // limbs receive sum_i x_i M[j][i] + ((t - sum_i x_i M[last][i] mod q_last) mod q_j), t = the limb before x
     int mdr;
@@ -340,22 +343,22 @@ struct BconvRows {
     // stores byte i of r = (t - sum_i x_i M[last][i]) mod q_last there, and the records of mx_tab multiply it by the
     // digits of 2^(8 i) mod q_r.
     const void *mx_last;
-    // levels with a prime from 2^50 on (mat_fp == nullptr): the matrix in integers, and, mdr, P^-1 mod q_j (Shoup pairs)
+    // levels with a prime from 2^50 on (rows_fp == nullptr): the matrix in integers, and, mdr, P^-1 mod q_j (Shoup pairs)
     const uint64_t *mat;
     const uint64_t *w;
-    // N = 2^16: the input limbs are in the order of conversion_word, as doubles with mat_fp (not for the matrix kernel); ModDown: in [items][units]
+    // N = 2^16: the input limbs are in the order of conversion_word, with rows_fp as doubles, less 2^49 (not for the matrix kernel); ModDown: in [items][units]
     // [K][N], mdr: [K + 1][N] with t's limb in front
     int tiled;
 };
 // What its kernels take: NttHead with in and out, h1 = units | K << 16, h2 = workgroups of a tile that compute | that copy << 16,
 // h5 = rows of one, and pro_mode 1 for ModUp; behind it
 struct BconvExtra {
-    const void *mat;             // mat_fp, mat or mx_tab
+    const void *mat;             // rows_fp, mat or mx_tab
     const void *w;               // w or mx_last
     const uint64_t *copy_base;
     size_t copy_item_stride;
 };
-constexpr uint32_t kMxRecord = 144;
+constexpr uint32_t kMxRecord = 144, kConversionRow = 10;
 // `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
 // and `backend` says what the blocks pass that follows runs on
 // whether `inv`, the inverse transform that ends in b's inputs, should leave them tiled (in a buffer of their own: its last pass is in

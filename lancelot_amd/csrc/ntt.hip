@@ -175,8 +175,7 @@ __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARA
         } else {
             const double scale = inverse_scale(a, job, ar.m);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) x[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], scale, ar.m), ar.m));
+            ar.template scale<T4::stages(0)>(x, v, scale);
         }
     }
     if constexpr (BE != NTT_BACKEND_FP) {
@@ -294,7 +293,7 @@ __device__ __forceinline__ void fuse_last(const double *ld, const double *twl, F
         double v[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = ld[swz8(base + ((uint32_t)j << 3))];
-        fp_ct_block<2, 2>(v, twl, 64u + upper, m);
+        fp_ct_block<2, 1>(v, twl, 64u + upper, m);   // (at most 1.8 q: see FpArith)
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const uint32_t e = base + ((uint32_t)j << 3);
@@ -593,7 +592,7 @@ void bconv_rows_mx_kernel(HE_HEAD_PARAMS, BconvExtra b) {
 // K = 6, L = 30: one 203.0 / 201.2; K = 4, L = 12: one 80.8 / 74.4, two 129.7 / 124.4, eight 410 / 403.  (Merged ModDown +
 // rescale, K = 8: eight 106 / 122 us.)
 static bool bconv_on_matrix_cores(uint32_t log_n, const BconvRows &b, const Tuning &tune) {
-    return log_n == 16 && b.mat_fp && b.mx_tab && !b.tiled && !tune.no_matrix_bconv && b.K > 4 && (!b.mdr || b.mx_last) &&
+    return log_n == 16 && b.rows_fp && b.mx_tab && !b.tiled && !tune.no_matrix_bconv && b.K > 4 && (!b.mdr || b.mx_last) &&
            ((uint64_t)b.units * (b.items ? b.items : 1) << (log_n - kFuseLog)) >= (tune.cus ? tune.cus : 256);
 }
 
@@ -604,7 +603,7 @@ static bool bconv_on_matrix_cores(uint32_t log_n, const BconvRows &b, const Tuni
 // 39.7 / 40.5; hoisting 24 + 8 238.6 / 235.6, 4 + 2 49.3 / 51.0; 60 / 40 bits: rotation 24 + 8 157.3 / 153.2, 8 + 2 65.2 / 63.3, 4 + 2 42.6 /
 // 42.8, product 24 + 8 189 / 187, 4 + 2 50.5 / 51.6.  At 2^15 the segments are whole lines already: rotation 24 + 8 68.0 / 67.3, 10 + 3 43.7 / 44.6.
 bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune) {
-    return inv.log_n == 16 && b.map.limbs >= 10 && !bconv_on_matrix_cores(inv.log_n, b, tune) && (b.mat_fp != nullptr) == (inv_backend == NTT_BACKEND_FP);
+    return inv.log_n == 16 && b.map.limbs >= 10 && !bconv_on_matrix_cores(inv.log_n, b, tune) && (b.rows_fp != nullptr) == (inv_backend == NTT_BACKEND_FP);
 }
 
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s) {
@@ -631,7 +630,7 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     uint32_t target = mx ? (forced + 3) / 4 * 4 : forced;
     if (!target) {
         uint64_t best = ~0ull;
-        const uint32_t single = b.mat_fp ? 23 : 25;
+        const uint32_t single = b.rows_fp ? 23 : 25;
         for (uint32_t r = step; r <= kFuseMaxRows && r < rows + step; r += step) {
             const uint64_t wgs = (uint64_t)b.units * items * tiles * ((rows + r - 1) / r);
             const uint64_t per_cu = (wgs + cus - 1) / cus;
@@ -650,7 +649,7 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     m.out = b.out;
     m.map = b.map;
     m.pro_mode = b.up;
-    if (!b.mat_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;
+    if (!b.rows_fp) m.fp_mask = backend == NTT_BACKEND_INT ? 0 : backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask;
     NttHead h = ntt_head(m, (uint32_t)wgs, target);
     h.h1 = b.units | b.K << 16;
     h.h2 = compute_groups | copy_groups << 16;

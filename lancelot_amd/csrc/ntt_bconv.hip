@@ -34,49 +34,41 @@ namespace {
 
 constexpr int kTileLog = 11;
 
-// Conversion in FP64 (every prime of the level below 2^50)
+// Conversion in FP64 (every prime of the level below 2^50).  The inputs are held as x' = x - 2^49 and the matrix entries centred, so that
+// a product is below 2^98 in magnitude; what the shift takes away comes back with the row's constant (BconvRows::rows_fp).
 template <int NIN, bool MDR, bool TILED>
 struct ConvFp {
     double x[NIN][4], rr[MDR ? 4 : 1];
-    // (tiled words are doubles)
-    static __device__ __forceinline__ double value(uint64_t w) { return TILED ? FpArith::from_word(w) : fp_from_u64(w); }
-    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = value(w); }
-    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
-        const uint32_t last = d.n_out - 1;
-        const FpMod m = fp_ctx(a, map_table(a.map, last)).m;
-        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + d.mat_off + (size_t)last * d.n_in;
-#pragma unroll
-        for (int j = 0; j < 4; j++) rr[j] = value(t[j]);
-#pragma unroll
-        for (int k = 0; k < NIN; k++) {
-            if ((uint32_t)k >= d.n_in) break;
-            const double w = row[k];
-#pragma unroll
-            for (int j = 0; j < 4; j++) rr[j] -= fp_mulmod(x[k][j], w, m);
-        }
-#pragma unroll
-        for (int j = 0; j < 4; j++) rr[j] = fp_canonical(rr[j], m);
+    // (tiled words are doubles, and shifted already)
+    static __device__ __forceinline__ double value(uint64_t w) {
+        return TILED ? FpArith::from_word(w) : __longlong_as_double((long long)(w | 0x4330000000000000ull)) - 0x1.2p52;
     }
-    // The sum as an exact pair (hi, lo) before any reduction, four operations per term.  hi runs in [2^103, 2^104), where
-    // doubles are the multiples of 2^51: t = fl(x w + hi) rounds the exact sum to such a multiple (eight products below 2^100 keep
-    // it under 2^104), t - hi is exact, x w - (t - hi) is the rounding error, an integer of at most 2^50 in magnitude that the
-    // second fused multiply-add returns exactly, and eight of those sum exactly.  (hi - 2^103) / 2^51 is an integer below
-    // 2^52; times 2^51 mod m it is congruent to the high part, and the modular product takes it as it is.
-    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t,
-                                            const FpArith &ar) const {
-        const ScalarF64 row = scalar(static_cast<const double *>(b.mat)) + d.mat_off + (size_t)r * d.n_in;
+    __device__ __forceinline__ void take(int k, int j, uint64_t w) { x[k][j] = value(w); }
+    static __device__ __forceinline__ ScalarF64 row_of(const BconvExtra &b, const BconvUnit &d, uint32_t r) {
+        return scalar(static_cast<const double *>(b.mat)) + (size_t)(d.row_off + r) * kConversionRow;
+    }
+    // v = sum of x M mod q, at most 1.01 q in magnitude, the sums' low part starting from lo.
+    // The sum as an exact pair (hi, lo) before any reduction, four operations per term.  hi runs in [2^102, 2^103], where doubles are the
+    // multiples of 2^50: t = fl(x w + hi) rounds the exact sum to such a multiple (eight products below 2^98 stay within 2^101 of
+    // 1.5 2^102), t - hi is exact, x w - (t - hi) is the rounding error, an integer of at most 2^49 that the second fused multiply-add
+    // returns exactly; eight of those, the row's constant below 2^49 and a residue below 2^50 sum exactly, to less than 2^52.5.
+    // With H = hi - 1.5 2^102, a multiple of 2^50 up to 2^101, and c = 2^50 mod q the sum is H 2^-50 c + lo = h + l + lo, h = fl(H 2^-50 c),
+    // up to 2^100, and one quotient serves all three: k = rint(lo / q + h / q), of which h's part is off by at most 3/8 (three roundings of a
+    // number up to 2^50) and their sum by 1/8; h - k q is within q + 2^47 of -lo, below 2^53 as is every sum after it, and exact.
+    static __device__ __forceinline__ void sum(double *v, const double (*x)[4], ScalarF64 row, uint32_t n_in, FpMod m, const double *lo0) {
         double hi[4], lo[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            hi[j] = 0x1p103;
-            lo[j] = 0.0;
+            hi[j] = 0x1.8p102;
+            lo[j] = lo0[j];
         }
         double w[NIN];
 #pragma unroll
-        for (int k = 0; k < NIN; k++) w[k] = row[k];   // (the matrices are padded: 8 entries can be read whatever the row's length)
+        for (int k = 0; k < NIN; k++) w[k] = row[k];
+        const double c = row[9];
 #pragma unroll
         for (int k = 0; k < NIN; k++) {
-            if ((uint32_t)k >= d.n_in) break;
+            if ((uint32_t)k >= n_in) break;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
                 const double t = __builtin_fma(x[k][j], w[k], hi[j]);
@@ -84,14 +76,31 @@ struct ConvFp {
                 hi[j] = t;
             }
         }
-        const FpMod m = ar.m;
-        const double c51 = fp_reduce(0x1p51, m);
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            v[j] = fp_mulmod((hi[j] - 0x1p103) * 0x1p-51, c51, m) + fp_reduce(lo[j], m);   // below 3 m
-            if constexpr (MDR) v[j] += rr[j];
+            const double big = hi[j] - 0x1.8p102, h = big * c, l = __builtin_fma(big, c, -h);
+            const double k = __builtin_rint(__builtin_fma(lo[j], m.qinv, h * m.qinv));
+            v[j] = (__builtin_fma(-k, m.q, h) + l) + lo[j];
         }
-        ar.reduce(v);   // (four stages without a reduction start from at most 1.27 q)
+    }
+    __device__ __forceinline__ void dropped(const NttArgs &a, const BconvExtra &b, const BconvUnit &d, const uint64_t *t) {
+        const uint32_t last = d.n_out - 1;
+        const FpMod m = fp_ctx(a, map_table(a.map, last)).m;
+        const ScalarF64 row = row_of(b, d, last);
+        double v[4], lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) lo[j] = row[8];
+        sum(v, x, row, d.n_in, m, lo);
+#pragma unroll
+        for (int j = 0; j < 4; j++) rr[j] = fp_canonical((value(t[j]) + 0x1p49) - v[j], m);
+    }
+    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t,
+                                            const FpArith &ar) const {
+        const ScalarF64 row = row_of(b, d, r);
+        double lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) lo[j] = MDR ? rr[j] + row[8] : row[8];
+        sum(v, x, row, d.n_in, ar.m, lo);
     }
 };
 
@@ -279,13 +288,13 @@ hipError_t launch_bconv_rows4(const NttHead &head, const BconvRows &b, hipStream
     NttHead h = head;
     const uint32_t log_n = h.h0 & 31, groups = (h.h2 & 0xffff) + (h.h2 >> 16);
     const uint64_t wgs = (uint64_t)b.units * (b.items ? b.items : 1) * (1u << (log_n - kTileLog)) * groups;
-    if (log_n < 12 || log_n > 16 || b.K == 0 || b.K > 8 || (!b.mat_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
+    if (log_n < 12 || log_n > 16 || b.K == 0 || b.K > 8 || (!b.rows_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
         return hipErrorInvalidValue;
     h.h4 = (uint32_t)wgs;
-    const BconvExtra x{b.mat_fp ? static_cast<const void *>(b.mat_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride};
+    const BconvExtra x{b.rows_fp ? static_cast<const void *>(b.rows_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride};
 #define HE_TILED(FP, NIN, MDR) (b.tiled ? launch_nin<FP, NIN, MDR, true>(h, log_n, x, s) : launch_nin<FP, NIN, MDR, false>(h, log_n, x, s))
 #define HE_NIN(FP, MDR) (b.K <= 4 ? HE_TILED(FP, 4, MDR) : HE_TILED(FP, 8, MDR))
-    if (b.mat_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
+    if (b.rows_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
     return b.mdr ? HE_NIN(false, true) : HE_NIN(false, false);
 #undef HE_NIN
 #undef HE_TILED

@@ -96,7 +96,7 @@ struct BconvUnit {
     const uint64_t *in;
     uint64_t *out;
     size_t mat_off;
-    uint32_t mx_off;
+    uint32_t mx_off, row_off;
     bool up;
     __device__ __forceinline__ uint32_t limb(uint32_t row) const { return up && row >= copy_first ? row + n_in : row; }
 };
@@ -107,7 +107,7 @@ __device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units
     BconvUnit u;
     u.up = a.pro_mode;
     u.item = index / units;
-    u.copy_first = u.mx_off = 0;
+    u.copy_first = u.mx_off = u.row_off = 0;
     u.mat_off = 0;
     u.n_in = K;
     u.n_out = L;
@@ -118,6 +118,7 @@ __device__ __forceinline__ BconvUnit bconv_unit(const NttArgs &a, uint32_t units
         u.n_out = LK - u.n_in;
         u.mat_off = (size_t)u.copy_first * (LK - K);
         u.mx_off = d * ((LK - K + 3) / 4);
+        u.row_off = d * (LK - K);
         u.in = a.in + (((size_t)u.item * L + u.copy_first) << a.log_n);
         u.out = a.out + ((size_t)index * LK << a.log_n);
     } else {
@@ -210,12 +211,12 @@ __device__ __forceinline__ FpCtx fp_ctx(const NttArgs &a, uint32_t table) {
     return FpCtx{FpMod{c[0], c[1]}, a.tw_fp + ((size_t)table << a.log_n)};
 }
 
-// (N^-1 [* w]) for the last multiplication of the inverse transform
+// (N^-1 [* w]) for the last multiplication of the inverse transform, centred
 __device__ __forceinline__ double inverse_scale(const NttArgs &a, const Job &job, FpMod m) {
     const ScalarF64 c = scalar(a.fp_consts) + 4 * (size_t)job.table;
     const double ninv = c[2];
     if (a.epi_mode != NTT_EPI_MUL) return ninv;
-    return fp_canonical(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
+    return fp_reduce(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
 }
 
 // coefficient at `at` of polynomial job.poly of an encoding, rounded (NTT_PRO_ROUND)
@@ -400,11 +401,17 @@ struct IntArith {
         gs_butterfly(v[1], v[3], t.s[0], m);
     }
     __device__ __forceinline__ void reduce(V *) const {}
+    __device__ __forceinline__ void settle(V *) const {}
 };
 
-// Bounds (in units of q, |v| < 8 keeps every value exact): forward, a stage takes b to 1.375 b + 0.5, so four stages
-// between reductions end at 5.3 (7.1 from canonical words); inverse, words are reduced before every two stages, whose
-// sums end at 2 (4 from canonical words) and whose products stay below that.
+// Bounds, in units of 2^50 > q: |v| < 8 keeps every value exact.  The twiddles are centred, so a product with a word below b is at most
+// 0.5 + 0.1875 b (the quotient's estimate is three roundings off).
+// Forward, a stage takes b to 1.1875 b + 0.5: six stages from 1 (canonical words, a conversion's sums up to 1.01) end at 7.7, from 0.5
+// (reduced) at 6.2, four from 2.63 at 7.9.  One reduction in a rows pass that leaves at most three stages behind it (2.63), one in the
+// middle of the blocks pass (3.63 at its end): see Tile4.
+// Inverse, a block of two stages leaves sums of four words at 4 b, sums of two products at 1 + 0.75 b, and 0.5 + 0.75 b and less in the
+// others.  Reducing the first two (settle) keeps b below 2 from canonical words on: 1, 1.25, 1.44, 1.58, 1.69, 1.77, 1.83, 1.87, ..., and 4 b
+// below 8.
 struct FpArith {
     using V = double;
     struct Tw {
@@ -459,6 +466,28 @@ struct FpArith {
 #pragma unroll
         for (int j = 0; j < 4; j++) v[j] = fp_reduce(v[j], m);
     }
+    __device__ __forceinline__ void settle(V *v) const {
+        v[0] = fp_reduce(v[0], m);
+        v[1] = fp_reduce(v[1], m);
+    }
+    // v s as canonical values for the words that the inverse's last block of ST stages has left: with v[0] (and v[1] after one stage)
+    // reduced they are at most 2.4, the products at most 0.95 q
+    template <int ST>
+    __device__ __forceinline__ void scale(V *v, double s) const {
+        v[0] = fp_reduce(v[0], m);
+        if (ST == 1) v[1] = fp_reduce(v[1], m);
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double p = fp_mulmod(v[j], s, m);
+            v[j] = p < 0.0 ? p + m.q : p;
+        }
+    }
+    template <int ST>
+    __device__ __forceinline__ void scale(uint64_t *w, V *v, double s) const {
+        scale<ST>(v, s);
+#pragma unroll
+        for (int j = 0; j < 4; j++) w[j] = fp_to_u64(v[j]);
+    }
 };
 
 // A tile of 2^B words, 4 per thread, whose stages 0 .. LD-1 pair the tile bits B-1, B-2, ...; block k holds the stages
@@ -470,6 +499,8 @@ struct Tile4 {
     static constexpr int kBlocks = (LD + 1) / 2;
     static_assert(B >= 8 && 2 * kBlocks <= B, "four words of every block lie inside the tile");
     static constexpr int stages(int k) { return LD - 2 * k >= 2 ? 2 : 1; }
+    // the forward block before which words are reduced (FpArith): whole limbs and the blocks pass (B = LD), rows passes
+    static constexpr int kReduceBefore = B == LD ? (LD <= 10 ? 2 : 3) : LD <= 2 ? kBlocks : LD <= 5 ? 1 : LD <= 7 ? 2 : 3;
     static __device__ __forceinline__ uint32_t word(int k, uint32_t t, int j) {
         const int low = B - 2 * k - 2;
         return ((t >> low) << (low + 2)) | ((uint32_t)j << low) | (t & ((1u << low) - 1));
@@ -522,7 +553,7 @@ struct Tile4 {
         ar.template ct<stages(K)>(v, tw[K]);
         if constexpr (K + 1 < kBlocks) {
             exchange<A, K, false>(v, lds, t);
-            if constexpr ((K + 1) % 2 == 0) ar.reduce(v);
+            if constexpr (K + 1 == kReduceBefore) ar.reduce(v);
             forward<A, K + 1>(v, tw, ar, lds, t);
         }
     }
@@ -530,9 +561,11 @@ struct Tile4 {
     static __device__ __forceinline__ void inverse(typename A::V *v, const typename A::Tw *tw, const A &ar, uint64_t *lds, uint32_t t) {
         ar.template gs<stages(K)>(v, tw[K]);
         if constexpr (K > 0) {
+            ar.settle(v);
             exchange<A, K - 1, true>(v, lds, t);
-            ar.reduce(v);
             inverse<A, K - 1>(v, tw, ar, lds, t);
+        } else if constexpr (B == 8 && LD == 8) {
+            ar.settle(v);   // (blocks pass: the rows pass goes on)
         }
     }
 };

@@ -101,12 +101,10 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
         for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(s[j]);
         FpArith::Tw tw[NB];
         T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
-        ar.reduce(v);
         T4::template inverse<FpArith>(v, tw, ar, lds, t);
         const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
         const double ninv = cc[2];
-#pragma unroll
-        for (int j = 0; j < 4; j++) s[j] = fp_to_u64(fp_canonical(fp_mulmod(v[j], ninv, ar.m), ar.m));
+        ar.template scale<T4::stages(0)>(s, v, ninv);
     } else {
         const uint64_t q = scalar(a.moduli)[st];
         const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
@@ -190,13 +188,11 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(job.in[glob(NB - 1, j)]);
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
             const double scale = inverse_scale(a, job, c.m);
-            ar.reduce(v);
             T4::template inverse<FpArith>(v, tw, ar, lds, t);
-#pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = fp_canonical(fp_mulmod(v[j], scale, c.m), c.m);
+            ar.template scale<T4::stages(0)>(v, scale);
             uint64_t w[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) w[j] = TILES && BE == NTT_BACKEND_FP ? FpArith::to_word(v[j]) : fp_to_u64(v[j]);
+            for (int j = 0; j < 4; j++) w[j] = TILES && BE == NTT_BACKEND_FP ? FpArith::to_word(v[j] - 0x1p49) : fp_to_u64(v[j]);
             leave(w);
         }
         return;
@@ -364,11 +360,10 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             if (FWD) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
-                ar.reduce(v);
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
                 turn_pairs(v);
                 if (EPI) {
-                    // (the word enters the difference as the last stage leaves it: at most 5.3 q, minuend below 1.9 q)
+                    // (the word enters the difference as the last stage leaves it: at most 3.7 q, minuend below 1.9 q)
                     const double ew = fp_from_u64(e.w.w);
                     if (e.fma) {
                         const double pw = fp_from_u64(e.pro_w.w);
@@ -452,8 +447,8 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
 }
 
 // Sum over the digits of (word x key word) for four words of both key polynomials.
-// FP64: a transformed word enters as the last stage leaves it (at most 5.3 q: a term below 2.5 q), the sums are reduced after
-// every second digit and stay below 6 q.  Integers: canonical words, 128-bit sums of at most 64 products below 2^122.
+// FP64: a transformed word enters as the last stage leaves it (at most 3.7 q: a term below 1.9 q), the sums are reduced after
+// every fourth digit and stay below 8 q.  Integers: canonical words, 128-bit sums of at most 64 products below 2^122.
 struct FpSums {
     double s[2][4];
     uint32_t pending = 0;
@@ -469,7 +464,7 @@ struct FpSums {
                 const double w = fp_from_u64(k[r][j]);
                 s[r][j] += fp_mulmod(v[j], w, ar.m);
             }
-        if (++pending == 2) {
+        if (++pending == 4) {
             pending = 0;
             ar.reduce(s[0]);
             ar.reduce(s[1]);
@@ -631,7 +626,6 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         // (behind a branch that may skip these loads the compiler waits for them with the keys; short chains fetch their last digit
         // again instead: n = 2^15, 10 of 12 limbs 71.5 -> 69.8 us.  One wave a block loses by it: L = 24, K = 8 153 against 156 us)
         if (SPLIT > 1 || d < beta) fetch(nx, d < beta ? d : now);
-        ar.reduce(v);
         T4::template forward<A>(v, tw, ar, nullptr, lane);
         turn_pairs(v);
         if constexpr (!FP) {
@@ -907,7 +901,6 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
     typename A::V v[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
-    ar.reduce(v);
     T4::template forward<A>(v, tw, ar, nullptr, lane);
     turn_pairs(v);
     if (w == 0) {
@@ -989,7 +982,6 @@ __device__ __forceinline__ void decrypt_block(const NttArgs &a, const DecryptArg
     typename A::V v[4];
 #pragma unroll
     for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
-    ar.reduce(v);
     T4::template forward<A>(v, tw, ar, nullptr, lane);
     turn_pairs(v);
     uint64_t o[4];
