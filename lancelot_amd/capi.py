@@ -83,6 +83,7 @@ SIGNATURES = {
     "he_sample": (C.c_int, [vp, C.c_int, C.POINTER(u32), u64, vp, u32, u32, u32, u32, vp, u32, vp]),
     "he_ckks_encode_batch_workspace_words": (C.c_size_t, [vp, u32]),
     "he_ckks_encode_batch": (C.c_int, [vp, vp, vp, u32, u32, C.c_double, u32, u32, C.c_size_t, vp, u32, vp, vp]),
+    "he_widen_rows": (C.c_int, [vp, vp, u32, C.c_size_t, C.c_size_t, vp]),
     "he_ckks_encode_bounded": (C.c_int, [vp, vp, vp, u32, u32, C.c_double, u32, u32, C.c_size_t, vp, u32, vp, vp]),
     "he_encrypt": (C.c_int, [vp, u32, vp, vp, C.POINTER(u32), u64, vp, vp, vp]),
     "he_decrypt_flood": (C.c_int, [vp, vp, u32, u32, vp, C.c_size_t, C.POINTER(u32), u64, vp, u32, vp, vp, vp]),

@@ -1593,6 +1593,13 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     return he_ntt_forward(ctx, out, items, out_poly_stride, limbs, 0, limbs, 0, s);
 }
 
+int he_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, he_stream s) {
+    if (!in || !out || rows == 0 || rows > 65535 || padded == 0 || padded % 2 || length > padded || (reinterpret_cast<uintptr_t>(out) & 15))
+        return HE_E_INVALID_ARGUMENT;
+    HE_HIP(launch_widen_rows(in, out, rows, length, padded, S(s)));
+    return HE_OK;
+}
+
 int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t slots,
                            double scale, uint32_t limbs, uint32_t items, size_t value_stride, uint64_t *out,
                            uint32_t out_poly_stride, uint64_t *ws, he_stream s) {

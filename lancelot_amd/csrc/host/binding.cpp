@@ -254,6 +254,19 @@ PYBIND11_MODULE(pyCAHEL, m) {
                  return e.encode_encrypt_many(c, pk, values, items, count, count, scale);
              },
              py::arg("context"), py::arg("public_key"), py::arg("values").noconvert(), py::arg("scale"))
+        .def("encode_encrypt_updates",
+             [](CAHELGPUCKKSEncoder &e, const CAHELGPUContext &c, const CAHELGPUPublicKey &pk,
+                const std::vector<py::array_t<float, py::array::c_style>> &updates, double scale) {
+                 std::vector<const float *> rows;
+                 for (const auto &u : updates) {
+                     if (u.size() != updates[0].size()) throw std::invalid_argument("all client updates must have the same length");
+                     rows.push_back(u.data());
+                 }
+                 const std::size_t length = updates.empty() ? 0 : (std::size_t)updates[0].size();
+                 py::gil_scoped_release release;
+                 return e.encode_encrypt_updates(c, pk, rows, length, scale);
+             },
+             py::arg("context"), py::arg("public_key"), py::arg("updates").noconvert(), py::arg("scale"))
         .def("decode_array",
              [](CAHELGPUCKKSEncoder &e, const CAHELGPUContext &c, const CAHELGPUPlaintext &p, std::size_t count) {
                  py::array_t<double> out((py::ssize_t)e.decode_count(c, p, count));

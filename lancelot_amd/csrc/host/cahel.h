@@ -432,6 +432,10 @@ public:
     std::vector<CAHELGPUCiphertext> encode_encrypt_many(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
                                                         const double *values, std::size_t items, std::size_t count,
                                                         std::size_t value_stride, double scale);
+    // The same for vectors of 32-bit floats of any one length, each split into messages of N / 2 values (zeros behind the last): row
+    // after row, its messages in order.
+    std::vector<CAHELGPUCiphertext> encode_encrypt_updates(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
+                                                           const std::vector<const float *> &rows, std::size_t length, double scale);
     void encode(const CAHELGPUContext &context, const std::vector<double> &values, std::size_t chain_index, double scale,
                 CAHELGPUPlaintext &destination);
     void encode(const CAHELGPUContext &context, const std::vector<double> &values, double scale,
@@ -470,6 +474,10 @@ public:
     }
 
 private:
+    int batch_bits(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const;
+    std::vector<CAHELGPUCiphertext> encode_encrypt_staged(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
+                                                          const double *d_values, bool small, std::size_t items, std::size_t count,
+                                                          std::size_t slots, double scale, int total_bits);
     std::size_t slots_ = 0, sparse_slots_ = 0;
     std::size_t first_chain_index_ = 1;  // include/ckks.h:325
 };

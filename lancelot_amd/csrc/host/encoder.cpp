@@ -21,12 +21,13 @@ namespace {
 constexpr std::size_t kChunkBytes = std::size_t(1) << 20;
 
 // dst = src, and the sum of the magnitudes
-double copy_sum(double *dst, const double *src, std::size_t count) {
+template <class T>
+double copy_sum(T *dst, const T *src, std::size_t count) {
     double s = 0.0;
 #pragma omp simd reduction(+ : s)
     for (std::size_t i = 0; i < count; i++) {
         dst[i] = src[i];
-        s += std::fabs(src[i]);
+        s += std::fabs((double)src[i]);
     }
     return s;
 }
@@ -73,18 +74,9 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_many(const C
                                                                          std::size_t items, std::size_t count,
                                                                          std::size_t value_stride, double scale) {
     if (items == 0) return {};
-    if (items > 8192) throw std::invalid_argument("too many messages");
-    if (!pk.gen_flag_) throw std::logic_error("public key has not been generated");
     if (count > slots_ || value_stride < count) throw std::invalid_argument("values_size is too large");
-    const std::size_t chain = first_chain_index_;
-    if (chain == 0 || context.size_p() == 0) throw std::logic_error("batched encryption needs a data level and special primes");
-    const int total_bits = context.total_coeff_modulus_bit_count(chain);
-    if (scale <= 0 || (static_cast<int>(std::log2(scale)) + 1 >= total_bits))
-        throw std::invalid_argument("scale out of bounds");
+    const int total_bits = batch_bits(context, pk, items, scale);
     const std::size_t ss = message_slots(count);
-    const std::size_t n = context.poly_degree();
-    const uint32_t L = (uint32_t)context.limbs_at(chain);
-    he_context *h = context.handle();
     he_stream st = context.stream();
 
     // values -> device, packed, some messages at a time through page-locked memory (the next ones are copied while the last
@@ -103,6 +95,67 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_many(const C
         ring.fence(st);
         check_status(status, "upload");
     }
+    return encode_encrypt_staged(context, pk, d_values, small, items, count, ss, scale, total_bits);
+}
+
+std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_updates(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
+                                                                            const std::vector<const float *> &rows, std::size_t length,
+                                                                            double scale) {
+    if (rows.empty() || length == 0) return {};
+    const std::size_t chunks = (length + slots_ - 1) / slots_;
+    if (chunks > 8192 || rows.size() > 8192) throw std::invalid_argument("too many messages");
+    const std::size_t items = rows.size() * chunks, padded = chunks * slots_;
+    const int total_bits = batch_bits(context, pk, items, scale);
+    const std::size_t ss = message_slots(slots_);
+    he_stream st = context.stream();
+    // the floats as they are, row after row, some messages at a time through page-locked memory; the device widens them
+    const std::size_t total = rows.size() * length;
+    DeviceBuffer narrow((total + 1) / 2), staging(items * slots_);
+    float *d_floats = reinterpret_cast<float *>(narrow.get());
+    double *d_values = reinterpret_cast<double *>(staging.get());
+    PinnedRing &ring = PinnedRing::of_thread();
+    const std::size_t room = std::max(kChunkBytes / sizeof(float), slots_);
+    bool small = true;
+    float *host = nullptr;
+    std::size_t filled = 0, sent = 0;
+    auto send = [&] {
+        const int status = he_memcpy_h2d_async(d_floats + sent, host, filled * sizeof(float), st);
+        ring.fence(st);
+        check_status(status, "upload");
+        sent += filled;
+        filled = 0;
+    };
+    for (const float *row : rows)
+        for (std::size_t at = 0; at < length; at += slots_) {
+            const std::size_t taken = std::min(slots_, length - at);
+            if (filled + taken > room) send();
+            if (filled == 0) host = static_cast<float *>(ring.take(room * sizeof(float)));
+            small = surely_small(copy_sum(host + filled, row + at, taken), scale, ss, total_bits) && small;
+            filled += taken;
+        }
+    send();
+    check_status(he_widen_rows(d_floats, d_values, (uint32_t)rows.size(), length, padded, st), "he_widen_rows");
+    return encode_encrypt_staged(context, pk, d_values, small, items, slots_, ss, scale, total_bits);
+}
+
+// the modulus' bits at the level where batches are encrypted, if this one can be
+int CAHELGPUCKKSEncoder::batch_bits(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const {
+    if (items > 8192) throw std::invalid_argument("too many messages");
+    if (!pk.gen_flag_) throw std::logic_error("public key has not been generated");
+    if (first_chain_index_ == 0 || context.size_p() == 0) throw std::logic_error("batched encryption needs a data level and special primes");
+    const int total_bits = context.total_coeff_modulus_bit_count(first_chain_index_);
+    if (scale <= 0 || (static_cast<int>(std::log2(scale)) + 1 >= total_bits)) throw std::invalid_argument("scale out of bounds");
+    return total_bits;
+}
+
+// d_values: [items][count] on the device; small: no coefficient can reach the bounds
+std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_staged(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
+                                                                           const double *d_values, bool small, std::size_t items,
+                                                                           std::size_t count, std::size_t ss, double scale, int total_bits) {
+    const std::size_t n = context.poly_degree(), chain = first_chain_index_;
+    const uint32_t L = (uint32_t)context.limbs_at(chain);
+    he_context *h = context.handle();
+    he_stream st = context.stream();
     // plaintexts straight into polynomial 0 of the ciphertexts
     const std::size_t words = 2 * (std::size_t)L * n;
     DeviceBuffer batch(items * words), ws(he_ckks_encode_batch_workspace_words(h, (uint32_t)items));

@@ -490,6 +490,8 @@ hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const doubl
                               uint32_t slots, double scale, double2 *v, uint64_t *max_bits, uint32_t items, size_t value_stride,
                               uint64_t *out, uint32_t limbs, size_t out_item_stride, hipStream_t s);
 // Only the transform: the slot vectors stay in v [items][slots] for NTT_PRO_ROUND.  re / im may be page-locked host memory.
+// rows of `length` floats -> rows of `padded` doubles, zeros behind the floats
+hipError_t launch_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, hipStream_t s);
 hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
                                    double2 *v, uint32_t items, size_t value_stride, hipStream_t s);
 // res: [limbs][N] coefficient-form residues of the first `limbs` primes -> v: `slots` complex values.

@@ -131,6 +131,21 @@ def split_updates(vectors, slots: int):
     return [[row[k:k + slots] for k in range(0, whole, slots)] for row in padded]
 
 
+def encrypt_all(state: KrumState, updates):
+    """split_updates and encrypt_updates in one: updates of 32-bit floats are split, padded and widened on the device."""
+    rows = [np.asarray(u) for u in updates] if state.config.batched else []
+    if not rows or any(r.dtype != np.float32 or r.size == 0 for r in rows):
+        return encrypt_updates(state, split_updates(updates, state.slots))
+    if any(r.size != rows[0].size for r in rows):
+        raise ValueError("all client updates must have the same length")
+    t0 = time.perf_counter()
+    cts = iter(state.encoder.encode_encrypt_updates(state.context, state.pk, [np.ascontiguousarray(r).reshape(-1) for r in rows],
+                                                    state.config.scale))
+    _sync(state.cahel)
+    state.timings["encode"] += time.perf_counter() - t0   # encode and encrypt are one pipeline here
+    return [[next(cts) for _ in range(-(-rows[0].size // state.slots))] for _ in rows]
+
+
 def encrypt_updates(state: KrumState, chunks):
     """One ciphertext per (client, chunk).  Batched: all chunks through encode and encrypt together.  Otherwise the
     chunks go over the lanes (unless the run is to be reproducible); the first one is then encoded on the calling
@@ -363,7 +378,7 @@ def _packed_distance_matrix(state: KrumState, updates):
     """distance_matrix's numbers without its ciphertexts: the squared differences have real slots, so two pairs share a ciphertext
     through relinearisation, rescale, slot sum and decryption."""
     c = state.cahel
-    cts = encrypt_updates(state, split_updates(updates, state.slots))
+    cts = encrypt_all(state, updates)
     n_clients = len(updates)
     pairs = [(i, j) for i in range(n_clients) for j in range(i + 1, n_clients)]
     t0 = time.perf_counter()
@@ -501,8 +516,7 @@ def gpu_krum_aggregate(updates, config: KrumConfig | None = None, state: KrumSta
     for k in list(state.timings):
         state.timings[k] = 0.0
     t0 = time.perf_counter()
-    chunks = split_updates(updates, state.slots)
-    cts = encrypt_updates(state, chunks)
+    cts = encrypt_all(state, updates)
     n_clients = len(updates)
     t1 = time.perf_counter()
     if state.config.batched and n_clients > 1:

@@ -143,6 +143,14 @@ int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double
     return HE_OK;
 }
 
+int he_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, he_stream stream) {
+    queues[stream].push_back([=] {
+        for (uint32_t r = 0; r < rows; r++)
+            for (size_t i = 0; i < padded; i++) out[r * padded + i] = i < length ? (double)in[r * length + i] : 0.0;
+    });
+    return HE_OK;
+}
+
 size_t he_ckks_encode_batch_workspace_words(const he_context *, uint32_t items) { return 8 * (size_t)items; }
 
 // (what encoder.cpp refers to besides)
