@@ -448,7 +448,8 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
 
 // Sum over the digits of (word x key word) for four words of both key polynomials.
 // FP64: a transformed word enters as the last stage leaves it (at most 3.7 q: a term below 1.9 q), the sums are reduced after
-// every fourth digit and stay below 8 q.  Integers: canonical words, 128-bit sums of at most 64 products below 2^122.
+// every fourth digit and stay below 8 q.  Integers: 128-bit sums of at most 64 products below 2^122 of canonical words, or, with primes
+// below 2^60, of at most 40 products of words as the last stage leaves them (below 6 q).
 struct FpSums {
     double s[2][4];
     uint32_t pending = 0;
@@ -593,6 +594,8 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
             fetch_addends(part);
         }
     }
+    bool canonical = false;
+    if constexpr (!FP) canonical = (ar.m.q >> 60) || beta > 40;
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = a.in + (size_t)t * n;
@@ -629,49 +632,55 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         T4::template forward<A>(v, tw, ar, nullptr, lane);
         turn_pairs(v);
         if constexpr (!FP) {
+            if (SPLIT == 1 || canonical) {   // (one wave a block: the branch costs what it saves)
 #pragma unroll
-            for (int j = 0; j < 4; j++) v[j] = reduce_6q(v[j], ar.m.q);
+                for (int j = 0; j < 4; j++) v[j] = reduce_6q(v[j], ar.m.q);
+            }
         }
         sums.add(v, k, ar);
     }
     if constexpr (SPLIT > 1) {
+        // (integers: the 128-bit sums as they are, so that each is reduced once, by the wave that finishes it, and not by all that share it;
+        // with the words' reductions left out where they can be, rotations: n = 2^15, 10 + 3 limbs of 60 / 40 bits 51.9 -> 50.8 us; 2^14, 4 + 1
+        // of 60 bits 23.6 -> 22.7; 2^16, 2 + 1 29.5 -> 28.8)
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             uint64_t w[4];
-            if constexpr (FP) ar.reduce(sums.s[r]);
+            if constexpr (FP) {
+                ar.reduce(sums.s[r]);
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (FP)
-                    w[j] = A::to_word(sums.s[r][j]);
-                else
-                    w[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, ar.m.q, r0, r1);
+                for (int j = 0; j < 4; j++) w[j] = A::to_word(sums.s[r][j]);
+                store_pairs(sums_lds + (2 * part + r) * 256 + pair_lane(lane), w);
+            } else {
+#pragma unroll
+                for (int j = 0; j < 4; j++) w[j] = sums.s[r][j].lo;
+                store_pairs(sums_lds + (4 * part + 2 * r) * 256 + pair_lane(lane), w);
+#pragma unroll
+                for (int j = 0; j < 4; j++) w[j] = sums.s[r][j].hi;
+                store_pairs(sums_lds + (4 * part + 2 * r + 1) * 256 + pair_lane(lane), w);
             }
-            store_pairs(sums_lds + (2 * part + r) * 256 + pair_lane(lane), w);
         }
         lds_barrier();
         if (part > 1) return;
     }
     if (SPLIT == 1 && invert) T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
+    // one wave finishes both polynomials, or waves 0 and 1 one each
 #pragma unroll
-    for (int r = 0; r < 2; r++) {
-        if (SPLIT > 1 && (uint32_t)r != part) continue;
+    for (int both = 0; both < (SPLIT > 1 ? 1 : 2); both++) {
+        const uint32_t r = SPLIT > 1 ? part : (uint32_t)both;
         typename A::V v[4];
-        uint64_t parts[SPLIT][4];
-        if constexpr (SPLIT > 1) {
-#pragma unroll
-            for (int i = 0; i < SPLIT; i++) load_pairs(parts[i], sums_lds + (2 * i + r) * 256 + pair_lane(lane));
-        }
         if (SPLIT == 1) fetch_addends(r);
         if constexpr (FP) {
             const FpMod m = ar.m;
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (SPLIT > 1) {
-                    v[j] = 0.0;
+            for (int j = 0; j < 4; j++) v[j] = SPLIT > 1 ? 0.0 : sums.s[both][j];
+            if constexpr (SPLIT > 1) {
 #pragma unroll
-                    for (int i = 0; i < SPLIT; i++) v[j] += A::from_word(parts[i][j]);
-                } else {
-                    v[j] = sums.s[r][j];
+                for (int i = 0; i < SPLIT; i++) {
+                    uint64_t w[4];
+                    load_pairs(w, sums_lds + (2 * i + r) * 256 + pair_lane(lane));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] += A::from_word(w[j]);
                 }
             }
             if (add && r == 0) {
@@ -688,16 +697,24 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
             for (int j = 0; j < 4; j++) v[j] = fp_canonical(v[j], m);
         } else {
             const uint64_t q = ar.m.q;
+            U128 total[4];
 #pragma unroll
-            for (int j = 0; j < 4; j++) {
-                if constexpr (SPLIT > 1) {
-                    v[j] = parts[0][j];
+            for (int j = 0; j < 4; j++) total[j] = SPLIT > 1 ? U128{0, 0} : sums.s[both][j];
+            if constexpr (SPLIT > 1) {
 #pragma unroll
-                    for (int i = 1; i < SPLIT; i++) v[j] = add_mod(v[j], parts[i][j], q);
-                } else {
-                    v[j] = barrett128(sums.s[r][j].lo, sums.s[r][j].hi, q, r0, r1);
+                for (int i = 0; i < SPLIT; i++) {
+                    uint64_t lo[4], hi[4];
+                    load_pairs(lo, sums_lds + (4 * i + 2 * r) * 256 + pair_lane(lane));
+                    load_pairs(hi, sums_lds + (4 * i + 2 * r + 1) * 256 + pair_lane(lane));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        total[j].lo += lo[j];
+                        total[j].hi += hi[j] + (total[j].lo < lo[j]);
+                    }
                 }
             }
+#pragma unroll
+            for (int j = 0; j < 4; j++) v[j] = barrett128(total[j].lo, total[j].hi, q, r0, r1);
             if (add && r == 0) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = add_mod(v[j], mul_shoup(c0[j], add_w, q), q);
@@ -733,7 +750,7 @@ constexpr int kInnerWaves = 4;
 
 template <int BE, int SPLIT, bool STREAM, class X>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PARAMS, X x) {
-    __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? 2 * SPLIT * 256 : 1];
+    __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? (BE == NTT_BACKEND_FP ? 2 : 4) * SPLIT * 256 : 1];
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
     set_inverse_block(a, x.itw);
