@@ -1,6 +1,6 @@
-"""Fused base conversions whose inputs the inverse rows pass leaves in the conversion's own order (N = 2^16, ten limbs of Ql u P and more)
-against the oracle, on every back end, on both sides of the line, with partial last digits, with scratch that is too small for the order
-(L < K: natural order in ModDown), and where data limbs and conversion run on different arithmetic."""
+"""Fused base conversions whose inputs the inverse rows pass leaves in the conversion's own order (N = 2^16, from 10 limbs of Ql u P on, 12 on
+FP64) against the oracle, on every back end, on both sides of the line, with partial last digits, with scratch that is too small for the
+order (the merged ModDown + rescale of one digit), and where data limbs and conversion run on different arithmetic."""
 import ctypes
 
 import numpy as np
@@ -11,9 +11,9 @@ from gpu_util import DeviceArray, make_pair, rand_limbs
 pytestmark = pytest.mark.gpu
 
 CASES = [  # bits, size_p, levels
-    ([50] * 8 + [50] * 4, 4, (8, 6, 5)),              # FP64: 12, 10 (half a digit) and 9 limbs (natural order)
-    ([50] * 8 + [50] * 8, 8, (8, 3)),                 # one digit: scratch for ModDown's inputs but not for the merged one's, and for neither
-    ([60] + [40] * 7 + [60] * 4, 4, (8, 6)),          # integer conversion, limbs of both arithmetics
+    ([50] * 12 + [50] * 4, 4, (10, 8, 7)),            # FP64: 14 (half a digit), 12 and 11 limbs (natural order)
+    ([50] * 8 + [50] * 8, 8, (8, 6)),                 # one digit: scratch for ModDown's inputs but not for the merged one's, and for neither
+    ([60] + [40] * 7 + [60] * 4, 4, (8, 6, 5)),       # integer conversion, limbs of both arithmetics; 5: natural order
     ([60] * 8 + [60] * 2, 2, (8, 7)),                 # integers throughout: 10 limbs, and 9
     ([45] * 8 + [60] * 4, 4, (7,)),                   # inverse transform of the data limbs on FP64 in front of an integer conversion
 ]
@@ -60,7 +60,7 @@ def test_key_switches_with_tiled_conversions(oracle, capi, bits, size_p, levels)
         assert (drot.numpy() == np.stack([p.add(p.galois_ntt(ct[0], elt), md[0]), md[1]])).all(), L
 
 
-@pytest.mark.parametrize("bits,size_p,L", [([50] * 10, 2, 8), ([60] + [40] * 7 + [60] * 2, 2, 8), ([50] * 16, 8, 4)])
+@pytest.mark.parametrize("bits,size_p,L", [([50] * 12, 2, 10), ([60] + [40] * 7 + [60] * 2, 2, 8), ([50] * 16, 8, 4)])
 def test_encryption_with_tiled_conversion(oracle, capi, bits, size_p, L):
     """ModDown's inputs lie where the encrypted u was, or in natural order where that is too short (L < K)."""
     cahel, parms, ctx, p = make_pair(oracle, 16, bits, size_p)
