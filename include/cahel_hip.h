@@ -382,6 +382,12 @@ size_t he_encrypt_batch_workspace_words(const he_context *ctx, uint32_t L, uint3
 int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
                      uint64_t stream_id, uint64_t *cts, uint64_t *workspace, he_stream stream);
 
+/* he_encrypt_batch in two calls on one stream and one workspace: what needs no plaintext (the device may be at it while the
+ * caller still prepares the messages), then the division by P onto the plaintexts in cts. */
+int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
+                     uint64_t stream_id, uint64_t *workspace, he_stream stream);
+int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *workspace, he_stream stream);
+
 /* One encryption of plain [L][N] (NTT form) into ct [2][L][N]: he_encrypt_batch of one item without the copy of the plaintext.
  * workspace: he_encrypt_batch_workspace_words(ctx, L, 1) words. */
 int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],

@@ -1642,35 +1642,50 @@ size_t he_encrypt_batch_workspace_words(const he_context *ctx, uint32_t L, uint3
 
 namespace {
 
-// plain: [items] plaintexts plain_stride limbs apart; nullptr: they lie in polynomial 0 of the ciphertexts
-int encrypt_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],
-                 uint64_t stream_id, uint64_t *cts, uint64_t *ws, he_stream s) {
-    if (!ctx || !pk || !key || !cts || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q || items == 0 || items > 8192)
-        return HE_E_INVALID_ARGUMENT;
-    const size_t n = ctx->n();
+bool encrypt_arguments_ok(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *ws) {
+    return ctx && ws && ctx->size_p != 0 && L != 0 && L <= ctx->size_q && items != 0 && items <= 8192;
+}
+
+// Workspace of `items` encryptions: u and wide one after the other, 3 * items polynomials of the same limbs, then ModDown's scratch
+struct EncryptWorkspace {
+    uint64_t *u, *wide, *tmp;
+};
+
+EncryptWorkspace encrypt_workspace(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *ws) {
+    const size_t words = (size_t)items * (L + ctx->size_p) * ctx->n();
+    return EncryptWorkspace{ws, ws + words, ws + 3 * words};
+}
+
+// (u pk_0 + e_0, u pk_1 + e_1) of every item, into the workspace
+int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8], uint64_t stream_id, uint64_t *ws,
+                  he_stream s) {
     const uint32_t K = ctx->size_p, Q = ctx->size_q, LK = L + K;
-    // u and wide lie one after the other: 3 * items polynomials of the same limbs
-    uint64_t *u = ws, *wide = u + (size_t)items * LK * n, *tmp = wide + (size_t)items * 2 * LK * n;
+    const EncryptWorkspace w = encrypt_workspace(ctx, L, items, ws);
     ChaChaKey k;
     memcpy(k.k, key, sizeof(k.k));
     // item k draws u, e0, e1 from the stream ids stream_id + 3 k, + 1, + 2: what `items` encryptions in a row draw.  The
     // samples stay bytes (in ModDown's scratch, which is written later) until the transform reads them.
-    int8_t *small = reinterpret_cast<int8_t *>(tmp);
+    int8_t *small = reinterpret_cast<int8_t *>(w.tmp);
     HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, small, items, S(s)));
     const int backend = backend_for_level(ctx, L);
     NttArgs a = base_args(ctx, true);
-    a.out = u;
+    a.out = w.u;
     a.out_poly_stride = LK;
     a.map = LimbMap{LK, 0, L, Q};
     a.pro_mode = NTT_PRO_SMALL;
-    a.pro_src = tmp;
+    a.pro_src = w.tmp;
     a.pro_itw = ctx->d_ipsi;
     a.pro_itw_fp = ctx->d_ipsi_fp;
     HE_HIP(launch_ntt_rows(a, 3 * items * LK, true, backend, S(s)));
     HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
-    // divide by P onto the plaintexts
-    return moddown_impl(ctx, L, wide, cts, 2 * items, 0x55555555u, tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
-                        plain ? L : 0, u, (size_t)items * LK);
+    return HE_OK;
+}
+
+// ... divided by P onto the plaintexts.  plain: that of one item; nullptr: they lie in polynomial 0 of the ciphertexts
+int encrypt_onto(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, uint64_t *cts, uint64_t *ws, he_stream s) {
+    const EncryptWorkspace w = encrypt_workspace(ctx, L, items, ws);
+    return moddown_impl(ctx, L, w.wide, cts, 2 * items, 0x55555555u, w.tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
+                        plain ? L : 0, w.u, (size_t)items * (L + ctx->size_p));
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
@@ -1741,15 +1756,29 @@ int decrypt_decode_impl(const he_context *ctx, const uint64_t *const *d_cts, uin
 
 extern "C" {
 
+int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8], uint64_t stream_id,
+                     uint64_t *ws, he_stream s) {
+    if (!encrypt_arguments_ok(ctx, L, items, ws) || !pk || !key) return HE_E_INVALID_ARGUMENT;
+    return encrypt_zeros(ctx, L, items, pk, key, stream_id, ws, s);
+}
+
+int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *ws, he_stream s) {
+    if (!encrypt_arguments_ok(ctx, L, items, ws) || !cts) return HE_E_INVALID_ARGUMENT;
+    return encrypt_onto(ctx, L, items, nullptr, cts, ws, s);
+}
+
 int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
                      uint64_t stream_id, uint64_t *cts, uint64_t *ws, he_stream s) {
-    return encrypt_impl(ctx, L, items, nullptr, pk, key, stream_id, cts, ws, s);
+    if (!encrypt_arguments_ok(ctx, L, items, ws) || !pk || !key || !cts) return HE_E_INVALID_ARGUMENT;
+    if (int rc = encrypt_zeros(ctx, L, items, pk, key, stream_id, ws, s)) return rc;
+    return encrypt_onto(ctx, L, items, nullptr, cts, ws, s);
 }
 
 int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],
                uint64_t stream_id, uint64_t *ct, uint64_t *ws, he_stream s) {
-    if (!plain) return HE_E_INVALID_ARGUMENT;
-    return encrypt_impl(ctx, L, 1, plain, pk, key, stream_id, ct, ws, s);
+    if (!encrypt_arguments_ok(ctx, L, 1, ws) || !plain || !pk || !key || !ct) return HE_E_INVALID_ARGUMENT;
+    if (int rc = encrypt_zeros(ctx, L, 1, pk, key, stream_id, ws, s)) return rc;
+    return encrypt_onto(ctx, L, 1, plain, ct, ws, s);
 }
 
 int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t size, uint32_t limbs, const uint64_t *sk, size_t sk_stride,

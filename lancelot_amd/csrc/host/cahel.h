@@ -166,6 +166,12 @@ public:
     void set_seed(uint64_t seed);
     const uint32_t *prng_key() const { return prng_key_; }
     uint64_t next_stream(uint64_t count = 1) const { return prng_stream_.fetch_add(count, std::memory_order_relaxed); }
+    // ids of a call that was refused before anything drawn from them left it, if no other call has taken any since: the next
+    // call draws what it would have drawn without the refused one
+    void give_back_streams(uint64_t first, uint64_t count) const {
+        uint64_t last = first + count;
+        prng_stream_.compare_exchange_strong(last, first, std::memory_order_relaxed);
+    }
     const uint64_t *gauss_cdt() const { return gauss_cdt_.get(); }
     uint32_t gauss_cdt_len() const { return gauss_cdt_len_; }
 
@@ -474,10 +480,19 @@ public:
     }
 
 private:
-    int batch_bits(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const;
-    std::vector<CAHELGPUCiphertext> encode_encrypt_staged(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
-                                                          const double *d_values, bool small, std::size_t items, std::size_t count,
-                                                          std::size_t slots, double scale, int total_bits);
+    // a batch on its way: the encryptions' random part is on the device's queue before the messages are copied
+    struct Batch {
+        std::size_t items;
+        double scale;
+        int total_bits;
+        uint64_t stream_id;
+        cahel::DeviceBuffer cts, ws;
+    };
+    void check_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const;
+    Batch begin_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale);
+    // d_values: [items][count] on the device; small: no coefficient can reach the bounds
+    std::vector<CAHELGPUCiphertext> end_batch(const CAHELGPUContext &context, Batch batch, const double *d_values, bool small,
+                                              std::size_t count, std::size_t slots);
     std::size_t slots_ = 0, sparse_slots_ = 0;
     std::size_t first_chain_index_ = 1;  // include/ckks.h:325
 };

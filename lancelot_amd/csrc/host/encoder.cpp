@@ -75,8 +75,9 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_many(const C
                                                                          std::size_t value_stride, double scale) {
     if (items == 0) return {};
     if (count > slots_ || value_stride < count) throw std::invalid_argument("values_size is too large");
-    const int total_bits = batch_bits(context, pk, items, scale);
+    check_batch(context, pk, items, scale);
     const std::size_t ss = message_slots(count);
+    Batch batch = begin_batch(context, pk, items, scale);
     he_stream st = context.stream();
 
     // values -> device, packed, some messages at a time through page-locked memory (the next ones are copied while the last
@@ -90,12 +91,12 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_many(const C
         const std::size_t taken = std::min(rows, items - first), bytes = taken * count * sizeof(double);
         double *host = static_cast<double *>(ring.take(bytes));
         for (std::size_t k = 0; k < taken; k++)
-            small = surely_small(copy_sum(host + k * count, values + (first + k) * value_stride, count), scale, ss, total_bits) && small;
+            small = surely_small(copy_sum(host + k * count, values + (first + k) * value_stride, count), scale, ss, batch.total_bits) && small;
         const int status = he_memcpy_h2d_async(d_values + first * count, host, bytes, st);
         ring.fence(st);
         check_status(status, "upload");
     }
-    return encode_encrypt_staged(context, pk, d_values, small, items, count, ss, scale, total_bits);
+    return end_batch(context, std::move(batch), d_values, small, count, ss);
 }
 
 std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_updates(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
@@ -105,8 +106,9 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_updates(cons
     const std::size_t chunks = (length + slots_ - 1) / slots_;
     if (chunks > 8192 || rows.size() > 8192) throw std::invalid_argument("too many messages");
     const std::size_t items = rows.size() * chunks, padded = chunks * slots_;
-    const int total_bits = batch_bits(context, pk, items, scale);
+    check_batch(context, pk, items, scale);
     const std::size_t ss = message_slots(slots_);
+    Batch batch = begin_batch(context, pk, items, scale);
     he_stream st = context.stream();
     // the floats as they are, row after row, some messages at a time through page-locked memory; the device widens them
     const std::size_t total = rows.size() * length;
@@ -130,58 +132,68 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_updates(cons
             const std::size_t taken = std::min(slots_, length - at);
             if (filled + taken > room) send();
             if (filled == 0) host = static_cast<float *>(ring.take(room * sizeof(float)));
-            small = surely_small(copy_sum(host + filled, row + at, taken), scale, ss, total_bits) && small;
+            small = surely_small(copy_sum(host + filled, row + at, taken), scale, ss, batch.total_bits) && small;
             filled += taken;
         }
     send();
     check_status(he_widen_rows(d_floats, d_values, (uint32_t)rows.size(), length, padded, st), "he_widen_rows");
-    return encode_encrypt_staged(context, pk, d_values, small, items, slots_, ss, scale, total_bits);
+    return end_batch(context, std::move(batch), d_values, small, slots_, ss);
 }
 
-// the modulus' bits at the level where batches are encrypted, if this one can be
-int CAHELGPUCKKSEncoder::batch_bits(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const {
+// what a batch needs of its key, level and scale
+void CAHELGPUCKKSEncoder::check_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const {
     if (items > 8192) throw std::invalid_argument("too many messages");
     if (!pk.gen_flag_) throw std::logic_error("public key has not been generated");
     if (first_chain_index_ == 0 || context.size_p() == 0) throw std::logic_error("batched encryption needs a data level and special primes");
-    const int total_bits = context.total_coeff_modulus_bit_count(first_chain_index_);
-    if (scale <= 0 || (static_cast<int>(std::log2(scale)) + 1 >= total_bits)) throw std::invalid_argument("scale out of bounds");
-    return total_bits;
+    if (scale <= 0 || (static_cast<int>(std::log2(scale)) + 1 >= context.total_coeff_modulus_bit_count(first_chain_index_)))
+        throw std::invalid_argument("scale out of bounds");
 }
 
-// d_values: [items][count] on the device; small: no coefficient can reach the bounds
-std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::encode_encrypt_staged(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk,
-                                                                           const double *d_values, bool small, std::size_t items,
-                                                                           std::size_t count, std::size_t ss, double scale, int total_bits) {
-    const std::size_t n = context.poly_degree(), chain = first_chain_index_;
+CAHELGPUCKKSEncoder::Batch CAHELGPUCKKSEncoder::begin_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items,
+                                                            double scale) {
+    const uint32_t L = (uint32_t)context.limbs_at(first_chain_index_);
+    he_context *h = context.handle();
+    Batch batch{items, scale, context.total_coeff_modulus_bit_count(first_chain_index_), 0,
+                DeviceBuffer(items * 2 * (std::size_t)L * context.poly_degree()),
+                DeviceBuffer(he_encrypt_batch_workspace_words(h, L, (uint32_t)items))};
+    batch.stream_id = context.next_stream(3 * items);
+    check_status(he_encrypt_begin(h, L, (uint32_t)items, pk.pk_.data(), context.prng_key(), batch.stream_id, batch.ws.get(), context.stream()),
+                 "he_encrypt_begin");
+    return batch;
+}
+
+std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::end_batch(const CAHELGPUContext &context, Batch batch, const double *d_values, bool small,
+                                                               std::size_t count, std::size_t ss) {
+    const std::size_t n = context.poly_degree(), chain = first_chain_index_, items = batch.items;
     const uint32_t L = (uint32_t)context.limbs_at(chain);
+    const double scale = batch.scale;
     he_context *h = context.handle();
     he_stream st = context.stream();
     // plaintexts straight into polynomial 0 of the ciphertexts
     const std::size_t words = 2 * (std::size_t)L * n;
-    DeviceBuffer batch(items * words), ws(he_ckks_encode_batch_workspace_words(h, (uint32_t)items));
+    DeviceBuffer ws(he_ckks_encode_batch_workspace_words(h, (uint32_t)items));
     if (small) {
         check_status(he_ckks_encode_bounded(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
-                                            batch.get(), 2 * L, ws.get(), st),
+                                            batch.cts.get(), 2 * L, ws.get(), st),
                      "he_ckks_encode_bounded");
     } else {
         check_status(he_ckks_encode_batch(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
-                                          batch.get(), 2 * L, ws.get(), st),
+                                          batch.cts.get(), 2 * L, ws.get(), st),
                      "he_ckks_encode_batch");
         std::vector<double> maxima(items);
         check_status(he_memcpy_d2h(maxima.data(), ws.get(), items * sizeof(double), st), "download");
         for (double max_coeff : maxima) {
             const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
-            if (max_coeff_bit_count >= total_bits || max_coeff_bit_count > 63)
+            if (max_coeff_bit_count >= batch.total_bits || max_coeff_bit_count > 63) {
+                context.give_back_streams(batch.stream_id, 3 * items);
                 throw std::invalid_argument("encoded values are too large");
+            }
         }
     }
-    DeviceBuffer ews(he_encrypt_batch_workspace_words(h, L, (uint32_t)items));
-    check_status(he_encrypt_batch(h, L, (uint32_t)items, pk.pk_.data(), context.prng_key(), context.next_stream(3 * items),
-                                  batch.get(), ews.get(), st),
-                 "he_encrypt_batch");
+    check_status(he_encrypt_end(h, L, (uint32_t)items, batch.cts.get(), batch.ws.get(), st), "he_encrypt_end");
     // one ciphertext object per message, each a slice of the batch (no copies)
     std::vector<CAHELGPUCiphertext> out(items);
-    auto shared = std::make_shared<DeviceBuffer>(std::move(batch));
+    auto shared = std::make_shared<DeviceBuffer>(std::move(batch.cts));
     for (std::size_t k = 0; k < items; k++) {
         CAHELGPUCiphertext &ct = out[k];
         ct.adopt(DeviceBuffer::slice(shared, k * words, words));

@@ -159,6 +159,10 @@ int he_ckks_encode(const he_context *, const double *, const double *, uint32_t,
 int he_ckks_encode_batch(const he_context *, const double *, const double *, uint32_t, uint32_t, double, uint32_t, uint32_t, size_t,
                          uint64_t *, uint32_t, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
 size_t he_encrypt_batch_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
+int he_encrypt_begin(const he_context *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, he_stream) {
+    return HE_E_UNSUPPORTED;
+}
+int he_encrypt_end(const he_context *, uint32_t, uint32_t, uint64_t *, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
 int he_encrypt_batch(const he_context *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, uint64_t *,
                      he_stream) { return HE_E_UNSUPPORTED; }
 size_t he_ckks_workspace_words(const he_context *, uint32_t) { return 0; }
