@@ -1483,8 +1483,32 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     fwd.w = lv->d_qlast_inv;
     fwd.epi_dst = out;
     fwd.epi_dst_poly_stride = L - 1;
+    if (tin && tin->last_only) {
+        if (!fused) HE_HIP(launch_ntt_rows(fwd, polys * (L - 1), true, backend_for(ctx, fwd.map, (int)L - 1), S(s)));
+        const ProductEnd end{cx, tin->ct1, tin->ct2, out, fwd.pro_w, fwd.w, L, LK, tin->square};
+        HE_HIP(launch_product_end(fwd, end, items, backend_for(ctx, fwd.map, (int)L - 1), S(s)));
+        return HE_OK;
+    }
     HE_HIP(launch_ntt_forward(fwd, polys, backend_for(ctx, fwd.map, (int)L - 1), S(s), fused));
     return HE_OK;
+}
+
+// Whether a product's last pass forms (d0, d1) from the factors itself (ProductEnd), not the first: 214 MB less of 3.5 GB for eight products
+// of 24 + 8 limbs of 2^16 words, but both polynomials of a limb are one wave's, and few waves take longer.  From 2^19 words a polynomial
+// of the whole batch on, 2^20 with integers alone, which issue as much as before and move less of it (products, us in the first pass / in the
+// last; FP64: 8 x 24 + 8 limbs of 2^16 words 776 / 745, 1 x 130.5 / 125.3, 16 x 3 + 1 192.5 / 182.3, 1 x 8 + 1 68.5 / 67.4, 4 x 5 + 1 of 2^15
+// 61.4 / 58.3, 2 x 5 + 1 42.7 / 43.0, 8 x 12 + 4 of 2^14 109.4 / 102.6, 2 x 8 + 2 37.2 / 37.7, 8 x 4 + 1 48.3 / 47.4, 32 x 6 + 2 of 2^13 104.9 /
+// 97.5, 4 x 8 + 1 41.2 / 41.1; 60 / 40 bits: 8 x 24 + 8 of 2^16 1121 / 1088, 1 x 8 + 2 72.4 / 71.8, 2 x 8 + 2 of 2^15 77.2 / 75.5, 1 x 8 + 2
+// 50.0 / 51.4, 8 x 4 + 1 of 2^14 62.0 / 61.3, 4 x 4 + 1 44.4 / 45.4; 60 bits: 8 x 24 + 8 of 2^16 1260 / 1233, 2 x 8 + 2 140.0 / 136.2, 1 x 8 + 2
+// 81.4 / 81.3, 8 x 8 + 2 of 2^14 119.5 / 118.5, 8 x 4 + 1 68.4 / 68.5, 4 x 4 + 1 49.5 / 51.9, 32 x 4 + 1 of 2^12 63.5 / 64.5).  The factors are
+// then read until the end: a result that lies over them (which is allowed) is written from (d0, d1) in the workspace.
+bool end_from_factors(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *ct1, const uint64_t *ct2, const uint64_t *out) {
+    const bool integers = backend_for(ctx, plain_map(L - 1, 0), (int)L - 1) == NTT_BACKEND_INT;
+    if (((uint64_t)items * L << ctx->log_n) < (uint64_t)(integers ? 16 : 8) << 16) return false;
+    const uintptr_t limb = ctx->n() * sizeof(uint64_t), size = (uintptr_t)items * 2 * L * limb, o = (uintptr_t)out;
+    const uintptr_t o_size = (uintptr_t)items * 2 * (L - 1) * limb;
+    auto apart = [&](const uint64_t *ct) { return o + o_size <= (uintptr_t)ct || (uintptr_t)ct + size <= o; };
+    return apart(ct1) && apart(ct2);
 }
 
 }  // namespace
@@ -1511,7 +1535,7 @@ int he_multiply_relin_rescale(const he_context *ctx, uint32_t L, const uint64_t 
     const size_t n = ctx->n();
     uint64_t *d01 = ws + he_keyswitch_workspace_words(ctx, L), *d2 = d01 + 2 * (size_t)L * n;
     if (tensor_fusion_ok(ctx, 1)) {
-        const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0};
+        const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0, end_from_factors(ctx, L, 1, ct1, ct2, out)};
         return ksr_impl(ctx, L, 1, d2, L, evk, d01, out, 0, ws, s, &tin);
     }
     // (d0, d1 | d2) are contiguous: the layout of he_tensor's output
@@ -1538,7 +1562,7 @@ int he_multiply_relin_rescale_batch(const he_context *ctx, uint32_t L, uint32_t 
     // [items] key-switch workspaces | (d0, d1) [items][2][L][N] | d2 [items][L][N]
     uint64_t *d01 = ws + (size_t)items * he_keyswitch_workspace_words(ctx, L), *d2 = d01 + (size_t)items * 2 * L * n;
     if (tensor_fusion_ok(ctx, items)) {
-        const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0};
+        const TensorFuse tin{ct1, ct2, d01, d2, L, ct1 == ct2 ? 1 : 0, end_from_factors(ctx, L, items, ct1, ct2, out)};
         return ksr_impl(ctx, L, items, d2, L, evk, d01, out, 0, ws, s, &tin);
     }
     HE_HIP(launch_tensor(ctx->tables(), ct1, ct2, d01, L, ct1 == ct2, S(s),

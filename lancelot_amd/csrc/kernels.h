@@ -227,8 +227,22 @@ struct TensorFuse {
     uint64_t *d2;                // [L][N]: d2 in NTT form
     uint32_t L;
     int square;                  // ct2 is ignored, (d0, d1, d2) = (a0^2, 2 a0 a1, a1^2)
+    int last_only;               // of d0 and d1 only limb L - 1 is formed (launch_product_end forms the others)
 };
 hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint32_t items, int backend, hipStream_t s);
+
+// The last blocks pass of a product with relinearisation and rescale: out_r = (cx_r P^-1 + d_r - NTT(delta_r)) q_last^-1 on the limbs
+// 0 .. L - 2 of both polynomials, with (d0, d1) = (a0 b0, a0 b1 + a1 b0) formed here from the factors.  `a`: forward base arguments, out = the
+// rows pass's words [items][2][L][N], map = the L - 1 limbs.
+struct ProductEnd {
+    const uint64_t *cx;          // [items][2][cx_stride][N]
+    const uint64_t *ct1, *ct2;   // [items][2][L][N]
+    uint64_t *out;               // [items][2][L - 1][N]
+    const uint64_t *p_inv, *q_last_inv;   // Shoup pairs, by limb
+    uint32_t L, cx_stride;
+    int square;
+};
+hipError_t launch_product_end(const NttArgs &a, const ProductEnd &x, uint32_t items, int backend, hipStream_t s);
 
 struct Tables {
     const uint64_t *moduli;

@@ -817,6 +817,22 @@ __device__ __forceinline__ void tensor4(const IntArith &ar, const NttArgs &a, ui
     }
 }
 
+// x y mod q of four canonical words: as the arithmetic's values and as words, canonical
+__device__ __forceinline__ void product4(const FpArith &ar, const NttArgs &, uint32_t, const uint64_t *x, const uint64_t *y, double *d, uint64_t *w) {
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        d[j] = fp_canonical(fp_mulmod(fp_from_u64(x[j]), fp_from_u64(y[j]), ar.m), ar.m);
+        w[j] = fp_to_u64(d[j]);
+    }
+}
+
+__device__ __forceinline__ void product4(const IntArith &ar, const NttArgs &a, uint32_t table, const uint64_t *x, const uint64_t *y, uint64_t *d,
+                                         uint64_t *w) {
+    const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
+#pragma unroll
+    for (int j = 0; j < 4; j++) w[j] = d[j] = mul_mod(x[j], y[j], ar.m.q, r0, r1);
+}
+
 // Tensor product fused with the blocks pass of the inverse transform of its third polynomial: a wave forms the three products
 // of one block of 256 words, stores them (d2 in NTT form is what the key switch multiplies by its own digit's key) and takes d2
 // through the 8 inverse stages; the lazy words are left in a.out for the rows pass.  One read of d2 and one launch less
@@ -868,19 +884,130 @@ __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse 
     for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(d2[j]);
 }
 
-template <int BE>
+// the third polynomial alone (TensorFuse::last_only)
+template <class A>
+__device__ __forceinline__ void third_block(const NttArgs &a, const TensorFuse &x, const Job &job, const A &ar, uint32_t blk, uint32_t lane) {
+    using T4 = Tile4<8, 8>;
+    const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + pair_lane(lane);
+    const size_t ct = (2 * job.poly + 1) * poly + job.limb * n + at;
+    uint64_t a1[4], b1[4];
+    load_pairs(a1, x.ct1 + ct);
+    load_pairs(b1, (x.square ? x.ct1 : x.ct2) + ct);
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    typename A::V d2[4];
+    uint64_t w[4];
+    product4(ar, a, job.table, a1, b1, d2, w);
+    store_pairs(x.d2 + job.poly * poly + job.limb * n + at, w);
+    turn_pairs(d2);
+    T4::template inverse<A>(d2, tw, ar, nullptr, lane);
+#pragma unroll
+    for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(d2[j]);
+}
+
+template <int BE, bool LAST_ONLY>
 __global__ __launch_bounds__(64 * kBlockWaves) void tensor_intt_blocks_kernel(HE_HEAD_PARAMS, const uint64_t *ct2, uint64_t *d01, uint64_t *d2) {
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
-    const TensorFuse x{h_in, ct2, d01, d2, a.map.limbs, (int)h5};
+    const TensorFuse x{h_in, ct2, d01, d2, a.map.limbs, (int)h5, LAST_ONLY};
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
     const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) tensor_block(a, x, job, fp_arith(a, job.table), blk, lane);
+    auto block = [&](const auto &ar) {
+        if (LAST_ONLY && job.limb + 1 != a.map.limbs)
+            third_block(a, x, job, ar, blk, lane);
+        else
+            tensor_block(a, x, job, ar, blk, lane);
+    };
+    if (BE != NTT_BACKEND_INT && fp) block(fp_arith(a, job.table));
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) tensor_block(a, x, job, int_arith(a, job.table), blk, lane);
+        if (!fp) block(int_arith(a, job.table));
+    }
+}
+
+// out = (c P^-1 + d - v) q_last^-1 of four words: v as the forward stages have left it, d = x y or x y + z w of canonical words
+__device__ __forceinline__ void end4(const FpArith &ar, const NttArgs &, uint32_t, const double *v, const uint64_t *c, const uint64_t *x, const uint64_t *y,
+                                     const uint64_t *z, const uint64_t *w, Shoup p_inv, Shoup q_inv, uint64_t *out) {
+    const FpMod m = ar.m;
+    const double pw = fp_from_u64(p_inv.w), ew = fp_from_u64(q_inv.w);
+    // (three products below q, less a word of at most 3.7 q: below 8 q)
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        double d = fp_mulmod(fp_from_u64(c[j]), pw, m) + fp_mulmod(fp_from_u64(x[j]), fp_from_u64(y[j]), m);
+        if (z) d += fp_mulmod(fp_from_u64(z[j]), fp_from_u64(w[j]), m);
+        out[j] = fp_to_u64(fp_canonical(fp_mulmod(d - v[j], ew, m), m));
+    }
+}
+
+__device__ __forceinline__ void end4(const IntArith &ar, const NttArgs &a, uint32_t table, const uint64_t *v, const uint64_t *c, const uint64_t *x,
+                                     const uint64_t *y, const uint64_t *z, const uint64_t *w, Shoup p_inv, Shoup q_inv, uint64_t *out) {
+    const uint64_t q = ar.m.q, r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        U128 d{0, 0};
+        mac128(d, x[j], y[j]);
+        if (z) mac128(d, z[j], w[j]);
+        const uint64_t lhs = add_mod(mul_shoup(c[j], p_inv, q), barrett128(d.lo, d.hi, q, r0, r1), q);
+        out[j] = mul_shoup(sub_mod(lhs, reduce_6q(v[j], q), q), q_inv, q);
+    }
+}
+
+// A product's last pass (ProductEnd): a wave takes one block of both polynomials, so that it reads the four factors once.  Bound by memory:
+// the factors are read again (four polynomials) in place of d0 and d1 (two), which the first pass then neither forms nor stores, and for which
+// it does not read two of the factors.  Eight products of 24 + 8 limbs of 2^16 words, the first and the last pass: 140 + 163 us -> @T@ + @E@.
+template <class A>
+__device__ __forceinline__ void product_end_block(const NttArgs &a, const ProductEnd &x, const Job &job, const A &ar, uint32_t blk,
+                                                  uint32_t lane) {
+    using T4 = Tile4<8, 8>;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane), item = job.poly;
+    const size_t ct = (2 * item * x.L + job.limb) * n + at, poly = (size_t)x.L * n;
+    const uint64_t *cx = x.cx + (2 * item * x.cx_stride + job.limb) * n + at, *ct2 = x.square ? x.ct1 : x.ct2;
+    uint64_t lazy[2][4], c[2][4], f[2][4], g[2][4];
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) lazy[r][j] = job.out[r * poly + off + T4::word(0, lane, j)];
+    }
+    typename A::Tw tw[4];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        load_pairs(c[r], cx + r * (size_t)x.cx_stride * n);
+        load_pairs(f[r], x.ct1 + ct + r * poly);
+        load_pairs(g[r], ct2 + ct + r * poly);
+    }
+    const Shoup p_inv = scalar_shoup(x.p_inv, job.limb), q_inv = scalar_shoup(x.q_last_inv, job.limb);
+    uint64_t *out = x.out + (2 * item * (x.L - 1) + job.limb) * n + at;
+#pragma unroll
+    for (int r = 0; r < 2; r++) {
+        typename A::V v[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) v[j] = A::from_word(lazy[r][j]);
+        T4::template forward<A>(v, tw, ar, nullptr, lane);
+        turn_pairs(v);
+        uint64_t o[4];
+        if (r == 0)
+            end4(ar, a, job.table, v, c[0], f[0], g[0], nullptr, nullptr, p_inv, q_inv, o);
+        else
+            end4(ar, a, job.table, v, c[1], f[0], g[1], f[1], g[0], p_inv, q_inv, o);
+        store_pairs(out + r * (size_t)(x.L - 1) * n, o);
+    }
+}
+
+template <int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_PARAMS, ProductEnd x) {
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
+    const Job job = decode_job(a, id >> lr);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
+    if (BE != NTT_BACKEND_INT && fp) product_end_block(a, x, job, fp_arith(a, job.table), blk, lane);
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) product_end_block(a, x, job, int_arith(a, job.table), blk, lane);
     }
 }
 
@@ -1388,12 +1515,39 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, u
     // 2^15 32.4 / 32.7, 8 x 10 of 2^13 62.5 / 61.9; 8 x 3 of 2^14 39.5 / 41.1, 8 x 8 of 2^12 58.7 / 61.6).
     a.spread = items > 1 && ((uint64_t)x.L * items << a.log_n) >= (uint64_t)(a.log_n >= 15 ? 6 : 10) << 16;
     const NttHead h = ntt_head(a, grid.x, x.square ? 1 : 0);
+#define HE_TENSOR(BE)                                                                                                             \
+    do {                                                                                                                          \
+        if (x.last_only)                                                                                                          \
+            hipLaunchKernelGGL((tensor_intt_blocks_kernel<BE, true>), grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);    \
+        else                                                                                                                      \
+            hipLaunchKernelGGL((tensor_intt_blocks_kernel<BE, false>), grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);   \
+    } while (0)
     if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
+        HE_TENSOR(NTT_BACKEND_MIXED);
     else if (backend)
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
+        HE_TENSOR(NTT_BACKEND_FP);
     else
-        hipLaunchKernelGGL(tensor_intt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(h), x.ct2, x.d01, x.d2);
+        HE_TENSOR(NTT_BACKEND_INT);
+#undef HE_TENSOR
+    return hipGetLastError();
+}
+
+hipError_t launch_product_end(const NttArgs &args, const ProductEnd &x, uint32_t items, int backend, hipStream_t s) {
+    NttArgs a = args;
+    a.in = nullptr;
+    a.out_poly_stride = 2 * x.L;   // (a job is both polynomials of a limb)
+    if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs + 1 != x.L || a.map.limbs == 0 || items == 0) return hipErrorInvalidValue;
+    const uint64_t wgs = ((uint64_t)a.map.limbs * items << (a.log_n - 8)) / kBlockWaves;
+    if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
+    const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
+    a.spread = items > 1;   // (as in launch_tensor_intt_blocks)
+    const NttHead h = ntt_head(a, grid.x, 0);
+    if (backend == NTT_BACKEND_MIXED)
+        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
+    else if (backend)
+        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
+    else
+        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
     return hipGetLastError();
 }
 
