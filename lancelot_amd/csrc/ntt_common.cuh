@@ -654,6 +654,14 @@ __device__ __forceinline__ void stream_pairs(uint64_t *v, const uint64_t *p) {
     v[3] = b.y;
 }
 
+template <bool STREAM>
+__device__ __forceinline__ void load_pairs_or_stream(uint64_t *v, const uint64_t *p) {
+    if constexpr (STREAM)
+        stream_pairs(v, p);
+    else
+        load_pairs(v, p);
+}
+
 __device__ __forceinline__ void store_pairs(uint64_t *p, const uint64_t *v) {
     reinterpret_cast<Words2 *>(p)[0] = Words2{v[0], v[1]};
     reinterpret_cast<Words2 *>(p + pair_word(2))[0] = Words2{v[2], v[3]};

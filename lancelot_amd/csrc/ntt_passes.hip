@@ -518,8 +518,8 @@ struct InnerMany {
 // FP64 kernel from 96 registers to 120).
 // SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
 // and waves 0 and 1 finish one polynomial each.
-// STREAM: the key words pass by the caches (launch_ntt_inner says when).
-template <int SPLIT, bool STREAM, class A, class X>
+// STREAM: 1: the key words pass by the caches; 2: the digits' words do, which nothing reads again; 3: both (launch_ntt_inner says when).
+template <int SPLIT, int STREAM, class A, class X>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32_t L, uint32_t LK, uint32_t beta, uint32_t t,
                                             uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
                                             uint64_t *sums_lds) {
@@ -539,16 +539,14 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
     };
     auto fetch = [&](uint64_t *w, uint32_t d) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) w[j] = lazy[d * digit_stride + T4::word(0, lane, j)];
+        for (int j = 0; j < 4; j++) {
+            const uint64_t *p = lazy + d * digit_stride + T4::word(0, lane, j);
+            w[j] = STREAM & 2 ? __builtin_nontemporal_load(p) : *p;
+        }
     };
     auto keys = [&](uint64_t (*k)[4], uint32_t d) {
-        if constexpr (STREAM) {
-            stream_pairs(k[0], x.evk[d] + key_off);
-            stream_pairs(k[1], x.evk[d] + key_poly + key_off);
-        } else {
-            load_pairs(k[0], x.evk[d] + key_off);
-            load_pairs(k[1], x.evk[d] + key_poly + key_off);
-        }
+        load_pairs_or_stream<(STREAM & 1) != 0>(k[0], x.evk[d] + key_off);
+        load_pairs_or_stream<(STREAM & 1) != 0>(k[1], x.evk[d] + key_poly + key_off);
     };
     typename A::Tw tw[4];
     uint64_t nx[4];
@@ -606,7 +604,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
 #pragma unroll
             for (int j = 0; j < 4; j++) c[j] = src[galois_index((uint32_t)at + pair_word(j), x.own_galois, a.log_n)];
         } else {
-            load_pairs(c, src + at);
+            load_pairs_or_stream<(STREAM & 2) != 0>(c, src + at);
         }
         typename A::V v[4];
 #pragma unroll
@@ -748,7 +746,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
 constexpr int kInnerWaves = 4;
 
-template <int BE, int SPLIT, bool STREAM, class X>
+template <int BE, int SPLIT, int STREAM, class X>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PARAMS, X x) {
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? (BE == NTT_BACKEND_FP ? 2 : 4) * SPLIT * 256 : 1];
     NttArgs a;
@@ -956,8 +954,10 @@ __device__ __forceinline__ void end4(const IntArith &ar, const NttArgs &a, uint3
 
 // A product's last pass (ProductEnd): a wave takes one block of both polynomials, so that it reads the four factors once.  Bound by memory:
 // the factors are read again (four polynomials) in place of d0 and d1 (two), which the first pass then neither forms nor stores, and for which
-// it does not read two of the factors.  Eight products of 24 + 8 limbs of 2^16 words, the first and the last pass: 140 + 163 us -> @T@ + @E@.
-template <class A>
+// it does not read two of the factors.  Eight products of 24 + 8 limbs of 2^16 words, the first and the last pass: 140 + 163 us -> 77
+// + 190, and 90 + 147 with words that pass by the caches.
+// STREAM: 1: the rows pass's words and the sums pass by the caches; 2: the factors do as well.
+template <int STREAM, class A>
 __device__ __forceinline__ void product_end_block(const NttArgs &a, const ProductEnd &x, const Job &job, const A &ar, uint32_t blk,
                                                   uint32_t lane) {
     using T4 = Tile4<8, 8>;
@@ -968,15 +968,18 @@ __device__ __forceinline__ void product_end_block(const NttArgs &a, const Produc
 #pragma unroll
     for (int r = 0; r < 2; r++) {
 #pragma unroll
-        for (int j = 0; j < 4; j++) lazy[r][j] = job.out[r * poly + off + T4::word(0, lane, j)];
+        for (int j = 0; j < 4; j++) {
+            const uint64_t *p = job.out + r * poly + off + T4::word(0, lane, j);
+            lazy[r][j] = STREAM ? __builtin_nontemporal_load(p) : *p;
+        }
     }
     typename A::Tw tw[4];
     T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
 #pragma unroll
     for (int r = 0; r < 2; r++) {
-        load_pairs(c[r], cx + r * (size_t)x.cx_stride * n);
-        load_pairs(f[r], x.ct1 + ct + r * poly);
-        load_pairs(g[r], ct2 + ct + r * poly);
+        load_pairs_or_stream<STREAM != 0>(c[r], cx + r * (size_t)x.cx_stride * n);
+        load_pairs_or_stream<STREAM == 2>(f[r], x.ct1 + ct + r * poly);
+        load_pairs_or_stream<STREAM == 2>(g[r], ct2 + ct + r * poly);
     }
     const Shoup p_inv = scalar_shoup(x.p_inv, job.limb), q_inv = scalar_shoup(x.q_last_inv, job.limb);
     uint64_t *out = x.out + (2 * item * (x.L - 1) + job.limb) * n + at;
@@ -996,7 +999,7 @@ __device__ __forceinline__ void product_end_block(const NttArgs &a, const Produc
     }
 }
 
-template <int BE>
+template <int BE, int STREAM>
 __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_PARAMS, ProductEnd x) {
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
@@ -1005,9 +1008,9 @@ __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_P
     const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) product_end_block(a, x, job, fp_arith(a, job.table), blk, lane);
+    if (BE != NTT_BACKEND_INT && fp) product_end_block<STREAM>(a, x, job, fp_arith(a, job.table), blk, lane);
     if constexpr (BE != NTT_BACKEND_FP) {
-        if (!fp) product_end_block(a, x, job, int_arith(a, job.table), blk, lane);
+        if (!fp) product_end_block<STREAM>(a, x, job, int_arith(a, job.table), blk, lane);
     }
 }
 
@@ -1428,6 +1431,14 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     return hipGetLastError();
 }
 
+// Words that are read for the last time pass by the caches (the digits' words and the sums of a product), from 2^20 words a polynomial of the
+// whole batch on: they leave the last-level cache to what the kernels behind them read.  Products, us with such words kept / passing by:
+// FP64: 8 x 24 + 8 limbs of 2^16 words 742 / 694, 4 x 389 / 364, 1 x 124.0 / 122.7, 16 x 12 + 4 695 / 648, 2 x 111.4 / 107.2, 2 x 8 + 2 85.5 / 83.3, 8 x
+// 12 + 4 of 2^15 186 / 175, 32 x 6 + 2 of 2^13 96.4 / 92.0; 60 / 40 bits: 8 x 12 + 4 of 2^16 456 / 435, 16 x 3 + 1 221 / 215; 60 bits: 8 x 12 + 4
+// 533 / 520, 2 x 8 + 2 136.1 / 134.5; below the line 8 x 8 + 1 of 2^13 57.5 / 58.0, 1 x 8 + 2 of 2^16 55.4 / 55.9, 2 x 12 + 4 of 2^15 67.3 / 67.6, but 4 x 3 +
+// 1 of 60 bits 86.4 / 84.4.  (The result stored past the caches would be 1 % more, and the caller's next call would read it from memory.)
+bool stream_products(uint32_t items, uint32_t L, uint32_t log_n) { return ((uint64_t)items * L << log_n) >= (uint64_t)16 << 16; }
+
 hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backend, hipStream_t s) {
     NttArgs a = args;
     if (a.log_n < 9 || a.log_n > 17 || x.items > 0xffffff || x.beta > 255) return hipErrorInvalidValue;
@@ -1472,7 +1483,9 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     // 104.9, 22 + 8 (414) 110.6 / 109.1, 18 + 4 (446) 104.7 / 103.7, 24 + 8 (448) 115.0 / 112.8, 12 + 1 (542) 105.6 / 104.9, 24 + 4 (656)
     // 140.5 / 131.8, 14 + 1 (720) 132.7 / 125.4; 60 / 40 bits 10 + 1 87.7 / 89.7, 22 + 8 154.4 / 152.1, 24 + 4 167.8 / 161.4.  A batch's
     // waves share their keys in a CU's cache: eight products 791 / 856.
-    const bool stream = items == 1 && (((3 * (uint64_t)x.beta + 2) * (x.L + x.K) + 4 * (uint64_t)x.L) << a.log_n) >= (uint64_t)400 << 16;
+    const bool stream_keys = items == 1 && (((3 * (uint64_t)x.beta + 2) * (x.L + x.K) + 4 * (uint64_t)x.L) << a.log_n) >= (uint64_t)400 << 16;
+    // The digits' words of products whose buffers go round the cache between two uses: see stream_products.
+    const bool stream_words = x.fold_ct && stream_products(items, x.L, a.log_n);
 #define HE_INNER_BE(BE, SPLIT, STREAM)                                                                                             \
     do {                                                                                                                          \
         if (items == 1 && x.beta <= InnerFew::kDigits)                                                                            \
@@ -1490,13 +1503,17 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
             HE_INNER_BE(NTT_BACKEND_INT, SPLIT, STREAM);         \
     } while (0)
     if (split == 4)
-        HE_INNER(4, false);
+        HE_INNER(4, 0);
     else if (split == 2)
-        HE_INNER(2, false);
-    else if (stream)
-        HE_INNER(1, true);
+        HE_INNER(2, 0);
+    else if (stream_keys && stream_words)
+        HE_INNER(1, 3);
+    else if (stream_keys)
+        HE_INNER(1, 1);
+    else if (stream_words)
+        HE_INNER(1, 2);
     else
-        HE_INNER(1, false);
+        HE_INNER(1, 0);
 #undef HE_INNER
 #undef HE_INNER_BE
     return hipGetLastError();
@@ -1542,12 +1559,24 @@ hipError_t launch_product_end(const NttArgs &args, const ProductEnd &x, uint32_t
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
     a.spread = items > 1;   // (as in launch_tensor_intt_blocks)
     const NttHead h = ntt_head(a, grid.x, 0);
+    // (the factors from half the last-level cache on: smaller ones may be in it for the caller's next product of them)
+    const int stream = !stream_products(items, x.L, a.log_n) ? 0 : ((uint64_t)items * x.L << a.log_n) >= (uint64_t)64 << 16 ? 2 : 1;
+#define HE_END(BE)                                                                                         \
+    do {                                                                                                   \
+        if (stream == 2)                                                                                   \
+            hipLaunchKernelGGL((product_end_kernel<BE, 2>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+        else if (stream)                                                                                   \
+            hipLaunchKernelGGL((product_end_kernel<BE, 1>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+        else                                                                                               \
+            hipLaunchKernelGGL((product_end_kernel<BE, 0>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+    } while (0)
     if (backend == NTT_BACKEND_MIXED)
-        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
+        HE_END(NTT_BACKEND_MIXED);
     else if (backend)
-        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
+        HE_END(NTT_BACKEND_FP);
     else
-        hipLaunchKernelGGL(product_end_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(h), x);
+        HE_END(NTT_BACKEND_INT);
+#undef HE_END
     return hipGetLastError();
 }
 

@@ -15,6 +15,8 @@ CASES = [  # log_n, bits, size_p, L, items
     (14, [60] * 8 + [60] * 2, 2, 8, 8),               # integers: on the line
     (13, [60] * 8 + [60], 1, 7, 19),                  # one special prime, L < size_q
     (16, [50] * 12 + [50] * 4, 4, 10, 1),             # one product, a partial last digit
+    (13, [60] + [40] * 5 + [60] * 2, 2, 6, 22),       # words that pass by the caches: from 16 * 2^16 on,
+    (13, [50] * 6 + [50] * 2, 2, 6, 86),              # with the factors from 64 * 2^16
     (17, [50, 50], 1, 2, 2),                          # two limbs: one stays (the largest ring)
 ]
 
