@@ -330,6 +330,7 @@ __device__ __forceinline__ double fp_canonical(double v, FpMod m) {
 // 2^50, for every q below 2^50: the first stage ends at 1 + 0.375 b and each later one at 1.375 b' + 0.5, which
 // is 5.92 after three stages from inputs of 4, 7.28 after three more, 5.63 after two more: for a chain of blocks of
 // at most 3, 3 and 2 stages whose first inputs are at most 4 x 2^50, and whose consumer reduces first.
+// (All of this for twiddles up to q; those of the tables are centred, so that a product grows by half of the 0.375.)
 template <int LOGR, int REDUCE_FIRST>
 __device__ __forceinline__ void fp_ct_block(double *v, const double *table, uint32_t idx, FpMod m) {
     constexpr int R = 1 << LOGR;

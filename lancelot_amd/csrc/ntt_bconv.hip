@@ -10,9 +10,9 @@
 // r = t - P^-1 sum_i x_i M[last][i] mod q_last (t: the limb right before the unit's inputs), output limb j receives
 // P^-1 sum_i x_i M[j][i] + (r mod q_j).  (FP64: the matrix carries the factor P^-1.)
 //
-// What bounds it: instruction issue, about 380 operations per output word of 64 lanes with 8 input limbs, and the wait for the inputs
-// that every workgroup starts with; 4 words a thread leave room for four waves per SIMD with 8 input limbs in registers (124 of
-// 128; on integers two or three), where 8 words left two.  One product against a kernel with 8 words per thread (FP64 only):
+// What bounds it: instruction issue, about 390 instructions for a thread's 4 words of an output limb with 8 input limbs (their loads and
+// set-up included), and the wait for the inputs that every workgroup starts with; 4 words a thread leave room for four waves per SIMD with 8
+// input limbs in registers (on integers two or three), where 8 words left two.  One product against a kernel with 8 words per thread (FP64 only):
 // n = 2^15, 10 of 12 limbs, K = 3 64.7 -> 55.8 us; n = 2^14, 8 limbs, K = 2 42.6 -> 38.4; a batch of 8, n = 2^15, 12 limbs, K = 4
 // 233 -> 219; L = 24, K = 8 the same 150 us.  Levels with a prime from 2^50 on against conversion kernel + rows pass: n = 2^15, 10 of
 // 12 limbs of 60 / 40 bits 77.5 -> 71.6 us; n = 2^13, 6 limbs, K = 2 45.4 -> 38.3; n = 2^16, 24 + 8 limbs 217 -> 204; a batch of 8,
