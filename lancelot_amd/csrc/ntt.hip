@@ -624,21 +624,25 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     const bool mx = bconv_on_matrix_cores(a.log_n, b, tune);
     // Output limbs per workgroup.  The kernel is bound by instruction issue, so a CU's time is the number of workgroups it is dealt
     // times a workgroup's work: r rows plus the fetching of the inputs and setting up, one row's worth and a half with 4 waves and a
-    // tile of 8 words per thread, half a row's with 8 waves and 4 words.  Few rows per workgroup pay that often, many leave
-    // CUs with one workgroup more than others.  A CU with a single workgroup has fewer waves to cover its waits with: as much as two
-    // take (4 waves), 15 % (8 waves, 25 % on integers: n = 2^14, 12 limbs of 60 bits, K = 4, one row 49.5 us, two
-    // 50.0).  Measured at n = 2^16 (8 waves), us with 1, 2, 3, 4, 5, 6, 8 rows a workgroup: K = 8, 24 rows
-    // for 96 tiles 37.5, 36.0, 30.5, 34.1, 30.9, 33.2, 38.4; K = 8, 23 rows for 64 tiles 33.3, 28.8, 24.4, 26.8, 30.5, 24.7, 28.4;
-    // K = 4, 12 rows for 96 tiles 16.7, 16.2, 15.8, 18.1, -, 17.0; K = 4, 11 rows for 64 tiles 13.3, 12.5, 11.4, 12.4, -, 16.0.
+    // tile of 8 words per thread; with 8 waves and 4 words half a row's with eight inputs and K / 16 of one with up to four (K / 20 on
+    // integers, whose rows take longer).  Few rows per workgroup pay that often, many leave CUs with one workgroup more than others.  A CU
+    // with a single workgroup has fewer waves to cover its waits with: as much as two take (4 waves), 15 % (8 waves, 10 % on
+    // integers), and some of it where an odd number leaves one for the end.  Measured at n = 2^16 (8 waves, inputs in their own order), us
+    // with 1, 2, 3, 4, 5, 6, 8 rows a workgroup: K = 8, 24 rows for 96 tiles 32.0, 25.0, 24.0, 31.3, 25.5, 28.7, 34.2; 23 rows for 64 tiles 26.0,
+    // 23.6, 21.0, 25.3, 27.6, 22.5, 27.0; 16 rows for 64 15.5, 14.6, 16.4, 15.0, 16.5, 17.4, 21.4; K = 4, 12 rows for 96 tiles 13.4, 14.2, 14.4, 16.2,
+    // 18.1, 16.0, 18.8; 12 for 64 9.6, 11.0, 10.5, 11.6, -, 14.2; 24 for 192 39.0, 35.4, 33.0, 34.1, 35.2, 35.3, 39.0; integers, K = 4, 12 rows for 96
+    // 19.3, 20.4, 21.6, 24.8, 26.3, 23.2, 25.2; n = 2^15, K = 3, 12 for 64 14.0, 14.4, 13.7, 15.0, 18.1, 18.8, 22.3.  Against half a row's set-up for every
+    // K: rotations, n = 2^16, 12 + 4 limbs 63.4 / 62.8 us, 9 of 12 + 4 59.8 / 58.6, of 60 / 40 bits 79.2 / 77.0, 73.4 / 71.0, 16 + 8 102.3 / 100.1.
     const uint32_t step = mx ? 4 : 1;
     uint32_t target = mx ? (forced + 3) / 4 * 4 : forced;
     if (!target) {
         uint64_t best = ~0ull;
-        const uint32_t single = b.rows_fp ? 23 : 25;
+        const uint32_t set_up = b.K > 4 ? 40 : b.rows_fp ? 5 * b.K : 4 * b.K, alone = b.rows_fp ? 23 : 22, odd = b.rows_fp ? 3 : 1;
         for (uint32_t r = step; r <= kFuseMaxRows && r < rows + step; r += step) {
             const uint64_t wgs = (uint64_t)b.units * items * tiles * ((rows + r - 1) / r);
             const uint64_t per_cu = (wgs + cus - 1) / cus;
-            const uint64_t cost = mx ? (per_cu < 2 ? 2 : per_cu) * (2 * r + 3) : (per_cu < 2 ? single : 20 * per_cu) * (2 * r + 1);
+            const uint64_t cost = mx ? (per_cu < 2 ? 2 : per_cu) * (2 * r + 3)
+                                     : (per_cu < 2 ? alone : 20 * per_cu + (per_cu & 1 ? odd : 0)) * (80 * r + set_up);
             if (cost < best) {
                 best = cost;
                 target = r;
