@@ -166,8 +166,8 @@ public:
     void set_seed(uint64_t seed);
     const uint32_t *prng_key() const { return prng_key_; }
     uint64_t next_stream(uint64_t count = 1) const { return prng_stream_.fetch_add(count, std::memory_order_relaxed); }
-    // ids of a call that was refused before anything drawn from them left it, if no other call has taken any since: the next
-    // call draws what it would have drawn without the refused one
+    // ids of a call that failed before anything drawn from them left it, if no other call has taken any since: the next
+    // call draws what it would have drawn without the failed one
     void give_back_streams(uint64_t first, uint64_t count) const {
         uint64_t last = first + count;
         prng_stream_.compare_exchange_strong(last, first, std::memory_order_relaxed);
@@ -480,13 +480,29 @@ public:
     }
 
 private:
+    // the stream ids of a batch on its way: given back unless it is kept, wherever it fails
+    class StreamIds {
+    public:
+        StreamIds(const CAHELGPUContext &context, std::size_t count) : context_(&context), first_(context.next_stream(count)), count_(count) {}
+        StreamIds(StreamIds &&o) noexcept : context_(o.context_), first_(o.first_), count_(o.count_) { o.context_ = nullptr; }
+        StreamIds &operator=(StreamIds &&) = delete;
+        ~StreamIds() {
+            if (context_) context_->give_back_streams(first_, count_);
+        }
+        uint64_t first() const { return first_; }
+        void keep() { context_ = nullptr; }
+
+    private:
+        const CAHELGPUContext *context_;
+        uint64_t first_, count_;
+    };
     // a batch on its way: the encryptions' random part is on the device's queue before the messages are copied
     struct Batch {
         std::size_t items;
         double scale;
         int total_bits;
-        uint64_t stream_id;
         cahel::DeviceBuffer cts, ws;
+        StreamIds ids;
     };
     void check_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale) const;
     Batch begin_batch(const CAHELGPUContext &context, const CAHELGPUPublicKey &pk, std::size_t items, double scale);

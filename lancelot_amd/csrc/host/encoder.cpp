@@ -153,11 +153,10 @@ CAHELGPUCKKSEncoder::Batch CAHELGPUCKKSEncoder::begin_batch(const CAHELGPUContex
                                                             double scale) {
     const uint32_t L = (uint32_t)context.limbs_at(first_chain_index_);
     he_context *h = context.handle();
-    Batch batch{items, scale, context.total_coeff_modulus_bit_count(first_chain_index_), 0,
+    Batch batch{items, scale, context.total_coeff_modulus_bit_count(first_chain_index_),
                 DeviceBuffer(items * 2 * (std::size_t)L * context.poly_degree()),
-                DeviceBuffer(he_encrypt_batch_workspace_words(h, L, (uint32_t)items))};
-    batch.stream_id = context.next_stream(3 * items);
-    check_status(he_encrypt_begin(h, L, (uint32_t)items, pk.pk_.data(), context.prng_key(), batch.stream_id, batch.ws.get(), context.stream()),
+                DeviceBuffer(he_encrypt_batch_workspace_words(h, L, (uint32_t)items)), StreamIds(context, 3 * items)};
+    check_status(he_encrypt_begin(h, L, (uint32_t)items, pk.pk_.data(), context.prng_key(), batch.ids.first(), batch.ws.get(), context.stream()),
                  "he_encrypt_begin");
     return batch;
 }
@@ -184,10 +183,8 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::end_batch(const CAHELGPUCon
         check_status(he_memcpy_d2h(maxima.data(), ws.get(), items * sizeof(double), st), "download");
         for (double max_coeff : maxima) {
             const int max_coeff_bit_count = static_cast<int>(std::ceil(std::log2(std::max(max_coeff, 1.0)))) + 1;
-            if (max_coeff_bit_count >= batch.total_bits || max_coeff_bit_count > 63) {
-                context.give_back_streams(batch.stream_id, 3 * items);
+            if (max_coeff_bit_count >= batch.total_bits || max_coeff_bit_count > 63)
                 throw std::invalid_argument("encoded values are too large");
-            }
         }
     }
     check_status(he_encrypt_end(h, L, (uint32_t)items, batch.cts.get(), batch.ws.get(), st), "he_encrypt_end");
@@ -206,6 +203,7 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::end_batch(const CAHELGPUCon
         ct.is_ntt_form_ = true;
         ct.is_asymmetric_ = true;
     }
+    batch.ids.keep();
     return out;
 }
 

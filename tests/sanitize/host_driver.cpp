@@ -16,6 +16,8 @@
 
 using namespace cahel;
 
+extern const char *mock_failing;   // mock_device.cpp
+
 #define REQUIRE(cond)                                                        \
     do {                                                                     \
         if (!(cond)) {                                                       \
@@ -250,6 +252,45 @@ int main(int argc, char **argv) {
         }
         synchronize_lanes();
         for (double *b : blocks) REQUIRE(std::memcmp(b, values.data(), bytes) == 0);
+    }
+
+    // ---- batches: the random part is on its way before the messages are looked at.  One that fails behind it, wherever that is, leaves
+    // the next one the stream ids that it would have drawn from without it. ----
+    {
+        set_lane(0);
+        CAHELGPUCKKSEncoder encoder(context);
+        CAHELGPUPublicKey pk(context);
+        pk.pk_.resize(context, 0, 2);
+        pk.gen_flag_ = true;
+        const std::size_t L1 = context.limbs_at(1), items = 3, count = n / 2;
+        std::vector<double> values(items * count, 0.5), huge(items * count, 1e30);
+        std::vector<float> floats(items * count, 0.5f);
+        const std::vector<const float *> rows{floats.data(), floats.data() + count, floats.data() + 2 * count};
+        const double scale = 1099511627776.0;
+        const uint64_t first = context.next_stream(0);
+        auto refused = [&](const char *call, const std::vector<double> &v) {
+            DeviceBuffer::trim_pool();
+            { DeviceBuffer cts(items * 2 * L1 * n), ws(items); }   // (in the pool: what he_malloc is asked for is the staging between the two calls)
+            mock_failing = call;
+            const bool threw = refuses([&] { encoder.encode_encrypt_many(context, pk, v.data(), items, count, count, scale); });
+            mock_failing = nullptr;
+            return threw && context.next_stream(0) == first;
+        };
+        REQUIRE(refused("", huge));
+        REQUIRE(refused("he_encrypt_begin", values));
+        REQUIRE(refused("he_memcpy_h2d_async", values));
+        REQUIRE(refused("he_ckks_encode_bounded", values));
+        REQUIRE(refused("he_ckks_encode_batch", huge));
+        REQUIRE(refused("he_encrypt_end", values));
+        REQUIRE(refused("he_malloc", values));
+        mock_failing = "he_memcpy_h2d_async";
+        REQUIRE(refuses([&] { encoder.encode_encrypt_updates(context, pk, rows, count, scale); }) && context.next_stream(0) == first);
+        mock_failing = nullptr;
+        auto cts = encoder.encode_encrypt_many(context, pk, values.data(), items, count, count, scale);
+        REQUIRE(cts.size() == items && context.next_stream(0) == first + 3 * items);
+        synchronize_lanes();
+        for (std::size_t k = 0; k < items; k++)
+            REQUIRE(cts[k].data()[0] == cts[0].data()[0] && cts[k].data()[L1 * n] == first + 3 * k && cts[k].data()[2 * L1 * n - 1] == first + 3 * k);
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused

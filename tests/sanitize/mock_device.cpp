@@ -3,6 +3,7 @@
 // CPU code paths can run under AddressSanitizer and UndefinedBehaviorSanitizer without a GPU.  Test infrastructure: "device" memory is malloc'ed host memory, copies
 // are memcpy, a context is an opaque token.  Nothing here computes.  Streams are queues: an encoding that nothing waits for writes its
 // plaintext when its stream is next used or waited for, as late as a device may.
+#include <cmath>
 #include <cstdlib>
 #include <cstring>
 #include <functional>
@@ -15,9 +16,14 @@ struct he_context {
     uint32_t log_n, size_q, size_p;
 };
 
+// the call that fails from now on, or nullptr
+const char *mock_failing = nullptr;
+
 namespace {
 
 std::map<he_stream, std::vector<std::function<void()>>> queues;
+
+bool fails(const char *call) { return mock_failing && !std::strcmp(mock_failing, call); }
 
 void run(he_stream stream) {
     for (auto &work : queues[stream]) work();
@@ -32,11 +38,13 @@ const char *he_error_string(int status) { return status == 0 ? "success" : "mock
 
 int he_malloc(void **dev_ptr, size_t bytes) {
     if (!dev_ptr) return HE_E_INVALID_ARGUMENT;
+    if (fails("he_malloc")) return HE_E_OUT_OF_MEMORY;
     *dev_ptr = bytes ? std::malloc(bytes) : nullptr;
     return (bytes && !*dev_ptr) ? HE_E_OUT_OF_MEMORY : HE_OK;
 }
 
-int he_free(void *dev_ptr) {
+int he_free(void *dev_ptr) {   // (waits for the device, as hipFree does)
+    for (auto &q : queues) run(q.first);
     std::free(dev_ptr);
     return HE_OK;
 }
@@ -74,7 +82,9 @@ int he_stream_synchronize(he_stream stream) {
 
 int he_host_malloc(void **host_ptr, size_t bytes) { return he_malloc(host_ptr, bytes); }
 int he_host_free(void *host_ptr) { return he_free(host_ptr); }
-int he_memcpy_h2d_async(void *dst, const void *src, size_t bytes, he_stream stream) { return he_memcpy_h2d(dst, src, bytes, stream); }
+int he_memcpy_h2d_async(void *dst, const void *src, size_t bytes, he_stream stream) {
+    return fails("he_memcpy_h2d_async") ? HE_E_UNSUPPORTED : he_memcpy_h2d(dst, src, bytes, stream);
+}
 
 // an event knows the stream it was recorded on
 int he_event_create(he_event *event) {
@@ -133,12 +143,32 @@ int he_context_destroy(he_context *ctx) {
 
 // "Encodes" later: the bits of value i as word i of every limb, zeros behind them.
 int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t, double, uint32_t limbs,
-                           uint32_t items, size_t, uint64_t *out, uint32_t, uint64_t *ws, he_stream stream) {
-    if (!ctx || !re || im || !out || !ws || items != 1) return HE_E_INVALID_ARGUMENT;
+                           uint32_t items, size_t value_stride, uint64_t *out, uint32_t out_poly_stride, uint64_t *ws, he_stream stream) {
+    if (!ctx || !re || im || !out || !ws || items == 0) return HE_E_INVALID_ARGUMENT;
+    if (fails("he_ckks_encode_bounded")) return HE_E_UNSUPPORTED;
     const size_t n = (size_t)1 << ctx->log_n;
     queues[stream].push_back([=] {
-        std::memset(out, 0, limbs * n * sizeof(uint64_t));
-        for (uint32_t l = 0; l < limbs; l++) std::memcpy(out + l * n, re, count * sizeof(double));
+        for (uint32_t k = 0; k < items; k++)
+            for (uint32_t l = 0; l < limbs; l++) {
+                uint64_t *limb = out + ((size_t)k * out_poly_stride + l) * n;
+                std::memset(limb, 0, n * sizeof(uint64_t));
+                std::memcpy(limb, re + k * value_stride, count * sizeof(double));
+            }
+    });
+    return HE_OK;
+}
+
+// The same, and the largest |value| times the scale in place of the largest coefficient
+int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *im, uint32_t count, uint32_t slots, double scale, uint32_t limbs,
+                         uint32_t items, size_t value_stride, uint64_t *out, uint32_t out_poly_stride, uint64_t *ws, he_stream stream) {
+    if (fails("he_ckks_encode_batch")) return HE_E_UNSUPPORTED;
+    if (int rc = he_ckks_encode_bounded(ctx, re, im, count, slots, scale, limbs, items, value_stride, out, out_poly_stride, ws, stream)) return rc;
+    queues[stream].push_back([=] {
+        for (uint32_t k = 0; k < items; k++) {
+            double largest = 0.0;
+            for (uint32_t i = 0; i < count; i++) largest = std::fmax(largest, std::fabs(re[k * value_stride + i]) * scale);
+            std::memcpy(ws + k, &largest, sizeof(double));
+        }
     });
     return HE_OK;
 }
@@ -153,16 +183,30 @@ int he_widen_rows(const float *in, double *out, uint32_t rows, size_t length, si
 
 size_t he_ckks_encode_batch_workspace_words(const he_context *, uint32_t items) { return 8 * (size_t)items; }
 
+// "Encrypts" in two calls: what item k draws from, its first stream id, goes to the workspace, and from there into every word of polynomial 1.
+size_t he_encrypt_batch_workspace_words(const he_context *, uint32_t, uint32_t items) { return items; }
+int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t *key, uint64_t stream_id, uint64_t *ws,
+                     he_stream stream) {
+    if (!ctx || L == 0 || items == 0 || !pk || !key || !ws) return HE_E_INVALID_ARGUMENT;
+    queues[stream].push_back([=] {
+        for (uint32_t k = 0; k < items; k++) ws[k] = stream_id + 3 * k;
+    });
+    return fails("he_encrypt_begin") ? HE_E_UNSUPPORTED : HE_OK;
+}
+int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *ws, he_stream stream) {
+    if (!ctx || L == 0 || items == 0 || !cts || !ws) return HE_E_INVALID_ARGUMENT;
+    if (fails("he_encrypt_end")) return HE_E_UNSUPPORTED;
+    const size_t poly = (size_t)L << ctx->log_n;
+    queues[stream].push_back([=] {
+        for (uint32_t k = 0; k < items; k++)
+            for (size_t i = 0; i < poly; i++) cts[(2 * (size_t)k + 1) * poly + i] = ws[k];
+    });
+    return HE_OK;
+}
+
 // (what encoder.cpp refers to besides)
 int he_ckks_encode(const he_context *, const double *, const double *, uint32_t, uint32_t, double, uint32_t, uint64_t *, uint64_t *,
                    he_stream) { return HE_E_UNSUPPORTED; }
-int he_ckks_encode_batch(const he_context *, const double *, const double *, uint32_t, uint32_t, double, uint32_t, uint32_t, size_t,
-                         uint64_t *, uint32_t, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
-size_t he_encrypt_batch_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
-int he_encrypt_begin(const he_context *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, he_stream) {
-    return HE_E_UNSUPPORTED;
-}
-int he_encrypt_end(const he_context *, uint32_t, uint32_t, uint64_t *, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
 int he_encrypt_batch(const he_context *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, uint64_t *,
                      he_stream) { return HE_E_UNSUPPORTED; }
 size_t he_ckks_workspace_words(const he_context *, uint32_t) { return 0; }
