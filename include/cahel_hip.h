@@ -383,7 +383,12 @@ int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const ui
                      uint64_t stream_id, uint64_t *cts, uint64_t *workspace, he_stream stream);
 
 /* he_encrypt_batch in two calls on one stream and one workspace: what needs no plaintext (the device may be at it while the
- * caller still prepares the messages), then the division by P onto the plaintexts in cts. */
+ * caller still prepares the messages), then the division by P onto the plaintexts in cts.  Nothing records what a workspace
+ * holds, so the caller keeps to this: he_encrypt_end takes the L and items of the he_encrypt_begin before it, the workspace is
+ * left alone in between, and he_encrypt_end uses it up: one he_encrypt_end for every he_encrypt_begin.  A second one would
+ * return HE_OK and either words that decrypt to nothing or, worse, ciphertexts of other messages under the same (u, e_0, e_1),
+ * whose difference shows the difference of the messages.  To try again with other messages, begin again, with other stream ids
+ * if a ciphertext of the first ones has been given away. */
 int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],
                      uint64_t stream_id, uint64_t *workspace, he_stream stream);
 int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *workspace, he_stream stream);
