@@ -303,8 +303,11 @@ int he_keyswitch_rescale(const he_context *ctx, uint32_t L, const uint64_t *c, c
                          he_stream stream);
 
 /* out [2][L-1][N] = rescale(relinearize(ct1 * ct2)) for two size-2 ciphertexts ct1, ct2 [2][L][N] (ct2 == ct1
- * squares): he_tensor, he_keyswitch and he_rescale with the same limbs in one call; the tensor product is formed by the
- * first pass of the key switch's inverse transform (its third polynomial is not read back for it).
+ * squares): he_tensor, he_keyswitch and he_rescale with the same limbs in one call.  The third polynomial of the tensor product
+ * is formed by the first pass of the key switch's inverse transform (and is not read back for it), the other two there as
+ * well or, in large calls, by the last pass: ct1 and ct2 are read until the call's work on the stream has ended.  out may
+ * lie over ct1 or ct2, wholly or in part (large calls then keep the first two polynomials in the workspace, the slower
+ * way); the workspace lies apart from all three.
  * workspace: he_multiply_relin_rescale_workspace_words words.
  * Replaces the sequence multiply (src/evaluate.cu:447-501: tensor_prod_2x2_rns_poly), relinearize_inplace
  * (src/eval_key_switch.cu:80-216) and rescale_to_next (src/evaluate.cu:2058-2085). */
@@ -314,7 +317,8 @@ int he_multiply_relin_rescale(const he_context *ctx, uint32_t L, const uint64_t 
 
 /* he_multiply_relin_rescale over `items` independent products with one launch per stage: ct1, ct2 [items][2][L][N]
  * -> out [items][2][L-1][N] (ct2 == ct1 squares every item), all with the same relinearisation key.  The limbs are
- * those of `items` separate calls.  Contexts with more than 8 special primes are not served (HE_E_UNSUPPORTED: the
+ * those of `items` separate calls.  When ct1 and ct2 are read and where out may lie: as for he_multiply_relin_rescale, over the whole
+ * batch.  Contexts with more than 8 special primes are not served (HE_E_UNSUPPORTED: the
  * batched base conversion holds at most 8 input limbs per thread); call he_multiply_relin_rescale per item there.
  * No counterpart in the reference, which multiplies one pair per call.
  * workspace: he_multiply_relin_rescale_batch_workspace_words words. */
