@@ -291,6 +291,29 @@ int main(int argc, char **argv) {
         synchronize_lanes();
         for (std::size_t k = 0; k < items; k++)
             REQUIRE(cts[k].data()[0] == cts[0].data()[0] && cts[k].data()[L1 * n] == first + 3 * k && cts[k].data()[2 * L1 * n - 1] == first + 3 * k);
+        // floats: rows that end inside, at and right behind a message, and more than all staging blocks hold (the fifth one is the first
+        // again, which its copy has to have left)
+        const std::size_t one_block = (std::size_t(1) << 20) / sizeof(float);
+        for (const std::size_t length : {std::size_t(1), count - 1, count, count + 1, 3 * count + 77, one_block + 5, 2 * one_block - 1}) {
+            const std::size_t chunks = (length + count - 1) / count, clients = length > count ? 3 : 2;
+            std::vector<std::vector<float>> updates(clients);
+            std::vector<const float *> starts;
+            for (std::size_t r = 0; r < clients; r++) {
+                for (std::size_t i = 0; i < length; i++) updates[r].push_back(0.25f + 1e-6f * (float)((i * 7 + r) % 1000));
+                starts.push_back(updates[r].data());
+            }
+            auto encrypted = encoder.encode_encrypt_updates(context, pk, starts, length, scale);
+            REQUIRE(encrypted.size() == clients * chunks);
+            synchronize_lanes();
+            for (std::size_t k = 0; k < encrypted.size(); k++)
+                for (std::size_t i = 0; i < count; i++) {
+                    const std::size_t at = k % chunks * count + i;
+                    double got;
+                    std::memcpy(&got, encrypted[k].data() + i, sizeof(got));
+                    REQUIRE(got == (at < length ? (double)updates[k / chunks][at] : 0.0));
+                }
+        }
+        REQUIRE(encoder.encode_encrypt_updates(context, pk, {}, 5, scale).empty());
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused

@@ -1,8 +1,8 @@
 // Host-memory stand-in for the C-ABI entry points that the host layer's table construction, record parsing and
 // containers call (he_malloc .. he_context_destroy, and he_keyswitch for a deferred relinearisation), so that those
 // CPU code paths can run under AddressSanitizer and UndefinedBehaviorSanitizer without a GPU.  Test infrastructure: "device" memory is malloc'ed host memory, copies
-// are memcpy, a context is an opaque token.  Nothing here computes.  Streams are queues: an encoding that nothing waits for writes its
-// plaintext when its stream is next used or waited for, as late as a device may.
+// are memcpy, a context is an opaque token.  Nothing here computes.  Streams are queues: an asynchronous copy reads its source, an encoding
+// writes its plaintext, when the stream is next waited for, as late as a device may.
 #include <cmath>
 #include <cstdlib>
 #include <cstring>
@@ -83,7 +83,9 @@ int he_stream_synchronize(he_stream stream) {
 int he_host_malloc(void **host_ptr, size_t bytes) { return he_malloc(host_ptr, bytes); }
 int he_host_free(void *host_ptr) { return he_free(host_ptr); }
 int he_memcpy_h2d_async(void *dst, const void *src, size_t bytes, he_stream stream) {
-    return fails("he_memcpy_h2d_async") ? HE_E_UNSUPPORTED : he_memcpy_h2d(dst, src, bytes, stream);
+    if (fails("he_memcpy_h2d_async")) return HE_E_UNSUPPORTED;
+    queues[stream].push_back([=] { std::memcpy(dst, src, bytes); });
+    return HE_OK;
 }
 
 // an event knows the stream it was recorded on
