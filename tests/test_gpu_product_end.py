@@ -1,5 +1,6 @@
 """Products whose last pass forms d0 and d1 from the factors, against the tensor product, key switch and rescale call by call, and against
-themselves with a result that lies over a factor (which takes (d0, d1) from the workspace): the same words, on both sides of the line."""
+themselves with a result that lies over a factor (which takes (d0, d1) from the workspace): the same words, on both sides of the line.  On
+integers and on both arithmetics also against the oracle (FP64: test_gpu_fullsize.py)."""
 import numpy as np
 import pytest
 
@@ -57,3 +58,26 @@ def test_products_equal_their_steps(oracle, capi, log_n, bits, size_p, L, items,
         capi.check(lib.he_tensor(h, da.at(at), db.at(at), d.ptr, L, None))
         capi.check(lib.he_keyswitch_rescale(h, L, d.at(2 * L * n), evk, d.ptr, one.ptr, 0, ws.ptr, None))
         assert (got[k] == one.numpy()).all(), k
+
+
+@pytest.mark.parametrize("log_n,bits,size_p,L,items", [(13, [60] * 8 + [60] * 2, 2, 8, 16),             # integers: on the line, 2^20 words
+                                                        (15, [60] * 6 + [60], 1, 6, 6),                  # one special prime
+                                                        (14, [60] + [40] * 5 + [60] * 2, 2, 6, 6)])      # both arithmetics
+def test_products_equal_the_oracle(oracle, capi, log_n, bits, size_p, L, items):
+    cahel, parms, ctx, p = make_pair(oracle, log_n, bits, size_p)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    assert items * L << log_n >= (16 if bits[1] > 50 else 8) << 16
+    rng = np.random.default_rng(log_n)
+    host_evk = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(p.size_q // size_p)]
+    dev_evk = [DeviceArray(capi, host=k) for k in host_evk]
+    evk = capi.evk_array([k.ptr for k in dev_evk])
+    a, b = (np.stack([rand_limbs(p, rng, range(L), n_polys=2) for _ in range(items)]) for _ in range(2))
+    a[0, 0, 0, :4] = b[-1, 1, 0, :4] = [0, 1, p.moduli[0] - 1, p.moduli[0] - 2]
+    da, db = DeviceArray(capi, host=a), DeviceArray(capi, host=b)
+    ws = DeviceArray(capi, shape=(lib.he_multiply_relin_rescale_batch_workspace_words(h, L, items),))
+    out = DeviceArray(capi, shape=(items, 2, L - 1, n))
+    for x, y, dx, dy in ((a, b, da, db), (b, b, db, db)):
+        capi.check(lib.he_multiply_relin_rescale_batch(h, L, items, dx.ptr, dy.ptr, evk, out.ptr, ws.ptr, None))
+        got = out.numpy()
+        for k in sorted({0, items // 2, items - 1}):
+            assert (got[k] == p.rescale(p.relinearize(p.tensor(x[k], y[k]), host_evk))).all(), k

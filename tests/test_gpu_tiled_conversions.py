@@ -60,6 +60,31 @@ def test_key_switches_with_tiled_conversions(oracle, capi, bits, size_p, levels)
         assert (drot.numpy() == np.stack([p.add(p.galois_ntt(ct[0], elt), md[0]), md[1]])).all(), L
 
 
+@pytest.mark.parametrize("bits", [[60] * 8 + [60] * 2, [60] + [40] * 7 + [60] * 2])
+def test_batch_of_merged_moddown_with_tiled_conversion(oracle, capi, bits):
+    """Three key switches with rescale in one call, conversions in integers: ModDown's inputs lie at the strides of the tiled order, K + 1
+    limbs a polynomial, two polynomials an item."""
+    L, size_p, items = 8, 2, 3
+    cahel, parms, ctx, p = make_pair(oracle, 16, bits, size_p)
+    rng = np.random.default_rng(5)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    # the order is taken: limbs in all, and its inputs within what is left of the digits
+    assert L + size_p >= 10 and (L + size_p) * items <= 64 and 2 * items * (size_p + 1) <= items * (L // size_p) * (L + size_p)
+    host_evk = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(L // size_p)]
+    dev_evk = [DeviceArray(capi, host=k) for k in host_evk]
+    c = rand_limbs(p, rng, range(L), n_polys=items)
+    ct = np.stack([rand_limbs(p, rng, range(L), n_polys=2) for _ in range(items)])
+    dc, dct = DeviceArray(capi, host=c), DeviceArray(capi, host=ct)
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_batch_workspace_words(h, L, items),))
+    out = DeviceArray(capi, shape=(items, 2, L - 1, n))
+    capi.check(lib.he_keyswitch_rescale_batch(h, L, items, dc.ptr, L, capi.evk_array([d.ptr for d in dev_evk]), dct.ptr, out.ptr, 0, ws.ptr,
+                                              None))
+    got = out.numpy()
+    for k in range(items):
+        ks = p.key_switch(c[k], host_evk)
+        assert (got[k] == p.rescale(np.stack([p.add(ct[k][r], ks[r]) for r in range(2)]))).all(), k
+
+
 @pytest.mark.parametrize("bits,size_p,L", [([50] * 12, 2, 10), ([60] + [40] * 7 + [60] * 2, 2, 8), ([50] * 16, 8, 4)])
 def test_encryption_with_tiled_conversion(oracle, capi, bits, size_p, L):
     """ModDown's inputs lie where the encrypted u was, or in natural order where that is too short (L < K)."""
