@@ -1114,6 +1114,7 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
                  uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0,
                  uint64_t *scratch = nullptr, size_t scratch_limbs = 0) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
+    if (n_polys == 0) return HE_OK;
     const int accumulate = add_mask != 0;
     const size_t n = ctx->n();
     const uint32_t K = ctx->size_p, LK = L + K;

@@ -221,6 +221,18 @@ def test_limbs_past_the_last_prime_are_refused(oracle, capi, first, count):
     assert calls == [-1] * len(calls)
 
 
+@pytest.mark.parametrize("bits,size_p", [([50, 40, 40, 50], 1), ([50, 40, 40, 40, 50, 50], 2), ([60, 40, 40, 40, 60, 60], 2)])
+@pytest.mark.parametrize("logn", [9, 12])
+def test_moddown_of_no_polynomials(oracle, capi, logn, bits, size_p):
+    """Nothing to do, with any number of special primes (the number is a divisor where the conversions are batched)."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    words = np.full((p.size_qp, p.n), 7, dtype=np.uint64)
+    cx, out, ws = (DeviceArray(capi, host=words) for _ in range(3))
+    for add in (0, 1):
+        assert capi.lib().he_moddown(ctx.he_handle(), p.size_q, cx.ptr, out.ptr, 0, add, ws.ptr, None) == 0
+    assert all((a.numpy() == words).all() for a in (cx, out, ws))
+
+
 class OddArray(DeviceArray):
     """A device buffer that starts 8 bytes behind a 16-byte boundary."""
 
