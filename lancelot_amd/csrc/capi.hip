@@ -1486,7 +1486,7 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     fwd.epi_dst_poly_stride = L - 1;
     if (tin && tin->last_only) {
         if (!fused) HE_HIP(launch_ntt_rows(fwd, polys * (L - 1), true, backend_for(ctx, fwd.map, (int)L - 1), S(s)));
-        const ProductEnd end{cx, tin->ct1, tin->ct2, out, fwd.pro_w, fwd.w, L, LK, tin->square};
+        const ProductEnd end{cx, tin->ct1, tin->square ? tin->ct1 : tin->ct2, out, fwd.pro_w, fwd.w, L, LK};
         HE_HIP(launch_product_end(fwd, end, items, backend_for(ctx, fwd.map, (int)L - 1), S(s)));
         return HE_OK;
     }

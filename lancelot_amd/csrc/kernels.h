@@ -236,11 +236,10 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &a, const TensorFuse &x, uint
 // rows pass's words [items][2][L][N], map = the L - 1 limbs.
 struct ProductEnd {
     const uint64_t *cx;          // [items][2][cx_stride][N]
-    const uint64_t *ct1, *ct2;   // [items][2][L][N]
+    const uint64_t *ct1, *ct2;   // [items][2][L][N]; a square: both the same
     uint64_t *out;               // [items][2][L - 1][N]
     const uint64_t *p_inv, *q_last_inv;   // Shoup pairs, by limb
     uint32_t L, cx_stride;
-    int square;
 };
 hipError_t launch_product_end(const NttArgs &a, const ProductEnd &x, uint32_t items, int backend, hipStream_t s);
 

@@ -952,18 +952,27 @@ __device__ __forceinline__ void end4(const IntArith &ar, const NttArgs &a, uint3
     }
 }
 
+// what ProductEnd has behind the head, whose input is the first factor
+struct EndExtra {
+    const uint64_t *cx, *ct2;
+    uint64_t *out;
+    const uint64_t *p_inv, *q_last_inv;
+    uint32_t cx_stride;
+};
+
 // A product's last pass (ProductEnd): a wave takes one block of both polynomials, so that it reads the four factors once.  Bound by memory:
 // the factors are read again (four polynomials) in place of d0 and d1 (two), which the first pass then neither forms nor stores, and for which
 // it does not read two of the factors.  Eight products of 24 + 8 limbs of 2^16 words, the first and the last pass: 140 + 163 us -> 77
 // + 190, and 90 + 147 with words that pass by the caches.
 // STREAM: 1: the rows pass's words and the sums pass by the caches; 2: the factors do as well.
 template <int STREAM, class A>
-__device__ __forceinline__ void product_end_block(const NttArgs &a, const ProductEnd &x, const Job &job, const A &ar, uint32_t blk,
+__device__ __forceinline__ void product_end_block(const NttArgs &a, const EndExtra &x, const Job &job, const A &ar, uint32_t blk,
                                                   uint32_t lane) {
     using T4 = Tile4<8, 8>;
+    const uint32_t L = a.map.limbs + 1;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane), item = job.poly;
-    const size_t ct = (2 * item * x.L + job.limb) * n + at, poly = (size_t)x.L * n;
-    const uint64_t *cx = x.cx + (2 * item * x.cx_stride + job.limb) * n + at, *ct2 = x.square ? x.ct1 : x.ct2;
+    const size_t ct = (2 * item * L + job.limb) * n + at, poly = (size_t)L * n;
+    const uint64_t *cx = x.cx + (2 * item * x.cx_stride + job.limb) * n + at;
     uint64_t lazy[2][4], c[2][4], f[2][4], g[2][4];
 #pragma unroll
     for (int r = 0; r < 2; r++) {
@@ -978,11 +987,11 @@ __device__ __forceinline__ void product_end_block(const NttArgs &a, const Produc
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         load_pairs_or_stream<STREAM != 0>(c[r], cx + r * (size_t)x.cx_stride * n);
-        load_pairs_or_stream<STREAM == 2>(f[r], x.ct1 + ct + r * poly);
-        load_pairs_or_stream<STREAM == 2>(g[r], ct2 + ct + r * poly);
+        load_pairs_or_stream<STREAM == 2>(f[r], a.in + ct + r * poly);
+        load_pairs_or_stream<STREAM == 2>(g[r], x.ct2 + ct + r * poly);
     }
     const Shoup p_inv = scalar_shoup(x.p_inv, job.limb), q_inv = scalar_shoup(x.q_last_inv, job.limb);
-    uint64_t *out = x.out + (2 * item * (x.L - 1) + job.limb) * n + at;
+    uint64_t *out = x.out + (2 * item * (L - 1) + job.limb) * n + at;
 #pragma unroll
     for (int r = 0; r < 2; r++) {
         typename A::V v[4];
@@ -995,12 +1004,12 @@ __device__ __forceinline__ void product_end_block(const NttArgs &a, const Produc
             end4(ar, a, job.table, v, c[0], f[0], g[0], nullptr, nullptr, p_inv, q_inv, o);
         else
             end4(ar, a, job.table, v, c[1], f[0], g[1], f[1], g[0], p_inv, q_inv, o);
-        store_pairs(out + r * (size_t)(x.L - 1) * n, o);
+        store_pairs(out + r * (size_t)(L - 1) * n, o);
     }
 }
 
 template <int BE, int STREAM>
-__global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_PARAMS, ProductEnd x) {
+__global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_PARAMS, EndExtra x) {
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
     const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63;
@@ -1519,6 +1528,16 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     return hipGetLastError();
 }
 
+// Whether a pass over the products of a batch deals a limb's workgroups to all XCDs (limb_block).  A limb's twiddles serve all items:
+// dealt out, an XCD keeps its eighth of all of them.  The first pass gains by it once the operands do not fit into the
+// L2s, where the launch before has left them otherwise: from 6 * 2^16 words a polynomial on, 10 * 2^16 with limbs of 2^14 and less
+// (products of a batch, us together / dealt: 8 x 24 limbs of 2^16 782 / 772, 2 x 3 of 2^16 43.2 / 42.6, 20 x 3 of 2^15 122 / 118, 2 x 3 of
+// 2^15 32.4 / 32.7, 8 x 10 of 2^13 62.5 / 61.9; 8 x 3 of 2^14 39.5 / 41.1, 8 x 8 of 2^12 58.7 / 61.6).  The last pass gains a little over the same
+// line (8 x 24 + 8 of 2^16 709 / 704, 8 x 12 + 4 of 2^15 182.9 / 180.9, 4 x 6 + 1 of 2^15, 60 / 40 bits, 86.1 / 85.0; 10 x 4 + 1 of 2^14 55.9 / 56.0).
+bool spread_products(uint32_t items, uint32_t L, uint32_t log_n) {
+    return items > 1 && ((uint64_t)L * items << log_n) >= (uint64_t)(log_n >= 15 ? 6 : 10) << 16;
+}
+
 hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, uint32_t items, int backend, hipStream_t s) {
     NttArgs a = args;
     a.in = x.ct1;
@@ -1526,11 +1545,7 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, u
     const uint64_t wgs = ((uint64_t)x.L * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
-    // A limb's twiddles serve all items: dealt out, an XCD keeps its eighth of all of them.  It pays once the operands do not fit into the
-    // L2s, where the launch before has left them otherwise: from 6 * 2^16 words a polynomial on, 10 * 2^16 with limbs of 2^14 and less
-    // (products of a batch, us together / dealt: 8 x 24 limbs of 2^16 782 / 772, 2 x 3 of 2^16 43.2 / 42.6, 20 x 3 of 2^15 122 / 118, 2 x 3 of
-    // 2^15 32.4 / 32.7, 8 x 10 of 2^13 62.5 / 61.9; 8 x 3 of 2^14 39.5 / 41.1, 8 x 8 of 2^12 58.7 / 61.6).
-    a.spread = items > 1 && ((uint64_t)x.L * items << a.log_n) >= (uint64_t)(a.log_n >= 15 ? 6 : 10) << 16;
+    a.spread = spread_products(items, x.L, a.log_n);
     const NttHead h = ntt_head(a, grid.x, x.square ? 1 : 0);
 #define HE_TENSOR(BE)                                                                                                             \
     do {                                                                                                                          \
@@ -1551,24 +1566,25 @@ hipError_t launch_tensor_intt_blocks(const NttArgs &args, const TensorFuse &x, u
 
 hipError_t launch_product_end(const NttArgs &args, const ProductEnd &x, uint32_t items, int backend, hipStream_t s) {
     NttArgs a = args;
-    a.in = nullptr;
+    a.in = x.ct1;
     a.out_poly_stride = 2 * x.L;   // (a job is both polynomials of a limb)
     if (a.log_n < 9 || a.log_n > 17 || a.jobs || a.map.limbs + 1 != x.L || a.map.limbs == 0 || items == 0) return hipErrorInvalidValue;
     const uint64_t wgs = ((uint64_t)a.map.limbs * items << (a.log_n - 8)) / kBlockWaves;
     if (wgs > most_workgroups(64 * kBlockWaves)) return hipErrorInvalidValue;
     const dim3 grid((uint32_t)wgs), block(64 * kBlockWaves);
-    a.spread = items > 1;   // (as in launch_tensor_intt_blocks)
+    a.spread = spread_products(items, x.L, a.log_n);
     const NttHead h = ntt_head(a, grid.x, 0);
+    const EndExtra extra{x.cx, x.ct2, x.out, x.p_inv, x.q_last_inv, x.cx_stride};
     // (the factors from half the last-level cache on: smaller ones may be in it for the caller's next product of them)
     const int stream = !stream_products(items, x.L, a.log_n) ? 0 : ((uint64_t)items * x.L << a.log_n) >= (uint64_t)64 << 16 ? 2 : 1;
 #define HE_END(BE)                                                                                         \
     do {                                                                                                   \
         if (stream == 2)                                                                                   \
-            hipLaunchKernelGGL((product_end_kernel<BE, 2>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+            hipLaunchKernelGGL((product_end_kernel<BE, 2>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
         else if (stream)                                                                                   \
-            hipLaunchKernelGGL((product_end_kernel<BE, 1>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+            hipLaunchKernelGGL((product_end_kernel<BE, 1>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
         else                                                                                               \
-            hipLaunchKernelGGL((product_end_kernel<BE, 0>), grid, block, 0, s, HE_HEAD_ARGS(h), x);        \
+            hipLaunchKernelGGL((product_end_kernel<BE, 0>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
     } while (0)
     if (backend == NTT_BACKEND_MIXED)
         HE_END(NTT_BACKEND_MIXED);
