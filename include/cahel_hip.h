@@ -372,8 +372,8 @@ int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double
                            double scale, uint32_t limbs, uint32_t items, size_t value_stride, uint64_t *out,
                            uint32_t out_poly_stride, uint64_t *workspace, he_stream stream);
 
-/* out[row] = in[row] as doubles, zeros behind them: `rows` rows of `length` floats, dense, to rows of `padded` (even) doubles.  What an
- * encoding takes from updates that travel in the 32 bits they are held in.  No counterpart in the reference. */
+/* out[row] = in[row] as doubles, zeros behind them: `rows` rows of `length` floats, dense, to rows of `padded` (even) doubles on a
+ * 16-byte boundary.  What an encoding takes from updates that travel in the 32 bits they are held in.  No counterpart in the reference. */
 int he_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, he_stream stream);
 
 /* Public-key encryption of `items` plaintexts with one launch per stage: cts [items][2][L][N] holds plaintext k in

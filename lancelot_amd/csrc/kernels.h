@@ -372,11 +372,11 @@ struct BconvExtra {
     size_t copy_item_stride;
 };
 constexpr uint32_t kMxRecord = 144, kConversionRow = 10;
-// `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
-// and `backend` says what the blocks pass that follows runs on
 // whether `inv`, the inverse transform that ends in b's inputs, should leave them tiled (in a buffer of their own: its last pass is in
 // place otherwise)
 bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune);
+// `a` supplies the FP64 twiddles and constants of a forward transform (base_args)
+// and `backend` says what the blocks pass that follows runs on
 hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, const Tuning &tune, hipStream_t s);
 hipError_t launch_bconv_rows4(const NttHead &h, const BconvRows &b, hipStream_t s);
 
@@ -502,9 +502,9 @@ struct FftTables {
 hipError_t launch_ckks_encode(const FftTables &t, const Tables &tab, const double *re, const double *im, uint32_t count,
                               uint32_t slots, double scale, double2 *v, uint64_t *max_bits, uint32_t items, size_t value_stride,
                               uint64_t *out, uint32_t limbs, size_t out_item_stride, hipStream_t s);
-// Only the transform: the slot vectors stay in v [items][slots] for NTT_PRO_ROUND.  re / im may be page-locked host memory.
 // rows of `length` floats -> rows of `padded` doubles, zeros behind the floats
 hipError_t launch_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, hipStream_t s);
+// launch_ckks_encode's transform alone: the slot vectors stay in v [items][slots] for NTT_PRO_ROUND.  re / im may be page-locked host memory.
 hipError_t launch_ckks_fft_inverse(const FftTables &t, const double *re, const double *im, uint32_t count, uint32_t slots,
                                    double2 *v, uint32_t items, size_t value_stride, hipStream_t s);
 // res: [limbs][N] coefficient-form residues of the first `limbs` primes -> v: `slots` complex values.

@@ -598,12 +598,14 @@ static bool bconv_on_matrix_cores(uint32_t log_n, const BconvRows &b, const Tuni
 
 // Tiled inputs (conversion_word): what a workgroup of the vector kernel fetches first, 64 KB to 144 KB, lay in segments of 64 bytes at N = 2^16,
 // which took 10 us of a launch's 28 with all workgroups at it.  The rows pass before it needs a buffer to leave them in, whose lines no cache
-// holds yet; that costs what is gained while there are few limbs, and more where a batch's words go past the caches.  us natural / tiled,
-// n = 2^16, L + K limbs: rotation 24 + 8 113.1 / 108.8, 16 + 8 78.4 / 75.1, 8 + 8 50.9 / 49.1, 10 + 3 65.7 / 64.7, 16 + 2 105.0 / 103.5, 8 + 2 52.9 /
-// 53.2, 6 + 4 43.6 / 44.4; product 24 + 8 136.9 / 132.1, 16 + 8 94.6 / 90.5, 4 + 2 39.7 / 40.5; hoisting 24 + 8 238.6 / 235.6; products of a
-// batch, limbs x items: 12 + 4 x 2 123.6 / 118.8, x 4 199.7 / 199.2, x 8 380 / 386, x 16 730 / 756, 24 + 8 x 2 229.8 / 227.2, 24 + 4 x 4 489 / 494, 8 + 2
-// x 4 152 / 149, x 16 507 / 529; 60 / 40 bits: rotation 24 + 8 157.3 / 153.2, 8 + 2 65.4 / 64.2, 8 + 3 63.7 / 62.1, 6 + 4 55.1 / 54.0, 3 + 8 52.1 / 53.5,
-// batches 12 + 4 x 4 257 / 256, x 8 474 / 481.  At 2^15 the segments are whole lines already: rotation 24 + 8 68.0 / 67.3, 10 + 3 43.7 / 44.6.
+// holds yet; that costs rotations what they gain while there are few limbs, and batches past 64 limbs, whose words go past the caches.  us
+// natural / tiled, n = 2^16, L + K limbs.  Rotation 24 + 8 113.1 / 108.8, 16 + 8 78.4 / 75.1, 8 + 8 50.9 / 49.1, 10 + 3 65.7 / 64.7, 16 + 2 105.0 /
+// 103.5, 8 + 2 52.9 / 53.2, 6 + 4 43.6 / 44.4; hoisting 24 + 8 238.6 / 235.6; 60 / 40 bits: rotation 24 + 8 157.3 / 153.2, 8 + 2 65.4 / 64.2, 8 + 3
+// 63.7 / 62.1, 6 + 4 55.1 / 54.0, 3 + 8 52.1 / 53.5.  Products, limbs x items: 24 + 8 136.9 / 132.1, 16 + 8 94.6 / 90.5, 9 + 3 55.9 / 53.8, 12 + 4 x 2
+// 111.8 / 108.8, x 3 151.3 / 148.7, x 4 182.1 / 180.5, x 5 240 / 242, 16 + 4 x 3 201 / 197, x 4 252 / 254, 9 + 3 x 4 141.8 / 141.3; 60 / 40 bits 12 + 4
+// x 4 244.4 / 245.9, x 6 366 / 367; 60 bits x 4 292.7 / 292.7.  Products that would gain below the lower line, which is the rotations': 8 + 2 55.3 /
+// 53.2, x 4 139.9 / 137.1, x 6 201 / 195, 6 + 2 x 4 105.4 / 100.0, but 6 + 3 x 4 98.5 / 98.3; 60 / 40 bits 6 + 2 63.6 / 62.0, x 4 138.8 / 137.3, but 6 +
+// 3 x 4 129.6 / 131.9.  At 2^15 the segments are whole lines already: rotation 24 + 8 68.0 / 67.3, 10 + 3 43.7 / 44.6.
 bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune) {
     const uint32_t limbs = b.map.limbs, items = b.items ? b.items : 1;
     if (inv.log_n != 16 || b.map.split < 6 || limbs < (b.rows_fp ? 12 : 10) || (uint64_t)limbs * items > 64) return false;

@@ -631,8 +631,8 @@ __device__ __forceinline__ void store_tiled(uint64_t *p, const uint64_t *v) {
 // (Tile4<8, 8>) but two pairs, 128 words apart, so that a 16-byte access of the wave covers 1 KiB without holes.  Four neighbours took
 // two accesses that touched the same sixteen lines one after the other, half of each.  turn_pairs goes from one layout to the other:
 // word bit 1 (a register's) and word bit 7 (lane bit 5) change places, four instructions.  Everything between the stages and memory
-// (products, epilogues) works on pairs.  2 x 24 limbs of 2^16 words back 24.7 -> 24.1 us; L = 24, K = 8: a rotation 121.3 -> 117.8, a
-// product 142.5 -> 140.1, eight 784 -> 774; n = 2^15, 10 of 12 limbs of 60 / 40 bits 64.0 -> 63.6; 2^16, 12 + 1 of them 114.2 -> 110.7.
+// (products, epilogues) works on pairs.  Before / after, us: L = 24, K = 8 a product 141.6 / 140.9, eight 782 / 769, a rotation 116.9 / 116.6;
+// n = 2^15, 10 of 12 limbs of 60 / 40 bits 63.6 / 62.4; 2 x 24 limbs of 2^16 words back the same 24.4.
 __device__ __forceinline__ uint32_t pair_lane(uint32_t lane) { return 4 * (lane & 31) + 2 * (lane >> 5); }
 __device__ __forceinline__ constexpr uint32_t pair_word(uint32_t j) { return (j & 1) + (j >> 1) * 128; }
 
