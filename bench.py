@@ -596,7 +596,8 @@ def main():
         duration is the traffic-weighted rate of its kernels."""
         prof = PROFILE[kind]
         issue_ms = prof["valu_wave_instr"] * 64 / rate.value * 1e3
-        floor_ms = 920 * limb_bytes / 6.0e12 * 1e3
+        floor_limbs = 736 + 192.0 / ops_per_launch
+        floor_ms = floor_limbs * limb_bytes / 6.0e12 * 1e3
         return {"bound": "hbm", "kernel": what + prof["kernels"],
                 "achieved": alg_bytes / (ms_per_op * 1e-3) / 1e9, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                 "frac": frac(ms_per_op),
@@ -609,8 +610,9 @@ def main():
                 "traffic": int(prof["traffic_limbs"] * limb_bytes * ops_per_launch),
                 "traffic_source": "profiles/hmult_relin_rescale_n65536_l24_k8.md (counter profile, not this run)",
                 "frac_of_dataflow_floor": floor_ms / ms_per_op,
-                "dataflow_floor": "920 limbs of traffic per operation (two-pass transforms, every fusion of "
-                                  "neighbouring pointwise stages) at the 6 TB/s a streaming kernel reaches on this GPU",
+                "dataflow_floor": "%.0f limbs of traffic per operation (what its kernels read and write, each word once per "
+                                  "kernel, the key once per launch, no twiddles) at the 6 TB/s a streaming kernel "
+                                  "reaches on this GPU" % floor_limbs,
                 "valu": {"wave_instructions_per_operation": prof["valu_wave_instr"],
                          "source": "SQ_INSTS_VALU summed over the kernels, same profile",
                          "fp64_issue_peak_lane_ops_per_s": rate.value, "issue_bound_ms": issue_ms,
