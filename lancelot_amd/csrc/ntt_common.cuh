@@ -382,6 +382,8 @@ struct IntArith {
         }
         return t;
     }
+    // (FpArith::load_last; in pairs a product and its quotient take as many multiplications as a butterfly and a half)
+    __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const { return load<2, false>((scale << 6) + t); }
     template <int ST>
     __device__ __forceinline__ void ct(V *v, const Tw &t) const {
         ct_butterfly(v[0], v[2], t.s[0], m);
@@ -433,6 +435,18 @@ struct FpArith {
             t.w[2] = at(2 * (size_t)idx + 1);
         }
         return t;
+    }
+    // a b mod q, centred, for centred a and b
+    __device__ __forceinline__ double twiddle(double a, double b) const { return fp_reduce(fp_mulmod(a, b, m), m); }
+    // The last block of a wave's 256 words (Tile4<8, 8>, `scale` as in load_tw), whose twiddles are three quarters of those of the pass
+    // and, read from their own places, as many bytes as the words: entry i is psi to the power of i bit-reversed, so for numbers
+    // without a common bit entry x + y = entry x times entry y, one of the wave's block times one of the first 128, which every block of
+    // the limb reads.  us before / after: 2 x 24 limbs of 2^16 words back 24.18 / 22.48 (its blocks pass 14.5 / 13.4 under the tracer), a product of
+    // 24 + 8 limbs 132.5 / 130.0, hoisting 238.2 / 235.3, a rotation 109.2 / 108.2; 4 + 1 limbs of 2^14 the same.
+    __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const {
+        const double r0 = table[t], r1 = table[2 * t], r2 = table[2 * t + 1];
+        const double b0 = scalar(table)[(size_t)scale << 6], b1 = scalar(table)[(size_t)scale << 7];
+        return Tw{{twiddle(r0, b0), twiddle(r1, b1), twiddle(r2, b1)}};
     }
     __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
         const double t = fp_mulmod(y, w, m);
@@ -510,7 +524,10 @@ struct Tile4 {
     template <class A, int K>
     static __device__ __forceinline__ void load_tw(typename A::Tw *tw, const A &ar, uint32_t scale, uint32_t t) {
         // scale: the tile's number within the limb enters the index as its upper bits (blocks pass), 1 for a rows pass
-        tw[K] = ar.template load<stages(K), (B - 2 * K - 2 >= 6)>(((scale - 1) << (2 * K)) + index(K, t));
+        if constexpr (B == 8 && LD == 8 && K == kBlocks - 1)
+            tw[K] = ar.load_last(scale, t);
+        else
+            tw[K] = ar.template load<stages(K), (B - 2 * K - 2 >= 6)>(((scale - 1) << (2 * K)) + index(K, t));
         if constexpr (K + 1 < kBlocks) load_tw<A, K + 1>(tw, ar, scale, t);
     }
     // From the layout of block KLO to that of block KLO + 1, or back: the register bits and the thread bits low - 1 and low - 2
