@@ -590,7 +590,7 @@ int he_context_create(const he_context_desc *d, he_context **out) {
                 psi_fp[t * n + i] = centred(w, q);
                 ipsi_fp[t * n + i] = centred(iw, q);
             }
-            psi_fp[t * n] = ipsi_fp[t * n] = 1.0;   // (psi^0, whatever the caller's entry: FpArith::load_last multiplies by it)
+            psi_fp[t * n] = ipsi_fp[t * n] = 1.0;   // (psi^0, whatever the caller's entry: FpProducts multiplies by it)
             const uint64_t ninv = q - (q - 1) / n;  // q = 1 mod 2N, so N * (q - (q-1)/N) = 1 mod q
             consts[4 * t] = qd;
             consts[4 * t + 1] = 1.0 / qd;

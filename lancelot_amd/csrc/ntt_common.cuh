@@ -382,7 +382,6 @@ struct IntArith {
         }
         return t;
     }
-    // (FpArith::load_last; in pairs a product and its quotient take as many multiplications as a butterfly and a half)
     __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const { return load<2, false>((scale << 6) + t); }
     template <int ST>
     __device__ __forceinline__ void ct(V *v, const Tw &t) const {
@@ -438,16 +437,8 @@ struct FpArith {
     }
     // a b mod q, centred, for centred a and b
     __device__ __forceinline__ double twiddle(double a, double b) const { return fp_reduce(fp_mulmod(a, b, m), m); }
-    // The last block of a wave's 256 words (Tile4<8, 8>, `scale` as in load_tw), whose twiddles are three quarters of those of the pass
-    // and, read from their own places, as many bytes as the words: entry i is psi to the power of i bit-reversed, so for numbers
-    // without a common bit entry x + y = entry x times entry y, one of the wave's block times one of the first 128, which every block of
-    // the limb reads.  us before / after: 2 x 24 limbs of 2^16 words back 24.18 / 22.48 (its blocks pass 14.5 / 13.4 under the tracer), a product of
-    // 24 + 8 limbs 132.5 / 130.0, hoisting 238.2 / 235.3, a rotation 109.2 / 108.2; 4 + 1 limbs of 2^14 the same.
-    __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const {
-        const double r0 = table[t], r1 = table[2 * t], r2 = table[2 * t + 1];
-        const double b0 = scalar(table)[(size_t)scale << 6], b1 = scalar(table)[(size_t)scale << 7];
-        return Tw{{twiddle(r0, b0), twiddle(r1, b1), twiddle(r2, b1)}};
-    }
+    // the last block of a wave's 256 words (Tile4<8, 8>, `scale` as in load_tw)
+    __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const { return load<2, false>((scale << 6) + t); }
     __device__ __forceinline__ void ct1(V &x, V &y, double w) const {
         const double t = fp_mulmod(y, w, m);
         y = x - t;
@@ -501,6 +492,30 @@ struct FpArith {
         scale<ST>(v, s);
 #pragma unroll
         for (int j = 0; j < 4; j++) w[j] = fp_to_u64(v[j]);
+    }
+};
+
+// The same with the twiddles of the last block of a wave's 256 words (Tile4<8, 8>) worked out.  They are three quarters of those of a blocks
+// pass and, read from their own places, nearly as many bytes as its words; but entry i of the table is psi to the power of i bit-reversed, so
+// for numbers without a common bit entry x + y is entry x times entry y: one of the wave's block times one of the first 128, which all
+// blocks of the limb read.  It pays where a kernel is bound by what it moves.  us with the entries read / worked out, n = 2^16: the last
+// blocks pass of a product of 12 + 4 limbs 11.0 / 9.5, of 24 + 8 18.4 / 16.9, of eight of those (product_end_kernel) 146 / 140, of a
+// rotation 8.8 / 8.0 and 15.5 / 14.1, 2^14, 12 + 4 4.6 / 4.5; the inner product of rotations 17.8 / 16.4 and 35.4 / 33.9.  Not where waves wait for
+// each other or for scattered words: inner product with blocks shared by two waves, 2^14, 12 + 4 6.8 / 7.2, encryption, 12 + 4 16.8 / 17.5,
+// rotation's first pass 8.7 / 9.2 and 8.8 / 10.5, the first pass of eight products 92 / 94.  (In pairs for the integer butterflies a product and
+// its quotient would take as many multiplications as a butterfly and a half.)
+// The product of two centred entries is at most 0.6 q.  Inverse: the first block of two stages then leaves at most 1.4 in place of 1.25,
+// and the bounds above still rise to 2.  Forward: the last two stages end at 3.8 in place of 3.63; CENTRED keeps 3.63, which the inner
+// product's sums need (FpSums).
+template <bool CENTRED>
+struct FpProducts : FpArith {
+    __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const {
+        const double b0 = scalar(table)[(size_t)scale << 6], b1 = scalar(table)[(size_t)scale << 7];
+        Tw w{{fp_mulmod(table[t], b0, m), fp_mulmod(table[2 * t], b1, m), fp_mulmod(table[2 * t + 1], b1, m)}};
+#pragma unroll
+        for (int i = 0; i < 3; i++)
+            if (CENTRED) w.w[i] = fp_reduce(w.w[i], m);
+        return w;
     }
 };
 

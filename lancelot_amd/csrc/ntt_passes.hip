@@ -325,7 +325,7 @@ template <bool FWD, bool EPI, bool LOOP, class A>
 __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &unit, Job job, const A &ar, uint64_t q, uint32_t blk,
                                               uint32_t lane) {
     using T4 = Tile4<8, 8>;
-    constexpr bool FP = std::is_same<A, FpArith>::value;
+    constexpr bool FP = std::is_base_of<FpArith, A>::value;
     const size_t off = (size_t)blk * 256;
     auto fetch = [&](uint64_t *x, const Job &j) {
         if (FWD) {
@@ -363,7 +363,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
                 turn_pairs(v);
                 if (EPI) {
-                    // (the word enters the difference as the last stage leaves it: at most 3.7 q, minuend below 1.9 q)
+                    // (the word enters the difference as the last stage leaves it: at most 3.8 q, minuend below 1.9 q)
                     const double ew = fp_from_u64(e.w.w);
                     if (e.fma) {
                         const double pw = fp_from_u64(e.pro_w.w);
@@ -428,7 +428,8 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
     }
 }
 
-template <bool FWD, bool EPI, bool LOOP, int BE>
+// PRODUCTS: see FpProducts (launch_ntt_blocks says when)
+template <bool FWD, bool EPI, bool LOOP, int BE, bool PRODUCTS>
 __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PARAMS, BlocksExtra x) {
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
@@ -440,7 +441,10 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
     const uint32_t blk = id & ((1u << lr) - 1);
     const Job job = decode_job<false, true>(a, unit.job(0));
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, fp_arith(a, job.table), 0, blk, lane);
+    if (BE != NTT_BACKEND_INT && fp) {
+        const typename std::conditional<PRODUCTS, FpProducts<false>, FpArith>::type ar{fp_arith(a, job.table)};
+        blocks_pass<FWD, EPI, LOOP>(a, unit, job, ar, 0, blk, lane);
+    }
     if constexpr (BE != NTT_BACKEND_FP) {
         if (!fp) blocks_pass<FWD, EPI, LOOP>(a, unit, job, int_arith(a, job.table), scalar(a.moduli)[job.table], blk, lane);
     }
@@ -524,7 +528,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
                                             uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
                                             uint64_t *sums_lds) {
     using T4 = Tile4<8, 8>;
-    constexpr bool FP = std::is_same<A, FpArith>::value;
+    constexpr bool FP = std::is_base_of<FpArith, A>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     const uint32_t own = t < L ? t / (LK - L) : 0xffffffffu;
     const uint64_t *lazy = a.out + (size_t)t * n + off;   // words left by the rows pass, digit 0
@@ -782,7 +786,10 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PAR
     const uint32_t blk = pair & ((1u << lr) - 1), table = map_table(a.map, t);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
-    if (BE != NTT_BACKEND_INT && fp) inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, fp_arith(a, table), part, sums);
+    if (BE != NTT_BACKEND_INT && fp) {
+        const typename std::conditional<SPLIT == 1, FpProducts<true>, FpArith>::type ar{fp_arith(a, table)};
+        inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, ar, part, sums);
+    }
     if constexpr (BE != NTT_BACKEND_FP) {
         if (!fp) inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, int_arith(a, table), part, sums);
     }
@@ -839,7 +846,7 @@ template <class A>
 __device__ __forceinline__ void tensor_block(const NttArgs &a, const TensorFuse &x, const Job &job, const A &ar, uint32_t blk,
                                              uint32_t lane) {
     using T4 = Tile4<8, 8>;
-    constexpr bool FP = std::is_same<A, FpArith>::value;
+    constexpr bool FP = std::is_base_of<FpArith, A>::value;
     const size_t n = (size_t)1 << a.log_n, poly = (size_t)x.L * n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     const size_t ct = 2 * job.poly * poly + job.limb * n + at;
     uint64_t a0[4], a1[4], b0[4], b1[4];
@@ -930,7 +937,7 @@ __device__ __forceinline__ void end4(const FpArith &ar, const NttArgs &, uint32_
                                      const uint64_t *z, const uint64_t *w, Shoup p_inv, Shoup q_inv, uint64_t *out) {
     const FpMod m = ar.m;
     const double pw = fp_from_u64(p_inv.w), ew = fp_from_u64(q_inv.w);
-    // (three products below q, less a word of at most 3.7 q: below 8 q)
+    // (three products below q, less a word of at most 3.8 q: below 8 q)
 #pragma unroll
     for (int j = 0; j < 4; j++) {
         double d = fp_mulmod(fp_from_u64(c[j]), pw, m) + fp_mulmod(fp_from_u64(x[j]), fp_from_u64(y[j]), m);
@@ -1017,7 +1024,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_P
     const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) product_end_block<STREAM>(a, x, job, fp_arith(a, job.table), blk, lane);
+    if (BE != NTT_BACKEND_INT && fp) product_end_block<STREAM>(a, x, job, FpProducts<false>{fp_arith(a, job.table)}, blk, lane);
     if constexpr (BE != NTT_BACKEND_FP) {
         if (!fp) product_end_block<STREAM>(a, x, job, int_arith(a, job.table), blk, lane);
     }
@@ -1044,7 +1051,7 @@ __device__ __forceinline__ void encrypt_block(const NttArgs &a, const uint64_t *
                                               uint32_t table, uint32_t blk, uint32_t item, uint32_t items, uint32_t w, uint32_t lane,
                                               const A &ar, uint64_t *u_lds) {
     using T4 = Tile4<8, 8>;
-    constexpr bool FP = std::is_same<A, FpArith>::value;
+    constexpr bool FP = std::is_base_of<FpArith, A>::value;
     const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane);
     uint64_t *poly = a.out + ((size_t)(w == 0 ? item : items + 2 * item + w - 1) * LK + t) * n;
     const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
@@ -1414,28 +1421,36 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     a.spread = epi && spread_epilogue(a, backend, kinds, repeats, wgs);
     const NttHead head = ntt_head(a, grid.x, a.batch);
     const BlocksExtra extra = blocks_extra(a, forward);
-#define HE_LAUNCH(FWD, EPI, LOOP)                                                                                       \
-    do {                                                                                                                \
-        if (backend == NTT_BACKEND_MIXED)                                                                               \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_MIXED>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
-        else if (backend)                                                                                               \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_FP>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
-        else                                                                                                            \
-            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
+#define HE_LAUNCH(FWD, EPI, LOOP, PRODUCTS)                                                                                       \
+    do {                                                                                                                          \
+        if (backend == NTT_BACKEND_MIXED)                                                                                         \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_MIXED, PRODUCTS>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
+        else if (backend)                                                                                                         \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_FP, PRODUCTS>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
+        else                                                                                                                      \
+            hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT, false>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
     } while (0)
     const bool loop = a.batch > 1 || a.groups;
+    // Twiddles worked out (FpProducts): in front of an epilogue always; by itself a pass over 32 * 2^16 words finds them in the L2s in a repeated
+    // transform, one over 36 does not.  Transforms, us read / worked out: 2 x 16 limbs of 2^16 words 15.1 / 15.6, 2 x 20 19.1 / 18.0, 2 x 24 back 22.8 /
+    // 21.0, of 60 / 40 bits 23.7 / 22.0, 3 x 24 of 2^15 17.3 / 16.8, 4 x 24 of 2^14 12.1 / 12.7.
+    const bool products = ((uint64_t)kinds * repeats << a.log_n) >= (uint64_t)36 << 16 && !a.in_galois;
     if (epi && loop)
-        HE_LAUNCH(true, true, true);
+        HE_LAUNCH(true, true, true, false);
     else if (epi)
-        HE_LAUNCH(true, true, false);
+        HE_LAUNCH(true, true, false, true);
     else if (forward && loop)
-        HE_LAUNCH(true, false, true);
+        HE_LAUNCH(true, false, true, false);
+    else if (forward && products)
+        HE_LAUNCH(true, false, false, true);
     else if (forward)
-        HE_LAUNCH(true, false, false);
+        HE_LAUNCH(true, false, false, false);
     else if (loop)
-        HE_LAUNCH(false, false, true);
+        HE_LAUNCH(false, false, true, false);
+    else if (products)
+        HE_LAUNCH(false, false, false, true);
     else
-        HE_LAUNCH(false, false, false);
+        HE_LAUNCH(false, false, false, false);
 #undef HE_LAUNCH
     return hipGetLastError();
 }
