@@ -522,7 +522,7 @@ __global__ __launch_bounds__(256 * LIMBS) void decode_rows_compose_kernel(HE_HEA
         T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
         T4::template inverse<IntArith>(x, tw, ar, lds, t);
 #pragma unroll
-        for (int j = 0; j < 4; j++) x[j] = reduce_3q(x[j], ar.m.q);
+        for (int j = 0; j < 4; j++) x[j] = reduce_4q(x[j], ar.m);
     }
     uint64_t d[2][LIMBS];
     if constexpr (LIMBS > 1) {

@@ -1,6 +1,6 @@
 // Device-side 64-bit modular arithmetic for gfx950 (wave64, VALU integer multiplies).
 //
-// All routines work on residues of primes below 2^61.  "lazy" values live in [0, 3q) or [0, 6q) and
+// All routines work on residues of primes below 2^61.  "lazy" values live in [0, 4q) or [0, 8q) and
 // never leave a kernel: every store to HBM that a caller can observe is the canonical residue, which
 // is what makes limb-for-limb comparison with the CPU oracle meaningful.
 //
@@ -181,14 +181,14 @@ __device__ __forceinline__ U128 total_sum3(const Sum3 &h, const Sum3 &s) {
     return U128{(uint64_t)t, (uint64_t)(t >> 64)};
 }
 
-// The butterflies' view of a modulus: q, 3q, 4q and their negatives modulo 2^64.  With the negatives at hand a Shoup
-// product is y w + hi (2^64 - q) and a conditional subtraction is x + (2^64 - 3q) followed by a select on the sign, i.e.
-// 64-bit additions (one instruction each) where subtractions would be borrow chains through VCC, which on this GPU need
-// two idle issue slots between producer and consumer.  The negatives pass through an empty asm statement so that the
-// compiler does not fold them back into subtractions: 27.5 -> 24.5 vector instructions and 4.0 -> 2.9 idle slots per
-// butterfly, 32.5 -> 30.5 and 3.1 -> 2.6 in the inverse direction.
+// The butterflies' view of a modulus: q, and modulo 2^64 the numbers that make every sum, difference and conditional subtraction of a
+// butterfly 64-bit additions (one instruction each): -q, -2q, -4q, and 4q + 1, with which x + 4q - t is (x + 4q + 1) + ~t.  Borrow chains
+// through VCC need two idle issue slots between producer and consumer on this GPU, which a SIMD with one wave cannot fill (a slot costs
+// such a wave 1.6 ns, any vector instruction 2.0 to 2.2; with eight waves 1.0 for the simplest and 1.75 for all others, 32-bit
+// multiplications included).  The numbers pass through an empty asm statement so that the compiler does not fold them back into
+// subtractions.
 struct IntMod {
-    uint64_t q, q3, q4, nq, nq3, nq4;
+    uint64_t q, q4p, nq, nq2, nq4;
 };
 
 // (q is the same in every lane of a wave: a workgroup works on one limb; read from lane 0 so that the constants are
@@ -196,65 +196,59 @@ struct IntMod {
 __device__ __forceinline__ IntMod int_mod(uint64_t q_any_lane) {
     const uint32_t q_hi = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)(q_any_lane >> 32));
     const uint32_t q_lo = (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)q_any_lane);   // (the builtin returns int)
-    const uint64_t q = ((uint64_t)q_hi << 32) | q_lo, q3 = 3 * q, q4 = 4 * q;
+    const uint64_t q = ((uint64_t)q_hi << 32) | q_lo, q2 = 2 * q, q4 = 4 * q, q4p = q4 + 1;
     // (as 32-bit scalars)
     uint32_t a0 = (uint32_t)(0 - q), a1 = (uint32_t)((0 - q) >> 32);
-    uint32_t b0 = (uint32_t)(0 - q3), b1 = (uint32_t)((0 - q3) >> 32);
+    uint32_t b0 = (uint32_t)(0 - q2), b1 = (uint32_t)((0 - q2) >> 32);
     uint32_t c0 = (uint32_t)(0 - q4), c1 = (uint32_t)((0 - q4) >> 32);
-    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(b0), "+s"(b1), "+s"(c0), "+s"(c1));
-    return IntMod{q, q3, q4, ((uint64_t)a1 << 32) | a0, ((uint64_t)b1 << 32) | b0, ((uint64_t)c1 << 32) | c0};
+    uint32_t d0 = (uint32_t)q4p, d1 = (uint32_t)(q4p >> 32);
+    asm volatile("" : "+s"(a0), "+s"(a1), "+s"(b0), "+s"(b1), "+s"(c0), "+s"(c1), "+s"(d0), "+s"(d1));
+    return IntMod{q, ((uint64_t)d1 << 32) | d0, ((uint64_t)a1 << 32) | a0, ((uint64_t)b1 << 32) | b0, ((uint64_t)c1 << 32) | c0};
 }
 
-// floor(a b / 2^64) or one less: the product of the lower halves, below 2^64, is left out
+// floor(a b / 2^64) or up to two less: the products with one lower half enter with their upper words, that of both lower halves not at
+// all (three fractions below 1 are lost)
 __device__ __forceinline__ uint64_t mulhi64_low(uint64_t a, uint64_t b) {
     const uint32_t a0 = (uint32_t)a, a1 = (uint32_t)(a >> 32), b0 = (uint32_t)b, b1 = (uint32_t)(b >> 32);
-    const uint64_t t = (uint64_t)a0 * b1, u = (uint64_t)a1 * b0 + (uint32_t)t;
-    return (uint64_t)a1 * b1 + (t >> 32) + (u >> 32);
+    return (uint64_t)a1 * b1 + __umulhi(a0, b1) + __umulhi(a1, b0);
 }
 
-// y w mod q up to two subtractions of q, in [0, 3q), for any 64-bit y
+// y w mod q up to three subtractions of q, in [0, 4q), for any 64-bit y
 __device__ __forceinline__ uint64_t mul_shoup_lazy(uint64_t y, Shoup s, const IntMod &m) {
     return y * s.w + mulhi64_low(y, s.wq) * m.nq;
 }
 
-// v - k q if that is not negative, else v; nkq = 2^64 - k q (v below 6q: the difference fits 63 bits)
+// v - k q if that is not negative, else v; nkq = 2^64 - k q (v below 8q: the difference fits 63 bits)
 __device__ __forceinline__ uint64_t reduce_once(uint64_t v, uint64_t nkq) {
     const uint64_t d = v + nkq;
-    return (int64_t)d < 0 ? v : d;
+    return (int32_t)(d >> 32) < 0 ? v : d;
 }
 
-// Cooley-Tukey butterfly, inputs in [0, 6q), outputs in [0, 6q): below 2^64 for q < 2^61.  (The range is what the shorter product
-// costs: a reduction more per word at the end of a transform, against one of ten multiplications and a link of the
-// chain per butterfly: multiplication with 4 limbs of 2^16 words and 60 bits 56.5 -> 54.8 us, 10 of 12 limbs of 2^15 with 60 and
-// 40 bits 65.8 -> 65.0, a transform of 2 x 24 limbs back 33.4 -> 33.0.)
+// Cooley-Tukey butterfly, inputs in [0, 8q), outputs in [0, 8q): below 2^64 for q < 2^61.  21 vector instructions.  (With a quotient one
+// less at most, in multiply-adds that wait for each other and need their addends moved, and ranges of 6q: 27, and a whole blocks pass 692
+// against 502.  us: rotation on [60, 40, 40, 60], n = 2^16 27.0 -> 26.1; 2^15, 12 + 3 of 60 / 40 bits 54.9 -> 53.7; 2^16, 12 + 4 of 60 bits 90.6 ->
+// 88.7; multiplication, 2^14, 4 + 1 28.6 -> 27.9 and 29.4 -> 29.0; eight limbs of 2^16 words and 60 bits 9.0 -> 8.8.)
 __device__ __forceinline__ void ct_butterfly(uint64_t &x, uint64_t &y, Shoup tw, const IntMod &m) {
     const uint64_t t = mul_shoup_lazy(y, tw, m);
-    const uint64_t xr = reduce_once(x, m.nq3);
-    y = (xr + m.q3) - t;
+    const uint64_t xr = reduce_once(x, m.nq4);
+    y = (xr + m.q4p) + ~t;
     x = xr + t;
 }
 
 // Gentleman-Sande butterfly with the division by two folded in (the inverse twiddles are stored
-// pre-halved), inputs in [0, 3q), outputs in [0, 3q): the sum is below 6q, 4q once reduced, 2.5q once halved; the difference below
-// 7q (2^64 for q < 2^61).  4q, not 3q: both have the parity of x + y, so that the sum's halving does not wait for its reduction.
+// pre-halved), inputs in [0, 4q), outputs in [0, 4q): the sum is below 8q, 4q once reduced, 2.5q once halved; the difference below
+// 8q (2^64 for q < 2^61).  Both have the parity of x + y, so that the sum's halving does not wait for its reduction.
 __device__ __forceinline__ void gs_butterfly(uint64_t &x, uint64_t &y, Shoup tw, const IntMod &m) {
-    const uint64_t d = x + m.q4 - y;
+    const uint64_t d = (x + m.q4p) + ~y;
     uint64_t s = reduce_once(x + y, m.nq4);
     s += (d & 1) ? m.q : 0;
     x = s >> 1;
     y = mul_shoup_lazy(d, tw, m);
 }
 
-__device__ __forceinline__ uint64_t reduce_3q(uint64_t v, uint64_t q) {
-    const uint64_t q2 = q << 1;
-    v = v >= q2 ? v - q2 : v;
-    return v >= q ? v - q : v;
-}
-
-__device__ __forceinline__ uint64_t reduce_6q(uint64_t v, uint64_t q) {
-    const uint64_t q3 = 3 * q;
-    return reduce_3q(v >= q3 ? v - q3 : v, q);
-}
+// canonical from below 4q and 8q
+__device__ __forceinline__ uint64_t reduce_4q(uint64_t v, const IntMod &m) { return reduce_once(reduce_once(v, m.nq2), m.nq); }
+__device__ __forceinline__ uint64_t reduce_8q(uint64_t v, const IntMod &m) { return reduce_4q(reduce_once(v, m.nq4), m); }
 
 __device__ __forceinline__ Shoup load_shoup(const uint64_t *table, size_t idx) {
     const ulonglong2 v = reinterpret_cast<const ulonglong2 *>(table)[idx];

@@ -187,13 +187,13 @@ __global__ __launch_bounds__(1 << (LOGN - 2)) void ntt_limb4_kernel(HE_HEAD_PARA
             if (FWD) {
                 T4::template forward<IntArith>(x, tw, ar, lds, t);
 #pragma unroll
-                for (int j = 0; j < 4; j++) x[j] = reduce_6q(x[j], q);
+                for (int j = 0; j < 4; j++) x[j] = reduce_8q(x[j], ar.m);
             } else {
                 Shoup w{0, 0};
                 if (a.epi_mode == NTT_EPI_MUL) w = scalar_shoup(a.w, job.limb);
                 T4::template inverse<IntArith>(x, tw, ar, lds, t);
 #pragma unroll
-                for (int j = 0; j < 4; j++) x[j] = a.epi_mode == NTT_EPI_MUL ? mul_shoup(x[j], w, q) : reduce_3q(x[j], q);
+                for (int j = 0; j < 4; j++) x[j] = a.epi_mode == NTT_EPI_MUL ? mul_shoup(x[j], w, q) : reduce_4q(x[j], ar.m);
             }
         }
     }

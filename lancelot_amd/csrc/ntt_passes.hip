@@ -112,7 +112,7 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
         T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
         T4::template inverse<IntArith>(s, tw, ar, lds, t);
 #pragma unroll
-        for (int j = 0; j < 4; j++) s[j] = reduce_3q(s[j], q);
+        for (int j = 0; j < 4; j++) s[j] = reduce_4q(s[j], ar.m);
     }
 }
 
@@ -213,7 +213,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 rows_input_int<MDR, SRC_INTT>(v, a, job, q, [&](int j) { return glob(0, j); }, s, s2);
             }
             T4::template forward<IntArith>(v, tw, ar, lds, t);
-            // lazy values in [0, 6q) go to the blocks pass
+            // lazy values in [0, 8q) go to the blocks pass
 #pragma unroll
             for (int j = 0; j < 4; j++) job.out[glob(NB - 1, j)] = v[j];
         } else {
@@ -228,7 +228,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 for (int j = 0; j < 4; j++) v[j] = mul_shoup(v[j], w, q);
             } else {
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = reduce_3q(v[j], q);
+                for (int j = 0; j < 4; j++) v[j] = reduce_4q(v[j], ar.m);
             }
             leave(v);
         }
@@ -396,7 +396,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
                 T4::template forward<A>(v, tw, ar, nullptr, lane);
                 turn_pairs(v);
 #pragma unroll
-                for (int j = 0; j < 4; j++) x[j] = reduce_6q(v[j], q);
+                for (int j = 0; j < 4; j++) x[j] = reduce_8q(v[j], ar.m);
                 if (EPI) {
                     const Shoup ew = e.w;
                     if (e.fma) {
@@ -419,7 +419,7 @@ __device__ __forceinline__ void blocks_pass(const NttArgs &a, const BlockUnit &u
             }
         }
         if (!FWD) {
-            // lazy words (signed doubles, or integers in [0, 3q)) go to the rows pass
+            // lazy words (signed doubles, or integers in [0, 4q)) go to the rows pass
 #pragma unroll
             for (int j = 0; j < 4; j++) job.out[off + T4::word(0, lane, j)] = A::to_word(v[j]);
         }
@@ -453,7 +453,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
 // Sum over the digits of (word x key word) for four words of both key polynomials.
 // FP64: a transformed word enters as the last stage leaves it (at most 3.7 q: a term below 1.9 q), the sums are reduced after
 // every fourth digit and stay below 8 q.  Integers: 128-bit sums of at most 64 products below 2^122 of canonical words, or, with primes
-// below 2^60, of at most 40 products of words as the last stage leaves them (below 6 q).
+// below 2^60, of at most 32 products of words as the last stage leaves them (below 8 q).
 struct FpSums {
     double s[2][4];
     uint32_t pending = 0;
@@ -597,7 +597,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         }
     }
     bool canonical = false;
-    if constexpr (!FP) canonical = (ar.m.q >> 60) || beta > 40;
+    if constexpr (!FP) canonical = (ar.m.q >> 60) || beta > 32;
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = a.in + (size_t)t * n;
@@ -636,7 +636,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         if constexpr (!FP) {
             if (SPLIT == 1 || canonical) {   // (one wave a block: the branch costs what it saves)
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = reduce_6q(v[j], ar.m.q);
+                for (int j = 0; j < 4; j++) v[j] = reduce_8q(v[j], ar.m);
             }
         }
         sums.add(v, k, ar);
@@ -955,7 +955,7 @@ __device__ __forceinline__ void end4(const IntArith &ar, const NttArgs &a, uint3
         mac128(d, x[j], y[j]);
         if (z) mac128(d, z[j], w[j]);
         const uint64_t lhs = add_mod(mul_shoup(c[j], p_inv, q), barrett128(d.lo, d.hi, q, r0, r1), q);
-        out[j] = mul_shoup(sub_mod(lhs, reduce_6q(v[j], q), q), q_inv, q);
+        out[j] = mul_shoup(sub_mod(lhs, reduce_8q(v[j], ar.m), q), q_inv, q);
     }
 }
 
@@ -1032,7 +1032,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_P
 
 // a word that the forward stages have left (lazy) as a canonical residue, and a canonical word as the arithmetic's value
 __device__ __forceinline__ uint64_t canonical_word(double v, const FpArith &ar) { return fp_to_u64(fp_canonical(v, ar.m)); }
-__device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &ar) { return reduce_6q(v, ar.m.q); }
+__device__ __forceinline__ uint64_t canonical_word(uint64_t v, const IntArith &ar) { return reduce_8q(v, ar.m); }
 
 // v + x * y mod q for canonical words x, y and v as the forward stages have left it; canonical
 __device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y, const FpArith &ar, uint64_t, uint64_t) {
@@ -1040,7 +1040,7 @@ __device__ __forceinline__ uint64_t add_product(double v, uint64_t x, uint64_t y
     return fp_to_u64(fp_canonical(v + fp_mulmod(fp_from_u64(x), w, ar.m), ar.m));
 }
 __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t y, const IntArith &ar, uint64_t r0, uint64_t r1) {
-    return add_mod(reduce_6q(v, ar.m.q), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
+    return add_mod(reduce_8q(v, ar.m), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
 }
 
 // Encryption: three waves take their block of u, e0 and e1 of one limb through the last 8 stages; the transformed u stays in

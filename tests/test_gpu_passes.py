@@ -58,23 +58,23 @@ def test_whole_limb_transforms(oracle, capi, monkeypatch, chain, logn, limbs, po
     assert (d.numpy() == x).all()
 
 
-@pytest.mark.parametrize("bits", [50, 49, 30])
-@pytest.mark.parametrize("logn", [9, 11, 13, 16, 17])
-def test_last_twiddles_as_products(oracle, capi, monkeypatch, logn, bits):
-    """FP64 blocks passes form the twiddles of their last two stages from two entries of the table: every block of the smallest and
-    the largest degree, primes at both ends of the back end's range, words of q - 1 throughout."""
+@pytest.mark.parametrize("bits", [60, 50, 49, 30])
+@pytest.mark.parametrize("logn,limbs", [(9, 2), (11, 2), (13, 2), (16, 2), (16, 18), (17, 2), (17, 9)])
+def test_passes_of_the_largest_words(oracle, capi, monkeypatch, logn, limbs, bits):
+    """Lazy ranges of both back ends, primes at the ends of FP64's; words of q - 1 throughout, and random ones.  FP64 passes over 36 * 2^16
+    words and more work out the twiddles of their last two stages from two entries of the table: every block of the limb."""
     monkeypatch.setenv("CAHEL_HIP_NO_ONE_PASS", "1")
-    cahel, parms, ctx, p = make_pair(oracle, logn, [bits] * 3, 1)
+    cahel, parms, ctx, p = make_pair(oracle, logn, [bits] * (limbs + 1), 1)
     lib, h = capi.lib(), ctx.he_handle()
-    x = rand_limbs(p, np.random.default_rng(logn), range(2), n_polys=2)
-    for i in range(2):
+    x = rand_limbs(p, np.random.default_rng(logn), range(limbs), n_polys=2)
+    for i in range(limbs):
         x[1, i, :] = p.moduli[i] - 1
     d = DeviceArray(capi, host=x)
-    capi.check(lib.he_ntt_forward(h, d.ptr, 2, 2, 2, 0, 2, 0, None))
+    capi.check(lib.he_ntt_forward(h, d.ptr, 2, limbs, limbs, 0, limbs, 0, None))
     got = d.numpy()
     assert all((got[k] == p.ntt_fwd(x[k].copy())).all() for k in range(2))
     capi.check(lib.he_memcpy_h2d(d.ptr, x.ctypes.data, x.nbytes, None))
-    capi.check(lib.he_ntt_inverse(h, d.ptr, 2, 2, 2, 0, 2, 0, None))
+    capi.check(lib.he_ntt_inverse(h, d.ptr, 2, limbs, limbs, 0, limbs, 0, None))
     got = d.numpy()
     assert all((got[k] == p.ntt_inv(x[k].copy())).all() for k in range(2))
 
