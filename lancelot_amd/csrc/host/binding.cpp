@@ -185,6 +185,39 @@ PYBIND11_MODULE(pyCAHEL, m) {
                  return a;
              },
              py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count") = 1)
+        .def("decrypt_decode_each",
+             [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, CAHELGPUCKKSEncoder &e, const std::vector<const CAHELGPUCiphertext *> &cts) {
+                 py::array_t<double> out((py::ssize_t)(cts.size() * e.decoded_slots()));
+                 double *values = out.mutable_data();
+                 {
+                     py::gil_scoped_release release;
+                     k.decrypt_decode_each(c, e, cts, values);
+                 }
+                 return out;
+             },
+             py::arg("context"), py::arg("encoder"), py::arg("ciphertexts"))
+        // decrypt_decode_complex_many of the ciphertexts and encode_encrypt_many of the values (in this order, as far as what they draw is
+        // concerned); the encryption is on the device's queue before the decoded values are waited for
+        .def("decrypt_decode_complex_and_encrypt_many",
+             [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, const std::vector<const CAHELGPUCiphertext *> &cts,
+                std::size_t slots, std::size_t count, CAHELGPUCKKSEncoder &e, const CAHELGPUPublicKey &pk,
+                py::array_t<double, py::array::c_style> v, double scale) {
+                 if (v.ndim() != 2) throw std::invalid_argument("values must be a two-dimensional array");
+                 py::array_t<std::complex<double>> a(
+                     {(py::ssize_t)cts.size(), (py::ssize_t)(count > slots || slots > c.poly_degree() ? 0 : count)});
+                 double *decoded = reinterpret_cast<double *>(a.mutable_data());
+                 const double *values = v.data();
+                 const std::size_t items = (std::size_t)v.shape(0), length = (std::size_t)v.shape(1);
+                 std::vector<CAHELGPUCiphertext> encrypted;
+                 {
+                     py::gil_scoped_release release;
+                     k.decrypt_decode_many(c, cts, slots, count, decoded, true,
+                                           [&] { encrypted = e.encode_encrypt_many(c, pk, values, items, length, length, scale); });
+                 }
+                 return py::make_tuple(a, std::move(encrypted));
+             },
+             py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count"), py::arg("encoder"), py::arg("public_key"),
+             py::arg("values").noconvert(), py::arg("scale"))
         .def("to_numpy", [](const CAHELGPUSecretKey &s, const CAHELGPUContext &c) {
             return to_host(s.secret_key_array(), {(py::ssize_t)c.size_qp(), (py::ssize_t)c.poly_degree()});
         });
@@ -402,6 +435,8 @@ PYBIND11_MODULE(pyCAHEL, m) {
         return r;
     });
     m.def("_trim_pool", &DeviceBuffer::trim_pool);
+    // a point on the current lane's queue, for the time between two of them by the device's clock
+    py::class_<DeviceMark>(m, "_mark").def(py::init<>()).def("seconds_since", &DeviceMark::seconds_since, nogil);
     m.def("_synchronize", []() { cahel::synchronize_lanes(); });
     m.def("_set_lane", &cahel::set_lane);
     m.def("_current_lane", &cahel::current_lane);

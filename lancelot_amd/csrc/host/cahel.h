@@ -11,6 +11,7 @@
 #include <atomic>
 #include <cstddef>
 #include <cstdint>
+#include <functional>
 #include <iosfwd>
 #include <memory>
 #include <stdexcept>
@@ -117,6 +118,32 @@ private:
 // enqueues like the others, may be used on any lane at once: a plaintext waits for its encoding where another lane reads it.
 he_stream current_stream();
 int current_lane();
+
+// A point on the current lane's queue.
+class DeviceMark {
+public:
+    DeviceMark() {
+        check_status(he_event_create(&event_), "he_event_create");
+        if (const int status = he_event_record(event_, current_stream())) {
+            (void)he_event_destroy(event_);
+            check_status(status, "he_event_record");
+        }
+    }
+    DeviceMark(const DeviceMark &) = delete;
+    DeviceMark &operator=(const DeviceMark &) = delete;
+    ~DeviceMark() { (void)he_event_destroy(event_); }
+    // by the device's clock; waits for both
+    double seconds_since(const DeviceMark &earlier) const {
+        float ms = 0;
+        check_status(he_event_synchronize(earlier.event_), "he_event_synchronize");
+        check_status(he_event_synchronize(event_), "he_event_synchronize");
+        check_status(he_event_elapsed_ms(earlier.event_, event_, &ms), "he_event_elapsed_ms");
+        return 1e-3 * ms;
+    }
+
+private:
+    he_event event_ = nullptr;
+};
 int lane_count();
 void set_lane(int lane);
 void synchronize_lanes();
@@ -371,6 +398,8 @@ public:
     cahel::parms_id_type parms_id_ = cahel::parms_id_zero;
 };
 
+class CAHELGPUCKKSEncoder;
+
 // include/secretkey.h:412-659
 class CAHELGPUSecretKey {
 public:
@@ -399,9 +428,10 @@ public:
     // Real parts of the first `count` slots of every ciphertext, [items][count] row-major: decrypt + decode of all of
     // them with one launch per stage (not in the reference).  All ciphertexts: size 2, one level, one scale;
     // `slots` = the encoder's slot count.
-    // both: (re, im) pairs, [items][count][2].
+    // both: (re, im) pairs, [items][count][2].  meanwhile: what the caller enqueues behind this work before it waits for the values.
     void decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
-                             std::size_t slots, std::size_t count, double *destination, bool both = false);
+                             std::size_t slots, std::size_t count, double *destination, bool both = false,
+                             const std::function<void()> &meanwhile = nullptr);
     std::vector<double> decrypt_decode_many(const CAHELGPUContext &context,
                                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots,
                                             std::size_t count) {
@@ -409,6 +439,10 @@ public:
         decrypt_decode_many(context, ciphers, slots, count, out.data());
         return out;
     }
+    // The real parts of all slots of every ciphertext, one after the other in destination (decoded_slots() each): decrypt and decode of each,
+    // the next one's enqueued before the values of the one in front are waited for.  Not in the reference.
+    void decrypt_decode_each(const CAHELGPUContext &context, CAHELGPUCKKSEncoder &encoder,
+                             const std::vector<const CAHELGPUCiphertext *> &ciphers, double *destination);
     const uint64_t *secret_key_array() const { return sk_powers_.get(); }
 
 private:
@@ -462,6 +496,8 @@ public:
         return destination;
     }
     void decode(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::vector<double> &destination);
+    // values of a decoding (the full slot count where no message has fixed another)
+    std::size_t decoded_slots() const { return sparse_slots_ ? sparse_slots_ : slots_; }
     // complex values of the first `count` slots, interleaved
     void decode_values(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count,
                        std::vector<double> &interleaved);

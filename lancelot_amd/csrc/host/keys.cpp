@@ -5,6 +5,7 @@
 // sampled polynomial, handed out in the order the polynomials are drawn.
 #include <cmath>
 #include <cstring>
+#include <optional>
 #include <string>
 
 #include "cahel.h"
@@ -230,9 +231,13 @@ void CAHELGPUSecretKey::decrypt(const CAHELGPUContext &context, const CAHELGPUCi
 }
 
 void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, const std::vector<const CAHELGPUCiphertext *> &ciphers,
-                                            std::size_t slots, std::size_t count, double *destination, bool both) {
+                                            std::size_t slots, std::size_t count, double *destination, bool both,
+                                            const std::function<void()> &meanwhile) {
     if (!gen_flag_) throw std::logic_error("secret key has not been generated");
-    if (ciphers.empty()) return;
+    if (ciphers.empty()) {
+        if (meanwhile) meanwhile();
+        return;
+    }
     if (ciphers.size() > 16384) throw std::invalid_argument("too many ciphertexts");
     const CAHELGPUCiphertext &first = *ciphers[0];
     for (const CAHELGPUCiphertext *ct : ciphers) {
@@ -271,9 +276,47 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
     if (status != HE_OK && staged) ring.fence(st);   // (what was launched before the failure may still write the block)
     check_status(status, "he_decrypt_decode_batch");
     if (staged) {
-        check_status(he_stream_synchronize(st), "synchronisation failed");
+        PinnedRing::Held held(ring, st);
+        if (meanwhile) meanwhile();
+        held.wait();
         std::memcpy(destination, out, bytes);
     } else {
+        if (meanwhile) meanwhile();
         check_status(he_memcpy_d2h(destination, out, bytes, st), "download");
     }
+}
+
+void CAHELGPUSecretKey::decrypt_decode_each(const CAHELGPUContext &context, CAHELGPUCKKSEncoder &encoder,
+                                            const std::vector<const CAHELGPUCiphertext *> &ciphers, double *destination) {
+    he_context *h = context.handle();
+    he_stream st = context.stream();
+    PinnedRing &ring = PinnedRing::of_thread();
+    std::optional<PinnedRing::Held> ahead;   // of the ciphertext in front
+    const double *values = nullptr;
+    std::size_t count = 0;
+    auto finish = [&] {
+        if (!ahead) return;
+        ahead->wait();
+        std::memcpy(destination, values, count * sizeof(double));
+        destination += count;
+        ahead.reset();
+    };
+    for (const CAHELGPUCiphertext *ct : ciphers) {
+        if (!ct) throw std::invalid_argument("encrypted is not valid");
+        CAHELGPUPlaintext plain(context);
+        decrypt(context, *ct, plain);
+        const std::size_t taken = encoder.decode_count(context, plain, 0);   // (all slots)
+        const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
+        DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)taken));
+        double *host = static_cast<double *>(ring.take(taken * sizeof(double)));
+        const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)taken, plain.scale(), host, (uint32_t)taken,
+                                               ws.get(), st);
+        PinnedRing::Held held(ring, st);
+        check_status(status, "he_ckks_decode_real");
+        finish();
+        values = host;
+        count = taken;
+        ahead.emplace(std::move(held));
+    }
+    finish();
 }

@@ -10,6 +10,13 @@ namespace cahel {
 // work: it is rewritten only when the work is done, and nothing else waits for it.  Blocks grow on demand up to kMaxBytes and
 // are given back when the thread ends (worker threads of a pool come and go).
 class PinnedRing {
+    struct Block {
+        void *ptr = nullptr;
+        std::size_t bytes = 0;
+        he_event event = nullptr;
+        bool busy = false, held = false;
+    };
+
 public:
     static constexpr int kBlocks = 4;
     static constexpr std::size_t kMaxBytes = std::size_t(16) << 20;
@@ -30,7 +37,8 @@ public:
     // the next block, at least `bytes` (at most kMaxBytes) large, with no device work left on it
     void *take(std::size_t bytes) {
         if (bytes > kMaxBytes) throw std::logic_error("staging block too large");
-        current_ = (current_ + 1) % kBlocks;
+        do current_ = (current_ + 1) % kBlocks;
+        while (blocks_[current_].held);   // (at most two are)
         Block &b = blocks_[current_];
         if (b.busy) {
             check_status(he_event_synchronize(b.event), "he_event_synchronize");
@@ -54,13 +62,29 @@ public:
         b.busy = true;
     }
 
-private:
-    struct Block {
-        void *ptr = nullptr;
-        std::size_t bytes = 0;
-        he_event event = nullptr;
-        bool busy = false;
+    // The block taken last, which the work enqueued on `stream` so far writes, kept out of turn for what its owner does before it waits
+    // for the block: other blocks may be taken, and other work enqueued, in between.
+    class Held {
+    public:
+        Held(PinnedRing &ring, he_stream stream) : block_(&ring.blocks_[ring.current_]) {
+            ring.fence(stream);
+            block_->held = true;
+        }
+        Held(Held &&o) noexcept : block_(o.block_) { o.block_ = nullptr; }
+        Held &operator=(Held &&) = delete;
+        ~Held() {
+            if (block_) block_->held = false;
+        }
+        void wait() {
+            check_status(he_event_synchronize(block_->event), "he_event_synchronize");
+            block_->busy = false;
+        }
+
+    private:
+        Block *block_;
     };
+
+private:
     Block blocks_[kBlocks];
     int current_ = 0;
 };
