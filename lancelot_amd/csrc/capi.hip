@@ -43,6 +43,7 @@ struct Level {
     uint32_t modup_max_rows = 0, modup_max_copy = 0;
     bool batched = false;
     double *d_mats_fp = nullptr;         // the digit matrices as doubles, when every prime is below 2^50
+    double *d_rows_mixed = nullptr;      // FP64 rows of a level with other primes (BconvRows::rows_mixed)
     double *d_rows_up = nullptr;         // ... and as the fused kernel reads them (BconvRows::rows_fp)
     int32_t *d_mx_up = nullptr;          // the same matrices as 7-bit digits for the int8 matrix cores (N = 2^16)
 };
@@ -92,6 +93,7 @@ struct he_context {
     std::vector<uint64_t> h_phat_inv;    // host copy of d_phat_inv
     double *d_psi_fp = nullptr, *d_ipsi_fp = nullptr, *d_fp_consts = nullptr;  // FP64 back end tables
     double *d_phat_mod_q_fp = nullptr;   // the P -> Ql matrix as doubles
+    double *d_mixed_down = nullptr, *d_mixed_mdr = nullptr;   // BconvRows::rows_mixed
     double *d_rows_down = nullptr, *d_rows_mdr = nullptr;   // ... as the fused kernel reads it (BconvRows::rows_fp), and times P^-1 mod q_j (merged
                                                             // ModDown + rescale)
     bool fuse_rows = true;       // environment CAHEL_HIP_NO_FUSED_BCONV=1: conversion kernel, then the rows pass
@@ -140,6 +142,20 @@ void conversion_row(std::vector<double> &rows, uint32_t n_in, uint64_t q, Entry 
     }
     rows.push_back(centred(shift, q));
     rows.push_back(centred((uint64_t)((1ull << 50) % q), q) * 0x1p-50);
+}
+
+// One row of BconvRows::rows_mixed (nothing reads that of a prime from 2^50 on)
+template <class Entry>
+void mixed_row(std::vector<double> &rows, uint32_t n_in, uint64_t q, Entry entry) {
+    const size_t at = rows.size();
+    rows.resize(at + kMixedRow, 0.0);
+    if (q >> 50) return;
+    for (uint32_t i = 0; i < n_in && i < 8; i++) {
+        rows[at + i] = centred((uint64_t)(((unsigned __int128)entry(i) << 30) % q), q);
+        rows[at + 8 + i] = centred(entry(i) % q, q);
+    }
+    rows[at + 16] = centred((1ull << 34) % q, q) * 0x1p-34;
+    rows[at + 17] = centred((1ull << 30) % q, q);
 }
 
 // One record of BconvRows::mx_tab: up to four rows of a conversion matrix with at most 8 columns as 7-bit digits of
@@ -602,17 +618,21 @@ int he_context_create(const he_context_desc *d, he_context **out) {
             for (size_t i = 0; i < entries; i++) pfp[i] = (double)d->phat_mod_q[i];
             rc = upload(ctx, &ctx->d_phat_mod_q_fp, pfp.data(), pfp.size());
             if (!rc && d->size_p <= 8) {
-                std::vector<double> down, mdr;
+                std::vector<double> down, mdr, mixed_down, mixed_mdr;
                 for (uint32_t jq = 0; jq < d->size_q; jq++) {
                     const uint64_t q = d->moduli[jq];
                     auto entry = [&](uint32_t k) { return d->phat_mod_q[(size_t)jq * d->size_p + k]; };
                     conversion_row(down, d->size_p, q, entry);
                     // (P / p_k) P^-1 mod q_j: delta_j P^-1 straight from the conversion
-                    conversion_row(mdr, d->size_p, q,
-                                   [&](uint32_t k) { return (uint64_t)((unsigned __int128)entry(k) * d->pinv_mod_q[2 * jq] % q); });
+                    auto by_p = [&](uint32_t k) { return (uint64_t)((unsigned __int128)entry(k) * d->pinv_mod_q[2 * jq] % q); };
+                    conversion_row(mdr, d->size_p, q, by_p);
+                    mixed_row(mixed_down, d->size_p, q, entry);
+                    mixed_row(mixed_mdr, d->size_p, q, by_p);
                 }
                 rc = upload(ctx, &ctx->d_rows_down, down.data(), down.size());
                 if (!rc) rc = upload(ctx, &ctx->d_rows_mdr, mdr.data(), mdr.size());
+                if (!rc) rc = upload(ctx, &ctx->d_mixed_down, mixed_down.data(), mixed_down.size());
+                if (!rc) rc = upload(ctx, &ctx->d_mixed_mdr, mixed_mdr.data(), mixed_mdr.size());
             }
             if (!rc && d->log_n == 16 && d->size_p <= 8) {
                 // the same matrix for the int8 matrix cores: rows in groups of four with the bytes of the rescale term,
@@ -765,6 +785,17 @@ int he_context_set_level(he_context *ctx, const he_level_desc *d) {
                     rc = upload(ctx, &lv.d_mx_up, tab.data(), tab.size());
                     if (rc) return rc;
                 }
+            }
+            else if (ctx->use_fp) {
+                std::vector<double> rows;
+                for (uint32_t dg = 0; dg < beta; dg++) {
+                    const Digit &g = lv.digits[dg];
+                    for (uint32_t r = 0; r < g.n_out; r++)
+                        mixed_row(rows, g.size, ctx->h_moduli[table_of(ctx, L, r < g.start ? r : r + g.size)],
+                                  [&](uint32_t i) { return mats[g.mat_off + (size_t)r * g.size + i]; });
+                }
+                rc = upload(ctx, &lv.d_rows_mixed, rows.data(), rows.size());
+                if (rc) return rc;
             }
             rc = upload(ctx, &lv.d_modup_descs, up.data(), up.size());
             if (rc) return rc;
@@ -1023,7 +1054,7 @@ int modup_impl(const he_context *ctx, uint32_t L, const uint64_t *c, uint32_t c_
     const int inv_backend = backend_for(ctx, inv.map);
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, lv->n_modup_jobs * items);
     BconvRows conv{ws, out, skip_own ? nullptr : c, (size_t)c_item_stride * n, LimbMap{LK, 0, L, ctx->size_q}, ctx->size_p, lv->beta, items, 1,
-                   fp_for_level(ctx, L) ? lv->d_rows_up : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr, 0};
+                   fp_for_level(ctx, L) ? lv->d_rows_up : nullptr, 0, lv->d_mx_up, nullptr, lv->d_mats, nullptr, lv->d_rows_mixed, 0};
     if (fused && tiles) use_tiles(ctx, inv, inv_backend, conv, tiles, L);
     if (tin) HE_HIP(launch_tensor_intt_blocks(inv, *tin, items, inv_backend, S(s)));
     HE_HIP(launch_ntt_inverse(inv, items, inv_backend, S(s), tin != nullptr, source_intt));
@@ -1139,7 +1170,7 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     const bool source_intt = reduce_in_ntt && source_intt_ok(ctx, n_polys * L);
     const uint32_t units = n_polys <= 4 ? n_polys : 2, items = n_polys / units;
     BconvRows conv{cx, ws, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, units, items, 0,
-                   fp_for_level(ctx, L) ? ctx->d_rows_down : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr, 0};
+                   fp_for_level(ctx, L) ? ctx->d_rows_down : nullptr, 0, nullptr, nullptr, ctx->d_phat_mod_q, nullptr, ctx->d_mixed_down, 0};
     if (fused && (size_t)n_polys * K <= scratch_limbs) use_tiles(ctx, inv, inv_backend, conv, scratch, K);
     HE_HIP(launch_ntt_inverse(inv, n_polys, inv_backend, S(s), inverted, source_intt));
     if (reduce_in_ntt) {
@@ -1430,7 +1461,7 @@ int ksr_impl(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *
     const bool fused = fuse_rows_ok(ctx, lv, L);
     BconvRows conv{cx, delta, nullptr, 0, LimbMap{LK, 0, L, ctx->size_q}, K, 2, items, 0,
                    fp_for_level(ctx, L) ? ctx->d_rows_mdr : nullptr, 1, ctx->d_mx_down,
-                   ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q, 0};
+                   ctx->d_mx_last ? ctx->d_mx_last + (size_t)(L - 1) * 4 * kMxRecord : nullptr, ctx->d_phat_mod_q, ctx->d_pinv_mod_q, ctx->d_mixed_mdr, 0};
     if (fused && (size_t)polys * (K + 1) <= digit_limbs(ctx, lv, L, items)) use_tiles(ctx, inv, inv_backend, conv, w.y, K + 1);
     HE_HIP(launch_ntt_inverse(inv, polys, inv_backend, S(s), inverted, source_intt));
     // one special prime: the conversion is the reduction of its coefficients modulo every q_j, which the prologue of (4)

@@ -359,6 +359,9 @@ struct BconvRows {
     // levels with a prime from 2^50 on (rows_fp == nullptr): the matrix in integers, and, mdr, P^-1 mod q_j (Shoup pairs)
     const uint64_t *mat;
     const uint64_t *w;
+    // ... and of output limbs below 2^50 a row of kMixedRow doubles, in rows_fp's order: 8 entries times 2^30 mod q, the 8 entries (mdr: times
+    // P^-1), all in (-q/2, q/2), 2^34 mod q times 2^-34, 2^30 mod q
+    const double *rows_mixed;
     // N = 2^16: the input limbs are in the order of conversion_word, with rows_fp as doubles, less 2^49 (not for the matrix kernel); ModDown: in [items][units]
     // [K][N], mdr: [K + 1][N] with t's limb in front
     int tiled;
@@ -370,8 +373,9 @@ struct BconvExtra {
     const void *w;               // w or mx_last
     const uint64_t *copy_base;
     size_t copy_item_stride;
+    const double *rows_mixed;
 };
-constexpr uint32_t kMxRecord = 144, kConversionRow = 10;
+constexpr uint32_t kMxRecord = 144, kConversionRow = 10, kMixedRow = 18;
 // whether `inv`, the inverse transform that ends in b's inputs, should leave them tiled (in a buffer of their own: its last pass is in
 // place otherwise)
 bool bconv_wants_tiles(const NttArgs &inv, int inv_backend, const BconvRows &b, const Tuning &tune);

@@ -664,7 +664,7 @@ hipError_t launch_bconv_rows(const NttArgs &a, const BconvRows &b, int backend, 
     h.h1 = b.units | b.K << 16;
     h.h2 = compute_groups | copy_groups << 16;
     if (mx) {
-        const BconvExtra x{b.mx_tab, b.mx_last, b.copy_base, b.copy_item_stride};
+        const BconvExtra x{b.mx_tab, b.mx_last, b.copy_base, b.copy_item_stride, nullptr};
         if (b.mdr)
             hipLaunchKernelGGL(bconv_rows_mx_kernel<true>, dim3(h.h4), dim3(256), 0, s, HE_HEAD_ARGS(h), x);
         else

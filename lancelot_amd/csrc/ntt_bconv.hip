@@ -104,7 +104,7 @@ struct ConvFp {
     }
 };
 
-// Conversion in integers (any primes); the results go to the arithmetic of the output limb.
+// Conversion of integer inputs (any primes) in the arithmetic of the output limb.
 template <int NIN, bool MDR>
 struct ConvInt {
     Split30 x[NIN][4];
@@ -141,32 +141,76 @@ struct ConvInt {
 #pragma unroll
         for (int j = 0; j < 4; j++) rr[j] = sub_mod(t[j], mul_shoup(s[j], w, q), q);
     }
-    template <class A>
-    __device__ __forceinline__ void convert(typename A::V *v, const NttArgs &a, const BconvExtra &b, const BconvUnit &d, uint32_t r,
-                                            uint32_t table, const A &) const {
-        uint64_t s[4];
-        sums(s, a, b, d, r, table);
+    __device__ __forceinline__ void convert(uint64_t *v, const NttArgs &a, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t table,
+                                            const IntArith &) const {
+        sums(v, a, b, d, r, table);
         if constexpr (MDR) {
             const uint64_t q = scalar(a.moduli)[table], r1 = scalar(a.barrett)[2 * table + 1];
             const Shoup w = scalar_shoup(static_cast<const uint64_t *>(b.w), r);
 #pragma unroll
-            for (int j = 0; j < 4; j++) s[j] = add_mod(mul_shoup(s[j], w, q), barrett64(rr[j], q, r1), q);
+            for (int j = 0; j < 4; j++) v[j] = add_mod(mul_shoup(v[j], w, q), barrett64(rr[j], q, r1), q);
         }
+    }
+    // An output limb below 2^50: x = xh 2^30 + xl in FP64, sum of xh (M 2^30 mod q) + xl M (mod q), at most 1.01 q in magnitude.  As
+    // ConvFp::sum: a product is below 2^80, hi runs around 1.5 2^86, where doubles are the multiples of 2^34, with sums below 2^85, and
+    // what is left of a product is an integer of at most 2^33.  Four operations and a conversion a product, where integers take four
+    // multiply-adds a term and sixty instructions to put a word together and reduce it.  Chains of 60 / 40 bits, integers -> FP64, one
+    // product: n = 2^15, 10 of 12 limbs, K = 3 62.1 -> 60.7 us; n = 2^16, 12 + 4 limbs 91.6 -> 90.3, a batch of four 244 -> 239; a batch of
+    // 8, n = 2^14, 8 limbs, K = 2 98.4 -> 94.6.
+    __device__ __forceinline__ void convert(double *v, const NttArgs &, const BconvExtra &b, const BconvUnit &d, uint32_t r, uint32_t,
+                                            const FpArith &ar) {
+        // (the halves stay integers between the rows: as doubles of all inputs they would not fit in the registers)
+#pragma unroll
+        for (int k = 0; k < NIN; k++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) asm volatile("" : "+v"(x[k][j].lo), "+v"(x[k][j].hi));
+        if constexpr (MDR) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) asm volatile("" : "+v"(rr[j]));
+        }
+        const ScalarF64 row = scalar(b.rows_mixed) + (size_t)(d.row_off + r) * kMixedRow;
+        const FpMod m = ar.m;
+        double hi[4], lo[4];
+        auto add = [&](int j, double x, double w) {
+            const double t = __builtin_fma(x, w, hi[j]);
+            lo[j] += __builtin_fma(x, w, -(t - hi[j]));
+            hi[j] = t;
+        };
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            if constexpr (std::is_same<A, FpArith>::value)
-                v[j] = fp_from_u64(s[j]);
-            else
-                v[j] = s[j];
+            hi[j] = 0x1.8p86;
+            lo[j] = 0.0;
+            if constexpr (MDR) {
+                const Split30 s = split30(rr[j]);
+                lo[j] = (double)s.lo;
+                add(j, (double)s.hi, row[17]);
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < NIN; k++) {
+            if ((uint32_t)k >= d.n_in) break;
+            const double wh = row[k], wl = row[8 + k];
+#pragma unroll
+            for (int j = 0; j < 4; j++) {
+                add(j, (double)x[k][j].hi, wh);
+                add(j, (double)x[k][j].lo, wl);
+            }
+        }
+        const double c = row[16];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const double big = hi[j] - 0x1.8p86, h = big * c, l = __builtin_fma(big, c, -h);
+            const double k = __builtin_rint(__builtin_fma(lo[j], m.qinv, h * m.qinv));
+            v[j] = (__builtin_fma(-k, m.q, h) + l) + lo[j];
         }
     }
 };
 
-// FP: the whole level is below 2^50; otherwise the conversion is done in integers and bit `table` of a.fp_mask says in which
-// arithmetic the limb is transformed
+// BE: NTT_BACKEND_FP: the whole level is below 2^50; otherwise the inputs are integers, and MIXED: bit `table` of a.fp_mask says in which
+// arithmetic the limb is converted and transformed
 // TILED: the input limbs are in the order of conversion_word (BconvRows::tiled)
-template <int LD, bool FP, int NIN, bool MDR, bool TILED>
-__global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(FP || NIN <= 4 ? 4 : 2)))
+template <int LD, int BE, int NIN, bool MDR, bool TILED>
+__global__ __launch_bounds__(1 << (kTileLog - 2)) __attribute__((amdgpu_waves_per_eu(BE == NTT_BACKEND_FP || NIN <= 4 ? 4 : 2)))
 void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     using T4 = Tile4<kTileLog, LD>;
     constexpr int LOGC = kTileLog - LD, NB = T4::kBlocks;
@@ -210,7 +254,7 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     const uint32_t n_rows = MDR ? d.n_out - 1 : d.n_out, r_begin = grp * rows_per;
     const uint32_t r_end = r_begin + rows_per < n_rows ? r_begin + rows_per : n_rows;
     if (r_begin >= n_rows) return;
-    typename std::conditional<FP, ConvFp<NIN, MDR, TILED>, ConvInt<NIN, MDR>>::type conv;
+    typename std::conditional<BE == NTT_BACKEND_FP, ConvFp<NIN, MDR, TILED>, ConvInt<NIN, MDR>>::type conv;
     const uint64_t *x = d.in;
     {
         uint64_t w[NIN][4], tw[4];
@@ -250,8 +294,10 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
 #pragma unroll
             for (int j = 0; j < 4; j++) (dst + step(NB - 1, j))[out0] = A::to_word(v[j]);
         };
-        if constexpr (FP) {
+        if constexpr (BE == NTT_BACKEND_FP) {
             row(fp_arith(a, table));
+        } else if constexpr (BE == NTT_BACKEND_INT) {
+            row(int_arith(a, table));
         } else {
             if ((a.fp_mask >> table) & 1)
                 row(fp_arith(a, table));
@@ -261,11 +307,11 @@ void bconv_rows4_kernel(HE_HEAD_PARAMS, BconvExtra b) {
     }
 }
 
-template <bool FP, int NIN, bool MDR, bool TILED>
+template <int BE, int NIN, bool MDR, bool TILED>
 hipError_t launch_nin(const NttHead &h, uint32_t log_n, const BconvExtra &b, hipStream_t s) {
 #define HE_CASE(LD)                                                                                                              \
     case LD:                                                                                                                     \
-        hipLaunchKernelGGL((bconv_rows4_kernel<LD, FP, NIN, MDR, TILED>), dim3(h.h4), dim3(1 << (kTileLog - 2)), 0, s, HE_HEAD_ARGS(h), b); \
+        hipLaunchKernelGGL((bconv_rows4_kernel<LD, BE, NIN, MDR, TILED>), dim3(h.h4), dim3(1 << (kTileLog - 2)), 0, s, HE_HEAD_ARGS(h), b); \
         break;
     if constexpr (TILED) {
         switch (log_n - 8) {
@@ -288,14 +334,17 @@ hipError_t launch_bconv_rows4(const NttHead &head, const BconvRows &b, hipStream
     NttHead h = head;
     const uint32_t log_n = h.h0 & 31, groups = (h.h2 & 0xffff) + (h.h2 >> 16);
     const uint64_t wgs = (uint64_t)b.units * (b.items ? b.items : 1) * (1u << (log_n - kTileLog)) * groups;
-    if (log_n < 12 || log_n > 16 || b.K == 0 || b.K > 8 || (!b.rows_fp && !b.mat) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
+    if (log_n < 12 || log_n > 16 || b.K == 0 || b.K > 8 || (!b.rows_fp && (!b.mat || (h.fp_mask && !b.rows_mixed))) || wgs == 0 || wgs > most_workgroups(1 << (kTileLog - 2)))
         return hipErrorInvalidValue;
     h.h4 = (uint32_t)wgs;
-    const BconvExtra x{b.rows_fp ? static_cast<const void *>(b.rows_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride};
-#define HE_TILED(FP, NIN, MDR) (b.tiled ? launch_nin<FP, NIN, MDR, true>(h, log_n, x, s) : launch_nin<FP, NIN, MDR, false>(h, log_n, x, s))
-#define HE_NIN(FP, MDR) (b.K <= 4 ? HE_TILED(FP, 4, MDR) : HE_TILED(FP, 8, MDR))
-    if (b.rows_fp) return b.mdr ? HE_NIN(true, true) : HE_NIN(true, false);
-    return b.mdr ? HE_NIN(false, true) : HE_NIN(false, false);
+    const BconvExtra x{b.rows_fp ? static_cast<const void *>(b.rows_fp) : b.mat, b.w, b.copy_base, b.copy_item_stride, b.rows_mixed};
+#define HE_TILED(BE, NIN, MDR) (b.tiled ? launch_nin<BE, NIN, MDR, true>(h, log_n, x, s) : launch_nin<BE, NIN, MDR, false>(h, log_n, x, s))
+#define HE_NIN(BE, MDR) (b.K <= 4 ? HE_TILED(BE, 4, MDR) : HE_TILED(BE, 8, MDR))
+#define HE_MDR(BE) (b.mdr ? HE_NIN(BE, true) : HE_NIN(BE, false))
+    if (b.rows_fp) return HE_MDR(NTT_BACKEND_FP);
+    // (no limb on FP64: without that branch the kernel needs fewer registers)
+    return h.fp_mask ? HE_MDR(NTT_BACKEND_MIXED) : HE_MDR(NTT_BACKEND_INT);
+#undef HE_MDR
 #undef HE_NIN
 #undef HE_TILED
 }

@@ -110,6 +110,44 @@ def test_entry_points_with_fused_conversion(oracle, capi, monkeypatch, logn, bit
                 assert (got[k] == p.rescale(np.stack([p.add(ct3[k][b], ks[b]) for b in range(2)]))).all(), ("batch", L, k)
 
 
+@pytest.mark.parametrize("logn,bits,size_p,levels", [
+    (12, [60, 50, 30, 49, 60, 20, 60, 60], 2, (6, 3)),
+    (13, [50, 20, 50, 60, 60, 60], 3, (3, 2)),
+    (14, [40] * 4 + [50] * 3 + [60], 4, (4, 3)),
+    (15, [60, 30, 50, 40, 40] + [60] * 5, 5, (5, 2)),
+    (16, [60] + [40] * 3 + [50] * 3 + [60] * 2 + [50] + [60] * 4, 7, (7, 4)),
+    (16, [50, 49, 30, 60] * 2 + [60, 30, 50, 60, 60, 60, 60, 60], 8, (8, 3)),
+    (16, [50, 49, 30, 60, 60, 60], 2, (4, 3)),
+])
+def test_mixed_conversions_of_the_largest_words(oracle, capi, logn, bits, size_p, levels):
+    """Conversions of integer inputs into limbs on FP64: every coefficient of every input q - 1, then random ones; digits of two to eight
+    limbs and part of one, with the data limbs or only some of them, and none or some of the special ones, below 2^50."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    rng = np.random.default_rng(300 + logn)
+    lib, h, K, n = capi.lib(), ctx.he_handle(), p.size_p, p.n
+    for L in levels:
+        tables = [p.table_index(L, t) for t in range(L + K)]
+        dy, ws = DeviceArray(capi, shape=(-(-L // K), L + K, n)), DeviceArray(capi, shape=(2 * L, n))
+        top = np.stack([np.full(n, p.moduli[t] - 1, dtype=np.uint64) for t in tables])
+        for fill in (top, rand_limbs(p, rng, tables)):
+            c = p.ntt_fwd(np.ascontiguousarray(fill[:L]), list(range(L)))
+            dc = DeviceArray(capi, host=c)
+            capi.check(lib.he_modup(h, L, dc.ptr, dy.ptr, ws.ptr, None))
+            assert (dy.numpy() == p.modup(c)).all(), ("modup", L)
+            cx = np.ascontiguousarray(p.ntt_fwd(fill.copy(), tables))
+            dcx, dout = DeviceArray(capi, host=cx), DeviceArray(capi, shape=(1, L, n))
+            capi.check(lib.he_moddown(h, L, dcx.ptr, dout.ptr, 1, 0, ws.ptr, None))
+            assert (dout.numpy()[0] == p.moddown(cx)).all(), ("moddown", L)
+        host_evk = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(p.size_q // K)]
+        dev_evk = [DeviceArray(capi, host=k) for k in host_evk]
+        c, ct = rand_limbs(p, rng, range(L)), rand_limbs(p, rng, range(L), n_polys=2)
+        dc, dct, dout = DeviceArray(capi, host=c), DeviceArray(capi, host=ct), DeviceArray(capi, shape=(2, L - 1, n))
+        kws = DeviceArray(capi, shape=(lib.he_keyswitch_workspace_words(h, L),))
+        capi.check(lib.he_keyswitch_rescale(h, L, dc.ptr, capi.evk_array([d.ptr for d in dev_evk]), dct.ptr, dout.ptr, 0, kws.ptr, None))
+        ks = p.key_switch(c, host_evk)
+        assert (dout.numpy() == p.rescale(np.stack([p.add(ct[b], ks[b]) for b in range(2)]))).all(), ("keyswitch_rescale", L)
+
+
 @pytest.mark.parametrize("no_fused", ["0", "1"])
 @pytest.mark.parametrize("logn,bits,size_p,levels", CASES + [(11, [45, 40, 40, 50], 1, (3, 2)), (12, [60, 40, 50, 45, 30, 59, 60, 60], 2, (6, 3))])
 def test_multiply_relin_rescale_entry_point(oracle, capi, monkeypatch, logn, bits, size_p, levels, no_fused):
