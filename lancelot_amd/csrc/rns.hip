@@ -785,7 +785,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) v
         } else {
             // two neighbouring words per thread (see turned) of half the items; the gathers of a step are independent of the running
             // sums, several steps' are in flight
-            constexpr int H = I / 2;
+            constexpr int H = (I + 1) / 2;
             const uint32_t half = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x / (kThreads / 2)) * H;
             const uint32_t j2 = bx * kThreads + 2 * (threadIdx.x % (kThreads / 2));
             const uint64_t *src[H];
@@ -1684,18 +1684,34 @@ hipError_t launch_hoist_inner(const Tables &t, const Tuning &tune, const uint64_
         return hipGetLastError();
     }
     const bool p_xcd_ok = !no_xcd && (nb * rows) % 8 == 0;
+    const bool stretches = !local && !no_contig && stretch_local && nb >= 128 && (nb >> 4) % 8 == 0;
     auto launch = [&](auto kernel, uint32_t per) {
         p.groups = (items + per - 1) / per;
-        p.xcd_map = p_xcd_ok && p.groups > 1 ? (local || no_contig || !stretch_local || nb < 128 || (nb >> 4) % 8 != 0 ? 1 : 2) : 0;
+        // (one group shares its keys with nobody, but its gathers still want a stretch's words in one L2: 4 items of 2^16 words, steps
+        // that are multiples of 8, the whole call 99.9 -> 76.3 us)
+        p.xcd_map = !p_xcd_ok ? 0 : stretches ? 2 : p.groups > 1 ? 1 : 0;
         const uint64_t wgs = (uint64_t)nb * rows * p.groups;
         if (wgs > most_workgroups(kThreads)) return hipErrorInvalidValue;
         hipLaunchKernelGGL(kernel, dim3((uint32_t)wgs), dim3(kThreads), 0, s, p);
         return hipGetLastError();
     };
+    // Items of a thread.  More of them read the keys less often but need more registers (5, 6 and 8 at 3, 2 and 2 waves per SIMD: 6 %,
+    // 5 to 20 % and 20 % slower than 4 at 4 waves), and a thread multiplies for all of its places, also those past the last item: 5 as 4
+    // and 1 cost what 8 do, as 3 and 2 what 6 do.  A group's own cost is about an item's.  Calls on [60, 40 | 60] bits, 15 steps, as 4 / as
+    // 3: 2^16 words, 5 items block-local 98.2 / 94.1 us, from memory 109.6 / 104.2, 9 items 138.7 / 133.1 and 156.8 / 148.1, but 7 items
+    // 111.0 / 116.1 and 8 items 126.9 / 136.9; 3 items as 2 and 1 / as 3, block-local 71.5 / 64.8.
+    // Below five workgroups for every two CUs two items, block-local below two a CU: more waves hide more than fewer key words save.  As 4 /
+    // 3 / 2: 9 items of 2^14 words from memory 67.4 / 65.4 / 62.9, 23 of 2^13 71.8 / 67.6 / 68.1; block-local 11 of 2^14 (576 workgroups)
+    // 61.2 / 59.2 / 63.8, 7 of 2^14 (384) 47.9 / 48.4 / 46.6.
+    auto cost = [&](uint32_t per) { return (items + per - 1) / per * (per + 1); };
+    uint32_t per = 4;
+    for (uint32_t i = 3; i >= 2; i--)
+        if (cost(i) < cost(per)) per = i;
+    const uint64_t heavy = (uint64_t)nb * (L + K) * ((items + per - 1) / per);
+    if (2 * heavy < (local ? 4 : 5) * (uint64_t)tune.cus) per = 2;
 #define HE_HOIST(I) return local ? launch(hoist_inner_kernel<I, true>, I) : launch(hoist_inner_kernel<I, false>, I)
-    // (more items per thread read the keys less often but need more registers: 5, 6 and 8 items at 3, 2 and 2 waves per
-    // SIMD measured 6 %, 5 to 20 % and 20 % slower than 4 items at 4 waves)
-    if (items >= 4) HE_HOIST(4);
+    if (per == 4) HE_HOIST(4);
+    if (per == 3) HE_HOIST(3);
     HE_HOIST(2);
 #undef HE_HOIST
 }
