@@ -1142,9 +1142,10 @@ namespace {
 // (addend: where the words to add come from, limb stride addend_stride between polynomials; nullptr: out itself)
 // inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
 // deal: see NttArgs; scratch: as many limbs that nothing else needs (inputs of the fused conversion in its own order)
+// small (single_limb_digits): [n_polys][N] bytes, coefficients that cx has still to gain (NttArgs::pro_small)
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
                  uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0,
-                 uint64_t *scratch = nullptr, size_t scratch_limbs = 0) {
+                 uint64_t *scratch = nullptr, size_t scratch_limbs = 0, const int8_t *small = nullptr) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     if (n_polys == 0) return HE_OK;
     const int accumulate = add_mask != 0;
@@ -1204,13 +1205,12 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     fwd.epi_dst = out;
     fwd.epi_dst_poly_stride = L;
     if (reduce_in_ntt) {
-        fwd.pro_mode = NTT_PRO_SOURCE_REDUCE;
+        fwd.pro_mode = small ? NTT_PRO_SOURCE_SMALL_REDUCE : NTT_PRO_SOURCE_REDUCE;
         fwd.pro_src = cx + (size_t)L * n;
         fwd.pro_poly_stride = LK;
-        if (source_intt) {
-            set_source_intt(ctx, fwd, inv_backend);
-            fwd.pro_src_table = ctx->size_q;
-        }
+        fwd.pro_src_table = ctx->size_q;
+        fwd.pro_small = small;
+        if (source_intt) set_source_intt(ctx, fwd, inv_backend);
     }
     HE_HIP(launch_ntt_forward(fwd, n_polys, backend_for(ctx, fwd.map), S(s), fused));
     return HE_OK;
@@ -1703,17 +1703,22 @@ bool encrypt_arguments_ok(const he_context *ctx, uint32_t L, uint32_t items, con
     return ctx && ws && ctx->size_p != 0 && L != 0 && L <= ctx->size_q && items != 0 && items <= 8192;
 }
 
-// Workspace of `items` encryptions: u and wide one after the other, 3 * items polynomials of the same limbs, then ModDown's scratch
+// Workspace of `items` encryptions: the places of u and wide one after the other, 3 * items polynomials of the same limbs, then ModDown's scratch
 struct EncryptWorkspace {
     uint64_t *u, *wide, *tmp;
+    int8_t *small;   // the samples, one byte each: u of every item, then e0 and e1 of every item
 };
 
 EncryptWorkspace encrypt_workspace(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *ws) {
     const size_t words = (size_t)items * (L + ctx->size_p) * ctx->n();
-    return EncryptWorkspace{ws, ws + words, ws + 3 * words};
+    // One special prime: the errors stay bytes until ModDown's transform reads them (launch_encrypt_products), in the place of u, whose
+    // 3 N bytes an item it has, and u lies in ModDown's scratch.  More of them: all three are transformed, the samples lie in ModDown's scratch.
+    uint64_t *tmp = ws + 3 * words;
+    const bool late = ctx->single_limb_digits;
+    return EncryptWorkspace{late ? tmp : ws, ws + words, tmp, reinterpret_cast<int8_t *>(late ? ws : tmp)};
 }
 
-// (u pk_0 + e_0, u pk_1 + e_1) of every item, into the workspace
+// (u pk_0 + e_0, u pk_1 + e_1) of every item, into the workspace; with one special prime the errors beside them
 int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8], uint64_t stream_id, uint64_t *ws,
                   he_stream s) {
     const uint32_t K = ctx->size_p, Q = ctx->size_q, LK = L + K;
@@ -1721,28 +1726,33 @@ int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint6
     ChaChaKey k;
     memcpy(k.k, key, sizeof(k.k));
     // item k draws u, e0, e1 from the stream ids stream_id + 3 k, + 1, + 2: what `items` encryptions in a row draw.  The
-    // samples stay bytes (in ModDown's scratch, which is written later) until the transform reads them.
-    int8_t *small = reinterpret_cast<int8_t *>(w.tmp);
-    HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, small, items, S(s)));
+    // samples stay bytes until a transform reads them.
+    HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, w.small, items, S(s)));
+    const bool late = ctx->single_limb_digits;
     const int backend = backend_for_level(ctx, L);
     NttArgs a = base_args(ctx, true);
     a.out = w.u;
     a.out_poly_stride = LK;
     a.map = LimbMap{LK, 0, L, Q};
     a.pro_mode = NTT_PRO_SMALL;
-    a.pro_src = w.tmp;
+    a.pro_src = reinterpret_cast<const uint64_t *>(w.small);
     a.pro_itw = ctx->d_ipsi;
     a.pro_itw_fp = ctx->d_ipsi_fp;
-    HE_HIP(launch_ntt_rows(a, 3 * items * LK, true, backend, S(s)));
-    HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
+    HE_HIP(launch_ntt_rows(a, (late ? 1 : 3) * items * LK, true, backend, S(s)));
+    if (late)
+        HE_HIP(launch_encrypt_products(a, pk, w.wide, L, K, Q, items, backend, S(s)));
+    else
+        HE_HIP(launch_encrypt_blocks(a, pk, L, K, Q, items, backend, S(s)));
     return HE_OK;
 }
 
 // ... divided by P onto the plaintexts.  plain: that of one item; nullptr: they lie in polynomial 0 of the ciphertexts
 int encrypt_onto(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, uint64_t *cts, uint64_t *ws, he_stream s) {
     const EncryptWorkspace w = encrypt_workspace(ctx, L, items, ws);
+    const bool late = ctx->single_limb_digits;
     return moddown_impl(ctx, L, w.wide, cts, 2 * items, 0x55555555u, w.tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
-                        plain ? L : 0, w.u, (size_t)items * (L + ctx->size_p));
+                        plain ? L : 0, late ? nullptr : w.u, late ? 0 : (size_t)items * (L + ctx->size_p),
+                        late ? w.small + (size_t)items * ctx->n() : nullptr);
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts

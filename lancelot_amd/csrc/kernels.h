@@ -88,6 +88,9 @@ enum : int {
     // imaginary part x of value (c mod N/2) / gap of the transformed slot vector (const double2 *)pro_src + p * 2^pro_log_slots,
     // which holds value i at bitrev(i); 0 where gap does not divide c.  Magnitudes below 2^62.
     NTT_PRO_ROUND = 11,
+    // NTT_PRO_SOURCE_REDUCE in map mode with small coefficients, one byte each, polynomial p at pro_small + p * N, added to the source
+    // modulo its prime (table pro_src_table) and taken from its residue.  NTT_PRO_SOURCE_INTT_REDUCE does the same where pro_small is set.
+    NTT_PRO_SOURCE_SMALL_REDUCE = 12,
 };
 
 // NttArgs::deal
@@ -138,7 +141,8 @@ struct NttArgs {
     const uint64_t *pro_src;  // [poly][pro_poly_stride limbs], the first limb of each poly is the source
     uint32_t pro_poly_stride;
     size_t pro_item_stride;   // NTT_PRO_SOURCE_REDUCE in list mode: words between the sources of consecutive items
-    uint32_t pro_src_table;   // NTT_PRO_SOURCE_INTT_REDUCE in map mode: table of the source limb
+    uint32_t pro_src_table;   // NTT_PRO_SOURCE_INTT_REDUCE and NTT_PRO_SOURCE_SMALL_REDUCE in map mode: table of the source limb
+    const int8_t *pro_small;  // ... and the small coefficients
     double pro_fix;           // NTT_PRO_ROUND: scale / slots
     uint32_t pro_log_slots;
     uint64_t pro_src_fp_mask; // NTT_PRO_SOURCE_INTT_REDUCE: tables whose inverse blocks pass left FP64 lazy words
@@ -458,6 +462,10 @@ hipError_t launch_ntt_inner(const NttArgs &a, const KsFuseArgs &x, int backend, 
 // others as canonical residues.
 hipError_t launch_encrypt_blocks(const NttArgs &a, const uint64_t *pk, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
                                  int backend, hipStream_t s);
+// The same for one special prime, without the errors, which the ModDown that follows brings in (NttArgs::pro_small): a.out holds the words of u [items][L+K][N]
+// alone, u pk_i goes to wide [items][2][L+K][N].
+hipError_t launch_encrypt_products(const NttArgs &a, const uint64_t *pk, uint64_t *wide, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
+                                   int backend, hipStream_t s);
 
 // Blocks pass of the flooding noise's transform fused with a decryption: a.out [items][limbs][N] holds the words that the
 // rows pass left; c0 + sum_i c_i s^i of the ciphertext is added to them (sizes 2 and 3).

@@ -229,6 +229,13 @@ __device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Jo
     return round(v[2 * slot + (at >= half ? 1 : 0)] * a.pro_fix);
 }
 
+// s + e modulo q for a residue s and a small e
+__device__ __forceinline__ uint64_t add_small(uint64_t s, int e, uint64_t q) {
+    int64_t t = (int64_t)s + e;
+    t += t < 0 ? (int64_t)q : 0;
+    return (uint64_t)(t >= (int64_t)q ? t - (int64_t)q : t);
+}
+
 // Input of a forward rows pass (a.pro_mode): word j of the thread from global offset glob(j) of its limb, as exact
 // doubles; returns whether they have to be reduced before the first stage (else they are canonical).
 // MDR: the launch's mode is NTT_PRO_MODDOWN_RESCALE (a template argument: its operands cost the other modes registers, 90 instead of
@@ -266,6 +273,14 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(barrett64(job.src[glob(j)], q, r1));
+    } else if (a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
+        const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1], p = scalar(a.moduli)[a.pro_src_table];
+        const int8_t *small = a.pro_small + ((size_t)job.poly << a.log_n);
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const int e = small[glob(j)];
+            v[j] = fp_from_u64(add_small(barrett64(add_small(job.src[glob(j)], e, p), q, r1), -e, q));
+        }
     } else if (a.pro_mode == NTT_PRO_SMALL) {
         const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll
@@ -305,6 +320,14 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
         const uint64_t *src = job.src;
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = barrett64(src[glob(j)], q, r1);
+    } else if (a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
+        const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1], p = scalar(a.moduli)[a.pro_src_table];
+        const int8_t *small = a.pro_small + ((size_t)job.poly << a.log_n);
+#pragma unroll
+        for (int j = 0; j < W; j++) {
+            const int e = small[glob(j)];
+            v[j] = add_small(barrett64(add_small(job.src[glob(j)], e, p), q, r1), -e, q);
+        }
     } else if (a.pro_mode == NTT_PRO_SMALL) {
         const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll

@@ -25,9 +25,9 @@ namespace {
 
 // What a rows pass's mode needs behind NttHead.
 struct RowsExtra {
-    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_INTT_REDUCE: pro_itw; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2 (or pro_itw), pro_w
+    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_[INTT_|SMALL_]REDUCE: pro_itw, pro_small; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2 (or pro_itw), pro_w
     uint64_t u0, u1, mask;          // list: item_stride, pro_item_stride; NTT_PRO_ROUND: pro_fix; NTT_PRO_MODDOWN_RESCALE: strides, pro_last and pro_k1
-    uint32_t w0;                    // inverse: epi_mode; NTT_PRO_SOURCE_INTT_REDUCE in map mode: pro_src_table
+    uint32_t w0;                    // inverse: epi_mode; NTT_PRO_SOURCE_[INTT_|SMALL_]REDUCE in map mode: pro_src_table
 };
 
 RowsExtra rows_extra(const NttArgs &a, bool fwd) {
@@ -35,8 +35,9 @@ RowsExtra rows_extra(const NttArgs &a, bool fwd) {
     if (!fwd) {
         e.p0 = a.w;
         e.w0 = (uint32_t)a.epi_mode;
-    } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
+    } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE || a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
         e.p0 = a.pro_itw;
+        e.p1 = reinterpret_cast<const uint64_t *>(a.pro_small);
         e.w0 = a.pro_src_table;
     } else if (a.pro_mode == NTT_PRO_MODDOWN_RESCALE && a.pro_itw) {
         e.p0 = a.pro_src;
@@ -64,6 +65,8 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
     a.item_stride = e.u0;
     a.pro_item_stride = e.u1;
     a.pro_fix = __longlong_as_double((long long)e.u0);
+    a.pro_small = reinterpret_cast<const int8_t *>(e.p1);
+    if constexpr (FWD && !MDR) a.pro_src_table = e.w0;
     if constexpr (SRC_INTT) {
         set_inverse_block(a, MDR ? e.p1 : e.p0);
         a.pro_src_fp_mask = e.mask;
@@ -123,7 +126,8 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
 // one behind it, which every output limb's workgroup transforms anew: a launch less, and CUs that were idle (see ntt_two_sources_ok).
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
 // TILES (inverse): the coefficients leave where a fused conversion looks for them (conversion_word), on the FP64 back end as doubles.
-template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B, bool TILES>
+// SMALL (SRC_INTT without MDR): pro_small is there.
+template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B, bool TILES, bool SMALL>
 __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, RowsExtra x) {
     NttArgs a;
     using T4 = Tile4<B, LD>;
@@ -150,8 +154,19 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             for (int j = 0; j < 4; j++) s2[j] = (src + ((size_t)1 << a.log_n))[glob(NB - 1, j)];
         }
     }
+    int small[4] = {0, 0, 0, 0};   // an encryption's errors (pro_small)
     auto sources = [&]() {
+        // (here and not with the words: the pointer comes late, and the forward twiddles are not to wait for it)
+        if constexpr (SMALL) {
+#pragma unroll
+            for (int j = 0; j < 4; j++) small[j] = (a.pro_small + ((size_t)job.poly << a.log_n))[glob(0, j)];
+        }
         source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t);
+        if constexpr (SMALL) {
+            const uint64_t p = scalar(a.moduli)[job.src_table];
+#pragma unroll
+            for (int j = 0; j < 4; j++) s[j] = add_small(s[j], small[j], p);
+        }
         if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t);
     };
     // the last words of an inverse pass: to their places in the limb, or where a conversion looks for them
@@ -175,7 +190,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             if constexpr (SRC_INTT && !MDR) {
                 const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(barrett64(s[j], q, r1));
+                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1));
             } else if (rows_input_fp<MDR, SRC_INTT>(v, a, job, c, [&](int j) { return glob(0, j); }, s, s2)) {
                 ar.reduce(v);
             }
@@ -208,7 +223,7 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             if constexpr (SRC_INTT && !MDR) {
                 const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = barrett64(s[j], q, r1);
+                for (int j = 0; j < 4; j++) v[j] = SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1);
             } else {
                 rows_input_int<MDR, SRC_INTT>(v, a, job, q, [&](int j) { return glob(0, j); }, s, s2);
             }
@@ -1043,7 +1058,7 @@ __device__ __forceinline__ uint64_t add_product(uint64_t v, uint64_t x, uint64_t
     return add_mod(reduce_8q(v, ar.m), mul_mod(x, y, ar.m.q, r0, r1), ar.m.q);
 }
 
-// Encryption: three waves take their block of u, e0 and e1 of one limb through the last 8 stages; the transformed u stays in
+// Encryption with several special primes: three waves take their block of u, e0 and e1 of one limb through the last 8 stages; the transformed u stays in
 // LDS, from where the other two add u pk_i to their e_i and store the sums, a special limb's through the inverse blocks pass
 // (ModDown follows).  (One wave for all three: 14.8 against 11.4 us for 4 limbs of 2^16 words.)
 template <class A>
@@ -1118,6 +1133,100 @@ __global__ __launch_bounds__(192) void encrypt_blocks_kernel(HE_HEAD_PARAMS, con
         encrypt_block(a, pk, L, LK, a.size_qp, t, table, blk, item, items, w, lane, fp_arith(a, table), u_lds);
     if constexpr (BE != NTT_BACKEND_FP) {
         if (!fp) encrypt_block(a, pk, L, LK, a.size_qp, t, table, blk, item, items, w, lane, int_arith(a, table), u_lds);
+    }
+}
+
+// x times v as the forward stages have left it, mod q, canonical
+__device__ __forceinline__ uint64_t lazy_product(double v, uint64_t x, const FpArith &ar, uint64_t, uint64_t) {
+    return fp_to_u64(fp_canonical(fp_mulmod(fp_canonical(v, ar.m), fp_from_u64(x), ar.m), ar.m));
+}
+__device__ __forceinline__ uint64_t lazy_product(uint64_t v, uint64_t x, const IntArith &ar, uint64_t r0, uint64_t r1) {
+    return mul_mod(reduce_8q(v, ar.m), x, ar.m.q, r0, r1);
+}
+
+// Encryption with one special prime P: the errors e_i never come here.  With d = (u pk_i + e_i) mod P,
+// (u pk_i + e_i - d) / P = (u pk_i - NTT(d - e_i)) / P modulo q, so ModDown's transform of d takes e_i along, and the
+// special limb gains it as the coefficients that it is: L + 1 transforms of u, 2 L of d - e_i, where those of e_0 and e_1 were
+// 2 (L + 1) more.  A wave transforms its block of u and multiplies by both pk_i; a special limb's two products go through the inverse
+// blocks pass on a wave each, with the block of u on both (one after the other they would be the launch's longest chain).
+// Encryption against three transforms each, us: [60, 40, 40 | 60], 2^16 words, 1, 4, 20 items 29.5 -> 26.7, 66.0 -> 52.5, 212 -> 168,
+// primes of 60 bits 33.7 -> 29.0, 71.5 -> 57.8, 249 -> 186, of 50 bits 26.1 -> 23.9, 51.8 -> 46.3, 175 -> 141; 2^12 and 2^13 words, 1 or 2
+// items the same within 1 %.
+template <bool SPECIAL, class A>
+__device__ __forceinline__ void encrypt_products(const NttArgs &a, const uint64_t *pk, uint64_t *wide, uint32_t LK, uint32_t t, uint32_t table,
+                                                 uint32_t r, uint32_t blk, uint32_t item, uint32_t lane, const A &ar) {
+    using T4 = Tile4<8, 8>;
+    constexpr bool FP = std::is_base_of<FpArith, A>::value;
+    const size_t n = (size_t)1 << a.log_n, off = (size_t)blk * 256, at = off + pair_lane(lane), key_poly = (size_t)a.size_qp * n;
+    const uint64_t *u = a.out + ((size_t)item * LK + t) * n;
+    const uint64_t *key = pk + (size_t)table * n + r * key_poly + at;
+    uint64_t *out = wide + ((size_t)(2 * item + r) * LK + t) * n;
+    const uint64_t r0 = scalar(a.barrett)[2 * table], r1 = scalar(a.barrett)[2 * table + 1];
+    uint64_t x[4], k[4], k1[4], o[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) x[j] = u[off + T4::word(0, lane, j)];
+    typename A::Tw tw[T4::kBlocks];
+    T4::template load_tw<A, 0>(tw, ar, (1u << (a.log_n - 8)) + blk, lane);
+    load_pairs(k, key);
+    if constexpr (!SPECIAL) load_pairs(k1, key + key_poly);
+    typename A::V v[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = A::from_word(x[j]);
+    T4::template forward<A>(v, tw, ar, nullptr, lane);
+    A iar = ar;
+    if constexpr (SPECIAL) {
+        if constexpr (FP)
+            iar.table = a.pro_itw_fp + ((size_t)table << a.log_n);
+        else
+            iar.table = a.pro_itw + ((size_t)table << (a.log_n + 1));
+        T4::template load_tw<A, 0>(tw, iar, (1u << (a.log_n - 8)) + blk, lane);
+    }
+    turn_pairs(v);
+#pragma unroll
+    for (int j = 0; j < 4; j++) o[j] = lazy_product(v[j], k[j], ar, r0, r1);
+    if constexpr (SPECIAL) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            if constexpr (FP)
+                v[j] = fp_from_u64(o[j]);
+            else
+                v[j] = o[j];
+        }
+        turn_pairs(v);
+        T4::template inverse<A>(v, tw, iar, nullptr, lane);
+#pragma unroll
+        for (int j = 0; j < 4; j++) out[off + T4::word(0, lane, j)] = A::to_word(v[j]);
+    } else {
+        store_pairs(out + at, o);
+#pragma unroll
+        for (int j = 0; j < 4; j++) o[j] = lazy_product(v[j], k1[j], ar, r0, r1);
+        store_pairs(out + LK * n + at, o);
+    }
+}
+
+// (units of an item: its L data limbs, then both polynomials of the special ones)
+template <int BE>
+__global__ __launch_bounds__(64 * kBlockWaves) void encrypt_products_kernel(HE_HEAD_PARAMS, const uint64_t *itw, uint64_t *wide) {
+    NttArgs a;
+    set_head(a, HE_HEAD_NAMES);
+    set_inverse_block(a, itw);
+    const uint64_t *pk = a.in;
+    const uint32_t lr = a.log_n - 8, lane = threadIdx.x & 63, LK = a.map.limbs, L = a.map.split, units = 2 * LK - L;
+    const uint32_t w = (uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1), it = id >> lr;
+    const uint32_t of_launch = it / units, unit = it - of_launch * units, item = h5 + of_launch;
+    const bool special = unit >= L;
+    const uint32_t t = special ? L + ((unit - L) >> 1) : unit, r = (unit - L) & 1, table = map_table(a.map, t);
+    const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
+    auto block = [&](const auto &ar) {
+        if (special)
+            encrypt_products<true>(a, pk, wide, LK, t, table, r, blk, item, lane, ar);
+        else
+            encrypt_products<false>(a, pk, wide, LK, t, table, 0, blk, item, lane, ar);
+    };
+    if (BE != NTT_BACKEND_INT && fp) block(fp_arith(a, table));
+    if constexpr (BE != NTT_BACKEND_FP) {
+        if (!fp) block(int_arith(a, table));
     }
 }
 
@@ -1272,7 +1381,7 @@ bool spread_epilogue(const NttArgs &a, int backend, uint32_t limbs, uint32_t pol
 // Words of a tile, log2: 1024 (4 columns at N = 2^16) for launches that would otherwise leave CUs without a workgroup, 2048
 // (twice the columns of a memory access) from 32 limbs of 2^16 words on (2 x 24 limbs 28.0 against 27.3 us); N < 2^12 takes
 // tiles of one wave, N = 2^17 needs 2048.
-template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false, bool TILES = false>
+template <bool FWD, int BE, bool SRC_INTT = false, bool MDR = false, bool TILES = false, bool SMALL = false>
 hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
     const uint32_t ld = a.log_n - 8;
     const bool large = ((uint64_t)n_jobs << a.log_n) >= ((uint64_t)32 << 16);
@@ -1280,14 +1389,14 @@ hipError_t launch_rows(NttArgs a, uint32_t n_jobs, hipStream_t s) {
     // (from 2^34 words on, 137 GB, one launch does not hold the threads)
     const uint32_t per_launch = most_workgroups(1u << (b - 2)) >> (a.log_n - b);
     while (n_jobs > per_launch) {
-        if (hipError_t e = launch_rows<FWD, BE, SRC_INTT, MDR, TILES>(a, per_launch, s)) return e;
+        if (hipError_t e = launch_rows<FWD, BE, SRC_INTT, MDR, TILES, SMALL>(a, per_launch, s)) return e;
         a.first_job += per_launch;
         n_jobs -= per_launch;
     }
     const dim3 grid(n_jobs << (a.log_n - b)), block(1u << (b - 2));
     const NttHead head = ntt_head(a, grid.x, a.first_job);
     const RowsExtra extra = rows_extra(a, FWD);
-#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B, TILES>), grid, block, 0, s, HE_HEAD_ARGS(head), extra)
+#define HE_ROWS(LD, B) hipLaunchKernelGGL((ntt_rows_kernel<LD, FWD, BE, SRC_INTT, MDR, B, TILES, SMALL>), grid, block, 0, s, HE_HEAD_ARGS(head), extra)
 #define HE_CASE(LD)         \
     case LD:                \
         if (large)          \
@@ -1349,6 +1458,7 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
         // one instantiation per degree, which follows fp_mask limb by limb: the mask stands for the launch's back end here
         if (!forward || !a.pro_itw || (a.pro_src_fp_mask && !a.pro_itw_fp)) return hipErrorInvalidValue;
         a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+        if (a.pro_small) return launch_rows<true, NTT_BACKEND_MIXED, true, false, false, true>(a, n_jobs, s);
         return launch_rows<true, NTT_BACKEND_MIXED, true>(a, n_jobs, s);
     }
     if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE && a.pro_itw) {
@@ -1631,6 +1741,31 @@ hipError_t launch_encrypt_blocks(const NttArgs &args, const uint64_t *pk, uint32
             hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);
         else
             hipLaunchKernelGGL(encrypt_blocks_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw);
+        if (hipError_t e = hipGetLastError()) return e;
+    }
+    return hipSuccess;
+}
+
+hipError_t launch_encrypt_products(const NttArgs &args, const uint64_t *pk, uint64_t *wide, uint32_t L, uint32_t K, uint32_t size_q, uint32_t items,
+                                   int backend, hipStream_t s) {
+    NttArgs a = args;
+    if (a.log_n < 9 || a.log_n > 17 || items == 0) return hipErrorInvalidValue;
+    a.in = pk;
+    a.map = LimbMap{L + K, 0, L, size_q};
+    const dim3 block(64 * kBlockWaves);
+    const uint32_t wgs_per_item = ((L + 2 * K) << (a.log_n - 8)) / kBlockWaves, per_launch = most_workgroups(block.x) / wgs_per_item;
+    if (per_launch == 0) return hipErrorInvalidValue;
+    for (uint32_t first = 0; first < items; first += per_launch) {
+        const uint32_t now = items - first < per_launch ? items - first : per_launch;
+        const dim3 grid(now * wgs_per_item);
+        a.spread = spread_encryption(a, backend, items, (uint64_t)now * (L + K) << (a.log_n - 8));
+        const NttHead head = ntt_head(a, grid.x, first);
+        if (backend == NTT_BACKEND_MIXED)
+            hipLaunchKernelGGL(encrypt_products_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw, wide);
+        else if (backend)
+            hipLaunchKernelGGL(encrypt_products_kernel<NTT_BACKEND_FP>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw, wide);
+        else
+            hipLaunchKernelGGL(encrypt_products_kernel<NTT_BACKEND_INT>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw, wide);
         if (hipError_t e = hipGetLastError()) return e;
     }
     return hipSuccess;
