@@ -94,8 +94,9 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
 // The inverse rows pass of a source limb's tile: lazy words of the last block's layout become canonical coefficients in the first
 // block's.  (Behind the request of the forward twiddles: the exchanges' compiler barriers would hold that back until the inverse
 // pass has ended.)
-template <class T4>
-__device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a, uint32_t st, uint64_t *lds, uint32_t t) {
+// behind: requests what is needed after the pass (loads return in order: in front of the twiddles, the pass would wait for them)
+template <class T4, class Behind>
+__device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a, uint32_t st, uint64_t *lds, uint32_t t, Behind &&behind) {
     constexpr int NB = T4::kBlocks;
     if ((a.pro_src_fp_mask >> st) & 1) {
         const FpArith ar{fp_ctx(a, st).m, a.pro_itw_fp + ((size_t)st << a.log_n)};
@@ -104,6 +105,7 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
         for (int j = 0; j < 4; j++) v[j] = FpArith::from_word(s[j]);
         FpArith::Tw tw[NB];
         T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
+        behind();
         T4::template inverse<FpArith>(v, tw, ar, lds, t);
         const ScalarF64 cc = scalar(a.fp_consts) + 4 * (size_t)st;
         const double ninv = cc[2];
@@ -113,6 +115,7 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
         const IntArith ar{int_mod(q), a.pro_itw + ((size_t)st << (a.log_n + 1))};
         IntArith::Tw tw[NB];
         T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
+        behind();
         T4::template inverse<IntArith>(s, tw, ar, lds, t);
 #pragma unroll
         for (int j = 0; j < 4; j++) s[j] = reduce_4q(s[j], ar.m);
@@ -156,18 +159,18 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
     }
     int small[4] = {0, 0, 0, 0};   // an encryption's errors (pro_small)
     auto sources = [&]() {
-        // (here and not with the words: the pointer comes late, and the forward twiddles are not to wait for it)
-        if constexpr (SMALL) {
+        source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t, [&]() {
+            if constexpr (SMALL) {
 #pragma unroll
-            for (int j = 0; j < 4; j++) small[j] = (a.pro_small + ((size_t)job.poly << a.log_n))[glob(0, j)];
-        }
-        source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t);
+                for (int j = 0; j < 4; j++) small[j] = (a.pro_small + ((size_t)job.poly << a.log_n))[glob(0, j)];
+            }
+        });
         if constexpr (SMALL) {
             const uint64_t p = scalar(a.moduli)[job.src_table];
 #pragma unroll
             for (int j = 0; j < 4; j++) s[j] = add_small(s[j], small[j], p);
         }
-        if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t);
+        if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t, []() {});
     };
     // the last words of an inverse pass: to their places in the limb, or where a conversion looks for them
     auto leave = [&](const uint64_t *w) {
