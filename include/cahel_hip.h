@@ -397,6 +397,12 @@ int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const ui
                      uint64_t stream_id, uint64_t *workspace, he_stream stream);
 int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *workspace, he_stream stream);
 
+/* he_ckks_encode_bounded of real values (DEVICE; the arguments and the bound on the coefficients as there) followed by he_encrypt_end: the
+ * same ciphertexts, without the plaintexts where they are not needed.  cts [items][2][L][N] is only written.  encode_workspace:
+ * he_ckks_encode_batch_workspace_words words.  No counterpart in the reference. */
+int he_encrypt_end_values(const he_context *ctx, uint32_t L, uint32_t items, const double *re, uint32_t count, uint32_t slots, double scale,
+                          size_t value_stride, uint64_t *cts, uint64_t *workspace, uint64_t *encode_workspace, he_stream stream);
+
 /* One encryption of plain [L][N] (NTT form) into ct [2][L][N]: he_encrypt_batch of one item without the copy of the plaintext.
  * workspace: he_encrypt_batch_workspace_words(ctx, L, 1) words. */
 int he_encrypt(const he_context *ctx, uint32_t L, const uint64_t *plain, const uint64_t *pk, const uint32_t key[8],

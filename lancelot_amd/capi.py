@@ -97,6 +97,7 @@ SIGNATURES = {
     "he_encrypt_batch_workspace_words": (C.c_size_t, [vp, u32, u32]),
     "he_encrypt_begin": (C.c_int, [vp, u32, u32, vp, C.POINTER(u32), u64, vp, vp]),
     "he_encrypt_end": (C.c_int, [vp, u32, u32, vp, vp, vp]),
+    "he_encrypt_end_values": (C.c_int, [vp, u32, u32, vp, u32, u32, C.c_double, C.c_size_t, vp, vp, vp, vp]),
     "he_encrypt_batch": (C.c_int, [vp, u32, u32, vp, C.POINTER(u32), u64, vp, vp, vp]),
     "he_sample_batch": (C.c_int, [vp, C.c_int, C.POINTER(u32), u64, vp, u32, u32, u32, u32, vp, u32, u32, vp]),
     "he_decrypt_decode_batch_workspace_words": (C.c_size_t, [vp, u32, u32, u32]),

@@ -1138,14 +1138,23 @@ int he_ks_inner_product(const he_context *ctx, uint32_t L, const uint64_t *y, co
 
 namespace {
 
+// Parts of an encryption that join it where ModDown's transform begins: its errors, [polys][N] bytes, and, unless they are ciphertexts by
+// themselves already (nullptr; not with source_intt_ok), the messages of the even polynomials (NttArgs::pro_values)
+struct LateParts {
+    const int8_t *small;
+    const double *values;
+    double fix;
+    uint32_t log_slots;
+};
+
 // add_mask: which polynomials of `out` are added onto (bit p set) instead of overwritten
 // (addend: where the words to add come from, limb stride addend_stride between polynomials; nullptr: out itself)
 // inverted: the special limbs have been through their inverse blocks pass on the level's back end (ks_accumulate)
 // deal: see NttArgs; scratch: as many limbs that nothing else needs (inputs of the fused conversion in its own order)
-// small (single_limb_digits): [n_polys][N] bytes, coefficients that cx has still to gain (NttArgs::pro_small)
+// late (single_limb_digits): what cx has still to gain
 int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out, uint32_t n_polys, uint32_t add_mask,
                  uint64_t *ws, he_stream s, uint32_t deal, bool inverted = false, const uint64_t *addend = nullptr, uint32_t addend_stride = 0,
-                 uint64_t *scratch = nullptr, size_t scratch_limbs = 0, const int8_t *small = nullptr) {
+                 uint64_t *scratch = nullptr, size_t scratch_limbs = 0, const LateParts *late = nullptr) {
     if (!ctx || !cx || !out || !ws || ctx->size_p == 0 || L == 0 || L > ctx->size_q) return HE_E_INVALID_ARGUMENT;
     if (n_polys == 0) return HE_OK;
     const int accumulate = add_mask != 0;
@@ -1205,11 +1214,16 @@ int moddown_impl(const he_context *ctx, uint32_t L, uint64_t *cx, uint64_t *out,
     fwd.epi_dst = out;
     fwd.epi_dst_poly_stride = L;
     if (reduce_in_ntt) {
-        fwd.pro_mode = small ? NTT_PRO_SOURCE_SMALL_REDUCE : NTT_PRO_SOURCE_REDUCE;
+        fwd.pro_mode = late ? NTT_PRO_SOURCE_SMALL_REDUCE : NTT_PRO_SOURCE_REDUCE;
         fwd.pro_src = cx + (size_t)L * n;
         fwd.pro_poly_stride = LK;
         fwd.pro_src_table = ctx->size_q;
-        fwd.pro_small = small;
+        if (late) {
+            fwd.pro_small = late->small;
+            fwd.pro_values = late->values;
+            fwd.pro_fix = late->fix;
+            fwd.pro_log_slots = late->log_slots;
+        }
         if (source_intt) set_source_intt(ctx, fwd, inv_backend);
     }
     HE_HIP(launch_ntt_forward(fwd, n_polys, backend_for(ctx, fwd.map), S(s), fused));
@@ -1624,6 +1638,21 @@ size_t he_ckks_workspace_words(const he_context *ctx, uint32_t limbs) {
     return enc > dec ? enc : dec;
 }
 
+}  // extern "C"
+
+namespace {
+
+bool encode_arguments_ok(const he_context *ctx, uint32_t count, uint32_t slots, double scale, uint32_t items, size_t value_stride) {
+    return slots >= 2 && !(slots & (slots - 1)) && slots <= ctx->n() / 2 && count <= slots && scale > 0 && (items <= 1 || value_stride >= count);
+}
+
+// the slot vectors of an encoding's workspace, behind the maxima (he_ckks_encode_batch_workspace_words)
+double2 *encode_vectors(uint64_t *ws, uint32_t items) { return reinterpret_cast<double2 *>(ws + (((size_t)items + 7) & ~(size_t)7)); }
+
+}  // namespace
+
+extern "C" {
+
 size_t he_ckks_encode_batch_workspace_words(const he_context *ctx, uint32_t items) {
     if (!ctx) return 0;
     // [items words rounded up to 8: the maxima] [items][N words: complex scratch]
@@ -1636,12 +1665,9 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     if (!ctx || !re || !out || !ws || limbs == 0 || limbs > ctx->size_qp || items == 0 || items > 16384 ||
         out_poly_stride < limbs)
         return HE_E_INVALID_ARGUMENT;
-    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || count > slots || !(scale > 0) ||
-        (items > 1 && value_stride < count))
-        return HE_E_INVALID_ARGUMENT;
+    if (!encode_arguments_ok(ctx, count, slots, scale, items, value_stride)) return HE_E_INVALID_ARGUMENT;
     const size_t n = ctx->n();
-    const size_t head = ((size_t)items + 7) & ~(size_t)7;
-    double2 *v = reinterpret_cast<double2 *>(ws + head);
+    double2 *v = encode_vectors(ws, items);
     const FftTables ft = ctx->fft();
     // (the complex scratch of an item is `slots` values = at most N words: the items are packed `slots` apart)
     // (the rounding kernel writes the residues itself: the coefficients never exist as an array of doubles)
@@ -1663,10 +1689,8 @@ int he_ckks_encode_bounded(const he_context *ctx, const double *re, const double
     if (!ctx || !re || !out || !ws || limbs == 0 || limbs > ctx->size_qp || items == 0 || items > 16384 ||
         out_poly_stride < limbs)
         return HE_E_INVALID_ARGUMENT;
-    if (slots < 2 || (slots & (slots - 1)) || slots > ctx->n() / 2 || count > slots || !(scale > 0) ||
-        (items > 1 && value_stride < count))
-        return HE_E_INVALID_ARGUMENT;
-    double2 *v = reinterpret_cast<double2 *>(ws + (((size_t)items + 7) & ~(size_t)7));
+    if (!encode_arguments_ok(ctx, count, slots, scale, items, value_stride)) return HE_E_INVALID_ARGUMENT;
+    double2 *v = encode_vectors(ws, items);
     const FftTables ft = ctx->fft();
     HE_HIP(launch_ckks_fft_inverse(ft, re, im, count, slots, v, items, value_stride, S(s)));
     // rounding and residues happen where the transform reads its input
@@ -1746,13 +1770,16 @@ int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint6
     return HE_OK;
 }
 
-// ... divided by P onto the plaintexts.  plain: that of one item; nullptr: they lie in polynomial 0 of the ciphertexts
-int encrypt_onto(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, uint64_t *cts, uint64_t *ws, he_stream s) {
+// ... divided by P onto the plaintexts.  plain: that of one item; nullptr: they lie in polynomial 0 of the ciphertexts.  values: the
+// messages instead of plaintexts, one special prime only (NttArgs::pro_values)
+int encrypt_onto(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *plain, uint64_t *cts, uint64_t *ws, he_stream s,
+                 const double *values = nullptr, double fix = 0, uint32_t log_slots = 0) {
     const EncryptWorkspace w = encrypt_workspace(ctx, L, items, ws);
     const bool late = ctx->single_limb_digits;
-    return moddown_impl(ctx, L, w.wide, cts, 2 * items, 0x55555555u, w.tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
+    const LateParts parts{w.small + (size_t)items * ctx->n(), values, fix, log_slots};
+    return moddown_impl(ctx, L, w.wide, cts, 2 * items, values ? 0u : 0x55555555u, w.tmp, s, items == 1 ? NTT_DEAL_ALWAYS : NTT_DEAL_LONG, true, plain,
                         plain ? L : 0, late ? nullptr : w.u, late ? 0 : (size_t)items * (L + ctx->size_p),
-                        late ? w.small + (size_t)items * ctx->n() : nullptr);
+                        late ? &parts : nullptr);
 }
 
 // the inverse blocks pass over `items` dense plaintexts, then the composition of their coefficients, the transform and the real parts
@@ -1832,6 +1859,24 @@ int he_encrypt_begin(const he_context *ctx, uint32_t L, uint32_t items, const ui
 int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *ws, he_stream s) {
     if (!encrypt_arguments_ok(ctx, L, items, ws) || !cts) return HE_E_INVALID_ARGUMENT;
     return encrypt_onto(ctx, L, items, nullptr, cts, ws, s);
+}
+
+int he_encrypt_end_values(const he_context *ctx, uint32_t L, uint32_t items, const double *re, uint32_t count, uint32_t slots, double scale,
+                          size_t value_stride, uint64_t *cts, uint64_t *ws, uint64_t *encode_ws, he_stream s) {
+    if (!encrypt_arguments_ok(ctx, L, items, ws) || !cts || !re || !encode_ws) return HE_E_INVALID_ARGUMENT;
+    // With one special prime P, (c - NTT(d)) / P + NTT(m) = (c - NTT(d - P m)) / P: the message joins ModDown's coefficients, and neither
+    // its transform nor the words of a plaintext are needed.  Not where a small launch transforms the special limb anew for every limb
+    // (there the message would be one more thing that every limb repeats).  20 messages on three limbs of 2^16 words: two launches of 20
+    // and 15 us and a seventh of the last pass's words less, a Krum round 1190 -> 1171 us.
+    if (!ctx->single_limb_digits || source_intt_ok(ctx, 2 * items * L)) {
+        if (int rc = he_ckks_encode_bounded(ctx, re, nullptr, count, slots, scale, L, items, value_stride, cts, 2 * L, encode_ws, s)) return rc;
+        return he_encrypt_end(ctx, L, items, cts, ws, s);
+    }
+    if (!encode_arguments_ok(ctx, count, slots, scale, items, value_stride)) return HE_E_INVALID_ARGUMENT;
+    double2 *v = encode_vectors(encode_ws, items);
+    HE_HIP(launch_ckks_fft_inverse(ctx->fft(), re, nullptr, count, slots, v, items, value_stride, S(s)));
+    return encrypt_onto(ctx, L, items, nullptr, cts, ws, s, reinterpret_cast<const double *>(v), scale / (double)slots,
+                        31 - __builtin_clz(slots));
 }
 
 int he_encrypt_batch(const he_context *ctx, uint32_t L, uint32_t items, const uint64_t *pk, const uint32_t key[8],

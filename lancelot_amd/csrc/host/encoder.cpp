@@ -168,13 +168,13 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::end_batch(const CAHELGPUCon
     const double scale = batch.scale;
     he_context *h = context.handle();
     he_stream st = context.stream();
-    // plaintexts straight into polynomial 0 of the ciphertexts
+    // plaintexts, where there are any, straight into polynomial 0 of the ciphertexts
     const std::size_t words = 2 * (std::size_t)L * n;
     DeviceBuffer ws(he_ckks_encode_batch_workspace_words(h, (uint32_t)items));
     if (small) {
-        check_status(he_ckks_encode_bounded(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
-                                            batch.cts.get(), 2 * L, ws.get(), st),
-                     "he_ckks_encode_bounded");
+        check_status(he_encrypt_end_values(h, L, (uint32_t)items, d_values, (uint32_t)count, (uint32_t)ss, scale, count, batch.cts.get(),
+                                           batch.ws.get(), ws.get(), st),
+                     "he_encrypt_end_values");
     } else {
         check_status(he_ckks_encode_batch(h, d_values, nullptr, (uint32_t)count, (uint32_t)ss, scale, L, (uint32_t)items, count,
                                           batch.cts.get(), 2 * L, ws.get(), st),
@@ -186,8 +186,8 @@ std::vector<CAHELGPUCiphertext> CAHELGPUCKKSEncoder::end_batch(const CAHELGPUCon
             if (max_coeff_bit_count >= batch.total_bits || max_coeff_bit_count > 63)
                 throw std::invalid_argument("encoded values are too large");
         }
+        check_status(he_encrypt_end(h, L, (uint32_t)items, batch.cts.get(), batch.ws.get(), st), "he_encrypt_end");
     }
-    check_status(he_encrypt_end(h, L, (uint32_t)items, batch.cts.get(), batch.ws.get(), st), "he_encrypt_end");
     // one ciphertext object per message, each a slice of the batch (no copies)
     std::vector<CAHELGPUCiphertext> out(items);
     auto shared = std::make_shared<DeviceBuffer>(std::move(batch.cts));

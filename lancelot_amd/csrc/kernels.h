@@ -90,6 +90,7 @@ enum : int {
     NTT_PRO_ROUND = 11,
     // NTT_PRO_SOURCE_REDUCE in map mode with small coefficients, one byte each, polynomial p at pro_small + p * N, added to the source
     // modulo its prime (table pro_src_table) and taken from its residue.  NTT_PRO_SOURCE_INTT_REDUCE does the same where pro_small is set.
+    // pro_values set: P times coefficient c of encoding p / 2 (NTT_PRO_ROUND's, its vectors there) is taken from an even polynomial too.
     NTT_PRO_SOURCE_SMALL_REDUCE = 12,
 };
 
@@ -143,6 +144,7 @@ struct NttArgs {
     size_t pro_item_stride;   // NTT_PRO_SOURCE_REDUCE in list mode: words between the sources of consecutive items
     uint32_t pro_src_table;   // NTT_PRO_SOURCE_INTT_REDUCE and NTT_PRO_SOURCE_SMALL_REDUCE in map mode: table of the source limb
     const int8_t *pro_small;  // ... and the small coefficients
+    const double *pro_values;
     double pro_fix;           // NTT_PRO_ROUND: scale / slots
     uint32_t pro_log_slots;
     uint64_t pro_src_fp_mask; // NTT_PRO_SOURCE_INTT_REDUCE: tables whose inverse blocks pass left FP64 lazy words

@@ -219,14 +219,22 @@ __device__ __forceinline__ double inverse_scale(const NttArgs &a, const Job &job
     return fp_reduce(fp_mulmod(fp_from_u64(scalar(a.w)[2 * job.limb]), ninv, m), m);
 }
 
-// coefficient at `at` of polynomial job.poly of an encoding, rounded (NTT_PRO_ROUND)
-__device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Job &job, uint32_t at) {
-    const uint32_t log_slots = a.in_poly_stride, half = 1u << (a.log_n - 1), log_gap = a.log_n - 1 - log_slots;
+// coefficient at `at` of encoding `poly`, whose slot vector lies in `values`, rounded (NTT_PRO_ROUND)
+__device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const double *values, uint32_t poly, uint32_t log_slots, uint32_t at) {
+    const uint32_t half = 1u << (a.log_n - 1), log_gap = a.log_n - 1 - log_slots;
     const uint32_t k = at & (half - 1);
     if (k & ((1u << log_gap) - 1)) return 0.0;
-    const double *v = reinterpret_cast<const double *>(a.in) + ((size_t)job.poly << (log_slots + 1));
+    const double *v = values + ((size_t)poly << (log_slots + 1));
     const uint32_t slot = __brev(k >> log_gap) >> (32 - log_slots);
     return round(v[2 * slot + (at >= half ? 1 : 0)] * a.pro_fix);
+}
+__device__ __forceinline__ double rounded_coefficient(const NttArgs &a, const Job &job, uint32_t at) {
+    return rounded_coefficient(a, reinterpret_cast<const double *>(a.in), job.poly, a.in_poly_stride, at);
+}
+// ... as a residue
+__device__ __forceinline__ uint64_t rounded_residue(double x, uint64_t q, uint64_t r1) {
+    const uint64_t r = barrett64((uint64_t)fabs(x), q, r1);
+    return x < 0 ? neg_mod(r, q) : r;
 }
 
 // s + e modulo q for a residue s and a small e
@@ -273,14 +281,6 @@ __device__ __forceinline__ bool rows_input_fp(double (&v)[W], const NttArgs &a, 
         const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = fp_from_u64(barrett64(job.src[glob(j)], q, r1));
-    } else if (a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
-        const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1], p = scalar(a.moduli)[a.pro_src_table];
-        const int8_t *small = a.pro_small + ((size_t)job.poly << a.log_n);
-#pragma unroll
-        for (int j = 0; j < W; j++) {
-            const int e = small[glob(j)];
-            v[j] = fp_from_u64(add_small(barrett64(add_small(job.src[glob(j)], e, p), q, r1), -e, q));
-        }
     } else if (a.pro_mode == NTT_PRO_SMALL) {
         const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll
@@ -320,14 +320,6 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
         const uint64_t *src = job.src;
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = barrett64(src[glob(j)], q, r1);
-    } else if (a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
-        const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1], p = scalar(a.moduli)[a.pro_src_table];
-        const int8_t *small = a.pro_small + ((size_t)job.poly << a.log_n);
-#pragma unroll
-        for (int j = 0; j < W; j++) {
-            const int e = small[glob(j)];
-            v[j] = add_small(barrett64(add_small(job.src[glob(j)], e, p), q, r1), -e, q);
-        }
     } else if (a.pro_mode == NTT_PRO_SMALL) {
         const int8_t *src = reinterpret_cast<const int8_t *>(a.in) + ((size_t)job.poly << a.log_n);
 #pragma unroll
@@ -338,15 +330,30 @@ __device__ __forceinline__ void rows_input_int(uint64_t (&v)[W], const NttArgs &
     } else if (a.pro_mode == NTT_PRO_ROUND) {
         const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
-        for (int j = 0; j < W; j++) {
-            const double x = rounded_coefficient(a, job, (uint32_t)glob(j));
-            const uint64_t r = barrett64((uint64_t)fabs(x), q, r1);
-            v[j] = x < 0 ? neg_mod(r, q) : r;
-        }
+        for (int j = 0; j < W; j++) v[j] = rounded_residue(rounded_coefficient(a, job, (uint32_t)glob(j)), q, r1);
     } else {
 #pragma unroll
         for (int j = 0; j < W; j++) v[j] = job.in[glob(j)];
     }
+}
+
+// Input of a forward rows pass in the mode NTT_PRO_SOURCE_SMALL_REDUCE.  x: the rounded coefficients (pro_values)
+template <typename Glob>
+__device__ __forceinline__ void small_source(uint64_t (&v)[4], double (&x)[4], const NttArgs &a, const Job &job, bool values, Glob glob) {
+    const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1], p = scalar(a.moduli)[a.pro_src_table];
+    const int8_t *small = a.pro_small + ((size_t)job.poly << a.log_n);
+    int e[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        v[j] = job.src[glob(j)];
+        e[j] = small[glob(j)];
+    }
+    if (values) {
+#pragma unroll
+        for (int j = 0; j < 4; j++) x[j] = rounded_coefficient(a, a.pro_values, job.poly >> 1, a.pro_log_slots, (uint32_t)glob(j));
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) v[j] = add_small(barrett64(add_small(v[j], e[j], p), q, r1), -e[j], q);
 }
 
 // a of the lanes whose bit BIT is set and b of the lanes where it is not change places: the words' register bit becomes that

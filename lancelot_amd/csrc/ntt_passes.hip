@@ -25,8 +25,8 @@ namespace {
 
 // What a rows pass's mode needs behind NttHead.
 struct RowsExtra {
-    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_[INTT_|SMALL_]REDUCE: pro_itw, pro_small; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2 (or pro_itw), pro_w
-    uint64_t u0, u1, mask;          // list: item_stride, pro_item_stride; NTT_PRO_ROUND: pro_fix; NTT_PRO_MODDOWN_RESCALE: strides, pro_last and pro_k1
+    const uint64_t *p0, *p1, *p2;   // inverse: w; NTT_PRO_SOURCE_[INTT_|SMALL_]REDUCE: pro_itw or pro_values, pro_small; NTT_PRO_MODDOWN_RESCALE: pro_src, pro_src2 (or pro_itw), pro_w
+    uint64_t u0, u1, mask;          // list: item_stride, pro_item_stride; NTT_PRO_ROUND, NTT_PRO_SOURCE_SMALL_REDUCE: pro_fix (, pro_log_slots); NTT_PRO_MODDOWN_RESCALE: strides, pro_last and pro_k1
     uint32_t w0;                    // inverse: epi_mode; NTT_PRO_SOURCE_[INTT_|SMALL_]REDUCE in map mode: pro_src_table
 };
 
@@ -35,7 +35,13 @@ RowsExtra rows_extra(const NttArgs &a, bool fwd) {
     if (!fwd) {
         e.p0 = a.w;
         e.w0 = (uint32_t)a.epi_mode;
-    } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE || a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
+    } else if (a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE) {
+        e.p0 = reinterpret_cast<const uint64_t *>(a.pro_values);
+        e.p1 = reinterpret_cast<const uint64_t *>(a.pro_small);
+        memcpy(&e.u0, &a.pro_fix, sizeof(e.u0));
+        e.u1 = a.pro_log_slots;
+        e.w0 = a.pro_src_table;
+    } else if (a.pro_mode == NTT_PRO_SOURCE_INTT_REDUCE) {
         e.p0 = a.pro_itw;
         e.p1 = reinterpret_cast<const uint64_t *>(a.pro_small);
         e.w0 = a.pro_src_table;
@@ -66,6 +72,8 @@ __device__ __forceinline__ void set_extra(NttArgs &a, const RowsExtra &e) {
     a.pro_item_stride = e.u1;
     a.pro_fix = __longlong_as_double((long long)e.u0);
     a.pro_small = reinterpret_cast<const int8_t *>(e.p1);
+    a.pro_values = reinterpret_cast<const double *>(e.p0);
+    a.pro_log_slots = (uint32_t)e.u1;
     if constexpr (FWD && !MDR) a.pro_src_table = e.w0;
     if constexpr (SRC_INTT) {
         set_inverse_block(a, MDR ? e.p1 : e.p0);
@@ -129,7 +137,7 @@ __device__ __forceinline__ void source_words(uint64_t (&s)[4], const NttArgs &a,
 // one behind it, which every output limb's workgroup transforms anew: a launch less, and CUs that were idle (see ntt_two_sources_ok).
 // B = log2(words of a tile): 2^LD rows x 2^(B - LD) columns
 // TILES (inverse): the coefficients leave where a fused conversion looks for them (conversion_word), on the FP64 back end as doubles.
-// SMALL (SRC_INTT without MDR): pro_small is there.
+// SMALL: NTT_PRO_SOURCE_SMALL_REDUCE, or SRC_INTT with pro_small.
 template <int LD, bool FWD, int BE, bool SRC_INTT, bool MDR, int B, bool TILES, bool SMALL>
 __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, RowsExtra x) {
     NttArgs a;
@@ -194,6 +202,18 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = fp_from_u64(SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1));
+            } else if constexpr (SMALL) {
+                const bool values = a.pro_values && !(job.poly & 1);
+                double r[4];
+                small_source(s, r, a, job, values, [&](int j) { return glob(0, j); });
+#pragma unroll
+                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(s[j]);
+                if (values) {
+                    const double p = fp_from_u64(scalar_shoup(a.barrett + p_constants_from_barrett(a.size_qp), job.limb).w);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] -= fp_mulmod(fp_reduce(r[j], c.m), p, c.m);
+                    ar.reduce(v);
+                }
             } else if (rows_input_fp<MDR, SRC_INTT>(v, a, job, c, [&](int j) { return glob(0, j); }, s, s2)) {
                 ar.reduce(v);
             }
@@ -227,6 +247,16 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
                 const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
                 for (int j = 0; j < 4; j++) v[j] = SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1);
+            } else if constexpr (SMALL) {
+                const bool values = a.pro_values && !(job.poly & 1);
+                const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
+                double r[4];
+                small_source(v, r, a, job, values, [&](int j) { return glob(0, j); });
+                if (values) {
+                    const Shoup p = scalar_shoup(a.barrett + p_constants_from_barrett(a.size_qp), job.limb);
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[j] = sub_mod(v[j], mul_shoup(rounded_residue(r[j], q, r1), p, q), q);
+                }
             } else {
                 rows_input_int<MDR, SRC_INTT>(v, a, job, q, [&](int j) { return glob(0, j); }, s, s2);
             }
@@ -1464,6 +1494,10 @@ hipError_t launch_ntt_rows(const NttArgs &args, uint32_t n_jobs, bool forward, i
         if (a.pro_small) return launch_rows<true, NTT_BACKEND_MIXED, true, false, false, true>(a, n_jobs, s);
         return launch_rows<true, NTT_BACKEND_MIXED, true>(a, n_jobs, s);
     }
+    if (forward && a.pro_mode == NTT_PRO_SOURCE_SMALL_REDUCE)
+        return backend == NTT_BACKEND_MIXED ? launch_rows<true, NTT_BACKEND_MIXED, false, false, false, true>(a, n_jobs, s)
+               : backend                    ? launch_rows<true, NTT_BACKEND_FP, false, false, false, true>(a, n_jobs, s)
+                                            : launch_rows<true, NTT_BACKEND_INT, false, false, false, true>(a, n_jobs, s);
     if (forward && a.pro_mode == NTT_PRO_MODDOWN_RESCALE && a.pro_itw) {
         if (!a.pro_k1 || a.pro_poly_stride != a.pro2_poly_stride || a.pro_src2 != a.pro_src + ((size_t)1 << a.log_n)) return hipErrorInvalidValue;
         a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);

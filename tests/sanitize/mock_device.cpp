@@ -175,6 +175,13 @@ int he_ckks_encode_batch(const he_context *ctx, const double *re, const double *
     return HE_OK;
 }
 
+int he_encrypt_end(const he_context *ctx, uint32_t L, uint32_t items, uint64_t *cts, uint64_t *ws, he_stream stream);
+int he_encrypt_end_values(const he_context *ctx, uint32_t L, uint32_t items, const double *re, uint32_t count, uint32_t slots, double scale,
+                          size_t value_stride, uint64_t *cts, uint64_t *ws, uint64_t *encode_ws, he_stream stream) {
+    if (int rc = he_ckks_encode_bounded(ctx, re, nullptr, count, slots, scale, L, items, value_stride, cts, 2 * L, encode_ws, stream)) return rc;
+    return he_encrypt_end(ctx, L, items, cts, ws, stream);
+}
+
 int he_widen_rows(const float *in, double *out, uint32_t rows, size_t length, size_t padded, he_stream stream) {
     queues[stream].push_back([=] {
         for (uint32_t r = 0; r < rows; r++)
