@@ -1751,7 +1751,6 @@ int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint6
     memcpy(k.k, key, sizeof(k.k));
     // item k draws u, e0, e1 from the stream ids stream_id + 3 k, + 1, + 2: what `items` encryptions in a row draw.  The
     // samples stay bytes until a transform reads them.
-    HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, w.small, items, S(s)));
     const bool late = ctx->single_limb_digits;
     const int backend = backend_for_level(ctx, L);
     NttArgs a = base_args(ctx, true);
@@ -1762,7 +1761,12 @@ int encrypt_zeros(const he_context *ctx, uint32_t L, uint32_t items, const uint6
     a.pro_src = reinterpret_cast<const uint64_t *>(w.small);
     a.pro_itw = ctx->d_ipsi;
     a.pro_itw_fp = ctx->d_ipsi_fp;
-    HE_HIP(launch_ntt_rows(a, (late ? 1 : 3) * items * LK, true, backend, S(s)));
+    if (late && encrypt_rows_ok(ctx->log_n, LK, items, ctx->tune.cus)) {
+        HE_HIP(launch_encrypt_rows(a, k, stream_id, w.small, items, backend, S(s)));
+    } else {
+        HE_HIP(launch_sample_encrypt(ctx->log_n, k, stream_id, w.small, items, S(s)));
+        HE_HIP(launch_ntt_rows(a, (late ? 1 : 3) * items * LK, true, backend, S(s)));
+    }
     if (late)
         HE_HIP(launch_encrypt_products(a, pk, w.wide, L, K, Q, items, backend, S(s)));
     else

@@ -33,6 +33,13 @@ __device__ void chacha20_block(const ChaChaKey &key, uint64_t counter, uint64_t 
     for (int i = 0; i < 16; i++) out[i] = x[i] + s[i];
 }
 
+// A ternary coefficient of one word, and an error (centred binomial, 21 bits a side) of two
+__device__ __forceinline__ int ternary_value(uint32_t w) { return (int)(((uint64_t)w * 3) >> 32) - 1; }
+__device__ __forceinline__ int error_value(uint32_t w0, uint32_t w1) { return __popc(w0 & 0x1FFFFFu) - __popc(w1 & 0x1FFFFFu); }
+__device__ __forceinline__ uint32_t four_bytes(int a, int b, int c, int d) {
+    return (uint32_t)(a & 255) | ((uint32_t)(b & 255) << 8) | ((uint32_t)(c & 255) << 16) | ((uint32_t)(d & 255) << 24);
+}
+
 // The cumulative table of the discrete Gaussian, padded to 128 entries that nothing reaches, so that all searches take the same seven
 // steps and those of a thread go together, their LDS reads behind one another instead of each search after the one before
 // (one polynomial of 2^16 coefficients 7.9 -> 5.1 us).

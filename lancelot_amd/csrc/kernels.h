@@ -501,6 +501,9 @@ hipError_t launch_sample_gauss_small(uint32_t log_n, ChaChaKey key, uint64_t str
 // ... or that polynomial's residues, with the rows pass of their forward transform done: limb l of item k at a.out (a: map mode,
 // dense).  flood_rows_ok: whether that is the faster way.
 bool flood_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items, uint32_t cus);
+// The same for u of public-key encryptions, whose errors go to small + items * N as launch_sample_encrypt writes them (u's bytes are nowhere).
+bool encrypt_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items, uint32_t cus);
+hipError_t launch_encrypt_rows(const NttArgs &a, ChaChaKey key, uint64_t stream_id, int8_t *small, uint32_t items, int backend, hipStream_t s);
 hipError_t launch_flood_rows(const NttArgs &a, ChaChaKey key, uint64_t stream_id, const uint64_t *cdt, uint32_t cdt_len, uint32_t items,
                              int backend, hipStream_t s);
 

@@ -1319,26 +1319,42 @@ struct FloodExtra {
     uint64_t stream;
     const uint64_t *cdt;
     uint32_t cdt_len;
+    int8_t *errors;
 };
 
 // The rows pass of a small Gaussian polynomial that is sampled on the spot: a thread makes four neighbouring coefficients of its tile
 // (half of its ChaCha block), a byte each in LDS.  Every limb's workgroups sample anew, on CUs that a launch of a few limbs leaves
 // idle, which costs less than a sampler's launch and the bytes' way through memory: decryption of two limbs of
 // 2^16 coefficients 10.7 -> 8.9 us.
-template <int LD>
+// ENCRYPT: u instead (a quarter of a ChaCha block a thread); the workgroups behind the tiles make a block's errors a
+// thread.  he_encrypt_batch on three limbs and a special one of 2^15, 2^14, 2^12 words 23.2 -> 22.4, 19.1 -> 18.2, 18.0 -> 17.1 us.
+template <int LD, bool ENCRYPT>
 __global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodExtra f) {
     using T4 = Tile4<10, LD>;
     constexpr int LOGC = 10 - LD, NB = T4::kBlocks;
     constexpr uint32_t C = 1u << LOGC, tiles_per_limb = 256u >> LOGC;
-    __shared__ uint64_t lds[(1 << 10) + (1 << 6)], cdt[kSmallCdt];
+    __shared__ uint64_t lds[(1 << 10) + (1 << 6)], cdt[ENCRYPT ? 1 : kSmallCdt];
     __shared__ uint32_t noise[256];
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
+    if constexpr (ENCRYPT) {
+        if (blockIdx.x >= h4) {
+            const uint32_t i = blockIdx.x - h4, poly = i >> (LD - 3), b = (i & ((1u << (LD - 3)) - 1)) * 256 + threadIdx.x;
+            uint32_t w[16];
+            chacha20_block(f.key, b, f.stream + 3 * (uint64_t)(poly >> 1) + 1 + (poly & 1), w);
+            uint32_t *dst = reinterpret_cast<uint32_t *>(f.errors + ((size_t)poly << a.log_n) + 8 * (size_t)b);
+#pragma unroll
+            for (int e = 0; e < 2; e++)
+                dst[e] = four_bytes(error_value(w[8 * e], w[8 * e + 1]), error_value(w[8 * e + 2], w[8 * e + 3]),
+                                    error_value(w[8 * e + 4], w[8 * e + 5]), error_value(w[8 * e + 6], w[8 * e + 7]));
+            return;
+        }
+    }
     const uint32_t lb = logical_block(h4);
     const Job job = decode_job(a, lb / tiles_per_limb);
     const uint32_t col0 = (lb % tiles_per_limb) << LOGC;
     const uint32_t t = ((uint32_t)__builtin_amdgcn_readfirstlane(threadIdx.x >> 6) << 6) | (threadIdx.x & 63);
-    if (t < kSmallCdt) cdt[t] = padded_cdt(f.cdt, f.cdt_len, t);
+    if (!ENCRYPT && t < kSmallCdt) cdt[t] = padded_cdt(f.cdt, f.cdt_len, t);
     auto glob = [&](int k, int j) {
         const uint32_t e = T4::word(k, t, j);
         return (size_t)(e >> LOGC) * 256 + col0 + (e & (C - 1));
@@ -1346,6 +1362,16 @@ __global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodEx
     auto sample = [&]() {
         const uint32_t at = ((4 * t) >> LOGC) * 256 + col0 + ((4 * t) & (C - 1));
         uint32_t w[16];
+        if constexpr (ENCRYPT) {
+            chacha20_block(f.key, at >> 4, f.stream + 3 * (uint64_t)job.poly, w);
+#pragma unroll
+            for (int e = 0; e < 8; e++) w[e] = at & 8 ? w[8 + e] : w[e];
+#pragma unroll
+            for (int e = 0; e < 4; e++) w[e] = at & 4 ? w[4 + e] : w[e];
+            noise[t] = four_bytes(ternary_value(w[0]), ternary_value(w[1]), ternary_value(w[2]), ternary_value(w[3]));
+            lds_barrier();
+            return;
+        }
         chacha20_block(f.key, at >> 3, f.stream + job.poly, w);
         const bool upper = at & 4;
 #pragma unroll
@@ -1534,9 +1560,33 @@ hipError_t launch_flood_rows(const NttArgs &args, ChaChaKey key, uint64_t stream
     a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
     const dim3 grid(n_jobs << (a.log_n - 10));
     const NttHead head = ntt_head(a, grid.x, 0);
-    const FloodExtra f{key, stream_id, cdt, cdt_len};
+    const FloodExtra f{key, stream_id, cdt, cdt_len, nullptr};
     switch (a.log_n - 8) {
-#define HE_CASE(LD) case LD: hipLaunchKernelGGL(flood_rows_kernel<LD>, grid, dim3(256), 0, s, HE_HEAD_ARGS(head), f); break;
+#define HE_CASE(LD) case LD: hipLaunchKernelGGL((flood_rows_kernel<LD, false>), grid, dim3(256), 0, s, HE_HEAD_ARGS(head), f); break;
+        HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
+#undef HE_CASE
+        default: return hipErrorInvalidValue;
+    }
+    return hipGetLastError();
+}
+
+// One workgroup for every CU, those with the errors counted: 4 limbs of 2^16 words, 256 of tiles and 64 of errors, take as long as the two
+// launches (8.0 us)
+bool encrypt_rows_ok(uint32_t log_n, uint32_t limbs, uint32_t items, uint32_t cus) {
+    return flood_rows_ok(log_n, limbs, items, cus) && ((uint64_t)items * (limbs + 1) << (log_n - 10)) <= cus;
+}
+
+hipError_t launch_encrypt_rows(const NttArgs &args, ChaChaKey key, uint64_t stream_id, int8_t *small, uint32_t items, int backend, hipStream_t s) {
+    const uint32_t n_jobs = items * args.map.limbs;
+    if (items == 0 || args.jobs || !encrypt_rows_ok(args.log_n, args.map.limbs, items, args.cus)) return hipErrorInvalidValue;
+    NttArgs a = args;
+    a.fp_mask = backend == NTT_BACKEND_INT ? 0 : (backend == NTT_BACKEND_FP ? ~(uint64_t)0 : a.fp_mask);
+    const uint32_t tiles = n_jobs << (a.log_n - 10);
+    const dim3 grid(tiles + (2 * items << (a.log_n - 11)));
+    const NttHead head = ntt_head(a, tiles, 0);
+    const FloodExtra f{key, stream_id, nullptr, 0, small + ((size_t)items << a.log_n)};
+    switch (a.log_n - 8) {
+#define HE_CASE(LD) case LD: hipLaunchKernelGGL((flood_rows_kernel<LD, true>), grid, dim3(256), 0, s, HE_HEAD_ARGS(head), f); break;
         HE_CASE(4) HE_CASE(5) HE_CASE(6) HE_CASE(7) HE_CASE(8)
 #undef HE_CASE
         default: return hipErrorInvalidValue;

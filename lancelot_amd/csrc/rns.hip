@@ -1274,9 +1274,9 @@ __device__ __forceinline__ void signed_values(int *v, const uint32_t *w, const u
 #pragma unroll
     for (int e = 0; e < per_block; e++) {
         if (KIND == SAMPLE_TERNARY) {
-            v[e] = (int)(((uint64_t)w[e] * 3) >> 32) - 1;
+            v[e] = ternary_value(w[e]);
         } else if (KIND == SAMPLE_ERROR) {
-            v[e] = __popc(w[2 * e] & 0x1FFFFFu) - __popc(w[2 * e + 1] & 0x1FFFFFu);
+            v[e] = error_value(w[2 * e], w[2 * e + 1]);
         } else {
             uint64_t u = ((uint64_t)w[2 * e + 1] << 32) | w[2 * e];
             const bool neg = u >> 63;
@@ -1332,8 +1332,7 @@ __device__ __forceinline__ void sample_bytes(const SmallArgs &p, uint64_t stream
     signed_values<KIND>(v, w, nullptr, 0);
     uint32_t *dst = reinterpret_cast<uint32_t *>(out + (size_t)per_block * b);
 #pragma unroll
-    for (int e = 0; e < per_block; e += 4)
-        dst[e / 4] = (uint32_t)(v[e] & 255) | ((uint32_t)(v[e + 1] & 255) << 8) | ((uint32_t)(v[e + 2] & 255) << 16) | ((uint32_t)(v[e + 3] & 255) << 24);
+    for (int e = 0; e < per_block; e += 4) dst[e / 4] = four_bytes(v[e], v[e + 1], v[e + 2], v[e + 3]);
 }
 
 // u of every item, then e0, e1 of every item; blockIdx.y = polynomial
