@@ -166,17 +166,24 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
         }
     }
     int small[4] = {0, 0, 0, 0};   // an encryption's errors (pro_small)
+    uint64_t src_q = 0, dst_q = 0, dst_r1 = 0;
     auto sources = [&]() {
+        if constexpr (!MDR) {
+            src_q = scalar(a.moduli)[job.src_table];
+            dst_q = scalar(a.moduli)[job.table];
+            dst_r1 = scalar(a.barrett)[2 * job.table + 1];
+        }
         source_words<T4>(s, a, MDR ? a.pro_last : job.src_table, lds, t, [&]() {
+            // (the moduli too: behind the pass they would be another trip to memory)
+            if constexpr (!MDR) asm volatile("" ::"s"(src_q), "s"(dst_q), "s"(dst_r1));
             if constexpr (SMALL) {
 #pragma unroll
                 for (int j = 0; j < 4; j++) small[j] = (a.pro_small + ((size_t)job.poly << a.log_n))[glob(0, j)];
             }
         });
         if constexpr (SMALL) {
-            const uint64_t p = scalar(a.moduli)[job.src_table];
 #pragma unroll
-            for (int j = 0; j < 4; j++) s[j] = add_small(s[j], small[j], p);
+            for (int j = 0; j < 4; j++) s[j] = add_small(s[j], small[j], src_q);
         }
         if constexpr (MDR) source_words<T4>(s2, a, a.pro_src_table, lds2, t, []() {});
     };
@@ -199,9 +206,11 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             T4::template load_tw<FpArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) sources();
             if constexpr (SRC_INTT && !MDR) {
-                const uint64_t q = scalar(a.moduli)[job.table], r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = fp_from_u64(SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1));
+                for (int j = 0; j < 4; j++) {
+                    const uint64_t w = barrett64(s[j], dst_q, dst_r1);
+                    v[j] = fp_from_u64(SMALL ? add_small(w, -small[j], dst_q) : w);
+                }
             } else if constexpr (SMALL) {
                 const bool values = a.pro_values && !(job.poly & 1);
                 double r[4];
@@ -244,9 +253,11 @@ __global__ __launch_bounds__(1 << (B - 2)) void ntt_rows_kernel(HE_HEAD_PARAMS, 
             T4::template load_tw<IntArith, 0>(tw, ar, 1, t);
             if constexpr (SRC_INTT) sources();
             if constexpr (SRC_INTT && !MDR) {
-                const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
 #pragma unroll
-                for (int j = 0; j < 4; j++) v[j] = SMALL ? add_small(barrett64(s[j], q, r1), -small[j], q) : barrett64(s[j], q, r1);
+                for (int j = 0; j < 4; j++) {
+                    const uint64_t w = barrett64(s[j], dst_q, dst_r1);
+                    v[j] = SMALL ? add_small(w, -small[j], dst_q) : w;
+                }
             } else if constexpr (SMALL) {
                 const bool values = a.pro_values && !(job.poly & 1);
                 const uint64_t r1 = scalar(a.barrett)[2 * job.table + 1];
