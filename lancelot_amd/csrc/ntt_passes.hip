@@ -581,7 +581,7 @@ struct InnerMany {
 // FP64 kernel from 96 registers to 120).
 // SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
 // and waves 0 and 1 finish one polynomial each.
-// STREAM: 1: the key words pass by the caches; 2: the digits' words do, which nothing reads again; 3: both (launch_ntt_inner says when).
+// STREAM: 1: the key words pass by the caches; 2: the digits' words do, which nothing reads again; 3: both; 4: neither, with twiddles read (launch_ntt_inner says when).
 template <int SPLIT, int STREAM, class A, class X>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32_t L, uint32_t LK, uint32_t beta, uint32_t t,
                                             uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
@@ -846,7 +846,7 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PAR
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
     if (BE != NTT_BACKEND_INT && fp) {
-        const typename std::conditional<SPLIT == 1, FpProducts<true>, FpArith>::type ar{fp_arith(a, table)};
+        const typename std::conditional<SPLIT == 1 && STREAM != 4, FpProducts<true>, FpArith>::type ar{fp_arith(a, table)};
         inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, ar, part, sums);
     }
     if constexpr (BE != NTT_BACKEND_FP) {
@@ -1718,6 +1718,11 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     const bool stream_keys = items == 1 && (((3 * (uint64_t)x.beta + 2) * (x.L + x.K) + 4 * (uint64_t)x.L) << a.log_n) >= (uint64_t)400 << 16;
     // The digits' words of products whose buffers go round the cache between two uses: see stream_products.
     const bool stream_words = x.fold_ct && stream_products(items, x.L, a.log_n);
+    // Twiddles worked out (FpProducts) where the waves are many enough to be bound by what they move, read elsewhere: one product, us worked out /
+    // read, by waves, 50 bits and less: 832 (2^14, 5 + 8 limbs) 31.4 / 31.0, 1664 (2^15, 5 + 8) 39.7 / 38.8, 2048 (2^15, 8 + 8) 42.3 / 40.7, 2816 (2^16,
+    // 5 + 6) 45.1 / 44.8, 2560 (2^16, 8 + 2) 52.7 / 53.1, 4096 (2^16, 8 + 8 and 12 + 4) 51.5 / 51.5, 63.3 / 63.4, and a rotation 17.8 -> 16.4 in this
+    // kernel; batches, whose waves find them in their CU's cache: 4 of 3 + 1 limbs of 2^16 57.4 / 57.0, 16 of 8 + 2 of 2^13 70.7 / 69.8.
+    const bool read_twiddles = items > 1 || pairs < 3072;
 #define HE_INNER_BE(BE, SPLIT, STREAM)                                                                                             \
     do {                                                                                                                          \
         if (items == 1 && x.beta <= InnerFew::kDigits)                                                                            \
@@ -1744,6 +1749,8 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
         HE_INNER(1, 1);
     else if (stream_words)
         HE_INNER(1, 2);
+    else if (read_twiddles)
+        HE_INNER(1, 4);
     else
         HE_INNER(1, 0);
 #undef HE_INNER
