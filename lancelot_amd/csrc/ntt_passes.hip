@@ -1424,7 +1424,7 @@ __global__ __launch_bounds__(256) void flood_rows_kernel(HE_HEAD_PARAMS, FloodEx
 // the passes need that go over the same words one after the other: they meet them in the XCD's L2 (2 x 6 limbs of 2^16 words 10.8 us, dealt
 // out 13.1).  But with few limbs of both arithmetics, two XCDs have all the work of a 60-bit limb and two that of a 40-bit one.
 //
-// Encryption's blocks pass: up to four items, of which an XCD's range is half of one or less; a range over more evens itself out.
+// Encryption's blocks pass with several special primes (the lines were measured with one as well): up to four items, of which an XCD's range is half of one or less; a range over more evens itself out.
 // Together / dealt, us of an encryption on 60 + 40 .. + 60 bits, L + K limbs x items: 2^16, 3 + 1 x 1 32.4 / 29.2, x 2 48.1 / 44.0, x 4
 // 64.4 / 63.5, x 6 81.3 / 83.0, x 20 210 / 211, 20 + 4 x 1 96.9 / 84.2, x 4 254 / 240; 2^15, 10 + 2 x 1 43.3 / 38.2, x 4 82.5 / 80.9.  Short
 // limbs need more workgroups: 2^14, 12 + 4 x 1 35.0 / 31.1, 3 + 1 x 2 23.4 / 24.1, x 3 27.1 / 29.1, x 6 33.6 / 38.5, 12 + 4 x 2 47.3 / 45.4, x 4
@@ -1433,6 +1433,15 @@ bool spread_encryption(const NttArgs &a, int backend, uint32_t items, uint64_t w
     if (backend != NTT_BACKEND_MIXED || items > 4) return false;
     const uint64_t halves = a.log_n >= 15 || items == 1 ? 3 : items == 2 ? 6 : 24;   // workgroups for every two CUs
     return 2 * wgs >= halves * a.cus;
+}
+
+// Encryption with one special prime (encrypt_products_kernel), which is shorter: limbs of 2^16 words always, of 2^15 up to 16 of them, of fewer a
+// single encryption's.  Together / dealt, us, limbs x items: 2^16, 4 x 1 27.8 / 27.0, 4 x 10 97.5 / 93.3, 4 x 20 172 / 165, 10 x 10 189 / 178, 21 x 1
+// 55.8 / 54.6, but 4 x 4 52.2 / 53.0; 2^15, 10 x 1 28.8 / 27.8, 4 x 4 36.2 / 35.1, 10 x 2 38.5 / 39.5, 21 x 1 40.4 / 41.0, 4 x 6 45.4 / 46.8, 10 x 4
+// 54.2 / 56.2; 2^14, 13 x 1 23.7 / 22.6, 21 x 1 28.3 / 27.2, 4 x 2 21.2 / 21.1, 4 x 4 24.8 / 25.7, 10 x 4 39.8 / 41.3; 2^13, 10 x 1 18.5 / 18.6, 10 x 4 26.5 / 28.0.
+bool spread_products(const NttArgs &a, int backend, uint32_t items, uint32_t limbs) {
+    if (backend != NTT_BACKEND_MIXED || 2 * ((uint64_t)items * limbs << (a.log_n - 8)) < 3 * (uint64_t)a.cus) return false;
+    return a.log_n >= 16 || (a.log_n == 15 ? (uint64_t)items * limbs <= 16 : items == 1);
 }
 
 // A blocks pass with an epilogue, where its caller asks for it (NttArgs::deal) and from three workgroups per CU on.  Behind an inner
@@ -1863,7 +1872,7 @@ hipError_t launch_encrypt_products(const NttArgs &args, const uint64_t *pk, uint
     for (uint32_t first = 0; first < items; first += per_launch) {
         const uint32_t now = items - first < per_launch ? items - first : per_launch;
         const dim3 grid(now * wgs_per_item);
-        a.spread = spread_encryption(a, backend, items, (uint64_t)now * (L + K) << (a.log_n - 8));
+        a.spread = spread_products(a, backend, items, L + K);
         const NttHead head = ntt_head(a, grid.x, first);
         if (backend == NTT_BACKEND_MIXED)
             hipLaunchKernelGGL(encrypt_products_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw, wide);
