@@ -187,11 +187,12 @@ PYBIND11_MODULE(pyCAHEL, m) {
              py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count") = 1)
         .def("decrypt_decode_each",
              [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, CAHELGPUCKKSEncoder &e, const std::vector<const CAHELGPUCiphertext *> &cts) {
-                 py::array_t<double> out((py::ssize_t)(cts.size() * e.decoded_slots()));
+                 const std::size_t slots = e.decoded_slots();   // (once, under the interpreter's lock: what the array holds)
+                 py::array_t<double> out((py::ssize_t)(cts.size() * slots));
                  double *values = out.mutable_data();
                  {
                      py::gil_scoped_release release;
-                     k.decrypt_decode_each(c, e, cts, values);
+                     k.decrypt_decode_each(c, e, cts, slots, values);
                  }
                  return out;
              },

@@ -287,35 +287,34 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
 }
 
 void CAHELGPUSecretKey::decrypt_decode_each(const CAHELGPUContext &context, CAHELGPUCKKSEncoder &encoder,
-                                            const std::vector<const CAHELGPUCiphertext *> &ciphers, double *destination) {
+                                            const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots,
+                                            double *destination) {
     he_context *h = context.handle();
     he_stream st = context.stream();
     PinnedRing &ring = PinnedRing::of_thread();
     std::optional<PinnedRing::Held> ahead;   // of the ciphertext in front
     const double *values = nullptr;
-    std::size_t count = 0;
     auto finish = [&] {
         if (!ahead) return;
         ahead->wait();
-        std::memcpy(destination, values, count * sizeof(double));
-        destination += count;
+        std::memcpy(destination, values, slots * sizeof(double));
+        destination += slots;
         ahead.reset();
     };
     for (const CAHELGPUCiphertext *ct : ciphers) {
         if (!ct) throw std::invalid_argument("encrypted is not valid");
         CAHELGPUPlaintext plain(context);
         decrypt(context, *ct, plain);
-        const std::size_t taken = encoder.decode_count(context, plain, 0);   // (all slots)
+        (void)encoder.decode_count(context, plain, 0);   // (checks the plaintext; the encoder's own count may change meanwhile, the array does not)
         const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
-        DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)taken));
-        double *host = static_cast<double *>(ring.take(taken * sizeof(double)));
-        const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)taken, plain.scale(), host, (uint32_t)taken,
+        DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)slots));
+        double *host = static_cast<double *>(ring.take(slots * sizeof(double)));
+        const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)slots, plain.scale(), host, (uint32_t)slots,
                                                ws.get(), st);
         PinnedRing::Held held(ring, st);
         check_status(status, "he_ckks_decode_real");
         finish();
         values = host;
-        count = taken;
         ahead.emplace(std::move(held));
     }
     finish();

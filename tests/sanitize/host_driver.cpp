@@ -5,6 +5,7 @@
 // a record (any std::exception), it may not crash or touch memory it does not own.  Exit code 0 = clean.
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <random>
 #include <sstream>
 #include <stdexcept>
@@ -17,6 +18,8 @@
 using namespace cahel;
 
 extern const char *mock_failing;   // mock_device.cpp
+extern bool mock_decodes;
+extern std::function<void()> mock_meanwhile;
 
 #define REQUIRE(cond)                                                        \
     do {                                                                     \
@@ -314,6 +317,58 @@ int main(int argc, char **argv) {
                 }
         }
         REQUIRE(encoder.encode_encrypt_updates(context, pk, {}, 5, scale).empty());
+    }
+
+    // ---- decryptions that are enqueued before the values in front are waited for: the values of every ciphertext in their place, in an array
+    // of the slot count that the encoder had at the start, whatever becomes of that meanwhile ----
+    {
+        set_lane(0);
+        CAHELGPUCKKSEncoder encoder(context);
+        CAHELGPUSecretKey secret(parms);
+        secret.gen_secretkey(context);
+        const std::size_t L2 = context.limbs_at(2), few = n / 8;
+        auto value = [](std::size_t k, std::size_t i) { return 1.0 + (double)k + 1e-6 * (double)i; };
+        std::vector<CAHELGPUCiphertext> cts;
+        std::vector<const CAHELGPUCiphertext *> ptrs;
+        for (std::size_t k = 0; k < 7; k++) {
+            cts.emplace_back(context);
+            cts.back().resize(context, 2, 2);
+            cts.back().scale() = 1048576.0;
+            cts.back().is_ntt_form() = true;
+            for (std::size_t i = 0; i < L2 * n; i++) {
+                const double v = value(k, i);
+                std::memcpy(cts.back().data() + i, &v, sizeof(v));
+            }
+        }
+        for (const auto &ct : cts) ptrs.push_back(&ct);
+        CAHELGPUPlaintext message(context);
+        encoder.encode(context, std::vector<double>(few, 0.5), 1048576.0, message);   // fixes the slot count
+        mock_decodes = true;
+        auto decoded = [&](std::size_t slots) {
+            std::vector<double> out(cts.size() * slots);
+            secret.decrypt_decode_each(context, encoder, ptrs, slots, out.data());
+            for (std::size_t k = 0; k < cts.size(); k++)
+                for (std::size_t i = 0; i < slots; i++)
+                    if (out[k * slots + i] != value(k, i)) return false;
+            return true;
+        };
+        REQUIRE(encoder.decoded_slots() == few && decoded(few));
+        int calls = 0;
+        mock_meanwhile = [&] {
+            if (++calls == 3) encoder.reset_sparse_slots();
+        };
+        REQUIRE(decoded(few) && encoder.decoded_slots() == n / 2);   // (a decoding fixes the full count)
+        calls = 0;
+        mock_meanwhile = [&] {
+            if (++calls == 2) {
+                encoder.reset_sparse_slots();
+                CAHELGPUPlaintext p(context);
+                encoder.encode(context, std::vector<double>(few, 0.5), 1048576.0, p);
+            }
+        };
+        REQUIRE(decoded(n / 2) && encoder.decoded_slots() == few);
+        mock_meanwhile = nullptr;
+        mock_decodes = false;
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused

@@ -18,6 +18,9 @@ struct he_context {
 
 // the call that fails from now on, or nullptr
 const char *mock_failing = nullptr;
+// whether he_ckks_decode_real succeeds; what happens during each he_decrypt_flood (another thread's doing)
+bool mock_decodes = false;
+std::function<void()> mock_meanwhile;
 
 namespace {
 
@@ -223,12 +226,59 @@ int he_ckks_decode(const he_context *, const uint64_t *, uint32_t, uint32_t, dou
     return HE_E_UNSUPPORTED;
 }
 size_t he_ckks_decode_real_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
-// Fails behind its first launches: what they write comes later all the same.
-int he_ckks_decode_real(const he_context *, const uint64_t *, uint32_t, uint32_t, double, double *out, uint32_t count, uint64_t *,
+// "Decodes" later: the bits of word i as value i.  Unless mock_decodes, fails behind its first launches: what they write comes later all the same.
+int he_ckks_decode_real(const he_context *, const uint64_t *plain, uint32_t, uint32_t slots, double, double *out, uint32_t count, uint64_t *,
                         he_stream stream) {
+    if (count > slots) return HE_E_INVALID_ARGUMENT;
+    if (mock_decodes) {
+        queues[stream].push_back([=] { std::memcpy(out, plain, count * sizeof(double)); });
+        return HE_OK;
+    }
     queues[stream].push_back([=] { std::memset(out, 0x66, count * sizeof(double)); });
     return HE_E_UNSUPPORTED;
 }
+
+// "Decrypts" later: the words of polynomial 0.
+int he_decrypt_flood(const he_context *ctx, const uint64_t *ct, uint32_t, uint32_t limbs, const uint64_t *, size_t, const uint32_t *, uint64_t,
+                     const uint64_t *, uint32_t, uint64_t *plain, uint64_t *, he_stream stream) {
+    queues[stream].push_back([=] { std::memcpy(plain, ct, ((size_t)limbs << ctx->log_n) * sizeof(uint64_t)); });
+    if (mock_meanwhile) mock_meanwhile();
+    return HE_OK;
+}
+size_t he_decrypt_decode_real_workspace_words(const he_context *, uint32_t, uint32_t, uint32_t) { return 1; }
+// Decryption and decoding of a batch, later: the first `count` words of polynomial 0 of every ciphertext, as (re, im) pairs of equal values
+int he_decrypt_decode_flood_batch(const he_context *, const uint64_t *const *d_cts, uint32_t items, uint32_t, const uint64_t *, const uint32_t *,
+                                  uint64_t, const uint64_t *, uint32_t, uint32_t, double, uint32_t count, double *out, uint64_t *,
+                                  he_stream stream) {
+    queues[stream].push_back([=] {
+        for (size_t k = 0; k < items; k++)
+            for (size_t i = 0; i < 2 * (size_t)count; i++) std::memcpy(out + 2 * k * count + i, d_cts[k] + i / 2, sizeof(double));
+    });
+    return HE_OK;
+}
+
+// (what keys.cpp refers to besides; a secret key is sampled and transformed)
+int he_sample(const he_context *ctx, int, const uint32_t *, uint64_t stream_id, uint64_t *out, uint32_t limbs, uint32_t, uint32_t, uint32_t,
+              const uint64_t *, uint32_t, he_stream stream) {
+    queues[stream].push_back([=] {
+        for (size_t i = 0; i < (size_t)limbs << ctx->log_n; i++) out[i] = stream_id;
+    });
+    return HE_OK;
+}
+int he_ntt_forward(const he_context *, uint64_t *, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, he_stream) { return HE_OK; }
+int he_add(const he_context *, const uint64_t *, const uint64_t *, uint64_t *, uint32_t, uint32_t, uint32_t, he_stream) { return HE_E_UNSUPPORTED; }
+int he_multiply(const he_context *, const uint64_t *, const uint64_t *, uint64_t *, uint32_t, uint32_t, uint32_t, he_stream) {
+    return HE_E_UNSUPPORTED;
+}
+int he_multiply_add(const he_context *, const uint64_t *, const uint64_t *, const uint64_t *, uint64_t *, uint32_t, uint32_t, uint32_t, int,
+                    he_stream) { return HE_E_UNSUPPORTED; }
+int he_add_p_multiple(const he_context *, const uint64_t *, const uint64_t *, uint64_t *, uint32_t, uint32_t, he_stream) { return HE_E_UNSUPPORTED; }
+int he_galois_ntt(const he_context *, const uint64_t *, uint64_t *, uint32_t, uint32_t, he_stream) { return HE_E_UNSUPPORTED; }
+int he_encrypt(const he_context *, uint32_t, const uint64_t *, const uint64_t *, const uint32_t *, uint64_t, uint64_t *, uint64_t *, he_stream) {
+    return HE_E_UNSUPPORTED;
+}
+int he_decrypt_decode_real_batch(const he_context *, const uint64_t *const *, uint32_t, uint32_t, const uint64_t *, const uint32_t *, uint64_t,
+                                 const uint64_t *, uint32_t, uint32_t, double, uint32_t, double *, uint64_t *, he_stream) { return HE_E_UNSUPPORTED; }
 
 size_t he_keyswitch_workspace_words(const he_context *ctx, uint32_t L) { return ctx ? (size_t)L << ctx->log_n : 0; }
 

@@ -40,6 +40,21 @@ def test_decrypt_and_decode_one_after_the_other(log_n, items, size):
     assert a.sk.decrypt_decode_each(a.context, a.encoder, []).size == 0
 
 
+@pytest.mark.parametrize("length", [100, 1025])
+def test_each_decoded_with_the_slot_count_of_the_encoder(length):
+    """An encoder whose first message has fixed fewer slots than the ring has."""
+    state = state_of(8, 13)
+    values = np.random.default_rng(length).uniform(-1, 1, (3, length))
+    cts = state.encoder.encode_encrypt_many(state.context, state.pk, values, SCALE)
+    slots = 1 << (length - 1).bit_length()
+    got = state.sk.decrypt_decode_each(state.context, state.encoder, cts)
+    assert got.shape == (3 * slots,)
+    got = got.reshape(3, slots)
+    assert np.abs(got[:, :length] - values).max() < 1e-4 and np.abs(got[:, length:]).max() < 1e-4
+    state.encoder.reset_sparse_slots()
+    assert state.sk.decrypt_decode_each(state.context, state.encoder, cts[:1]).shape == (state.slots,)
+
+
 @pytest.mark.parametrize("log_n,items,messages", [(13, 1, 2), (13, 5, 1), (15, 2, 17)])   # 17: five blocks of messages in a ring of four
 def test_values_and_encryptions_at_once(log_n, items, messages):
     a, b = state_of(6, log_n), state_of(6, log_n)

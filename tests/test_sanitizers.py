@@ -2,8 +2,8 @@
 
 * oracle/ckks_oracle.c: a sanitizer build of the oracle is loaded by a child interpreter (sanitizer runtime
   preloaded) that runs the oracle's own pinning tests against it;
-* the host layer's number theory, table construction, record parsing and encodings in flight (hostmath.cpp, context.cpp,
-  serialize.cpp, encoder.cpp):
+* the host layer's number theory, table construction, record parsing, encodings and decryptions in flight (hostmath.cpp, context.cpp,
+  serialize.cpp, encoder.cpp, keys.cpp):
   tests/sanitize/host_driver.cpp over the host-memory mock of the device ABI, ending with a bounded seeded loop of
   damaged and random records into every load() entry (it stops at the first report: the sanitizers abort).
 """
@@ -53,7 +53,7 @@ def test_host_layer_under_asan_ubsan(tmp_path):
     exe = str(tmp_path / "host_driver")
     sources = [os.path.join(ROOT, "tests", "sanitize", "host_driver.cpp"), os.path.join(ROOT, "tests", "sanitize", "mock_device.cpp"),
                os.path.join(HOST, "hostmath.cpp"), os.path.join(HOST, "context.cpp"), os.path.join(HOST, "serialize.cpp"),
-               os.path.join(HOST, "encoder.cpp")]
+               os.path.join(HOST, "encoder.cpp"), os.path.join(HOST, "keys.cpp")]
     subprocess.check_call(["g++", "-std=c++17", *SAN, "-I", os.path.join(ROOT, "include"), "-I", HOST, *sources, "-o", exe])
     env = dict(os.environ)
     env["ASAN_OPTIONS"] = "abort_on_error=1:detect_leaks=1"
