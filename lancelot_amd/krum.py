@@ -61,6 +61,8 @@ class KrumState:
     rlk: object
     encoder: object
     slots: int
+    # Seconds a phase.  Those of a batched round between marks on the device's queue, by its clock, each from the end of the phase in front;
+    # all others, and the total, by the host's.
     timings: dict = field(default_factory=lambda: {"encode": 0.0, "encrypt": 0.0, "evaluate": 0.0, "decrypt": 0.0})
     marks: list = field(default_factory=list)   # (phase, mark at its start, mark at its end) of the round on its way
 
@@ -476,6 +478,11 @@ def _mask(state: KrumState, scores, constants=None):
     return [[one if order[r] == k else zero for k in range(n_clients)] for r in range(n_clients)], order
 
 
+def _masked_sum(state: KrumState, cts, mask_row):
+    sums = state.cahel.multiply_sum(state.context, [[client[chunk] for client in cts[:len(mask_row)]] for chunk in range(len(cts[0]))], mask_row)
+    return state.sk.decrypt_decode_each(state.context, state.encoder, sums)
+
+
 def mul_mask_weight(state: KrumState, cts, mask_row):
     """sum_k mask_row[k] * update_k chunk by chunk with lazy relinearisation: the products stay size-3
     ciphertexts, are added, and are decrypted as such (byzantine_fl.py:371-429, lazy_relin_flag branch).
@@ -484,8 +491,7 @@ def mul_mask_weight(state: KrumState, cts, mask_row):
     t0 = time.perf_counter()
     n_chunks = len(cts[0])
     if state.config.batched:
-        sums = c.multiply_sum(ctx, [[client[chunk] for client in cts[:len(mask_row)]] for chunk in range(n_chunks)], mask_row)
-        out = state.sk.decrypt_decode_each(ctx, state.encoder, sums)
+        out = _masked_sum(state, cts, mask_row)
         state.timings["mask_multiply"] = state.timings.get("mask_multiply", 0.0) + time.perf_counter() - t0
         return out
     out = []
@@ -558,14 +564,17 @@ def gpu_krum_aggregate(updates, config: KrumConfig | None = None, state: KrumSta
         scores, constants = state.sk.decrypt_decode_complex_and_encrypt_many(
             state.context, packed, state.slots, 1, state.encoder, state.pk, _mask_constants(state), state.config.scale)
         mask, order = _mask(state, _unpacked(scores, n_clients), constants)
-        _mark(state, "mask", evaluated)
+        masked = _mark(state, "mask", evaluated)
+        # (by the device's clock too: the constants are the mask's time, and the host does not wait for them)
+        weights = _masked_sum(state, cts, mask[0])
+        _mark(state, "mask_multiply", masked)
     else:
         t1 = time.perf_counter()
         enc = [[None] * n_clients for _ in range(n_clients)]
         all_pair_distances(state, cts, enc)
         state.timings["evaluate"] += time.perf_counter() - t1
         mask, order, _ = decrypt_sort_mask(state, enc)
-    weights = mul_mask_weight(state, cts, mask[0])
+        weights = mul_mask_weight(state, cts, mask[0])
     total = time.perf_counter() - t0
     _settle(state)
     length = len(np.asarray(updates[0]).reshape(-1))

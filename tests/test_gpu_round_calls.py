@@ -86,3 +86,18 @@ def test_phases_of_a_round_add_up(aggregate):
     phases = ["encode", "evaluate", "mask", "mask_multiply"] if aggregate else ["encode", "evaluate", "decrypt"]
     assert all(timings[k] > 0 for k in phases) and not state.marks
     assert timings["encode"] + timings["evaluate"] < timings["total"]
+
+
+@pytest.mark.parametrize("aggregate", [False, True])
+def test_no_time_of_a_round_is_in_two_phases(aggregate):
+    """At 2^16 the mask's constants take the device some 50 us, which are the mask's and not the masked sum's as well.  15 us: by what the device
+    reaches the last mark behind the clock that ends the round."""
+    from lancelot_amd import krum
+    state = state_of(9, 16)
+    rng = np.random.default_rng(2)
+    updates = [rng.normal(0, 0.01, 40000).astype(np.float32) for _ in range(4)]
+    over = []
+    for _ in range(9):
+        timings = dict((krum.gpu_krum_aggregate if aggregate else krum.gpu_krum)(updates, state=state)[2])
+        over.append(sum(timings.values()) - 2 * timings["total"])
+    assert np.median(over[2:]) < 15e-6, (over, timings)
