@@ -512,7 +512,8 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
 // Sum over the digits of (word x key word) for four words of both key polynomials.
 // FP64: a transformed word enters as the last stage leaves it (at most 3.7 q: a term below 1.9 q), the sums are reduced after
 // every fourth digit and stay below 8 q.  Integers: 128-bit sums of at most 64 products below 2^122 of canonical words, or, with primes
-// below 2^60, of at most 32 products of words as the last stage leaves them (below 8 q).
+// below 2^60, of at most 32 products of words as the last stage leaves them (below 8 q):
+// a wave's share of kMaxDigits, since only waves that share a block leave them so.
 struct FpSums {
     double s[2][4];
     uint32_t pending = 0;
@@ -656,7 +657,7 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
         }
     }
     bool canonical = false;
-    if constexpr (!FP) canonical = (ar.m.q >> 60) || beta > 32;
+    if constexpr (!FP) canonical = ar.m.q >> 60;
     typename std::conditional<FP, FpSums, IntSums>::type sums;
     if (own != 0xffffffffu && part == 0) {
         const uint64_t *src = a.in + (size_t)t * n;
@@ -703,7 +704,19 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
     if constexpr (SPLIT > 1) {
         // (integers: the 128-bit sums as they are, so that each is reduced once, by the wave that finishes it, and not by all that share it;
         // with the words' reductions left out where they can be, rotations: n = 2^15, 10 + 3 limbs of 60 / 40 bits 51.9 -> 50.8 us; 2^14, 4 + 1
-        // of 60 bits 23.6 -> 22.7; 2^16, 2 + 1 29.5 -> 28.8)
+        // of 60 bits 23.6 -> 22.7; 2^16, 2 + 1 29.5 -> 28.8.  A wave's sum of lazy words is below 2^128 q^2 / 2^120 (two waves) or half of that
+        // (four); from 33 digits on all of them could pass 2^128, so one that has reached 2^127 (2^126) gives q 2^67 (q 2^66) away and is below it
+        // again.  A reduction of every word instead took 2 to 3.5 % of a whole product: 36 digits of 2^13 and 60 bits 141.5 / 137.0 us.)
+        static_assert(kMaxDigits <= 64, "a wave's sum fits 128 bits");
+        if constexpr (!FP) {
+            constexpr int top = SPLIT == 2 ? 63 : 62;
+            if (beta > 32 && !canonical) {
+#pragma unroll
+                for (int r = 0; r < 2; r++)
+#pragma unroll
+                    for (int j = 0; j < 4; j++) sums.s[r][j].hi -= sums.s[r][j].hi >> top ? ar.m.q << (top - 60) : 0;
+            }
+        }
 #pragma unroll
         for (int r = 0; r < 2; r++) {
             uint64_t w[4];

@@ -1,5 +1,5 @@
 """Inner products whose blocks are shared by two or four waves, on integers: the waves' 128-bit sums meet before they are reduced, and words
-enter them as the last stage leaves them where primes and digits allow it (below 2^60, up to 32 digits).  Against the oracle, with keys of the
+enter them as the last stage leaves them where primes and digits allow it (below 2^60, the waves' sums are cut back from 33 digits on).  Against the oracle, with keys of the
 largest residues."""
 import numpy as np
 import pytest
@@ -19,9 +19,12 @@ def capi():
 @pytest.mark.parametrize("logn,bits,size_p,L", [(12, [60] * 5, 1, 4),                # four waves a block, lazy words
                                                  (13, [60] + [40] * 11 + [60] * 4, 4, 10),   # two waves, limbs of both arithmetics
                                                  (12, [60] * 33, 1, 32),              # the last number of digits with lazy words
-                                                 (12, [60] * 34, 1, 33),              # the first with canonical ones
+                                                 (12, [60] * 34, 1, 33),              # the first whose waves' sums could pass 2^128 together
                                                  (12, [60] * 41, 1, 40),
-                                                 (12, [60] * 42, 1, 41)])
+                                                 (12, [60] * 42, 1, 41),
+                                                 (12, [60] * 64, 1, 63),              # the most digits of a chain of 64 primes
+                                                 (13, [60] * 50, 1, 49),
+                                                 (11, [60] * 64, 1, 63)])             # four waves a block
 def test_split_inner_products(oracle, capi, logn, bits, size_p, L):
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     rng = np.random.default_rng(L)
