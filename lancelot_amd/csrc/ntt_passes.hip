@@ -582,7 +582,7 @@ struct InnerMany {
 // FP64 kernel from 96 registers to 120).
 // SPLIT waves share a block when there are few: wave `part` takes every SPLIT-th digit, the partial sums meet in LDS (`sums_lds`),
 // and waves 0 and 1 finish one polynomial each.
-// STREAM: 1: the key words pass by the caches; 2: the digits' words do, which nothing reads again; 3: both; 4: neither, with twiddles read (launch_ntt_inner says when).
+// STREAM: 1: the key words pass by the caches; 2: the digits' words do, which nothing reads again; 3: both (launch_ntt_inner says when).
 template <int SPLIT, int STREAM, class A, class X>
 __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32_t L, uint32_t LK, uint32_t beta, uint32_t t,
                                             uint32_t table, uint32_t blk, uint32_t item, uint32_t lane, const A &ar, uint32_t part,
@@ -822,7 +822,8 @@ __device__ __forceinline__ void inner_block(const NttArgs &a, const X &x, uint32
 // key words of the first in the CU's cache.  Across workgroups the items of a block run next to each other on one XCD.
 constexpr int kInnerWaves = 4;
 
-template <int BE, int SPLIT, int STREAM, class X>
+// PRODUCTS: see FpProducts (launch_ntt_inner says when)
+template <int BE, int SPLIT, int STREAM, bool PRODUCTS, class X>
 __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PARAMS, X x) {
     __shared__ uint64_t sums_all[SPLIT > 1 ? kInnerWaves / SPLIT : 1][SPLIT > 1 ? (BE == NTT_BACKEND_FP ? 2 : 4) * SPLIT * 256 : 1];
     NttArgs a;
@@ -859,7 +860,7 @@ __global__ __launch_bounds__(64 * kInnerWaves) void ntt_inner_kernel(HE_HEAD_PAR
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> table) & 1));
     uint64_t *sums = sums_all[SPLIT > 1 ? w / SPLIT : 0];
     if (BE != NTT_BACKEND_INT && fp) {
-        const typename std::conditional<SPLIT == 1 && STREAM != 4, FpProducts<true>, FpArith>::type ar{fp_arith(a, table)};
+        const typename std::conditional<PRODUCTS, FpProducts<true>, FpArith>::type ar{fp_arith(a, table)};
         inner_block<SPLIT, STREAM>(a, x, L, LK, h5 & 255, t, table, blk, item, lane, ar, part, sums);
     }
     if constexpr (BE != NTT_BACKEND_FP) {
@@ -1740,41 +1741,54 @@ hipError_t launch_ntt_inner(const NttArgs &args, const KsFuseArgs &x, int backen
     const bool stream_keys = items == 1 && (((3 * (uint64_t)x.beta + 2) * (x.L + x.K) + 4 * (uint64_t)x.L) << a.log_n) >= (uint64_t)400 << 16;
     // The digits' words of products whose buffers go round the cache between two uses: see stream_products.
     const bool stream_words = x.fold_ct && stream_products(items, x.L, a.log_n);
-    // Twiddles worked out (FpProducts) where the waves are many enough to be bound by what they move, read elsewhere: one product, us worked out /
-    // read, by waves, 50 bits and less: 832 (2^14, 5 + 8 limbs) 31.4 / 31.0, 1664 (2^15, 5 + 8) 39.7 / 38.8, 2048 (2^15, 8 + 8) 42.3 / 40.7, 2816 (2^16,
-    // 5 + 6) 45.1 / 44.8, 2560 (2^16, 8 + 2) 52.7 / 53.1, 4096 (2^16, 8 + 8 and 12 + 4) 51.5 / 51.5, 63.3 / 63.4, and a rotation 17.8 -> 16.4 in this
-    // kernel; batches, whose waves find them in their CU's cache: 4 of 3 + 1 limbs of 2^16 57.4 / 57.0, 16 of 8 + 2 of 2^13 70.7 / 69.8.
-    const bool read_twiddles = items > 1 || pairs < 3072;
-#define HE_INNER_BE(BE, SPLIT, STREAM)                                                                                             \
+    // Twiddles worked out (FpProducts) where one ciphertext's waves are many enough to be bound by what they move: from 3072 on, or with words
+    // that pass by the caches; with limbs of both arithmetics up to 11 digits, since a wave works them out once for all of its digits and the waves of
+    // integer limbs keep the launch waiting.  One product, us in this kernel read / worked out: 2^16, 24 + 8 limbs 35.2 / 34.7, 20 + 8 30.1 / 28.0, 12 + 3
+    // 19.9 / 18.9, 10 + 1 (2816 waves, keys streamed) 30.9 / 30.7, 24 + 2 90.1 / 87.2; 60 / 40 bits 24 + 4 57.3 / 55.9, 16 + 2 (8 digits) 52.2 / 52.5, rotation 50.8 /
+    // 50.1, 44 + 4 of 2^14 (11) 39.8 / 39.6, but 24 + 2 of 2^15 (12) 53.4 / 55.3, 24 + 1 100.2 / 101.4, 39 + 1 of 2^14 113.0 / 117.1; whole calls below the line: 832
+    // (2^14, 5 + 8 limbs) 31.0 / 31.4, 2816 (2^16, 5 + 6) 44.8 / 45.1.  A batch's waves find them in their
+    // CU's cache, read / worked out in this kernel: 4 x 24 + 8 limbs of 2^16 91.3 / 92.6, 16 x 3 + 1 33.6 / 33.8, 8 x 12 + 4 of 2^15 51.7 / 52.2, 60 / 40 bits 8 x 24 + 8
+    // 225.9 / 228.8, 4 x 24 + 8 119.1 / 120.4; but with 8192 blocks of FP64, 16 MB of twiddles, they are no loss, 8 x 24 + 8 178.6 / 177.3, and the whole
+    // call gains, 691 / 688, 2 x 24 + 8 205.2 / 204.4 (16 x 12 + 4, 4096 blocks, 649 / 652).
+    const bool products = backend == NTT_BACKEND_MIXED ? items == 1 && (pairs >= 3072 || stream_keys || stream_words) && x.beta < 12
+                          : items == 1                 ? pairs >= 3072 || stream_keys || stream_words
+                                                       : pairs >= 8192;
+#define HE_INNER_BE(BE, SPLIT, STREAM, PRODUCTS)                                                                                   \
     do {                                                                                                                          \
         if (items == 1 && x.beta <= InnerFew::kDigits)                                                                            \
-            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, InnerFew>), grid, block, 0, s, HE_HEAD_ARGS(head), few);       \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, PRODUCTS, InnerFew>), grid, block, 0, s, HE_HEAD_ARGS(head), few);   \
         else                                                                                                                      \
-            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, InnerMany>), grid, block, 0, s, HE_HEAD_ARGS(head), many);     \
+            hipLaunchKernelGGL((ntt_inner_kernel<BE, SPLIT, STREAM, PRODUCTS, InnerMany>), grid, block, 0, s, HE_HEAD_ARGS(head), many); \
     } while (0)
-#define HE_INNER(SPLIT, STREAM)                                  \
+#define HE_INNER(SPLIT, STREAM, PRODUCTS)                        \
     do {                                                         \
         if (backend == NTT_BACKEND_MIXED)                        \
-            HE_INNER_BE(NTT_BACKEND_MIXED, SPLIT, STREAM);       \
+            HE_INNER_BE(NTT_BACKEND_MIXED, SPLIT, STREAM, PRODUCTS); \
         else if (backend)                                        \
-            HE_INNER_BE(NTT_BACKEND_FP, SPLIT, STREAM);          \
+            HE_INNER_BE(NTT_BACKEND_FP, SPLIT, STREAM, PRODUCTS);    \
         else                                                     \
-            HE_INNER_BE(NTT_BACKEND_INT, SPLIT, STREAM);         \
+            HE_INNER_BE(NTT_BACKEND_INT, SPLIT, STREAM, false);  \
+    } while (0)
+#define HE_INNER_ONE(STREAM)            \
+    do {                                \
+        if (products)                   \
+            HE_INNER(1, STREAM, true);  \
+        else                            \
+            HE_INNER(1, STREAM, false); \
     } while (0)
     if (split == 4)
-        HE_INNER(4, 0);
+        HE_INNER(4, 0, false);
     else if (split == 2)
-        HE_INNER(2, 0);
+        HE_INNER(2, 0, false);
     else if (stream_keys && stream_words)
-        HE_INNER(1, 3);
+        HE_INNER_ONE(3);
     else if (stream_keys)
-        HE_INNER(1, 1);
+        HE_INNER_ONE(1);
     else if (stream_words)
-        HE_INNER(1, 2);
-    else if (read_twiddles)
-        HE_INNER(1, 4);
+        HE_INNER_ONE(2);
     else
-        HE_INNER(1, 0);
+        HE_INNER_ONE(0);
+#undef HE_INNER_ONE
 #undef HE_INNER
 #undef HE_INNER_BE
     return hipGetLastError();

@@ -17,7 +17,9 @@ def capi():
 
 
 @pytest.mark.parametrize("bits,size_p,L", [([60] + [40] * 23 + [60] * 8, 8, 24),     # three digits: 448 limbs in all
-                                            ([60] + [40] * 17 + [60] * 3, 3, 16)])    # five digits and a limb: 444
+                                            ([60] + [40] * 17 + [60] * 3, 3, 16),     # five digits and a limb: 444
+                                            ([60] + [40] * 10 + [60], 1, 11),         # the most digits that work their twiddles out: 464
+                                            ([60] + [40] * 11 + [60], 1, 12)])        # the first that read them: 542
 def test_key_words_past_the_caches_on_mixed_chains(oracle, capi, bits, size_p, L):
     cahel, parms, ctx, p = make_pair(oracle, 16, bits, size_p)
     lib, h, n, beta = capi.lib(), ctx.he_handle(), p.n, -(-L // size_p)
