@@ -1662,14 +1662,21 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
             hipLaunchKernelGGL((ntt_blocks_kernel<FWD, EPI, LOOP, NTT_BACKEND_INT, false>), grid, block, 0, s, HE_HEAD_ARGS(head), extra); \
     } while (0)
     const bool loop = a.batch > 1 || a.groups;
-    // Twiddles worked out (FpProducts): in front of an epilogue always; by itself a pass over 32 * 2^16 words finds them in the L2s in a repeated
+    // Twiddles worked out (FpProducts).  In front of an epilogue, on FP64 from one wave for every SIMD on: fewer wait for their two products
+    // more than for what they move.  us in this pass, waves, read / worked out: 64 3.40 / 3.50, 256 3.24 / 3.42, 448 3.68 / 3.78, 512 3.36 / 3.52, 1024 4.16 / 4.16,
+    // 1280 4.68 / 4.56, 2048 5.60 / 5.10, 4096 8.24 / 7.42; a whole product of 4 + 1 limbs of 2^14 (384 waves) 22.95 / 23.04, of 8 + 2 of 2^12 26.60 / 26.69, of 3 + 1
+    // of 2^13 19.96 / 20.06.  With limbs of both arithmetics the integers' waves are the longer ones: 4 + 1 of 2^13 24.53 / 24.39, rotation, 2 + 1 of 2^14 20.55 /
+    // 20.48, 24 + 8 of 2^12 42.58 / 42.54.  By itself a pass over 32 * 2^16 words finds them in the L2s in a repeated
     // transform, one over 36 does not.  Transforms, us read / worked out: 2 x 16 limbs of 2^16 words 15.1 / 15.6, 2 x 20 19.1 / 18.0, 2 x 24 back 22.8 /
     // 21.0, of 60 / 40 bits 23.7 / 22.0, 3 x 24 of 2^15 17.3 / 16.8, 4 x 24 of 2^14 12.1 / 12.7.
     const bool products = ((uint64_t)kinds * repeats << a.log_n) >= (uint64_t)36 << 16 && !a.in_galois;
+    const bool epi_products = backend == NTT_BACKEND_MIXED || (uint64_t)kinds * repeats * blocks >= 4 * (uint64_t)a.cus;
     if (epi && loop)
         HE_LAUNCH(true, true, true, false);
-    else if (epi)
+    else if (epi && epi_products)
         HE_LAUNCH(true, true, false, true);
+    else if (epi)
+        HE_LAUNCH(true, true, false, false);
     else if (forward && loop)
         HE_LAUNCH(true, false, true, false);
     else if (forward && products)

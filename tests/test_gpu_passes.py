@@ -484,6 +484,24 @@ def test_moddown_and_rescale_of_a_mixed_chain(oracle, capi, logn, L, polys):
     assert (low.numpy() == p.rescale(np.ascontiguousarray(cx[:, :L]))).all()
 
 
+@pytest.mark.parametrize("bits", [[50] * 17, [50, 49, 30] * 5 + [50, 49], [60] + [40] * 15 + [60]])
+@pytest.mark.parametrize("L", [15, 16])
+def test_epilogues_on_both_sides_of_the_twiddles_worked_out(oracle, capi, bits, L):
+    """FP64: 1024 waves at 256 CUs, ModDown of 16 limbs of 2^13 words; the rescale has a limb less.  Words of q - 1 throughout, and random ones."""
+    cahel, parms, ctx, p = make_pair(oracle, 13, bits, 1)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    tables = list(range(L)) + [p.size_q]
+    cx = rand_limbs(p, np.random.default_rng(L), tables, n_polys=2)
+    for i, t in enumerate(tables):
+        cx[1, i] = p.moduli[t] - 1
+    dcx, dct, ws = DeviceArray(capi, host=cx), DeviceArray(capi, host=cx[:, :L]), DeviceArray(capi, shape=(2, L, n))
+    down, low = DeviceArray(capi, shape=(2, L, n)), DeviceArray(capi, shape=(2, L - 1, n))
+    capi.check(lib.he_moddown(h, L, dcx.ptr, down.ptr, 2, 0, ws.ptr, None))
+    capi.check(lib.he_rescale(h, dct.ptr, low.ptr, 2, L, ws.ptr, None))
+    assert (down.numpy() == np.stack([p.moddown(x) for x in cx])).all()
+    assert (low.numpy() == p.rescale(np.ascontiguousarray(cx[:, :L]))).all()
+
+
 @pytest.mark.parametrize("chain", sorted(CHAINS))
 @pytest.mark.parametrize("logn,L,items", [(12, 8, 19), (12, 8, 20), (13, 5, 16), (15, 2, 5), (15, 2, 6)])
 def test_products_on_both_sides_of_the_dealt_tensor_product(oracle, capi, chain, logn, L, items):
