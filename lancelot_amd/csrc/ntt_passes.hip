@@ -1668,8 +1668,11 @@ hipError_t launch_ntt_blocks(NttArgs a, uint32_t n_polys, bool forward, int back
     // of 2^13 19.96 / 20.06.  With limbs of both arithmetics the integers' waves are the longer ones: 4 + 1 of 2^13 24.53 / 24.39, rotation, 2 + 1 of 2^14 20.55 /
     // 20.48, 24 + 8 of 2^12 42.58 / 42.54.  By itself a pass over 32 * 2^16 words finds them in the L2s in a repeated
     // transform, one over 36 does not.  Transforms, us read / worked out: 2 x 16 limbs of 2^16 words 15.1 / 15.6, 2 x 20 19.1 / 18.0, 2 x 24 back 22.8 /
-    // 21.0, of 60 / 40 bits 23.7 / 22.0, 3 x 24 of 2^15 17.3 / 16.8, 4 x 24 of 2^14 12.1 / 12.7.
-    const bool products = ((uint64_t)kinds * repeats << a.log_n) >= (uint64_t)36 << 16 && !a.in_galois;
+    // 21.0, of 60 / 40 bits 23.7 / 22.0, 3 x 24 of 2^15 17.3 / 16.8, 4 x 24 of 2^14 12.1 / 12.7.  A job list's words (hoisting's ModUp) come from one
+    // buffer and go to another: FP64 from 64 on, 36 limbs 10.46 / 10.50, 49 12.40 / 12.56, 64 15.26 / 15.24, 72 17.38 / 17.20, 100 20.80 / 20.38; 60 / 40 bits 36 limbs
+    // 13.32 / 13.28, 49 16.12 / 16.02, 72 22.02 / 21.68.
+    const uint64_t line = a.jobs && backend == NTT_BACKEND_FP ? 64 : 36;
+    const bool products = ((uint64_t)kinds * repeats << a.log_n) >= line << 16 && !a.in_galois;
     const bool epi_products = backend == NTT_BACKEND_MIXED || (uint64_t)kinds * repeats * blocks >= 4 * (uint64_t)a.cus;
     if (epi && loop)
         HE_LAUNCH(true, true, true, false);

@@ -484,6 +484,20 @@ def test_moddown_and_rescale_of_a_mixed_chain(oracle, capi, logn, L, polys):
     assert (low.numpy() == p.rescale(np.ascontiguousarray(cx[:, :L]))).all()
 
 
+@pytest.mark.parametrize("bits", [[50] * 20, [60] + [40] * 15 + [60] * 4])
+@pytest.mark.parametrize("L", [15, 16])
+def test_modup_on_both_sides_of_the_twiddles_worked_out(oracle, capi, bits, L):
+    """FP64: 61 and 64 transformed limbs of 2^16 words.  Both arithmetics work them out from 36 on."""
+    cahel, parms, ctx, p = make_pair(oracle, 16, bits, 4)
+    lib, h, n = capi.lib(), ctx.he_handle(), p.n
+    c = rand_limbs(p, np.random.default_rng(L), range(L))
+    for i in range(0, L, 3):
+        c[i] = p.moduli[i] - 1
+    dc, dy, ws = DeviceArray(capi, host=c), DeviceArray(capi, shape=(4, L + 4, n)), DeviceArray(capi, shape=(2 * L, n))
+    capi.check(lib.he_modup(h, L, dc.ptr, dy.ptr, ws.ptr, None))
+    assert (dy.numpy() == p.modup(c)).all()
+
+
 @pytest.mark.parametrize("bits", [[50] * 17, [50, 49, 30] * 5 + [50, 49], [60] + [40] * 15 + [60]])
 @pytest.mark.parametrize("L", [15, 16])
 def test_epilogues_on_both_sides_of_the_twiddles_worked_out(oracle, capi, bits, L):
