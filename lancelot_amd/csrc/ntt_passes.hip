@@ -1088,7 +1088,8 @@ __device__ __forceinline__ void product_end_block(const NttArgs &a, const EndExt
     }
 }
 
-template <int BE, int STREAM>
+// PRODUCTS: see FpProducts (launch_product_end says when)
+template <int BE, int STREAM, bool PRODUCTS>
 __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_PARAMS, EndExtra x) {
     NttArgs a;
     set_head(a, HE_HEAD_NAMES);
@@ -1097,7 +1098,10 @@ __global__ __launch_bounds__(64 * kBlockWaves) void product_end_kernel(HE_HEAD_P
     const uint32_t id = limb_block(h4, lr - 1, h0) * kBlockWaves + w, blk = id & ((1u << lr) - 1);
     const Job job = decode_job(a, id >> lr);
     const bool fp = BE == NTT_BACKEND_FP || (BE == NTT_BACKEND_MIXED && ((a.fp_mask >> job.table) & 1));
-    if (BE != NTT_BACKEND_INT && fp) product_end_block<STREAM>(a, x, job, FpProducts<false>{fp_arith(a, job.table)}, blk, lane);
+    if (BE != NTT_BACKEND_INT && fp) {
+        const typename std::conditional<PRODUCTS, FpProducts<false>, FpArith>::type ar{fp_arith(a, job.table)};
+        product_end_block<STREAM>(a, x, job, ar, blk, lane);
+    }
     if constexpr (BE != NTT_BACKEND_FP) {
         if (!fp) product_end_block<STREAM>(a, x, job, int_arith(a, job.table), blk, lane);
     }
@@ -1853,21 +1857,29 @@ hipError_t launch_product_end(const NttArgs &args, const ProductEnd &x, uint32_t
     const EndExtra extra{x.cx, x.ct2, x.out, x.p_inv, x.q_last_inv, x.cx_stride};
     // (the factors from half the last-level cache on: smaller ones may be in it for the caller's next product of them)
     const int stream = !stream_products(items, x.L, a.log_n) ? 0 : ((uint64_t)items * x.L << a.log_n) >= (uint64_t)64 << 16 ? 2 : 1;
-#define HE_END(BE)                                                                                         \
-    do {                                                                                                   \
-        if (stream == 2)                                                                                   \
-            hipLaunchKernelGGL((product_end_kernel<BE, 2>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
-        else if (stream)                                                                                   \
-            hipLaunchKernelGGL((product_end_kernel<BE, 1>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
-        else                                                                                               \
-            hipLaunchKernelGGL((product_end_kernel<BE, 0>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);    \
+    // Twiddles worked out (FpProducts): FP64 always; with limbs of both arithmetics, whose integers keep a launch waiting, from 11 limbs of
+    // 2^16 words on, when a launch's twiddles are more than its L2s keep for all of its items.  us in this kernel read / worked out, FP64: 8 x 4 + 1
+    // limbs of 2^14 8.22 / 7.44, 2 x 8 + 2 of 2^16 13.16 / 12.64, 16 x 3 + 1 26.90 / 27.24, 8 x 24 + 8 147.1 / 141.4; 60 / 40 bits 8 x 4 + 1 of 2^14 9.18 / 9.66, 2 x 8 + 2 of
+    // 2^16 14.54 / 14.96, 32 x 6 + 2 of 2^14 34.74 / 35.60, 8 x 8 + 2 of 2^16 45.38 / 45.52, 8 x 12 + 4 68.21 / 68.07, 2 x 16 + 4 27.84 / 26.78, 3 x 24 + 8 of 2^15 29.64 /
+    // 28.64, 8 x 24 + 8 of 2^16 147.0 / 141.9.
+    const bool products = ((uint64_t)a.map.limbs << a.log_n) >= (uint64_t)11 << 16;
+#define HE_END(BE, PRODUCTS)                                                                                       \
+    do {                                                                                                           \
+        if (stream == 2)                                                                                           \
+            hipLaunchKernelGGL((product_end_kernel<BE, 2, PRODUCTS>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);  \
+        else if (stream)                                                                                           \
+            hipLaunchKernelGGL((product_end_kernel<BE, 1, PRODUCTS>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);  \
+        else                                                                                                       \
+            hipLaunchKernelGGL((product_end_kernel<BE, 0, PRODUCTS>), grid, block, 0, s, HE_HEAD_ARGS(h), extra);  \
     } while (0)
-    if (backend == NTT_BACKEND_MIXED)
-        HE_END(NTT_BACKEND_MIXED);
+    if (backend == NTT_BACKEND_MIXED && products)
+        HE_END(NTT_BACKEND_MIXED, true);
+    else if (backend == NTT_BACKEND_MIXED)
+        HE_END(NTT_BACKEND_MIXED, false);
     else if (backend)
-        HE_END(NTT_BACKEND_FP);
+        HE_END(NTT_BACKEND_FP, true);
     else
-        HE_END(NTT_BACKEND_INT);
+        HE_END(NTT_BACKEND_INT, false);
 #undef HE_END
     return hipGetLastError();
 }

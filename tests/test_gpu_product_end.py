@@ -63,7 +63,9 @@ def test_products_equal_their_steps(oracle, capi, log_n, bits, size_p, L, items,
 @pytest.mark.parametrize("log_n,bits,size_p,L,items", [(13, [60] * 8 + [60] * 2, 2, 8, 16),             # integers: on the line, 2^20 words
                                                         (15, [60] * 6 + [60], 1, 6, 6),                  # one special prime
                                                         (14, [60] + [40] * 5 + [60] * 2, 2, 6, 6),       # both arithmetics
-                                                        (16, [50] * 4 + [50] * 2, 2, 4, 4)])             # FP64: on the line
+                                                        (16, [50] * 4 + [50] * 2, 2, 4, 4),              # FP64: on the line
+                                                        (16, [60] + [40] * 11 + [60] * 4, 4, 12, 2),     # both: twiddles worked out, the fewest
+                                                        (16, [60] + [40] * 11 + [60] * 4, 4, 11, 2)])    # ... and read
 def test_products_equal_the_oracle(oracle, capi, log_n, bits, size_p, L, items):
     cahel, parms, ctx, p = make_pair(oracle, log_n, bits, size_p)
     lib, h, n = capi.lib(), ctx.he_handle(), p.n
