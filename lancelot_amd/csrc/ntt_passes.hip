@@ -1453,12 +1453,14 @@ bool spread_encryption(const NttArgs &a, int backend, uint32_t items, uint64_t w
     return 2 * wgs >= halves * a.cus;
 }
 
-// Encryption with one special prime (encrypt_products_kernel), which is shorter: limbs of 2^16 words always, of 2^15 up to 16 of them, of fewer a
-// single encryption's.  Together / dealt, us, limbs x items: 2^16, 4 x 1 27.8 / 27.0, 4 x 10 97.5 / 93.3, 4 x 20 172 / 165, 10 x 10 189 / 178, 21 x 1
-// 55.8 / 54.6, but 4 x 4 52.2 / 53.0; 2^15, 10 x 1 28.8 / 27.8, 4 x 4 36.2 / 35.1, 10 x 2 38.5 / 39.5, 21 x 1 40.4 / 41.0, 4 x 6 45.4 / 46.8, 10 x 4
-// 54.2 / 56.2; 2^14, 13 x 1 23.7 / 22.6, 21 x 1 28.3 / 27.2, 4 x 2 21.2 / 21.1, 4 x 4 24.8 / 25.7, 10 x 4 39.8 / 41.3; 2^13, 10 x 1 18.5 / 18.6, 10 x 4 26.5 / 28.0.
-bool spread_products(const NttArgs &a, int backend, uint32_t items, uint32_t limbs) {
+// Encryption with one special prime (encrypt_products_kernel), which is shorter: limbs of 2^16 words, of 2^15 up to 16 of them, of fewer a
+// single encryption's; not four items of up to eight limbs: half an item an XCD, together or dealt out.  Together / dealt, us, limbs x items: 2^16, 4 x 1
+// 27.0 / 25.8, 4 x 3 46.9 / 46.1, 4 x 4 51.9 / 54.1, 4 x 5 64.0 / 61.7, 4 x 10 96.3 / 93.4, 4 x 20 169 / 163, 3 x 4 44.9 / 44.9, 7 x 1 32.9 / 32.4, 7 x 2 47.8 / 48.3,
+// 7 x 4 69.6 / 70.5, 7 x 8 120 / 114, 13 x 1 44.9 / 43.0, 13 x 4 106.6 / 102.2; 2^15, 10 x 1 28.4 / 27.3, 4 x 2 26.9 / 26.5, 4 x 4 34.9 / 35.4, 4 x 5 39.7 / 40.5, 10 x 2
+// 37.8 / 38.3, 4 x 8 50.5 / 53.1; 2^14, 13 x 1 23.8 / 22.9, 21 x 1 27.9 / 26.6, 4 x 2 22.0 / 22.1; 2^13, 10 x 1 18.5 / 18.6, 10 x 4 26.5 / 28.0.
+bool spread_encrypt_products(const NttArgs &a, int backend, uint32_t items, uint32_t limbs) {
     if (backend != NTT_BACKEND_MIXED || 2 * ((uint64_t)items * limbs << (a.log_n - 8)) < 3 * (uint64_t)a.cus) return false;
+    if (items == 4 && limbs <= 8) return false;
     return a.log_n >= 16 || (a.log_n == 15 ? (uint64_t)items * limbs <= 16 : items == 1);
 }
 
@@ -1921,7 +1923,7 @@ hipError_t launch_encrypt_products(const NttArgs &args, const uint64_t *pk, uint
     for (uint32_t first = 0; first < items; first += per_launch) {
         const uint32_t now = items - first < per_launch ? items - first : per_launch;
         const dim3 grid(now * wgs_per_item);
-        a.spread = spread_products(a, backend, items, L + K);
+        a.spread = spread_encrypt_products(a, backend, items, L + K);
         const NttHead head = ntt_head(a, grid.x, first);
         if (backend == NTT_BACKEND_MIXED)
             hipLaunchKernelGGL(encrypt_products_kernel<NTT_BACKEND_MIXED>, grid, block, 0, s, HE_HEAD_ARGS(head), a.pro_itw, wide);

@@ -445,10 +445,12 @@ def test_conversions_on_both_sides_of_the_matrix_kernel(oracle, capi, size_p, L,
 
 
 @pytest.mark.parametrize("logn,L,size_p,items", [(14, 3, 1, 1), (13, 8, 1, 1), (13, 10, 2, 1), (14, 3, 1, 2), (14, 4, 2, 2), (12, 24, 8, 2), (14, 8, 1, 4),
-                                                 (14, 10, 2, 4), (15, 2, 1, 4), (15, 2, 1, 5), (15, 10, 2, 2)])
+                                                 (14, 10, 2, 4), (15, 2, 1, 4), (15, 2, 1, 5), (15, 10, 2, 2),
+                                                 (16, 3, 1, 4), (16, 3, 1, 5), (15, 3, 1, 3), (15, 8, 1, 2)])
 def test_encryption_of_a_mixed_chain(oracle, capi, logn, L, size_p, items):
     """Encryption's blocks pass deals the limbs' workgroups to all XCDs for up to four items, from 3 workgroups for two CUs on, with limbs
-    of 2^14 words and less from 3 a CU for two items and from 12 for more; its ModDown from 3 a CU on for one item or limbs of 2^15."""
+    of 2^14 words and less from 3 a CU for two items and from 12 for more; with one special prime limbs of 2^16 words, up to 16 of 2^15 and
+    single encryptions, but not four items of few limbs; its ModDown from 3 a CU on for one item or limbs of 2^15."""
     bits = [60] + [40] * (L - 1) + [60] * size_p
     cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
     lib, h, n = capi.lib(), ctx.he_handle(), p.n
