@@ -465,8 +465,6 @@ struct FpArith {
         }
         return t;
     }
-    // a b mod q, centred, for centred a and b
-    __device__ __forceinline__ double twiddle(double a, double b) const { return fp_reduce(fp_mulmod(a, b, m), m); }
     // the last block of a wave's 256 words (Tile4<8, 8>, `scale` as in load_tw)
     __device__ __forceinline__ Tw load_last(uint32_t scale, uint32_t t) const { return load<2, false>((scale << 6) + t); }
     __device__ __forceinline__ void ct1(V &x, V &y, double w) const {

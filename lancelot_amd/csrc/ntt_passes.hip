@@ -510,7 +510,7 @@ __global__ __launch_bounds__(64 * kBlockWaves) void ntt_blocks_kernel(HE_HEAD_PA
 }
 
 // Sum over the digits of (word x key word) for four words of both key polynomials.
-// FP64: a transformed word enters as the last stage leaves it (at most 3.7 q: a term below 1.9 q), the sums are reduced after
+// FP64: a transformed word enters as the last stage leaves it (at most 3.63 q: a term below 1.9 q), the sums are reduced after
 // every fourth digit and stay below 8 q.  Integers: 128-bit sums of at most 64 products below 2^122 of canonical words, or, with primes
 // below 2^60, of at most 32 products of words as the last stage leaves them (below 8 q):
 // a wave's share of kMaxDigits, since only waves that share a block leave them so.
