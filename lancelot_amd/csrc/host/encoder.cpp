@@ -257,9 +257,9 @@ void CAHELGPUCKKSEncoder::encode(const CAHELGPUContext &context, const std::vect
 // the first `count` complex values of the decoding, interleaved (re, im), into v
 void CAHELGPUCKKSEncoder::decode_values(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain,
                                         std::size_t count, std::vector<double> &v) {
-    count = decode_count(context, plain, count);
+    const std::size_t ss = decode_count(context, plain, 0);   // (once: it may change on another thread)
+    if (count == 0 || count > ss) count = ss;
     const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
-    const std::size_t ss = sparse_slots_;
 
     he_context *h = context.handle();
     DeviceBuffer ws(he_ckks_workspace_words(h, limbs));
@@ -299,12 +299,11 @@ std::size_t CAHELGPUCKKSEncoder::decode_count(const CAHELGPUContext &context, co
 void CAHELGPUCKKSEncoder::decode_real(const CAHELGPUContext &context, const CAHELGPUPlaintext &plain, std::size_t count,
                                       double *destination) {
     he_context *h = context.handle();
-    const uint32_t limbs = (uint32_t)plain.coeff_modulus_size();
-    DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, (uint32_t)sparse_slots_));
+    const uint32_t limbs = (uint32_t)plain.coeff_modulus_size(), slots = (uint32_t)sparse_slots_;   // (once: it may change on another thread)
+    DeviceBuffer ws(he_ckks_decode_real_workspace_words(h, limbs, slots));
     PinnedRing &ring = PinnedRing::of_thread();
     double *host = static_cast<double *>(ring.take(count * sizeof(double)));
-    const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, (uint32_t)sparse_slots_, plain.scale(), host, (uint32_t)count, ws.get(),
-                                           context.stream());
+    const int status = he_ckks_decode_real(h, plain.lane_data(), limbs, slots, plain.scale(), host, (uint32_t)count, ws.get(), context.stream());
     if (status != HE_OK) ring.fence(context.stream());   // (what was launched before the failure may still write the block)
     check_status(status, "he_ckks_decode_real");
     check_status(he_stream_synchronize(context.stream()), "synchronisation failed");

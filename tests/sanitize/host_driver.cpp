@@ -353,6 +353,21 @@ int main(int argc, char **argv) {
             return true;
         };
         REQUIRE(encoder.decoded_slots() == few && decoded(few));
+        {   // a decoding by itself: its workspace is for the slots that it decodes
+            CAHELGPUPlaintext p(context);
+            secret.decrypt(context, cts[1], p);
+            std::vector<double> out(few);
+            mock_meanwhile = [&] {
+                encoder.reset_sparse_slots();
+                CAHELGPUPlaintext q(context);
+                encoder.encode(context, std::vector<double>(2 * few, 0.5), 1048576.0, q);
+            };
+            encoder.decode_real(context, p, few, out.data());
+            REQUIRE(out[0] == value(1, 0) && out[few - 1] == value(1, few - 1) && encoder.decoded_slots() == 2 * few);
+            mock_meanwhile = nullptr;
+            encoder.reset_sparse_slots();
+            encoder.encode(context, std::vector<double>(few, 0.5), 1048576.0, message);
+        }
         int calls = 0;
         mock_meanwhile = [&] {
             if (++calls == 3) encoder.reset_sparse_slots();

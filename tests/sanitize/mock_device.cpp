@@ -18,7 +18,8 @@ struct he_context {
 
 // the call that fails from now on, or nullptr
 const char *mock_failing = nullptr;
-// whether he_ckks_decode_real succeeds; what happens during each he_decrypt_flood (another thread's doing)
+// whether he_ckks_decode_real succeeds; what happens during each he_decrypt_flood and each
+// question for a decoding's workspace (another thread's doing)
 bool mock_decodes = false;
 std::function<void()> mock_meanwhile;
 
@@ -225,11 +226,18 @@ size_t he_ckks_workspace_words(const he_context *, uint32_t) { return 0; }
 int he_ckks_decode(const he_context *, const uint64_t *, uint32_t, uint32_t, double, double *, uint64_t *, he_stream) {
     return HE_E_UNSUPPORTED;
 }
-size_t he_ckks_decode_real_workspace_words(const he_context *, uint32_t, uint32_t) { return 0; }
+// a workspace is for as many slots as were asked for last
+static uint32_t decode_workspace_slots = 0;
+size_t he_ckks_decode_real_workspace_words(const he_context *, uint32_t, uint32_t slots) {
+    decode_workspace_slots = slots;
+    if (mock_meanwhile) mock_meanwhile();
+    return 0;
+}
 // "Decodes" later: the bits of word i as value i.  Unless mock_decodes, fails behind its first launches: what they write comes later all the same.
 int he_ckks_decode_real(const he_context *, const uint64_t *plain, uint32_t, uint32_t slots, double, double *out, uint32_t count, uint64_t *,
                         he_stream stream) {
     if (count > slots) return HE_E_INVALID_ARGUMENT;
+    if (slots > decode_workspace_slots) std::abort();
     if (mock_decodes) {
         queues[stream].push_back([=] { std::memcpy(out, plain, count * sizeof(double)); });
         return HE_OK;
