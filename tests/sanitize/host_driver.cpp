@@ -384,6 +384,67 @@ int main(int argc, char **argv) {
         REQUIRE(decoded(n / 2) && encoder.decoded_slots() == few);
         mock_meanwhile = nullptr;
         mock_decodes = false;
+
+        // a batch whose caller enqueues more work, staging blocks of its own with it, before the values are waited for, or fails there
+        const std::size_t items = cts.size(), count = 5;
+        std::vector<double> pairs(2 * items * count);
+        PinnedRing &ring = PinnedRing::of_thread();
+        secret.decrypt_decode_many(context, ptrs, few, count, pairs.data(), true, [&] {
+            for (int i = 0; i < 2 * PinnedRing::kBlocks + 1; i++) {
+                std::memset(ring.take(2 * items * count * sizeof(double)), 0x55, 2 * items * count * sizeof(double));
+                ring.fence(current_stream());
+            }
+        });
+        for (std::size_t i = 0; i < pairs.size(); i++) REQUIRE(pairs[i] == value(i / (2 * count), i / 2 % count));
+        REQUIRE(refuses([&] { secret.decrypt_decode_many(context, ptrs, few, count, pairs.data(), true, [] { throw std::runtime_error("meanwhile"); }); }));
+        secret.decrypt_decode_many(context, {}, few, count, pairs.data(), true, [&] { pairs[0] = -1.0; });
+        REQUIRE(pairs[0] == -1.0);
+    }
+
+    // ---- blocks of the page-locked ring that are held: never handed out meanwhile, afterwards only when their work is done ----
+    {
+        set_lane(0);
+        const he_stream stream = current_stream();
+        const std::vector<double> written(16, 3.5);
+        const std::size_t bytes = written.size() * sizeof(double);
+        PinnedRing ring;
+        auto started = [&] {   // a block that work on the stream will write
+            void *block = ring.take(bytes);
+            std::memset(block, 0, bytes);
+            check_status(he_memcpy_h2d_async(block, written.data(), bytes, stream), "copy");
+            return block;
+        };
+        auto handed_out = [&](const void *block, int times) {
+            bool met = false;
+            for (int i = 0; i < times; i++) met = ring.take(bytes) == block || met;
+            return met;
+        };
+        auto done = [&](const void *block) { return std::memcmp(block, written.data(), bytes) == 0; };
+        for (int turn = 0; turn < PinnedRing::kBlocks; turn++) {   // (the held blocks lie at every place of the ring)
+            void *one = started();
+            {
+                PinnedRing::Held held(ring, stream);
+                REQUIRE(!handed_out(one, 2 * PinnedRing::kBlocks) && !done(one));
+                void *two = started();
+                REQUIRE(two != one);
+                PinnedRing::Held first(ring, stream);
+                PinnedRing::Held second = std::move(first);
+                REQUIRE(!handed_out(one, 2 * PinnedRing::kBlocks) && !handed_out(two, 2 * PinnedRing::kBlocks) && !done(two));
+                second.wait();
+                REQUIRE(done(two) && !handed_out(two, 2 * PinnedRing::kBlocks));
+            }
+            REQUIRE(done(one) && handed_out(one, PinnedRing::kBlocks));
+            void *thrown = nullptr;
+            REQUIRE(refuses([&] {
+                thrown = started();
+                PinnedRing::Held held(ring, stream);
+                throw std::runtime_error("while a block is held");
+            }));
+            REQUIRE(!done(thrown));   // (nobody has waited)
+            while (ring.take(bytes) != thrown) REQUIRE(!done(thrown));
+            REQUIRE(done(thrown));    // its event was waited for before it was handed out
+            (void)ring.take(bytes);
+        }
     }
 
     // a record of another level, a truncated one and one with a wrong degree are refused
