@@ -148,6 +148,53 @@ def test_mixed_conversions_of_the_largest_words(oracle, capi, logn, bits, size_p
         assert (dout.numpy() == p.rescale(np.stack([p.add(ct[b], ks[b]) for b in range(2)]))).all(), ("keyswitch_rescale", L)
 
 
+def inverses(x, q):
+    """x^-1 mod q of every word (none of them 0): one power and three products a word."""
+    x = [int(w) for w in x]
+    upto = [1]
+    for w in x:
+        upto.append(upto[-1] * w % q)
+    inv, out = pow(upto[-1], q - 2, q), [0] * len(x)
+    for i in range(len(x) - 1, -1, -1):
+        out[i] = upto[i] * inv % q
+        inv = inv * x[i] % q
+    return out
+
+
+@pytest.mark.parametrize("logn,bits,size_p,L", [
+    (12, [60, 50, 30, 49, 60, 20, 60, 60], 2, 6), (12, [60, 50, 30, 49, 60, 60, 60, 60], 2, 5), (14, [40] * 4 + [50] * 3 + [60], 4, 4),
+    (16, [60] + [40] * 3 + [50] * 2 + [60] + [50] + [60] * 8, 8, 7), (16, [50, 49, 30, 60, 60, 60], 2, 4)])
+def test_merged_conversions_of_the_largest_words(oracle, capi, logn, bits, size_p, L):
+    """ModDown and rescale in one: every coefficient of every special limb, and of the limb that the rescale drops, q - 1.  The keys' words
+    are chosen for that: those of the first digit are the wanted sum over its transformed words, those of the others 0."""
+    cahel, parms, ctx, p = make_pair(oracle, logn, bits, size_p)
+    rng = np.random.default_rng(400 + logn)
+    lib, h, K, Q, n = capi.lib(), ctx.he_handle(), p.size_p, p.size_q, p.n
+    special = [Q + i for i in range(K)]
+    top = p.ntt_fwd(np.stack([np.full(n, p.moduli[t] - 1, dtype=np.uint64) for t in special]), special)
+    c = rand_limbs(p, rng, range(L))
+    y = p.modup(c)
+    assert (y[0, L:] != 0).all()
+    evk = [rand_limbs(p, rng, range(p.size_qp), n_polys=2) for _ in range(Q // K)]
+    for d, key in enumerate(evk):
+        for i, t in enumerate(special):
+            q = p.moduli[t]
+            key[:, t] = 0 if d else np.array([int(w) * v % q for w, v in zip(top[i], inverses(y[0, L + i], q))], dtype=np.uint64)
+    cx = p.inner_prod(y, evk)
+    assert all((cx[r, L:] == top).all() for r in range(2))
+    ks = p.key_switch(c, evk)
+    ct, last = rand_limbs(p, rng, range(L), n_polys=2), p.moduli[L - 1]
+    dropped = p.ntt_fwd(np.full((1, n), last - 1, dtype=np.uint64), [L - 1])[0]
+    for r in range(2):
+        ct[r, L - 1] = (dropped + (np.uint64(last) - ks[r, L - 1])) % np.uint64(last)
+    want = p.rescale(np.stack([p.add(ct[r], ks[r]) for r in range(2)]))
+    dev = [DeviceArray(capi, host=k) for k in evk]
+    dc, dct, dout = DeviceArray(capi, host=c), DeviceArray(capi, host=ct), DeviceArray(capi, shape=(2, L - 1, n))
+    ws = DeviceArray(capi, shape=(lib.he_keyswitch_workspace_words(h, L),))
+    capi.check(lib.he_keyswitch_rescale(h, L, dc.ptr, capi.evk_array([d.ptr for d in dev]), dct.ptr, dout.ptr, 0, ws.ptr, None))
+    assert (dout.numpy() == want).all()
+
+
 @pytest.mark.parametrize("no_fused", ["0", "1"])
 @pytest.mark.parametrize("logn,bits,size_p,levels", CASES + [(11, [45, 40, 40, 50], 1, (3, 2)), (12, [60, 40, 50, 45, 30, 59, 60, 60], 2, (6, 3))])
 def test_multiply_relin_rescale_entry_point(oracle, capi, monkeypatch, logn, bits, size_p, levels, no_fused):
