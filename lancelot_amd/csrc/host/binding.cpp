@@ -26,6 +26,19 @@ py::array_t<uint64_t> to_host(const uint64_t *dev, std::vector<py::ssize_t> shap
     return out;
 }
 
+// the values of all slots of every ciphertext; the slot count is read once, under the interpreter's lock: it is what the array holds
+py::array_t<double> decrypt_decode_each(CAHELGPUSecretKey &k, const CAHELGPUContext &c, CAHELGPUCKKSEncoder &e,
+                                        const std::vector<const CAHELGPUCiphertext *> &cts, const std::function<void()> &behind) {
+    const std::size_t slots = e.decoded_slots();
+    py::array_t<double> out((py::ssize_t)(cts.size() * slots));
+    double *values = out.mutable_data();
+    {
+        py::gil_scoped_release release;
+        k.decrypt_decode_each(c, e, cts, slots, values, behind);
+    }
+    return out;
+}
+
 // save / load / to_bytes / from_bytes on top of the C++ stream members (the reference binds none of them)
 template <typename T, typename C>
 void def_serialization(C &cls) {
@@ -187,14 +200,15 @@ PYBIND11_MODULE(pyCAHEL, m) {
              py::arg("context"), py::arg("ciphertexts"), py::arg("slots"), py::arg("count") = 1)
         .def("decrypt_decode_each",
              [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, CAHELGPUCKKSEncoder &e, const std::vector<const CAHELGPUCiphertext *> &cts) {
-                 const std::size_t slots = e.decoded_slots();   // (once, under the interpreter's lock: what the array holds)
-                 py::array_t<double> out((py::ssize_t)(cts.size() * slots));
-                 double *values = out.mutable_data();
-                 {
-                     py::gil_scoped_release release;
-                     k.decrypt_decode_each(c, e, cts, slots, values);
-                 }
-                 return out;
+                 return decrypt_decode_each(k, c, e, cts, nullptr);
+             },
+             py::arg("context"), py::arg("encoder"), py::arg("ciphertexts"))
+        // ... and a mark behind the last of them, which is there when the values are
+        .def("decrypt_decode_each_marked",
+             [](CAHELGPUSecretKey &k, const CAHELGPUContext &c, CAHELGPUCKKSEncoder &e, const std::vector<const CAHELGPUCiphertext *> &cts) {
+                 std::unique_ptr<DeviceMark> mark;
+                 py::array_t<double> values = decrypt_decode_each(k, c, e, cts, [&] { mark = std::make_unique<DeviceMark>(); });
+                 return py::make_tuple(values, std::move(mark));
              },
              py::arg("context"), py::arg("encoder"), py::arg("ciphertexts"))
         // decrypt_decode_complex_many of the ciphertexts and encode_encrypt_many of the values (in this order, as far as what they draw is

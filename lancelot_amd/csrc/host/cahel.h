@@ -441,9 +441,10 @@ public:
     }
     // The real parts of all slots of every ciphertext, one after the other in destination, `slots` each (the encoder's decoded_slots(), read
     // once by who has made the destination): decrypt and decode of each, the next one's enqueued before the values of the one in front are
-    // waited for.  Not in the reference.
+    // waited for.  behind: what the caller enqueues behind all of it before the last values are waited for.  Not in the reference.
     void decrypt_decode_each(const CAHELGPUContext &context, CAHELGPUCKKSEncoder &encoder,
-                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots, double *destination);
+                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots, double *destination,
+                             const std::function<void()> &behind = nullptr);
     const uint64_t *secret_key_array() const { return sk_powers_.get(); }
 
 private:

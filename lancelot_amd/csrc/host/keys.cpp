@@ -288,7 +288,7 @@ void CAHELGPUSecretKey::decrypt_decode_many(const CAHELGPUContext &context, cons
 
 void CAHELGPUSecretKey::decrypt_decode_each(const CAHELGPUContext &context, CAHELGPUCKKSEncoder &encoder,
                                             const std::vector<const CAHELGPUCiphertext *> &ciphers, std::size_t slots,
-                                            double *destination) {
+                                            double *destination, const std::function<void()> &behind) {
     he_context *h = context.handle();
     he_stream st = context.stream();
     PinnedRing &ring = PinnedRing::of_thread();
@@ -317,5 +317,6 @@ void CAHELGPUSecretKey::decrypt_decode_each(const CAHELGPUContext &context, CAHE
         values = host;
         ahead.emplace(std::move(held));
     }
+    if (behind) behind();
     finish();
 }

@@ -478,9 +478,8 @@ def _mask(state: KrumState, scores, constants=None):
     return [[one if order[r] == k else zero for k in range(n_clients)] for r in range(n_clients)], order
 
 
-def _masked_sum(state: KrumState, cts, mask_row):
-    sums = state.cahel.multiply_sum(state.context, [[client[chunk] for client in cts[:len(mask_row)]] for chunk in range(len(cts[0]))], mask_row)
-    return state.sk.decrypt_decode_each(state.context, state.encoder, sums)
+def _masked_sums(state: KrumState, cts, mask_row):
+    return state.cahel.multiply_sum(state.context, [[client[chunk] for client in cts[:len(mask_row)]] for chunk in range(len(cts[0]))], mask_row)
 
 
 def mul_mask_weight(state: KrumState, cts, mask_row):
@@ -491,7 +490,7 @@ def mul_mask_weight(state: KrumState, cts, mask_row):
     t0 = time.perf_counter()
     n_chunks = len(cts[0])
     if state.config.batched:
-        out = _masked_sum(state, cts, mask_row)
+        out = state.sk.decrypt_decode_each(ctx, state.encoder, _masked_sums(state, cts, mask_row))
         state.timings["mask_multiply"] = state.timings.get("mask_multiply", 0.0) + time.perf_counter() - t0
         return out
     out = []
@@ -565,9 +564,10 @@ def gpu_krum_aggregate(updates, config: KrumConfig | None = None, state: KrumSta
             state.context, packed, state.slots, 1, state.encoder, state.pk, _mask_constants(state), state.config.scale)
         mask, order = _mask(state, _unpacked(scores, n_clients), constants)
         masked = _mark(state, "mask", evaluated)
-        # (by the device's clock too: the constants are the mask's time, and the host does not wait for them)
-        weights = _masked_sum(state, cts, mask[0])
-        _mark(state, "mask_multiply", masked)
+        # (by the device's clock too: the constants are the mask's time, and the host does not wait for them.  The mark lies in front of the
+        # wait for the values: one behind it would be another trip to the device, 15 us of a round at 2^13)
+        weights, end = state.sk.decrypt_decode_each_marked(state.context, state.encoder, _masked_sums(state, cts, mask[0]))
+        state.marks.append(("mask_multiply", masked, end))
     else:
         t1 = time.perf_counter()
         enc = [[None] * n_clients for _ in range(n_clients)]

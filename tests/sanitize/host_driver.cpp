@@ -353,6 +353,19 @@ int main(int argc, char **argv) {
             return true;
         };
         REQUIRE(encoder.decoded_slots() == few && decoded(few));
+        {   // what is to be enqueued behind them comes once, in front of the last values
+            std::vector<double> out(cts.size() * few, 0.0);
+            int times = 0;
+            bool early = false;
+            secret.decrypt_decode_each(context, encoder, ptrs, few, out.data(), [&] {
+                times++;
+                early = out[(cts.size() - 1) * few] == 0.0;
+            });
+            REQUIRE(times == 1 && early && out.back() == value(cts.size() - 1, few - 1));
+            secret.decrypt_decode_each(context, encoder, {}, few, nullptr, [&] { times++; });
+            REQUIRE(times == 2);
+            REQUIRE(refuses([&] { secret.decrypt_decode_each(context, encoder, ptrs, few, out.data(), [] { throw std::runtime_error("behind"); }); }));
+        }
         {   // a decoding by itself: its workspace is for the slots that it decodes
             CAHELGPUPlaintext p(context);
             secret.decrypt(context, cts[1], p);
