@@ -52,11 +52,11 @@ BLOCKS = 5
 # with 1 and 8 items), per operation: L2-miss traffic in limbs of 8 N bytes (FETCH_SIZE scaled by 2, WRITE_SIZE by 1: the
 # factors a copy of known size gives) and SQ_INSTS_VALU summed over the kernels.  Constants of the profile, not
 # measured in this run.
-PROFILE = {"single": {"traffic_limbs": 1020.6, "valu_wave_instr": 30.51e6,
+PROFILE = {"single": {"traffic_limbs": 982.0, "valu_wave_instr": 30.65e6,
                       "kernels": "tensor_intt_blocks, ntt_rows (inverse), bconv_rows4 (ModUp), ntt_inner (special "
                                  "limbs leave through the inverse blocks pass), ntt_rows (inverse), bconv_rows4, "
                                  "product_end (d0, d1 and the rescale epilogue)"},
-           "batch": {"traffic_limbs": 808.9, "valu_wave_instr": 26.56e6,
+           "batch": {"traffic_limbs": 793.6, "valu_wave_instr": 26.91e6,
                      "kernels": "per call of 8 operations: tensor_intt_blocks, ntt_rows (inverse), bconv_rows_mx, "
                                 "ntt_inner (items of a block on one XCD, key words shared through L2), ntt_rows "
                                 "(inverse), bconv_rows_mx, product_end (d0, d1 and the rescale epilogue)"}}
