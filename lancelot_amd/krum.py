@@ -62,7 +62,7 @@ class KrumState:
     encoder: object
     slots: int
     # Seconds a phase.  Those of a batched round between marks on the device's queue, by its clock, each from the end of the phase in front;
-    # all others, and the total, by the host's.
+    # all others (the encryption of updates that are not 32-bit floats among them), and the total, by the host's.
     timings: dict = field(default_factory=lambda: {"encode": 0.0, "encrypt": 0.0, "evaluate": 0.0, "decrypt": 0.0})
     marks: list = field(default_factory=list)   # (phase, mark at its start, mark at its end) of the round on its way
 
